@@ -184,8 +184,8 @@ typedef struct kh_model_opts {
 #define KH_FLAG_ATTN_MERGE_FENCED 2
 /* The prompt phase of kh_model_generate*.  The reference feeds the prompt one token per forward pass
  * (demo/main.cpp:20-22), so its prompt phase is, bit for bit, its decode path.  Two batched prompt paths exist here:
- *  - default: prompts with >= 16 fed-only tokens run as fp32-MFMA GEMMs (kh_model_prefill_gemm, 45-60 k prompt
- *    tokens/s on Llama-3.2-1B): K/V rows equal to fp32 round-off, i.e. the greedy continuation can differ from the
+ *  - default: prompts with >= 16 fed-only tokens run as GEMMs on the matrix cores (kh_model_prefill_gemm, 63-130 k
+ *    prompt tokens/s on Llama-3.2-1B): K/V rows equal to fp32 round-off, i.e. the greedy continuation can differ from the
  *    reference's at near-ties (kh_model_first_sample reports the margin of the first sampled step);
  *  - KH_FLAG_PREFILL_EXACT: every prompt runs on the B-token VALU kernels (kh_model_prefill, 5.9 k prompt
  *    tokens/s): K/V rows and every later logit are bit-identical to the token-by-token prompt phase - what a
@@ -324,10 +324,13 @@ int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int32_t n_prom
  * geometries outside the mirrored kernels (head_size <= 32, dim > 4096). */
 int kh_model_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t pos0);
 
-/* The same contract with the contractions as fp32-MFMA GEMMs (csrc/kh_gemm.h): up to 512 prompt
- * tokens share one pass over the weights (a longer prompt is cut into 512-token passes plus a
- * remainder; env KH_PG_CHUNK = 16..512 sets another pass size) (v_mfma_f32_16x16x4_f32, exact fp32 arithmetic, tokens on
- * the MFMA N dimension; int8 weights dequantised per element in registers).  The K/V rows agree
+/* The same contract with the contractions as GEMMs on the matrix cores: up to 2048 prompt tokens share one pass over the
+ * weights (never more than the cache holds; a longer prompt is cut into such passes plus a remainder; env KH_PG_CHUNK =
+ * 16..512 sets another pass size).  Activations and fp32 weights travel as pairs of halves that keep fp32 accuracy, int8
+ * weights are exact in one (csrc/kh_pair.h; the K/V rows are closer to their 64-bit values than those of an fp32 fmaf
+ * chain).  The first call of a model computes a scale per weight row; the weights must not change afterwards.  Widths
+ * that are no multiple of 32 - and hook KH_PG_PAIR=0 - take fp32-MFMA GEMMs instead (csrc/kh_gemm.h: v_mfma_f32_16x16x4_f32,
+ * passes of up to 512 tokens, int8 weights dequantised per element in registers).  The K/V rows agree
  * with the token-by-token path to fp32 round-off (different summation order), not bit for bit.
  * kh_model_generate* use it for prompts with >= 16 fed-only tokens unless the model was created with
  * KH_FLAG_PREFILL_EXACT - so for such prompts the greedy tokens carry this tolerance too and can differ from the
@@ -378,7 +381,8 @@ int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32
 
 /* Tuning / test hooks.  Every hook the library honours (KH_SHAPE_<QKV|WO|FFN|W2|CLS>, KH_RING, KH_ATTN_WG, KH_ATTN_FENCED,
  * KH_ATTN_TLONG, KH_ATTN_DEFER (0 = never merge time splits in the wo kernel), KH_ATTN_DEFER_MAX (active splits up to
- * which it does), KH_PREFILL, KH_PG_<CHUNK|SHAPE_*|SOLO|KZ|ATTN|ATTN_QT|ROPE_FUSE|DEBUG>,
+ * which it does), KH_PREFILL, KH_PG_<CHUNK|PAIR|SHAPE_*|SOLO|KZ|ATTN|ATTN_QT|ROPE_FUSE|DEBUG> (SHAPE_*, SOLO, KZ and
+ * DEBUG belong to the fp32-MFMA GEMMs; a SHAPE_* hook selects them), KH_PAIR_SHAPE (tile,K split of the pair GEMMs),
  * KH_SHAPE_DEBUG, KH_HY_DECODE (0 = single-token batches of layer-list models run on the pass kernels), KH_HY_EXPAND (0 = latent
  * attention of prompts in its absorbed form), KH_HY_TMAX (tokens of one pass, 32 ... 2048), KH_HY_ROWS (16, 64 or 128: row tiles
  * of the attention kernels of a pass)) lives in ONE process-wide key -> value table, seeded once from the KH_* variables of

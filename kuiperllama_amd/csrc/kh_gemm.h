@@ -1,11 +1,12 @@
-// kh_gemm.h — prompt prefill as real GEMMs on the matrix cores.
+// kh_gemm.h — prompt GEMMs on the fp32 matrix cores: the path of widths that are no multiple of 32 (fp32), and the exact
+// counterpart that the pair GEMMs (kh_pair.h, the usual path) are tested against (KH_PG_PAIR=0).
 //
 // The reference feeds the prompt one token per forward pass (demo/main.cpp:20-22): every prompt
 // token streams all weights.  kh_prefill.h already shares one weight pass between 8 (fp32) / 4
 // (int8) tokens on the VALU; here up to KH_PG_TMAX = 512 prompt tokens share ONE pass and the
 // contraction runs on MFMA:  C[rows, T] = W[rows, K] . Xn[T, K]^T  with
 //     v_mfma_f32_16x16x4_f32   (f32 in, f32 accumulate: bit-for-bit a k-ordered fmaf chain,
-//                               MI355X guide §3 — exact fp32, no reduced-precision path)
+//                               exact fp32, no reduced-precision path)
 // Tokens sit on the MFMA N dimension, weight rows on M.  Arithmetic intensity at T = 128 is
 // 64 flop per weight byte (fp32) against a machine balance of ~22, so the GEMMs are MFMA-bound
 // (157 TF f32 peak) and the weights cross HBM once per 128 tokens.

@@ -61,17 +61,6 @@ struct LgCfg {
   static constexpr int LDS = NSTAGE * STAGE;
 };
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// 64 lanes x 16 B from (base + voff[lane]) to LDS [dst + 16 lane], default cache policy
-__device__ __forceinline__ void dma_x4_keep(const void* base, unsigned voff, unsigned dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(voff), "s"(base), "s"(dst)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 template <class T, int BM, int BN, int EPI>
 __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   typedef Tile<T> TL;

@@ -49,6 +49,7 @@ struct Hybrid;  // kh_hybrid.h: a layer-list model
 }  // namespace khm
 using khm::LayerW;
 
+#define KH_PAIR_TMAX 2048   // prompt tokens of one pass on the pair GEMMs
 #define KH_STEP_VARIANTS 3  // kh_model_step.hip::step_variant
 struct kh_model {
   khm::Hybrid* hy = nullptr;  // layer-list model (checkpoint folder); nullptr: a .bin image
@@ -114,6 +115,13 @@ struct kh_model {
   float* pg_part = nullptr;     // partial rows of residual GEMMs that split K across workgroups
   void* pg_ws = nullptr;        // KH_PG_TMAX attention split workspaces
   size_t pg_ws_tok_bytes = 0;
+  // pair GEMMs (kh_pair.h): per layer four scales (k_pair_scales) and the scale of every weight row (fp32), then one scale
+  // per attention output of a pass, then three words per layer
+  float* pair_ws = nullptr;
+  size_t pair_ws_layer = 0;
+  bool pair_ready = false;
+  bool kv_foreign = false;  // cache rows may hold values that this model did not compute (kh_model_write_kv, _get_kv)
+  int pg_rows = 0;  // token rows of the slabs above
   bool pf_ready = false, pg_ready = false;  // set when ALL prefill slabs exist (allocation can fail half-way)
   bool pg_launch_failed = false;
   int32_t* h_words_pin = nullptr;  // pinned mirror of d_words (stop-token check, final copy-out)
@@ -207,4 +215,9 @@ int run_selftests(kh_model* m);
 // ---- kh_model_prefill.hip -------------------------------------------------------------------
 bool prefill_supported(const kh_model* m);  // B-token VALU path
 bool pg_supported(const kh_model* m);       // MFMA GEMM path
+bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int tcap, const float* pair_scale);
+// pair GEMMs (kh_model_pair.hip)
+bool pair_geometry(const kh_config& c);
+int ensure_pair(kh_model* m);  // scales of the weights, once
+int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0);
 }  // namespace khm

@@ -1,0 +1,218 @@
+// kh_model_pair.hip — prompt passes of .bin models on the pair GEMMs (kh_pair.h): scales once per model, launch shapes,
+// one pass of up to KH_PAIR_TMAX prompt tokens.  The reference feeds the prompt one token per forward pass
+// (demo/main.cpp:20-22).  gfx950 only.
+#include <stdio.h>
+#include <stdlib.h>
+
+#include <algorithm>
+#include <vector>
+
+#include "kh_model_internal.h"
+#include "kh_pair.h"
+
+using namespace khm;
+
+namespace {
+// Tile and K split of one GEMM from a model of the busiest CU: a workgroup's stage takes at least `lat` (one or more stages
+// in flight against memory latency), and `n` workgroups side by side on a CU take n `sat` per stage together.  Both numbers
+// (us) were fitted to 18 tile / split combinations of the four GEMMs of Llama-3.2-1B fp32 and Llama-2-7B int8 at 40 ... 2000
+// tokens: the choice is on average 0.6 % (fp32) and 0.3 % (int8) behind the fastest combination measured, 5 % at worst.
+// Against the tiled fp32-MFMA kernel (k_pg_gemm), us at 40 / 128 / 512 / 2000 tokens, w1 + w3 of either model:
+// 34 / 45 / 102 / 376 against 46 / 76 / 287 / 1089 (fp32); 55 / 85 / 222 / 767 against 126 / 210 / 792 / 3032 (int8).
+// Only wq + wk + wv of 64 fp32 tokens or less were faster there (18 us against 24).
+struct PairShape {
+  int tile;  // index into kPairTiles
+  int kz;    // K slices across workgroups (residual GEMMs)
+};
+struct PairTile {
+  int bm, bn, occ;  // occ: workgroups that share a CU
+  double lat, sat;
+};
+const PairTile kPairTiles[2][4] = {
+    {{128, 128, 2, 1.44, 0.73}, {64, 128, 2, 0.57, 0.445}, {32, 128, 2, 0.40, 0.315}, {32, 64, 2, 0.20, 0.30}},  // fp32
+    {{112, 128, 2, 1.22, 0.95}, {64, 128, 2, 0.72, 0.63}, {32, 128, 2, 0.53, 0.42}, {128, 256, 1, 1.95, 1.95}}};  // int8
+
+PairShape pair_shape(bool q, int T, int N, int K, bool resid) {
+  PairShape best{0, 1};
+  double best_us = -1.0;
+  for (int i = 0; i < 4; ++i)
+    for (int kz = 1; kz <= (resid ? KH_PG_KZ_MAX : 1); kz *= 2) {
+      const PairTile& t = kPairTiles[q][i];
+      const int stages = K / (q ? 64 : 32);
+      if (kz > 1 && stages / kz < 4) break;
+      const long wgs = (long)((N + t.bn - 1) / t.bn) * ((T + t.bm - 1) / t.bm) * kz;
+      const long per_cu = (wgs + 255) / 256, rest = per_cu % t.occ;
+      double us = (double)(per_cu / t.occ) * std::max(t.lat, t.occ * t.sat);
+      if (rest) us += std::max(t.lat, (double)rest * t.sat);
+      us *= (double)stages / kz;
+      if (kz > 1) us += (double)kz * T * N * 8 / 4.0e6;  // partial rows, written and read back at 4 TB/s
+      if (best_us < 0 || us < best_us) {
+        best_us = us;
+        best = PairShape{i, kz};
+      }
+    }
+  return best;
+}
+
+template <bool Q, int EPI, int TM, int TN, int WM, int WN, int NST>
+int pair_go(hipStream_t s, KhPairArgs a, int kz) {
+  typedef PairCfg<Q, TM, TN, WM, WN, NST> C;
+  auto kern = k_pair_gemm<Q, EPI, TM, TN, WM, WN, NST>;
+  if (C::LDS > 64 * 1024) {  // the dynamic-LDS opt-in is per (device, kernel): once
+    static thread_local std::vector<int> done;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    bool hit = false;
+    for (int d : done) hit = hit || d == dev;
+    if (!hit) {
+      KH_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
+      done.push_back(dev);
+    }
+  }
+  a.tiles_t = (a.T + C::BM - 1) / C::BM;
+  a.tiles_f = (a.N + C::BN - 1) / C::BN;
+  hipLaunchKernelGGL(kern, dim3((a.tiles_f + 7) / 8 * 8 * a.tiles_t, kz), dim3(64 * C::NW), C::LDS, s, a);
+  return KH_OK;
+}
+// *kz_out: K slices whose partial rows the next RMSNorm has to add (0: the epilogue added itself)
+template <int EPI>
+int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out) {
+  PairShape sh = pair_shape(m->cfg.is_quant, a.T, a.N, a.K, EPI == KH_PG_RESID);
+  if (const char* e = dbg("KH_PAIR_SHAPE")) {  // test hook "tile,kz"
+    int t = 0, kz = 1;
+    if (sscanf(e, "%d,%d", &t, &kz) == 2 && t >= 0 && t < 4 && (kz == 1 || kz == 2 || kz == 4))
+      sh = PairShape{t, EPI == KH_PG_RESID ? kz : 1};
+  }
+  if (kz_out) *kz_out = sh.kz > 1 ? sh.kz : 0;
+  if (m->cfg.is_quant) {
+    switch (sh.tile) {
+      case 0: return pair_go<true, EPI, 7, 2, 1, 4, 2>(m->stream, a, sh.kz);
+      case 1: return pair_go<true, EPI, 4, 2, 1, 4, 3>(m->stream, a, sh.kz);
+      case 2: return pair_go<true, EPI, 2, 2, 1, 4, 4>(m->stream, a, sh.kz);
+      default: return pair_go<true, EPI, 4, 4, 2, 4, 3>(m->stream, a, sh.kz);
+    }
+  }
+  switch (sh.tile) {
+    case 0: return pair_go<false, EPI, 8, 2, 1, 4, 2>(m->stream, a, sh.kz);
+    case 1: return pair_go<false, EPI, 4, 2, 1, 4, 3>(m->stream, a, sh.kz);
+    case 2: return pair_go<false, EPI, 2, 2, 1, 4, 4>(m->stream, a, sh.kz);
+    default: return pair_go<false, EPI, 1, 2, 2, 2, 6>(m->stream, a, sh.kz);
+  }
+}
+}  // namespace
+
+namespace khm {
+// pair slabs advance in 32-column blocks, int8 groups in 64; other widths stay with k_pg_gemm
+bool pair_geometry(const kh_config& c) {
+  const int g = c.is_quant ? 64 : 32;
+  return c.dim % g == 0 && c.hidden_dim % g == 0;
+}
+
+int ensure_pair(kh_model* m) {
+  if (m->pair_ready) return KH_OK;
+  const kh_config& c = m->cfg;
+  if (m->pair_ws) (void)hipFree(m->pair_ws);
+  m->pair_ws = nullptr;
+  const size_t rows = 3 * (size_t)c.dim + 2 * (size_t)c.kv_dim + 2 * (size_t)c.hidden_dim;  // wq wk wv wo w1 w3 w2
+  const size_t per = (c.is_quant ? 0 : rows) + 4;
+  int rc;
+  if ((rc = dalloc(&m->pair_ws, per * c.layer_num + KH_PAIR_TMAX + 3 * c.layer_num)) != KH_OK) return rc;
+  m->pair_ws_layer = per;
+  unsigned* norms = (unsigned*)(m->pair_ws + per * c.layer_num + KH_PAIR_TMAX);
+  KH_CHECK_HIP(hipMemsetAsync(norms, 0, 3 * sizeof(unsigned) * c.layer_num, m->stream));
+  for (int l = 0; l < c.layer_num; ++l) {
+    const LayerW& W = m->layers[l];
+    unsigned* nm = norms + 3 * l;
+    const KhPairMats mats = {{{W.wq, c.dim, c.dim, nullptr, nullptr},
+                              {W.wk, c.kv_dim, c.dim, nullptr, nullptr},
+                              {W.wv, c.kv_dim, c.dim, W.att_norm, nm + 2},
+                              {W.wo, c.dim, c.dim, nullptr, nullptr},
+                              {W.w1, c.hidden_dim, c.dim, W.ffn_norm, nm},
+                              {W.w3, c.hidden_dim, c.dim, W.ffn_norm, nm + 1},
+                              {W.w2, c.dim, c.hidden_dim, nullptr, nullptr}}};
+    if (c.is_quant) hipLaunchKernelGGL(k_pair_rows<true>, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, (float*)nullptr, (int)rows);
+    else hipLaunchKernelGGL(k_pair_rows<false>, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, m->pair_ws + per * l + 4, (int)rows);
+    hipLaunchKernelGGL(k_pair_scales, dim3(1), dim3(256), 0, m->stream, W.att_norm, W.ffn_norm, W.wv.bias, (const unsigned*)nm, c.dim,
+                       c.kv_dim, m->pair_ws + per * l);
+  }
+  if ((rc = kh_launch_status()) != KH_OK) return rc;
+  m->pair_ready = true;
+  return KH_OK;
+}
+
+// forward of T (<= pg_rows) prompt tokens at positions pos0..: fills their K/V cache rows
+int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0) {
+  const kh_config& c = m->cfg;
+  int rc;
+  if ((rc = kh_embedding_f32_host(toks, T, m->tok_emb, m->pg_x, c.dim, c.vocab_size, (void*)m->stream)) != KH_OK) return rc;
+  char *xn = (char*)m->pg_xn, *h = (char*)m->pg_h;  // pair slabs: four bytes a number, like the fp32 slabs
+  float* att_s = m->pair_ws + m->pair_ws_layer * c.layer_num;
+  int kz = 0;  // K slices of the last residual GEMM still to be added to pg_x
+  const bool rope_fuse = !dbg_off("KH_PG_ROPE_FUSE");
+  for (int l = 0; l < c.layer_num; ++l) {
+    const LayerW& W = m->layers[l];
+    const float* sc = m->pair_ws + m->pair_ws_layer * l;
+    const float* ws = sc + 4;  // row scales: wq, wk, wv, wo, w1, w3, w2
+    const float* ws_o = ws + c.dim + 2 * c.kv_dim;
+    const float* ws_1 = ws_o + c.dim;
+    auto rmsnorm = [&](const float* w, const float* scale) {
+      hipLaunchKernelGGL(k_pair_rmsnorm, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_x, w, xn, scale, c.dim, c.rms_eps, m->pg_rows,
+                         (const float*)m->pg_part, kz);
+      kz = 0;
+    };
+    KhPairArgs base{};
+    base.T = T;
+    base.pos0 = pos0;
+    base.tcap = m->pg_rows;
+    base.part = m->pg_part;
+    base.head_size = c.head_size;
+    base.sin_cache = m->sin_cache;
+    base.cos_cache = m->cos_cache;
+    rmsnorm(W.att_norm, sc);
+    {
+      KhPairArgs a = base;
+      a.w[0] = W.wq; a.w[1] = W.wk; a.w[2] = W.wv;
+      a.ws[0] = ws; a.ws[1] = ws + c.dim; a.ws[2] = ws + c.dim + c.kv_dim;
+      a.X = xn; a.xs = sc; a.out = m->pg_q;
+      a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
+      a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
+      a.rows0 = c.dim; a.rows1 = c.kv_dim; a.N = c.dim + 2 * c.kv_dim; a.ldo = c.dim; a.K = c.dim;
+      a.rope = !rope_fuse ? KH_PG_ROPE_OFF
+               : (c.rope_mode == KH_ROPE_HALF ? (c.head_size % 32 == 0 ? KH_PG_ROPE_TILES : KH_PG_ROPE_OFF) : KH_PG_ROPE_PAIRS);
+      if ((rc = pair_launch<KH_PG_QKV>(m, a, nullptr)) != KH_OK) return rc;
+      if (a.rope == KH_PG_ROPE_OFF)
+        hipLaunchKernelGGL(k_pg_rope, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_q, a.kc, m->sin_cache, m->cos_cache, c.dim, c.kv_dim,
+                           c.head_size, pos0, c.rope_mode);
+    }
+    // the prompt phase leaves K/V rows and nothing else: the last layer's attention, wo and feed-forward feed nothing
+    if (l == c.layer_num - 1) break;
+    // the attention kernel leaves pairs where the static bound of the value rows holds
+    const bool pairs = pg_slice_attention(m, l, T, pos0, 0, m->kv_foreign ? nullptr : sc + 3);
+    if (!pairs) hipLaunchKernelGGL(k_pair_convert, dim3(T), dim3(KH_WG), 0, m->stream, (const float*)m->pg_att, xn, att_s, c.dim);
+    {
+      KhPairArgs a = base;
+      a.w[0] = W.wo; a.ws[0] = ws_o;
+      a.X = pairs ? (const char*)m->pg_att : xn; a.xs = pairs ? sc + 3 : att_s; a.xs_tok = !pairs; a.out = m->pg_x;
+      a.rows0 = a.N = a.ldo = a.K = c.dim;
+      if ((rc = pair_launch<KH_PG_RESID>(m, a, &kz)) != KH_OK) return rc;
+    }
+    rmsnorm(W.ffn_norm, sc + 1);
+    {
+      KhPairArgs a = base;
+      a.w[0] = W.w1; a.w[1] = W.w3;
+      a.ws[0] = ws_1; a.ws[1] = ws_1 + c.hidden_dim;
+      a.X = xn; a.xs = sc + 1; a.pairs = h; a.out_s = sc + 2;
+      a.rows0 = c.hidden_dim; a.N = 2 * c.hidden_dim; a.ldo = c.hidden_dim; a.K = c.dim;
+      if ((rc = pair_launch<KH_PG_SWIGLU>(m, a, nullptr)) != KH_OK) return rc;
+    }
+    {
+      KhPairArgs a = base;
+      a.w[0] = W.w2; a.ws[0] = ws_1 + 2 * c.hidden_dim;
+      a.X = h; a.xs = sc + 2; a.out = m->pg_x;
+      a.rows0 = a.N = a.ldo = c.dim; a.K = c.hidden_dim;
+      if ((rc = pair_launch<KH_PG_RESID>(m, a, &kz)) != KH_OK) return rc;
+    }
+  }
+  return kh_launch_status();
+}
+}  // namespace khm

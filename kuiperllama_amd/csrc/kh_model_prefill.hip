@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "kh_gemm.h"
@@ -227,8 +228,13 @@ void launch_prefill_chunk(kh_model* m, const int32_t* toks, int nvalid, int pos0
 
 // ---- GEMM prefill (kh_gemm.h) ------------------------------------------------------------------
 namespace {
-int ensure_pg_buffers(kh_model* m) {
-  if (m->pg_ready) return KH_OK;
+// slabs for a prompt of n tokens: at least KH_PG_TMAX rows, more for the longer passes of the pair GEMMs
+int ensure_pg_buffers(kh_model* m, int n) {
+  int rows = KH_PG_TMAX;
+  if (pair_geometry(m->cfg)) rows = std::max(rows, std::min((n + 127) / 128 * 128, KH_PAIR_TMAX));
+  if (m->pg_ready && m->pg_rows >= rows) return KH_OK;
+  if (m->pg_ready) KH_CHECK_HIP(hipStreamSynchronize(m->stream));  // passes on the smaller slabs
+  m->pg_ready = false;
   // a previous attempt may have failed half-way (out of memory): start from a clean slate so a
   // later call never launches GEMMs on null slabs
   for (float** p : {&m->pg_x, &m->pg_xn, &m->pg_q, &m->pg_att, &m->pg_h, &m->pg_part}) {
@@ -238,7 +244,7 @@ int ensure_pg_buffers(kh_model* m) {
   if (m->pg_ws) (void)hipFree(m->pg_ws);
   m->pg_ws = nullptr;
   const kh_config& c = m->cfg;
-  const size_t T = KH_PG_TMAX;
+  const size_t T = (size_t)rows;
   int rc;
   auto zalloc = [&](float** p, size_t n) -> int {
     if ((rc = dalloc(p, n)) != KH_OK) return rc;
@@ -252,6 +258,7 @@ int ensure_pg_buffers(kh_model* m) {
   if ((rc = zalloc(&m->pg_att, T * c.dim)) != KH_OK) return rc;
   if ((rc = zalloc(&m->pg_h, T * c.hidden_dim)) != KH_OK) return rc;
   if ((rc = zalloc(&m->pg_part, (size_t)KH_PG_KZ_MAX * T * c.dim)) != KH_OK) return rc;  // K-slice partial rows
+  m->pg_rows = rows;
   m->pg_ready = true;
   return KH_OK;
 }
@@ -421,6 +428,43 @@ int pg_launch(kh_model* m, int rows_total, bool r2_ok, KhPgGemmArgs a) {
   if (EPI == KH_PG_RESID) return sh.kz > 1 ? sh.kz : 0;
   return EPI == KH_PG_QKV && a.rope != KH_PG_ROPE_OFF;
 }
+}  // namespace
+namespace khm {
+// Attention of T prompt tokens whose K/V rows have just been written: pg_q -> pg_att, as the tiled slab of k_pg_gemm
+// (tcap > 0), as pairs of the scale at pair_scale (returns true) or as rows [T][dim] (the decode kernel always).
+// MFMA kernel (kh_pattn.h) unless KH_PG_ATTN=0 or an odd head size.
+bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int tcap, const float* pair_scale) {
+  const kh_config& c = m->cfg;
+  if (pg_mfma_attn(m)) {
+    KhPgAttnArgs a{};
+    a.q = m->pg_q;
+    a.kc = m->kcache + (size_t)layer * c.cache_len * c.kv_dim;
+    a.vc = m->vcache + (size_t)layer * c.cache_len * c.kv_dim;
+    a.out = m->pg_att;
+    a.dim = c.dim; a.kv_dim = c.kv_dim; a.kv_heads = c.kv_head_num; a.kv_mul = c.kv_mul;
+    a.T = T; a.pos0 = pos0; a.tcap = tcap;
+    a.layout = tcap > 0 ? (c.is_quant ? KH_PA_TILED_Q8 : KH_PA_TILED_F32) : (pair_scale ? KH_PA_PAIRS : KH_PA_ROWS);
+    a.out_s = pair_scale;
+    launch_pg_attn(a, c.head_size, m->stream);
+    return a.layout == KH_PA_PAIRS;
+  }
+  KhAttnArgs a = fill_attn(m, layer);
+  a.defer = 0;  // multi-token slices merge in the launch
+  a.nsplit_g = m->attn_ns_g;  // not the decode step's variant: launch_attn_decode decides from the slice's positions
+  a.q = m->pg_q;
+  a.out = m->pg_att;
+  a.d_pos = nullptr;
+  a.ws = m->pg_ws;
+  a.tok_stride = c.dim;
+  a.ws_tok_bytes = m->pg_ws_tok_bytes;
+  // head sizes without an MFMA instantiation (and KH_PG_ATTN=0): the decode kernel, one grid
+  // slice per token, 256-thread workgroups (4096 latency-bound (head, token) workgroups: twice
+  // as many fit a CU as with the decode width, 28.7 -> 19.6 us per layer)
+  launch_attn_decode(a, pos0, KH_WG, m->stream, T, pos0 + T - 1);
+  return false;
+}
+}  // namespace khm
+namespace {
 // forward of T (<= KH_PG_TMAX) prompt tokens at positions pos0..: fills their K/V cache rows
 void launch_prefill_gemm_chunk(kh_model* m, const int32_t* toks, int T, int pos0) {
   const kh_config& c = m->cfg;
@@ -462,27 +506,7 @@ void launch_prefill_gemm_chunk(kh_model* m, const int32_t* toks, int T, int pos0
     // the prompt phase leaves K/V rows and nothing else (no logits): the last layer's K/V rows are
     // written, its attention, wo and FFN feed nothing (1/L of the pass minus one QKV GEMM)
     if (l == c.layer_num - 1) break;
-    if (mfma_attn) {
-      KhPgAttnArgs a{};
-      a.q = m->pg_q; a.kc = kc; a.vc = vc; a.out = m->pg_att;
-      a.dim = c.dim; a.kv_dim = c.kv_dim; a.kv_heads = c.kv_head_num; a.kv_mul = c.kv_mul;
-      a.T = T; a.pos0 = pos0; a.layout = q ? KH_PA_TILED_Q8 : KH_PA_TILED_F32; a.tcap = tcap;
-      launch_pg_attn(a, c.head_size, m->stream);
-    } else {
-      KhAttnArgs a = fill_attn(m, l);
-      a.defer = 0;  // multi-token slices merge in the launch
-      a.nsplit_g = m->attn_ns_g;  // not the decode step's variant: launch_attn_decode decides from the slice's positions
-      a.q = m->pg_q;
-      a.out = m->pg_att;
-      a.d_pos = nullptr;
-      a.ws = m->pg_ws;
-      a.tok_stride = c.dim;
-      a.ws_tok_bytes = m->pg_ws_tok_bytes;
-      // head sizes without an MFMA instantiation (and KH_PG_ATTN=0): the decode kernel, one grid
-      // slice per token, 256-thread workgroups (4096 latency-bound (head, token) workgroups: twice
-      // as many fit a CU as with the decode width, 28.7 -> 19.6 us per layer)
-      launch_attn_decode(a, pos0, KH_WG, m->stream, T, pos0 + T - 1);
-    }
+    pg_slice_attention(m, l, T, pos0, tcap, nullptr);
     {
       KhPgGemmArgs a{};
       a.w[0] = W.wo;
@@ -539,14 +563,22 @@ extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32
     const HyEntry e{0, n, pos0, h_tokens};
     return kh_api_guard([&] { return hy_forward(m, &e, 1, nullptr, 0, nullptr); });
   }
-  if ((rc = ensure_pg_buffers(m)) != KH_OK) return rc;
+  if ((rc = ensure_pg_buffers(m, n)) != KH_OK) return rc;
   if ((rc = ensure_pg_ws(m)) != KH_OK) return rc;
   m->pg_launch_failed = false;
+  // KH_PG_PAIR=0 and the shape hooks of k_pg_gemm select the fp32-MFMA GEMMs
+  const bool pair = pair_geometry(c) && !dbg_off("KH_PG_PAIR") && !dbg("KH_PG_SHAPE_QKV") && !dbg("KH_PG_SHAPE_RESID") && !dbg("KH_PG_SHAPE_SWIGLU");
+  if (pair && (rc = ensure_pair(m)) != KH_OK) return rc;
   // tuning / test hook: KH_PG_CHUNK=<tokens per weight pass> (16 .. KH_PG_TMAX), read per call
-  int chunk = KH_PG_TMAX;
+  int chunk = pair && pg_mfma_attn(m) ? m->pg_rows : KH_PG_TMAX;
   if (const char* e = dbg("KH_PG_CHUNK")) {
     const int v = atoi(e);
     chunk = v < 16 ? 16 : (v > KH_PG_TMAX ? KH_PG_TMAX : v);
+  }
+  if (pair) {
+    for (int t0 = 0; t0 < n; t0 += chunk)
+      if ((rc = launch_prefill_pair_chunk(m, h_tokens + t0, n - t0 < chunk ? n - t0 : chunk, pos0 + t0)) != KH_OK) return rc;
+    return kh_launch_status();
   }
   for (int t0 = 0; t0 < n; t0 += chunk)
     launch_prefill_gemm_chunk(m, h_tokens + t0, n - t0 < chunk ? n - t0 : chunk, pos0 + t0);
@@ -644,7 +676,7 @@ extern "C" int kh_model_time_prefill(kh_model* m, const int32_t* h_tokens, int32
   } else if (mode == KH_PREFILL_GEMM) {
     if (!pg_supported(m)) return KH_ERR_UNSUPPORTED;
     if (!m->hy) {
-      if ((rc = ensure_pg_buffers(m)) != KH_OK) return rc;
+      if ((rc = ensure_pg_buffers(m, n)) != KH_OK) return rc;
       if ((rc = ensure_pg_ws(m)) != KH_OK) return rc;
     }
     KH_CHECK_HIP(hipEventRecord(m->ev0, m->stream));

@@ -1,0 +1,605 @@
+// kh_pair.h — prompt GEMMs on the fp16 matrix cores with both operands kept to 32-bit accuracy (.bin models; the
+// reference multiplies the prompt one token at a time: cpu/matmul_kernel.cpp:5-41, cuda/matmul_kernel.cu:56-87).
+//
+//   C[rows, T] = W[rows, K] . X[T, K]^T      every number v of X and of fp32 weights travels as a PAIR of halves
+//       hi = fp16(s v),  lo = fp16(s v - hi)          s a power of two
+// hi + lo is s v to at most one unit in the last place of fp32 (11 + 11 bits and the sign of lo) as long as |s v| lies
+// between 2^-8 and 2^15, and to 2^-25 absolutely below that; a product takes three matrix instructions (hi hi, hi lo,
+// lo hi; lo lo is 2^-22 of it at most) of v_mfma_f32_16x16x32_f16 into fp32 accumulators.  int8 weights are exact in
+// fp16 and take two; their group scale is applied in fp32 to the sum of each 64-column group.
+// Against v_mfma_f32_16x16x4_f32 the unit is 16 times as fast, so 5.3 (8) times the work per cycle is left, and a sum is
+// rounded once per 32 columns and product instead of once per 4 columns.
+//
+// Scales.  An activation row leaves RMSNorm with a Euclidean norm of at most sqrt(dim), so static bounds hold for every
+// input: |xn| <= sqrt(dim) max|g| and, for the gated unit, |h| <= max_j |w1_j * g| max_j |w3_j * g| dim (Cauchy-Schwarz;
+// typically 2^8 above the largest h, the pair spans 2^40 below its bound).  Attention outputs are averages of value rows,
+// |v| <= max_j |wv_j * g| sqrt(dim) + max|bias|.  k_pair_rows and k_pair_scales compute these and a scale for every weight
+// row once per model.  Once a caller has had its hands on the cache (kh_model_write_kv, kh_model_get_kv) the scale of an
+// attention output is its row maximum instead, found by a pass over the rows (k_pair_convert).
+//
+// Kernel: the stage ring of kh_lgemm.h.  A workgroup owns BM tokens x BN weight rows; a stage of 32 (int8: 64) columns
+// is moved to LDS by global_load_lds_dwordx4 in 128-byte rows (pairs: 32 hi | 32 lo; fp32 weights as they lie in the
+// file; int8 64-byte rows), swizzled so that the 16 rows of a fragment touch all banks.  fp32 weights are split in
+// registers behind the LDS read: two v_fma_mix per number.  Weights are the first MFMA operand, so a lane ends with four
+// consecutive rows of one token.
+#pragma once
+#include <type_traits>
+
+#include "kh_gemm.h"
+#include "kh_q8ring.h"
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// Chunk c (16 bytes) of a 128-byte LDS row r lies in slot c ^ pair_swz(r).  ds_read_b128 serves 16 lanes at a time - 0-3,
+// 12-15, 20-27 and 4-11, 16-19, 28-31 of each half wave (found by fitting SQ_LDS_BANK_CONFLICT of four layouts) - and
+// 64 banks hold two rows: with this table every fragment read of the kernel (16 rows; chunk h, 2 h or 2 (h & 1) by lane
+// group h) is free of conflicts, with r & 7 a third of the LDS cycles were.
+__device__ __forceinline__ int pair_swz(int r) { return ((r & 2) << 1) | ((r & 4) ? 3 : 0); }
+#define KH_PAIR_TOP 14  // a bound is scaled to at most 2^14: a factor of four below the largest fp16
+
+struct KhPairArgs {
+  KhLin w[3];          // QKV: wq, wk, wv; RESID: w[0]; SWIGLU: w1, w3
+  const float* ws[3];  // fp32 weights: the scale of every row
+  const char* X;       // pair slab: [T][K / 32][32 hi | 32 lo]
+  const float* xs;     // its scale: one value, or one per token
+  int xs_tok;
+  float* out;          // QKV: Q [T][ldo]; RESID: X [T][ldo] (+=)
+  char* pairs;         // SWIGLU: pair slab of the gated unit, [T][ldo / 32]
+  const float* out_s;  // SWIGLU: its scale
+  float* kc;           // QKV: K / V cache rows of this layer, row (pos0 + t) * rows1
+  float* vc;
+  float* part;         // RESID with gridDim.y > 1: partial rows [z][tcap][ldo], added by the k_pair_rmsnorm that follows
+  int rows0, rows1;    // QKV: rows of wq, of wk = wv; else rows0 = rows of one matrix
+  int N;               // rows of all matrices together
+  int ldo, K, T, pos0, tcap, tiles_t, tiles_f;
+  int rope, head_size; // QKV: KH_PG_ROPE_* in the epilogue
+  const float* sin_cache;
+  const float* cos_cache;
+};
+
+__device__ __forceinline__ f32x4 mfma_pair(const f16x8& a, const f16x8& b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+// two floats to two halves, round to nearest even (v_cvt_pk_f16_f32)
+__device__ __forceinline__ f16x2 pair_cvt(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_convertvector((f32x2{a, b}), f16x2);
+}
+// byte offset of the hi half of column k of a row of pairs; the lo half lies 64 bytes further
+__host__ __device__ __forceinline__ size_t pair_at(int k) { return (size_t)(k >> 5) * 128 + (k & 31) * 2; }
+__device__ __forceinline__ void pair_store4(char* row, int k, const f32x4& v, float s) {
+  f16x4 hi, lo;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    hi[i] = (_Float16)(v[i] * s);
+    lo[i] = (_Float16)__builtin_fmaf(v[i], s, -(float)hi[i]);
+  }
+  *(f16x4*)(row + pair_at(k)) = hi;
+  *(f16x4*)(row + pair_at(k) + 64) = lo;
+}
+// power of two that brings `bound` to at most 2^KH_PAIR_TOP (1 for 0, the smallest one for infinities and NaN)
+__device__ __forceinline__ float pair_scale(float bound) {
+  if (bound == 0.f) return 1.0f;
+  int e = (int)((__float_as_uint(bound) >> 23) & 255) - 126;  // |bound| < 2^e
+  int k = KH_PAIR_TOP - e;
+  k = k < -100 ? -100 : (k > 100 ? 100 : k);
+  return __uint_as_float((unsigned)(k + 127) << 23);
+}
+__device__ __forceinline__ float pair_inv(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }  // 1 / s
+// eight int8, times sgn = +-1 -> fp16, exact: 0x6400 + u is 1024 + u, u = q + 128
+__device__ __forceinline__ f16x8 pair_q8(unsigned a, unsigned b, float sgn) {
+  const f16x2 one = {(_Float16)sgn, (_Float16)sgn}, bias = {(_Float16)(-1152.0f * sgn), (_Float16)(-1152.0f * sgn)};
+  union { f16x8 v; f16x2 p[4]; } r;
+  const unsigned src[2] = {a ^ 0x80808080u, b ^ 0x80808080u};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    union { unsigned u; f16x2 h; } lo, hi;
+    lo.u = __builtin_amdgcn_perm(0x64646464u, src[i], 0x04010400u);
+    hi.u = __builtin_amdgcn_perm(0x64646464u, src[i], 0x04030402u);
+    r.p[2 * i] = __builtin_elementwise_fma(lo.h, one, bias);
+    r.p[2 * i + 1] = __builtin_elementwise_fma(hi.h, one, bias);
+  }
+  return r.v;
+}
+
+template <bool Q, int TM, int TN, int WM, int WN, int NST>
+struct PairCfg {
+  static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN, NW = WM * WN;
+  static constexpr int XB = Q ? 2 : 1;                     // 128-byte blocks of a token per stage
+  static constexpr int XR = BM * XB / 8;                   // 1-KiB requests: activations
+  static constexpr int WR = Q ? BN / 16 : BN / 8;          // weights
+  static constexpr int SR = Q ? BN / 64 : 0;               // 256-byte requests: group scales
+  static constexpr int STAGE = (XR + WR) * 1024 + SR * 256;
+  static constexpr int NL = XR / NW + WR / NW + (Q ? 1 : 0);  // requests of a wave per stage
+  static constexpr int LDS = NST * STAGE;
+  static_assert(NW % 2 == 0 && XR % NW == 0 && WR % NW == 0, "every wave issues the same number of requests");
+};
+
+// blockIdx.x -> (row tile, token tile): the token tiles of a row tile run on one XCD (blocks go round the XCDs) one after
+// the other, so its weights cross HBM once.  blockIdx.y = K slice (RESID).
+template <bool Q, int EPI, int TM, int TN, int WM, int WN, int NST>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs a) {
+  typedef PairCfg<Q, TM, TN, WM, WN, NST> C;
+  extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = (int)blockIdx.x & 7, bj = (int)blockIdx.x >> 3;
+  const int ft = bj / a.tiles_t * 8 + xcd, tt = bj % a.tiles_t;
+  if (ft >= a.tiles_f) return;  // uniform: the grid is rounded up to eight row tiles
+  const int t0 = tt * C::BM, f0 = ft * C::BN;
+  const int K = a.K;
+  // place f of the stacked rows -> matrix, row.  Runs of 16 places are runs of 16 rows: SWIGLU takes 16 rows of w1, the
+  // same 16 of w3, ...; half-mode RoPE takes 16 rows of a head, then their 16 partners half a head further.
+  auto place = [&](int f, int& mat, int& row) __attribute__((always_inline)) {
+    mat = 0;
+    row = f;
+    if (EPI == KH_PG_SWIGLU) {
+      mat = (f >> 4) & 1;
+      row = (f >> 5) * 16 + (f & 15);
+    } else if (EPI == KH_PG_QKV) {
+      if (f >= a.rows0 + a.rows1) {
+        mat = 2;
+        row = f - a.rows0 - a.rows1;
+      } else if (f >= a.rows0) {
+        mat = 1;
+        row = f - a.rows0;
+      }
+      if (a.rope == KH_PG_ROPE_TILES) {
+        const int head = row / a.head_size, q = row - head * a.head_size;
+        row = head * a.head_size + (q >> 5) * 16 + (q & 15) + ((q & 16) ? a.head_size >> 1 : 0);
+      }
+    }
+  };
+  // ---- staging addresses
+  static_assert(TN % 2 == 0, "both tiles of a SWIGLU or half-mode RoPE pair lie in one wave");
+  constexpr int NX = C::XR / C::NW, NWR = C::WR / C::NW;
+  unsigned xoff[NX], woff[NWR];
+  const char* wbase[NWR];
+  const char* sbase = nullptr;
+  const int sub = lane >> 3, ch8 = (lane & 7) ^ pair_swz(sub);
+  const int z0 = (int)((long)blockIdx.y * (K >> (Q ? 6 : 5)) / gridDim.y);
+  const int z1 = (int)((long)(blockIdx.y + 1) * (K >> (Q ? 6 : 5)) / gridDim.y);
+#pragma unroll
+  for (int j = 0; j < NX; ++j) {
+    const int r = 8 * (j * C::NW + wave) + sub;  // LDS row: block-major for int8
+    int t = t0 + (Q ? r % C::BM : r);
+    t = t < a.T ? t : a.T - 1;
+    xoff[j] = (unsigned)t * (unsigned)(4 * K) + (Q ? (unsigned)(r / C::BM) * 128u : 0u) + 16u * ch8 + (unsigned)z0 * (128u * C::XB);
+  }
+#pragma unroll
+  for (int j = 0; j < NWR; ++j) {
+    const int run = Q ? 16 : 8;
+    int f = f0 + run * (j * C::NW + wave);
+    f = f < a.N - run ? f : a.N - run;
+    int mat, row;
+    place(f, mat, row);
+    wbase[j] = (const char*)a.w[mat].w;
+    if (Q) {
+      const int rr = lane >> 2, ch = (lane & 3) ^ ((rr & 4) >> 1);
+      woff[j] = (unsigned)(row + rr) * (unsigned)K + 16u * ch + (unsigned)z0 * 64u;
+    } else {
+      woff[j] = (unsigned)(row + sub) * (unsigned)(4 * K) + 16u * ch8 + (unsigned)z0 * 128u;
+    }
+  }
+  if (Q) {  // scales of 64 places: one dword a lane (SWIGLU and RoPE runs of 16 may lie in two matrices: 64-bit addresses)
+    int f = f0 + 64 * (wave % (C::SR ? C::SR : 1)) + lane;
+    f = f < a.N ? f : a.N - 1;
+    int mat, row;
+    place(f, mat, row);
+    sbase = (const char*)(mat == 0 ? a.w[0].scales : (mat == 1 ? a.w[1].scales : a.w[2].scales)) +
+            ((size_t)row * (K >> 6) + z0) * 4;
+  }
+  const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane((int)kh_lds_addr(smem_raw)) + 1024u * wave;
+  auto issue = [&](int slot) __attribute__((always_inline)) {
+    const unsigned d = lds0 + (unsigned)(slot * C::STAGE);
+#pragma unroll
+    for (int j = 0; j < NWR; ++j) {
+      dma_x4_keep(wbase[j], woff[j], d + (unsigned)(C::XR * 1024 + j * C::NW * 1024));
+      woff[j] += Q ? 64 : 128;
+    }
+#pragma unroll
+    for (int j = 0; j < NX; ++j) {
+      dma_x4_keep(a.X, xoff[j], d + (unsigned)(j * C::NW * 1024));
+      xoff[j] += 128 * C::XB;
+    }
+    if (Q) {
+      const unsigned sd = lds0 - 1024u * wave + (unsigned)(slot * C::STAGE + (C::XR + C::WR) * 1024) +
+                          256u * (unsigned)(wave % (C::SR ? C::SR : 1));
+      dma_x1_keep(sbase, sd);
+      sbase += 4;
+    }
+  };
+  const int nk = z1 - z0;
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int n = 0; n < TN; ++n)
+#pragma unroll
+    for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wm = wave % WM, wn = wave / WM;
+  const int fr = lane & 15, fh = lane >> 4;
+  float wsc[TN];
+#pragma unroll
+  for (int n = 0; n < TN; ++n) {
+    wsc[n] = 1.0f;
+    if (!Q) {
+      int f = f0 + (wn * TN + n) * 16;
+      f = f < a.N - 16 ? f : a.N - 16;
+      int mat, row;
+      place(f, mat, row);
+      wsc[n] = a.ws[mat][row + fr];
+    }
+  }
+  // wait for them here: a wait left to their first use would sit in the loop and drain the ring
+#pragma unroll
+  for (int n = 0; n < TN; ++n) asm volatile("" : "+v"(wsc[n]));
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nk) issue(s);
+  int slot = 0, fill = NST - 1;
+  f32x4 grp[Q ? 1 : TN][Q ? 1 : TM];  // fp32 weights: the sums of two stages
+  // The matrix unit rounds its sums down: a bias that the mean over many cached rows keeps while it averages everything else
+  // (logits behind 1900 prompt tokens: 1.7e-6 from 64 bits instead of 1.3e-6 on fp32 fma chains).  Every other group takes
+  // its weights with the sign turned and is subtracted, which cancels it: 1.1e-6.
+  float sgn = 1.0f;
+  auto stage = [&](int k, auto open) __attribute__((always_inline)) {
+    constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a group
+    // stage k has landed when at most the requests of the stages behind it are outstanding
+    if (NST > 2 && k + NST - 2 < nk) wait_vm<(NST - 2) * C::NL>();
+    else wait_vm<0>();
+    __syncthreads();
+    if (k + NST - 1 < nk) issue(fill);
+    const char* st = smem_raw + slot * C::STAGE;
+    const char* wst = st + C::XR * 1024;
+    if constexpr (!Q) {
+      f16x8 xh[TM], xl[TM];
+      f32x4 wv[TN][2];
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const int r = (wn * TN + n) * 16 + fr;
+        wv[n][0] = *(const f32x4*)(wst + r * 128 + (((2 * fh) ^ pair_swz(r)) << 4));
+        wv[n][1] = *(const f32x4*)(wst + r * 128 + (((2 * fh + 1) ^ pair_swz(r)) << 4));
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        const int r = (wm * TM + m) * 16 + fr;
+        xh[m] = *(const f16x8*)(st + r * 128 + ((fh ^ pair_swz(r)) << 4));
+        xl[m] = *(const f16x8*)(st + r * 128 + (((4 + fh) ^ pair_swz(r)) << 4));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        f16x8 wh, wl;
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const float v0 = wv[n][e >> 2][e & 3], v1 = wv[n][e >> 2][(e & 3) + 1];
+          const f16x2 hi = pair_cvt(v0 * wsc[n], v1 * wsc[n]);
+          const f16x2 lo = pair_cvt(__builtin_fmaf(v0, wsc[n], -(float)hi.x), __builtin_fmaf(v1, wsc[n], -(float)hi.y));
+          wh[e] = hi.x; wh[e + 1] = hi.y;
+          wl[e] = lo.x; wl[e + 1] = lo.y;
+        }
+#pragma unroll
+        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wl, xh[m], OPEN ? f32x4{0.f, 0.f, 0.f, 0.f} : grp[n][m]);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wh, xl[m], grp[n][m]);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wh, xh[m], grp[n][m]);
+      }
+    } else {
+      // lane (i, h) takes columns 16 h .. + 15 of its 64-column group; either product takes eight of them
+      f16x8 xh[TM][2], xl[TM][2];
+      i32x4 qv[TN];
+      f32x4 sc[TN];
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const int r = (wn * TN + n) * 16 + fr;
+        qv[n] = *(const i32x4*)(wst + r * 64 + ((fh ^ ((r & 4) >> 1)) << 4));
+        sc[n] = *(const f32x4*)(wst + C::WR * 1024 + ((wn * TN + n) * 16 + 4 * fh) * 4);
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        const int r = (wm * TM + m) * 16 + fr;
+        const char* row = st + ((fh >> 1) * C::BM + r) * 128;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const int c = 2 * (fh & 1) + b;
+          xh[m][b] = *(const f16x8*)(row + ((c ^ pair_swz(r)) << 4));
+          xl[m][b] = *(const f16x8*)(row + (((4 + c) ^ pair_swz(r)) << 4));
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const f16x8 w0 = pair_q8((unsigned)qv[n].x, (unsigned)qv[n].y, sgn), w1 = pair_q8((unsigned)qv[n].z, (unsigned)qv[n].w, sgn);
+        const f32x4 sg = {sc[n].x * sgn, sc[n].y * sgn, sc[n].z * sgn, sc[n].w * sgn};
+        f32x4 g[TM];
+#pragma unroll
+        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w0, xl[m][0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w1, xl[m][1], g[m]);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w0, xh[m][0], g[m]);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w1, xh[m][1], g[m]);
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(sg[i], g[m][i], acc[n][m][i]);
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    slot = slot + 1 == NST ? 0 : slot + 1;
+    fill = fill + 1 == NST ? 0 : fill + 1;
+  };
+  auto close = [&]() __attribute__((always_inline)) {
+    if constexpr (!Q) {
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(sgn, grp[n][m][i], acc[n][m][i]);
+        wsc[n] = -wsc[n];
+      }
+    }
+    sgn = -sgn;
+  };
+  const std::true_type first{};
+  const std::false_type second{};
+  if constexpr (Q) {
+    for (int k = 0; k < nk; ++k) {
+      stage(k, first);
+      close();
+    }
+  } else {
+    int k = 0;
+    for (; k + 1 < nk; k += 2) {
+      stage(k, first);
+      stage(k + 1, second);
+      close();
+    }
+    if (k < nk) {
+      stage(k, first);
+      close();
+    }
+  }
+  // ---- epilogue: lane (fr, fh) of tile (n, m) holds rows 4 fh .. + 3 of the tile for token t0 + .. + fr
+  float xs = a.xs_tok ? 1.0f : a.xs[0];
+  const float os = EPI == KH_PG_SWIGLU ? a.out_s[0] : 1.0f;
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int tok = t0 + (wm * TM + m) * 16 + fr;
+    if (tok >= a.T) continue;
+    if (a.xs_tok) xs = a.xs[tok];
+    const float ix = pair_inv(xs);
+    auto value = [&](int n, int mat, int row) __attribute__((always_inline)) {
+      f32x4 v = acc[n][m];
+      if (!Q) {
+        const f32x4 s = *(const f32x4*)(a.ws[mat] + row);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = v[i] * ix * pair_inv(s[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= ix;
+      }
+      return v;
+    };
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const int f = f0 + (wn * TN + n) * 16;
+      if (f >= a.N) continue;
+      int mat, row;
+      place(f, mat, row);
+      row += 4 * fh;
+      if (EPI == KH_PG_SWIGLU) {
+        if (n & 1) continue;
+        const f32x4 g = value(n, 0, row), u = value(n + 1, 1, row);
+        f32x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = swiglu1(g[i], u[i]);
+        pair_store4(a.pairs + (size_t)tok * a.ldo * 4, row, o, os);
+      } else if (EPI == KH_PG_RESID) {
+        const f32x4 v = value(n, 0, row);
+        if (gridDim.y > 1) {
+          *(f32x4*)(a.part + ((size_t)blockIdx.y * a.tcap + tok) * a.ldo + row) = v;
+        } else {  // residual add (llama3.cpp:686,719)
+          f32x4* dst = (f32x4*)(a.out + (size_t)tok * a.ldo + row);
+          f32x4 x = *dst;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] += v[i];
+          *dst = x;
+        }
+      } else {
+        auto biased = [&](f32x4 v, int r) __attribute__((always_inline)) {  // before RoPE (matmul.cpp:74-77)
+          if (a.w[mat].bias) {
+            const f32x4 b = *(const f32x4*)(a.w[mat].bias + r);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += b[i];
+          }
+          return v;
+        };
+        float* dst = mat == 0 ? a.out + (size_t)tok * a.ldo : (mat == 1 ? a.kc : a.vc) + (size_t)(a.pos0 + tok) * a.rows1;
+        const int hs = a.head_size;
+        const float* sn = a.sin_cache + (size_t)(a.pos0 + tok) * hs;
+        const float* cs = a.cos_cache + (size_t)(a.pos0 + tok) * hs;
+        if (a.rope == KH_PG_ROPE_TILES) {
+          if (n & 1) continue;
+          // tile n + 1 holds the partners, half a head further; cache column 2 j (cpu/rope_kernel.cpp:18-42)
+          const f32x4 lo = biased(value(n, mat, row), row), hi = biased(value(n + 1, mat, row + (hs >> 1)), row + (hs >> 1));
+          f32x4 olo = lo, ohi = hi;
+          if (mat < 2) {
+            const int j = row % hs;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float s = sn[2 * (j + i)], c = cs[2 * (j + i)];
+              olo[i] = lo[i] * c - hi[i] * s;
+              ohi[i] = lo[i] * s + hi[i] * c;
+            }
+          }
+          *(f32x4*)(dst + row) = olo;
+          *(f32x4*)(dst + row + (hs >> 1)) = ohi;
+        } else {
+          f32x4 v = biased(value(n, mat, row), row);
+          if (mat < 2 && a.rope == KH_PG_ROPE_PAIRS) {  // pairs (row, row + 1) (cpu/rope_kernel.cpp:98-121)
+            const int c = row % hs;
+            const float s0 = sn[c], c0 = cs[c], s1 = sn[c + 2], c1 = cs[c + 2];
+            v = f32x4{v.x * c0 - v.y * s0, v.x * s0 + v.y * c0, v.z * c1 - v.w * s1, v.z * s1 + v.w * c1};
+          }
+          *(f32x4*)(dst + row) = v;
+        }
+      }
+    }
+  }
+}
+
+// ---- scales, once per model ----------------------------------------------------------------------------------------
+struct KhPairMats {  // the matrices of a layer
+  struct {
+    KhLin w;
+    int rows, K;
+    const float* g;   // norm weights in front of it (w1, w3, wv)
+    unsigned* norm;
+  } m[7];
+};
+// One wave per row of the stacked matrices: fp32 weights get the row's scale; with norm weights g the largest |w_row * g| of
+// the matrix goes to *norm (its bits: the values are positive).  16 bytes a lane; K is a multiple of 32 (int8: 64).
+template <bool Q>
+__global__ __launch_bounds__(256) void k_pair_rows(const KhPairMats a, float* ws, int total) {
+  const int at = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (at >= total) return;
+  int row = at, i = 0;
+  while (i < 6 && row >= a.m[i].rows) row -= a.m[i++].rows;
+  const KhLin w = a.m[i].w;
+  const int K = a.m[i].K;
+  const float* g = a.m[i].g;
+  unsigned* norm = a.m[i].norm;
+  if (Q && !g) return;
+  float top = 0.f, sum = 0.f;
+  auto add4 = [&](f32x4 v, int k) __attribute__((always_inline)) {
+    top = fmaxf(fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+    if (g) {
+      const f32x4 y = *(const f32x4*)(g + k);
+      v = f32x4{v.x * y.x, v.y * y.y, v.z * y.z, v.w * y.w};
+      sum = fma4(v, v, sum);
+    }
+  };
+  if constexpr (Q) {
+    for (int k = 16 * lane; k < K; k += 1024) {
+      const i32x4 q = ld_nt((const i32x4*)((const int8_t*)w.w + (size_t)row * K + k));
+      const float s = w.scales[(size_t)row * (K >> 6) + (k >> 6)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        add4(f32x4{s * (float)(int8_t)q[i], s * (float)(int8_t)(q[i] >> 8), s * (float)(int8_t)(q[i] >> 16), s * (float)(q[i] >> 24)},
+             k + 4 * i);
+    }
+  } else {
+#pragma unroll 4
+    for (int k = 4 * lane; k < K; k += 256) add4(ld_nt((const f32x4*)((const float*)w.w + (size_t)row * K + k)), k);
+  }
+  for (int o = 32; o; o >>= 1) {
+    top = fmaxf(top, __shfl_xor(top, o));
+    sum += __shfl_xor(sum, o);
+  }
+  if (lane == 0) {
+    if (!Q) ws[at] = pair_scale(top);
+    if (norm) atomicMax(norm, __float_as_uint(sqrtf(sum)));
+  }
+}
+// out: scales of the rows behind the attention and the feed-forward norm, of the gated unit and of the attention output.
+// norms: of w1, w3, wv; bv: bias of the value rows or null
+static __global__ __launch_bounds__(256) void k_pair_scales(const float* g_att, const float* g_ffn, const float* bv,
+                                                            const unsigned* norms, int dim, int kv_dim, float* out) {
+  __shared__ float red[3][4];
+  float m[3] = {0.f, 0.f, 0.f};
+  for (int k = threadIdx.x; k < dim; k += 256) {
+    m[0] = fmaxf(m[0], fabsf(g_att[k]));
+    m[1] = fmaxf(m[1], fabsf(g_ffn[k]));
+  }
+  if (bv)
+    for (int k = threadIdx.x; k < kv_dim; k += 256) m[2] = fmaxf(m[2], fabsf(bv[k]));
+  for (int i = 0; i < 3; ++i) {
+    for (int o = 32; o; o >>= 1) m[i] = fmaxf(m[i], __shfl_xor(m[i], o));
+    if ((threadIdx.x & 63) == 0) red[i][threadIdx.x >> 6] = m[i];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 0; i < 3; ++i) m[i] = fmaxf(fmaxf(red[i][0], red[i][1]), fmaxf(red[i][2], red[i][3]));
+    const float x = sqrtf((float)dim);  // |x| / rms(x) at most
+    out[0] = pair_scale(m[0] * x);
+    out[1] = pair_scale(m[1] * x);
+    out[2] = pair_scale(__uint_as_float(norms[0]) * x * __uint_as_float(norms[1]) * x);
+    out[3] = pair_scale(__uint_as_float(norms[2]) * x + m[2]);
+  }
+}
+
+// ---- the per-token kernels between the GEMMs ------------------------------------------------------------------------
+// k_pg_rmsnorm (kh_gemm.h) with a row of pairs as its output; one workgroup per token
+static __global__ __launch_bounds__(KH_WG) void k_pair_rmsnorm(float* __restrict__ X, const float* __restrict__ w, char* __restrict__ out,
+                                                               const float* __restrict__ scale, int dim, float eps, int tcap,
+                                                               const float* __restrict__ part, int kz) {
+  __shared__ float red[KH_WAVES_MAX];
+  const int t = blockIdx.x;
+  f32x4* x4 = (f32x4*)(X + (size_t)t * dim);
+  const f32x4* w4 = (const f32x4*)w;
+  const int n4 = dim >> 2;
+  constexpr int KEEP = 4;  // the row stays in registers between the two passes for dim <= 4096
+  f32x4 keep[KEEP];
+  float ss = 0.f;
+  auto load = [&](int k) __attribute__((always_inline)) {
+    f32x4 v = x4[k];
+    if (kz > 0) {  // the residual GEMM in front split K: its partial rows, in fixed order
+      for (int z = 0; z < kz; ++z) {
+        const f32x4 p = *(const f32x4*)(part + ((size_t)z * tcap + t) * dim + 4 * k);
+        v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
+      }
+      x4[k] = v;
+    }
+    return v;
+  };
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int k = (int)threadIdx.x + i * KH_WG;
+    if (k < n4) {
+      keep[i] = load(k);
+      ss = fma4(keep[i], keep[i], ss);
+    }
+  }
+  for (int k = (int)threadIdx.x + KEEP * KH_WG; k < n4; k += KH_WG) {
+    const f32x4 v = load(k);  // (re-read by this same thread below)
+    ss = fma4(v, v, ss);
+  }
+  ss = block_sum(ss, red);
+  const float rs = 1.0f / sqrtf(ss / (float)dim + eps), s = *scale;
+  auto emit = [&](int k, const f32x4& v) __attribute__((always_inline)) {
+    const f32x4 g = w4[k];
+    pair_store4(out + (size_t)t * dim * 4, 4 * k, f32x4{g.x * (rs * v.x), g.y * (rs * v.y), g.z * (rs * v.z), g.w * (rs * v.w)}, s);
+  };
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int k = (int)threadIdx.x + i * KH_WG;
+    if (k < n4) emit(k, keep[i]);
+  }
+  for (int k = (int)threadIdx.x + KEEP * KH_WG; k < n4; k += KH_WG) emit(k, x4[k]);
+}
+// rows of pairs and their scales (from the row maximum) from rows of fp32; one workgroup per token
+static __global__ __launch_bounds__(KH_WG) void k_pair_convert(const float* __restrict__ A, char* __restrict__ out, float* __restrict__ xs,
+                                                               int dim) {
+  __shared__ float red[KH_WAVES_MAX];
+  const int t = blockIdx.x, n4 = dim >> 2;
+  const f32x4* a4 = (const f32x4*)(A + (size_t)t * dim);
+  float top = 0.f;
+  for (int k = threadIdx.x; k < n4; k += KH_WG) {
+    const f32x4 v = a4[k];
+    top = fmaxf(top, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+  }
+  for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = top;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < KH_WG / 64; ++i) top = fmaxf(top, red[i]);
+  const float s = pair_scale(top);
+  if (threadIdx.x == 0) xs[t] = s;
+  for (int k = threadIdx.x; k < n4; k += KH_WG) pair_store4(out + (size_t)t * dim * 4, 4 * k, a4[k], s);
+}

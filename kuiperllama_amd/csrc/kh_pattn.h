@@ -27,17 +27,18 @@
 //
 // Output goes straight into the tiled activation slab the wo GEMM reads (pg_tiled_index).
 #pragma once
-#include "kh_gemm.h"
+#include "kh_pair.h"
 
 struct KhPgAttnArgs {
   const float* q;   // [T][dim] row-major, RoPE applied
   const float* kc;  // this layer's K cache rows [cache_len][kv_dim]; rows pos0 .. pos0+T-1 just written
   const float* vc;
   float* out;       // layout 0 / 1: tiled slab [dim x tcap] of an fp32 / int8 model
-                    // (pg_tiled_index, T <= tcap); layout 2: row-major [T][dim]
+                    // (pg_tiled_index, T <= tcap); layout 2: row-major [T][dim]; layout 3: rows of pairs (kh_pair.h)
+  const float* out_s;  // layout 3: their scale
   int dim, kv_dim, kv_heads, kv_mul, T, pos0, layout, tcap;
 };
-enum { KH_PA_TILED_F32 = 0, KH_PA_TILED_Q8 = 1, KH_PA_ROWS = 2 };
+enum { KH_PA_TILED_F32 = 0, KH_PA_TILED_Q8 = 1, KH_PA_ROWS = 2, KH_PA_PAIRS = 3 };
 
 template <int HB /* head_size / 16 */, int NW /* waves that split the timesteps: 4 or 8 */,
           int QT /* 16-token query tiles per workgroup: every K/V fragment a wave loads feeds QT tiles */>
@@ -219,6 +220,10 @@ __global__ __launch_bounds__(64 * NW) void k_pg_attn(const KhPgAttnArgs a) {
         }
         r.x /= L; r.y /= L; r.z /= L; r.w /= L;
         const int k = h * HS + 4 * grp;
+        if (a.layout == KH_PA_PAIRS) {
+          pair_store4((char*)a.out + (size_t)t * a.dim * 4, k, r, *a.out_s);
+          continue;
+        }
         const size_t at = a.layout == KH_PA_ROWS ? (size_t)t * a.dim + k
                                                  : pg_tiled_index(a.layout == KH_PA_TILED_Q8, k, t, a.tcap);
         *(f32x4*)(a.out + at) = r;

@@ -50,6 +50,17 @@ __device__ __forceinline__ void dma_x4(const void* base, unsigned voff, unsigned
                : "v"(voff), "s"(base), "s"(dst)
                : "memory", "m0");
 }
+// the same with the default cache policy: operands that other workgroups read as well
+__device__ __forceinline__ void dma_x4_keep(const void* base, unsigned voff, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(voff), "s"(base), "s"(dst)
+               : "memory", "m0");
+}
+// 64 lanes x 4 B, every lane from an address of its own
+__device__ __forceinline__ void dma_x1_keep(const void* addr, unsigned dst) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(addr), "s"(dst) : "memory", "m0");
+}
 // 64 lanes x 4 B to LDS [dst + 4 * lane]
 __device__ __forceinline__ void dma_x1(const void* base, unsigned voff, unsigned dst) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
