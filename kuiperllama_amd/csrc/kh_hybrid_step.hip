@@ -39,19 +39,11 @@ enum { TB_TOK = 0, TB_POS = KH_HY_DECODE_B, TB_SLOT = 2 * KH_HY_DECODE_B, TB_ZER
 template <class T>
 size_t vec_b(int n) { return Ld<T>::vec_bytes(n); }
 template <class T>
-size_t lds_out(const Hybrid& hy, const HyLayer& l, int B) {
-  const int nbv = Ld<T>::blocks(l.out_mat().ld);
-  const int nf = l.ff.on ? l.ff.top * Ld<T>::blocks(l.ff.ffp) + (l.ff.sffp ? Ld<T>::blocks(l.ff.sffp) : 0) : 0;
-  (void)hy;
-  return ((size_t)B * nbv + nf) * Ld<T>::BE * 4;
-}
-template <class T>
 bool fits(const Hybrid& hy, int B) {
   const size_t room = kMaxLds - 2048;  // static shared memory of the kernels
   if (hy.c.widthp > 8192 || B * vec_b<T>(hy.c.widthp) > room) return false;
   if (hy.enter.N && B * vec_b<T>(hy.enter.ld) > room) return false;
   for (auto& l : hy.layers) {
-    if (lds_out<T>(hy, l, B) > room) return false;
     if (l.mixer == HY_MAMBA1 && B * vec_b<T>(l.mb.innerp) > room) return false;
     if (l.mixer == HY_LATENT && (B * vec_b<T>(l.la.qrp) > room)) return false;
   }
@@ -109,7 +101,7 @@ int with_rp(int n_out, F&& f) {
   return f(std::integral_constant<int, 16>());
 }
 
-// waves of a row pair over nblk blocks (k_ld_out, k_ld_enter): as many as keep each wave's share within its two tiles and
+// waves of a row pair over nblk blocks (k_ld_enter): as many as keep each wave's share within its two tiles and
 // give every CU a workgroup, while the launch has at most four per CU
 int split_waves(int rows, int nblk) {
   int ks = 1;
@@ -317,7 +309,6 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
       LdOutArgs a{};
       a.wo = wo.w;
       a.v = st.v;
-      a.n4v = wo.ld / 4;
       a.ld = Wp;
       a.ld_v = wo.ld;
       a.ldv = wo.ld;
@@ -340,8 +331,11 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
         a.ffp = f.ffp;
         a.sffp = f.sffp;
       }
-      a.ks = split_waves(W, Ld<T>::blocks(wo.ld) + (f.on ? f.top * Ld<T>::blocks(f.ffp) + (f.sff ? Ld<T>::blocks(f.sffp) : 0) : 0));
-      TRY(go(k_ld_out<T, B>, dim3(cdiv(cdiv(W, 2) * a.ks, 8)), 512, lds_out<T>(hy, l, B), s, a));
+      // two workgroups per CU at most: 16 waves a CU hide the latency, a second round would not (four sequences, us a step:
+      // width 1024: 535 with ks 4, 520 with 8; width 2048: 606 with 4, 616 with 8)
+      a.ks = 1;
+      while (a.ks < 8 && cdiv(cdiv(W, 2) * a.ks * 2, 8) <= 512) a.ks *= 2;
+      TRY(go(k_ld_out<T, B>, dim3(cdiv(cdiv(W, 2) * a.ks, 8)), 512, 0, s, a));
     }
     x_in = x_out;
   }

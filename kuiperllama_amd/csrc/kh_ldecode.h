@@ -844,39 +844,37 @@ __global__ __launch_bounds__(512) void k_ld_enter(const LdEnterArgs a) {
 // ---- k_ld_out ----------------------------------------------------------------------------------------------------
 struct LdOutArgs {
   const void* wo;         // [W][ldv]
-  const float* v;         // [B][ld_v] mixer vector (4 n4v readable)
+  const float* v;         // [B][ld_v] mixer vector
   const void *down, *sdown;  // experts [W][ffp] each; shared [W][sffp]
   const float *he, *hs;   // [B][top][ffp] (weighted), [B][sffp]
   const int32_t* ids;     // [B][top]
   const float *id_w, *sh_g, *xn2, *x_cur;  // id_w, sh_g: nullptr = none, 1
   const float* bias;      // of W_o, or nullptr
   float* x_out;           // [B][ld]
-  int W, ld, n4v, ld_v, ldv, top, ffp, sffp, moe, ks;
+  int W, ld, ld_v, ldv, top, ffp, sffp, moe, ks;
   float mult;             // of everything that is added to the residual
 };
-// Workgroup = 8 waves = 8 / ks groups of ks waves; a group owns R rows, its waves share the blocks of the concatenation
-// [mixer | shared | expert 0 | expert 1 ...] (blocks of identity experts are skipped).  Experts differ between
-// sequences, so for B > 1 the feed-forward part runs once per sequence.  A block's place follows from its number, so
-// the first two tiles of a wave are requested before the vectors are staged.
+// Workgroup = 8 waves = 8 / ks groups of ks waves; a group owns R rows, its waves share the blocks: first those that all
+// sequences share (mixer, shared expert: a weight block meets B vectors), then every sequence's experts.  The vectors come
+// from the caches as they are needed, lanes behind a row's end repeat its last chunk against zeros: no LDS but the final sum,
+// no barrier before it, and 16 waves a CU run freely.  Bound by latency: with the vectors staged in LDS, four sequences of
+// 2048 columns took 96 KB (8 waves a CU, two rounds of workgroups) and a load, a staging and two barriers per sequence:
+// 44.9 -> 26.3 us a layer at four (bf16, 105 ... 139 MB of weights), 8.0 -> 6.1 at one of 1024 (fp32).
 template <class T, int B>
-__global__ __launch_bounds__(512) void k_ld_out(const LdOutArgs a) {
+__global__ __launch_bounds__(512, 4) void k_ld_out(const LdOutArgs a) {
   constexpr int R = 2, U = 4;
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   typedef typename Tile<T>::frag frag;
-  constexpr int BE = Ld<T>::BE, E = Ld<T>::E;
+  constexpr int E = Ld<T>::E, P = Ld<T>::P;
   __shared__ float comb[8][R * B];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nbv = Ld<T>::blocks(a.ldv);
-  const int nbe = a.moe && a.top ? Ld<T>::blocks(a.ffp) : 1, nbs = a.moe && a.sffp ? Ld<T>::blocks(a.sffp) : 0;
-  const int nb = nbv + nbs + (a.moe ? a.top * nbe : 0);
-  float* xv = (float*)smem_raw;
-  float* xf = xv + (size_t)B * nbv * BE;
+  const int nbv = Ld<T>::blocks(a.ldv), nbs = a.moe && a.sffp ? Ld<T>::blocks(a.sffp) : 0, nbc = nbv + nbs;
+  const int nbe = Ld<T>::blocks(a.ffp), per_q = a.moe ? a.top * nbe : 0;
   const int kp = wave % a.ks, grp = (int)blockIdx.x * (8 / a.ks) + wave / a.ks;
   const int item = grp * R;
   int ri[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) ri[r] = item + r < a.W ? item + r : a.W - 1;
-  // residual operands of the rows this wave will finish
+  float acc[R][B] = {};
   float rx = 0.f, rn = 0.f, rw = 0.f, rb = 0.f;
   if (kp == 0 && lane < R * B) {
     const int q = lane / R, i = item + (lane & (R - 1));
@@ -889,83 +887,81 @@ __global__ __launch_bounds__(512) void k_ld_out(const LdOutArgs a) {
       }
     }
   }
-  frag w[2][R][U];
-  int nc[2][U];
-  auto fetch = [&](int set, int b0, int b1, int q) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int b = b0 + u;  // wave-uniform
-      nc[set][u] = 0;
-      if (b < b1) {
-        const T* p = (const T*)a.wo;
-        int stride = a.ldv, bb = b;
-        bool have = true;
-        if (b >= nbv + nbs) {
-          const int e = b - nbv - nbs, k = e / nbe, id = a.ids[q * a.top + k];
-          bb = e - k * nbe;
-          stride = a.ffp;
-          have = id >= 0;
-          p = (const T*)a.down + (size_t)(have ? id : 0) * a.W * a.ffp;
-        } else if (b >= nbv) {
-          bb = b - nbv;
-          stride = a.sffp;
-          p = (const T*)a.sdown;
-        }
-        const int left = stride / E - bb * 64, n = left < 64 ? left : 64;
-        nc[set][u] = have ? n : 0;
-        if (have) {
-          const int c = lane < n ? lane : n - 1;
-#pragma unroll
-          for (int r = 0; r < R; ++r) w[set][r][u] = ld_nt((const frag*)(p + (size_t)ri[r] * stride + (size_t)bb * BE) + c);
-        }
-      }
-    }
+  // chunk of the lane in block bb of a row of `n` elements
+  auto chunk = [&](int n, int bb, bool& in) __attribute__((always_inline)) {
+    const int left = n / E - bb * 64;
+    in = lane < left;
+    return bb * 64 + (in ? lane : left - 1);
   };
-  float acc[R][B] = {};
+  auto dot = [&](const frag& w, const f32x4 (&x)[P], float s) __attribute__((always_inline)) {
 #pragma unroll
-  for (int q = 0; q < B; ++q) {
-    const int b_lo = q == 0 ? 0 : nbv, per = (nb - b_lo + a.ks - 1) / a.ks;
-    const int b0 = b_lo + kp * per, b1 = b0 + per < nb ? b0 + per : nb;
-    fetch(0, b0, b1, q);
-    fetch(1, b0 + U, b1, q);
-    if (q == 0) {
-      for (int j = 0; j < B; ++j)
-        ld_stage<T, 512>((f32x4*)(xv + (size_t)j * nbv * BE), a.v + (size_t)j * a.ld_v, a.n4v, nbv * BE / 4, 1.f, threadIdx.x);
-    } else {
-      __syncthreads();  // the feed-forward vectors of the sequence before have been consumed
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s = __builtin_fmaf((float)w[4 * p + i], x[p][i], s);
+    return s;
+  };
+  // ---- blocks that all sequences share
+  {
+    const int per = (nbc + a.ks - 1) / a.ks, u0 = kp * per, u1 = u0 + per < nbc ? u0 + per : nbc;
+    for (int u = u0; u < u1; ++u) {
+      const bool sh = u >= nbv;
+      const int n = sh ? a.sffp : a.ldv, ldx = sh ? a.sffp : a.ld_v;
+      const T* base = (const T*)(sh ? a.sdown : a.wo);
+      const float* v = sh ? a.hs : a.v;
+      bool in;
+      const int c = chunk(n, sh ? u - nbv : u, in);
+      frag w[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) w[r] = ld_nt((const frag*)(base + (size_t)ri[r] * n) + c);
+      f32x4 x[B][P];
+#pragma unroll
+      for (int q = 0; q < B; ++q)
+#pragma unroll
+        for (int p = 0; p < P; ++p) x[q][p] = *(const f32x4*)(v + (size_t)q * ldx + (size_t)c * E + 4 * p);
+#pragma unroll
+      for (int q = 0; q < B; ++q) {
+        const float g = sh && a.sh_g ? a.sh_g[q] : 1.f;
+#pragma unroll
+        for (int p = 0; p < P; ++p) x[q][p] = in ? x[q][p] * g : f4_zero();
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r][q] = dot(w[r], x[q], acc[r][q]);
+      }
     }
-    if (a.moe) {
-      if (nbs) ld_stage<T, 512>((f32x4*)xf, a.hs + (size_t)q * a.sffp, a.sffp >> 2, nbs * BE / 4, a.sh_g ? a.sh_g[q] : 1.f,
-                                 threadIdx.x);
-      for (int k = 0; k < a.top; ++k)
-        ld_stage<T, 512>((f32x4*)(xf + (size_t)(nbs + k * nbe) * BE), a.he + (size_t)(q * a.top + k) * a.ffp, a.ffp >> 2,
-                         nbe * BE / 4, 1.f, threadIdx.x);
-    }
-    __syncthreads();
-    auto use = [&](int set, int b) __attribute__((always_inline)) {
+  }
+  // ---- expert blocks, sequence by sequence
+  if (per_q) {
+    const int per = (per_q + a.ks - 1) / a.ks, e0 = kp * per, e1 = e0 + per < per_q ? e0 + per : per_q;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (!nc[set][u]) continue;
-        if (b + u < nbv) {
+    for (int q = 0; q < B; ++q)
+      for (int e = e0; e < e1; e += U) {
+        frag w[R][U];
+        f32x4 x[U][P];
+        bool in[U];
 #pragma unroll
-          for (int j = 0; j < B; ++j) {
-            const f32x4* x = (const f32x4*)(xv + ((size_t)j * nbv + b + u) * BE) + lane;
+        for (int u = 0; u < U; ++u) {
+          in[u] = false;
+          if (e + u >= e1) continue;  // uniform
+          const int k = (e + u) / nbe, id = a.ids[q * a.top + k];
+          if (id < 0) continue;  // identity expert
+          const int c = chunk(a.ffp, e + u - k * nbe, in[u]);
+          const T* base = (const T*)a.down + (size_t)id * a.W * a.ffp;
 #pragma unroll
-            for (int r = 0; r < R; ++r) acc[r][j] = ld_dot<T>(w[set][r][u], x, acc[r][j]);
-          }
-        } else {
-          const f32x4* x = (const f32x4*)(xf + (size_t)(b + u - nbv) * BE) + lane;
+          for (int r = 0; r < R; ++r) w[r][u] = ld_nt((const frag*)(base + (size_t)ri[r] * a.ffp) + c);
+          const float* v = a.he + (size_t)(q * a.top + k) * a.ffp + (size_t)c * E;
 #pragma unroll
-          for (int r = 0; r < R; ++r) acc[r][q] = ld_dot<T>(w[set][r][u], x, acc[r][q]);
+          for (int p = 0; p < P; ++p) x[u][p] = *(const f32x4*)(v + 4 * p);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (e + u >= e1) continue;
+          const int k = (e + u) / nbe;
+          if (a.ids[q * a.top + k] < 0) continue;
+#pragma unroll
+          for (int p = 0; p < P; ++p) x[u][p] = in[u] ? x[u][p] : f4_zero();
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[r][q] = dot(w[r][u], x[u], acc[r][q]);
         }
       }
-    };
-    for (int b = b0; b < b1; b += 2 * U) {
-      use(0, b);
-      fetch(0, b + 2 * U, b1, q);
-      use(1, b + U);
-      fetch(1, b + 3 * U, b1, q);
-    }
   }
   ld_reduce<R, B>(acc);
   if (lane < R * B) comb[wave][lane] = ld_pick<R, B>(acc, lane & (R - 1), lane / R);

@@ -20,7 +20,8 @@
 // Kernel: the stage ring of kh_lgemm.h.  A workgroup owns BM tokens x BN weight rows; a stage of 32 (int8: 64) columns
 // is moved to LDS by global_load_lds_dwordx4 in 128-byte rows (pairs: 32 hi | 32 lo; fp32 weights as they lie in the
 // file; int8 64-byte rows), swizzled so that the 16 rows of a fragment touch all banks.  fp32 weights are split in
-// registers behind the LDS read: two v_fma_mix per number.  Weights are the first MFMA operand, so a lane ends with four
+// registers behind the LDS read: two numbers take two multiplications, two v_cvt_pk_f16_f32 and two v_fma_mix_f32
+// (v_fma_mixlo / mixhi would be fewer but run at half their rate: 462 -> 389 us for w1 + w3 of Llama-3.2-1B at 2048 tokens).  Weights are the first MFMA operand, so a lane ends with four
 // consecutive rows of one token.
 #pragma once
 #include <type_traits>
