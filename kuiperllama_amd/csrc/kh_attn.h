@@ -14,6 +14,8 @@
 // the output over its timesteps, then timestep-groups are folded with shuffles + one LDS
 // exchange across the 4 waves.
 #pragma once
+#include <type_traits>
+
 #include <stdlib.h>
 
 #include "kh_common.h"
@@ -46,6 +48,9 @@ static inline size_t attn_lds_bytes(int head_size, int wg = KH_WG) {
 // q_h: [hs] ; k_base/v_base: cache + layer offset + head column offset ; kv_stride = kv_dim.
 // out_h: [hs].  score_out (optional, global [>= pos+1]): receives the softmax probabilities like
 // the reference's score tensor.  smem: attn_lds_bytes(hs) bytes, 16-B aligned.
+// U timesteps per thread and batch; the next batch is requested before the current one is used, and the first values
+// before the softmax statistics.
+template <int U>
 __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
                                                  const float* __restrict__ k_base,
                                                  const float* __restrict__ v_base, int kv_stride,
@@ -75,27 +80,59 @@ __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
 
   for (int t0 = 0; t0 < nT; t0 += KH_ATTN_TC) {
     const int tc = min(KH_ATTN_TC, nT - t0);
-    // ---- scores: s[t] = (q . K[t]) * scale ---------------------------------------------
-    for (int tb = 0; tb < tc; tb += TPI * 4) {
-      f32x4 kv[4];
+    // row of timestep t0 + tb + u TPI + tg, clamped to the chunk; nothing is requested behind its end
+    auto load_as = [&](f32x4(&r)[U], const f32x4* base, int tb, auto f) __attribute__((always_inline)) {
+      constexpr bool full = decltype(f)::value;  // a whole batch: no guards between the requests
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = tb + u * TPI + tg;
-        const int tt = t < tc ? t : tc - 1;
-        kv[u] = active ? K4[(size_t)(t0 + tt) * stride4 + dl] : zero4;
+      for (int u = 0; u < U; ++u) {
+        r[u] = zero4;
+        if (!full && tb + u * TPI >= tc) continue;  // uniform
+        const int t = tb + u * TPI + tg, tt = t < tc ? t : tc - 1;
+        if (active) r[u] = base[(size_t)(t0 + tt) * stride4 + dl];
       }
+    };
+    const int step = TPI * U;
+    auto load = [&](f32x4(&r)[U], const f32x4* base, int tb) __attribute__((always_inline)) {
+      if (tb + step <= tc) load_as(r, base, tb, std::true_type{});
+      else load_as(r, base, tb, std::false_type{});
+    };
+    auto apply = [&](const f32x4(&r)[U], int tb, auto&& use) __attribute__((always_inline)) {
+      if (tb + step <= tc) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = tb + u * TPI + tg;
-        float d = fma4(q4, kv[u], 0.f);
-        for (int off = G >> 1; off > 0; off >>= 1) d += __shfl_xor(d, off, KH_WAVE);
-        if (dl == 0 && t < tc) {
-          const float s = d * scale;
-          sc[t] = s;
-          if (score_out) score_out[t0 + t] = s;  // raw score; normalised in the last pass
+        for (int u = 0; u < U; ++u) use(r[u], tb + u * TPI + tg);
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (tb + u * TPI >= tc) break;  // uniform
+          use(r[u], tb + u * TPI + tg);
         }
       }
-    }
+    };
+    // batches 0, step, ... through two register sets
+    auto stream = [&](const f32x4* base, f32x4(&r0)[U], auto&& use) __attribute__((always_inline)) {
+      f32x4 r1[U];
+      for (int tb = 0; tb < tc; tb += 2 * step) {
+        if (tb + step < tc) load(r1, base, tb + step);
+        apply(r0, tb, use);
+        if (tb + step < tc) {
+          if (tb + 2 * step < tc) load(r0, base, tb + 2 * step);
+          apply(r1, tb + step, use);
+        }
+      }
+    };
+    f32x4 kv[U], vv[U];
+    load(kv, K4, 0);
+    // ---- scores: s[t] = (q . K[t]) * scale ---------------------------------------------
+    stream(K4, kv, [&](const f32x4& k4, int t) __attribute__((always_inline)) {
+      float d = fma4(q4, k4, 0.f);
+      for (int off = G >> 1; off > 0; off >>= 1) d += __shfl_xor(d, off, KH_WAVE);
+      if (dl == 0 && t < tc) {
+        const float s = d * scale;
+        sc[t] = s;
+        if (score_out && !single) score_out[t0 + t] = s;  // raw score; normalised in the last pass
+      }
+    });
+    load(vv, V4, 0);
     __syncthreads();
     // ---- running softmax statistics --------------------------------------------------------
     float mx = -INFINITY;
@@ -119,24 +156,13 @@ __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
       __syncthreads();
     }
     // ---- o += sum_t p[t] * V[t] --------------------------------------------------------------
-    for (int tb = 0; tb < tc; tb += TPI * 4) {
-      f32x4 vv[4];
-      float p[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = tb + u * TPI + tg;
-        const int tt = t < tc ? t : tc - 1;
-        vv[u] = active ? V4[(size_t)(t0 + tt) * stride4 + dl] : zero4;
-        p[u] = t < tc ? sc[tt] : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        o4.x = __builtin_fmaf(p[u], vv[u].x, o4.x);
-        o4.y = __builtin_fmaf(p[u], vv[u].y, o4.y);
-        o4.z = __builtin_fmaf(p[u], vv[u].z, o4.z);
-        o4.w = __builtin_fmaf(p[u], vv[u].w, o4.w);
-      }
-    }
+    stream(V4, vv, [&](const f32x4& v4, int t) __attribute__((always_inline)) {
+      const float p = t < tc ? sc[t] : 0.f;
+      o4.x = __builtin_fmaf(p, v4.x, o4.x);
+      o4.y = __builtin_fmaf(p, v4.y, o4.y);
+      o4.z = __builtin_fmaf(p, v4.z, o4.z);
+      o4.w = __builtin_fmaf(p, v4.w, o4.w);
+    });
     __syncthreads();  // sc is rewritten by the next chunk
   }
 
@@ -161,7 +187,7 @@ __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
   if (score_out) {
     // probabilities as the reference leaves them in the score tensor
     const float inv_l = l_run;
-    for (int t = tid; t < nT; t += kh_wg()) score_out[t] = expf(score_out[t] - m_run) / inv_l;
+    for (int t = tid; t < nT; t += kh_wg()) score_out[t] = single ? sc[t] : expf(score_out[t] - m_run) / inv_l;
   }
 }
 

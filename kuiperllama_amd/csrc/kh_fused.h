@@ -173,7 +173,7 @@ static __global__ __launch_bounds__(KH_WG_MAX) void k_attn_generic(const KhAttnA
   const int pos = *a.d_pos;
   const int h = blockIdx.x;
   const size_t head_off = (size_t)(h / a.kv_mul) * a.head_size;
-  attn_head_decode(a.q + (size_t)h * a.head_size, a.kcache_layer + head_off,
+  attn_head_decode<4>(a.q + (size_t)h * a.head_size, a.kcache_layer + head_off,
                    a.vcache_layer + head_off, a.kv_dim, a.head_size, pos,
                    a.out + (size_t)h * a.head_size, nullptr, (float*)smem_raw);
 }

@@ -452,7 +452,10 @@ extern "C" int kh_sincos_cache_f32(int32_t head_size, int32_t max_seq_len, float
 
 // =============================================================================================
 // multi-head attention (decode).  Device core in kh_attn.h.
-__global__ __launch_bounds__(KH_WG) void k_mha(const int32_t* __restrict__ d_pos, int pos_val,
+// One workgroup of eight waves per head, eight timesteps per thread and batch, two batches in flight: the launch is a chain
+// of memory trips (scores, then values), so their number counts.  Back to back on Llama-3.2-1B's geometry, us at positions
+// 30 / 255 / 700 / 4000: 5.5 / 11.0 / 24.2 / 148 with four waves, four timesteps and one batch, 5.4 / 7.9 / 15.1 / 81 now.
+__global__ __launch_bounds__(KH_WG_MAX) void k_mha(const int32_t* __restrict__ d_pos, int pos_val,
                                                int layer_index, int seq_len, int kv_dim,
                                                int kv_mul, int head_size,
                                                float* __restrict__ mha_out,
@@ -465,7 +468,7 @@ __global__ __launch_bounds__(KH_WG) void k_mha(const int32_t* __restrict__ d_pos
   const int h = blockIdx.x;
   const size_t layer_off = (size_t)layer_index * (size_t)seq_len * (size_t)kv_dim;
   const size_t head_off = (size_t)(h / kv_mul) * head_size;
-  attn_head_decode(q + (size_t)h * head_size, kcache + layer_off + head_off,
+  attn_head_decode<8>(q + (size_t)h * head_size, kcache + layer_off + head_off,
                    vcache + layer_off + head_off, kv_dim, head_size, pos,
                    mha_out + (size_t)h * head_size, score ? score + (size_t)h * seq_len : nullptr,
                    (float*)smem_raw);
@@ -521,7 +524,7 @@ extern "C" int kh_mha_f32(const int32_t* d_pos, int32_t pos, int32_t head_num,
     // one workgroup per head (kh_mha_decode_f32 adds the long-context time split)
     return launch_mha_fast(d_pos, pos, head_num, layer_index, seq_len, kv_dim, kv_mul, head_size,
                            mha_out, q, kcache, vcache, 1, 0, 1, 1 << 30, nullptr, s);
-  hipLaunchKernelGGL(k_mha, dim3(head_num), dim3(KH_WG), attn_lds_bytes(head_size), s, d_pos,
+  hipLaunchKernelGGL(k_mha, dim3(head_num), dim3(KH_WG_MAX), attn_lds_bytes(head_size, KH_WG_MAX), s, d_pos,
                      pos, layer_index, seq_len, kv_dim, kv_mul, head_size, mha_out, q, score,
                      kcache, vcache);
   return kh_launch_status();

@@ -587,3 +587,29 @@ def test_softmax_scale_scalesum(gpu, oracle):
     ops.scale_sum(dev(v, gpu), dev(s, gpu), out, pos, size, stride)
     ref = (s[:, None].astype(np.float64) * v.reshape(pos + 1, stride)[:, :size]).sum(0)
     np.testing.assert_allclose(host(out), ref, rtol=0, atol=1e-5)
+
+
+@pytest.mark.parametrize("heads,kv_heads,hs", [(8, 2, 64), (4, 4, 128), (6, 6, 48), (2, 1, 256), (4, 2, 16)])
+def test_mha_score_form_batch_edges(gpu, oracle, heads, kv_heads, hs):
+    """k_mha: positions around one request of the workgroup (512 / lanes per timestep timesteps), a batch of eight, two
+    batches and the odd batch behind them, and the LDS score chunk of 2048."""
+    from kuiperllama_amd import ops
+    seq = 2400
+    rng = np.random.default_rng(hs)
+    kv_dim, kv_mul, dim = kv_heads * hs, heads // kv_heads, heads * hs
+    kc = rng.standard_normal((1, seq, kv_dim)).astype(np.float32)
+    vc = rng.standard_normal((1, seq, kv_dim)).astype(np.float32)
+    q = rng.standard_normal(dim).astype(np.float32)
+    kcd, vcd, qd = dev(kc, gpu), dev(vc, gpu), dev(q, gpu)
+    lanes = 1
+    while lanes < hs // 4:
+        lanes *= 2
+    one = 512 // lanes
+    edges = {n + d for n in (one, 2 * one, 8 * one, 16 * one, 24 * one, 2048) for d in (-2, -1, 0)}
+    for pos in sorted(p for p in edges if 0 <= p < seq):
+        out = torch.full((dim,), float("nan"), device=gpu)
+        score = torch.full((heads, seq), float("nan"), device=gpu)
+        ops.mha(pos, heads, 0, seq, kv_dim, kv_mul, hs, out, qd, score, kcd, vcd)
+        oo, so = oracle.mha(pos, heads, 0, seq, kv_dim, kv_mul, hs, q, kc, vc, acc=oracle.ACC_F64)
+        np.testing.assert_allclose(host(out), oo, rtol=0, atol=3e-5, err_msg=str(pos))
+        np.testing.assert_allclose(host(score)[:, : pos + 1], so[:, : pos + 1], rtol=0, atol=3e-6, err_msg=str(pos))
