@@ -50,6 +50,7 @@ struct Hybrid;  // kh_hybrid.h: a layer-list model
 using khm::LayerW;
 
 #define KH_PAIR_TMAX 2048   // prompt tokens of one pass on the pair GEMMs
+#define KH_PA_WS_MAX ((size_t)256 << 20)  // the most memory for one layer's K / V as pairs
 #define KH_STEP_VARIANTS 3  // kh_model_step.hip::step_variant
 struct kh_model {
   khm::Hybrid* hy = nullptr;  // layer-list model (checkpoint folder); nullptr: a .bin image
@@ -120,6 +121,8 @@ struct kh_model {
   float* pair_ws = nullptr;
   size_t pair_ws_layer = 0;
   bool pair_ready = false;
+  char* pa_ws = nullptr;     // K / V of one layer as pairs in fragment order (kh_pattn_pair.h)
+  size_t pa_ws_bytes = 0;
   bool kv_foreign = false;  // cache rows may hold values that this model did not compute (kh_model_write_kv, _get_kv)
   int pg_rows = 0;  // token rows of the slabs above
   bool pf_ready = false, pg_ready = false;  // set when ALL prefill slabs exist (allocation can fail half-way)

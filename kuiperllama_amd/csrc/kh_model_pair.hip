@@ -8,7 +8,7 @@
 #include <vector>
 
 #include "kh_model_internal.h"
-#include "kh_pair.h"
+#include "kh_pattn_pair.h"
 
 using namespace khm;
 
@@ -140,6 +140,62 @@ int ensure_pair(kh_model* m) {
   return KH_OK;
 }
 
+namespace {
+template <int HS, int QT>
+void pa_go(const KhPaArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_pa_pack<HS>, dim3((a.pos0 + a.T + 31) / 32, a.kv_heads), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((k_pa_attn<HS, 4, QT>), dim3(a.kv_heads * a.kv_mul * ((a.T + 16 * QT - 1) / (16 * QT))), dim3(256), 0, s, a);
+}
+template <int HS>
+size_t pa_bytes(int heads, int blocks) { return (size_t)heads * blocks * (PaGeom<HS>::FR * 1024 + sizeof(float)); }
+
+// Attention of a slice with its operands as pairs; false: the caller takes pg_slice_attention (fp32 matrix cores).
+// Packing reads all of the layer's rows whatever T is, so it needs enough query tokens and enough work.  Whole prompt
+// passes, ms, fp32 matrix cores against pairs, T @ first position: Llama-3.2-1B 128 @ 0 1.98 / 2.00, 256 @ 0 2.68 / 2.68,
+// 512 @ 0 4.05 / 3.94, 64 @ 2048 2.05 / 2.05, 256 @ 2048 3.42 / 3.06, 2048 @ 2048 20.3 / 14.6; Llama-2-7B int8
+// 128 @ 0 7.07 / 7.13, 256 @ 0 10.5 / 10.3, 128 @ 1024 8.08 / 7.83, 1024 @ 1024 41.5 / 34.5.
+// The slab of a layer is given up (not the call) above KH_PA_WS_MAX and where memory for it is refused.
+bool pair_attention(kh_model* m, int l, int T, int pos0, const float* out_s) {
+  const kh_config& c = m->cfg;
+  if (m->kv_foreign || dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
+  if (T < 128 || (size_t)T * (2 * (size_t)pos0 + T) < 65536) return false;
+  KhPaArgs a{};
+  a.blocks = (pos0 + T + 31) / 32;
+  size_t need = 0;
+  switch (c.head_size) {
+    case 48: need = pa_bytes<48>(c.kv_head_num, a.blocks); break;
+    case 64: need = pa_bytes<64>(c.kv_head_num, a.blocks); break;
+    case 128: need = pa_bytes<128>(c.kv_head_num, a.blocks); break;
+    default: return false;
+  }
+  if (need > KH_PA_WS_MAX) return false;
+  if (need > m->pa_ws_bytes) {
+    if (m->pa_ws) (void)hipFree(m->pa_ws);
+    m->pa_ws = nullptr;
+    m->pa_ws_bytes = 0;
+    if (dalloc(&m->pa_ws, need) != KH_OK) {
+      (void)hipGetLastError();
+      return false;
+    }
+    m->pa_ws_bytes = need;
+  }
+  a.q = m->pg_q;
+  a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
+  a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
+  a.slab = m->pa_ws;
+  a.kinv = (float*)(m->pa_ws + need - (size_t)c.kv_head_num * a.blocks * sizeof(float));
+  a.out_s = out_s;
+  a.out = (char*)m->pg_att;
+  a.dim = c.dim; a.kv_dim = c.kv_dim; a.kv_heads = c.kv_head_num; a.kv_mul = c.kv_mul; a.T = T; a.pos0 = pos0;
+  switch (c.head_size) {
+    case 48: pa_go<48, 2>(a, m->stream); break;
+    case 64: pa_go<64, 2>(a, m->stream); break;
+    default: pa_go<128, 1>(a, m->stream); break;
+  }
+  return true;
+}
+}  // namespace
+
 // forward of T (<= pg_rows) prompt tokens at positions pos0..: fills their K/V cache rows
 int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0) {
   const kh_config& c = m->cfg;
@@ -187,7 +243,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     // the prompt phase leaves K/V rows and nothing else: the last layer's attention, wo and feed-forward feed nothing
     if (l == c.layer_num - 1) break;
     // the attention kernel leaves pairs where the static bound of the value rows holds
-    const bool pairs = pg_slice_attention(m, l, T, pos0, 0, m->kv_foreign ? nullptr : sc + 3);
+    const bool pairs = pair_attention(m, l, T, pos0, sc + 3) || pg_slice_attention(m, l, T, pos0, 0, m->kv_foreign ? nullptr : sc + 3);
     if (!pairs) hipLaunchKernelGGL(k_pair_convert, dim3(T), dim3(KH_WG), 0, m->stream, (const float*)m->pg_att, xn, att_s, c.dim);
     {
       KhPairArgs a = base;

@@ -504,7 +504,7 @@ int ensure_pinned_words(kh_model* m, int n) {
 
 // The runtime moves logits to pageable memory by pinning or staging it.  Through pinned memory and a host copy one row of
 // 32 k takes 15 us instead of 59, of 128 k 30 instead of 31, and the steps of four sequences need no buffer allocated and
-// cleared per step: 20 us less of about 430 each.  One long prompt's single row gains nothing and is copied directly; above
+// cleared per step: 30 us less each.  One long prompt's single row gains nothing and is copied directly; above
 // 4 MB the second pass over the rows costs what the first saves.
 float* logits_pin(kh_model* m, size_t n) {
   if (n > (1u << 20)) return nullptr;
