@@ -80,7 +80,7 @@ int kh_embedding_f32(const int32_t* tokens, int32_t n_tokens, const float* w, fl
 
 /* The same with the token ids in HOST memory, which is what the reference's EmbeddingKernel
  * receives (the input tensor is a CPU tensor, op/embedding.cpp; emb_kernel.cu:25-29 uploads it per
- * call).  The ids travel in the kernel arguments, 64 per launch: no staging buffer, no copy. */
+ * call).  The ids travel in the kernel arguments, up to 512 per launch: no staging buffer, no copy. */
 int kh_embedding_f32_host(const int32_t* h_tokens, int32_t n_tokens, const float* w, float* out,
                           int32_t dim, int32_t vocab, void* stream);
 

@@ -71,7 +71,7 @@ def embedding(tokens, w, out):
 
 def embedding_host_tokens(tokens, w, out):
     """EmbeddingKernel as the reference calls it: `tokens` is a HOST int32 array (numpy); the ids
-    travel in the kernel arguments, 64 per launch (kh_embedding_f32_host)."""
+    travel in the kernel arguments, up to 512 per launch (kh_embedding_f32_host)."""
     import numpy as np
     t = np.ascontiguousarray(tokens, dtype=np.int32)
     _ffi.check(_ffi.lib().kh_embedding_f32_host(t.ctypes.data, t.size, _p(w), _p(out), w.shape[1],

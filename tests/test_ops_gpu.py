@@ -613,3 +613,18 @@ def test_mha_score_form_batch_edges(gpu, oracle, heads, kv_heads, hs):
         oo, so = oracle.mha(pos, heads, 0, seq, kv_dim, kv_mul, hs, q, kc, vc, acc=oracle.ACC_F64)
         np.testing.assert_allclose(host(out), oo, rtol=0, atol=3e-5, err_msg=str(pos))
         np.testing.assert_allclose(host(score)[:, : pos + 1], so[:, : pos + 1], rtol=0, atol=3e-6, err_msg=str(pos))
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 511, 512, 513, 576, 577, 1500])
+def test_embedding_host_tokens_launch_edges(gpu, n):
+    """Lists that fill a launch of 64 or of 512 ids, and one more; an id out of range leaves its row alone."""
+    from kuiperllama_amd import ops
+    rng = np.random.default_rng(n)
+    w = rng.standard_normal((300, 20)).astype(np.float32)
+    tok = rng.integers(0, 300, n).astype(np.int32)
+    tok[n // 2] = 300
+    out = torch.full((n, 20), 7.0, device=gpu)
+    ops.embedding_host_tokens(tok, dev(w, gpu), out)
+    want = w[np.minimum(tok, 299)]
+    want[n // 2] = 7.0
+    np.testing.assert_array_equal(host(out), want)
