@@ -271,8 +271,8 @@ class KuiperModel:
         torch.cuda.synchronize()
 
     def prefill_gemm(self, tokens: Sequence[int], pos0: int = 0) -> None:
-        """Forward of `tokens` at positions pos0.. as fp32-MFMA GEMMs (up to 128 tokens per weight
-        pass); K/V rows equal the token-by-token ones to fp32 round-off."""
+        """Forward of `tokens` at positions pos0.. as matrix-core GEMMs to fp32 accuracy (up to 2048 tokens
+        per weight pass); K/V rows equal the token-by-token ones to fp32 round-off."""
         _ffi.sync_env()
         t = (C.c_int32 * len(tokens))(*[int(x) for x in tokens])
         _ffi.check(_ffi.lib().kh_model_prefill_gemm(self._h, t, len(tokens), pos0),
@@ -284,7 +284,7 @@ class KuiperModel:
     def time_prefill(self, tokens: Sequence[int], pos0: int = 0, mode: str = "gemm") -> float:
         """Milliseconds (HIP events on the model stream) of the prompt phase alone for `tokens`:
         "token" = one forward pass per token (the reference), "gemv" = B-token VALU kernels,
-        "gemm" = fp32-MFMA GEMM prefill."""
+        "gemm" = matrix-core GEMM prefill."""
         _ffi.sync_env()
         t = (C.c_int32 * len(tokens))(*[int(x) for x in tokens])
         ms = C.c_float(0.0)
