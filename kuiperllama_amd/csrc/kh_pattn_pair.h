@@ -224,7 +224,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) sa[u][r] = p + 4 * u + r <= my ? sa[u][r] : -INFINITY;
       }
-      const float kq = ki0 * qs[qi];
+      const float kq = __builtin_amdgcn_fmed3f(ki0 * qs[qi], 0x1p-126f, 0x1p127f);  // 0 would make NaNs of the masked scores
       float tm = fmaxf(fmaxf(fmaxf(sa[0][0], sa[0][1]), fmaxf(sa[0][2], sa[0][3])),
                        fmaxf(fmaxf(sa[1][0], sa[1][1]), fmaxf(sa[1][2], sa[1][3])));
       tm = fmaxf(tm, __shfl_xor(tm, 16));

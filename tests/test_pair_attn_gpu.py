@@ -63,6 +63,22 @@ def test_spread_of_values_and_scores(gpu, hs, heads, kv_heads, half, monkeypatch
         elif base == "wq":
             w = binfmt.tensor_from_image(img, e)
             w.copy_(w * 16)
+    _close(monkeypatch, img, spec)
+
+
+@pytest.mark.parametrize("exp", [-30, -70, -90])
+def test_tiny_queries_and_keys(gpu, exp, monkeypatch):
+    """Scales of a block and of a token whose product leaves the range of fp32: every score is zero, masked ones stay masked."""
+    spec = _spec(64, 8, 2, True)
+    img = binfmt.synth_image(spec, seed=43, device=gpu)
+    for e in binfmt.layout(spec)[0]:
+        if e.name.split(".")[0] in ("wq", "wk"):
+            w = binfmt.tensor_from_image(img, e)
+            w.copy_(w * 2.0 ** exp)
+    _close(monkeypatch, img, spec)
+
+
+def _close(monkeypatch, img, spec):
     toks = [int(t) for t in np.random.default_rng(9).integers(0, spec.vocab_size, 600)]
     a, b = _both(monkeypatch, img, spec, [(toks, 0)])
     for x, y in zip(a, b):
