@@ -18,6 +18,7 @@
 #define KH_WAVES_MAX (KH_WG_MAX / KH_WAVE)
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f32x4 f4_zero() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 #define KH_CHECK_HIP(expr)                      \

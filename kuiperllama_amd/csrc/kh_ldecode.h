@@ -44,7 +44,6 @@ __device__ __forceinline__ int ld_slot(int i) {
   const int b = i / B4, r = i - b * B4;
   return b * B4 + (r % P) * 64 + r / P;
 }
-__device__ __forceinline__ f32x4 f4_zero() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 // n4 valid float4 of src -> slots [0, total4), zeros behind them; times g
 template <class T, int NT>
 __device__ __forceinline__ void ld_stage(f32x4* xs, const float* src, int n4, int total4, float g, int tid) {

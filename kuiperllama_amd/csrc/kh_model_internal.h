@@ -116,8 +116,11 @@ struct kh_model {
   float* pg_part = nullptr;     // partial rows of residual GEMMs that split K across workgroups
   void* pg_ws = nullptr;        // KH_PG_TMAX attention split workspaces
   size_t pg_ws_tok_bytes = 0;
-  // pair GEMMs (kh_pair.h): per layer four scales (k_pair_scales) and the scale of every weight row (fp32), then one scale
-  // per attention output of a pass, then three words per layer
+  // pair GEMMs (kh_pair.h): 1 / the scales of the rows of pairs: of normed rows one a token, of attention outputs and of the
+  // gated unit one a token and stage
+  float* pg_xs = nullptr;
+  unsigned char *pg_ae = nullptr, *pg_he = nullptr;
+  // per layer the scale of the value rows, three words unused and the scale of every weight row (fp32), then a word per layer
   float* pair_ws = nullptr;
   size_t pair_ws_layer = 0;
   bool pair_ready = false;
@@ -222,7 +225,7 @@ int run_selftests(kh_model* m);
 // ---- kh_model_prefill.hip -------------------------------------------------------------------
 bool prefill_supported(const kh_model* m);  // B-token VALU path
 bool pg_supported(const kh_model* m);       // MFMA GEMM path
-bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int tcap, const float* pair_scale);
+bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int layout, int tcap);
 // pair GEMMs (kh_model_pair.hip)
 bool pair_geometry(const kh_config& c);
 int ensure_pair(kh_model* m);  // scales of the weights, once

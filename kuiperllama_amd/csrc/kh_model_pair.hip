@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "kh_model_internal.h"
+#include "kh_pattn.h"
 #include "kh_pattn_pair.h"
 
 using namespace khm;
@@ -56,7 +57,7 @@ PairShape pair_shape(bool q, int T, int N, int K, bool resid) {
 
 template <bool Q, int EPI, int TM, int TN, int WM, int WN, int NST>
 int pair_go(hipStream_t s, KhPairArgs a, int kz) {
-  typedef PairCfg<Q, TM, TN, WM, WN, NST> C;
+  typedef PairCfg<Q, EPI == KH_PG_RESID, TM, TN, WM, WN, NST> C;
   auto kern = k_pair_gemm<Q, EPI, TM, TN, WM, WN, NST>;
   if (C::LDS > 64 * 1024) {  // the dynamic-LDS opt-in is per (device, kernel): once
     static thread_local std::vector<int> done;
@@ -75,14 +76,16 @@ int pair_go(hipStream_t s, KhPairArgs a, int kz) {
   return KH_OK;
 }
 // *kz_out: K slices whose partial rows the next RMSNorm has to add (0: the epilogue added itself)
+// *fine_out: SWIGLU left a scale per 32 columns instead of 64
 template <int EPI>
-int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out) {
+int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out, int* fine_out = nullptr) {
   PairShape sh = pair_shape(m->cfg.is_quant, a.T, a.N, a.K, EPI == KH_PG_RESID);
   if (const char* e = dbg("KH_PAIR_SHAPE")) {  // test hook "tile,kz"
     int t = 0, kz = 1;
     if (sscanf(e, "%d,%d", &t, &kz) == 2 && t >= 0 && t < 4 && (kz == 1 || kz == 2 || kz == 4))
       sh = PairShape{t, EPI == KH_PG_RESID ? kz : 1};
   }
+  if (fine_out) *fine_out = kPairTiles[m->cfg.is_quant][sh.tile].bn < 128;
   if (kz_out) *kz_out = sh.kz > 1 ? sh.kz : 0;
   if (m->cfg.is_quant) {
     switch (sh.tile) {
@@ -95,7 +98,7 @@ int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out) {
   switch (sh.tile) {
     case 0: return pair_go<false, EPI, 8, 2, 1, 4, 2>(m->stream, a, sh.kz);
     case 1: return pair_go<false, EPI, 4, 2, 1, 4, 3>(m->stream, a, sh.kz);
-    case 2: return pair_go<false, EPI, 2, 2, 1, 4, 4>(m->stream, a, sh.kz);
+    case 2: return pair_go<false, EPI, 2, 2, 1, 4, EPI == KH_PG_RESID ? 3 : 4>(m->stream, a, sh.kz);
     default: return pair_go<false, EPI, 1, 2, 2, 2, 6>(m->stream, a, sh.kz);
   }
 }
@@ -116,24 +119,24 @@ int ensure_pair(kh_model* m) {
   const size_t rows = 3 * (size_t)c.dim + 2 * (size_t)c.kv_dim + 2 * (size_t)c.hidden_dim;  // wq wk wv wo w1 w3 w2
   const size_t per = (c.is_quant ? 0 : rows) + 4;
   int rc;
-  if ((rc = dalloc(&m->pair_ws, per * c.layer_num + KH_PAIR_TMAX + 3 * c.layer_num)) != KH_OK) return rc;
+  if ((rc = dalloc(&m->pair_ws, (per + 1) * c.layer_num)) != KH_OK) return rc;
   m->pair_ws_layer = per;
-  unsigned* norms = (unsigned*)(m->pair_ws + per * c.layer_num + KH_PAIR_TMAX);
-  KH_CHECK_HIP(hipMemsetAsync(norms, 0, 3 * sizeof(unsigned) * c.layer_num, m->stream));
+  unsigned* norms = (unsigned*)(m->pair_ws + per * c.layer_num);
+  KH_CHECK_HIP(hipMemsetAsync(norms, 0, sizeof(unsigned) * c.layer_num, m->stream));
   for (int l = 0; l < c.layer_num; ++l) {
     const LayerW& W = m->layers[l];
-    unsigned* nm = norms + 3 * l;
+    unsigned* nm = norms + l;
     const KhPairMats mats = {{{W.wq, c.dim, c.dim, nullptr, nullptr},
                               {W.wk, c.kv_dim, c.dim, nullptr, nullptr},
-                              {W.wv, c.kv_dim, c.dim, W.att_norm, nm + 2},
+                              {W.wv, c.kv_dim, c.dim, W.att_norm, nm},
                               {W.wo, c.dim, c.dim, nullptr, nullptr},
-                              {W.w1, c.hidden_dim, c.dim, W.ffn_norm, nm},
-                              {W.w3, c.hidden_dim, c.dim, W.ffn_norm, nm + 1},
+                              {W.w1, c.hidden_dim, c.dim, nullptr, nullptr},
+                              {W.w3, c.hidden_dim, c.dim, nullptr, nullptr},
                               {W.w2, c.dim, c.hidden_dim, nullptr, nullptr}}};
     if (c.is_quant) hipLaunchKernelGGL(k_pair_rows<true>, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, (float*)nullptr, (int)rows);
     else hipLaunchKernelGGL(k_pair_rows<false>, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, m->pair_ws + per * l + 4, (int)rows);
-    hipLaunchKernelGGL(k_pair_scales, dim3(1), dim3(256), 0, m->stream, W.att_norm, W.ffn_norm, W.wv.bias, (const unsigned*)nm, c.dim,
-                       c.kv_dim, m->pair_ws + per * l);
+    hipLaunchKernelGGL(k_pair_scales, dim3(1), dim3(256), 0, m->stream, W.wv.bias, (const unsigned*)nm, c.dim, c.kv_dim,
+                       m->pair_ws + per * l);
   }
   if ((rc = kh_launch_status()) != KH_OK) return rc;
   m->pair_ready = true;
@@ -155,7 +158,7 @@ size_t pa_bytes(int heads, int blocks) { return (size_t)heads * blocks * (PaGeom
 // 512 @ 0 4.05 / 3.94, 64 @ 2048 2.05 / 2.05, 256 @ 2048 3.42 / 3.06, 2048 @ 2048 20.3 / 14.6; Llama-2-7B int8
 // 128 @ 0 7.07 / 7.13, 256 @ 0 10.5 / 10.3, 128 @ 1024 8.08 / 7.83, 1024 @ 1024 41.5 / 34.5.
 // The slab of a layer is given up (not the call) above KH_PA_WS_MAX and where memory for it is refused.
-bool pair_attention(kh_model* m, int l, int T, int pos0, const float* out_s) {
+bool pair_attention(kh_model* m, int l, int T, int pos0, const float* v_s) {
   const kh_config& c = m->cfg;
   if (m->kv_foreign || dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
   if (T < 128 || (size_t)T * (2 * (size_t)pos0 + T) < 65536) return false;
@@ -184,8 +187,11 @@ bool pair_attention(kh_model* m, int l, int T, int pos0, const float* out_s) {
   a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
   a.slab = m->pa_ws;
   a.kinv = (float*)(m->pa_ws + need - (size_t)c.kv_head_num * a.blocks * sizeof(float));
-  a.out_s = out_s;
-  a.out = (char*)m->pg_att;
+  a.v_s = v_s;
+  a.out = m->pg_att;
+  a.out_e = m->pg_ae;
+  a.stage = KH_PAIR_STAGE(c.is_quant);
+  a.tcap = m->pg_rows;
   a.dim = c.dim; a.kv_dim = c.kv_dim; a.kv_heads = c.kv_head_num; a.kv_mul = c.kv_mul; a.T = T; a.pos0 = pos0;
   switch (c.head_size) {
     case 48: pa_go<48, 2>(a, m->stream); break;
@@ -202,7 +208,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
   int rc;
   if ((rc = kh_embedding_f32_host(toks, T, m->tok_emb, m->pg_x, c.dim, c.vocab_size, (void*)m->stream)) != KH_OK) return rc;
   char *xn = (char*)m->pg_xn, *h = (char*)m->pg_h;  // pair slabs: four bytes a number, like the fp32 slabs
-  float* att_s = m->pair_ws + m->pair_ws_layer * c.layer_num;
+  int fine = 0;
   int kz = 0;  // K slices of the last residual GEMM still to be added to pg_x
   const bool rope_fuse = !dbg_off("KH_PG_ROPE_FUSE");
   for (int l = 0; l < c.layer_num; ++l) {
@@ -211,25 +217,26 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     const float* ws = sc + 4;  // row scales: wq, wk, wv, wo, w1, w3, w2
     const float* ws_o = ws + c.dim + 2 * c.kv_dim;
     const float* ws_1 = ws_o + c.dim;
-    auto rmsnorm = [&](const float* w, const float* scale) {
-      hipLaunchKernelGGL(k_pair_rmsnorm, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_x, w, xn, scale, c.dim, c.rms_eps, m->pg_rows,
+    auto rmsnorm = [&](const float* w) {
+      hipLaunchKernelGGL(k_pair_rmsnorm, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_x, w, xn, m->pg_xs, c.dim, c.rms_eps, m->pg_rows,
                          (const float*)m->pg_part, kz);
       kz = 0;
     };
     KhPairArgs base{};
     base.T = T;
     base.pos0 = pos0;
-    base.tcap = m->pg_rows;
+    base.tcap = base.xe_ld = m->pg_rows;
+    base.xs = m->pg_xs;
     base.part = m->pg_part;
     base.head_size = c.head_size;
     base.sin_cache = m->sin_cache;
     base.cos_cache = m->cos_cache;
-    rmsnorm(W.att_norm, sc);
+    rmsnorm(W.att_norm);
     {
       KhPairArgs a = base;
       a.w[0] = W.wq; a.w[1] = W.wk; a.w[2] = W.wv;
       a.ws[0] = ws; a.ws[1] = ws + c.dim; a.ws[2] = ws + c.dim + c.kv_dim;
-      a.X = xn; a.xs = sc; a.out = m->pg_q;
+      a.X = xn; a.out = m->pg_q;
       a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
       a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
       a.rows0 = c.dim; a.rows1 = c.kv_dim; a.N = c.dim + 2 * c.kv_dim; a.ldo = c.dim; a.K = c.dim;
@@ -242,29 +249,31 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     }
     // the prompt phase leaves K/V rows and nothing else: the last layer's attention, wo and feed-forward feed nothing
     if (l == c.layer_num - 1) break;
-    // the attention kernel leaves pairs where the static bound of the value rows holds
-    const bool pairs = pair_attention(m, l, T, pos0, sc + 3) || pg_slice_attention(m, l, T, pos0, 0, m->kv_foreign ? nullptr : sc + 3);
-    if (!pairs) hipLaunchKernelGGL(k_pair_convert, dim3(T), dim3(KH_WG), 0, m->stream, (const float*)m->pg_att, xn, att_s, c.dim);
+    // the attention kernels leave pairs where 64 columns are of one head
+    bool pairs = c.head_size % 64 == 0;
+    if (!pair_attention(m, l, T, pos0, sc)) pairs = pg_slice_attention(m, l, T, pos0, pairs ? KH_PA_PAIRS : KH_PA_ROWS, m->pg_rows);
+    if (!pairs) hipLaunchKernelGGL(k_pair_convert, dim3(T), dim3(KH_WG), 0, m->stream, (const float*)m->pg_att, xn, m->pg_ae, c.dim, m->pg_rows,
+                                   KH_PAIR_STAGE(c.is_quant) / 4);
     {
       KhPairArgs a = base;
       a.w[0] = W.wo; a.ws[0] = ws_o;
-      a.X = pairs ? (const char*)m->pg_att : xn; a.xs = pairs ? sc + 3 : att_s; a.xs_tok = !pairs; a.out = m->pg_x;
+      a.X = pairs ? (const char*)m->pg_att : xn; a.xe = m->pg_ae; a.out = m->pg_x;
       a.rows0 = a.N = a.ldo = a.K = c.dim;
       if ((rc = pair_launch<KH_PG_RESID>(m, a, &kz)) != KH_OK) return rc;
     }
-    rmsnorm(W.ffn_norm, sc + 1);
+    rmsnorm(W.ffn_norm);
     {
       KhPairArgs a = base;
       a.w[0] = W.w1; a.w[1] = W.w3;
       a.ws[0] = ws_1; a.ws[1] = ws_1 + c.hidden_dim;
-      a.X = xn; a.xs = sc + 1; a.pairs = h; a.out_s = sc + 2;
+      a.X = xn; a.pairs = h; a.out_e = m->pg_he;
       a.rows0 = c.hidden_dim; a.N = 2 * c.hidden_dim; a.ldo = c.hidden_dim; a.K = c.dim;
-      if ((rc = pair_launch<KH_PG_SWIGLU>(m, a, nullptr)) != KH_OK) return rc;
+      if ((rc = pair_launch<KH_PG_SWIGLU>(m, a, nullptr, &fine)) != KH_OK) return rc;
     }
     {
       KhPairArgs a = base;
       a.w[0] = W.w2; a.ws[0] = ws_1 + 2 * c.hidden_dim;
-      a.X = h; a.xs = sc + 2; a.out = m->pg_x;
+      a.X = h; a.xe = m->pg_he; a.fine = fine; a.out = m->pg_x;
       a.rows0 = a.N = a.ldo = c.dim; a.K = c.hidden_dim;
       if ((rc = pair_launch<KH_PG_RESID>(m, a, &kz)) != KH_OK) return rc;
     }

@@ -237,7 +237,11 @@ int ensure_pg_buffers(kh_model* m, int n) {
   m->pg_ready = false;
   // a previous attempt may have failed half-way (out of memory): start from a clean slate so a
   // later call never launches GEMMs on null slabs
-  for (float** p : {&m->pg_x, &m->pg_xn, &m->pg_q, &m->pg_att, &m->pg_h, &m->pg_part}) {
+  for (float** p : {&m->pg_x, &m->pg_xn, &m->pg_q, &m->pg_att, &m->pg_h, &m->pg_part, &m->pg_xs}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  }
+  for (unsigned char** p : {&m->pg_ae, &m->pg_he}) {
     if (*p) (void)hipFree(*p);
     *p = nullptr;
   }
@@ -258,6 +262,11 @@ int ensure_pg_buffers(kh_model* m, int n) {
   if ((rc = zalloc(&m->pg_att, T * c.dim)) != KH_OK) return rc;
   if ((rc = zalloc(&m->pg_h, T * c.hidden_dim)) != KH_OK) return rc;
   if ((rc = zalloc(&m->pg_part, (size_t)KH_PG_KZ_MAX * T * c.dim)) != KH_OK) return rc;  // K-slice partial rows
+  if (pair_geometry(c)) {
+    if ((rc = dalloc(&m->pg_xs, T)) != KH_OK) return rc;
+    if ((rc = dalloc(&m->pg_ae, pair_exp_bytes(c.dim, c.is_quant, rows))) != KH_OK) return rc;
+    if ((rc = dalloc(&m->pg_he, pair_exp_bytes(c.hidden_dim, c.is_quant, rows))) != KH_OK) return rc;
+  }
   m->pg_rows = rows;
   m->pg_ready = true;
   return KH_OK;
@@ -430,10 +439,10 @@ int pg_launch(kh_model* m, int rows_total, bool r2_ok, KhPgGemmArgs a) {
 }
 }  // namespace
 namespace khm {
-// Attention of T prompt tokens whose K/V rows have just been written: pg_q -> pg_att, as the tiled slab of k_pg_gemm
-// (tcap > 0), as pairs of the scale at pair_scale (returns true) or as rows [T][dim] (the decode kernel always).
-// MFMA kernel (kh_pattn.h) unless KH_PG_ATTN=0 or an odd head size.
-bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int tcap, const float* pair_scale) {
+// Attention of T prompt tokens whose K/V rows have just been written: pg_q -> pg_att in a layout of kh_pattn.h (pairs:
+// their scales to pg_ae; returns true) or as rows [T][dim] (the decode kernel always).  MFMA kernel (kh_pattn.h) unless
+// KH_PG_ATTN=0 or an odd head size.
+bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int layout, int tcap) {
   const kh_config& c = m->cfg;
   if (pg_mfma_attn(m)) {
     KhPgAttnArgs a{};
@@ -443,8 +452,9 @@ bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int tcap, const
     a.out = m->pg_att;
     a.dim = c.dim; a.kv_dim = c.kv_dim; a.kv_heads = c.kv_head_num; a.kv_mul = c.kv_mul;
     a.T = T; a.pos0 = pos0; a.tcap = tcap;
-    a.layout = tcap > 0 ? (c.is_quant ? KH_PA_TILED_Q8 : KH_PA_TILED_F32) : (pair_scale ? KH_PA_PAIRS : KH_PA_ROWS);
-    a.out_s = pair_scale;
+    a.layout = layout;
+    a.out_e = m->pg_ae;
+    a.stage = KH_PAIR_STAGE(c.is_quant);
     launch_pg_attn(a, c.head_size, m->stream);
     return a.layout == KH_PA_PAIRS;
   }
@@ -506,7 +516,7 @@ void launch_prefill_gemm_chunk(kh_model* m, const int32_t* toks, int T, int pos0
     // the prompt phase leaves K/V rows and nothing else (no logits): the last layer's K/V rows are
     // written, its attention, wo and FFN feed nothing (1/L of the pass minus one QKV GEMM)
     if (l == c.layer_num - 1) break;
-    pg_slice_attention(m, l, T, pos0, tcap, nullptr);
+    pg_slice_attention(m, l, T, pos0, c.is_quant ? KH_PA_TILED_Q8 : KH_PA_TILED_F32, tcap);
     {
       KhPgGemmArgs a{};
       a.w[0] = W.wo;

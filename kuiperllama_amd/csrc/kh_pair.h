@@ -3,26 +3,28 @@
 //
 //   C[rows, T] = W[rows, K] . X[T, K]^T      every number v of X and of fp32 weights travels as a PAIR of halves
 //       hi = fp16(s v),  lo = fp16(s v - hi)          s a power of two
-// hi + lo is s v to at most one unit in the last place of fp32 (11 + 11 bits and the sign of lo) as long as |s v| lies
-// between 2^-8 and 2^15, and to 2^-25 absolutely below that; a product takes three matrix instructions (hi hi, hi lo,
+// hi + lo is s v to at most one unit in the last place of fp32 (11 + 11 bits and the sign of lo) for |s v| from 2^-2 to 2^15
+// and to 2^-25 absolutely below that, where lo is a subnormal.  A product takes three matrix instructions (hi hi, hi lo,
 // lo hi; lo lo is 2^-22 of it at most) of v_mfma_f32_16x16x32_f16 into fp32 accumulators.  int8 weights are exact in
 // fp16 and take two; their group scale is applied in fp32 to the sum of each 64-column group.
 // Against v_mfma_f32_16x16x4_f32 the unit is 16 times as fast, so 5.3 (8) times the work per cycle is left, and a sum is
 // rounded once per 32 columns and product instead of once per 4 columns.
 //
-// Scales.  An activation row leaves RMSNorm with a Euclidean norm of at most sqrt(dim), so static bounds hold for every
-// input: |xn| <= sqrt(dim) max|g| and, for the gated unit, |h| <= max_j |w1_j * g| max_j |w3_j * g| dim (Cauchy-Schwarz;
-// typically 2^8 above the largest h, the pair spans 2^40 below its bound).  Attention outputs are averages of value rows,
-// |v| <= max_j |wv_j * g| sqrt(dim) + max|bias|.  k_pair_rows and k_pair_scales compute these and a scale for every weight
-// row once per model.  Once a caller has had its hands on the cache (kh_model_write_kv, kh_model_get_kv) the scale of an
-// attention output is its row maximum instead, found by a pass over the rows (k_pair_convert).
+// Scales bring the largest number that they cover to [2^14, 2^15): numbers down to 2^-16 of it keep the accuracy of fp32,
+// smaller ones have an error of 2^-39 of it.  Normed rows have one per token (k_pair_rmsnorm).  Attention outputs and the
+// gated unit have one per token and 64 columns, found where they are made (passes of few tokens: 32, see kPairTiles): a few
+// columns may be far above the others there, and a bound from the weights would have to hold for all of them (one row each
+// of w1 and w3 at 2^12 of its usual size, undone by w2: K/V rows 2.5e-2 from 64 bits instead of 4e-7).  Every weight row
+// has a scale, and the value rows have the bound |v| <= max_j |wv_j * g| sqrt(dim) + max|bias|, which k_pair_rows and
+// k_pair_scales compute once per model.  Once a caller has had its hands on the cache (kh_model_write_kv,
+// kh_model_get_kv) that bound does not hold and the attention keeps kh_pattn.h.
 //
 // Kernel: the stage ring of kh_lgemm.h.  A workgroup owns BM tokens x BN weight rows; a stage of 32 (int8: 64) columns
 // is moved to LDS by global_load_lds_dwordx4 in 128-byte rows (pairs: 32 hi | 32 lo; fp32 weights as they lie in the
 // file; int8 64-byte rows), swizzled so that the 16 rows of a fragment touch all banks.  fp32 weights are split in
-// registers behind the LDS read: two numbers take two multiplications, two v_cvt_pk_f16_f32 and two v_fma_mix_f32
-// (v_fma_mixlo / mixhi would be fewer but run at half their rate: 462 -> 389 us for w1 + w3 of Llama-3.2-1B at 2048 tokens).  Weights are the first MFMA operand, so a lane ends with four
-// consecutive rows of one token.
+// registers behind the LDS read: two numbers take two multiplications, two v_cvt_pk_f16_f32 and two v_fma_mix_f32.
+// (v_fma_mixlo / mixhi would be fewer, but they run at half the rate: w1 + w3 of Llama-3.2-1B at 2048 tokens took 462 us
+// with them and takes 389.)  Weights are the first MFMA operand, so a lane ends with four consecutive rows of one token.
 #pragma once
 #include <type_traits>
 
@@ -38,17 +40,20 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 // 64 banks hold two rows: with this table every fragment read of the kernel (16 rows; chunk h, 2 h or 2 (h & 1) by lane
 // group h) is free of conflicts, with r & 7 a third of the LDS cycles were.
 __device__ __forceinline__ int pair_swz(int r) { return ((r & 2) << 1) | ((r & 4) ? 3 : 0); }
-#define KH_PAIR_TOP 14  // a bound is scaled to at most 2^14: a factor of four below the largest fp16
+#define KH_PAIR_STAGE(Q) ((Q) ? 64 : 32)  // columns of a stage
+#define KH_PAIR_TOP 15  // a bound is scaled to less than 2^15: a factor of two below the largest fp16
 
 struct KhPairArgs {
   KhLin w[3];          // QKV: wq, wk, wv; RESID: w[0]; SWIGLU: w1, w3
   const float* ws[3];  // fp32 weights: the scale of every row
   const char* X;       // pair slab: [T][K / 32][32 hi | 32 lo]
-  const float* xs;     // its scale: one value, or one per token
-  int xs_tok;
+  const float* xs;     // QKV, SWIGLU: 1 / its scales, one per token
+  const unsigned char* xe;  // RESID: 1 / its scales, one per token and stage of columns, at pair_exp_at
+  int xe_ld;
+  int fine;            // RESID, fp32: the two stages of 64 columns may differ in scale
   float* out;          // QKV: Q [T][ldo]; RESID: X [T][ldo] (+=)
   char* pairs;         // SWIGLU: pair slab of the gated unit, [T][ldo / 32]
-  const float* out_s;  // SWIGLU: its scale
+  unsigned char* out_e;  // SWIGLU: 1 / its scales
   float* kc;           // QKV: K / V cache rows of this layer, row (pos0 + t) * rows1
   float* vc;
   float* part;         // RESID with gridDim.y > 1: partial rows [z][tcap][ldo], added by the k_pair_rmsnorm that follows
@@ -80,15 +85,21 @@ __device__ __forceinline__ void pair_store4(char* row, int k, const f32x4& v, fl
   *(f16x4*)(row + pair_at(k)) = hi;
   *(f16x4*)(row + pair_at(k) + 64) = lo;
 }
-// power of two that brings `bound` to at most 2^KH_PAIR_TOP (1 for 0, the smallest one for infinities and NaN)
+// power of two that brings `bound` to less than 2^KH_PAIR_TOP (1 for 0, the smallest one for infinities and NaN)
 __device__ __forceinline__ float pair_scale(float bound) {
   if (bound == 0.f) return 1.0f;
   int e = (int)((__float_as_uint(bound) >> 23) & 255) - 126;  // |bound| < 2^e
   int k = KH_PAIR_TOP - e;
-  k = k < -100 ? -100 : (k > 100 ? 100 : k);
+  k = k < -114 ? -114 : (k > 100 ? 100 : k);
   return __uint_as_float((unsigned)(k + 127) << 23);
 }
 __device__ __forceinline__ float pair_inv(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }  // 1 / s
+// 1 / s as its exponent, and where that of a token and a stage lies: 16 stages of a token side by side
+__device__ __forceinline__ unsigned char pair_exp(float s) { return (unsigned char)(254u - (__float_as_uint(s) >> 23)); }
+__device__ __forceinline__ size_t pair_exp_at(int stage, int t, int ld) { return ((size_t)(stage >> 4) * ld + t) * 16 + (stage & 15); }
+__host__ __device__ __forceinline__ size_t pair_exp_bytes(int K, bool q, int tokens) {
+  return (size_t)((K / KH_PAIR_STAGE(q) + 15) / 16) * 16 * tokens;
+}
 // eight int8, times sgn = +-1 -> fp16, exact: 0x6400 + u is 1024 + u, u = q + 128
 __device__ __forceinline__ f16x8 pair_q8(unsigned a, unsigned b, float sgn) {
   const f16x2 one = {(_Float16)sgn, (_Float16)sgn}, bias = {(_Float16)(-1152.0f * sgn), (_Float16)(-1152.0f * sgn)};
@@ -105,16 +116,18 @@ __device__ __forceinline__ f16x8 pair_q8(unsigned a, unsigned b, float sgn) {
   return r.v;
 }
 
-template <bool Q, int TM, int TN, int WM, int WN, int NST>
+// GROUP: whether X has a scale per group of columns
+template <bool Q, bool GROUP, int TM, int TN, int WM, int WN, int NST>
 struct PairCfg {
   static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN, NW = WM * WN;
   static constexpr int XB = Q ? 2 : 1;                     // 128-byte blocks of a token per stage
   static constexpr int XR = BM * XB / 8;                   // 1-KiB requests: activations
   static constexpr int WR = Q ? BN / 16 : BN / 8;          // weights
-  static constexpr int SR = Q ? BN / 64 : 0;               // 256-byte requests: group scales
+  static constexpr int SR = Q ? BN / 64 : 0;               // 256-byte requests: group scales of int8 weights
+  static constexpr int EX = GROUP ? (BM + 63) / 64 : 0;    // 1-KiB requests: scales of 16 stages, by the first waves
   static constexpr int STAGE = (XR + WR) * 1024 + SR * 256;
   static constexpr int NL = XR / NW + WR / NW + (Q ? 1 : 0);  // requests of a wave per stage
-  static constexpr int LDS = NST * STAGE;
+  static constexpr int LDS = NST * STAGE + 2 * EX * 1024;
   static_assert(NW % 2 == 0 && XR % NW == 0 && WR % NW == 0, "every wave issues the same number of requests");
 };
 
@@ -122,7 +135,8 @@ struct PairCfg {
 // the other, so its weights cross HBM once.  blockIdx.y = K slice (RESID).
 template <bool Q, int EPI, int TM, int TN, int WM, int WN, int NST>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs a) {
-  typedef PairCfg<Q, TM, TN, WM, WN, NST> C;
+  constexpr bool GROUP = EPI == KH_PG_RESID;
+  typedef PairCfg<Q, GROUP, TM, TN, WM, WN, NST> C;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int xcd = (int)blockIdx.x & 7, bj = (int)blockIdx.x >> 3;
@@ -159,8 +173,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   const char* wbase[NWR];
   const char* sbase = nullptr;
   const int sub = lane >> 3, ch8 = (lane & 7) ^ pair_swz(sub);
-  const int z0 = (int)((long)blockIdx.y * (K >> (Q ? 6 : 5)) / gridDim.y);
-  const int z1 = (int)((long)(blockIdx.y + 1) * (K >> (Q ? 6 : 5)) / gridDim.y);
+  const int groups = (K + 63) >> 6, stages = K >> (Q ? 6 : 5);  // slices begin at a multiple of 64 columns
+  const int z0 = (int)((long)blockIdx.y * groups / gridDim.y) * (Q ? 1 : 2);
+  int z1 = (int)((long)(blockIdx.y + 1) * groups / gridDim.y) * (Q ? 1 : 2);
+  z1 = z1 < stages ? z1 : stages;
 #pragma unroll
   for (int j = 0; j < NX; ++j) {
     const int r = 8 * (j * C::NW + wave) + sub;  // LDS row: block-major for int8
@@ -211,6 +227,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       sbase += 4;
     }
   };
+  // The scales of 16 stages: 16 bytes a token.  A request per stage (four bytes a token) made these GEMMs 5 % slower.
+  const int et = t0 + 64 * wave + lane;
+  const unsigned eoff = 16u * (unsigned)(et < a.T ? et : a.T - 1);
+  auto issue_exps = [&](int c) __attribute__((always_inline)) {
+    if (GROUP && wave < C::EX)
+      dma_x4_keep(a.xe + (size_t)c * a.xe_ld * 16, eoff, lds0 + (unsigned)(NST * C::STAGE + (c & 1) * C::EX * 1024));
+  };
   const int nk = z1 - z0;
   f32x4 acc[TN][TM];
 #pragma unroll
@@ -234,6 +257,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   // wait for them here: a wait left to their first use would sit in the loop and drain the ring
 #pragma unroll
   for (int n = 0; n < TN; ++n) asm volatile("" : "+v"(wsc[n]));
+  issue_exps(z0 >> 4);
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s)
     if (s < nk) issue(s);
@@ -242,13 +266,18 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   // The matrix unit rounds its sums down: a bias that the mean over many cached rows keeps while it averages everything else
   // (logits behind 1900 prompt tokens: 1.7e-6 from 64 bits instead of 1.3e-6 on fp32 fma chains).  Every other group takes
   // its weights with the sign turned and is subtracted, which cancels it: 1.1e-6.
-  float sgn = 1.0f;
+  float sgn = 1.0f, xinv[TM];
+  unsigned xe[TM];
   auto stage = [&](int k, auto open) __attribute__((always_inline)) {
-    constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a group
+    constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a sum
     // stage k has landed when at most the requests of the stages behind it are outstanding
+    // (and with it the scales, which were requested before those)
     if (NST > 2 && k + NST - 2 < nk) wait_vm<(NST - 2) * C::NL>();
     else wait_vm<0>();
     __syncthreads();
+    const int at = z0 + k;
+    if (GROUP && (k == 0 || (at & 15) == 0) && ((at >> 4) + 1) * 16 < z1) issue_exps((at >> 4) + 1);
+    const unsigned char* exps = (const unsigned char*)smem_raw + NST * C::STAGE + ((at >> 4) & 1) * C::EX * 1024 + (at & 15);
     if (k + NST - 1 < nk) issue(fill);
     const char* st = smem_raw + slot * C::STAGE;
     const char* wst = st + C::XR * 1024;
@@ -266,6 +295,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
         const int r = (wm * TM + m) * 16 + fr;
         xh[m] = *(const f16x8*)(st + r * 128 + ((fh ^ pair_swz(r)) << 4));
         xl[m] = *(const f16x8*)(st + r * 128 + (((4 + fh) ^ pair_swz(r)) << 4));
+      }
+      if constexpr (GROUP) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
       }
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(1);
@@ -309,8 +342,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
           xl[m][b] = *(const f16x8*)(row + (((4 + c) ^ pair_swz(r)) << 4));
         }
       }
+      if constexpr (GROUP) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
+      }
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+        if (GROUP) xinv[m] = sgn * __uint_as_float(xe[m] << 23);
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
         const f16x8 w0 = pair_q8((unsigned)qv[n].x, (unsigned)qv[n].y, sgn), w1 = pair_q8((unsigned)qv[n].z, (unsigned)qv[n].w, sgn);
@@ -327,7 +367,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(sg[i], g[m][i], acc[n][m][i]);
+          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(GROUP ? sc[n][i] * xinv[m] : sg[i], g[m][i], acc[n][m][i]);
       }
     }
     __builtin_amdgcn_s_setprio(0);
@@ -337,11 +377,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   auto close = [&]() __attribute__((always_inline)) {
     if constexpr (!Q) {
 #pragma unroll
+      for (int m = 0; m < TM; ++m) xinv[m] = GROUP ? sgn * __uint_as_float(xe[m] << 23) : sgn;
+#pragma unroll
       for (int n = 0; n < TN; ++n) {
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(sgn, grp[n][m][i], acc[n][m][i]);
+          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(xinv[m], grp[n][m][i], acc[n][m][i]);
         wsc[n] = -wsc[n];
       }
     }
@@ -358,6 +400,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     int k = 0;
     for (; k + 1 < nk; k += 2) {
       stage(k, first);
+      if (GROUP && a.fine) {  // uniform
+        close();
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+          for (int m = 0; m < TM; ++m) grp[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
       stage(k + 1, second);
       close();
     }
@@ -367,26 +416,75 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     }
   }
   // ---- epilogue: lane (fr, fh) of tile (n, m) holds rows 4 fh .. + 3 of the tile for token t0 + .. + fr
-  float xs = a.xs_tok ? 1.0f : a.xs[0];
-  const float os = EPI == KH_PG_SWIGLU ? a.out_s[0] : 1.0f;
+  float xi[TM];
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int tok = t0 + (wm * TM + m) * 16 + fr;
+    xi[m] = GROUP ? 1.0f : a.xs[tok < a.T ? tok : a.T - 1];
+  }
+  auto value = [&](int n, int m, int mat, int row) __attribute__((always_inline)) {
+    f32x4 v = acc[n][m];
+    f32x4 s = {1.f, 1.f, 1.f, 1.f};
+    if (!Q) s = *(const f32x4*)(a.ws[mat] + row);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (!GROUP) v[i] *= xi[m];
+      if (!Q) v[i] *= pair_inv(s[i]);
+    }
+    return v;
+  };
+  if constexpr (EPI == KH_PG_SWIGLU) {
+    // a wave holds 8 TN columns of the gated unit; 64 columns, those of `per` waves, share a scale, or the 32 of a workgroup
+    constexpr int per = WN * TN < 8 ? WN : 8 / TN, sub = KH_PAIR_STAGE(Q) / (8 * TN);  // sub: waves of a stage
+    static_assert(sub > 0 && per % sub == 0 && WN % per == 0, "whole stages in a workgroup");
+    float* tops = (float*)smem_raw;  // [WN][BM]
+    f32x4 o[TM][TN / 2];
+    __syncthreads();  // the last stage has been read
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      float top = 0.f;
+#pragma unroll
+      for (int n = 0; n < TN; n += 2) {
+        const int f = f0 + (wn * TN + n) * 16;
+        o[m][n / 2] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (f >= a.N) continue;
+        int mat, row;
+        place(f, mat, row);
+        row += 4 * fh;
+        const f32x4 g = value(n, m, 0, row), u = value(n + 1, m, 1, row);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o[m][n / 2][i] = swiglu1(g[i], u[i]);
+          top = fmaxf(top, fabsf(o[m][n / 2][i]));
+        }
+      }
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      if (fh == 0) tops[wn * C::BM + (wm * TM + m) * 16 + fr] = top;
+    }
+    __syncthreads();
+    const int stage = (f0 >> 1) / KH_PAIR_STAGE(Q) + wn / sub;
+#pragma unroll
+    for (int m = 0; m < TM; ++m) {
+      const int at = (wm * TM + m) * 16 + fr, tok = t0 + at;
+      if (tok >= a.T) continue;
+      float top = 0.f;
+#pragma unroll
+      for (int w = 0; w < per; ++w) top = fmaxf(top, tops[(wn / per * per + w) * C::BM + at]);
+      const float s = pair_scale(top);
+      if (fh == 0 && wn % sub == 0 && stage * 2 * KH_PAIR_STAGE(Q) < a.N) a.out_e[pair_exp_at(stage, tok, a.xe_ld)] = pair_exp(s);
+#pragma unroll
+      for (int n = 0; n < TN; n += 2) {
+        const int f = f0 + (wn * TN + n) * 16;
+        if (f < a.N) pair_store4(a.pairs + (size_t)tok * a.ldo * 4, (f >> 5) * 16 + 4 * fh, o[m][n / 2], s);
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
     const int tok = t0 + (wm * TM + m) * 16 + fr;
     if (tok >= a.T) continue;
-    if (a.xs_tok) xs = a.xs[tok];
-    const float ix = pair_inv(xs);
-    auto value = [&](int n, int mat, int row) __attribute__((always_inline)) {
-      f32x4 v = acc[n][m];
-      if (!Q) {
-        const f32x4 s = *(const f32x4*)(a.ws[mat] + row);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = v[i] * ix * pair_inv(s[i]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= ix;
-      }
-      return v;
-    };
 #pragma unroll
     for (int n = 0; n < TN; ++n) {
       const int f = f0 + (wn * TN + n) * 16;
@@ -394,15 +492,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       int mat, row;
       place(f, mat, row);
       row += 4 * fh;
-      if (EPI == KH_PG_SWIGLU) {
-        if (n & 1) continue;
-        const f32x4 g = value(n, 0, row), u = value(n + 1, 1, row);
-        f32x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = swiglu1(g[i], u[i]);
-        pair_store4(a.pairs + (size_t)tok * a.ldo * 4, row, o, os);
-      } else if (EPI == KH_PG_RESID) {
-        const f32x4 v = value(n, 0, row);
+      if (EPI == KH_PG_RESID) {
+        const f32x4 v = value(n, m, 0, row);
         if (gridDim.y > 1) {
           *(f32x4*)(a.part + ((size_t)blockIdx.y * a.tcap + tok) * a.ldo + row) = v;
         } else {  // residual add (llama3.cpp:686,719)
@@ -428,7 +519,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
         if (a.rope == KH_PG_ROPE_TILES) {
           if (n & 1) continue;
           // tile n + 1 holds the partners, half a head further; cache column 2 j (cpu/rope_kernel.cpp:18-42)
-          const f32x4 lo = biased(value(n, mat, row), row), hi = biased(value(n + 1, mat, row + (hs >> 1)), row + (hs >> 1));
+          const f32x4 lo = biased(value(n, m, mat, row), row), hi = biased(value(n + 1, m, mat, row + (hs >> 1)), row + (hs >> 1));
           f32x4 olo = lo, ohi = hi;
           if (mat < 2) {
             const int j = row % hs;
@@ -442,7 +533,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
           *(f32x4*)(dst + row) = olo;
           *(f32x4*)(dst + row + (hs >> 1)) = ohi;
         } else {
-          f32x4 v = biased(value(n, mat, row), row);
+          f32x4 v = biased(value(n, m, mat, row), row);
           if (mat < 2 && a.rope == KH_PG_ROPE_PAIRS) {  // pairs (row, row + 1) (cpu/rope_kernel.cpp:98-121)
             const int c = row % hs;
             const float s0 = sn[c], c0 = cs[c], s1 = sn[c + 2], c1 = cs[c + 2];
@@ -460,13 +551,13 @@ struct KhPairMats {  // the matrices of a layer
   struct {
     KhLin w;
     int rows, K;
-    const float* g;   // norm weights in front of it (w1, w3, wv)
+    const float* g;   // norm weights in front of it (wv)
     unsigned* norm;
   } m[7];
 };
-// Every row's atomicMax on one word took longer than the reading: only a larger norm sends one (a layer of Llama-3.2-1B
-// 209 -> 94 us, of Llama-2-7B int8 298 -> 107 us).  One wave per row of the stacked matrices: fp32 weights get the row's scale; with norm weights g the largest |w_row * g| of
-// the matrix goes to *norm (its bits: the values are positive).  16 bytes a lane; K is a multiple of 32 (int8: 64).
+// One wave per row of the stacked matrices: fp32 weights get the row's scale; with norm weights g the largest |w_row * g|
+// of the matrix goes to *norm (its bits: the values are positive).  16 bytes a lane; K is a multiple of 32 (int8: 64).
+// Every row's atomicMax on one word took longer than the reading, so only a larger norm sends one.
 template <bool Q>
 __global__ __launch_bounds__(256) void k_pair_rows(const KhPairMats a, float* ws, int total) {
   const int at = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -510,46 +601,46 @@ __global__ __launch_bounds__(256) void k_pair_rows(const KhPairMats a, float* ws
     if (norm && len > __hip_atomic_load(norm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(norm, len);
   }
 }
-// out: scales of the rows behind the attention and the feed-forward norm, of the gated unit and of the attention output.
-// norms: of w1, w3, wv; bv: bias of the value rows or null
-static __global__ __launch_bounds__(256) void k_pair_scales(const float* g_att, const float* g_ffn, const float* bv,
-                                                            const unsigned* norms, int dim, int kv_dim, float* out) {
-  __shared__ float red[3][4];
-  float m[3] = {0.f, 0.f, 0.f};
-  for (int k = threadIdx.x; k < dim; k += 256) {
-    m[0] = fmaxf(m[0], fabsf(g_att[k]));
-    m[1] = fmaxf(m[1], fabsf(g_ffn[k]));
-  }
+// out: scale of the value rows.  norm: of wv; bv: its bias or null
+static __global__ __launch_bounds__(256) void k_pair_scales(const float* bv, const unsigned* norm, int dim, int kv_dim, float* out) {
+  __shared__ float red[4];
+  float m = 0.f;
   if (bv)
-    for (int k = threadIdx.x; k < kv_dim; k += 256) m[2] = fmaxf(m[2], fabsf(bv[k]));
-  for (int i = 0; i < 3; ++i) {
-    for (int o = 32; o; o >>= 1) m[i] = fmaxf(m[i], __shfl_xor(m[i], o));
-    if ((threadIdx.x & 63) == 0) red[i][threadIdx.x >> 6] = m[i];
-  }
+    for (int k = threadIdx.x; k < kv_dim; k += 256) m = fmaxf(m, fabsf(bv[k]));
+  for (int o = 32; o; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 0; i < 3; ++i) m[i] = fmaxf(fmaxf(red[i][0], red[i][1]), fmaxf(red[i][2], red[i][3]));
-    const float x = sqrtf((float)dim);  // |x| / rms(x) at most
-    out[0] = pair_scale(m[0] * x);
-    out[1] = pair_scale(m[1] * x);
-    out[2] = pair_scale(__uint_as_float(norms[0]) * x * __uint_as_float(norms[1]) * x);
-    out[3] = pair_scale(__uint_as_float(norms[2]) * x + m[2]);
-  }
+  if (threadIdx.x == 0)  // |x| / rms(x) is at most sqrt(dim)
+    out[0] = pair_scale(__uint_as_float(norm[0]) * sqrtf((float)dim) + fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
 }
 
 // ---- the per-token kernels between the GEMMs ------------------------------------------------------------------------
+__device__ __forceinline__ float pair_top4(const f32x4& v) {
+  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+// Chunk k (four columns) of token t with a scale per 64 columns, whose chunks lie in 16 neighbouring lanes; chunks from n4 on
+// are zeros.  chunks: those of a stage (8 or 16), every stage gets the scale.
+__device__ __forceinline__ void pair_emit(char* row, unsigned char* exps, int ld, int t, int k, int n4, int chunks, const f32x4& v) {
+  float top = pair_top4(v);
+#pragma unroll
+  for (int o = 8; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+  if (k >= n4) return;
+  const float s = pair_scale(top);
+  pair_store4(row, 4 * k, v, s);
+  if ((k & (chunks - 1)) == 0) exps[pair_exp_at(k / chunks, t, ld)] = pair_exp(s);
+}
 // k_pg_rmsnorm (kh_gemm.h) with a row of pairs as its output; one workgroup per token
 static __global__ __launch_bounds__(KH_WG) void k_pair_rmsnorm(float* __restrict__ X, const float* __restrict__ w, char* __restrict__ out,
-                                                               const float* __restrict__ scale, int dim, float eps, int tcap,
+                                                               float* __restrict__ inv, int dim, float eps, int tcap,
                                                                const float* __restrict__ part, int kz) {
-  __shared__ float red[KH_WAVES_MAX];
+  __shared__ float red[KH_WG / KH_WAVE], tops[KH_WG / KH_WAVE];
   const int t = blockIdx.x;
   f32x4* x4 = (f32x4*)(X + (size_t)t * dim);
   const f32x4* w4 = (const f32x4*)w;
   const int n4 = dim >> 2;
   constexpr int KEEP = 4;  // the row stays in registers between the two passes for dim <= 4096
   f32x4 keep[KEEP];
-  float ss = 0.f;
+  float ss = 0.f, top = 0.f;
   auto load = [&](int k) __attribute__((always_inline)) {
     f32x4 v = x4[k];
     if (kz > 0) {  // the residual GEMM in front split K: its partial rows, in fixed order
@@ -559,22 +650,34 @@ static __global__ __launch_bounds__(KH_WG) void k_pair_rmsnorm(float* __restrict
       }
       x4[k] = v;
     }
+    const f32x4 g = w4[k];
+    ss = fma4(v, v, ss);
+    top = fmaxf(top, pair_top4(f32x4{g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w}));
     return v;
   };
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
     const int k = (int)threadIdx.x + i * KH_WG;
-    if (k < n4) {
-      keep[i] = load(k);
-      ss = fma4(keep[i], keep[i], ss);
-    }
+    if (k < n4) keep[i] = load(k);
   }
-  for (int k = (int)threadIdx.x + KEEP * KH_WG; k < n4; k += KH_WG) {
-    const f32x4 v = load(k);  // (re-read by this same thread below)
-    ss = fma4(v, v, ss);
+  for (int k = (int)threadIdx.x + KEEP * KH_WG; k < n4; k += KH_WG) (void)load(k);  // (re-read by this same thread below)
+  // the row's scale: the largest |g x|, found with the sum of squares
+  ss = wave_sum(ss);
+  for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = ss;
+    tops[threadIdx.x >> 6] = top;
   }
-  ss = block_sum(ss, red);
-  const float rs = 1.0f / sqrtf(ss / (float)dim + eps), s = *scale;
+  __syncthreads();
+  ss = red[0];
+  top = tops[0];
+#pragma unroll
+  for (int i = 1; i < KH_WG / KH_WAVE; ++i) {
+    ss += red[i];
+    top = fmaxf(top, tops[i]);
+  }
+  const float rs = 1.0f / sqrtf(ss / (float)dim + eps), s = pair_scale(rs * top);
+  if (threadIdx.x == 0) inv[t] = pair_inv(s);
   auto emit = [&](int k, const f32x4& v) __attribute__((always_inline)) {
     const f32x4 g = w4[k];
     pair_store4(out + (size_t)t * dim * 4, 4 * k, f32x4{g.x * (rs * v.x), g.y * (rs * v.y), g.z * (rs * v.z), g.w * (rs * v.w)}, s);
@@ -586,23 +689,13 @@ static __global__ __launch_bounds__(KH_WG) void k_pair_rmsnorm(float* __restrict
   }
   for (int k = (int)threadIdx.x + KEEP * KH_WG; k < n4; k += KH_WG) emit(k, x4[k]);
 }
-// rows of pairs and their scales (from the row maximum) from rows of fp32; one workgroup per token
-static __global__ __launch_bounds__(KH_WG) void k_pair_convert(const float* __restrict__ A, char* __restrict__ out, float* __restrict__ xs,
-                                                               int dim) {
-  __shared__ float red[KH_WAVES_MAX];
+// rows of pairs and their scales from rows of fp32; one workgroup per token
+static __global__ __launch_bounds__(KH_WG) void k_pair_convert(const float* __restrict__ A, char* __restrict__ out,
+                                                               unsigned char* __restrict__ exps, int dim, int tcap, int chunks) {
   const int t = blockIdx.x, n4 = dim >> 2;
   const f32x4* a4 = (const f32x4*)(A + (size_t)t * dim);
-  float top = 0.f;
-  for (int k = threadIdx.x; k < n4; k += KH_WG) {
-    const f32x4 v = a4[k];
-    top = fmaxf(top, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+  for (int k0 = 0; k0 < n4; k0 += KH_WG) {
+    const int k = k0 + (int)threadIdx.x;
+    pair_emit(out + (size_t)t * dim * 4, exps, tcap, t, k, n4, chunks, k < n4 ? a4[k] : f4_zero());
   }
-  for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = top;
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < KH_WG / 64; ++i) top = fmaxf(top, red[i]);
-  const float s = pair_scale(top);
-  if (threadIdx.x == 0) xs[t] = s;
-  for (int k = threadIdx.x; k < n4; k += KH_WG) pair_store4(out + (size_t)t * dim * 4, 4 * k, a4[k], s);
 }

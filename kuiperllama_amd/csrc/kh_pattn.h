@@ -34,8 +34,9 @@ struct KhPgAttnArgs {
   const float* kc;  // this layer's K cache rows [cache_len][kv_dim]; rows pos0 .. pos0+T-1 just written
   const float* vc;
   float* out;       // layout 0 / 1: tiled slab [dim x tcap] of an fp32 / int8 model
-                    // (pg_tiled_index, T <= tcap); layout 2: row-major [T][dim]; layout 3: rows of pairs (kh_pair.h)
-  const float* out_s;  // layout 3: their scale
+                    // (pg_tiled_index, T <= tcap); layout 2: row-major [T][dim]; layout 3: rows of pairs (kh_pair.h), heads of multiples of 64
+  unsigned char* out_e;  // layout 3: 1 / their scales, for tcap tokens
+  int stage;        // layout 3: columns of a stage
   int dim, kv_dim, kv_heads, kv_mul, T, pos0, layout, tcap;
 };
 enum { KH_PA_TILED_F32 = 0, KH_PA_TILED_Q8 = 1, KH_PA_ROWS = 2, KH_PA_PAIRS = 3 };
@@ -199,7 +200,9 @@ __global__ __launch_bounds__(64 * NW) void k_pg_attn(const KhPgAttnArgs a) {
       }
     }
     __syncthreads();
-    const int tok = tid & 15;
+    // pairs: the 16 chunks of 64 columns in neighbouring lanes
+    const bool pairs = HS % 64 == 0 && a.layout == KH_PA_PAIRS;
+    const int tok = pairs ? (tid >> 4) & 15 : tid & 15;
     const int t = t0 + 16 * qi + tok;
     if (t < a.T) {
       float M = m_lds[0][tok];
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(64 * NW) void k_pg_attn(const KhPgAttnArgs a) {
         f[w] = __builtin_amdgcn_exp2f(m_lds[w][tok] - M);  // waves without a timestep: m = -inf -> 0
         L += f[w] * l_lds[w][tok];
       }
-      for (int grp = tid >> 4; grp < HS / 4; grp += 4 * NW) {
+      for (int grp = pairs ? (tid >> 8) * 16 + (tid & 15) : tid >> 4; grp < HS / 4; grp += 4 * NW) {
         f32x4 r = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
@@ -220,8 +223,8 @@ __global__ __launch_bounds__(64 * NW) void k_pg_attn(const KhPgAttnArgs a) {
         }
         r.x /= L; r.y /= L; r.z /= L; r.w /= L;
         const int k = h * HS + 4 * grp;
-        if (a.layout == KH_PA_PAIRS) {
-          pair_store4((char*)a.out + (size_t)t * a.dim * 4, k, r, *a.out_s);
+        if (pairs) {
+          pair_emit((char*)a.out + (size_t)t * a.dim * 4, a.out_e, a.tcap, t, k >> 2, a.dim >> 2, a.stage >> 2, r);
           continue;
         }
         const size_t at = a.layout == KH_PA_ROWS ? (size_t)t * a.dim + k

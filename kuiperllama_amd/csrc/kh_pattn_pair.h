@@ -30,9 +30,11 @@ struct KhPaArgs {
   const float* vc;
   char* slab;          // [kv_heads][blocks][KF + VF] fragments of 1 KB
   float* kinv;         // [kv_heads][blocks] 1 / scale of a K block
-  const float* out_s;  // scale of V and of the output
-  char* out;           // rows of pairs [T][dim]
-  int dim, kv_dim, kv_heads, kv_mul, T, pos0, blocks;
+  const float* v_s;    // scale of V
+  float* out;          // heads of 64 and 128: rows of pairs [T][dim], else of fp32
+  unsigned char* out_e;  // 1 / the scales of the pairs, for tcap tokens
+  int stage;           // columns of a stage of the GEMM that reads them
+  int dim, kv_dim, kv_heads, kv_mul, T, pos0, blocks, tcap;
 };
 template <int HS>
 struct PaGeom {
@@ -99,7 +101,7 @@ __global__ __launch_bounds__(256) void k_pa_pack(const KhPaArgs a) {
       *(f16x8*)(dst + ((c * 2 + 1) * 2 + u) * 1024) = lo;
     }
   }
-  const float vs = *a.out_s;
+  const float vs = *a.v_s;
 #pragma unroll
   for (int k = 0; k < VT; ++k) {
     const int dt = wave + 4 * k;
@@ -272,7 +274,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
 #pragma unroll
     for (int d = 0; d < G::ND; ++d) *(f32x4*)&o_lds[wave][li][16 * d + 4 * lj] = o[qi][d];
     __syncthreads();
-    const int tok = tid & 15, t = t0 + 16 * qi + tok;
+    constexpr bool pairs = HS % 64 == 0;  // the 16 chunks of 64 columns in neighbouring lanes
+    const int tok = pairs ? (tid >> 4) & 15 : tid & 15, t = t0 + 16 * qi + tok;
     if (t < a.T) {
       float M = m_lds[0][tok];
 #pragma unroll
@@ -283,8 +286,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
         f[w] = __builtin_amdgcn_exp2f(m_lds[w][tok] - M);
         L += f[w] * l_lds[w][tok];
       }
-      L *= 16384.f;
-      for (int grp = tid >> 4; grp < HS / 4; grp += 4 * NW) {
+      L *= 16384.f * *a.v_s;
+      for (int grp = pairs ? (tid >> 8) * 16 + (tid & 15) : tid >> 4; grp < HS / 4; grp += 4 * NW) {
         f32x4 r = zero4;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
@@ -294,7 +297,9 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] /= L;
-        pair_store4(a.out + (size_t)t * a.dim * 4, h * HS + 4 * grp, r, 1.0f);
+        const int k = h * HS + 4 * grp;
+        if constexpr (pairs) pair_emit((char*)a.out + (size_t)t * a.dim * 4, a.out_e, a.tcap, t, k >> 2, a.dim >> 2, a.stage >> 2, r);
+        else *(f32x4*)(a.out + (size_t)t * a.dim + k) = r;
       }
     }
   }
