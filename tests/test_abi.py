@@ -121,3 +121,22 @@ def test_debug_hooks_live_in_one_table_not_in_getenv(lib, monkeypatch):
     csrc = os.path.join(ROOT, "kuiperllama_amd", "csrc")
     for f in os.listdir(csrc):
         assert "getenv" not in open(os.path.join(csrc, f)).read(), f
+
+
+def test_every_hook_of_the_sources_is_mirrored_from_the_environment(lib, monkeypatch):
+    """A hook whose prefix the mirror does not know is set in os.environ and never reaches the library."""
+    csrc = os.path.join(ROOT, "kuiperllama_amd", "csrc")
+    hooks = set()
+    for f in os.listdir(csrc):
+        if f.endswith((".h", ".hip", ".cpp")):
+            with open(os.path.join(csrc, f)) as src:
+                hooks.update(re.findall(r'"(KH_[A-Z0-9]+_[A-Z0-9_]*[A-Z0-9]|KH_[A-Z0-9]+)"', src.read()))
+    assert {"KH_PAIR_SHAPE", "KH_PAIR_ATTN", "KH_PG_PAIR", "KH_RING", "KH_HY_ROWS"} <= hooks
+    for h in sorted(hooks):
+        monkeypatch.setenv(h, "7")
+        _ffi.sync_env()
+        got = _ffi.debug_get(h)
+        monkeypatch.delenv(h)
+        _ffi.sync_env()
+        assert got == "7", h
+        assert _ffi.debug_get(h) is None, h
