@@ -120,13 +120,12 @@ struct kh_model {
   // gated unit one a token and stage
   float* pg_xs = nullptr;
   unsigned char *pg_ae = nullptr, *pg_he = nullptr;
-  // per layer the scale of the value rows, three words unused and the scale of every weight row (fp32), then a word per layer
+  // fp32: the scale of every weight row, layer by layer
   float* pair_ws = nullptr;
   size_t pair_ws_layer = 0;
   bool pair_ready = false;
   char* pa_ws = nullptr;     // K / V of one layer as pairs in fragment order (kh_pattn_pair.h)
   size_t pa_ws_bytes = 0;
-  bool kv_foreign = false;  // cache rows may hold values that this model did not compute (kh_model_write_kv, _get_kv)
   int pg_rows = 0;  // token rows of the slabs above
   bool pf_ready = false, pg_ready = false;  // set when ALL prefill slabs exist (allocation can fail half-way)
   bool pg_launch_failed = false;

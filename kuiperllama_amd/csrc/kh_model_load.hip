@@ -897,7 +897,6 @@ extern "C" int kh_model_get_kv(kh_model* m, float** d_kcache, float** d_vcache) 
   KH_CHECK_HIP(hipSetDevice(m->opts.device));
   const int rc = kv_ensure(m, m->cfg.cache_len);
   if (rc != KH_OK) return rc;
-  m->kv_foreign = true;
   *d_kcache = m->kcache;
   *d_vcache = m->vcache;
   return KH_OK;
@@ -946,7 +945,6 @@ extern "C" int kh_model_write_kv(kh_model* m, int32_t layer, int32_t row0, int32
     const int rc = kv_ensure_impl(m, row0, row0 + nrows, layer);  // only the chunks these rows live in
     if (rc != KH_OK) return rc;
   }
-  m->kv_foreign = true;
   const size_t off = ((size_t)layer * m->cfg.cache_len + row0) * m->cfg.kv_dim;
   const size_t nb = (size_t)nrows * m->cfg.kv_dim * sizeof(float);
   // hipMemcpyDefault: the source may be host memory or memory of this device (unified addressing)

@@ -112,31 +112,24 @@ bool pair_geometry(const kh_config& c) {
 }
 
 int ensure_pair(kh_model* m) {
-  if (m->pair_ready) return KH_OK;
+  if (m->pair_ready || m->cfg.is_quant) return KH_OK;
   const kh_config& c = m->cfg;
   if (m->pair_ws) (void)hipFree(m->pair_ws);
   m->pair_ws = nullptr;
   const size_t rows = 3 * (size_t)c.dim + 2 * (size_t)c.kv_dim + 2 * (size_t)c.hidden_dim;  // wq wk wv wo w1 w3 w2
-  const size_t per = (c.is_quant ? 0 : rows) + 4;
   int rc;
-  if ((rc = dalloc(&m->pair_ws, (per + 1) * c.layer_num)) != KH_OK) return rc;
-  m->pair_ws_layer = per;
-  unsigned* norms = (unsigned*)(m->pair_ws + per * c.layer_num);
-  KH_CHECK_HIP(hipMemsetAsync(norms, 0, sizeof(unsigned) * c.layer_num, m->stream));
+  if ((rc = dalloc(&m->pair_ws, rows * c.layer_num)) != KH_OK) return rc;
+  m->pair_ws_layer = rows;
   for (int l = 0; l < c.layer_num; ++l) {
     const LayerW& W = m->layers[l];
-    unsigned* nm = norms + l;
-    const KhPairMats mats = {{{W.wq, c.dim, c.dim, nullptr, nullptr},
-                              {W.wk, c.kv_dim, c.dim, nullptr, nullptr},
-                              {W.wv, c.kv_dim, c.dim, W.att_norm, nm},
-                              {W.wo, c.dim, c.dim, nullptr, nullptr},
-                              {W.w1, c.hidden_dim, c.dim, nullptr, nullptr},
-                              {W.w3, c.hidden_dim, c.dim, nullptr, nullptr},
-                              {W.w2, c.dim, c.hidden_dim, nullptr, nullptr}}};
-    if (c.is_quant) hipLaunchKernelGGL(k_pair_rows<true>, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, (float*)nullptr, (int)rows);
-    else hipLaunchKernelGGL(k_pair_rows<false>, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, m->pair_ws + per * l + 4, (int)rows);
-    hipLaunchKernelGGL(k_pair_scales, dim3(1), dim3(256), 0, m->stream, W.wv.bias, (const unsigned*)nm, c.dim, c.kv_dim,
-                       m->pair_ws + per * l);
+    const KhPairMats mats = {{{W.wq, c.dim, c.dim},
+                              {W.wk, c.kv_dim, c.dim},
+                              {W.wv, c.kv_dim, c.dim},
+                              {W.wo, c.dim, c.dim},
+                              {W.w1, c.hidden_dim, c.dim},
+                              {W.w3, c.hidden_dim, c.dim},
+                              {W.w2, c.dim, c.hidden_dim}}};
+    hipLaunchKernelGGL(k_pair_rows, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, m->pair_ws + rows * l, (int)rows);
   }
   if ((rc = kh_launch_status()) != KH_OK) return rc;
   m->pair_ready = true;
@@ -150,7 +143,7 @@ void pa_go(const KhPaArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((k_pa_attn<HS, 4, QT>), dim3(a.kv_heads * a.kv_mul * ((a.T + 16 * QT - 1) / (16 * QT))), dim3(256), 0, s, a);
 }
 template <int HS>
-size_t pa_bytes(int heads, int blocks) { return (size_t)heads * blocks * (PaGeom<HS>::FR * 1024 + sizeof(float)); }
+size_t pa_bytes(int heads, int blocks) { return (size_t)heads * blocks * (PaGeom<HS>::FR * 1024 + 2 * sizeof(float)); }
 
 // Attention of a slice with its operands as pairs; false: the caller takes pg_slice_attention (fp32 matrix cores).
 // Packing reads all of the layer's rows whatever T is, so it needs enough query tokens and enough work.  Whole prompt
@@ -158,9 +151,9 @@ size_t pa_bytes(int heads, int blocks) { return (size_t)heads * blocks * (PaGeom
 // 512 @ 0 4.05 / 3.94, 64 @ 2048 2.05 / 2.05, 256 @ 2048 3.42 / 3.06, 2048 @ 2048 20.3 / 14.6; Llama-2-7B int8
 // 128 @ 0 7.07 / 7.13, 256 @ 0 10.5 / 10.3, 128 @ 1024 8.08 / 7.83, 1024 @ 1024 41.5 / 34.5.
 // The slab of a layer is given up (not the call) above KH_PA_WS_MAX and where memory for it is refused.
-bool pair_attention(kh_model* m, int l, int T, int pos0, const float* v_s) {
+bool pair_attention(kh_model* m, int l, int T, int pos0) {
   const kh_config& c = m->cfg;
-  if (m->kv_foreign || dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
+  if (dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
   if (T < 128 || (size_t)T * (2 * (size_t)pos0 + T) < 65536) return false;
   KhPaArgs a{};
   a.blocks = (pos0 + T + 31) / 32;
@@ -186,8 +179,7 @@ bool pair_attention(kh_model* m, int l, int T, int pos0, const float* v_s) {
   a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
   a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
   a.slab = m->pa_ws;
-  a.kinv = (float*)(m->pa_ws + need - (size_t)c.kv_head_num * a.blocks * sizeof(float));
-  a.v_s = v_s;
+  a.inv = (float*)(m->pa_ws + need - 2 * (size_t)c.kv_head_num * a.blocks * sizeof(float));
   a.out = m->pg_att;
   a.out_e = m->pg_ae;
   a.stage = KH_PAIR_STAGE(c.is_quant);
@@ -213,8 +205,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
   const bool rope_fuse = !dbg_off("KH_PG_ROPE_FUSE");
   for (int l = 0; l < c.layer_num; ++l) {
     const LayerW& W = m->layers[l];
-    const float* sc = m->pair_ws + m->pair_ws_layer * l;
-    const float* ws = sc + 4;  // row scales: wq, wk, wv, wo, w1, w3, w2
+    const float* ws = m->pair_ws + m->pair_ws_layer * l;  // row scales: wq, wk, wv, wo, w1, w3, w2
     const float* ws_o = ws + c.dim + 2 * c.kv_dim;
     const float* ws_1 = ws_o + c.dim;
     auto rmsnorm = [&](const float* w) {
@@ -251,7 +242,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     if (l == c.layer_num - 1) break;
     // the attention kernels leave pairs where 64 columns are of one head
     bool pairs = c.head_size % 64 == 0;
-    if (!pair_attention(m, l, T, pos0, sc)) pairs = pg_slice_attention(m, l, T, pos0, pairs ? KH_PA_PAIRS : KH_PA_ROWS, m->pg_rows);
+    if (!pair_attention(m, l, T, pos0)) pairs = pg_slice_attention(m, l, T, pos0, pairs ? KH_PA_PAIRS : KH_PA_ROWS, m->pg_rows);
     if (!pairs) hipLaunchKernelGGL(k_pair_convert, dim3(T), dim3(KH_WG), 0, m->stream, (const float*)m->pg_att, xn, m->pg_ae, c.dim, m->pg_rows,
                                    KH_PAIR_STAGE(c.is_quant) / 4);
     {

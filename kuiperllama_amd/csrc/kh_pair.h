@@ -15,9 +15,7 @@
 // gated unit have one per token and 64 columns, found where they are made (passes of few tokens: 32, see kPairTiles): a few
 // columns may be far above the others there, and a bound from the weights would have to hold for all of them (one row each
 // of w1 and w3 at 2^12 of its usual size, undone by w2: K/V rows 2.5e-2 from 64 bits instead of 4e-7).  Every weight row
-// has a scale, and the value rows have the bound |v| <= max_j |wv_j * g| sqrt(dim) + max|bias|, which k_pair_rows and
-// k_pair_scales compute once per model.  Once a caller has had its hands on the cache (kh_model_write_kv,
-// kh_model_get_kv) that bound does not hold and the attention keeps kh_pattn.h.
+// of fp32 has a scale, which k_pair_rows finds once per model.
 //
 // Kernel: the stage ring of kh_lgemm.h.  A workgroup owns BM tokens x BN weight rows; a stage of 32 (int8: 64) columns
 // is moved to LDS by global_load_lds_dwordx4 in 128-byte rows (pairs: 32 hi | 32 lo; fp32 weights as they lie in the
@@ -84,6 +82,9 @@ __device__ __forceinline__ void pair_store4(char* row, int k, const f32x4& v, fl
   }
   *(f16x4*)(row + pair_at(k)) = hi;
   *(f16x4*)(row + pair_at(k) + 64) = lo;
+}
+__device__ __forceinline__ float pair_top4(const f32x4& v) {
+  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 // power of two that brings `bound` to less than 2^KH_PAIR_TOP (1 for 0, the smallest one for infinities and NaN)
 __device__ __forceinline__ float pair_scale(float bound) {
@@ -551,73 +552,24 @@ struct KhPairMats {  // the matrices of a layer
   struct {
     KhLin w;
     int rows, K;
-    const float* g;   // norm weights in front of it (wv)
-    unsigned* norm;
   } m[7];
 };
-// One wave per row of the stacked matrices: fp32 weights get the row's scale; with norm weights g the largest |w_row * g|
-// of the matrix goes to *norm (its bits: the values are positive).  16 bytes a lane; K is a multiple of 32 (int8: 64).
-// Every row's atomicMax on one word took longer than the reading, so only a larger norm sends one.
-template <bool Q>
-__global__ __launch_bounds__(256) void k_pair_rows(const KhPairMats a, float* ws, int total) {
+// One wave per row of the stacked matrices, 16 bytes a lane; K is a multiple of 32.
+static __global__ __launch_bounds__(256) void k_pair_rows(const KhPairMats a, float* ws, int total) {
   const int at = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (at >= total) return;
   int row = at, i = 0;
   while (i < 6 && row >= a.m[i].rows) row -= a.m[i++].rows;
-  const KhLin w = a.m[i].w;
   const int K = a.m[i].K;
-  const float* g = a.m[i].g;
-  unsigned* norm = a.m[i].norm;
-  if (Q && !g) return;
-  float top = 0.f, sum = 0.f;
-  auto add4 = [&](f32x4 v, int k) __attribute__((always_inline)) {
-    top = fmaxf(fmaxf(top, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
-    if (g) {
-      const f32x4 y = *(const f32x4*)(g + k);
-      v = f32x4{v.x * y.x, v.y * y.y, v.z * y.z, v.w * y.w};
-      sum = fma4(v, v, sum);
-    }
-  };
-  if constexpr (Q) {
-    for (int k = 16 * lane; k < K; k += 1024) {
-      const i32x4 q = ld_nt((const i32x4*)((const int8_t*)w.w + (size_t)row * K + k));
-      const float s = w.scales[(size_t)row * (K >> 6) + (k >> 6)];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        add4(f32x4{s * (float)(int8_t)q[i], s * (float)(int8_t)(q[i] >> 8), s * (float)(int8_t)(q[i] >> 16), s * (float)(q[i] >> 24)},
-             k + 4 * i);
-    }
-  } else {
+  const float* w = (const float*)a.m[i].w.w + (size_t)row * K;
+  float top = 0.f;
 #pragma unroll 4
-    for (int k = 4 * lane; k < K; k += 256) add4(ld_nt((const f32x4*)((const float*)w.w + (size_t)row * K + k)), k);
-  }
-  for (int o = 32; o; o >>= 1) {
-    top = fmaxf(top, __shfl_xor(top, o));
-    sum += __shfl_xor(sum, o);
-  }
-  if (lane == 0) {
-    if (!Q) ws[at] = pair_scale(top);
-    const unsigned len = __float_as_uint(sqrtf(sum));
-    if (norm && len > __hip_atomic_load(norm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(norm, len);
-  }
-}
-// out: scale of the value rows.  norm: of wv; bv: its bias or null
-static __global__ __launch_bounds__(256) void k_pair_scales(const float* bv, const unsigned* norm, int dim, int kv_dim, float* out) {
-  __shared__ float red[4];
-  float m = 0.f;
-  if (bv)
-    for (int k = threadIdx.x; k < kv_dim; k += 256) m = fmaxf(m, fabsf(bv[k]));
-  for (int o = 32; o; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0)  // |x| / rms(x) is at most sqrt(dim)
-    out[0] = pair_scale(__uint_as_float(norm[0]) * sqrtf((float)dim) + fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+  for (int k = 4 * lane; k < K; k += 256) top = fmaxf(top, pair_top4(ld_nt((const f32x4*)(w + k))));
+  for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+  if (lane == 0) ws[at] = pair_scale(top);
 }
 
 // ---- the per-token kernels between the GEMMs ------------------------------------------------------------------------
-__device__ __forceinline__ float pair_top4(const f32x4& v) {
-  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-}
 // Chunk k (four columns) of token t with a scale per 64 columns, whose chunks lie in 16 neighbouring lanes; chunks from n4 on
 // are zeros.  chunks: those of a stage (8 or 16), every stage gets the scale.
 __device__ __forceinline__ void pair_emit(char* row, unsigned char* exps, int ld, int t, int k, int n4, int chunks, const f32x4& v) {

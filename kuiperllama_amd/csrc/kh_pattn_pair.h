@@ -2,9 +2,9 @@
 // of halves (kh_pair.h; reference: cpu/mha_kernel.cpp:5-61, cuda/mha_kernel.cu:47-110, one query token at a time).
 //
 // k_pa_pack first lays this layer's K and V rows 0 .. pos0 + T - 1 out as pairs in the order of the MFMA fragments: blocks
-// of 32 positions, every fragment 64 lanes x 16 bytes, so that the attention reads nothing but whole kilobytes.  K blocks
-// carry a scale of their own (the largest number of the block), V the static bound of kh_pair.h, which is also the scale of
-// the output: a cache that a caller has written to has no such bound and keeps kh_pattn.h.
+// of 32 positions, every fragment 64 lanes x 16 bytes, so that the attention reads nothing but whole kilobytes.  The K and
+// the V part of a block carry a scale each, from the largest finite number in it (a row that is not finite must not take the
+// bits of the positions in front of it).  Nothing is kept from one pass to the next and nothing is assumed of the cache.
 //
 // k_pa_attn: one workgroup owns (head, QT x 16 query tokens), its NW waves split the 32-position blocks:
 //   S^T[pos, tok] = K . Q^T         rows of the two 16-row tiles u are positions 8 (i >> 2) + 4 u + (i & 3), so that a lane
@@ -12,7 +12,8 @@
 //   O^T[d, tok]  += V^T . P^T       the B operand of v_mfma_f32_16x16x32_f16 as it stands
 // Products lo hi, hi lo, hi hi in this order, so the sum is rounded at its full size only in the last ones.  Online softmax
 // in the log2 domain as in kh_pattn.h.  The matrix core rounds sums down, which would not average out over thousands of
-// positions: a block's P V starts from zero, is added to O in fp32, and every second block of a wave carries -P.
+// positions: a block's P V starts from zero, is added to O in fp32 (times 1 / the block's scale), and every second block of a
+// wave carries -P.
 //
 // Q is split once per workgroup and kept in LDS; K and V of the next block are requested when the last product of the
 // present one has read them: held twice they would not leave room for two waves per SIMD, which cover one another's softmax.
@@ -29,8 +30,7 @@ struct KhPaArgs {
   const float* kc;     // this layer's cache rows [cache_len][kv_dim]
   const float* vc;
   char* slab;          // [kv_heads][blocks][KF + VF] fragments of 1 KB
-  float* kinv;         // [kv_heads][blocks] 1 / scale of a K block
-  const float* v_s;    // scale of V
+  float* inv;          // [kv_heads][blocks] 1 / scale of K, of V
   float* out;          // heads of 64 and 128: rows of pairs [T][dim], else of fp32
   unsigned char* out_e;  // 1 / the scales of the pairs, for tcap tokens
   int stage;           // columns of a stage of the GEMM that reads them
@@ -51,16 +51,18 @@ __device__ __forceinline__ void pa_split(const float (&v)[8], float s, f16x8& hi
   }
 }
 
+// |v|, zero for infinities and NaN
+__device__ __forceinline__ float pa_finite(float v) { return fabsf(v) < INFINITY ? fabsf(v) : 0.f; }
 // one workgroup of four waves per (block of 32 positions, kv head); positions past the slice become zeros
 template <int HS>
 __global__ __launch_bounds__(256) void k_pa_pack(const KhPaArgs a) {
   using G = PaGeom<HS>;
   constexpr int KT = (2 * G::NC + 3) / 4, VT = (G::ND + 3) / 4;
-  __shared__ float top_lds[4];
+  __shared__ float top_lds[2][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lj = lane >> 4;
   const int blk = blockIdx.x, g = blockIdx.y, p0 = blk * 32, n = a.pos0 + a.T;
   char* dst = a.slab + ((size_t)g * a.blocks + blk) * G::FR * 1024 + lane * 16;
-  float kv[KT][8], vv[VT][8], top = 0.f;
+  float kv[KT][8], vv[VT][8], top = 0.f, vtop = 0.f;
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
     const int task = wave + 4 * k, u = task & 1, d = (task >> 1) * 32 + 8 * lj;
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(256) void k_pa_pack(const KhPaArgs a) {
     for (int e = 0; e < 4; ++e) {
       kv[k][e] = in ? x[e] : 0.f;
       kv[k][e + 4] = in ? y[e] : 0.f;
-      top = fmaxf(top, fmaxf(fabsf(kv[k][e]), fabsf(kv[k][e + 4])));
+      top = fmaxf(top, fmaxf(pa_finite(kv[k][e]), pa_finite(kv[k][e + 4])));
     }
   }
 #pragma unroll
@@ -84,13 +86,21 @@ __global__ __launch_bounds__(256) void k_pa_pack(const KhPaArgs a) {
       const bool in = p < n && d < HS;
       const float x = a.vc[(size_t)(in ? p : 0) * a.kv_dim + g * HS + (in ? d : 0)];
       vv[k][e] = in ? x : 0.f;
+      vtop = fmaxf(vtop, pa_finite(vv[k][e]));
     }
   }
-  for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
-  if (lane == 0) top_lds[wave] = top;
+  for (int o = 32; o; o >>= 1) {
+    top = fmaxf(top, __shfl_xor(top, o));
+    vtop = fmaxf(vtop, __shfl_xor(vtop, o));
+  }
+  if (lane == 0) {
+    top_lds[0][wave] = top;
+    top_lds[1][wave] = vtop;
+  }
   __syncthreads();
-  const float s = pair_scale(fmaxf(fmaxf(top_lds[0], top_lds[1]), fmaxf(top_lds[2], top_lds[3])));
-  if (threadIdx.x == 0) a.kinv[(size_t)g * a.blocks + blk] = pair_inv(s);
+  auto scale = [&](const float(&t)[4]) { return pair_scale(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]))); };
+  const float s = scale(top_lds[0]), vs = scale(top_lds[1]);
+  if (threadIdx.x == 0) *(float2*)(a.inv + 2 * ((size_t)g * a.blocks + blk)) = make_float2(pair_inv(s), pair_inv(vs));
   f16x8 hi, lo;
 #pragma unroll
   for (int k = 0; k < KT; ++k) {
@@ -101,7 +111,6 @@ __global__ __launch_bounds__(256) void k_pa_pack(const KhPaArgs a) {
       *(f16x8*)(dst + ((c * 2 + 1) * 2 + u) * 1024) = lo;
     }
   }
-  const float vs = *a.v_s;
 #pragma unroll
   for (int k = 0; k < VT; ++k) {
     const int dt = wave + 4 * k;
@@ -131,20 +140,21 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
   const int n_pb = ((a.pos0 + t_last) >> 5) + 1;
   const char* base = a.slab + (size_t)g * a.blocks * G::FR * 1024;  // uniform: fragments are read at scalar base + lane
   const unsigned lane16 = lane * 16;
-  const float* kinv = a.kinv + (size_t)g * a.blocks;
+  const float* inv = a.inv + 2 * (size_t)g * a.blocks;
 
   f16x8 kf[G::KF], vf[G::VF];
-  float ki = 1.f;
+  float ki = 1.f, vi = 1.f;
   auto load_k = [&](int pb) __attribute__((always_inline)) {
     const char* s = base + (size_t)pb * G::FR * 1024;
 #pragma unroll
     for (int i = 0; i < G::KF; ++i) kf[i] = *(const f16x8*)(s + i * 1024 + lane16);
-    ki = kinv[pb];
+    ki = inv[2 * pb];
   };
   auto load_v = [&](int pb) __attribute__((always_inline)) {
     const char* s = base + ((size_t)pb * G::FR + G::KF) * 1024;
 #pragma unroll
     for (int i = 0; i < G::VF; ++i) vf[i] = *(const f16x8*)(s + i * 1024 + lane16);
+    vi = inv[2 * pb + 1] * 0x1p-14f;  // P is scaled by 2^14
   };
   if (wave < n_pb) {
     load_k(wave);
@@ -195,7 +205,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
   auto block = [&](int pb, auto odd) __attribute__((always_inline)) {
     constexpr float PS = decltype(odd)::value ? -16384.f : 16384.f;  // p <= 1
     const int next = pb + NW;
-    const float ki0 = ki;
+    const float ki0 = ki, vi0 = decltype(odd)::value ? -vi : vi;
 #pragma unroll
     for (int qi = 0; qi < QT; ++qi) {
       const int first = a.pos0 + t0 + 16 * qi;        // position of the tile's first token
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
         t = mfma_pair(vf[2 * d], pl, t);
         t = mfma_pair(vf[2 * d], ph, t);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[qi][d][r] = __builtin_fmaf(o[qi][d][r], alpha, decltype(odd)::value ? -t[r] : t[r]);
+        for (int r = 0; r < 4; ++r) o[qi][d][r] = __builtin_fmaf(t[r], vi0, o[qi][d][r] * alpha);
       }
     }
     if (next < n_pb) load_v(next);
@@ -286,7 +296,6 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
         f[w] = __builtin_amdgcn_exp2f(m_lds[w][tok] - M);
         L += f[w] * l_lds[w][tok];
       }
-      L *= 16384.f * *a.v_s;
       for (int grp = pairs ? (tid >> 8) * 16 + (tid & 15) : tid >> 4; grp < HS / 4; grp += 4 * NW) {
         f32x4 r = zero4;
 #pragma unroll

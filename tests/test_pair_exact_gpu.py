@@ -46,18 +46,28 @@ def _norms(t, l, spec, f):  # one weight of either norm
             _scale(t, f"{k}.{l}", 70, 1 / f, 1)
 
 
-def errors(monkeypatch, img, spec, n, hook="KH_PG_PAIR", pos=0):
-    """Error of the rows of the layers behind the first: with pairs, and with `hook` off."""
+def _values(t, l, spec, f):  # one value column of a head
+    g, d = spec.n_kv_heads - 1, 3
+    _scale(t, f"wv.{l}", g * spec.head_size + d, f, 0)
+    for h in range(g * spec.kv_mul, (g + 1) * spec.kv_mul):
+        _scale(t, f"wo.{l}", h * spec.head_size + d, 1 / f, 1)
+
+
+def errors(monkeypatch, img, spec, n, hook="KH_PG_PAIR", front=None):
+    """Error of the rows of the layers behind the first: with pairs, and with `hook` off.  front: cache rows before them."""
     from kuiperllama_amd.model import KuiperModel
     toks = [int(t) for t in np.random.default_rng(17).integers(0, spec.vocab_size, n)]
-    want = exact_kv.rows(img, spec, toks)
+    want = exact_kv.rows(img, spec, toks, front)
+    old = 0 if front is None else len(front[0][0])
     out = []
     for off in (False, True):
         if off:
             monkeypatch.setenv(hook, "0")
         m = KuiperModel.from_device_image(img, spec)
-        m.prefill_gemm(toks, 0)
-        got = [m.read_kv(l, 0, n) for l in range(1, spec.n_layers)]
+        for l in range(spec.n_layers if old else 0):
+            m.write_kv(l, 0, *front[l])
+        m.prefill_gemm(toks, old)
+        got = [m.read_kv(l, old, n) for l in range(1, spec.n_layers)]
         out.append(max(exact_kv.error(g, w) for a, b in zip(got, want[1:]) for g, w in zip(a, b)))
         m.close()
         monkeypatch.delenv(hook, raising=False)
@@ -77,3 +87,50 @@ def test_sizes_that_cancel(gpu, name, change, e, n, monkeypatch):
     pair, fp32 = errors(monkeypatch, img, spec, n)
     print(f"{name} {change.__name__} 2^{e}, {n} tokens: {pair:.3g} with pairs, {fp32:.3g} without")
     assert pair <= 1.25 * fp32  # a quarter for the luck of the roundings
+
+
+@pytest.mark.parametrize("name", ["gqa-half", "mha-interleaved", "gqa-half-hs128", "int8"])
+@pytest.mark.parametrize("e", [0, 6, 12, 15])
+def test_value_columns_that_cancel(gpu, name, e, monkeypatch):
+    """Attention of a slice on pairs (csrc/kh_pattn_pair.h) against the fp32 matrix cores."""
+    spec = _PF_SPECS[name]
+    img = binfmt.synth_image(spec, seed=52, device=gpu)
+    t = exact_kv.tensors(img, spec)
+    for l in range(spec.n_layers):
+        _values(t, l, spec, 2.0 ** e)
+    pair, fp32 = errors(monkeypatch, img, spec, 300, "KH_PAIR_ATTN")
+    print(f"{name} values 2^{e}: {pair:.3g} with pairs, {fp32:.3g} without")
+    assert pair <= 1.25 * fp32
+
+
+@pytest.mark.parametrize("name", ["gqa-half", "gqa-half-hs128"])
+def test_rows_of_the_caller_in_front(gpu, name, monkeypatch):
+    """Cache rows that the model cannot have computed: values of 1e4, keys a thousandth of the usual ones."""
+    spec = _PF_SPECS[name]
+    img = binfmt.synth_image(spec, seed=53, device=gpu)
+    rng = np.random.default_rng(18)
+    draw = lambda size: (size * rng.standard_normal((70, spec.kv_dim))).astype(np.float32)
+    front = [(draw(1e-3), draw(1e4)) for _ in range(spec.n_layers)]
+    pair, fp32 = errors(monkeypatch, img, spec, 250, "KH_PAIR_ATTN", front)
+    print(f"{name} rows in front: {pair:.3g} with pairs, {fp32:.3g} without")
+    assert pair <= 1.25 * fp32
+
+
+def test_rows_handed_back_change_nothing(gpu):
+    """A caller that reads rows and writes them back gets the same rows behind them: the pass does not depend on who wrote
+    the cache."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = _PF_SPECS["gqa-half"]
+    img = binfmt.synth_image(spec, seed=54, device=gpu)
+    toks = [int(t) for t in np.random.default_rng(19).integers(0, spec.vocab_size, 400)]
+    out = []
+    for back in (False, True):
+        m = KuiperModel.from_device_image(img, spec)
+        m.prefill_gemm(toks[:100], 0)
+        for l in range(spec.n_layers if back else 0):
+            m.write_kv(l, 0, *m.read_kv(l, 0, 100))
+        m.prefill_gemm(toks[100:], 100)
+        out.append([m.read_kv(l, 100, 300) for l in range(spec.n_layers)])
+        m.close()
+    for a, b in zip(*out):
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
