@@ -328,9 +328,11 @@ int kh_model_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t po
  * weights (never more than the cache holds; a longer prompt is cut into such passes plus a remainder; env KH_PG_CHUNK =
  * 16..512 sets another pass size).  Activations and fp32 weights travel as pairs of halves that keep fp32 accuracy, int8
  * weights are exact in one (csrc/kh_pair.h; the K/V rows are closer to their 64-bit values than those of an fp32 fmaf
- * chain).  The first call of a model computes a scale per weight row; the weights must not change afterwards.  Widths
+ * chain as long as the numbers that share a scale - a normed row, 64 columns of the gated unit or of an attention output,
+ * 32 cached rows of a head, a weight row - are within about 2^12 of one another where they weigh alike in a result).  Widths
  * that are no multiple of 32 - and hook KH_PG_PAIR=0 - take fp32-MFMA GEMMs instead (csrc/kh_gemm.h: v_mfma_f32_16x16x4_f32,
- * passes of up to 512 tokens, int8 weights dequantised per element in registers).  The K/V rows agree
+ * passes of up to 512 tokens, int8 weights dequantised per element in registers).  Either way nothing about the weights is
+ * kept between calls: memory given to kh_model_create_from_device_weights may be written between them.  The K/V rows agree
  * with the token-by-token path to fp32 round-off (different summation order), not bit for bit.
  * kh_model_generate* use it for prompts with >= 16 fed-only tokens unless the model was created with
  * KH_FLAG_PREFILL_EXACT - so for such prompts the greedy tokens carry this tolerance too and can differ from the

@@ -120,10 +120,6 @@ struct kh_model {
   // gated unit one a token and stage
   float* pg_xs = nullptr;
   unsigned char *pg_ae = nullptr, *pg_he = nullptr;
-  // fp32: the scale of every weight row, layer by layer
-  float* pair_ws = nullptr;
-  size_t pair_ws_layer = 0;
-  bool pair_ready = false;
   char* pa_ws = nullptr;     // K / V of one layer as pairs in fragment order (kh_pattn_pair.h)
   size_t pa_ws_bytes = 0;
   int pg_rows = 0;  // token rows of the slabs above
@@ -227,6 +223,5 @@ bool pg_supported(const kh_model* m);       // MFMA GEMM path
 bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int layout, int tcap);
 // pair GEMMs (kh_model_pair.hip)
 bool pair_geometry(const kh_config& c);
-int ensure_pair(kh_model* m);  // scales of the weights, once
 int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0);
 }  // namespace khm

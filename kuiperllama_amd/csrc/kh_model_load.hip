@@ -664,7 +664,7 @@ extern "C" void kh_model_destroy(kh_model* m) {
   for (void* q : {(void*)m->pf_x, (void*)m->pf_q, (void*)m->pf_att, (void*)m->pf_h, m->pf_ws,
                   (void*)m->pg_x, (void*)m->pg_xn, (void*)m->pg_q, (void*)m->pg_att, (void*)m->pg_h, (void*)m->pg_part, (void*)m->pg_xs, (void*)m->pg_ae,
                   (void*)m->pg_he,
-                  m->pg_ws, (void*)m->pair_ws, (void*)m->pa_ws})
+                  m->pg_ws, (void*)m->pa_ws})
     if (q) (void)hipFree(q);
   for (auto e : m->ev_chunk)
     if (e) (void)hipEventDestroy(e);

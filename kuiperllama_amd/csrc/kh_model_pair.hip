@@ -1,6 +1,5 @@
-// kh_model_pair.hip — prompt passes of .bin models on the pair GEMMs (kh_pair.h): scales once per model, launch shapes,
-// one pass of up to KH_PAIR_TMAX prompt tokens.  The reference feeds the prompt one token per forward pass
-// (demo/main.cpp:20-22).  gfx950 only.
+// kh_model_pair.hip — prompt passes of .bin models on the pair GEMMs (kh_pair.h): launch shapes, one pass of up to
+// KH_PAIR_TMAX prompt tokens.  The reference feeds the prompt one token per forward pass (demo/main.cpp:20-22).  gfx950 only.
 #include <stdio.h>
 #include <stdlib.h>
 
@@ -111,31 +110,6 @@ bool pair_geometry(const kh_config& c) {
   return c.dim % g == 0 && c.hidden_dim % g == 0;
 }
 
-int ensure_pair(kh_model* m) {
-  if (m->pair_ready || m->cfg.is_quant) return KH_OK;
-  const kh_config& c = m->cfg;
-  if (m->pair_ws) (void)hipFree(m->pair_ws);
-  m->pair_ws = nullptr;
-  const size_t rows = 3 * (size_t)c.dim + 2 * (size_t)c.kv_dim + 2 * (size_t)c.hidden_dim;  // wq wk wv wo w1 w3 w2
-  int rc;
-  if ((rc = dalloc(&m->pair_ws, rows * c.layer_num)) != KH_OK) return rc;
-  m->pair_ws_layer = rows;
-  for (int l = 0; l < c.layer_num; ++l) {
-    const LayerW& W = m->layers[l];
-    const KhPairMats mats = {{{W.wq, c.dim, c.dim},
-                              {W.wk, c.kv_dim, c.dim},
-                              {W.wv, c.kv_dim, c.dim},
-                              {W.wo, c.dim, c.dim},
-                              {W.w1, c.hidden_dim, c.dim},
-                              {W.w3, c.hidden_dim, c.dim},
-                              {W.w2, c.dim, c.hidden_dim}}};
-    hipLaunchKernelGGL(k_pair_rows, dim3((rows + 3) / 4), dim3(256), 0, m->stream, mats, m->pair_ws + rows * l, (int)rows);
-  }
-  if ((rc = kh_launch_status()) != KH_OK) return rc;
-  m->pair_ready = true;
-  return KH_OK;
-}
-
 namespace {
 template <int HS, int QT>
 void pa_go(const KhPaArgs& a, hipStream_t s) {
@@ -205,9 +179,6 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
   const bool rope_fuse = !dbg_off("KH_PG_ROPE_FUSE");
   for (int l = 0; l < c.layer_num; ++l) {
     const LayerW& W = m->layers[l];
-    const float* ws = m->pair_ws + m->pair_ws_layer * l;  // row scales: wq, wk, wv, wo, w1, w3, w2
-    const float* ws_o = ws + c.dim + 2 * c.kv_dim;
-    const float* ws_1 = ws_o + c.dim;
     auto rmsnorm = [&](const float* w) {
       hipLaunchKernelGGL(k_pair_rmsnorm, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_x, w, xn, m->pg_xs, c.dim, c.rms_eps, m->pg_rows,
                          (const float*)m->pg_part, kz);
@@ -226,7 +197,6 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     {
       KhPairArgs a = base;
       a.w[0] = W.wq; a.w[1] = W.wk; a.w[2] = W.wv;
-      a.ws[0] = ws; a.ws[1] = ws + c.dim; a.ws[2] = ws + c.dim + c.kv_dim;
       a.X = xn; a.out = m->pg_q;
       a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
       a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
@@ -247,7 +217,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
                                    KH_PAIR_STAGE(c.is_quant) / 4);
     {
       KhPairArgs a = base;
-      a.w[0] = W.wo; a.ws[0] = ws_o;
+      a.w[0] = W.wo;
       a.X = pairs ? (const char*)m->pg_att : xn; a.xe = m->pg_ae; a.out = m->pg_x;
       a.rows0 = a.N = a.ldo = a.K = c.dim;
       if ((rc = pair_launch<KH_PG_RESID>(m, a, &kz)) != KH_OK) return rc;
@@ -256,14 +226,13 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     {
       KhPairArgs a = base;
       a.w[0] = W.w1; a.w[1] = W.w3;
-      a.ws[0] = ws_1; a.ws[1] = ws_1 + c.hidden_dim;
       a.X = xn; a.pairs = h; a.out_e = m->pg_he;
       a.rows0 = c.hidden_dim; a.N = 2 * c.hidden_dim; a.ldo = c.hidden_dim; a.K = c.dim;
       if ((rc = pair_launch<KH_PG_SWIGLU>(m, a, nullptr, &fine)) != KH_OK) return rc;
     }
     {
       KhPairArgs a = base;
-      a.w[0] = W.w2; a.ws[0] = ws_1 + 2 * c.hidden_dim;
+      a.w[0] = W.w2;
       a.X = h; a.xe = m->pg_he; a.fine = fine; a.out = m->pg_x;
       a.rows0 = a.N = a.ldo = c.dim; a.K = c.hidden_dim;
       if ((rc = pair_launch<KH_PG_RESID>(m, a, &kz)) != KH_OK) return rc;

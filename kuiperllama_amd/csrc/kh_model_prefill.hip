@@ -578,7 +578,6 @@ extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32
   m->pg_launch_failed = false;
   // KH_PG_PAIR=0 and the shape hooks of k_pg_gemm select the fp32-MFMA GEMMs
   const bool pair = pair_geometry(c) && !dbg_off("KH_PG_PAIR") && !dbg("KH_PG_SHAPE_QKV") && !dbg("KH_PG_SHAPE_RESID") && !dbg("KH_PG_SHAPE_SWIGLU");
-  if (pair && (rc = ensure_pair(m)) != KH_OK) return rc;
   // tuning / test hook: KH_PG_CHUNK=<tokens per weight pass> (16 .. KH_PG_TMAX), read per call
   int chunk = pair && pg_mfma_attn(m) ? m->pg_rows : KH_PG_TMAX;
   if (const char* e = dbg("KH_PG_CHUNK")) {

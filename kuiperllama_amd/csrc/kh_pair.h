@@ -14,8 +14,11 @@
 // smaller ones have an error of 2^-39 of it.  Normed rows have one per token (k_pair_rmsnorm).  Attention outputs and the
 // gated unit have one per token and 64 columns, found where they are made (passes of few tokens: 32, see kPairTiles): a few
 // columns may be far above the others there, and a bound from the weights would have to hold for all of them (one row each
-// of w1 and w3 at 2^12 of its usual size, undone by w2: K/V rows 2.5e-2 from 64 bits instead of 4e-7).  Every weight row
-// of fp32 has a scale, which k_pair_rows finds once per model.
+// of w1 and w3 at 2^12 of its usual size, undone by w2: K/V rows 2.5e-2 from 64 bits instead of 4e-7).  A row of fp32 weights
+// has one in every workgroup that reads it, from its first 32 columns, which it brings to [2^9, 2^10).  Where a number
+// behind them is too large for a half (2^6 times as large at least), the sums are no longer finite, and the wave starts
+// again with scales from all columns; a row that begins with zeros is read through at once.  (Following the largest number
+// in the loop instead made w1 + w3 of Llama-3.2-1B 5 % slower at 512 tokens.)  Nothing is kept from one pass to the next: weights may be written between two calls.
 //
 // Kernel: the stage ring of kh_lgemm.h.  A workgroup owns BM tokens x BN weight rows; a stage of 32 (int8: 64) columns
 // is moved to LDS by global_load_lds_dwordx4 in 128-byte rows (pairs: 32 hi | 32 lo; fp32 weights as they lie in the
@@ -43,7 +46,6 @@ __device__ __forceinline__ int pair_swz(int r) { return ((r & 2) << 1) | ((r & 4
 
 struct KhPairArgs {
   KhLin w[3];          // QKV: wq, wk, wv; RESID: w[0]; SWIGLU: w1, w3
-  const float* ws[3];  // fp32 weights: the scale of every row
   const char* X;       // pair slab: [T][K / 32][32 hi | 32 lo]
   const float* xs;     // QKV, SWIGLU: 1 / its scales, one per token
   const unsigned char* xe;  // RESID: 1 / its scales, one per token and stage of columns, at pair_exp_at
@@ -86,14 +88,14 @@ __device__ __forceinline__ void pair_store4(char* row, int k, const f32x4& v, fl
 __device__ __forceinline__ float pair_top4(const f32x4& v) {
   return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
-// power of two that brings `bound` to less than 2^KH_PAIR_TOP (1 for 0, the smallest one for infinities and NaN)
-__device__ __forceinline__ float pair_scale(float bound) {
-  if (bound == 0.f) return 1.0f;
-  int e = (int)((__float_as_uint(bound) >> 23) & 255) - 126;  // |bound| < 2^e
-  int k = KH_PAIR_TOP - e;
+// power of two that brings `bound` to [2^(top - 1), 2^top), 2^100 at most (the smallest one for infinities and NaN)
+__device__ __forceinline__ float pair_scale_to(float bound, int top) {
+  const int e = (int)((__float_as_uint(bound) >> 23) & 255) - 126;  // |bound| < 2^e
+  int k = top - e;
   k = k < -114 ? -114 : (k > 100 ? 100 : k);
   return __uint_as_float((unsigned)(k + 127) << 23);
 }
+__device__ __forceinline__ float pair_scale(float bound) { return bound == 0.f ? 1.0f : pair_scale_to(bound, KH_PAIR_TOP); }
 __device__ __forceinline__ float pair_inv(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }  // 1 / s
 // 1 / s as its exponent, and where that of a token and a stage lies: 16 stages of a token side by side
 __device__ __forceinline__ unsigned char pair_exp(float s) { return (unsigned char)(254u - (__float_as_uint(s) >> 23)); }
@@ -237,27 +239,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   };
   const int nk = z1 - z0;
   f32x4 acc[TN][TM];
+  const int wm = wave % WM, wn = wave / WM;
+  const int fr = lane & 15, fh = lane >> 4;
+  float wsc[TN];  // fp32 weights: the scale of row fr of every tile, with the sign of the present sum
 #pragma unroll
   for (int n = 0; n < TN; ++n)
 #pragma unroll
     for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int wm = wave % WM, wn = wave / WM;
-  const int fr = lane & 15, fh = lane >> 4;
-  float wsc[TN];
-#pragma unroll
-  for (int n = 0; n < TN; ++n) {
-    wsc[n] = 1.0f;
-    if (!Q) {
-      int f = f0 + (wn * TN + n) * 16;
-      f = f < a.N - 16 ? f : a.N - 16;
-      int mat, row;
-      place(f, mat, row);
-      wsc[n] = a.ws[mat][row + fr];
-    }
-  }
-  // wait for them here: a wait left to their first use would sit in the loop and drain the ring
-#pragma unroll
-  for (int n = 0; n < TN; ++n) asm volatile("" : "+v"(wsc[n]));
   issue_exps(z0 >> 4);
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s)
@@ -269,6 +257,34 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   // its weights with the sign turned and is subtracted, which cancels it: 1.1e-6.
   float sgn = 1.0f, xinv[TM];
   unsigned xe[TM];
+  auto row_top = [&](float v) __attribute__((always_inline)) {  // over the four lanes of row fr
+    v = fmaxf(v, __shfl_xor(v, 16));
+    return fmaxf(v, __shfl_xor(v, 32));
+  };
+  auto row_at = [&](int n) __attribute__((always_inline)) {
+    int f = f0, mat, row;
+    asm volatile("" : "+s"(f));  // or the addresses are kept in registers throughout the loop
+    f += (wn * TN + n) * 16;
+    f = f < a.N - 16 ? f : a.N - 16;
+    place(f, mat, row);
+    return (const float*)a.w[mat].w + (size_t)(row + fr) * K;
+  };
+  auto row_scale = [&](int n) __attribute__((always_inline)) {  // from all columns of the slice
+    const float* w = row_at(n);
+    float t = 0.f;
+    for (int k = z0 * 32 + 4 * fh; k < z1 * 32; k += 16) t = fmaxf(t, pair_top4(*(const f32x4*)(w + k)));
+    return pair_scale(row_top(t));
+  };
+  auto split = [&](const f32x4 (&wv)[2], float sc, f16x8& wh, f16x8& wl) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const float v0 = wv[e >> 2][e & 3], v1 = wv[e >> 2][(e & 3) + 1];
+      const f16x2 hi = pair_cvt(v0 * sc, v1 * sc);
+      const f16x2 lo = pair_cvt(__builtin_fmaf(v0, sc, -(float)hi.x), __builtin_fmaf(v1, sc, -(float)hi.y));
+      wh[e] = hi.x; wh[e + 1] = hi.y;
+      wl[e] = lo.x; wl[e + 1] = lo.y;
+    }
+  };
   auto stage = [&](int k, auto open) __attribute__((always_inline)) {
     constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a sum
     // stage k has landed when at most the requests of the stages behind it are outstanding
@@ -301,21 +317,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
 #pragma unroll
         for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
       }
+      if (OPEN && k == 0) {
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          const float t = row_top(fmaxf(pair_top4(wv[n][0]), pair_top4(wv[n][1])));
+          wsc[n] = pair_scale_to(t, 10);
+          if (__builtin_amdgcn_ballot_w64(t == 0.f)) wsc[n] = row_scale(n);
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
         f16x8 wh, wl;
+        split(wv[n], wsc[n], wh, wl);
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          const float v0 = wv[n][e >> 2][e & 3], v1 = wv[n][e >> 2][(e & 3) + 1];
-          const f16x2 hi = pair_cvt(v0 * wsc[n], v1 * wsc[n]);
-          const f16x2 lo = pair_cvt(__builtin_fmaf(v0, wsc[n], -(float)hi.x), __builtin_fmaf(v1, wsc[n], -(float)hi.y));
-          wh[e] = hi.x; wh[e + 1] = hi.y;
-          wl[e] = lo.x; wl[e + 1] = lo.y;
-        }
-#pragma unroll
-        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wl, xh[m], OPEN ? f32x4{0.f, 0.f, 0.f, 0.f} : grp[n][m]);
+        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wl, xh[m], OPEN ? f4_zero() : grp[n][m]);
 #pragma unroll
         for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wh, xl[m], grp[n][m]);
 #pragma unroll
@@ -390,6 +407,43 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     }
     sgn = -sgn;
   };
+  // The wave's tiles once more, from memory, with scales from all columns (x * 0 above: also where the inputs are not finite).
+  auto again = [&]() __attribute__((always_inline)) {
+    const float* w[TN];
+    sgn = 1.0f;
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      wsc[n] = row_scale(n);
+      w[n] = row_at(n) + 8 * fh;
+#pragma unroll
+      for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma nounroll
+    for (int k = z0; k < z1; ++k) {
+      f16x8 wh[TN], wl[TN];
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const f32x4 wv[2] = {*(const f32x4*)(w[n] + 32 * k), *(const f32x4*)(w[n] + 32 * k + 4)};
+        split(wv, sgn * wsc[n], wh[n], wl[n]);
+      }
+#pragma unroll
+      for (int m = 0; m < TM; ++m) {
+        int t = t0 + (wm * TM + m) * 16 + fr;
+        t = t < a.T ? t : a.T - 1;
+        const char* x = a.X + ((unsigned)t * (unsigned)(4 * K) + 128u * k + 16u * fh);
+        const f16x8 xh = *(const f16x8*)x, xl = *(const f16x8*)(x + 64);
+        const float f = GROUP ? sgn * __uint_as_float((unsigned)a.xe[pair_exp_at(k, t, a.xe_ld)] << 23) : sgn;
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          const f32x4 g = mfma_pair(wh[n], xh, mfma_pair(wh[n], xl, mfma_pair(wl[n], xh, f4_zero())));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(f, g[i], acc[n][m][i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      sgn = -sgn;
+    }
+  };
   const std::true_type first{};
   const std::false_type second{};
   if constexpr (Q) {
@@ -416,21 +470,37 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       close();
     }
   }
+  if constexpr (!Q) {
+    // a half that has overflowed has left infinities or NaN in its row
+    float all = 0.f;
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) all = __builtin_fmaf(acc[n][m][i], 0.f, all);
+    if (__builtin_amdgcn_ballot_w64(all != 0.f)) again();
+  }
   // ---- epilogue: lane (fr, fh) of tile (n, m) holds rows 4 fh .. + 3 of the tile for token t0 + .. + fr
+  f32x4 wi[TN];
+  if constexpr (!Q) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wi[n][i] = pair_inv(__shfl(fabsf(wsc[n]), 4 * fh + i));
+  }
   float xi[TM];
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
     const int tok = t0 + (wm * TM + m) * 16 + fr;
     xi[m] = GROUP ? 1.0f : a.xs[tok < a.T ? tok : a.T - 1];
   }
-  auto value = [&](int n, int m, int mat, int row) __attribute__((always_inline)) {
+  auto value = [&](int n, int m) __attribute__((always_inline)) {
     f32x4 v = acc[n][m];
-    f32x4 s = {1.f, 1.f, 1.f, 1.f};
-    if (!Q) s = *(const f32x4*)(a.ws[mat] + row);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (!GROUP) v[i] *= xi[m];
-      if (!Q) v[i] *= pair_inv(s[i]);
+      if (!Q) v[i] *= wi[n][i];
     }
     return v;
   };
@@ -449,10 +519,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
         const int f = f0 + (wn * TN + n) * 16;
         o[m][n / 2] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (f >= a.N) continue;
-        int mat, row;
-        place(f, mat, row);
-        row += 4 * fh;
-        const f32x4 g = value(n, m, 0, row), u = value(n + 1, m, 1, row);
+        const f32x4 g = value(n, m), u = value(n + 1, m);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           o[m][n / 2][i] = swiglu1(g[i], u[i]);
@@ -494,7 +561,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       place(f, mat, row);
       row += 4 * fh;
       if (EPI == KH_PG_RESID) {
-        const f32x4 v = value(n, m, 0, row);
+        const f32x4 v = value(n, m);
         if (gridDim.y > 1) {
           *(f32x4*)(a.part + ((size_t)blockIdx.y * a.tcap + tok) * a.ldo + row) = v;
         } else {  // residual add (llama3.cpp:686,719)
@@ -520,7 +587,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
         if (a.rope == KH_PG_ROPE_TILES) {
           if (n & 1) continue;
           // tile n + 1 holds the partners, half a head further; cache column 2 j (cpu/rope_kernel.cpp:18-42)
-          const f32x4 lo = biased(value(n, m, mat, row), row), hi = biased(value(n + 1, m, mat, row + (hs >> 1)), row + (hs >> 1));
+          const f32x4 lo = biased(value(n, m), row), hi = biased(value(n + 1, m), row + (hs >> 1));
           f32x4 olo = lo, ohi = hi;
           if (mat < 2) {
             const int j = row % hs;
@@ -534,7 +601,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
           *(f32x4*)(dst + row) = olo;
           *(f32x4*)(dst + row + (hs >> 1)) = ohi;
         } else {
-          f32x4 v = biased(value(n, m, mat, row), row);
+          f32x4 v = biased(value(n, m), row);
           if (mat < 2 && a.rope == KH_PG_ROPE_PAIRS) {  // pairs (row, row + 1) (cpu/rope_kernel.cpp:98-121)
             const int c = row % hs;
             const float s0 = sn[c], c0 = cs[c], s1 = sn[c + 2], c1 = cs[c + 2];
@@ -545,28 +612,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       }
     }
   }
-}
-
-// ---- scales, once per model ----------------------------------------------------------------------------------------
-struct KhPairMats {  // the matrices of a layer
-  struct {
-    KhLin w;
-    int rows, K;
-  } m[7];
-};
-// One wave per row of the stacked matrices, 16 bytes a lane; K is a multiple of 32.
-static __global__ __launch_bounds__(256) void k_pair_rows(const KhPairMats a, float* ws, int total) {
-  const int at = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (at >= total) return;
-  int row = at, i = 0;
-  while (i < 6 && row >= a.m[i].rows) row -= a.m[i++].rows;
-  const int K = a.m[i].K;
-  const float* w = (const float*)a.m[i].w.w + (size_t)row * K;
-  float top = 0.f;
-#pragma unroll 4
-  for (int k = 4 * lane; k < K; k += 256) top = fmaxf(top, pair_top4(ld_nt((const f32x4*)(w + k))));
-  for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
-  if (lane == 0) ws[at] = pair_scale(top);
 }
 
 // ---- the per-token kernels between the GEMMs ------------------------------------------------------------------------

@@ -134,3 +134,56 @@ def test_rows_handed_back_change_nothing(gpu):
         m.close()
     for a, b in zip(*out):
         assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("shape", [None, "0,1", "1,4", "2,2", "3,4"])
+@pytest.mark.parametrize("first", [0.0, 2.0 ** -24, 2.0 ** 10])
+def test_first_columns_of_another_size(gpu, first, shape, monkeypatch):
+    """The scale of a weight row comes from its first 32 columns: rows where these (and those in front of a K slice) are zero,
+    tiny or large.  Large ones meet inputs as much smaller."""
+    spec = _PF_SPECS["gqa-half"]
+    img = binfmt.synth_image(spec, seed=55, device=gpu)
+    t = exact_kv.tensors(img, spec)
+    for l in range(spec.n_layers):
+        for n, norm in (("wq", "att_norm"), ("wk", "att_norm"), ("wv", "att_norm"), ("w1", "ffn_norm"), ("w3", "ffn_norm"),
+                        ("wo", None), ("w2", None)):
+            w = t[f"{n}.{l}"]
+            if first > 1 and norm is None:
+                continue
+            w[::3, :32] *= first
+            if norm is None:
+                w[::3, w.shape[1] // 2: w.shape[1] // 2 + 32] *= first
+        if first > 1:
+            for norm in ("att_norm", "ffn_norm"):
+                t[f"{norm}.{l}"][:32] /= first
+    if shape:
+        monkeypatch.setenv("KH_PAIR_SHAPE", shape)
+    pair, fp32 = errors(monkeypatch, img, spec, 150)
+    print(f"first columns {first:.2g}, shape {shape}: {pair:.3g} with pairs, {fp32:.3g} without")
+    assert pair <= 1.25 * fp32
+
+
+@pytest.mark.parametrize("name", ["gqa-half", "qwen-bias", "int8"])
+def test_weights_written_in_place(gpu, name):
+    """Weights that the caller owns may be written between two calls: the rows are those of a model made afterwards."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = _PF_SPECS[name]
+    img = binfmt.synth_image(spec, seed=56, device=gpu)
+    toks = [int(t) for t in np.random.default_rng(20).integers(0, spec.vocab_size, 300)]
+    m = KuiperModel.from_device_image(img, spec)
+    m.prefill_gemm(toks, 0)
+    for e in binfmt.layout(spec)[0]:
+        w = binfmt.tensor_from_image(img, e)
+        base = e.name.split(".")[0]
+        if e.name.endswith("scales") or (w.dtype == torch.float32 and base[0] in "wb"):
+            k = torch.arange(w.numel(), device=gpu).reshape(w.shape) // w.shape[-1] % 3
+            w.mul_(torch.where(k == 0, 64.0, 1 / 64.0))
+    torch.cuda.synchronize()
+    m.prefill_gemm(toks, 0)
+    fresh = KuiperModel.from_device_image(img, spec)
+    fresh.prefill_gemm(toks, 0)
+    for l in range(spec.n_layers):
+        for a, b in zip(m.read_kv(l, 0, 300), fresh.read_kv(l, 0, 300)):
+            assert np.isfinite(a).all() and np.array_equal(a, b), l
+    m.close()
+    fresh.close()
