@@ -363,10 +363,15 @@ int kh_model_first_sample(kh_model* m, kh_first_sample* out);
 /* Launch plans, host-only (no device is touched; for tools and the CPU test-suite).
  * kh_plan_decode_shapes: {split, u, grid, wg} of the five GEMV kernels of a decode step (qkv, wo, ffn13, w2,
  * cls) for a geometry - what kh_model_create_* configures (env KH_SHAPE_* overrides included).
- * kh_plan_prefill_shape: {R, NT, ks, token slices, solo, kz, workgroups} of one GEMM of a T-token prefill
- * pass (epi 0 = QKV, 1 = residual GEMM wo / w2, 2 = SwiGLU pair; csrc/kh_model_prefill.hip::pg_shape). */
+ * kh_plan_prefill_shape: {R, NT, ks, token slices, solo, kz, workgroups} of one fp32-MFMA GEMM of a T-token prefill
+ * pass (epi 0 = QKV, 1 = residual GEMM wo / w2, 2 = SwiGLU pair; csrc/kh_model_prefill.hip::pg_shape): widths that are no
+ * multiple of 32, and hook KH_PG_PAIR=0. */
 int kh_plan_decode_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_dim, int32_t vocab_size,
                           int32_t is_quant, int32_t* out20);
+/* kh_plan_pair_shapes: {tokens, rows of a tile, K split, workgroups} of the four GEMMs (wq + wk + wv, wo, w1 + w3, w2) of a
+ * pass of T <= 2048 prompt tokens on pairs of halves (csrc/kh_model_pair.hip::pair_shape), the usual path;
+ * KH_ERR_UNSUPPORTED for the widths of kh_plan_prefill_shape. */
+int kh_plan_pair_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_dim, int32_t is_quant, int32_t T, int32_t* out16);
 /* kh_plan_decode_ring: out4 = {ffn13 ring slots per wave, ffn13 workgroups, cls ring slots, cls workgroups} - which
  * int8 GEMVs of a decode step run on the LDS-DMA ring kernels (csrc/kh_fused_ring.h; 0 slots = the register-tile
  * kernel of kh_plan_decode_shapes) and with how many 256-thread workgroups.  Hook KH_RING=0 turns them off. */

@@ -103,6 +103,28 @@ int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out, int* fine_out = n
 }
 }  // namespace
 
+// Host-only view of pair_shape for the four GEMMs of a layer; KH_PAIR_SHAPE is not applied.
+extern "C" int kh_plan_pair_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_dim, int32_t is_quant, int32_t T, int32_t* out16) {
+  if (!out16 || dim <= 0 || hidden_dim <= 0 || kv_dim <= 0 || T <= 0 || T > KH_PAIR_TMAX) return KH_ERR_INVALID_ARG;
+  kh_config c{};
+  c.dim = dim;
+  c.hidden_dim = hidden_dim;
+  c.kv_dim = kv_dim;
+  c.is_quant = is_quant != 0;
+  if (!pair_geometry(c)) return KH_ERR_UNSUPPORTED;
+  const int N[4] = {dim + 2 * kv_dim, dim, 2 * hidden_dim, dim}, K[4] = {dim, dim, dim, hidden_dim};
+  for (int i = 0; i < 4; ++i) {
+    const PairShape s = pair_shape(c.is_quant, T, N[i], K[i], i & 1);
+    const PairTile& t = kPairTiles[c.is_quant][s.tile];
+    int32_t* o = out16 + 4 * i;
+    o[0] = t.bm;
+    o[1] = t.bn;
+    o[2] = s.kz;
+    o[3] = (N[i] + t.bn - 1) / t.bn * ((T + t.bm - 1) / t.bm) * s.kz;
+  }
+  return KH_OK;
+}
+
 namespace khm {
 // pair slabs advance in 32-column blocks, int8 groups in 64; other widths stay with k_pg_gemm
 bool pair_geometry(const kh_config& c) {

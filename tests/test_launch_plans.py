@@ -1,6 +1,6 @@
 """Host-side launch planning (no GPU): the decode GEMV shapes (csrc/kh_model_step.hip::pick_shape) and the
 prefill GEMM shapes (csrc/kh_model_prefill.hip::pg_shape) through the host-only C-ABI entries
-kh_plan_decode_shapes / kh_plan_prefill_shape.  Invariants every plan must satisfy for every BASELINE
+kh_plan_decode_shapes / kh_plan_pair_shapes / kh_plan_prefill_shape.  Invariants every plan must satisfy for every BASELINE
 geometry, plus the plans DESIGN.md documents (so that a change of the heuristics shows up here and not
 only as a slower GPU run)."""
 import itertools
@@ -120,6 +120,40 @@ def test_prefill_plan_documented_shapes(monkeypatch):
         _ffi.plan_prefill_shape("qkv", 513, 3072, 2048, False, True)
     with pytest.raises(_ffi.KhError):
         _ffi.plan_prefill_shape("qkv", 128, 3072, 2040, False, True)
+
+
+@pytest.mark.parametrize("name", PRESETS + ["stories15M"])
+def test_pair_plan_invariants(name):
+    """The GEMMs that prompts run on (csrc/kh_model_pair.hip): tiles that exist, K slices of four stages at least and of the
+    residual products only, no fewer workgroups at more tokens with the same tile."""
+    sp = binfmt.PRESETS[name]
+    tiles = ((112, 128), (64, 128), (32, 128), (128, 256)) if sp.quant else ((128, 128), (64, 128), (32, 128), (32, 64))
+    N = {"qkv": sp.dim + 2 * sp.kv_dim, "wo": sp.dim, "w13": 2 * sp.hidden_dim, "w2": sp.dim}
+    last = {}
+    for T in (1, 16, 17, 32, 33, 64, 65, 112, 113, 128, 200, 256, 300, 511, 512, 777, 1024, 1900, 2048):
+        for g, p in _ffi.plan_pair_shapes(sp.dim, sp.hidden_dim, sp.kv_dim, sp.quant, T).items():
+            K = sp.hidden_dim if g == "w2" else sp.dim
+            assert (p["bm"], p["bn"]) in tiles, (T, g, p)
+            assert p["kz"] in ((1, 2, 4) if g in ("wo", "w2") else (1,)), (T, g, p)
+            assert p["kz"] == 1 or K // (64 if sp.quant else 32) // p["kz"] >= 4, (T, g, p)
+            assert p["workgroups"] == -(-N[g] // p["bn"]) * -(-T // p["bm"]) * p["kz"], (T, g, p)
+            shape = (p["bm"], p["bn"], p["kz"])
+            assert last.get((g, shape), 0) <= p["workgroups"], (T, g, p)
+            last[g, shape] = p["workgroups"]
+
+
+def test_pair_plan_of_prompts(monkeypatch):
+    """Llama-3.2-1B and Llama-2-7B int8: the plans that the measured prompt times belong to."""
+    sp = binfmt.PRESETS["llama3.2-1b"]
+    p = _ffi.plan_pair_shapes(sp.dim, sp.hidden_dim, sp.kv_dim, False, 512)
+    assert p == {"qkv": dict(bm=64, bn=128, kz=1, workgroups=192), "wo": dict(bm=64, bn=128, kz=2, workgroups=256),
+                 "w13": dict(bm=128, bn=128, kz=1, workgroups=512), "w2": dict(bm=64, bn=128, kz=4, workgroups=512)}
+    s7 = binfmt.PRESETS["llama2-7b-int8"]
+    p = _ffi.plan_pair_shapes(s7.dim, s7.hidden_dim, s7.kv_dim, True, 777)
+    assert p["w13"] == dict(bm=112, bn=128, kz=1, workgroups=1204) and p["qkv"]["workgroups"] == 672
+    for bad in ((2048, 8192, 512, False, 0), (2048, 8192, 512, False, 2049), (2064, 8192, 512, False, 512), (2080, 8192, 512, True, 512)):
+        with pytest.raises(_ffi.KhError):
+            _ffi.plan_pair_shapes(*bad)
 
 
 def test_attention_plan_and_split_geometry(monkeypatch):
