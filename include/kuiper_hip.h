@@ -330,7 +330,7 @@ int kh_model_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t po
  * weights are exact in one (csrc/kh_pair.h; the K/V rows are closer to their 64-bit values than those of an fp32 fmaf
  * chain as long as the numbers that share a scale - a normed row, 64 columns of the gated unit or of an attention output,
  * 32 cached rows of a head, a weight row - are within about 2^12 of one another where they weigh alike in a result).  Widths
- * that are no multiple of 32 - and hook KH_PG_PAIR=0 - take fp32-MFMA GEMMs instead (csrc/kh_gemm.h: v_mfma_f32_16x16x4_f32,
+ * that are no multiple of 32, matrices of more than 4 GiB - and hook KH_PG_PAIR=0 - take fp32-MFMA GEMMs instead (csrc/kh_gemm.h: v_mfma_f32_16x16x4_f32,
  * passes of up to 512 tokens, int8 weights dequantised per element in registers).  Either way nothing about the weights is
  * kept between calls: memory given to kh_model_create_from_device_weights may be written between them.  The K/V rows agree
  * with the token-by-token path to fp32 round-off (different summation order), not bit for bit.
@@ -365,7 +365,7 @@ int kh_model_first_sample(kh_model* m, kh_first_sample* out);
  * cls) for a geometry - what kh_model_create_* configures (env KH_SHAPE_* overrides included).
  * kh_plan_prefill_shape: {R, NT, ks, token slices, solo, kz, workgroups} of one fp32-MFMA GEMM of a T-token prefill
  * pass (epi 0 = QKV, 1 = residual GEMM wo / w2, 2 = SwiGLU pair; csrc/kh_model_prefill.hip::pg_shape): widths that are no
- * multiple of 32, and hook KH_PG_PAIR=0. */
+ * multiple of 32, matrices of more than 4 GiB, and hook KH_PG_PAIR=0. */
 int kh_plan_decode_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_dim, int32_t vocab_size,
                           int32_t is_quant, int32_t* out20);
 /* kh_plan_pair_shapes: {tokens, rows of a tile, K split, workgroups} of the four GEMMs (wq + wk + wv, wo, w1 + w3, w2) of a

@@ -126,10 +126,12 @@ extern "C" int kh_plan_pair_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_d
 }
 
 namespace khm {
-// pair slabs advance in 32-column blocks, int8 groups in 64; other widths stay with k_pg_gemm
+// Pair slabs advance in 32-column blocks, int8 groups in 64, and k_pair_gemm addresses a matrix and a slab with 32 bits:
+// other widths stay with k_pg_gemm.
 bool pair_geometry(const kh_config& c) {
   const int g = c.is_quant ? 64 : 32;
-  return c.dim % g == 0 && c.hidden_dim % g == 0;
+  const int64_t wide = std::max(c.dim, c.hidden_dim), lim = (int64_t)1 << 32;
+  return c.dim % g == 0 && c.hidden_dim % g == 0 && wide * c.dim * (c.is_quant ? 1 : 4) <= lim && wide * KH_PAIR_TMAX * 4 <= lim;
 }
 
 namespace {

@@ -150,8 +150,10 @@ def test_pair_plan_of_prompts(monkeypatch):
                  "w13": dict(bm=128, bn=128, kz=1, workgroups=512), "w2": dict(bm=64, bn=128, kz=4, workgroups=512)}
     s7 = binfmt.PRESETS["llama2-7b-int8"]
     p = _ffi.plan_pair_shapes(s7.dim, s7.hidden_dim, s7.kv_dim, True, 777)
+    assert _ffi.plan_pair_shapes(16384, 53248, 1024, False, 512) and _ffi.plan_pair_shapes(18432, 73728, 2304, True, 512)
     assert p["w13"] == dict(bm=112, bn=128, kz=1, workgroups=1204) and p["qkv"]["workgroups"] == 672
-    for bad in ((2048, 8192, 512, False, 0), (2048, 8192, 512, False, 2049), (2064, 8192, 512, False, 512), (2080, 8192, 512, True, 512)):
+    for bad in ((2048, 8192, 512, False, 0), (2048, 8192, 512, False, 2049), (2064, 8192, 512, False, 512), (2080, 8192, 512, True, 512),
+                (18432, 73728, 2304, False, 512), (18432, 245760, 2304, True, 512)):  # matrices of more than 4 GiB
         with pytest.raises(_ffi.KhError):
             _ffi.plan_pair_shapes(*bad)
 
