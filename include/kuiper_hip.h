@@ -388,7 +388,7 @@ int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32
 
 /* Tuning / test hooks.  Every hook the library honours (KH_SHAPE_<QKV|WO|FFN|W2|CLS>, KH_RING, KH_ATTN_WG, KH_ATTN_FENCED,
  * KH_ATTN_TLONG, KH_ATTN_DEFER (0 = never merge time splits in the wo kernel), KH_ATTN_DEFER_MAX (active splits up to
- * which it does), KH_PREFILL, KH_PG_<CHUNK|PAIR|SHAPE_*|SOLO|KZ|ATTN|ATTN_QT|ROPE_FUSE|DEBUG> (SHAPE_*, SOLO, KZ and
+ * which it does), KH_PREFILL, KH_PG_<CHUNK|ROWS (the most slab rows that memory is given for)|PAIR|SHAPE_*|SOLO|KZ|ATTN|ATTN_QT|ROPE_FUSE|DEBUG> (SHAPE_*, SOLO, KZ and
  * DEBUG belong to the fp32-MFMA GEMMs; a SHAPE_* hook selects them), KH_PAIR_SHAPE (tile,K split of the pair GEMMs),
  * KH_PAIR_ATTN (0 = attention of a prompt slice on the fp32 matrix cores; KH_PG_ATTN_QT selects it too),
  * KH_SHAPE_DEBUG, KH_HY_DECODE (0 = single-token batches of layer-list models run on the pass kernels), KH_HY_EXPAND (0 = latent

@@ -122,7 +122,7 @@ struct kh_model {
   unsigned char *pg_ae = nullptr, *pg_he = nullptr;
   char* pa_ws = nullptr;     // K / V of one layer as pairs in fragment order (kh_pattn_pair.h)
   size_t pa_ws_bytes = 0;
-  int pg_rows = 0;  // token rows of the slabs above
+  int pg_rows = 0, pg_part_rows = 0;  // token rows of the slabs above, rows of pg_part
   bool pf_ready = false, pg_ready = false;  // set when ALL prefill slabs exist (allocation can fail half-way)
   bool pg_launch_failed = false;
   int32_t* h_words_pin = nullptr;  // pinned mirror of d_words (stop-token check, final copy-out)
@@ -223,5 +223,7 @@ bool pg_supported(const kh_model* m);       // MFMA GEMM path
 bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int layout, int tcap);
 // pair GEMMs (kh_model_pair.hip)
 bool pair_geometry(const kh_config& c);
+int pair_part_rows(const kh_config& c, int rows);  // partial rows of passes of up to `rows` tokens
+void pair_prepare(kh_model* m, int n, int pos0);  // memory of the attention of a prompt's passes, if there is any
 int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0);
 }  // namespace khm

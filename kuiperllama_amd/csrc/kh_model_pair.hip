@@ -84,6 +84,7 @@ int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out, int* fine_out = n
     if (sscanf(e, "%d,%d", &t, &kz) == 2 && t >= 0 && t < 4 && (kz == 1 || kz == 2 || kz == 4))
       sh = PairShape{t, EPI == KH_PG_RESID ? kz : 1};
   }
+  while (sh.kz > 1 && sh.kz * a.T > m->pg_part_rows) sh.kz /= 2;  // (a hook set behind the allocation)
   if (fine_out) *fine_out = kPairTiles[m->cfg.is_quant][sh.tile].bn < 128;
   if (kz_out) *kz_out = sh.kz > 1 ? sh.kz : 0;
   if (m->cfg.is_quant) {
@@ -134,45 +135,74 @@ bool pair_geometry(const kh_config& c) {
   return c.dim % g == 0 && c.hidden_dim % g == 0 && wide * c.dim * (c.is_quant ? 1 : 4) <= lim && wide * KH_PAIR_TMAX * 4 <= lim;
 }
 
+int pair_part_rows(const kh_config& c, int rows) {
+  int most = 0;
+  for (int T = 1; T <= rows; ++T)
+    for (int K : {c.dim, c.hidden_dim}) {
+      const int kz = pair_shape(c.is_quant, T, c.dim, K, true).kz;
+      if (kz > 1) most = std::max(most, kz * T);
+    }
+  return most;
+}
+
 namespace {
 template <int HS, int QT>
 void pa_go(const KhPaArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_pa_pack<HS>, dim3((a.pos0 + a.T + 31) / 32, a.kv_heads), dim3(256), 0, s, a);
   hipLaunchKernelGGL((k_pa_attn<HS, 4, QT>), dim3(a.kv_heads * a.kv_mul * ((a.T + 16 * QT - 1) / (16 * QT))), dim3(256), 0, s, a);
 }
-template <int HS>
-size_t pa_bytes(int heads, int blocks) { return (size_t)heads * blocks * (PaGeom<HS>::FR * 1024 + 2 * sizeof(float)); }
+// bytes of one layer's K / V rows as pairs; 0: no kernel for this head size
+size_t pa_bytes(const kh_config& c, int positions) {
+  auto block = [](auto g) { return (size_t)decltype(g)::FR * 1024 + 2 * sizeof(float); };
+  const size_t n = (size_t)c.kv_head_num * ((positions + 31) / 32);
+  switch (c.head_size) {
+    case 48: return n * block(PaGeom<48>{});
+    case 64: return n * block(PaGeom<64>{});
+    case 128: return n * block(PaGeom<128>{});
+    default: return 0;
+  }
+}
 
 // Attention of a slice with its operands as pairs; false: the caller takes pg_slice_attention (fp32 matrix cores).
 // Packing reads all of the layer's rows whatever T is, so it needs enough query tokens and enough work.  Whole prompt
 // passes, ms, fp32 matrix cores against pairs, T @ first position: Llama-3.2-1B 128 @ 0 1.98 / 2.00, 256 @ 0 2.68 / 2.68,
 // 512 @ 0 4.05 / 3.94, 64 @ 2048 2.05 / 2.05, 256 @ 2048 3.42 / 3.06, 2048 @ 2048 20.3 / 14.6; Llama-2-7B int8
 // 128 @ 0 7.07 / 7.13, 256 @ 0 10.5 / 10.3, 128 @ 1024 8.08 / 7.83, 1024 @ 1024 41.5 / 34.5.
-// The slab of a layer is given up (not the call) above KH_PA_WS_MAX and where memory for it is refused.
+bool pa_pays(int T, int pos0) {
+  if (dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
+  return T >= 128 && (size_t)T * (2 * (size_t)pos0 + T) >= 65536;
+}
+}  // namespace
+// The slab of a layer is given up (not the call) above KH_PA_WS_MAX and where memory for it is refused.  It at least doubles.
+void pair_prepare(kh_model* m, int n, int pos0) {
+  const kh_config& c = m->cfg;
+  size_t need = 0;
+  for (int t0 = 0; t0 < n; t0 += m->pg_rows) {
+    const int T = std::min(n - t0, m->pg_rows);
+    const size_t b = pa_pays(T, pos0 + t0) ? pa_bytes(c, pos0 + t0 + T) : 0;
+    if (b <= KH_PA_WS_MAX) need = std::max(need, b);
+  }
+  if (need <= m->pa_ws_bytes) return;
+  const size_t most = std::min(KH_PA_WS_MAX, pa_bytes(c, c.cache_len)), twice = std::min(std::max(need, 2 * m->pa_ws_bytes), most);
+  if (m->pa_ws) (void)hipFree(m->pa_ws);
+  m->pa_ws = nullptr;
+  m->pa_ws_bytes = 0;
+  for (size_t b : {twice, need}) {
+    if (dalloc(&m->pa_ws, b) == KH_OK) {
+      m->pa_ws_bytes = b;
+      return;
+    }
+    (void)hipGetLastError();
+    m->pa_ws = nullptr;
+  }
+}
+namespace {
 bool pair_attention(kh_model* m, int l, int T, int pos0) {
   const kh_config& c = m->cfg;
-  if (dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
-  if (T < 128 || (size_t)T * (2 * (size_t)pos0 + T) < 65536) return false;
+  const size_t need = pa_bytes(c, pos0 + T);
+  if (!pa_pays(T, pos0) || need == 0 || need > m->pa_ws_bytes) return false;
   KhPaArgs a{};
   a.blocks = (pos0 + T + 31) / 32;
-  size_t need = 0;
-  switch (c.head_size) {
-    case 48: need = pa_bytes<48>(c.kv_head_num, a.blocks); break;
-    case 64: need = pa_bytes<64>(c.kv_head_num, a.blocks); break;
-    case 128: need = pa_bytes<128>(c.kv_head_num, a.blocks); break;
-    default: return false;
-  }
-  if (need > KH_PA_WS_MAX) return false;
-  if (need > m->pa_ws_bytes) {
-    if (m->pa_ws) (void)hipFree(m->pa_ws);
-    m->pa_ws = nullptr;
-    m->pa_ws_bytes = 0;
-    if (dalloc(&m->pa_ws, need) != KH_OK) {
-      (void)hipGetLastError();
-      return false;
-    }
-    m->pa_ws_bytes = need;
-  }
   a.q = m->pg_q;
   a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
   a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
@@ -204,14 +234,15 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
   for (int l = 0; l < c.layer_num; ++l) {
     const LayerW& W = m->layers[l];
     auto rmsnorm = [&](const float* w) {
-      hipLaunchKernelGGL(k_pair_rmsnorm, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_x, w, xn, m->pg_xs, c.dim, c.rms_eps, m->pg_rows,
+      hipLaunchKernelGGL(k_pair_rmsnorm, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_x, w, xn, m->pg_xs, c.dim, c.rms_eps, T,
                          (const float*)m->pg_part, kz);
       kz = 0;
     };
     KhPairArgs base{};
     base.T = T;
     base.pos0 = pos0;
-    base.tcap = base.xe_ld = m->pg_rows;
+    base.tcap = T;
+    base.xe_ld = m->pg_rows;
     base.xs = m->pg_xs;
     base.part = m->pg_part;
     base.head_size = c.head_size;

@@ -228,12 +228,15 @@ void launch_prefill_chunk(kh_model* m, const int32_t* toks, int nvalid, int pos0
 
 // ---- GEMM prefill (kh_gemm.h) ------------------------------------------------------------------
 namespace {
-// slabs for a prompt of n tokens: at least KH_PG_TMAX rows, more for the longer passes of the pair GEMMs
-int ensure_pg_buffers(kh_model* m, int n) {
-  int rows = KH_PG_TMAX;
-  if (pair_geometry(m->cfg)) rows = std::max(rows, std::min((n + 127) / 128 * 128, KH_PAIR_TMAX));
-  if (m->pg_ready && m->pg_rows >= rows) return KH_OK;
-  if (m->pg_ready) KH_CHECK_HIP(hipStreamSynchronize(m->stream));  // passes on the smaller slabs
+// does the prompt-slice attention run on the MFMA kernel (kh_pattn.h)?  KH_PG_ATTN=0 forces the fallback.
+bool pg_mfma_attn(const kh_model* m) { return !dbg_off("KH_PG_ATTN") && pg_attn_supported(m->cfg.head_size); }
+// prompt passes on the pair GEMMs?  KH_PG_PAIR=0 and the shape hooks of k_pg_gemm select the fp32-MFMA GEMMs.
+bool pg_pair(const kh_model* m) {
+  return pair_geometry(m->cfg) && !dbg_off("KH_PG_PAIR") && !dbg("KH_PG_SHAPE_QKV") && !dbg("KH_PG_SHAPE_RESID") &&
+         !dbg("KH_PG_SHAPE_SWIGLU");
+}
+// slabs of `rows` token rows and `part` partial rows
+int alloc_pg_buffers(kh_model* m, int rows, int part) {
   m->pg_ready = false;
   // a previous attempt may have failed half-way (out of memory): start from a clean slate so a
   // later call never launches GEMMs on null slabs
@@ -261,18 +264,44 @@ int ensure_pg_buffers(kh_model* m, int n) {
   if ((rc = zalloc(&m->pg_q, T * c.dim)) != KH_OK) return rc;
   if ((rc = zalloc(&m->pg_att, T * c.dim)) != KH_OK) return rc;
   if ((rc = zalloc(&m->pg_h, T * c.hidden_dim)) != KH_OK) return rc;
-  if ((rc = zalloc(&m->pg_part, (size_t)KH_PG_KZ_MAX * T * c.dim)) != KH_OK) return rc;  // K-slice partial rows
+  if ((rc = zalloc(&m->pg_part, (size_t)part * c.dim)) != KH_OK) return rc;  // K-slice partial rows
   if (pair_geometry(c)) {
     if ((rc = dalloc(&m->pg_xs, T)) != KH_OK) return rc;
     if ((rc = dalloc(&m->pg_ae, pair_exp_bytes(c.dim, c.is_quant, rows))) != KH_OK) return rc;
     if ((rc = dalloc(&m->pg_he, pair_exp_bytes(c.hidden_dim, c.is_quant, rows))) != KH_OK) return rc;
   }
   m->pg_rows = rows;
+  m->pg_part_rows = part;
   m->pg_ready = true;
   return KH_OK;
 }
-// does the prompt-slice attention run on the MFMA kernel (kh_pattn.h)?  KH_PG_ATTN=0 forces the fallback.
-bool pg_mfma_attn(const kh_model* m) { return !dbg_off("KH_PG_ATTN") && pg_attn_supported(m->cfg.head_size); }
+// Slabs for a prompt of n tokens: KH_PG_TMAX rows, two or four times as many for the longer passes of the pair GEMMs, so that
+// a conversation that grows turn by turn reallocates twice at most.  Where there is no memory for those (hook KH_PG_ROWS:
+// for more rows than it says), fewer rows: the prompt then takes more passes.
+int ensure_pg_buffers(kh_model* m, int n) {
+  const bool pair = pg_pair(m);
+  int rows = KH_PG_TMAX;
+  while (pair && pg_mfma_attn(m) && rows < n && rows < KH_PAIR_TMAX) rows *= 2;
+  // every split that pair_shape may choose for the slabs' rows, or all that k_pg_gemm and the hook may
+  const bool any_split = !pair || dbg("KH_PAIR_SHAPE");
+  auto done = [&](int r) { return m->pg_ready && m->pg_rows >= r && (!any_split || m->pg_part_rows >= KH_PG_KZ_MAX * r); };
+  if (done(rows)) return KH_OK;
+  if (m->pg_ready) KH_CHECK_HIP(hipStreamSynchronize(m->stream));  // passes on the smaller slabs
+  auto part = [&](int r) { return any_split ? KH_PG_KZ_MAX * r : std::max(KH_PG_KZ_MAX * KH_PG_TMAX, pair_part_rows(m->cfg, r)); };
+  auto bytes = [&](size_t r, size_t p) { return 4 * (r * (4 * (size_t)m->cfg.dim + m->cfg.hidden_dim) + p * m->cfg.dim); };
+  const char* most = dbg("KH_PG_ROWS");
+  for (; rows > KH_PG_TMAX; rows /= 2) {
+    if (done(rows)) return KH_OK;
+    const int p = part(rows);
+    size_t room = 0, total = 0;
+    if (hipMemGetInfo(&room, &total) != hipSuccess) room = ~(size_t)0;  // not known: try
+    else room += m->pg_ready ? bytes(m->pg_rows, m->pg_part_rows) : 0;
+    if ((most && atoi(most) < rows) || bytes(rows, p) > room) continue;
+    if (alloc_pg_buffers(m, rows, p) == KH_OK) return KH_OK;
+    (void)hipGetLastError();
+  }
+  return done(rows) ? KH_OK : alloc_pg_buffers(m, rows, part(rows));
+}
 // The split workspace of the decode-attention FALLBACK (one per token of a pass, ~270 KB per token at
 // Llama-3.2-1B geometry: 136 MB for a 512-token pass).  Every BASELINE head size has an MFMA
 // instantiation, so it is allocated on the first pass that actually takes the fallback.
@@ -576,8 +605,7 @@ extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32
   if ((rc = ensure_pg_buffers(m, n)) != KH_OK) return rc;
   if ((rc = ensure_pg_ws(m)) != KH_OK) return rc;
   m->pg_launch_failed = false;
-  // KH_PG_PAIR=0 and the shape hooks of k_pg_gemm select the fp32-MFMA GEMMs
-  const bool pair = pair_geometry(c) && !dbg_off("KH_PG_PAIR") && !dbg("KH_PG_SHAPE_QKV") && !dbg("KH_PG_SHAPE_RESID") && !dbg("KH_PG_SHAPE_SWIGLU");
+  const bool pair = pg_pair(m);
   // tuning / test hook: KH_PG_CHUNK=<tokens per weight pass> (16 .. KH_PG_TMAX), read per call
   int chunk = pair && pg_mfma_attn(m) ? m->pg_rows : KH_PG_TMAX;
   if (const char* e = dbg("KH_PG_CHUNK")) {
@@ -585,6 +613,7 @@ extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32
     chunk = v < 16 ? 16 : (v > KH_PG_TMAX ? KH_PG_TMAX : v);
   }
   if (pair) {
+    pair_prepare(m, n, pos0);
     for (int t0 = 0; t0 < n; t0 += chunk)
       if ((rc = launch_prefill_pair_chunk(m, h_tokens + t0, n - t0 < chunk ? n - t0 : chunk, pos0 + t0)) != KH_OK) return rc;
     return kh_launch_status();
@@ -687,6 +716,7 @@ extern "C" int kh_model_time_prefill(kh_model* m, const int32_t* h_tokens, int32
     if (!m->hy) {
       if ((rc = ensure_pg_buffers(m, n)) != KH_OK) return rc;
       if ((rc = ensure_pg_ws(m)) != KH_OK) return rc;
+      if (pg_pair(m)) pair_prepare(m, n, pos0);
     }
     KH_CHECK_HIP(hipEventRecord(m->ev0, m->stream));
     if ((rc = kh_model_prefill_gemm(m, h_tokens, n, pos0)) != KH_OK) return rc;
