@@ -50,7 +50,8 @@ def test_slices(gpu, hs, heads, kv_heads, half, monkeypatch):
 def test_spread_of_values_and_scores(gpu, hs, heads, kv_heads, half, monkeypatch):
     """Value rows between 2^-20 and 1 of their usual size, some zero; queries 16 times as large, so that a few positions
     carry a row.  An fp32 score of size s has an error of s 2^-24 per rounding, here s < 2^8 and some 2^3 roundings: the
-    weights, and with them the rows, move by 2^-13 at most between two orders of summation."""
+    weights, and with them the rows, move by 2^-13 at most between two orders of summation.  Columns far below the row's
+    largest entry are held by test_pair_exact_gpu.py."""
     spec = _spec(hs, heads, kv_heads, half)
     img = binfmt.synth_image(spec, seed=42, device=gpu)
     for e in binfmt.layout(spec)[0]:

@@ -187,3 +187,42 @@ def test_weights_written_in_place(gpu, name):
             assert np.isfinite(a).all() and np.array_equal(a, b), l
     m.close()
     fresh.close()
+
+
+_WIDTHS = {
+    # 480 = 7.5 groups of 64 columns, heads of 96 (attention outputs through k_pair_convert), hidden 1376 = 21.5 groups
+    "odd": binfmt.ModelSpec(480, 1376, 2, 5, 5, 500, 512, True, binfmt.FAMILY_LLAMA, False, 64, binfmt.ROPE_HALF, 10000.0, 1e-5, "odd"),
+    # rows that k_pair_rmsnorm does not keep in registers
+    "wide": binfmt.ModelSpec(4608, 512, 2, 36, 4, 500, 512, True, binfmt.FAMILY_LLAMA, False, 64, binfmt.ROPE_INTERLEAVED, 10000.0,
+                             1e-5, "wide"),
+}
+
+
+@pytest.mark.parametrize("name", sorted(_WIDTHS))
+@pytest.mark.parametrize("n", [3, 70, 300])
+def test_widths(gpu, name, n, monkeypatch):
+    spec = _WIDTHS[name]
+    img = binfmt.synth_image(spec, seed=57, device=gpu)
+    pair, fp32 = errors(monkeypatch, img, spec, n)
+    print(f"{name}, {n} tokens: {pair:.3g} with pairs, {fp32:.3g} without")
+    assert pair <= 1.25 * fp32
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_token_that_is_not_finite(gpu, bad):
+    """An embedding row that is not finite spoils its own position and those behind it: blocks of positions in front of it
+    stay within the error of the rest (the waves that meet it compute their tiles a second way)."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = _PF_SPECS["gqa-half"]
+    img = binfmt.synth_image(spec, seed=58, device=gpu)
+    toks = [int(t) for t in np.random.default_rng(24).integers(0, spec.vocab_size - 1, 300)]
+    toks[200] = spec.vocab_size - 1
+    want = exact_kv.rows(img, spec, toks[:192])
+    exact_kv.tensors(img, spec)["tok_emb"][spec.vocab_size - 1, 17] = bad
+    m = KuiperModel.from_device_image(img, spec)
+    m.prefill_gemm(toks, 0)
+    for l in range(spec.n_layers):
+        for got, w in zip(m.read_kv(l, 0, 192), want[l]):
+            assert exact_kv.error(got, w) < 2e-6, l  # 1.2e-6: the largest on the fp32 matrix cores without it
+        assert not np.isfinite(m.read_kv(l, 200, 1)[0]).all()
+    m.close()

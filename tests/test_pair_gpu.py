@@ -64,9 +64,10 @@ def test_long_pass_and_second_pass(gpu, name, monkeypatch):
 
 @pytest.mark.parametrize("name", ["gqa-half", "mha-interleaved"])
 def test_scales_follow_weights_and_cache(gpu, name, monkeypatch):
-    """Weight rows between 2^-20 and 2^20 of their usual size (row scales; the bound of the gated unit then lies far above
-    most of it), a zero row, and cache rows of 1e6 in front of the prompt (scales of the attention output).  Rows are held
-    to 2e-5 of their largest entry: 2^-24 per operand, 2^-22 per product, some hundred roundings to fp32 behind them."""
+    """Weight rows between 2^-20 and 2^20 of their usual size (scales of the rows and of the gated unit), a zero row, and
+    cache rows of 1e6 in front of the prompt (scales of the attention output).  Rows are held to 2e-5 of their largest entry:
+    2^-24 per operand, 2^-22 per product, some hundred roundings to fp32 behind them.  What lies far below the largest entry
+    is held by test_pair_exact_gpu.py."""
     spec = dataclasses.replace(SPECS[name], seq_len=512)
     img = binfmt.synth_image(spec, seed=33, device=gpu)
     for e in binfmt.layout(spec)[0]:
