@@ -570,8 +570,8 @@ def measure(spec, args, rank, world, local_rank, primary):
                 out["prefill"][names[mode] + "_tok_s"] = len(pp) / (ms * 1e-3)
         if pf.get("gemm") and pf.get("token"):
             out["prefill"]["speedup_gemm_vs_token"] = pf["token"] / pf["gemm"]
-        # longer prompts: one weight pass takes up to 512 tokens (the small-M GEMMs then get the big
-        # register tile), 1024 = two such passes with causal attention over up to 1024 timesteps
+        # longer prompts: one weight pass takes up to 2048 tokens (the small-M GEMMs then get the big
+        # register tile), with causal attention over up to 1024 timesteps
         if pf.get("gemm"):
             for n in (512, 1024):
                 if spec.seq_len < n:
@@ -583,8 +583,9 @@ def measure(spec, args, rank, world, local_rank, primary):
                     out["prefill"][f"mfma_gemm_{n}_prompt_tok_s"] = len(lp) / (ms * 1e-3)
                 except Exception as e:  # noqa: BLE001
                     log(f"[bench] {n}-token prefill: {e!r}")
-        out["prefill"]["note"] = ("mfma_gemm: fp32-MFMA GEMMs + MFMA causal attention, weights streamed once per "
-                                  "pass of up to 512 prompt tokens (prompt_tokens = 128: one 128-token pass), fp32 "
+        out["prefill"]["note"] = ("mfma_gemm: GEMMs and causal attention on the fp16 matrix cores with operands as pairs of "
+                                  "halves (fp32 accuracy; int8 weights exact in one), weights streamed once per pass of up "
+                                  "to 2048 prompt tokens (prompt_tokens = 128: one 128-token pass), fp32 "
                                   "tolerance vs the oracle; b_token_gemv: 8/4 tokens per weight pass on the VALU, "
                                   "bit-identical to token_by_token (the reference's prompt phase)")
     # per-kernel durations measured live with HIP events on the model's stream.  The roofline

@@ -184,7 +184,7 @@ typedef struct kh_model_opts {
 #define KH_FLAG_ATTN_MERGE_FENCED 2
 /* The prompt phase of kh_model_generate*.  The reference feeds the prompt one token per forward pass
  * (demo/main.cpp:20-22), so its prompt phase is, bit for bit, its decode path.  Two batched prompt paths exist here:
- *  - default: prompts with >= 16 fed-only tokens run as GEMMs on the matrix cores (kh_model_prefill_gemm, 63-130 k
+ *  - default: prompts with >= 16 fed-only tokens run as GEMMs on the matrix cores (kh_model_prefill_gemm, 62-158 k
  *    prompt tokens/s on Llama-3.2-1B): K/V rows equal to fp32 round-off, i.e. the greedy continuation can differ from the
  *    reference's at near-ties (kh_model_first_sample reports the margin of the first sampled step);
  *  - KH_FLAG_PREFILL_EXACT: every prompt runs on the B-token VALU kernels (kh_model_prefill, 5.9 k prompt
@@ -220,7 +220,8 @@ int kh_model_create_from_host_image(const void* h_image, size_t nbytes,
                                     const kh_model_opts* opts, kh_model** out);
 /* weights already resident in HBM: h_header = the 7 (fp32) or 8 (int8) header ints,
  * d_weight_data = the file bytes AFTER the header, 16-byte aligned, not owned
- * (the reference's "external buffer", layer.cpp:190-202). */
+ * (the reference's "external buffer", layer.cpp:190-202).  It is read by every call and may be written between two calls
+ * (cache rows computed before keep the old weights' values). */
 int kh_model_create_from_device_weights(const int32_t* h_header, const void* d_weight_data,
                                         size_t weight_nbytes, const kh_model_opts* opts,
                                         kh_model** out);
@@ -404,7 +405,7 @@ int64_t kh_debug_list(char* buf, int64_t cap); /* '\n'-separated names; returns 
 /* Duration (ms, HIP events on the model stream) of the prompt phase alone for n fed-only tokens:
  * KH_PREFILL_TOKEN = the reference's prompt phase, one forward pass per token (demo/main.cpp:20-22)
  * replayed from the decode hipGraph; KH_PREFILL_GEMV = kh_model_prefill's bit-identical B-token
- * kernels; KH_PREFILL_GEMM = the fp32-MFMA GEMM prefill.  Leaves the K/V rows of those positions. */
+ * kernels; KH_PREFILL_GEMM = kh_model_prefill_gemm.  Leaves the K/V rows of those positions. */
 enum { KH_PREFILL_TOKEN = 0, KH_PREFILL_GEMV = 1, KH_PREFILL_GEMM = 2 };
 int kh_model_time_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t pos0,
                           int32_t mode, float* h_ms);

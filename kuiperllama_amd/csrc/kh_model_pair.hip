@@ -16,10 +16,14 @@ namespace {
 // Tile and K split of one GEMM from a model of the busiest CU: a workgroup's stage takes at least `lat` (one or more stages
 // in flight against memory latency), and `n` workgroups side by side on a CU take n `sat` per stage together.  Both numbers
 // (us) were fitted to 18 tile / split combinations of the four GEMMs of Llama-3.2-1B fp32 and Llama-2-7B int8 at 40 ... 2000
-// tokens: the choice is on average 0.6 % (fp32) and 0.3 % (int8) behind the fastest combination measured, 5 % at worst.
+// tokens: the choice was on average 0.6 % (fp32) and 0.3 % (int8) behind the fastest combination measured, 5 % at worst.  They
+// belong to the tile and the 256 CUs, not to a model; other widths take them as they are.
+// The largest tile of a type is the largest whose registers do not spill: 8 x 2 fragments a wave for fp32, 7 x 2 (112
+// tokens) for int8, where 8 x 2 spills 18 to 24 registers, the sums of a 64-column group standing beside the accumulators.
 // Against the tiled fp32-MFMA kernel (k_pg_gemm), us at 40 / 128 / 512 / 2000 tokens, w1 + w3 of either model:
-// 34 / 45 / 102 / 376 against 46 / 76 / 287 / 1089 (fp32); 55 / 85 / 222 / 767 against 126 / 210 / 792 / 3032 (int8).
-// Only wq + wk + wv of 64 fp32 tokens or less were faster there (18 us against 24).
+// 38 / 48 / 108 / 388 against 46 / 76 / 287 / 1089 (fp32); 56 / 88 / 232 / 816 against 126 / 210 / 792 / 3032 (int8).
+// Only wq + wk + wv of 64 fp32 tokens or less were faster there (18 us against 24); whole prompts of 32 tokens and less take
+// 0.67 to 0.94 of its time, on Llama-3.2-1B 1.03.
 struct PairShape {
   int tile;  // index into kPairTiles
   int kz;    // K slices across workgroups (residual GEMMs)
@@ -165,9 +169,9 @@ size_t pa_bytes(const kh_config& c, int positions) {
 
 // Attention of a slice with its operands as pairs; false: the caller takes pg_slice_attention (fp32 matrix cores).
 // Packing reads all of the layer's rows whatever T is, so it needs enough query tokens and enough work.  Whole prompt
-// passes, ms, fp32 matrix cores against pairs, T @ first position: Llama-3.2-1B 128 @ 0 1.98 / 2.00, 256 @ 0 2.68 / 2.68,
-// 512 @ 0 4.05 / 3.94, 64 @ 2048 2.05 / 2.05, 256 @ 2048 3.42 / 3.06, 2048 @ 2048 20.3 / 14.6; Llama-2-7B int8
-// 128 @ 0 7.07 / 7.13, 256 @ 0 10.5 / 10.3, 128 @ 1024 8.08 / 7.83, 1024 @ 1024 41.5 / 34.5.
+// passes, ms, fp32 matrix cores against pairs, T @ first position: Llama-3.2-1B 256 @ 0 2.78 / 2.79, 512 @ 0 4.14 / 4.03,
+// 256 @ 2048 3.45 / 3.11, 2048 @ 2048 18.8 / 14.2; Llama-2-7B int8 256 @ 0 10.7 / 10.6, 128 @ 1024 8.35 / 8.19,
+// 1024 @ 1024 41.8 / 35.2.  128 @ 0 and 64 @ 2048 gain nothing.
 bool pa_pays(int T, int pos0) {
   if (dbg_off("KH_PG_ATTN") || dbg("KH_PG_ATTN_QT") || dbg_off("KH_PAIR_ATTN")) return false;
   return T >= 128 && (size_t)T * (2 * (size_t)pos0 + T) >= 65536;

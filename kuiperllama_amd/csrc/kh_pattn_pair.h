@@ -17,11 +17,10 @@
 //
 // Q is split once per workgroup and kept in LDS; K and V of the next block are requested when the last product of the
 // present one has read them: held twice they would not leave room for two waves per SIMD, which cover one another's softmax.
-// Bound by the softmax and the matrix cores about evenly.  Two query tiles for heads of 48 and 64 (one: 13.37 instead of
-// 13.14 ms for 1899 tokens of TinyLlama; four: 12.88 instead of 12.84, fewer workgroups for short prompts; eight waves
-// instead of four 13.14), one for 128 (two spill).  Attention of one layer, us, fp32 matrix cores -> pack + attention:
-// TinyLlama, 1899 tokens 187 -> 5.2 + 70; Llama-2-7B, 776 tokens 106 -> 10.1 + 39; Llama-3.2-1B, 511 tokens 23.5 -> 5.1 + 10.8.
-// Logits against 64 bits, rms of three prompts: TinyLlama, 1900 tokens 1.27e-6 -> 1.05e-6, Llama-3.2-1B, 512 1.48e-6 -> 1.03e-6.
+// Bound by the softmax and the matrix cores about evenly.  Two query tiles for heads of 48 and 64 (one was 2 % slower over a
+// whole prompt of 1899 tokens of TinyLlama, four 0.3 %, with fewer workgroups for short prompts; eight waves instead of four
+// 2 %), one for 128 (two spill).  Attention of one layer, us, fp32 matrix cores -> pack + attention: TinyLlama, 1899 tokens
+// 187 -> 5.1 + 70; Llama-2-7B, 776 tokens 106 -> 10.8 + 40; Llama-3.2-1B, 512 tokens 23.5 -> 5.0 + 11.5.
 #pragma once
 #include "kh_pair.h"
 
