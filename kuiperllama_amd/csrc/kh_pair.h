@@ -250,7 +250,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   for (int n = 0; n < TN; ++n)
 #pragma unroll
     for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Scales are requested 16 stages ahead of their first use, those of a slice's second 16 with the first: a slice may begin at
+  // the end of 16 stages, and stage k only waits for what was requested NST - 2 stages before it.
+  static_assert(NST - 2 < 16, "scales have landed when they are read");
   issue_exps(z0 >> 4);
+  if (((z0 >> 4) + 1) * 16 < z1) issue_exps((z0 >> 4) + 1);
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s)
     if (s < nk) issue(s);
@@ -297,7 +301,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     else wait_vm<0>();
     __syncthreads();
     const int at = z0 + k;
-    if (GROUP && (k == 0 || (at & 15) == 0) && ((at >> 4) + 1) * 16 < z1) issue_exps((at >> 4) + 1);
+    if (GROUP && k > 0 && (at & 15) == 0 && ((at >> 4) + 1) * 16 < z1) issue_exps((at >> 4) + 1);
     const unsigned char* exps = (const unsigned char*)smem_raw + NST * C::STAGE + ((at >> 4) & 1) * C::EX * 1024 + (at & 15);
     if (k + NST - 1 < nk) issue(fill);
     const char* st = smem_raw + slot * C::STAGE;

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import exact_kv
-from kuiperllama_amd import binfmt
+from kuiperllama_amd import _ffi, binfmt
 from test_model_gpu import _PF_SPECS
 
 pytestmark = pytest.mark.gpu
@@ -203,6 +203,32 @@ _WIDTHS = {
 def test_widths(gpu, name, n, monkeypatch):
     spec = _WIDTHS[name]
     img = binfmt.synth_image(spec, seed=57, device=gpu)
+    pair, fp32 = errors(monkeypatch, img, spec, n)
+    print(f"{name}, {n} tokens: {pair:.3g} with pairs, {fp32:.3g} without")
+    assert pair <= 1.25 * fp32
+
+
+_SLICES = {
+    # wo in four slices: the second begins at stage 14 of the 16 whose scales travel together (Qwen2.5-0.5B up to 128 tokens)
+    "fp32": (binfmt.ModelSpec(896, 1792, 2, 14, 2, 500, 512, True, binfmt.FAMILY_LLAMA, False, 64, binfmt.ROPE_HALF, 10000.0, 1e-5,
+                              "slices"), None),
+    # w2 in four slices that begin at stages 15, 31 and 47
+    "int8": (binfmt.ModelSpec(512, 4032, 2, 8, 2, 500, 512, False, binfmt.FAMILY_LLAMA, True, 64, binfmt.ROPE_HALF, 10000.0, 1e-5,
+                              "slices8"), "2,4"),
+}
+
+
+@pytest.mark.parametrize("name", sorted(_SLICES))
+@pytest.mark.parametrize("n", [16, 41, 128])
+def test_slices_that_begin_behind_the_first_scales(gpu, name, n, monkeypatch):
+    """A K slice whose second stages need the next 16 scales: those have landed too."""
+    spec, shape = _SLICES[name]
+    if shape:
+        monkeypatch.setenv("KH_PAIR_SHAPE", shape)
+    else:
+        plan = _ffi.plan_pair_shapes(spec.dim, spec.hidden_dim, spec.kv_dim, False, n)["wo"]
+        assert (plan["bm"], plan["bn"], plan["kz"]) == (32, 64, 4)
+    img = binfmt.synth_image(spec, seed=59, device=gpu)
     pair, fp32 = errors(monkeypatch, img, spec, n)
     print(f"{name}, {n} tokens: {pair:.3g} with pairs, {fp32:.3g} without")
     assert pair <= 1.25 * fp32
