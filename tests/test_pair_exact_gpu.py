@@ -1,5 +1,7 @@
 """Prompt passes on pairs of halves (csrc/kh_pair.h) against 64 bits, with weights whose sizes differ by powers of two that
 cancel over two matrices: the rows are held to the error of the fp32 matrix cores on the same weights (KH_PG_PAIR=0)."""
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -187,6 +189,28 @@ def test_weights_written_in_place(gpu, name):
             assert np.isfinite(a).all() and np.array_equal(a, b), l
     m.close()
     fresh.close()
+
+
+def test_uneven_rows_cost_a_second_pass(gpu):
+    """Rows with one number far above their first 32 columns: the waves that meet them compute their tiles a second time
+    behind a search for the scales: 1.9 to 2.2 times the time of even rows; 3.3 with one request in flight."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = dataclasses.replace(binfmt.PRESETS["llama3.2-1b"], n_layers=3, vocab_size=2000, seq_len=1024)
+    toks = [int(t) for t in np.random.default_rng(25).integers(0, spec.vocab_size, 512)]
+    ms = []
+    for uneven in (False, True):
+        img = binfmt.synth_image(spec, seed=60, device=gpu)
+        t = exact_kv.tensors(img, spec)
+        for l in range(spec.n_layers if uneven else 0):
+            for n in ("wq", "wk", "wv", "wo", "w1", "w3", "w2"):
+                w = t[f"{n}.{l}"]
+                w[7::100, 1000] = 200 * w.abs().max()
+        m = KuiperModel.from_device_image(img, spec)
+        m.time_prefill(toks, 0)
+        ms.append(min(m.time_prefill(toks, 0) for _ in range(8)))
+        m.close()
+    print(f"{ms[0]:.3f} ms, with uneven rows {ms[1]:.3f}")
+    assert ms[1] < 2.6 * ms[0]
 
 
 _WIDTHS = {
