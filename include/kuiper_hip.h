@@ -184,7 +184,7 @@ typedef struct kh_model_opts {
 #define KH_FLAG_ATTN_MERGE_FENCED 2
 /* The prompt phase of kh_model_generate*.  The reference feeds the prompt one token per forward pass
  * (demo/main.cpp:20-22), so its prompt phase is, bit for bit, its decode path.  Two batched prompt paths exist here:
- *  - default: prompts with >= 16 fed-only tokens run as GEMMs on the matrix cores (kh_model_prefill_gemm, 62-158 k
+ *  - default: prompts with >= 16 fed-only tokens run as GEMMs on the matrix cores (kh_model_prefill_gemm, 58-158 k
  *    prompt tokens/s on Llama-3.2-1B): K/V rows equal to fp32 round-off, i.e. the greedy continuation can differ from the
  *    reference's at near-ties (kh_model_first_sample reports the margin of the first sampled step);
  *  - KH_FLAG_PREFILL_EXACT: every prompt runs on the B-token VALU kernels (kh_model_prefill, 5.9 k prompt
