@@ -335,7 +335,8 @@ int kh_model_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t po
  * passes of up to 512 tokens, int8 weights dequantised per element in registers).  Either way nothing about the weights is
  * kept between calls: memory given to kh_model_create_from_device_weights may be written between them.  The K/V rows agree
  * with the token-by-token path to fp32 round-off (different summation order), not bit for bit.
- * kh_model_generate* use it for prompts with >= 16 fed-only tokens unless the model was created with
+ * kh_model_generate* use it for prompts with >= 16 fed-only tokens (and take the prompt's last token through every layer
+ * but the last with them, where that is cheaper than a step of its own) unless the model was created with
  * KH_FLAG_PREFILL_EXACT - so for such prompts the greedy tokens carry this tolerance too and can differ from the
  * token-by-token prompt phase at near-ties;
  * hook KH_PREFILL = 0 | token | gemv | gemm overrides (gemv = the bit-identical path; any other

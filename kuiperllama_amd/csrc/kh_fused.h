@@ -545,13 +545,13 @@ static __global__ __launch_bounds__(KH_WG) void k_sample(const KhSampleArgs a) {
 
 // set (token, pos) from the host and gather the embedding row: start of generate / predict
 static __global__ __launch_bounds__(KH_WG) void k_set_state(int token, int pos, int32_t* d_token,
-                                                     int32_t* d_pos, const float* tok_emb,
+                                                     int32_t* d_pos, const float* row,
                                                      float* x, int dim) {
   if (threadIdx.x == 0) {
     *d_token = token;
     *d_pos = pos;
   }
-  const f32x4* src = (const f32x4*)(tok_emb + (size_t)token * dim);
+  const f32x4* src = (const f32x4*)row;
   f32x4* dst = (f32x4*)x;
   for (int i = threadIdx.x; i < (dim >> 2); i += KH_WG) dst[i] = src[i];
 }

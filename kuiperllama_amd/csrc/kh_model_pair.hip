@@ -36,7 +36,7 @@ const PairTile kPairTiles[2][4] = {
     {{128, 128, 2, 1.44, 0.73}, {64, 128, 2, 0.57, 0.445}, {32, 128, 2, 0.40, 0.315}, {32, 64, 2, 0.20, 0.30}},  // fp32
     {{112, 128, 2, 1.22, 0.95}, {64, 128, 2, 0.72, 0.63}, {32, 128, 2, 0.53, 0.42}, {128, 256, 1, 1.95, 1.95}}};  // int8
 
-PairShape pair_shape(bool q, int T, int N, int K, bool resid) {
+PairShape pair_shape(bool q, int T, int N, int K, bool resid, double* time_us = nullptr) {
   PairShape best{0, 1};
   double best_us = -1.0;
   for (int i = 0; i < 4; ++i)
@@ -55,7 +55,15 @@ PairShape pair_shape(bool q, int T, int N, int K, bool resid) {
         best = PairShape{i, kz};
       }
     }
+  if (time_us) *time_us = best_us;
   return best;
+}
+// the four GEMMs of a layer
+struct PairDims {
+  int N[4], K[4];
+};
+PairDims pair_dims(const kh_config& c) {
+  return {{c.dim + 2 * c.kv_dim, c.dim, 2 * c.hidden_dim, c.dim}, {c.dim, c.dim, c.dim, c.hidden_dim}};
 }
 
 template <bool Q, int EPI, int TM, int TN, int WM, int WN, int NST>
@@ -117,15 +125,15 @@ extern "C" int kh_plan_pair_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_d
   c.kv_dim = kv_dim;
   c.is_quant = is_quant != 0;
   if (!pair_geometry(c)) return KH_ERR_UNSUPPORTED;
-  const int N[4] = {dim + 2 * kv_dim, dim, 2 * hidden_dim, dim}, K[4] = {dim, dim, dim, hidden_dim};
+  const PairDims d = pair_dims(c);
   for (int i = 0; i < 4; ++i) {
-    const PairShape s = pair_shape(c.is_quant, T, N[i], K[i], i & 1);
+    const PairShape s = pair_shape(c.is_quant, T, d.N[i], d.K[i], i & 1);
     const PairTile& t = kPairTiles[c.is_quant][s.tile];
     int32_t* o = out16 + 4 * i;
     o[0] = t.bm;
     o[1] = t.bn;
     o[2] = s.kz;
-    o[3] = (N[i] + t.bn - 1) / t.bn * ((T + t.bm - 1) / t.bm) * s.kz;
+    o[3] = (d.N[i] + t.bn - 1) / t.bn * ((T + t.bm - 1) / t.bm) * s.kz;
   }
   return KH_OK;
 }
@@ -137,6 +145,26 @@ bool pair_geometry(const kh_config& c) {
   const int g = c.is_quant ? 64 : 32;
   const int64_t wide = std::max(c.dim, c.hidden_dim), lim = (int64_t)1 << 32;
   return c.dim % g == 0 && c.hidden_dim % g == 0 && wide * c.dim * (c.is_quant ? 1 : 4) <= lim && wide * KH_PAIR_TMAX * 4 <= lim;
+}
+
+// Is the last of T tokens of a pass cheaper in the pass than as a step of its own?  The step reads a layer's weights once more
+// (5 TB/s behind 10 us of launches a layer); in the pass the token may open another row of tiles, and where the model of
+// pair_shape sees a near tie the step was faster.  Time to the first token, ms, step of its own / in the pass, T tokens:
+// Llama-3.2-1B 17 2.62 / 1.88, 193 3.75 / 2.99, 512 5.18 / 4.37, 641 6.45 / 5.96; Qwen2.5-0.5B 41 2.35 / 1.79; TinyLlama 1793
+// 13.9 / 13.2; Llama-2-7B int8 33 6.28 / 5.10, 225 12.1 / 10.7, 561 21.1 / 21.3 (the one length measured where the rule errs);
+// not taken: Llama-3.2-1B 513 5.18 / 5.43, 1025 8.10 / 9.05; Llama-2-7B int8 65 6.83 / 7.07, 449 17.1 / 17.3.
+bool pair_takes_last(const kh_config& c, int T) {
+  if (T < 2) return false;
+  const PairDims d = pair_dims(c);
+  double more = 0.0, bytes = 0.0;
+  for (int i = 0; i < 4; ++i) {
+    double with = 0.0, without = 0.0;
+    (void)pair_shape(c.is_quant, T, d.N[i], d.K[i], i & 1, &with);
+    (void)pair_shape(c.is_quant, T - 1, d.N[i], d.K[i], i & 1, &without);
+    more += with - without;
+    bytes += (double)d.N[i] * d.K[i] * (c.is_quant ? 1 : 4);
+  }
+  return more < 0.8 * (10.0 + bytes / 5.0e6);
 }
 
 int pair_part_rows(const kh_config& c, int rows) {
@@ -259,7 +287,8 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
       a.X = xn; a.out = m->pg_q;
       a.kc = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
       a.vc = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
-      a.rows0 = c.dim; a.rows1 = c.kv_dim; a.N = c.dim + 2 * c.kv_dim; a.ldo = c.dim; a.K = c.dim;
+      a.rows0 = l == c.layer_num - 1 ? 0 : c.dim;  // nobody asks for the last layer's queries
+      a.rows1 = c.kv_dim; a.N = a.rows0 + 2 * c.kv_dim; a.ldo = c.dim; a.K = c.dim;
       a.rope = !rope_fuse ? KH_PG_ROPE_OFF
                : (c.rope_mode == KH_ROPE_HALF ? (c.head_size % 32 == 0 ? KH_PG_ROPE_TILES : KH_PG_ROPE_OFF) : KH_PG_ROPE_PAIRS);
       if ((rc = pair_launch<KH_PG_QKV>(m, a, nullptr)) != KH_OK) return rc;

@@ -588,14 +588,13 @@ extern "C" int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32
   return KH_OK;
 }
 
-extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t pos0) {
-  if (!m || !h_tokens || n <= 0 || pos0 < 0) return KH_ERR_INVALID_ARG;
+int khm::prefill_gemm(kh_model* m, const int32_t* h_tokens, int n, int pos0, const float** last) {
   const kh_config& c = m->cfg;
-  if ((int64_t)pos0 + n > c.cache_len) return KH_ERR_RANGE;
-  for (int i = 0; i < n; ++i)
-    if (h_tokens[i] < 0 || h_tokens[i] >= c.vocab_size) return KH_ERR_RANGE;
-  if (!pg_supported(m)) return KH_ERR_UNSUPPORTED;
-  KH_CHECK_HIP(hipSetDevice(m->opts.device));
+  const bool pair = pg_pair(m);
+  if (last) {
+    *last = nullptr;
+    if (m->hy || !pair) last = nullptr, --n;
+  }
   int rc;
   if ((rc = kv_ensure(m, pos0 + n)) != KH_OK) return rc;
   if (m->hy) {
@@ -605,23 +604,35 @@ extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32
   if ((rc = ensure_pg_buffers(m, n)) != KH_OK) return rc;
   if ((rc = ensure_pg_ws(m)) != KH_OK) return rc;
   m->pg_launch_failed = false;
-  const bool pair = pg_pair(m);
   // tuning / test hook: KH_PG_CHUNK=<tokens per weight pass> (16 .. KH_PG_TMAX), read per call
   int chunk = pair && pg_mfma_attn(m) ? m->pg_rows : KH_PG_TMAX;
   if (const char* e = dbg("KH_PG_CHUNK")) {
     const int v = atoi(e);
     chunk = v < 16 ? 16 : (v > KH_PG_TMAX ? KH_PG_TMAX : v);
   }
+  if (last && !pair_takes_last(c, (n - 1) % chunk + 1)) last = nullptr, --n;
   if (pair) {
     pair_prepare(m, n, pos0);
     for (int t0 = 0; t0 < n; t0 += chunk)
       if ((rc = launch_prefill_pair_chunk(m, h_tokens + t0, n - t0 < chunk ? n - t0 : chunk, pos0 + t0)) != KH_OK) return rc;
+    if (last) *last = m->pg_x + (size_t)((n - 1) % chunk) * c.dim;
     return kh_launch_status();
   }
   for (int t0 = 0; t0 < n; t0 += chunk)
     launch_prefill_gemm_chunk(m, h_tokens + t0, n - t0 < chunk ? n - t0 : chunk, pos0 + t0);
   if (m->pg_launch_failed) return KH_ERR_UNSUPPORTED;  // a GEMM shape's LDS opt-in was refused
   return kh_launch_status();
+}
+
+extern "C" int kh_model_prefill_gemm(kh_model* m, const int32_t* h_tokens, int32_t n, int32_t pos0) {
+  if (!m || !h_tokens || n <= 0 || pos0 < 0) return KH_ERR_INVALID_ARG;
+  const kh_config& c = m->cfg;
+  if ((int64_t)pos0 + n > c.cache_len) return KH_ERR_RANGE;
+  for (int i = 0; i < n; ++i)
+    if (h_tokens[i] < 0 || h_tokens[i] >= c.vocab_size) return KH_ERR_RANGE;
+  if (!pg_supported(m)) return KH_ERR_UNSUPPORTED;
+  KH_CHECK_HIP(hipSetDevice(m->opts.device));
+  return prefill_gemm(m, h_tokens, n, pos0, nullptr);
 }
 
 // Operator-level entry of the MFMA slice attention (kh_pattn.h): the multi-token form of MHAKernel.

@@ -409,6 +409,19 @@ int step_variant(const kh_model* m, int pos_lo, int pos_hi) {
   // (head, split) workgroups at position 4094 +3.6 us per layer (profiles/r4_attn_pipe_ab.txt); per-head-only: 115.
   return m->attn_ns_g > 0 ? 2 : 0;
 }
+template <class F>
+static void launch_layer(kh_model* m, int l, F&& mark) {
+  launch_qkv(m, l);
+  mark();
+  launch_attn(m, l);
+  mark();
+  launch_wo(m, l);
+  mark();
+  launch_ffn13(m, l);
+  mark();
+  launch_w2(m, l);
+  mark();
+}
 // one fused decode step = 5L + 2 launches.  ev (optional) receives an event after each launch.
 void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant) {
   if (m->hy) return hy_launch_step(m, advance, n_forced);
@@ -418,18 +431,7 @@ void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, i
     if (ev) (void)hipEventRecord(ev[e++], m->stream);
   };
   mark();
-  for (int l = 0; l < m->cfg.layer_num; ++l) {
-    launch_qkv(m, l);
-    mark();
-    launch_attn(m, l);
-    mark();
-    launch_wo(m, l);
-    mark();
-    launch_ffn13(m, l);
-    mark();
-    launch_w2(m, l);
-    mark();
-  }
+  for (int l = 0; l < m->cfg.layer_num; ++l) launch_layer(m, l, mark);
   launch_cls(m);
   mark();
   launch_sample(m, advance, n_forced);
@@ -484,8 +486,19 @@ int launch_step_unfused(kh_model* m, int pos) {
 }
 
 void set_state(kh_model* m, int token, int pos) {
-  hipLaunchKernelGGL(k_set_state, dim3(1), dim3(KH_WG), 0, m->stream, token, pos, m->d_token,
-                     m->d_pos, m->tok_emb, m->x, m->hy ? 0 : m->cfg.dim);  // layer lists gather it in their first kernel
+  const int dim = m->hy ? 0 : m->cfg.dim;  // layer lists gather it in their first kernel
+  hipLaunchKernelGGL(k_set_state, dim3(1), dim3(KH_WG), 0, m->stream, token, pos, m->d_token, m->d_pos,
+                     m->tok_emb + (size_t)token * dim, m->x, dim);
+}
+
+// The step of a prompt's last token behind a prompt pass that took it through every layer but the last (prefill_gemm): `row`
+// is its residual there.  It reads one layer's weights and the classifier instead of all of them.
+static void launch_tail_step(kh_model* m, int token, int pos, const float* row, int n_forced) {
+  hipLaunchKernelGGL(k_set_state, dim3(1), dim3(KH_WG), 0, m->stream, token, pos, m->d_token, m->d_pos, row, m->x, m->cfg.dim);
+  m->step_var = step_variant(m, pos, pos);
+  launch_layer(m, m->cfg.layer_num - 1, [] {});
+  launch_cls(m);
+  launch_sample(m, 1, n_forced);
 }
 
 int ensure_pinned_words(kh_model* m, int n) {
@@ -818,6 +831,7 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
   //                  on, "gemv" below that
   // any other value is an error (KH_ERR_INVALID_ARG), not a silent choice.
   int start = 0;
+  const float* last_row = nullptr;  // the prompt pass went through with the prompt's last token as well
   KH_CHECK_HIP(hipEventRecord(m->ev0, m->stream));
   if (n_prompt - 1 >= 2 && n_prompt - 1 < total_steps) {
     const char* e = dbg("KH_PREFILL");
@@ -829,7 +843,7 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
       else return KH_ERR_INVALID_ARG;
     }
     if (want_gemm && pg_supported(m)) {
-      if ((rc = kh_model_prefill_gemm(m, h_prompt, n_prompt - 1, 0)) != KH_OK) return rc;
+      if ((rc = prefill_gemm(m, h_prompt, n_prompt, 0, &last_row)) != KH_OK) return rc;
       start = n_prompt - 1;
       m->first_mode = 2;
     } else if (want_gemv && prefill_supported(m)) {
@@ -845,8 +859,13 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
     if (!m->first_logits) KH_CHECK_HIP(hipMalloc(&m->first_logits, sizeof(float) * (size_t)c.vocab_size));
     m->first_pos = start;
   }
-  set_state(m, h_prompt[start], start);
+  if (!last_row) set_state(m, h_prompt[start], start);
   auto launch_chunk = [&](int s) -> int {  // enqueue the next 1 or KH_GRAPH_STEPS steps (positions s ..)
+    if (s == start && last_row) {
+      launch_tail_step(m, h_prompt[s], s, last_row, n_forced);
+      return hipMemcpyAsync(m->first_logits, m->logits, sizeof(float) * (size_t)c.vocab_size, hipMemcpyDeviceToDevice,
+                            m->stream) == hipSuccess ? 1 : -1;
+    }
     if (exec == KH_EXEC_GRAPH) {
       // the largest of 8 / 4 / 2 / 1 steps that still fits (a single-step launch costs ~15 us of graph-launch gap:
       // the 20-step form of the bench ran 8 + 8 + 1 + 1 + 1 + 1 and lost 0.3 % to it; now 8 + 8 + 4)

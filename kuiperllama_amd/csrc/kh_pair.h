@@ -24,6 +24,7 @@
 // 512 / 1900 tokens as without, 1.8 / 0.95 / 0.7 times as long as on the fp32 matrix cores.  (With one request in flight in
 // the second way and in the search for the scales: 3.5 / 3.3 / 3.2 times as long as without.  The workgroup once more through
 // its ring, decided by a vote: 2.35 / 2.0 / 1.95, and 1 % slower where nothing overflows.)
+// Where the last token of a prompt is in the pass (pair_takes_last), logits come from it: see fold.
 // K/V rows of models of eight layers and 400 tokens, rms against 64 bits: 4.3e-7 (int8), 5.6e-7 (fp32); on the fp32 matrix
 // cores 1.2e-6 and 1.3e-6.  That needs numbers that weigh alike in a result to lie within about 2^12 of one another where
 // they share a scale.
@@ -177,10 +178,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       }
     }
   };
+  // Row r of the tile -> token: as it comes, but for the last tile, whose 16-row tiles turn within a wave until the last token
+  // lies in the last of them: that one's sums are kept longer (fold).
+  const int turn = t0 + C::BM < a.T ? 0 : ((a.T - 1 - t0) >> 4) + 1;
+  auto token_of = [&](int r) __attribute__((always_inline)) {
+    const int m = r >> 4;
+    return t0 + ((m / TM * TM + (m + turn) % TM) << 4) + (r & 15);
+  };
   // ---- staging addresses
   static_assert(TN % 2 == 0, "both tiles of a SWIGLU or half-mode RoPE pair lie in one wave");
   constexpr int NX = C::XR / C::NW, NWR = C::WR / C::NW;
-  unsigned xoff[NX], woff[NWR];
+  unsigned xoff[NX], woff;  // per lane; the rows of a wave's weight requests differ by their bases
   const char* wbase[NWR];
   const char* sbase = nullptr;
   const int sub = lane >> 3, ch8 = (lane & 7) ^ pair_swz(sub);
@@ -191,7 +199,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
 #pragma unroll
   for (int j = 0; j < NX; ++j) {
     const int r = 8 * (j * C::NW + wave) + sub;  // LDS row: block-major for int8
-    int t = t0 + (Q ? r % C::BM : r);
+    int t = token_of(Q ? r % C::BM : r);
     t = t < a.T ? t : a.T - 1;
     xoff[j] = (unsigned)t * (unsigned)(4 * K) + (Q ? (unsigned)(r / C::BM) * 128u : 0u) + 16u * ch8 + (unsigned)z0 * (128u * C::XB);
   }
@@ -202,13 +210,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     f = f < a.N - run ? f : a.N - run;
     int mat, row;
     place(f, mat, row);
-    wbase[j] = (const char*)a.w[mat].w;
-    if (Q) {
-      const int rr = lane >> 2, ch = (lane & 3) ^ ((rr & 4) >> 1);
-      woff[j] = (unsigned)(row + rr) * (unsigned)K + 16u * ch + (unsigned)z0 * 64u;
-    } else {
-      woff[j] = (unsigned)(row + sub) * (unsigned)(4 * K) + 16u * ch8 + (unsigned)z0 * 128u;
-    }
+    wbase[j] = (const char*)a.w[mat].w + ((size_t)(unsigned)row * (unsigned)K + (unsigned)z0 * (Q ? 64u : 32u)) * (Q ? 1 : 4);
+  }
+  if (Q) {
+    const int rr = lane >> 2, ch = (lane & 3) ^ ((rr & 4) >> 1);
+    woff = (unsigned)rr * (unsigned)K + 16u * ch;
+  } else {
+    woff = (unsigned)sub * (unsigned)(4 * K) + 16u * ch8;
   }
   if (Q) {  // scales of 64 places: one dword a lane (SWIGLU and RoPE runs of 16 may lie in two matrices: 64-bit addresses)
     int f = f0 + 64 * (wave % (C::SR ? C::SR : 1)) + lane;
@@ -223,8 +231,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     const unsigned d = lds0 + (unsigned)(slot * C::STAGE);
 #pragma unroll
     for (int j = 0; j < NWR; ++j) {
-      dma_x4_keep(wbase[j], woff[j], d + (unsigned)(C::XR * 1024 + j * C::NW * 1024));
-      woff[j] += Q ? 64 : 128;
+      dma_x4_keep(wbase[j], woff, d + (unsigned)(C::XR * 1024 + j * C::NW * 1024));
+      wbase[j] += Q ? 64 : 128;
     }
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
@@ -239,11 +247,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     }
   };
   // The scales of 16 stages: 16 bytes a token.  A request per stage (four bytes a token) made these GEMMs 5 % slower.
-  const int et = t0 + 64 * wave + lane;
-  const unsigned eoff = 16u * (unsigned)(et < a.T ? et : a.T - 1);
   auto issue_exps = [&](int c) __attribute__((always_inline)) {
-    if (GROUP && wave < C::EX)
-      dma_x4_keep(a.xe + (size_t)c * a.xe_ld * 16, eoff, lds0 + (unsigned)(NST * C::STAGE + (c & 1) * C::EX * 1024));
+    if (!GROUP || wave >= C::EX) return;
+    int r = 64 * wave + lane;
+    asm volatile("" : "+v"(r));  // or the offset takes a register throughout the loop
+    const int t = token_of(r);
+    const unsigned eoff = 16u * (unsigned)(t < a.T ? t : a.T - 1);
+    dma_x4_keep(a.xe + (size_t)c * a.xe_ld * 16, eoff, lds0 + (unsigned)(NST * C::STAGE + (c & 1) * C::EX * 1024));
   };
   const int nk = z1 - z0;
   f32x4 acc[TN][TM];
@@ -267,6 +277,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   // The matrix unit rounds its sums down: a bias that the mean over many cached rows keeps while it averages everything else
   // (logits behind 1900 prompt tokens: 1.7e-6 from 64 bits instead of 1.3e-6 on fp32 fma chains).  Every other group takes
   // its weights with the sign turned and is subtracted, which cancels it: 1.1e-6.
+  // Every group's sum is folded into the accumulators with one rounding of them, the largest error of a long dot product.
+  // For the last 16 tokens of a wave it is kept and added at the end (lost): the logits behind the prompt come from the last
+  // token, while the rows of the others are averaged over by those that attend to them.  Logits from 64 bits (mean of six
+  // models), steps of their own on fp32 fma chains / in the pass without this / with it, Llama-3.2-1B 40, 150, 512 tokens:
+  // 1.20 1.17 1.08e-6 / 1.29 1.36 1.23 / 1.02 1.13 1.00; Qwen2.5-0.5B 300: 7.1e-7 / - / 7.5; Llama-2-7B int8 60, 225: 3.7
+  // 3.4e-6 / 3.6 3.6 / 3.4 3.3.  It takes 1 to 2 % of a prompt.  The largest tile spills with it in RESID, whose sums are
+  // shorter (kz); int8 loses 3 % with it everywhere.
+  constexpr bool KEEP = Q ? EPI == KH_PG_QKV : EPI != KH_PG_RESID || TM <= 4;
+  f32x4 lost[TN];
+#pragma unroll
+  for (int n = 0; n < TN; ++n) lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto fold = [&](int n, int m, int i, float f, float g) __attribute__((always_inline)) {
+    const float s = __builtin_fmaf(f, g, acc[n][m][i]);
+    if (KEEP && m == TM - 1) lost[n][i] += __builtin_fmaf(f, g, acc[n][m][i] - s);
+    acc[n][m][i] = s;
+  };
   float sgn = 1.0f, xinv[TM];
   unsigned xe[TM];
   auto row_top = [&](float v) __attribute__((always_inline)) {  // over the four lanes of row fr
@@ -398,7 +424,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(GROUP ? sc[n][i] * xinv[m] : sg[i], g[m][i], acc[n][m][i]);
+          for (int i = 0; i < 4; ++i) fold(n, m, i, GROUP ? sc[n][i] * xinv[m] : sg[i], g[m][i]);
       }
     }
     __builtin_amdgcn_s_setprio(0);
@@ -414,7 +440,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[n][m][i] = __builtin_fmaf(xinv[m], grp[n][m][i], acc[n][m][i]);
+          for (int i = 0; i < 4; ++i) fold(n, m, i, xinv[m], grp[n][m][i]);
         wsc[n] = -wsc[n];
       }
     }
@@ -428,6 +454,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     for (int n = 0; n < TN; ++n) {
       wsc[n] = row_scale(n);
       w[n] = row_at(n) + 8 * fh;
+      lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -447,7 +474,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
         unsigned e[PART];
 #pragma unroll
         for (int m = 0; m < PART; ++m) {
-          int t = t0 + (wm * TM + m0 + m) * 16 + fr;
+          int t = token_of((wm * TM + m0 + m) * 16 + fr);
           t = t < a.T ? t : a.T - 1;
           const char* x = a.X + ((unsigned)t * (unsigned)(4 * K) + 128u * k + 16u * fh);
           xh[m] = *(const f16x8*)x;
@@ -466,12 +493,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
           for (int n = 0; n < TN; ++n) {
             const f32x4 g = mfma_pair(wh[n], xh[m], mfma_pair(wh[n], xl[m], mfma_pair(wl[n], xh[m], f4_zero())));
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[n][m0 + m][i] = __builtin_fmaf(f, g[i], acc[n][m0 + m][i]);
+            for (int i = 0; i < 4; ++i) fold(n, m0 + m, i, f, g[i]);
           }
         }
       }
       sgn = -sgn;
     }
+#pragma unroll
+    for (int n = 0; n < TN; ++n) acc[n][TM - 1] += lost[n];
   };
   const std::true_type first{};
   const std::false_type second{};
@@ -499,6 +528,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       close();
     }
   }
+#pragma unroll
+  for (int n = 0; n < TN; ++n) acc[n][TM - 1] += lost[n];
   if constexpr (!Q) {
     // a half that has overflowed has left infinities or NaN in its row
     float all = 0.f;
@@ -521,7 +552,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   float xi[TM];
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
-    const int tok = t0 + (wm * TM + m) * 16 + fr;
+    const int tok = token_of((wm * TM + m) * 16 + fr);
     xi[m] = GROUP ? 1.0f : a.xs[tok < a.T ? tok : a.T - 1];
   }
   auto value = [&](int n, int m) __attribute__((always_inline)) {
@@ -563,7 +594,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     const int stage = (f0 >> 1) / KH_PAIR_STAGE(Q) + wn / sub;
 #pragma unroll
     for (int m = 0; m < TM; ++m) {
-      const int at = (wm * TM + m) * 16 + fr, tok = t0 + at;
+      const int at = (wm * TM + m) * 16 + fr, tok = token_of(at);
       if (tok >= a.T) continue;
       float top = 0.f;
 #pragma unroll
@@ -580,7 +611,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   }
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
-    const int tok = t0 + (wm * TM + m) * 16 + fr;
+    const int tok = token_of((wm * TM + m) * 16 + fr);
     if (tok >= a.T) continue;
 #pragma unroll
     for (int n = 0; n < TN; ++n) {
@@ -670,10 +701,12 @@ static __global__ __launch_bounds__(KH_WG) void k_pair_rmsnorm(float* __restrict
   auto load = [&](int k) __attribute__((always_inline)) {
     f32x4 v = x4[k];
     if (kz > 0) {  // the residual GEMM in front split K: its partial rows, in fixed order
+      f32x4 s = f4_zero();
       for (int z = 0; z < kz; ++z) {
         const f32x4 p = *(const f32x4*)(part + ((size_t)z * tcap + t) * dim + 4 * k);
-        v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
+        s.x += p.x; s.y += p.y; s.z += p.z; s.w += p.w;
       }
+      v.x += s.x; v.y += s.y; v.z += s.z; v.w += s.w;  // the residual, the largest of them, is rounded once
       x4[k] = v;
     }
     const f32x4 g = w4[k];

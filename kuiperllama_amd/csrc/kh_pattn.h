@@ -20,6 +20,11 @@
 // As in kh_gemm.h the K-side contraction visits the head dimension in the order of the lanes'
 // float4 loads (k-quad {16b+s, 16b+4+s, ...}); any order is a valid dot product.
 //
+// The matrix unit rounds its sums down.  In scores that is a shift that grows with their size, so large weights come out too
+// small, alike in every layer: each score is four sums (by the component s of its fragments), two of them with the sign
+// turned.  Logits behind 60 and 225 prompt tokens of Llama-2-7B int8, all rows but the cache from this pass: 5.0e-6 and
+// 4.9e-6 from 64 bits with one sum (kh_pattn_pair.h alike), 3.6e-6 with four (steps on the decode kernels: 3.7e-6 and 3.4e-6).
+//
 // Row statistics: a token's scores sit in 4 registers x 4 lane groups (l>>4); the tile maximum is
 // combined across the groups with two ds_bpermute, so every lane of a token uses the same m and
 // the P values fed to the matrix core are consistently scaled.  The row sum is kept per lane and
@@ -106,7 +111,10 @@ __global__ __launch_bounds__(64 * NW) void k_pg_attn(const KhPgAttnArgs a) {
     my_pos[qi] = a.pos0 + tq;
     const float* qrow = a.q + (size_t)tq * a.dim + (size_t)h * HS + 4 * lj;
 #pragma unroll
-    for (int bb = 0; bb < HB; ++bb) qf[qi][bb] = *(const f32x4*)(qrow + 16 * bb);
+    for (int bb = 0; bb < HB; ++bb) {
+      const f32x4 v = *(const f32x4*)(qrow + 16 * bb);
+      qf[qi][bb] = f32x4{v.x, -v.y, v.z, -v.w};  // signs of the four sums of a score
+    }
   }
   float m[QT], l[QT];
   f32x4 oacc[QT][NC][4];
@@ -126,14 +134,17 @@ __global__ __launch_bounds__(64 * NW) void k_pg_attn(const KhPgAttnArgs a) {
     for (int qi = 0; qi < QT; ++qi) {
       // position tiles wholly above the diagonal of this query tile: nothing to add (wave-uniform)
       if (QT > 1 && pt * 16 > a.pos0 + t0 + 16 * qi + 15) continue;
-      f32x4 sacc = zero4;
+      f32x4 sacc[4] = {zero4, zero4, zero4, zero4};
 #pragma unroll
       for (int bb = 0; bb < HB; ++bb)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) sacc = mfma16(pg_comp(kc_[bb], s), pg_comp(qf[qi][bb], s), sacc);
+        for (int s = 0; s < 4; ++s) sacc[s] = mfma16(pg_comp(kc_[bb], s), pg_comp(qf[qi][bb], s), sacc[s]);
       float sv[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sv[r] = (pb + r <= my_pos[qi]) ? pg_comp(sacc, r) * scale : -INFINITY;
+      for (int r = 0; r < 4; ++r) {
+        const float dot = (pg_comp(sacc[0], r) - pg_comp(sacc[1], r)) + (pg_comp(sacc[2], r) - pg_comp(sacc[3], r));
+        sv[r] = (pb + r <= my_pos[qi]) ? dot * scale : -INFINITY;
+      }
       float tm = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
       tm = fmaxf(tm, __shfl_xor(tm, 16));
       tm = fmaxf(tm, __shfl_xor(tm, 32));

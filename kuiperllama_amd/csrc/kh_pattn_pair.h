@@ -12,7 +12,7 @@
 //   O^T[d, tok]  += V^T . P^T       the B operand of v_mfma_f32_16x16x32_f16 as it stands
 // Products lo hi, hi lo, hi hi in this order, so the sum is rounded at its full size only in the last ones.  Online softmax
 // in the log2 domain as in kh_pattn.h.  The matrix core rounds sums down, which would not average out over thousands of
-// positions: a block's P V starts from zero, is added to O in fp32 (times 1 / the block's scale), and every second block of a
+// positions and shifts scores by their size: half of a score's columns are summed with the sign turned (kh_pattn.h), a block's P V starts from zero, is added to O in fp32 (times 1 / the block's scale), and every second block of a
 // wave carries -P.
 //
 // Q is split once per workgroup and kept in LDS; K and V of the next block are requested when the last product of the
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
 #pragma unroll
     for (int c = 0; c < G::NC; ++c) {
       f16x8 hi, lo;
-      pa_split(v[c], s, hi, lo);
+      pa_split(v[c], 2 * c < G::NC ? s : -s, hi, lo);
       *(f16x8*)&q_lds[qi][2 * c][lane * 16] = hi;
       *(f16x8*)&q_lds[qi][2 * c + 1][lane * 16] = lo;
     }
@@ -211,22 +211,30 @@ __global__ __launch_bounds__(64 * NW, 2) void k_pa_attn(const KhPaArgs a) {
       if (qi < QT - 1 && pb * 32 > first + 15) continue;  // wholly above the diagonal (never the last tile)
       int at = lane * 16;
       if constexpr (HS > 64) asm volatile("" : "+v"(at));  // or all of Q is kept in registers across the blocks, and they spill
-      f32x4 sa[2] = {zero4, zero4};
+      f32x4 sa[2] = {zero4, zero4}, sb[2] = {zero4, zero4};
 #pragma unroll
       for (int c = 0; c < G::NC; ++c) {
         const f16x8 qh = *(const f16x8*)&q_lds[qi][2 * c][at], ql = *(const f16x8*)&q_lds[qi][2 * c + 1][at];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          sa[u] = mfma_pair(kf[(c * 2 + 1) * 2 + u], qh, sa[u]);
-          sa[u] = mfma_pair(kf[c * 4 + u], ql, sa[u]);
+          f32x4& t = 2 * c < G::NC ? sa[u] : sb[u];
+          t = mfma_pair(kf[(c * 2 + 1) * 2 + u], qh, t);
+          t = mfma_pair(kf[c * 4 + u], ql, t);
         }
       }
 #pragma unroll
       for (int c = 0; c < G::NC; ++c) {
         const f16x8 qh = *(const f16x8*)&q_lds[qi][2 * c][at];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) sa[u] = mfma_pair(kf[c * 4 + u], qh, sa[u]);
+        for (int u = 0; u < 2; ++u) {
+          f32x4& t = 2 * c < G::NC ? sa[u] : sb[u];
+          t = mfma_pair(kf[c * 4 + u], qh, t);
+        }
       }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sa[u][r] -= sb[u][r];
       if (qi == QT - 1 && next < n_pb) load_k(next);
       if (pb * 32 + 31 > first) {
         const int my = first + li, p = pb * 32 + 8 * lj;

@@ -1,0 +1,65 @@
+"""The last token of a prompt inside the prompt's pass (csrc/kh_model_pair.hip: pair_takes_last) against its step behind the
+bit-identical prompt path: logits, words, cache rows, at pass borders and for a model of one layer."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from kuiperllama_amd import _ffi, binfmt
+from test_model_gpu import _PF_SPECS, KV_ATOL_GEMM, _atol
+
+pytestmark = pytest.mark.gpu
+
+SPECS = {n: _PF_SPECS[n] for n in ("gqa-half", "int8")}
+SPECS["one-layer"] = dataclasses.replace(_PF_SPECS["gqa-half"], n_layers=1)
+
+
+@pytest.mark.parametrize("name", sorted(SPECS))
+@pytest.mark.parametrize("chunk", [None, "16", "64"])
+def test_last_token_in_the_pass(gpu, name, chunk, monkeypatch):
+    from kuiperllama_amd.model import KuiperModel
+    spec = dataclasses.replace(SPECS[name], seq_len=512)
+    m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=41, device=gpu), spec)
+    toks = [int(t) for t in np.random.default_rng(7).integers(0, spec.vocab_size, 300)]
+    # n - 1 a multiple of the pass: the last token keeps its own step; n == total: nothing behind it
+    for n in (17, 18, 32, 33, 65, 66, 129, 130, 300):
+        for more in (0, 3):
+            out = {}
+            for mode in ("gemv", "gemm"):
+                monkeypatch.setenv("KH_PREFILL", mode)
+                if chunk and mode == "gemm":
+                    monkeypatch.setenv("KH_PG_CHUNK", chunk)
+                words, _ = m.generate(toks[:n], n + more, exec="fused" if n == 33 else "graph")
+                fs = m.first_sample()
+                out[mode] = (words, fs, m.logits(), [m.read_kv(l, 0, n) for l in range(spec.n_layers)])
+                monkeypatch.delenv("KH_PG_CHUNK", raising=False)
+            (wa, fa, la, ka), (wb, fb, lb, kb) = out["gemv"], out["gemm"]
+            assert fb["pos"] == n - 1 and fb["prefill_mode"] == "gemm" and wb[: n - 1] == toks[1:n]
+            assert abs(fa["top1"] - fb["top1"]) <= _atol(spec), (n, more)
+            if fa["margin"] > 2 * _atol(spec):
+                assert fb["top1_id"] == fa["top1_id"] == wb[n - 1]
+            if wa == wb:
+                np.testing.assert_allclose(lb, la, rtol=0, atol=_atol(spec), err_msg=f"n={n} more={more}")
+            for l, (x, y) in enumerate(zip(ka, kb)):
+                for a, b in zip(x, y):
+                    np.testing.assert_allclose(b, a, rtol=0, atol=KV_ATOL_GEMM * (4 if spec.quant else 1), err_msg=f"n={n} layer {l}")
+    monkeypatch.delenv("KH_PREFILL")
+    prompt = toks[:40]
+    words, _ = m.generate(prompt, 60)
+    assert m.generate(prompt, 60, stop=[words[39]])[0] == words[:39]  # the stop token comes from the pass
+    later = next((i for i in range(40, 60) if words[i] not in words[39:i]), None)
+    if later:
+        assert m.generate(prompt, 60, stop=[words[later]])[0] == words[:later]
+    m.close()
+
+
+def test_prompt_of_the_whole_cache(gpu):
+    from kuiperllama_amd.model import KuiperModel
+    spec = dataclasses.replace(SPECS["gqa-half"], seq_len=48)
+    m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=42, device=gpu), spec)
+    toks = [int(t) for t in np.random.default_rng(8).integers(0, spec.vocab_size, 48)]
+    words, _ = m.generate(toks, 48)
+    assert len(words) == 48 and words[:47] == toks[1:]
+    with pytest.raises(_ffi.KhError):
+        m.generate(toks, 49)
+    m.close()
