@@ -215,5 +215,10 @@ int hy_step_init(kh_model* m);
 void hy_launch_step(kh_model* m, int advance, int n_forced);
 int hy_decode_max(const kh_model* m);  // sequences the fused step can take at once
 int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits);
+struct HyTail {  // device lists of the wanted tokens of a pass: their rows, ids, positions, slots
+  const int32_t *rows, *tok, *pos, *slot;
+};
+bool hy_tail_pays(const kh_model* m, int T, int want);
+int hy_tail(kh_model* m, const HyTail& t, int n, float* h_logits);
 int hy_launches(const kh_model* m);  // kernel launches of one decode step
 }  // namespace khm

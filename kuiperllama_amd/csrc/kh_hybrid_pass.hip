@@ -43,6 +43,8 @@ struct Pass {
   const int32_t* base = nullptr;
   std::vector<RowTiles> tiles;
   bool no_logits = false;  // nothing of the last layer's output is wanted: only its cache rows / state
+  bool tail = false;       // ... or that of few tokens: they take the last layer as a decode step (hy_tail)
+  HyTail wanted{};
 };
 
 // ---- tables ------------------------------------------------------------------------------------------------------
@@ -392,7 +394,7 @@ struct Runner {
     for (size_t i = 0; i < hy.runs.size(); ++i) {
       const HyRun& r = hy.runs[i];
       const HyLayer& l = hy.layers[(size_t)r.layer];
-      const bool state_only = ps.no_logits && i + 1 == hy.runs.size() && !hy.probe;
+      const bool state_only = (ps.no_logits || ps.tail) && i + 1 == hy.runs.size() && !hy.probe;
       const bool through = r.pass >= 0 && hy.enter.N;
       if (through) TRY(enter(i == 0));
       TRY(combine(&l, i == 0 && !through, r.pass));
@@ -432,6 +434,7 @@ int run_pass(kh_model* m, const Pass& ps, float* h_logits) {
   Runner<T> r(m, ps);
   TRY(r.layers());
   if (!ps.n_want) return KH_OK;
+  if (ps.tail) return hy_tail(m, ps.wanted, ps.n_want, h_logits);
   TRY(r.combine(nullptr, false, -1));
   for (int w = 0; w < ps.n_want; w += hy.wl_rows) {
     const int n = std::min(hy.wl_rows, ps.n_want - w);
@@ -467,7 +470,7 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
   std::vector<Pass> passes;
   std::vector<int32_t> all;
   struct Off {
-    int tok, pos, seg, slot, row0, sn, pos0, ck, m0, mn, want;
+    int tok, pos, seg, slot, row0, sn, pos0, ck, m0, mn, want, wtok, wpos, wslot;
   };
   std::vector<Off> offs;
   std::vector<size_t> bases;
@@ -513,6 +516,7 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
     while (wi < n_want && want[wi] < row_base + p.T) wr.push_back(want[wi++] - row_base);
     p.n_want = (int)wr.size();
     p.no_logits = wr.empty();
+    p.tail = !hy.probe && hy_tail_pays(m, p.T, p.n_want);
     p.expand = hy.any_latent && p.S <= 8 && !dbg_off("KH_HY_EXPAND");
     for (int i = 0; i < p.S; ++i) {
       p.segs.push_back({slot[(size_t)i], row0[(size_t)i], sn[(size_t)i], pos0[(size_t)i]});
@@ -535,6 +539,14 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
     o.m0 = tb.put(m0);
     o.mn = tb.put(mn);
     o.want = tb.put(wr);
+    auto of_wanted = [&](auto&& f) {
+      std::vector<int32_t> v;
+      for (int32_t r : wr) v.push_back(f((size_t)r));
+      return tb.put(v);
+    };
+    o.wtok = of_wanted([&](size_t r) { return tok[r]; });
+    o.wpos = of_wanted([&](size_t r) { return pos[r]; });
+    o.wslot = of_wanted([&](size_t r) { return slot[(size_t)seg[r]]; });
     for (const RowKind& kd : kinds) {
       RowTiles t{kd, row_tiles(sn, kd, &lt), 0, (int)lt.size() / 2};
       t.off = tb.put(lt);
@@ -571,6 +583,7 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
     p.multi0 = b + o.m0;
     p.multin = b + o.mn;
     p.want = b + o.want;
+    p.wanted = HyTail{b + o.want, b + o.wtok, b + o.wpos, b + o.wslot};
     TRY(hy.f32 ? run_pass<float>(m, p, out) : run_pass<bf16>(m, p, out));
     if (out) out += (size_t)p.n_want * hy.c.vocab;
   }

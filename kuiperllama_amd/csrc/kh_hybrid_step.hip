@@ -112,20 +112,22 @@ int split_waves(int rows, int nblk) {
 
 // One token of B sequences: tables at (tok, pos, slot); logits to `logits` [B][V]; argmax partials of sequence 0 to
 // the model's sampler buffers.
+// tail: the last layer run only, behind a pass that has left the residual rows in front of it in x[0] (complete: nothing of a
+// loop's entry is missing) and, where its mixer is a scan, that one's outputs in v.
 template <class T, int B>
-int step(kh_model* m, const LdTabs tb, float* logits) {
+int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
   Hybrid& hy = *m->hy;
   Hybrid::Step& st = *hy.step_st;
   hipStream_t s = m->stream;
   const int W = hy.c.width, Wp = hy.c.widthp;
   float* x_in = st.x[0];
-  for (size_t ri = 0; ri < hy.runs.size(); ++ri) {
+  for (size_t ri = tail ? hy.runs.size() - 1 : 0; ri < hy.runs.size(); ++ri) {
     const HyRun& r = hy.runs[ri];
     const HyLayer& l = hy.layers[(size_t)r.layer];
     const HyMoe& f = l.ff;
     const HyHeads& ha = l.ha;
-    const bool mamba = l.mixer == HY_MAMBA1, heads = l.mixer == HY_HEADS, through = r.pass >= 0 && hy.enter.N;
-    const bool changed = !through && (ri == 0 || r.pass >= 0);
+    const bool mamba = l.mixer == HY_MAMBA1, heads = l.mixer == HY_HEADS, through = r.pass >= 0 && hy.enter.N && !tail;
+    const bool changed = !through && !tail && (ri == 0 || r.pass >= 0), mixed = tail && mamba;
     float* x_cur = through || changed ? st.x[2] : x_in;
     float* x_out = x_in == st.x[0] ? st.x[1] : st.x[0];
     const HyMat& w_in = mamba ? l.mb.in : (heads ? ha.qkvg : l.la.dqkv);
@@ -147,8 +149,9 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
         g.kind = kind;
         g.norm2 = norm2;
       };
-      seg(w_in, st.in, in_ld, in_ld, mamba ? LDI_CONV : LDI_PLAIN, 0);
+      if (!mixed) seg(w_in, st.in, in_ld, in_ld, mamba ? LDI_CONV : LDI_PLAIN, 0);
       if (heads) a.seg[0].bias = ha.qkvg_b.p;
+      const int router = a.nseg;
       if (f.top) seg(f.zr, st.z, f.zr.N, f.zr.N, LDI_PLAIN, 1);
       if (f.sff) seg(f.sgu, st.hs, f.sffp, f.sffp, LDI_GATED, 1);
       a.act = f.sact;
@@ -164,20 +167,21 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
       a.x_in = through ? x_cur : x_in;
       a.x_cur = changed ? x_cur : nullptr;
       a.emb = emb;
-      a.step = r.pass >= 0 && hy.step.on ? hy.step.p + (size_t)r.pass * Wp : nullptr;
+      a.step = r.pass >= 0 && hy.step.on && !tail ? hy.step.p + (size_t)r.pass * Wp : nullptr;
       a.w1 = l.n1.p;
       a.b1 = l.n1b.p;
       a.w2 = l.norm2().p;
       a.b2 = l.norm2_b().p;
       a.xn2 = f.top ? st.xn2 : nullptr;
+      a.xn2_wg = a.seg[router].wg0;
       a.W = W;
       a.ld = Wp;
-      a.from_embed = ri == 0 && !through;
-      a.add_x0 = r.pass > 0 && !through;
+      a.from_embed = ri == 0 && !through && !tail;
+      a.add_x0 = r.pass > 0 && !through && !tail;
       a.rms = hy.c.rms;
       a.eps = hy.c.eps;
       a.t = tb;
-      if (mamba) {
+      if (mamba && !mixed) {
         a.conv_w = l.mb.conv.p;
         a.conv_b = l.mb.conv_b.p;
         a.conv_st = hy.state + r.conv_off;
@@ -187,9 +191,9 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
         a.taps = l.mb.taps;
         a.xc_ld = l.mb.innerp;
       }
-      TRY(with_nv<T>(Wp, [&](auto nv) { return go(k_ld_in<T, B, decltype(nv)::value>, dim3(wg), 256, B * vec_b<T>(Wp), s, a); }));
+      if (wg) TRY(with_nv<T>(Wp, [&](auto nv) { return go(k_ld_in<T, B, decltype(nv)::value>, dim3(wg), 256, B * vec_b<T>(Wp), s, a); }));
     }
-    {
+    if (!mixed || f.top) {
       LdMidArgs a{};
       a.t = tb;
       a.eps = hy.c.eps;
@@ -225,7 +229,7 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
         a.raw = st.in;
         a.cache = (T*)m->kcache + r.kv_off;
         a.slot_elems = hy.kv_slot;
-      } else {
+      } else if (!mixed) {
         const HyMat& wm = mamba ? l.mb.x : l.la.uq;
         a.wm = wm.w;
         a.rows = wm.N;
@@ -262,7 +266,8 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
         });
       }));
     }
-    if (mamba) {
+    if (mixed) {
+    } else if (mamba) {
       const HyMamba& mb = l.mb;
       LdScanArgs a{st.xc, st.in, st.mid, mb.dt.w, mb.dt_b.p, mb.A2.p, mb.D.p, hy.state + r.st_off, st.v, hy.st_slot,
                    mb.inner, mb.state, mb.rankp, mb.innerp, mb.innerp, tb};
@@ -344,13 +349,22 @@ int step(kh_model* m, const LdTabs tb, float* logits) {
   return with_nv<T>(Wp, [&](auto nv) { return go(k_ld_head<T, B, decltype(nv)::value>, dim3(st.head_wg), 256, B * vec_b<T>(Wp), s, h); });
 }
 template <class T>
-int step_b(kh_model* m, int B, const LdTabs& tb, float* logits) {
-  if (B == 1) return step<T, 1>(m, tb, logits);
-  if (B == 2) return step<T, 2>(m, tb, logits);
-  return step<T, 4>(m, tb, logits);
+int step_b(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail) {
+  if (B == 1) return step<T, 1>(m, tb, logits, tail);
+  if (B == 2) return step<T, 2>(m, tb, logits, tail);
+  return step<T, 4>(m, tb, logits, tail);
 }
-int step_any(kh_model* m, int B, const LdTabs& tb, float* logits) {
-  return m->hy->f32 ? step_b<float>(m, B, tb, logits) : step_b<bf16>(m, B, tb, logits);
+int step_any(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail = false) {
+  return m->hy->f32 ? step_b<float>(m, B, tb, logits, tail) : step_b<bf16>(m, B, tb, logits, tail);
+}
+// rows of the residual stream, and of a scan's outputs (mix nullptr: none), to the step's buffers; grid (rows of the step)
+template <class T>
+__global__ __launch_bounds__(256) void k_tail_rows(const int32_t* rows, const float* x, float* x_out, int ld, const T* mix, float* v,
+                                                   int ldv) {
+  const size_t from = (size_t)rows[blockIdx.x], to = blockIdx.x;
+  for (int i = threadIdx.x; i < ld / 4; i += 256) ((f32x4*)(x_out + to * ld))[i] = ((const f32x4*)(x + from * ld))[i];
+  if (!mix) return;
+  for (int i = threadIdx.x; i < ldv / 4; i += 256) ((f32x4*)(v + to * ldv))[i] = quad_f(mix + from * ldv + 4 * i);
 }
 }  // namespace
 
@@ -441,6 +455,38 @@ int hy_launches(const kh_model* m) {
   return n;
 }
 int hy_decode_max(const kh_model* m) { return m->hy->step_st->bmax; }
+// Is the last layer of a pass over T tokens cheaper for its `want` tokens alone?  A step of up to four tokens reads the layer's
+// weights, and the experts of each of them, once more.  Whole calls, us, the layer for all tokens / for the last of each
+// sequence: Gufanex 2048 x 4 bf16 1 x 4 801 / 718, 1 x 300 1330 / 1162, 1 x 2048 2820 / 2365, 4 x 64 1317 / 1170, 6 x 22 1107 /
+// 1150; Gusorax 1024 x 8 bf16 1 x 17 602 / 590, 1 x 1100 1461 / 1339, 4 x 16 699 / 716, 4 x 64 822 / 825, 6 x 64 880 / 951;
+// Gusorax 2048 x 2 fp32 1 x 300 1195 / 705.
+bool hy_tail_pays(const kh_model* m, int T, int want) {
+  const int bmax = m->hy->step_st->bmax;
+  return bmax >= 1 && want > 0 && !dbg_off("KH_HY_DECODE") && !dbg_off("KH_HY_TAIL") && T >= 4 && T >= 32 * (want - 1) &&
+         (want <= bmax || (long)((want + bmax - 1) / bmax) * 256 <= T);
+}
+// the last layer run for the wanted rows of a pass (HyTail), logits [n][vocab] to the host
+int hy_tail(kh_model* m, const HyTail& t, int n, float* h_logits) {
+  Hybrid& hy = *m->hy;
+  Hybrid::Step& st = *hy.step_st;
+  const HyLayer& l = hy.layers[(size_t)hy.runs.back().layer];
+  const bool mamba = l.mixer == HY_MAMBA1;
+  for (int i = 0; i < n;) {
+    const int B = std::min(st.bmax, n - i >= 4 ? 4 : (n - i >= 2 ? 2 : 1));
+    const LdTabs tb{t.tok + i, t.pos + i, t.slot + i};
+    auto rows = [&](auto type) {
+      typedef decltype(type) T;
+      hipLaunchKernelGGL(k_tail_rows<T>, dim3(B), dim3(256), 0, m->stream, t.rows + i, (const float*)hy.x, st.x[0], hy.c.widthp,
+                         mamba ? (const T*)hy.a2 : (const T*)nullptr, st.v, mamba ? l.mb.innerp : 0);
+    };
+    if (hy.f32) rows(0.f);
+    else rows((bf16)0.f);
+    TRY(step_any(m, B, tb, st.logits, true));
+    KH_CHECK_HIP(hipMemcpyAsync(h_logits + (size_t)i * hy.c.vocab, st.logits, (size_t)B * hy.c.vocab * 4, hipMemcpyDeviceToHost, m->stream));
+    i += B;
+  }
+  return kh_launch_status();
+}
 // one token of each of n sequences (n <= hy_decode_max), logits [n][vocab] to the host
 int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits) {
   Hybrid& hy = *m->hy;

@@ -205,7 +205,8 @@ struct LdInArgs {
   LdEmbed emb;
   const float* step;
   const float *w1, *b1, *w2, *b2;  // b: nullptr with rms
-  float* xn2;          // [B][ld], written by the router's first workgroup (nullptr: nobody reads it)
+  float* xn2;          // [B][ld], written by the router's first workgroup xn2_wg (nullptr: nobody reads it)
+  int xn2_wg;
   int W, ld, from_embed, add_x0, rms;
   float eps;
   GateAct act;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
           if ((int)threadIdx.x + 256 * j < n4) ((f32x4*)(a.x_cur + (size_t)q * a.ld))[threadIdx.x + 256 * j] = v[j];
       }
       // the router's first workgroup leaves the second norm for the launches that follow
-      f32x4* keep = a.xn2 && wg == a.seg[1].wg0 ? (f32x4*)(a.xn2 + (size_t)q * a.ld) : nullptr;
+      f32x4* keep = a.xn2 && wg == a.xn2_wg ? (f32x4*)(a.xn2 + (size_t)q * a.ld) : nullptr;
       float shift = 0.f;
       if (!a.rms) shift = a.from_embed ? (float)((const T*)a.emb.embed)[(size_t)a.t.tok[q] * a.ld] : a.x_in[(size_t)q * a.ld];
       if (q) __syncthreads();  // red is free again
