@@ -208,7 +208,7 @@ struct Runner {
     cv.ldo = mb.innerp;
     cv.taps = mb.taps;
     cv.p = ps.p;
-    conv_launch<T>(s, cv, ps.T);
+    conv_launch<T>(s, cv, ps.chunks, ps.n_chunks);
     hipLaunchKernelGGL(k_conv_state<T>, dim3((I + 255) / 256, ps.S), dim3(256), 0, s, cv);
     {
       LgArgs a = gemm(mb.x, hy.a1, mb.innerp, hy.a2, mb.rankp);

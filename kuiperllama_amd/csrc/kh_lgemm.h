@@ -61,6 +61,53 @@ struct LgCfg {
   static constexpr int LDS = NSTAGE * STAGE;
 };
 
+// features f .. f + 3 of one token, f a multiple of four
+template <class T, int EPI>
+__device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 v) {
+  typedef Tile<T> TL;
+  if ((EPI == LG_T || EPI == LG_F32) && a.bias) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += a.bias[f + i < a.N ? f + i : 0];
+  }
+  if (EPI == LG_T) {
+    T* o = (T*)a.out + (size_t)blockIdx.z * a.o_z + (size_t)tok * a.ldo + f;
+    if (f + 3 < a.N && (a.ldo & 3) == 0) {
+      *(typename TL::quad*)o = to_quad<T>(v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (f + i < a.N) o[i] = (T)v[i];
+    }
+  } else {
+    f32x4 y = v;
+    if (EPI == LG_SOFTPLUS) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = softplus1(v[i] + a.bias[f + i < a.N ? f + i : 0]);
+    } else if (EPI == LG_SOFTCAP) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = a.cap > 0.f ? a.cap * tanhf(v[i] / a.cap) : v[i];
+    }
+    // destination of the four features: one array, unless they straddle LG_SPLIT's border
+    const bool to_t = EPI == LG_SPLIT && f + 3 < a.n_split, cut = EPI == LG_SPLIT && !to_t && f < a.n_split;
+    float* o = EPI == LG_SPLIT ? a.out2 + (size_t)tok * a.ldo2 + (f - a.n_split) : (float*)a.out + (size_t)tok * a.ldo + f;
+    const int ld = EPI == LG_SPLIT ? a.ldo2 : a.ldo;
+    if (to_t) {
+      T* ot = (T*)a.out + (size_t)tok * a.ldo + f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ot[i] = (T)y[i];
+    } else if (!cut && f + 3 < a.N && (ld & 3) == 0) {
+      *(f32x4*)o = y;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (f + i >= a.N) continue;
+        if (EPI == LG_SPLIT && f + i < a.n_split) ((T*)a.out)[(size_t)tok * a.ldo + f + i] = (T)y[i];
+        else o[i] = y[i];
+      }
+    }
+  }
+}
+
 template <class T, int BM, int BN, int EPI>
 __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   typedef Tile<T> TL;
@@ -175,51 +222,7 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
       }
     } else {
 #pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        const int f = f0 + wn * (BN / 2) + n * 16 + 4 * fh;
-        f32x4 v = acc[n][m];
-        if ((EPI == LG_T || EPI == LG_F32) && a.bias) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] += a.bias[f + i < a.N ? f + i : 0];
-        }
-        if (EPI == LG_T) {
-          T* o = (T*)a.out + (size_t)blockIdx.z * a.o_z + (size_t)tok * a.ldo + f;
-          if (f + 3 < a.N && (a.ldo & 3) == 0) {
-            *(typename TL::quad*)o = to_quad<T>(v);
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (f + i < a.N) o[i] = (T)v[i];
-          }
-        } else {
-          f32x4 y = v;
-          if (EPI == LG_SOFTPLUS) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) y[i] = softplus1(v[i] + a.bias[f + i < a.N ? f + i : 0]);
-          } else if (EPI == LG_SOFTCAP) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) y[i] = a.cap > 0.f ? a.cap * tanhf(v[i] / a.cap) : v[i];
-          }
-          // destination of the four features: one array, unless they straddle LG_SPLIT's border
-          const bool to_t = EPI == LG_SPLIT && f + 3 < a.n_split, cut = EPI == LG_SPLIT && !to_t && f < a.n_split;
-          float* o = EPI == LG_SPLIT ? a.out2 + (size_t)tok * a.ldo2 + (f - a.n_split) : (float*)a.out + (size_t)tok * a.ldo + f;
-          const int ld = EPI == LG_SPLIT ? a.ldo2 : a.ldo;
-          if (to_t) {
-            T* ot = (T*)a.out + (size_t)tok * a.ldo + f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ot[i] = (T)y[i];
-          } else if (!cut && f + 3 < a.N && (ld & 3) == 0) {
-            *(f32x4*)o = y;
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              if (f + i >= a.N) continue;
-              if (EPI == LG_SPLIT && f + i < a.n_split) ((T*)a.out)[(size_t)tok * a.ldo + f + i] = (T)y[i];
-              else o[i] = y[i];
-            }
-          }
-        }
-      }
+      for (int n = 0; n < TN; ++n) lg_store<T, EPI>(a, tok, f0 + wn * (BN / 2) + n * 16 + 4 * fh, acc[n][m]);
     }
   }
 }

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void k_gather_norm(const float* x, const int32
 
 // ---- causal depthwise convolution + silu -----------------------------------------------------------------------
 // Inputs are the first C columns of xz rows.  Inputs before a segment's first row come from the sequence's conv state
-// [taps - 1][C] (position 0: zeros).  grid (C / 256, T).
+// [taps - 1][C] (position 0: zeros).
 template <class T>
 struct ConvArgs {
   const T* xz;          // [T][ldx]
@@ -159,94 +159,113 @@ struct ConvArgs {
   int C, ldx, ldo, taps;
   PassTabs p;
 };
-// E channels (16 bytes) of KH_CONV_TT consecutive tokens per thread; the taps of the channels stay in registers.
-// TAPS: number of taps, 0 = any (weights re-read per token).  grid (C / (256 E), T / KH_CONV_TT)
+// E channels (16 bytes) of KH_CONV_TT consecutive tokens of one chunk (kh_scan.h: tokens of one segment) per thread; the taps
+// of the channels stay in registers.  With four taps all rows are requested at once (2048 tokens of 4096 channels: 20
+// us; token by token, every token's rows behind the one before it, 32).
+// TAPS: number of taps, 0 = any (weights re-read per token).  grid (C / (256 E), chunks x KH_CONV_PER)
 #define KH_CONV_TT 8
+#define KH_CONV_CH 64  // tokens of a chunk
+#define KH_CONV_PER (KH_CONV_CH / KH_CONV_TT)
+struct ScanChunk {
+  int seg, row0, n, flags;  // flags: 1 = first of its segment, 2 = last of its segment
+};
 template <class T, int TAPS>
-__global__ __launch_bounds__(256) void k_conv_silu(const ConvArgs<T> a, int T_all) {
-  constexpr int E = Tile<T>::N;
+__global__ __launch_bounds__(256) void k_conv_silu(const ConvArgs<T> a, const ScanChunk* chunks) {
+  constexpr int E = Tile<T>::N, TT = KH_CONV_TT;
   typedef typename Tile<T>::frag frag;
+  const ScanChunk ck = chunks[blockIdx.y / KH_CONV_PER];
+  const int u0 = (int)(blockIdx.y % KH_CONV_PER) * TT, n = ck.n - u0;
   const int c = (blockIdx.x * 256 + threadIdx.x) * E;
-  if (c >= a.C) return;
-  const bool vec = c + E <= a.C && (a.ldx & (E - 1)) == 0;
+  if (n <= 0 || c >= a.C) return;
+  const bool vec = (a.C & (E - 1)) == 0 && (a.ldx & (E - 1)) == 0;
+  const int t0 = ck.row0 + u0, i0 = t0 - a.p.seg_row0[ck.seg];  // rows of the segment in front of the first token
   const int taps = TAPS ? TAPS : a.taps;
-  float w[E][TAPS ? TAPS : 1], bias[E];
+  const bool fresh = a.p.seg_pos0[ck.seg] == 0;
+  const float* st = a.state + (size_t)a.p.seg_slot[ck.seg] * a.slot_stride;
+  auto row = [&](int t, float (&in)[E]) __attribute__((always_inline)) {
+    const T* x = a.xz + (size_t)t * a.ldx;
+    if (vec) {
+      const frag f = *(const frag*)(x + c);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    bias[e] = c + e < a.C ? a.b[c + e] : 0.f;
-    if (TAPS)
-#pragma unroll
-      for (int k = 0; k < TAPS; ++k) w[e][k] = c + e < a.C ? a.w[(size_t)(c + e) * TAPS + k] : 0.f;
-  }
-  for (int u = 0; u < KH_CONV_TT; ++u) {
-    const int t = blockIdx.y * KH_CONV_TT + u;
-    if (t >= T_all) return;
-    const int sg = a.p.seg[t], i = t - a.p.seg_row0[sg];
-    float v[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = bias[e];
-    auto tap = [&](int k, const float (&in)[E]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int e = 0; e < E; ++e)
-        v[e] = __builtin_fmaf(TAPS ? w[e][TAPS ? k : 0] : (c + e < a.C ? a.w[(size_t)(c + e) * taps + k] : 0.f), in[e], v[e]);
-    };
-    auto from_row = [&](int j, float (&in)[E]) __attribute__((always_inline)) {
-      const T* x = a.xz + (size_t)(t - i + j) * a.ldx + c;
-      if (vec) {
-        const frag f = *(const frag*)x;
-#pragma unroll
-        for (int e = 0; e < E; ++e) in[e] = (float)f[e];
-      } else {
-#pragma unroll
-        for (int e = 0; e < E; ++e) in[e] = c + e < a.C ? (float)x[e] : 0.f;
-      }
-    };
-    float in[E];
-    if (i >= taps - 1) {  // every input is a row of the segment
-      if (TAPS) {
-#pragma unroll
-        for (int k = 0; k < TAPS; ++k) {
-          from_row(i - (TAPS - 1) + k, in);
-          tap(k, in);
-        }
-      } else {
-        for (int k = 0; k < taps; ++k) {
-          from_row(i - (taps - 1) + k, in);
-          tap(k, in);
-        }
-      }
+      for (int e = 0; e < E; ++e) in[e] = (float)f[e];
     } else {
-      const bool fresh = a.p.seg_pos0[sg] == 0;
-      const float* st = a.state + (size_t)a.p.seg_slot[sg] * a.slot_stride;
-      auto edge = [&](int k) __attribute__((always_inline)) {
-        const int j = i - (taps - 1) + k;
-        if (j >= 0) {
-          from_row(j, in);
-        } else {
 #pragma unroll
-          for (int e = 0; e < E; ++e) in[e] = !fresh && c + e < a.C ? st[(size_t)(taps - 1 + j) * a.C + c + e] : 0.f;
-        }
-        tap(k, in);
-      };
-      if constexpr (TAPS != 0) {
+      for (int e = 0; e < E; ++e) in[e] = c + e < a.C ? (float)x[c + e] : 0.f;
+    }
+  };
+  auto before = [&](int j, float (&in)[E]) __attribute__((always_inline)) {  // input j < 0 of the segment
 #pragma unroll
-        for (int k = 0; k < TAPS; ++k) edge(k);
+    for (int e = 0; e < E; ++e) in[e] = !fresh && c + e < a.C ? st[(size_t)(taps - 1 + j) * a.C + c + e] : 0.f;
+  };
+  auto emit = [&](int t, const float (&v)[E]) __attribute__((always_inline)) {  // output rows are padded to whole fragments
+    frag f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) f[e] = (T)(c + e < a.C ? silu_t<T>(v[e]) : 0.f);
+    *(frag*)(a.out + (size_t)t * a.ldo + c) = f;
+  };
+  float bias[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) bias[e] = c + e < a.C ? a.b[c + e] : 0.f;
+  if constexpr (TAPS != 0) {
+    float w[E][TAPS], pre[TAPS - 1][E];
+    frag x[TT];
+#pragma unroll
+    for (int k = 0; k < TAPS - 1; ++k) {
+      const int j = i0 - (TAPS - 1) + k;
+      if (j >= 0) row(t0 - (TAPS - 1) + k, pre[k]);
+      else before(j, pre[k]);
+    }
+#pragma unroll
+    for (int u = 0; u < TT; ++u) {
+      const int t = t0 + (u < n ? u : n - 1);
+      if (vec) {
+        x[u] = *(const frag*)(a.xz + (size_t)t * a.ldx + c);
       } else {
-        for (int k = 0; k < taps; ++k) edge(k);
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[u][e] = c + e < a.C ? a.xz[(size_t)t * a.ldx + c + e] : (T)0.f;
       }
     }
-    frag f;  // output rows are padded to whole fragments
 #pragma unroll
-    for (int e = 0; e < E; ++e) f[e] = (T)(c + e < a.C ? silu1(v[e]) : 0.f);
-    *(frag*)(a.out + (size_t)t * a.ldo + c) = f;
+    for (int e = 0; e < E; ++e)
+#pragma unroll
+      for (int k = 0; k < TAPS; ++k) w[e][k] = c + e < a.C ? a.w[(size_t)(c + e) * TAPS + k] : 0.f;
+#pragma unroll
+    for (int u = 0; u < TT; ++u) {
+      if (u >= n) break;
+      float v[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        v[e] = bias[e];
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) {
+          const int r = u - (TAPS - 1) + k;
+          v[e] = __builtin_fmaf(w[e][k], r < 0 ? pre[r < 0 ? TAPS - 1 + r : 0][e] : (float)x[r < 0 ? 0 : r][e], v[e]);
+        }
+      }
+      emit(t0 + u, v);
+    }
+  } else {
+    for (int u = 0; u < TT && u < n; ++u) {
+      float v[E], in[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = bias[e];
+      for (int k = 0; k < taps; ++k) {
+        const int j = i0 + u - (taps - 1) + k;
+        if (j >= 0) row(t0 + u - (taps - 1) + k, in);
+        else before(j, in);
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = __builtin_fmaf(c + e < a.C ? a.w[(size_t)(c + e) * taps + k] : 0.f, in[e], v[e]);
+      }
+      emit(t0 + u, v);
+    }
   }
 }
 template <class T>
-void conv_launch(hipStream_t s, const ConvArgs<T>& a, int T_all) {
+void conv_launch(hipStream_t s, const ConvArgs<T>& a, const ScanChunk* chunks, int n_chunks) {
   constexpr int CW = 256 * Tile<T>::N;
-  const dim3 g((a.C + CW - 1) / CW, (T_all + KH_CONV_TT - 1) / KH_CONV_TT);
-  if (a.taps == 4) hipLaunchKernelGGL((k_conv_silu<T, 4>), g, dim3(256), 0, s, a, T_all);
-  else hipLaunchKernelGGL((k_conv_silu<T, 0>), g, dim3(256), 0, s, a, T_all);
+  const dim3 g((a.C + CW - 1) / CW, n_chunks * KH_CONV_PER);
+  if (a.taps == 4) hipLaunchKernelGGL((k_conv_silu<T, 4>), g, dim3(256), 0, s, a, chunks);
+  else hipLaunchKernelGGL((k_conv_silu<T, 0>), g, dim3(256), 0, s, a, chunks);
 }
 // the last taps - 1 inputs of every segment become its sequence's state.  grid (C / 256, S)
 template <class T>

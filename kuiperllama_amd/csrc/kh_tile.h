@@ -49,6 +49,13 @@ __device__ __forceinline__ typename Tile<T>::quad to_quad(f32x4 v) {
 
 __device__ __forceinline__ float sigmoid1(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float silu1(float z) { return z * sigmoid1(z); }
+// the same for a result that is rounded to T at once: for bf16 on the hardware's exponential and reciprocal (a few units in
+// the last place of fp32)
+template <class T>
+__device__ __forceinline__ float silu_t(float z) {
+  if constexpr (sizeof(T) == 2) return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896f * z));
+  else return silu1(z);
+}
 // Gated unit of a feed-forward: gate times sigmoid(alpha gate) times (up + shift), both sides limited first.  SwiGLU is
 // {INFINITY, 1, 0}.
 struct GateAct {
@@ -59,6 +66,25 @@ __device__ __forceinline__ float gated1(const GateAct& c, float g, float u) {
   u = fminf(fmaxf(u, -c.limit), c.limit);
   return g * sigmoid1(c.alpha * g) * (u + c.shift);
 }
-// log(1 + e^z) without overflow
-__device__ __forceinline__ float softplus1(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
+// log(1 + e^z) without overflow: max(z, 0) + log1p(e), e = e^-|z|, log1p(e) = 2 atanh(s), s = e / (2 + e) <= 1/3 by its series (the
+// first term left out is below 2^-26 of the sum).  The library's log1pf and expf cost three times as much.
+__device__ __forceinline__ float softplus1(float z) {
+  float a = fabsf(z);
+  a = a > 126.f ? 126.f : a;  // (NaN stays)
+  constexpr float L = 1.44269502f, L_lo = 1.92596299e-8f;  // log2(e)
+  const float t = -a * L, lo = __builtin_fmaf(-a, L_lo, __builtin_fmaf(-a, L, -t));
+  float e = __builtin_amdgcn_exp2f(t);
+  e = __builtin_fmaf(e, lo * 0.693147181f, e);
+  const float d = 2.0f + e;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(r, __builtin_fmaf(-d, r, 1.0f), r);
+  const float s = e * r, q = s * s;
+  float p = __builtin_fmaf(q, 1.f / 13, 1.f / 11);
+  p = __builtin_fmaf(q, p, 1.f / 9);
+  p = __builtin_fmaf(q, p, 1.f / 7);
+  p = __builtin_fmaf(q, p, 1.f / 5);
+  p = __builtin_fmaf(q, p, 1.f / 3);
+  const float s2 = s + s;
+  return fmaxf(z, 0.f) + __builtin_fmaf(s2 * q, p, s2);
+}
 }  // namespace khm
