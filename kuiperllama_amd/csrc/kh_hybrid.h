@@ -146,7 +146,7 @@ struct Hybrid {
   void *kx = nullptr, *vx = nullptr;
   int exp_keys = 0;
   bool any_latent = false;
-  int32_t *moe_id = nullptr, *moe_rows = nullptr, *moe_slot = nullptr, *n_tiles = nullptr;
+  int32_t *moe_id = nullptr, *moe_rows = nullptr, *moe_slot = nullptr, *moe_count = nullptr, *n_tiles = nullptr;
   LgTile* tiles = nullptr;
   int max_tiles = 0;
   int wl_rows = 0;        // rows wlogits / xw hold

@@ -607,7 +607,7 @@ int cache_rows(const HyLayer& l, int cache_len) { return l.mixer == HY_HEADS ? l
 int alloc_workspace(kh_model* m) {
   Hybrid& hy = *m->hy;
   const size_t T = (size_t)hy.tmax, Wp = (size_t)hy.c.widthp, es = hy.elem();
-  size_t f32a = 1, a0 = 1, a1 = 1, a2 = 1, dt = 1, bc = 1, z = 1, ends = 1, dtsum = 1, h = 1, hs = 1, y = 1, top = 1, tiles = 1;
+  size_t f32a = 1, a0 = 1, a1 = 1, a2 = 1, dt = 1, bc = 1, z = 1, ends = 1, dtsum = 1, h = 1, hs = 1, y = 1, top = 1, tiles = 1, experts = 1;
   auto up = [](size_t& v, size_t n) { v = v > n ? v : n; };
   const size_t multi = T / KH_SCAN_CH * 2 + 2;  // chunks of segments that have more than one
   if (hy.enter.N) up(a2, T * 2 * Wp);
@@ -642,6 +642,7 @@ int alloc_workspace(kh_model* m) {
       up(h, T * (size_t)f.top * (size_t)f.ffp);
       up(y, T * (size_t)f.top * Wp);
       up(top, (size_t)f.top);
+      up(experts, (size_t)f.E);
       up(hs, T * (size_t)f.sffp);
       up(tiles, T * (size_t)f.top / 32 + (size_t)f.E + 1);
     }
@@ -685,6 +686,7 @@ int alloc_workspace(kh_model* m) {
   TRY(zi(&hy.moe_id, T * top));
   TRY(zi(&hy.moe_rows, T * top));
   TRY(zi(&hy.moe_slot, T * top));
+  TRY(zi(&hy.moe_count, (size_t)moe_blocks((int)T) * experts));
   TRY(zi(&hy.n_tiles, 1));
   TRY(zi((int32_t**)&hy.tiles, tiles * 4));
   hy.max_tiles = (int)tiles;
@@ -877,7 +879,7 @@ void hy_destroy(kh_model* m) {
   if (!h) return;
   void* dev[] = {h->farena, h->state, h->x, h->x0, h->mix, h->f32a, h->y, h->sh, h->dt, h->bc, h->z, h->ends, h->dtsum,
                  h->moe_w, h->id_w, h->sh_g, h->wlogits, h->xn1, h->xn2, h->a0, h->a1, h->a2, h->h, h->hs, h->xw,
-                 h->moe_id, h->moe_rows, h->moe_slot, h->n_tiles, h->tiles, h->kx, h->vx, h->d_tab, h->d_one};
+                 h->moe_id, h->moe_rows, h->moe_slot, h->moe_count, h->n_tiles, h->tiles, h->kx, h->vx, h->d_tab, h->d_one};
   for (void* p : dev)
     if (p) (void)hipFree(p);
   for (float2* t : h->rope_tabs) (void)hipFree(t);

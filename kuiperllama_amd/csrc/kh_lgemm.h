@@ -1,11 +1,18 @@
 // kh_lgemm.h — GEMM of the layer-list models on the matrix cores: out[token][feature] = X[token][K] . W[feature][K],
 // storage type T = bf16 or fp32 on both sides (kh_tile.h), fp32 accumulation.
 //
-//   * One workgroup = 4 waves (2 x 2) = a BM-token x BN-feature tile; K advances 128 bytes per stage through a ring
-//     of NSTAGE LDS stages filled by the LDS-DMA path (global_load_lds_dwordx4): no staging registers, and
-//     NSTAGE - 1 stages are in flight while one is multiplied.  The big tiles use two stages, which leaves room for
-//     two workgroups per CU: one multiplies while the other waits (128 x 128: 0.43 - 0.50 of the bf16 peak, against
-//     0.28 - 0.33 with three stages and one workgroup).
+//   * One workgroup = 4 waves (2 x 2) = a BM-token x BN-feature tile; K advances 128 bytes per stage through two rings of
+//     LDS stages, XS of tokens and WS of weights, filled by the LDS-DMA path (global_load_lds_dwordx4): no staging
+//     registers, and XS - 1 and WS - 1 stages are in flight while one is multiplied.  The big tiles use two stages, which
+//     leaves room for two workgroups per CU: one multiplies while the other waits (128 x 128: 0.43 - 0.50 of the bf16 peak,
+//     against 0.28 - 0.33 with three stages and one workgroup).  Experts' weights come from HBM, each tile for two or three
+//     workgroups only, and wait for it longer than a stage's products take: the 80 KB that two workgroups leave each other
+//     hold a third stage of weights (2048 tokens, 6 of 32 experts, 2048 x 2048: 141 -> 130 us; 1100 tokens, 7 of 32,
+//     1024 x 1024: 41 -> 36).  Weights that all tokens share come from the L2, and two stages do as well there.  Measured
+//     and not kept: stages of 64 bytes, five of them (30 % slower: requests of half lines), fragments read one half stage
+//     ahead of their products (up to 20 % slower), the tiles of an expert on one XCD (+3 % at 2048 columns, -2 % at 1024).
+//   * Token tiles of 16 go to the two waves of a column in turn; a wave multiplies those that hold rows, so a tile that is
+//     not full costs what it holds.
 //   * LDS rows are 128 bytes.  Chunk c (16 bytes) of row r sits in slot c ^ (r & 7): the lanes of a fragment read
 //     (16 rows, same chunk) touch all 64 banks.  The DMA writes slots in lane order, so the permutation is applied
 //     to the GLOBAL address each lane requests.
@@ -16,6 +23,7 @@
 //   * Grouped form (experts): a device-side tile list maps blockIdx.y to (expert, first row, rows); the rows of X are
 //     gathered through an index list.  Batched form (heads): blockIdx.z strides.
 #pragma once
+#include <type_traits>
 #include <vector>
 
 #include "kh_q8ring.h"
@@ -54,11 +62,11 @@ struct LgArgs {
   GateAct act;          // LG_GATED
 };
 
-template <class T, int BM, int BN>
+template <class T, int BM, int BN, bool GROUPED>
 struct LgCfg {
-  static constexpr int NSTAGE = BM + BN >= 192 ? 2 : (BM + BN >= 128 ? 3 : 4);
-  static constexpr int STAGE = (BM + BN) * 128;
-  static constexpr int LDS = NSTAGE * STAGE;
+  static constexpr int XS = BM + BN >= 192 ? 2 : (BM + BN >= 128 ? 3 : 4);  // stages of the tokens' ring
+  static constexpr int WS = BM + BN >= 256 && GROUPED ? 3 : XS;             // ... of the weights'
+  static constexpr int LDS = (XS * BM + WS * BN) * 128;
 };
 
 // features f .. f + 3 of one token, f a multiple of four
@@ -108,20 +116,21 @@ __device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 
   }
 }
 
-template <class T, int BM, int BN, int EPI>
+template <class T, int BM, int BN, int EPI, bool GROUPED>
 __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   typedef Tile<T> TL;
   typedef typename TL::frag frag;
-  constexpr int NST = LgCfg<T, BM, BN>::NSTAGE, STAGE = LgCfg<T, BM, BN>::STAGE;
+  constexpr int XS = LgCfg<T, BM, BN, GROUPED>::XS, WS = LgCfg<T, BM, BN, GROUPED>::WS;
+  static_assert(XS >= 2 && WS >= XS, "order of the requests");
   constexpr int TM = BM / 32, TN = BN / 32;  // 16-wide tiles per wave: tokens, features
-  constexpr int NL = (BM + BN) / 32;         // LDS-DMA requests per wave and stage
+  constexpr int NX = BM / 32, NW = BN / 32;  // LDS-DMA requests per wave and stage
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const char* W = (const char*)a.W;
   const char* X = (const char*)a.X;
   int m_lo = 0, m_n = a.M;  // rows [m_lo, m_lo + m_n) of the row index space belong to this launch / group
   int mt0;                  // first row of the tile
-  if (a.tiles) {
+  if (GROUPED) {
     if ((int)blockIdx.y >= *a.n_tiles) return;  // uniform: the grid is an upper bound
     const LgTile t = a.tiles[blockIdx.y];
     W += (size_t)t.group * a.w_group * sizeof(T);
@@ -135,29 +144,35 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   X += (size_t)blockIdx.z * a.x_z * sizeof(T);
   const int f0 = (int)blockIdx.x * BN;
   const int m_last = m_lo + m_n - 1;
-  // ---- staging addresses: request j of wave w covers rows 8 (4 j + w) .. +8 of the stacked (tokens, features) tile
-  unsigned voff[NL];
+  // ---- staging addresses: request j of wave w covers rows 8 (4 j + w) .. +8 of the token tile, or of the feature tile
+  unsigned xoff[NX], woff[NW];
   const int sub = lane >> 3, ch = (lane & 7) ^ sub;
 #pragma unroll
-  for (int j = 0; j < NL; ++j) {
-    const int r = 8 * (4 * j + wave) + sub;
-    if (j < BM / 32) {
-      int m = mt0 + r;
-      m = m < m_last ? m : m_last;
-      const int row = a.gather ? a.gather[m] : m;
-      voff[j] = (unsigned)row * (unsigned)(a.ldx * (int)sizeof(T)) + 16u * ch;
-    } else {
-      int f = f0 + r - BM;
-      f = f < a.N ? f : a.N - 1;
-      voff[j] = (unsigned)f * (unsigned)(a.ldw * (int)sizeof(T)) + 16u * ch;
-    }
+  for (int j = 0; j < NX; ++j) {
+    int m = mt0 + 8 * (4 * j + wave) + sub;
+    m = m < m_last ? m : m_last;
+    const int row = GROUPED && a.gather ? a.gather[m] : m;
+    xoff[j] = (unsigned)row * (unsigned)(a.ldx * (int)sizeof(T)) + 16u * ch;
+  }
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    int f = f0 + 8 * (4 * j + wave) + sub;
+    f = f < a.N ? f : a.N - 1;
+    woff[j] = (unsigned)f * (unsigned)(a.ldw * (int)sizeof(T)) + 16u * ch;
   }
   const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane((int)kh_lds_addr(smem_raw)) + 1024u * wave;
-  auto issue = [&](int slot) __attribute__((always_inline)) {
+  auto issue_x = [&](int slot) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < NL; ++j) {
-      dma_x4_keep(j < BM / 32 ? (const void*)X : (const void*)W, voff[j], lds0 + (unsigned)(slot * STAGE + j * 4096));
-      voff[j] += 128;
+    for (int j = 0; j < NX; ++j) {
+      dma_x4_keep(X, xoff[j], lds0 + (unsigned)(slot * BM * 128 + j * 4096));
+      xoff[j] += 128;
+    }
+  };
+  auto issue_w = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      dma_x4_keep(W, woff[j], lds0 + (unsigned)(XS * BM * 128 + slot * BN * 128 + j * 4096));
+      woff[j] += 128;
     }
   };
   const int nk = a.K * (int)sizeof(T) / 128;  // stages
@@ -167,48 +182,61 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
 #pragma unroll
     for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (s < nk) issue(s);
+  for (int j = 0; j < WS - 1; ++j) {  // as WS - 1 steps before the first would request them
+    if (j >= WS - XS && j - (WS - XS) < nk) issue_x(j - (WS - XS));
+    if (j < nk) issue_w(j);
+  }
   const int wm = wave & 1, wn = wave >> 1;
   const int fr = lane & 15, fh = lane >> 4;
-  int slot = 0, fill = NST - 1;
-  for (int k = 0; k < nk; ++k) {
-    // stage k has landed when at most the requests of the stages behind it are outstanding
-    if (k + NST - 2 < nk) wait_vm<(NST - 2) * NL>();
-    else wait_vm<0>();
-    __syncthreads();
-    if (k + NST - 1 < nk) issue(fill);
-    const char* st = smem_raw + slot * STAGE;
-    // both halves of the stage are requested from LDS before the first product: the second half arrives under the
-    // products of the first (left to itself the compiler reads one half at a time; 0.40 -> 0.43 ... 0.50 of the peak)
-    frag fx[2][TM], fw[2][TN];
+  const int fo0 = fr * 128 + ((fh ^ (fr & 7)) << 4);  // this lane's fragment within 16 rows, first half of the stage
+  constexpr int LATER = WS > XS ? NW : 0;             // requests of a step behind the ones that are waited for
+  // LIVE: token tiles of this wave that hold rows
+  auto loop = [&](auto live) __attribute__((always_inline)) {
+    constexpr int LIVE = decltype(live)::value;
+    int xslot = 0, wslot = 0, xfill = XS - 1, wfill = WS - 1;
+    auto next = [](int s, int n) __attribute__((always_inline)) { return s + 1 == n ? 0 : s + 1; };
+    for (int k = 0; k < nk; ++k) {
+      // stage k has landed when at most the requests behind it are outstanding
+      if (k + WS - 2 < nk) wait_vm<LATER + (XS - 2) * (NX + NW)>();
+      else wait_vm<0>();
+      __syncthreads();
+      if (k + XS - 1 < nk) issue_x(xfill);
+      if (k + WS - 1 < nk) issue_w(wfill);
+      // both halves of the stage are requested from LDS before the first product: the second half arrives under the
+      // products of the first (left to itself the compiler reads one half at a time; 0.40 -> 0.43 ... 0.50 of the peak)
+      frag fx[2][LIVE], fw[2][TN];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+      for (int b = 0; b < 2; ++b) {
+        const char* sx = smem_raw + xslot * BM * 128 + (fo0 ^ (b << 6));
+        const char* sw = smem_raw + XS * BM * 128 + wslot * BN * 128 + (fo0 ^ (b << 6));
 #pragma unroll
-      for (int m = 0; m < TM; ++m) {
-        const int r = wm * (BM / 2) + m * 16 + fr;
-        fx[b][m] = *(const frag*)(st + r * 128 + (((4 * b + fh) ^ (r & 7)) << 4));
+        for (int m = 0; m < LIVE; ++m) fx[b][m] = *(const frag*)(sx + (2 * m + wm) * 2048);
+#pragma unroll
+        for (int n = 0; n < TN; ++n) fw[b][n] = *(const frag*)(sw + (wn * TN + n) * 2048);
       }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        const int r = BM + wn * (BN / 2) + n * 16 + fr;
-        fw[b][n] = *(const frag*)(st + r * 128 + (((4 * b + fh) ^ (r & 7)) << 4));
-      }
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+          for (int m = 0; m < LIVE; ++m) acc[n][m] = TL::mma(fw[b][n], fx[b][m], acc[n][m]);
+      xslot = next(xslot, XS);
+      wslot = next(wslot, WS);
+      xfill = next(xfill, XS);
+      wfill = next(wfill, WS);
     }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int n = 0; n < TN; ++n)
-#pragma unroll
-        for (int m = 0; m < TM; ++m) acc[n][m] = TL::mma(fw[b][n], fx[b][m], acc[n][m]);
-    slot = slot + 1 == NST ? 0 : slot + 1;
-    fill = fill + 1 == NST ? 0 : fill + 1;
-  }
+  };
+  const int tiles_m = (m_last - mt0) / 16 + 1;  // of the workgroup, with rows in them; they go to the waves in turn
+  const int live = (tiles_m - wm + 1) / 2;
+  if (TM == 1 || live <= 1) loop(std::integral_constant<int, 1>{});
+  else if (TM == 2 || live == 2) loop(std::integral_constant<int, TM < 2 ? 1 : 2>{});
+  else if (live == 3) loop(std::integral_constant<int, TM < 3 ? 1 : 3>{});
+  else loop(std::integral_constant<int, TM>{});
   // ---- epilogue: lane (fr, fh) of tile (n, m): token mt0 + .. + fr, features f .. f + 3
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
-    const int tok = mt0 + wm * (BM / 2) + m * 16 + fr;
+    const int tok = mt0 + (2 * m + wm) * 16 + fr;
     if (tok > m_last) continue;
     if (EPI == LG_GATED) {
 #pragma unroll
@@ -227,9 +255,8 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   }
 }
 
-// Tile choice.  Plain / batched launches: the largest tile that still gives the chip enough workgroups (one per CU is
-// not: nobody covers its barriers).  Grouped
-// launches: BM = the row granule the tile list was built with (lg_group_bm).
+// Tile choice.  Plain / batched launches: the largest tile that still gives the chip enough workgroups (one per CU is not:
+// nobody covers its barriers).  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
 static inline int lg_group_bm(long rows, int groups) {
   const long per = rows / (groups > 0 ? groups : 1);
   return per > 64 ? 128 : (per > 24 ? 64 : 32);
@@ -255,10 +282,20 @@ int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, in
     return KH_OK;
   };
   auto tiles = [&](int BM, int BN) { return (long)((a.N + BN - 1) / BN) * ((a.M + BM - 1) / BM) * zdim; };
-  if (a.tiles ? group_bm == 128 : a.M > 64 && tiles(128, 128) >= 400)
-    return go(k_lgemm<T, 128, 128, EPI>, 128, 128, LgCfg<T, 128, 128>::LDS);
-  if (a.tiles ? group_bm == 32 : a.M <= 32) return go(k_lgemm<T, 32, 64, EPI>, 32, 64, LgCfg<T, 32, 64>::LDS);
-  if (a.tiles || tiles(64, 128) >= 400) return go(k_lgemm<T, 64, 128, EPI>, 64, 128, LgCfg<T, 64, 128>::LDS);
-  return go(k_lgemm<T, 64, 64, EPI>, 64, 64, LgCfg<T, 64, 64>::LDS);
+#define KH_LG_GO(BM, BN, G) return go(k_lgemm<T, BM, BN, EPI, G>, BM, BN, LgCfg<T, BM, BN, G>::LDS)
+  if constexpr (EPI == LG_T || EPI == LG_GATED) {
+    if (a.tiles) {
+      if (group_bm == 128) KH_LG_GO(128, 128, true);
+      if (group_bm == 64) KH_LG_GO(64, 128, true);
+      KH_LG_GO(32, 64, true);
+    }
+  } else if (a.tiles) {
+    return KH_ERR_INTERNAL;
+  }
+  if (a.M > 64 && tiles(128, 128) >= 400) KH_LG_GO(128, 128, false);
+  if (a.M <= 32) KH_LG_GO(32, 64, false);
+  if (tiles(64, 128) >= 400) KH_LG_GO(64, 128, false);
+  KH_LG_GO(64, 64, false);
+#undef KH_LG_GO
 }
 }  // namespace khm

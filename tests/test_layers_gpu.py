@@ -71,6 +71,22 @@ def test_experts_alone(gpu, dtype, kw):
 
 
 @BOTH
+@pytest.mark.parametrize("n,kw", [(15, dict(experts=2, top=1)), (16, dict(experts=2, top=2)), (17, dict(experts=3, top=2)),
+                                  (129, dict(experts=1, top=1)), (130, dict(experts=2, top=2)), (209, dict(experts=3, top=2)),
+                                  (257, dict(experts=5, identity=0, top=4)), (400, dict(experts=2, top=1, ff=70)),
+                                  (95, dict(experts=1000, identity=20, top=3, ff=4))])
+def test_expert_tiles(gpu, dtype, n, kw):
+    """Rows of an expert around the tiles of 32, 64 and 128 and the units of 16 that a tile is made of, counts of the routing
+    workgroups (16 tokens each) that end inside one, as many experts as the lists hold."""
+    mod = U.Model(U.config([U.with_ff(U.mamba(), **kw), U.mamba()]))
+    m = mod.load(dtype)
+    toks = mod.tokens(n)
+    got = m.forward([(m.open_seq(), toks, list(range(n)))])
+    m.close()
+    U.check(got, mod.logits(toks), dtype, "prompt")
+
+
+@BOTH
 @pytest.mark.parametrize("loop", [None, (0, 1, 1), (0, 2, 3), (1, 3, 2), (2, 3, 2)])
 def test_loop_ranges(gpu, dtype, loop):
     layers = [U.with_ff(U.latent()), U.mamba(), U.with_ff(U.latent(2), identity=0)]
