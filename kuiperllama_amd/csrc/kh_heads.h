@@ -94,19 +94,28 @@ struct HeadsArgs {
   PassTabs p;
 };
 
-// KN, KV: key and value size in units of 64.  CP = 4: 16 rows per workgroup; CP = 1: 64 MR rows.
+// stages of a key tile of tb bytes, ks sets of them
+constexpr int heads_stages(int tb, int ks) { return tb <= 24 * 1024 && 3 * ks * tb <= 144 * 1024 ? 3 : 2; }
+
+// KN, KV: key and value size in units of 64.  CP = 4: 16 rows per workgroup; CP = 1: 64 MR rows.  KS = 2: eight waves, the
+// second four take every other key tile of the same rows and are merged at the end through LDS.  A tile of 32 keys is a serial
+// chain (keys from LDS, scores, maximum, exponentials, values: 1.1 us for 0.1 us of products), so a wave needs another one on
+// its SIMD; where the rows of a launch make one workgroup per CU, KS = 2 is where it comes from.
 // Two waves per SIMD where the accumulators allow it: within 256 registers the compiler keeps them where the rescaling can
 // reach them (beyond, it moves them between two register files in every tile).
-template <class T, int KN, int KV, int CP, int MR>
-__global__ __launch_bounds__(256, KN + KV > 4 ? 1 : 2) void k_heads_attn(const HeadsArgs a) {
+template <class T, int KN, int KV, int CP, int MR, int KS>
+__global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_heads_attn(const HeadsArgs a) {
   typedef Tile<T> TL;
   typedef typename TL::frag frag;
   constexpr int E = TL::N, KT = 4 * E, NS = KT / 16, ES = (int)sizeof(T);
   constexpr int DK = 64 * KN, DV = 64 * KV, ROW = DK + DV, CB = ROW / E;
   constexpr int NQ = DK / (4 * E), NT = DV / 16 / CP, NL = ROW / 64;
-  constexpr int TB = KT * ROW * ES, NST = TB <= 24 * 1024 ? 3 : 2, WR = 4 / CP, ROWS = 16 * MR * WR;
+  constexpr int TB = KT * ROW * ES, NST = heads_stages(TB, KS), WR = 4 / CP, ROWS = 16 * MR * WR;
+  constexpr int BOX = 4 * MR * NT * 1024 + 2048 * MR;  // what a set of four waves hands over
+  static_assert((KS - 1) * BOX <= KS * NST * TB, "fits the stages");
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave8 & 3, ks = KS == 1 ? 0 : wave8 >> 2;
   const int fr = lane & 15, fh = lane >> 4, wr = wave % WR, wc = wave / WR;
   const int g = blockIdx.x, per = a.H / a.G;
   LatTile tl;
@@ -153,6 +162,33 @@ __global__ __launch_bounds__(256, KN + KV > 4 ? 1 : 2) void k_heads_attn(const H
   int my_first[MR];
 #pragma unroll
   for (int q = 0; q < MR; ++q) my_first[q] = a.span.first(my_pos[q]);
+  // ---- staging: request j of a wave covers chunks (4 j + wave) 64 .. of the tile; slot s of row r holds chunk s ^ (r & 7)
+  int kr[NL];
+  unsigned kc[NL];
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {
+    const int c = (4 * j + wave) * 64 + lane;
+    kr[j] = c / CB;
+    kc[j] = (unsigned)(((c - kr[j] * CB) ^ (kr[j] & 7)) << 4);
+  }
+  const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane((int)kh_lds_addr(smem_raw)) + 1024u * wave + (unsigned)(ks * NST * TB);
+  const unsigned row_b = (unsigned)(a.G * ROW * ES);
+  int fill_row = (k_lo + ks * KT) % a.ring;  // cache row of the next tile to request
+  auto issue = [&](int slot, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int k = k0 + kr[j] < n_keys ? kr[j] : n_keys - 1 - k0;  // rows behind the sequence's last may not be backed
+      int r = fill_row + k;
+      r = r < a.ring ? r : r - a.ring;
+      dma_x4_keep(cache, (unsigned)r * row_b + kc[j], lds0 + (unsigned)(slot * TB + 4096 * j));
+    }
+    fill_row += KS * KT;
+    if (fill_row >= a.ring) fill_row -= a.ring;
+  };
+  constexpr int DK0 = KS * KT;  // from one tile of a wave to its next
+#pragma unroll
+  for (int i = 0; i < NST - 1; ++i)
+    if (k_lo + ks * KT + i * DK0 < k_hi) issue(i, k_lo + ks * KT + i * DK0);
   // ---- queries: norm and scale in registers (a row's elements lie in the four lanes fr, fr + 16, ...)
   frag fq[MR][NQ];
 #pragma unroll
@@ -191,59 +227,35 @@ __global__ __launch_bounds__(256, KN + KV > 4 ? 1 : 2) void k_heads_attn(const H
       }
   }
   // ---- distance bias: the group's rows of the table to LDS when a key of this workgroup is near enough to need them
-  float* tab = (float*)(smem_raw + NST * TB);
+  float* tab = (float*)(smem_raw + KS * NST * TB);
   float far[MR];
 #pragma unroll
   for (int q = 0; q < MR; ++q) far[q] = a.bias ? a.bias[(size_t)head[q] * a.nbias + a.nbias - 1] : 0.f;
   if (a.bias && a.bias_lds && pos_of(tl.r0) - (k_hi - 1) < a.nbias - 1)
-    for (int i = threadIdx.x; i < per * a.nbias; i += 256) tab[i] = a.bias[(size_t)g * per * a.nbias + i];
-  // ---- staging: request j of a wave covers chunks (4 j + wave) 64 .. of the tile; slot s of row r holds chunk s ^ (r & 7)
-  int kr[NL];
-  unsigned kc[NL];
-#pragma unroll
-  for (int j = 0; j < NL; ++j) {
-    const int c = (4 * j + wave) * 64 + lane;
-    kr[j] = c / CB;
-    kc[j] = (unsigned)(((c - kr[j] * CB) ^ (kr[j] & 7)) << 4);
-  }
-  const unsigned lds0 = (unsigned)__builtin_amdgcn_readfirstlane((int)kh_lds_addr(smem_raw)) + 1024u * wave;
-  const unsigned row_b = (unsigned)(a.G * ROW * ES);
-  int fill_row = k_lo % a.ring;  // cache row of the next tile to request
-  auto issue = [&](int slot, int k0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < NL; ++j) {
-      const int k = k0 + kr[j] < n_keys ? kr[j] : n_keys - 1 - k0;  // rows behind the sequence's last may not be backed
-      int r = fill_row + k;
-      r = r < a.ring ? r : r - a.ring;
-      dma_x4_keep(cache, (unsigned)r * row_b + kc[j], lds0 + (unsigned)(slot * TB + 4096 * j));
-    }
-    fill_row += KT;
-    if (fill_row >= a.ring) fill_row -= a.ring;
-  };
+    for (int i = threadIdx.x; i < per * a.nbias; i += 256 * KS) tab[i] = a.bias[(size_t)g * per * a.nbias + i];
   float m[MR], l[MR];
   f32x4 o[MR][NT];
 #pragma unroll
   for (int q = 0; q < MR; ++q) {
-    const bool sinks = a.sink && (a.nsplit == 1 || blockIdx.z == 0);
+    const bool sinks = a.sink && (a.nsplit == 1 || blockIdx.z == 0) && ks == 0;
     m[q] = sinks ? 0.f : -1e30f;  // finite: a row without a visible key yet keeps weights of zero, not NaN
     l[q] = sinks && fh == 0 ? 1.f : 0.f;
 #pragma unroll
     for (int n = 0; n < NT; ++n) o[q][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-#pragma unroll
-  for (int i = 0; i < NST - 1; ++i)
-    if (k_lo + i * KT < k_hi) issue(i, k_lo + i * KT);
   int slot = -1, fill = NST - 2;
-  for (int k0 = k_lo; k0 < k_hi; k0 += KT) {
+  for (int kb = k_lo; kb < k_hi; kb += DK0) {
+    const int k0 = kb + ks * KT;
     slot = slot + 1 == NST ? 0 : slot + 1;
     fill = fill + 1 == NST ? 0 : fill + 1;
     // this stage has landed when only the younger NST - 2 stages are outstanding
-    if (k0 + (NST - 2) * KT < k_hi) wait_vm<(NST - 2) * NL>();
+    if (k0 + (NST - 2) * DK0 < k_hi) wait_vm<(NST - 2) * NL>();
     else wait_vm<0>();
     __syncthreads();
-    if (k0 + (NST - 1) * KT < k_hi) issue(fill, k0 + (NST - 1) * KT);
-    if (k0 > p_hi || k0 + KT <= w_first) continue;  // nothing in this tile for the wave (barriers stay uniform)
-    const char* Kt = smem_raw + slot * TB;
+    if (k0 + (NST - 1) * DK0 < k_hi) issue(fill, k0 + (NST - 1) * DK0);
+    // nothing in this tile for the wave (barriers stay uniform)
+    if (k0 > p_hi || k0 + KT <= w_first || (KS > 1 && k0 >= k_hi)) continue;
+    const char* Kt = smem_raw + (ks * NST + slot) * TB;
     f32x4 s[MR][NS];
 #pragma unroll
     for (int q = 0; q < MR; ++q)
@@ -331,8 +343,45 @@ __global__ __launch_bounds__(256, KN + KV > 4 ? 1 : 2) void k_heads_attn(const H
   }
 #pragma unroll
   for (int q = 0; q < MR; ++q) {
-    float sum = xor16_sum(l[q]);
-    sum = xor32_sum(sum);
+    l[q] = xor16_sum(l[q]);
+    l[q] = xor32_sum(l[q]);
+  }
+  if (KS > 1) {  // the sets of waves hold the same rows and columns lane by lane
+    __syncthreads();
+    auto box = [&](int set) __attribute__((always_inline)) { return (f32x4*)(smem_raw + (set - 1) * BOX) + wave * MR * NT * 64 + lane; };
+    auto ml = [&](int set) __attribute__((always_inline)) {
+      return (float*)(smem_raw + (set - 1) * BOX + 4 * MR * NT * 1024) + wave * MR * 128 + lane;
+    };
+    if (ks) {
+#pragma unroll
+      for (int q = 0; q < MR; ++q) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) box(ks)[(q * NT + n) * 64] = o[q][n];
+        ml(ks)[q * 128] = m[q];
+        ml(ks)[q * 128 + 64] = l[q];
+      }
+    }
+    __syncthreads();
+    if (ks) return;
+#pragma unroll
+    for (int set = 1; set < KS; ++set)
+#pragma unroll
+      for (int q = 0; q < MR; ++q) {
+        const float m1 = ml(set)[q * 128], l1 = ml(set)[q * 128 + 64], mx = fmaxf(m[q], m1);
+        const float f0 = __builtin_amdgcn_exp2f(m[q] - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
+        m[q] = mx;
+        l[q] = __builtin_fmaf(l1, f1, l[q] * f0);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const f32x4 b = box(set)[(q * NT + n) * 64];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[q][n][i] = __builtin_fmaf(b[i], f1, o[q][n][i] * f0);
+        }
+      }
+  }
+#pragma unroll
+  for (int q = 0; q < MR; ++q) {
+    const float sum = l[q];
     if (!live[q]) continue;
     if (a.nsplit == 1) {
       const float inv = 1.0f / sum;

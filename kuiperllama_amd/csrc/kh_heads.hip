@@ -12,8 +12,8 @@ int heads_attn_launch(hipStream_t s, HeadsArgs a, int ntiles, int rows) {
     return KH_ERR_INTERNAL;
   const size_t table = (size_t)(a.H / a.G) * a.nbias * sizeof(float);
   a.bias_lds = a.bias && table <= KH_HEADS_BIAS_LDS;
-  auto go = [&](auto kern, size_t stage) -> int {
-    const size_t lds = stage * (stage <= 24 * 1024 ? 3 : 2) + (a.bias_lds ? table : 0);
+  auto go = [&](auto kern, size_t stage, int ks) -> int {
+    const size_t lds = stage * heads_stages((int)stage, ks) * ks + (a.bias_lds ? table : 0);
     if (lds > 64 * 1024) {
       struct Done { int dev; const void* fn; size_t lds; };
       static thread_local std::vector<Done> done;
@@ -27,16 +27,21 @@ int heads_attn_launch(hipStream_t s, HeadsArgs a, int ntiles, int rows) {
         done.push_back({dev, (const void*)kern, lds});
       }
     }
-    hipLaunchKernelGGL(kern, dim3(a.G, ntiles, a.nsplit), dim3(256), lds, s, a);
+    hipLaunchKernelGGL(kern, dim3(a.G, ntiles, a.nsplit), dim3(256 * ks), lds, s, a);
     return KH_OK;
   };
   auto by_rows = [&](auto kn, auto kv) -> int {
     constexpr int KN = decltype(kn)::value, KV = decltype(kv)::value;
     const size_t stage = (size_t)4 * Tile<T>::N * (a.dkp + a.dvp) * sizeof(T);
-    if (rows == 16) return go(k_heads_attn<T, KN, KV, 4, 1>, stage);
-    if (rows == 64) return go(k_heads_attn<T, KN, KV, 1, 1>, stage);
+    if (rows == 16) return go(k_heads_attn<T, KN, KV, 4, 1, 1>, stage, 1);
+    // at most one workgroup per CU: two sets of waves, which share the keys (1100 tokens of 2 x 4 heads of 128, 138 workgroups:
+    // 37.2 -> 27.6 us; four sets on tiles of 32 rows 25.9, at twice the key traffic).  Keys and values of more than 256
+    // elements together need the registers of a wave alone on its SIMD.
+    if constexpr (KN + KV <= 4)
+      if (rows == 64 && a.tiles && (long)ntiles * a.G <= 256) return go(k_heads_attn<T, KN, KV, 1, 1, 2>, stage, 2);
+    if (rows == 64) return go(k_heads_attn<T, KN, KV, 1, 1, 1>, stage, 1);
     if constexpr (sizeof(T) == 2 && KN <= 2 && KV <= 2)
-      if (rows == 128) return go(k_heads_attn<T, KN, KV, 1, 2>, stage);
+      if (rows == 128) return go(k_heads_attn<T, KN, KV, 1, 2, 1>, stage, 1);
     return KH_ERR_INTERNAL;
   };
   auto by_value = [&](auto kn) -> int {

@@ -163,6 +163,19 @@ def test_every_row_tile(gpu, dtype, rows, kw, hook):
     m.close()
 
 
+@BOTH
+@pytest.mark.parametrize("n,heads,kv_heads", [(33, 4, 2), (65, 2, 1), (160, 6, 2), (256, 64, 32), (257, 64, 32)])
+def test_waves_that_share_keys(gpu, dtype, n, heads, kv_heads):
+    """64-row tiles on fewer workgroups than CUs (two sets of waves, every other key tile) and on more (one set): one and two key
+    tiles, an odd number of them, the first launch that fills the chip."""
+    kw = dict(heads=heads, kv_heads=kv_heads, dim=32, vdim=48)
+    mod = U.Model(U.gusorax([U.windowed(window=70, rows=16, far=50.0, **kw), U.chunked(chunk=90, **kw), U.chunked(chunk=400, **kw)]))
+    toks = mod.tokens(n)
+    m = mod.load(dtype)
+    U.check(U.run_alone(m, toks), mod.logits(toks), dtype, "prompt")
+    m.close()
+
+
 def test_prompt_of_several_passes(gpu):
     """More tokens than one pass holds."""
     mod = U.Model(U.gusorax([U.windowed(8, 2, 16, 16, 0.4, 300, 16, 100.0), dict(U.chunked(16, 8, 8, 8, 0.5, 256), mlp=U.clamped(3, 2, 8))],
