@@ -356,9 +356,15 @@ struct Runner {
   }
   int experts(const HyMoe& f, const void* in) {
     const int W = hy.c.width, Wp = hy.c.widthp;
-    TRY((lg_launch<T, LG_F32>(s, gemm(f.zr, in, Wp, hy.z, f.zr.N))));
-    RouteArgs ra{hy.z, f.corr.p, hy.moe_id, hy.moe_w, hy.id_w, hy.sh_g, hy.moe_count, hy.moe_slot, ps.T, f.zr.N, f.n_out(), f.E, f.top, f.sgate, f.over_chosen};
-    moe_route_launch(s, ra);
+    const RouteArgs ra{hy.z, f.corr.p, hy.moe_id, hy.moe_w, hy.id_w, hy.sh_g, hy.moe_count, hy.moe_slot, ps.T, f.zr.N, f.n_out(),
+                       f.E, f.top, f.sgate, f.over_chosen};
+    const LgArgs zr = gemm(f.zr, in, Wp, hy.z, f.zr.N);
+    if (f.zr.N <= 64) {
+      moe_gate_launch<T>(s, MoeGateArgs{zr.X, zr.W, zr.ldx, zr.ldw, zr.K, ra});
+    } else {
+      TRY((lg_launch<T, LG_F32>(s, zr)));
+      moe_route_launch(s, ra);
+    }
     const int bm = lg_group_bm((long)ps.T * f.top, f.n_out());
     ListArgs li{hy.moe_id, hy.moe_count, hy.moe_rows, hy.moe_slot, hy.tiles, hy.n_tiles, ps.T, f.top, f.E, bm};
     hipLaunchKernelGGL(k_moe_lists, dim3(moe_blocks(ps.T)), dim3(KH_MOE_LT), 0, s, li);

@@ -82,8 +82,7 @@ struct RouteArgs {
   int T, ldz, n_out, n_expert, top, shared, over_chosen;
 };
 template <int PER>
-__device__ __forceinline__ void moe_route_token(const RouteArgs& a, int t, int lane, int32_t* cnt) {
-  const float* z = a.z + (size_t)t * a.ldz;
+__device__ __forceinline__ void moe_route_token(const RouteArgs& a, const float* z, int t, int lane, int32_t* cnt) {
   float idw = 0.f, my_w = 0.f;
   int my_id = 0;
   const float f = moe_route<PER>(z, a.corr, a.n_out, a.top, a.over_chosen, lane, [&](int k, int id, float w) __attribute__((always_inline)) {
@@ -107,7 +106,7 @@ __global__ __launch_bounds__(64 * KH_MOE_RT) void k_moe_route(const RouteArgs a)
   for (int e = threadIdx.x; e < a.n_expert; e += 64 * KH_MOE_RT) cnt[e] = 0;
   __syncthreads();
   const int t = blockIdx.x * KH_MOE_RT + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t < a.T) moe_route_token<PER>(a, t, lane, cnt);
+  if (t < a.T) moe_route_token<PER>(a, a.z + (size_t)t * a.ldz, t, lane, cnt);
   __syncthreads();
   for (int e = threadIdx.x; e < a.n_expert; e += 64 * KH_MOE_RT) a.count[(size_t)blockIdx.x * a.n_expert + e] = cnt[e];
 }
@@ -115,10 +114,90 @@ static inline int moe_blocks(int T) { return (T + KH_MOE_RT - 1) / KH_MOE_RT; }
 static inline int moe_per(int n_out) { return n_out <= 64 ? 1 : (n_out <= 256 ? 4 : 16); }
 static inline void moe_route_launch(hipStream_t s, const RouteArgs& a) {
   const dim3 g(moe_blocks(a.T)), b(64 * KH_MOE_RT);
-  const int per = moe_per(a.n_out);
-  if (per == 1) hipLaunchKernelGGL(k_moe_route<1>, g, b, 0, s, a);
-  else if (per == 4) hipLaunchKernelGGL(k_moe_route<4>, g, b, 0, s, a);
+  if (moe_per(a.n_out) <= 4) hipLaunchKernelGGL(k_moe_route<4>, g, b, 0, s, a);
   else hipLaunchKernelGGL(k_moe_route<16>, g, b, 0, s, a);
+}
+
+// Router of at most 64 outputs, product and choice in one launch: a workgroup takes 16 tokens, its 16 waves 128 bytes of K each
+// in turn, straight from memory to fragments (nobody reads a row twice), and then a token each.  Bound by what one CU can
+// pull, and by the chain of the choices: as a GEMM tile of 64 tokens every workgroup drew 64 rows of activations and 64 of
+// weights through its CU, 13.3 us for 2048 tokens x 37 outputs x 2048 on 32 CUs, and the choices took 6.3 more; this 14.3
+// (1100 tokens x 32 x 1024: 13.6 -> 10.4).  More outputs than 64 go through the GEMM.  NT: 16-wide tiles of outputs.
+struct MoeGateArgs {
+  const void *X, *W;  // [T][ldx], [n_out + shared][ldw], the storage type
+  int ldx, ldw, K;
+  RouteArgs r;
+};
+template <class T, int NT>
+__global__ __launch_bounds__(64 * KH_MOE_RT) void k_moe_gate(const MoeGateArgs a) {
+  typedef Tile<T> TL;
+  typedef typename TL::frag frag;
+  constexpr int N = 16 * NT, LD = N + 4, HALF = KH_MOE_RT / 2;
+  __shared__ __attribute__((aligned(16))) float part[HALF][16][LD];
+  __shared__ float zs[16][N + 1];
+  __shared__ int32_t cnt[64];
+  const RouteArgs& r = a.r;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fh = lane >> 4;
+  const int t0 = (int)blockIdx.x * KH_MOE_RT, rows = r.n_out + r.shared;
+  if (threadIdx.x < 64) cnt[threadIdx.x] = 0;
+  const char* x = (const char*)a.X + (size_t)(t0 + fr < r.T ? t0 + fr : r.T - 1) * a.ldx * sizeof(T) + 16 * fh;
+  const char* w[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+    w[n] = (const char*)a.W + (size_t)(16 * n + fr < rows ? 16 * n + fr : rows - 1) * a.ldw * sizeof(T) + 16 * fh;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int np = a.K * (int)sizeof(T) / 128;
+  for (int p = wave; p < np; p += 2 * KH_MOE_RT) {
+    const bool two = p + KH_MOE_RT < np;  // uniform
+    frag fx[4], fw[4][NT];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const size_t at = (size_t)(b < 2 || !two ? p : p + KH_MOE_RT) * 128 + 64 * (b & 1);
+      fx[b] = *(const frag*)(x + at);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) fw[b][n] = *(const frag*)(w[n] + at);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (b < 2 || two)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = TL::mma(fw[b][n], fx[b], acc[n]);
+  }
+  // lane: outputs 16 n + 4 fh + i of token fr
+  if (wave >= HALF)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) *(f32x4*)&part[wave - HALF][fr][16 * n + 4 * fh] = acc[n];
+  __syncthreads();
+  if (wave < HALF)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      f32x4* q = (f32x4*)&part[wave][fr][16 * n + 4 * fh];
+      *q = acc[n] + *q;
+    }
+  __syncthreads();
+  if (threadIdx.x < 16 * N) {
+    const int t = threadIdx.x / N, f = threadIdx.x - t * N;
+    float z = part[0][t][f];
+#pragma unroll
+    for (int h = 1; h < HALF; ++h) z += part[h][t][f];
+    zs[t][f] = z;
+  }
+  __syncthreads();
+  if (t0 + wave < r.T) moe_route_token<1>(r, zs[wave], t0 + wave, lane, cnt);
+  __syncthreads();
+  if ((int)threadIdx.x < r.n_expert) r.count[(size_t)blockIdx.x * r.n_expert + threadIdx.x] = cnt[threadIdx.x];
+}
+template <class T>
+void moe_gate_launch(hipStream_t s, const MoeGateArgs& a) {
+  const dim3 g(moe_blocks(a.r.T)), b(64 * KH_MOE_RT);
+  switch ((a.r.n_out + a.r.shared + 15) / 16) {
+    case 1: hipLaunchKernelGGL((k_moe_gate<T, 1>), g, b, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_moe_gate<T, 2>), g, b, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((k_moe_gate<T, 3>), g, b, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_moe_gate<T, 4>), g, b, 0, s, a); break;
+  }
 }
 
 // Dispatch lists: rows grouped by expert (row -> token), slot of every (token, choice) in that order (-1: identity expert),
@@ -126,7 +205,7 @@ static inline void moe_route_launch(hipStream_t s, const RouteArgs& a) {
 // what a tile lacks in units of 16 rows).  Latency alone: one workgroup per routing workgroup adds up the counts of all of
 // them, four requests a thread at once, and places its own tokens.  One workgroup that counted every choice in LDS, where 64
 // lanes meet on a few counters, took 11.5 us for 2048 x 6 choices of 32 experts and 8.4 for 1100 x 7; with the counts from the
-// router (4.8 -> 6.2 us there) this takes 4.9.
+// router this takes 4.9.
 struct ListArgs {
   const int32_t *id, *count;  // [T][top], [blocks][n_expert]
   int32_t *rows, *slot;       // slot: ranks before, slots behind

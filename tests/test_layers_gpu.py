@@ -74,10 +74,13 @@ def test_experts_alone(gpu, dtype, kw):
 @pytest.mark.parametrize("n,kw", [(15, dict(experts=2, top=1)), (16, dict(experts=2, top=2)), (17, dict(experts=3, top=2)),
                                   (129, dict(experts=1, top=1)), (130, dict(experts=2, top=2)), (209, dict(experts=3, top=2)),
                                   (257, dict(experts=5, identity=0, top=4)), (400, dict(experts=2, top=1, ff=70)),
-                                  (95, dict(experts=1000, identity=20, top=3, ff=4))])
+                                  (19, dict(experts=14, identity=1, top=2)), (33, dict(experts=32, identity=0, top=5, shared=0)),
+                                  (47, dict(experts=60, identity=3, top=4, shared=0)), (48, dict(experts=60, identity=4, top=4)),
+                                  (31, dict(experts=62, identity=3, top=4, shared=0)), (95, dict(experts=1000, identity=20, top=3, ff=4))])
 def test_expert_tiles(gpu, dtype, n, kw):
     """Rows of an expert around the tiles of 32, 64 and 128 and the units of 16 that a tile is made of, counts of the routing
-    workgroups (16 tokens each) that end inside one, as many experts as the lists hold."""
+    workgroups (16 tokens each) that end inside one, as many experts as the lists hold; router outputs around the tiles of 16
+    and the 64 that routing does in one launch."""
     mod = U.Model(U.config([U.with_ff(U.mamba(), **kw), U.mamba()]))
     m = mod.load(dtype)
     toks = mod.tokens(n)
