@@ -84,7 +84,8 @@ struct HeadsArgs {
   const void* cache;     // + slot * slot_elems + row * G (dkp + dvp)
   size_t slot_elems;
   const float* bias;     // [H][nbias] by distance, in units of log2(e); the last entry holds for everything beyond.  nullptr: none
-  void* out;             // T [T][ldo], heads dvr apart (one split)
+  void* out;             // [T][ldo], heads dvr apart (one split): T, or fp32
+  int out_f32;
   float* part;           // splits > 1: [T H][splits][dvp + 4]: o (unnormalised), m, l.  One token per segment then
   const LatTile* tiles;  // nullptr: one token per segment, ceil((H / G) / rows of a tile) workgroups each
   int H, G, dk, dkr, dkp, dvr, dvp, ldr, ldo, ring, nsplit, nbias, bias_lds;
@@ -162,6 +163,29 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
   int my_first[MR];
 #pragma unroll
   for (int q = 0; q < MR; ++q) my_first[q] = a.span.first(my_pos[q]);
+  // ---- queries as they lie, requested ahead of all that depends on the position
+  float qx[MR][NQ][E];
+#pragma unroll
+  for (int q = 0; q < MR; ++q) {
+    const size_t at = (size_t)(row0 + tok[q]) * a.ldr + (size_t)head[q] * a.dkr;
+#pragma unroll
+    for (int b = 0; b < NQ; ++b) {
+      const int e0 = 4 * E * b + E * fh;  // dkr is a multiple of 16: a fragment is inside or outside as a whole
+      if (a.raw_f32) {
+#pragma unroll
+        for (int i = 0; i < E; i += 4) {
+          const f32x4 v = e0 < a.dkr ? *(const f32x4*)((const float*)a.raw + at + e0 + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) qx[q][b][i + j] = v[j];
+        }
+      } else {
+        const bool in = e0 < a.dkr;
+        const frag v = *(const frag*)((const T*)a.raw + at + (in ? e0 : 0));
+#pragma unroll
+        for (int i = 0; i < E; ++i) qx[q][b][i] = in ? (float)v[i] : 0.f;
+      }
+    }
+  }
   // ---- staging: request j of a wave covers chunks (4 j + wave) 64 .. of the tile; slot s of row r holds chunk s ^ (r & 7)
   int kr[NL];
   unsigned kc[NL];
@@ -193,27 +217,11 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
   frag fq[MR][NQ];
 #pragma unroll
   for (int q = 0; q < MR; ++q) {
-    float x[NQ][E], s = 0.f;
-    const size_t at = (size_t)(row0 + tok[q]) * a.ldr + (size_t)head[q] * a.dkr;
+    float s = 0.f;
 #pragma unroll
-    for (int b = 0; b < NQ; ++b) {
-      const int e0 = 4 * E * b + E * fh;  // dkr is a multiple of 16: a fragment is inside or outside as a whole
-      if (a.raw_f32) {
+    for (int b = 0; b < NQ; ++b)
 #pragma unroll
-        for (int i = 0; i < E; i += 4) {
-          const f32x4 v = e0 < a.dkr ? *(const f32x4*)((const float*)a.raw + at + e0 + i) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) x[b][i + j] = v[j];
-        }
-      } else {
-        const bool in = e0 < a.dkr;
-        const frag v = *(const frag*)((const T*)a.raw + at + (in ? e0 : 0));
-#pragma unroll
-        for (int i = 0; i < E; ++i) x[b][i] = in ? (float)v[i] : 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < E; ++i) s = __builtin_fmaf(x[b][i], x[b][i], s);
-    }
+      for (int i = 0; i < E; ++i) s = __builtin_fmaf(qx[q][b][i], qx[q][b][i], s);
     s = xor16_sum(s);
     s = xor32_sum(s);
     const float f = a.qn ? a.scale2 / sqrtf(s / (float)a.dk + a.eps) : a.scale2;
@@ -223,7 +231,7 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
       for (int i = 0; i < E; i += 4) {
         const f32x4 w = a.qn ? *(const f32x4*)(a.qn + 4 * E * b + E * fh + i) : f32x4{1.f, 1.f, 1.f, 1.f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) fq[q][b][i + j] = (T)(x[b][i + j] * f * w[j]);
+        for (int j = 0; j < 4; ++j) fq[q][b][i + j] = (T)(qx[q][b][i + j] * f * w[j]);
       }
   }
   // ---- distance bias: the group's rows of the table to LDS when a key of this workgroup is near enough to need them
@@ -233,6 +241,19 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
   for (int q = 0; q < MR; ++q) far[q] = a.bias ? a.bias[(size_t)head[q] * a.nbias + a.nbias - 1] : 0.f;
   if (a.bias && a.bias_lds && pos_of(tl.r0) - (k_hi - 1) < a.nbias - 1)
     for (int i = threadIdx.x; i < per * a.nbias; i += 256 * KS) tab[i] = a.bias[(size_t)g * per * a.nbias + i];
+  // a decoded token's gate logits, ahead of their use
+  constexpr bool EARLY = CP == 4 && KS > 1;
+  f32x4 zg[EARLY ? NT : 1];
+  if constexpr (EARLY) {
+    if (a.g_off >= 0 && a.raw_f32 && ks == 0) {
+      const float* z = (const float*)a.raw + (size_t)(row0 + tok[0]) * a.ldr + a.g_off + (size_t)head[0] * a.dvr;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const int c = (wc * NT + n) * 16 + 4 * fh;
+        zg[n] = *(const f32x4*)(z + (c < a.dvr ? c : 0));
+      }
+    }
+  }
   float m[MR], l[MR];
   f32x4 o[MR][NT];
 #pragma unroll
@@ -395,11 +416,15 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
         for (int i = 0; i < 4; ++i) v[i] = o[q][n][i] * inv;
         if (a.g_off >= 0) {
           const size_t at = t * a.ldr + a.g_off + (size_t)head[q] * a.dvr + c;
-          const f32x4 z = a.raw_f32 ? *(const f32x4*)((const float*)a.raw + at) : quad_f((const T*)a.raw + at);
+          f32x4 z;
+          if (EARLY && a.raw_f32) z = zg[EARLY ? n : 0];
+          else z = a.raw_f32 ? *(const f32x4*)((const float*)a.raw + at) : quad_f((const T*)a.raw + at);
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[i] *= sigmoid1(z[i]);
         }
-        *(typename TL::quad*)((T*)a.out + t * a.ldo + (size_t)head[q] * a.dvr + c) = to_quad<T>(v);
+        const size_t to = t * a.ldo + (size_t)head[q] * a.dvr + c;
+        if (a.out_f32) *(f32x4*)((float*)a.out + to) = v;
+        else *(typename TL::quad*)((T*)a.out + to) = to_quad<T>(v);
       }
     } else {
       float* pt = a.part + (((size_t)(row0 + tok[q]) * a.H + head[q]) * a.nsplit + blockIdx.z) * (size_t)(DV + 4);
@@ -415,6 +440,10 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
 
 #define KH_HEADS_MAX_DIM 256
 #define KH_HEADS_BIAS_LDS (32 * 1024)
+// One token per sequence over at most `keys` keys: is a group one workgroup, without splits and the launch that merges them?
+// Where its keys and values are 64 KB, two microseconds of what one CU can pull; the merge costs three (8 heads of 128 on 2
+// groups in fp32, 24 ... 64 keys: 6.7 + 4.7 -> 9.0 us a layer; Gusorax 1024 x 8, 24 + 40 tokens 12 255 -> 11 950).
+__host__ __device__ inline bool heads_one_split(int keys, int dkp, int dvp, size_t elem) { return (size_t)keys * (dkp + dvp) * elem <= 64 * 1024; }
 // rows of a workgroup's tile: 16, 64 or, for bf16 heads of up to 128, 128 (two row tiles per wave share every operand)
 static inline bool heads_wide_rows(int dkp, int dvp, size_t elem) { return elem == 2 && dkp <= 128 && dvp <= 128; }
 template <class T>

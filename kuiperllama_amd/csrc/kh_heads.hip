@@ -33,6 +33,8 @@ int heads_attn_launch(hipStream_t s, HeadsArgs a, int ntiles, int rows) {
   auto by_rows = [&](auto kn, auto kv) -> int {
     constexpr int KN = decltype(kn)::value, KV = decltype(kv)::value;
     const size_t stage = (size_t)4 * Tile<T>::N * (a.dkp + a.dvp) * sizeof(T);
+    if constexpr (KN + KV <= 4)  // one token per sequence and one split: four sets of waves, a key tile each
+      if (rows == 16 && !a.tiles && a.nsplit == 1) return go(k_heads_attn<T, KN, KV, 4, 1, 4>, stage, 4);
     if (rows == 16) return go(k_heads_attn<T, KN, KV, 4, 1, 1>, stage, 1);
     // at most one workgroup per CU: two sets of waves, which share the keys (1100 tokens of 2 x 4 heads of 128, 138 workgroups:
     // 37.2 -> 27.6 us; four sets on tiles of 32 rows 25.9, at twice the key traffic).  Keys and values of more than 256

@@ -6,6 +6,9 @@
 //   kh_hybrid_pass.hip   a pass of T tokens of several sequences on the matrix cores (prompts, mixed lengths)
 //   kh_hybrid_step.hip   the fused decode step, batches, C-ABI
 #pragma once
+#include <limits.h>
+
+#include <algorithm>
 #include <memory>
 #include <string>
 #include <vector>
@@ -195,6 +198,19 @@ inline HeadsArgs heads_args(const Hybrid& hy, const HyHeads& a, const void* cach
   return h;
 }
 
+// decode steps up to position pos_hi: no attention over heads is split (step variant 0; 1 else)
+inline bool hy_one_split(const Hybrid& hy, const HyHeads& a, int pos_hi) {
+  int keys = pos_hi + 1;
+  if (a.span.window > 0) keys = std::min(keys, a.span.window);
+  if (a.span.chunk > 0) keys = std::min(keys, a.span.chunk);
+  return heads_one_split(keys, a.dkp, a.dvp, hy.elem());
+}
+inline int hy_step_variant(const Hybrid& hy, int pos_hi) {
+  for (auto& l : hy.layers)
+    if (l.mixer == HY_HEADS && !hy_one_split(hy, l.ha, pos_hi)) return 1;
+  return 0;
+}
+
 // ---- kh_hybrid_load.hip
 int hy_create(const char* config, size_t config_len, const void* tensors, size_t nbytes, const kh_model_opts* o, kh_model** out);
 void hy_destroy(kh_model* m);
@@ -220,5 +236,5 @@ struct HyTail {  // device lists of the wanted tokens of a pass: their rows, ids
 };
 bool hy_tail_pays(const kh_model* m, int T, int want);
 int hy_tail(kh_model* m, const HyTail& t, int n, float* h_logits);
-int hy_launches(const kh_model* m);  // kernel launches of one decode step
+int hy_launches(const kh_model* m);  // kernel launches of one decode step (variant 1; variant 0 does without the merges)
 }  // namespace khm

@@ -277,14 +277,21 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       a.raw = st.in;
       a.raw_f32 = 1;
       a.ldr = in_ld;
-      a.part = st.part;
-      a.nsplit = ha.nsplit;
       a.p.seg_slot = tb.slot;
       a.p.seg_pos0 = tb.pos;
+      const bool one = m->step_var == 0 || hy_one_split(hy, ha, INT_MAX - 1);
+      if (one) {
+        a.out = st.v;
+        a.out_f32 = 1;
+        a.ldo = ha.o.ld;
+      } else {
+        a.part = st.part;
+        a.nsplit = ha.nsplit;
+      }
       TRY(heads_attn_launch<T>(s, a, B * cdiv(ha.H / ha.G, 16), 16));
       LdMergeArgs mg{st.part, ha.gate ? st.in + ha.g_off() : nullptr, st.v, ha.H, ha.nsplit, ha.dvp, ha.dvr, in_ld, ha.o.ld,
                      ha.span, tb.pos};
-      TRY(go(k_ld_merge, dim3(ha.H, B), 256, 256 * 16, s, mg));
+      if (!one) TRY(go(k_ld_merge, dim3(ha.H, B), 256, 256 * 16, s, mg));
     } else {
       const HyLatent& la = l.la;
       LdAbsorbArgs ab{st.mid, la.ukT.w, la.rope, st.Q, la.H, std::max(1, std::min(cdiv(la.Rp, 32), cdiv(512, la.H * B))),
@@ -499,6 +506,7 @@ int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits) {
     st.h_tabs[TB_SLOT + i] = e[i].slot;
   }
   KH_CHECK_HIP(hipMemcpyAsync(st.tabs, st.h_tabs, TB_ZERO * 4, hipMemcpyHostToDevice, m->stream));
+  m->step_var = hy_step_variant(hy, *std::max_element(st.h_tabs + TB_POS, st.h_tabs + TB_POS + n));
   for (int i = 0; i < n;) {  // n = 3: 2 + 1
     const int B = n - i >= 4 ? 4 : (n - i >= 2 ? 2 : 1);
     const LdTabs tb{st.tabs + TB_TOK + i, st.tabs + TB_POS + i, st.tabs + TB_SLOT + i};

@@ -8,6 +8,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "kh_fused.h"
@@ -399,7 +400,7 @@ void launch_sample(kh_model* m, int advance, int n_forced) {
 // OVERLAP) defer only up to 4 splits (profiles/r4_attn_defer_ab.txt: Llama-2-7B int8 loses from 8 on).
 int step_variant(const kh_model* m, int pos_lo, int pos_hi) {
   (void)pos_lo;
-  if (m->hy) return 0;
+  if (m->hy) return hy_step_variant(*m->hy, pos_hi);
   if (pos_hi < KH_ATTN_MIN_TS) return 0;         // pos + 1 <= 256 everywhere: one split
   if (pos_hi + 1 >= m->attn_t_long) return 0;    // some step runs the group path
   if (m->attn_defer && attn_active_splits(pos_hi, m->attn_ns, m->attn_ts_shift) <= m->attn_defer_max) return 1;
@@ -424,8 +425,8 @@ static void launch_layer(kh_model* m, int l, F&& mark) {
 }
 // one fused decode step = 5L + 2 launches.  ev (optional) receives an event after each launch.
 void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant) {
-  if (m->hy) return hy_launch_step(m, advance, n_forced);
   m->step_var = variant;
+  if (m->hy) return hy_launch_step(m, advance, n_forced);
   int e = 0;
   auto mark = [&]() {
     if (ev) (void)hipEventRecord(ev[e++], m->stream);
@@ -805,18 +806,20 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
     // a generate owns rows [0, max(total_steps, 8)) of the cache).  Skipped when the cache is shorter than that.
     // (Launching only the graphs of at most total_steps steps - the first r5 form - left the 8-step graph's first
     // launch inside the timed loop of a 20-step run behind a 5-step warm-up: 1018 instead of 1036-1042 tok/s.)
+    // A layer-list model's variant 1 runs at any position: the variant that this call's first steps take.
+    const int v0 = m->hy ? step_variant(m, n_prompt - 1, std::min(total_steps, n_prompt - 1 + KH_GRAPH_STEPS) - 1) : 0;
     bool fresh[4] = {false, false, false, false};
     hipGraphExec_t ge = nullptr;
     for (int n = 1, k = 0; n <= KH_GRAPH_STEPS; n *= 2, ++k) {
-      fresh[k] = m->sg[0][k].e == nullptr;
-      if ((rc = step_graph_n(m, n_forced, 0, n, &ge)) != KH_OK) return rc;
+      fresh[k] = m->sg[v0][k].e == nullptr;
+      if ((rc = step_graph_n(m, n_forced, v0, n, &ge)) != KH_OK) return rc;
     }
     bool dry = false;
     if (c.cache_len >= KH_GRAPH_STEPS && m->seq_cap >= KH_GRAPH_STEPS)
       for (int k = 3; k >= 0; --k)
         if (fresh[k]) {
           set_state(m, h_prompt[0], 0);
-          KH_CHECK_HIP(hipGraphLaunch(m->sg[0][k].e, m->stream));
+          KH_CHECK_HIP(hipGraphLaunch(m->sg[v0][k].e, m->stream));
           dry = true;
         }
     if (dry) KH_CHECK_HIP(hipStreamSynchronize(m->stream));

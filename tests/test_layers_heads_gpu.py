@@ -176,6 +176,31 @@ def test_waves_that_share_keys(gpu, dtype, n, heads, kv_heads):
     m.close()
 
 
+@BOTH
+@pytest.mark.parametrize("kw", [dict(dim=20, vdim=28), dict(dim=100, vdim=70), dict(dim=200, vdim=40, heads=18, kv_heads=1)])
+def test_steps_with_one_split_and_more(gpu, dtype, kw):
+    """Decode steps around the last position whose keys and values stay in one workgroup: 128, 64 and 51 positions in fp32, twice
+    that in bf16; steps of one and of four sequences, and the graphs of generate()."""
+    mod = U.Model(U.gusorax([U.windowed(window=70, rows=16, far=50.0, **kw), U.chunked(chunk=400, **kw)]))
+    last = 64 * 1024 // ((-(-kw["dim"] // 64) + -(-kw["vdim"] // 64)) * 64 * (4 if dtype == "float32" else 2))
+    toks = mod.tokens(last + 9)
+    want = mod.logits(toks)
+    m = mod.load(dtype, max_seqs=4)
+    U.check(U.run_alone(m, toks, tuple(range(last - 6, last + 8))), want, dtype, "steps")
+    seqs = [m.open_seq() for _ in range(4)]
+    at = [last - 3, 1, last // 2, last + 2]
+    m.forward([(s, toks[:n], []) for s, n in zip(seqs, at)])
+    for k in range(5):
+        U.check(m.forward([(s, [toks[n + k]], [0]) for s, n in zip(seqs, at)]), want[[n + k for n in at]], dtype, "batch")
+    m.close()
+    for n, steps in ((3, 30), (last - 5, last + 6), (last + 3, last + 9)):
+        m = mod.load(dtype)
+        words, _ = m.generate(toks[:n], steps)
+        seq = toks[:n] + [int(t) for t in words[n - 1: steps - 1]]
+        U.check(m.logits()[None], mod.logits(seq)[-1:], dtype, "generate")
+        m.close()
+
+
 def test_prompt_of_several_passes(gpu):
     """More tokens than one pass holds."""
     mod = U.Model(U.gusorax([U.windowed(8, 2, 16, 16, 0.4, 300, 16, 100.0), dict(U.chunked(16, 8, 8, 8, 0.5, 256), mlp=U.clamped(3, 2, 8))],
