@@ -412,7 +412,9 @@ struct LdMidArgs {
   const float *corr, *xn2;
   const void* gu;        // experts [2 ffp][ldw]
   float* he;             // [B][top][ffp], weighted
-  int32_t* ids;          // [B][top] (-1: identity), written for k_ld_out
+  // [B][top], written for k_ld_out.  ids: -1 for an identity expert, and for one that an earlier sequence chose as well: the
+  // first of them multiplies its weights for all.  mates: byte q is 1 + the place where later sequence q chose the same expert
+  int32_t *ids, *mates;
   float *id_w, *sh_g;    // [B]
   int nwg_e, top, n_out, n_expert, shared, ffp, ldz, W, ldw, over_chosen;
   GateAct act;
@@ -440,12 +442,14 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float* xs = (float*)smem_raw;
   __shared__ float red[KH_WAVES_MAX];
+  __shared__ int32_t rid[B][KH_MOE_MAX_TOP];
+  __shared__ float rwt[B][KH_MOE_MAX_TOP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int wg = blockIdx.x;
   LdTile<T, R, U> t;
   const T* row[R];
   const int ne = B * a.top * a.nwg_e;
-  if (wg < ne) {  // ---- one chosen expert of one sequence
+  if (wg < ne) {  // ---- one chosen expert of one sequence, and of those behind it that chose it too
     const int pair = wg / a.nwg_e, part = wg - pair * a.nwg_e, q = pair / a.top, k = pair - q * a.top;
     const int nblk = Ld<T>::blocks(a.ldw), nch = a.ldw / Ld<T>::E;
     const int n4 = a.ldw >> 2, total4 = nblk * Ld<T>::BE / 4;
@@ -455,9 +459,50 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
       const int i = threadIdx.x + 256 * j;
       x[j] = i < n4 ? ((const f32x4*)(a.xn2 + (size_t)q * a.ldw))[i] : f4_zero();
     }
-    // every wave makes the choice for itself: its weight loads leave without a barrier
+    // one sequence: every wave makes the choice for itself: its weight loads leave without a barrier.  Several: the waves make
+    // one sequence's each, and an expert that several chose is read once.  Bound by the bytes of the experts (2048 x 1024 in bf16,
+    // four sequences, 6 of 32 and 4 identities each: 21 choices of 17 experts): 39.4 -> 35.5 us in front of latent attention,
+    // 31.6 -> 28.3 of mamba, k_ld_out 26.3 -> 24.6
     float idw = 0.f, w = 0.f;
     int id = -1;
+    unsigned mates = 0;
+    if constexpr (B > 1) {
+      const int qw = wave % B;
+      int my_id = 0;
+      float my_w = 0.f;
+      const float wf = moe_route<RP>(a.z + (size_t)qw * a.ldz, a.corr, a.n_out, a.top, a.over_chosen, lane,
+                                     [&](int kk, int i, float wt) __attribute__((always_inline)) {
+        if (i >= a.n_expert) idw += wt;
+        my_id = lane == kk ? (i >= a.n_expert ? -1 : i) : my_id;
+        my_w = lane == kk ? wt : my_w;
+      });
+      if (lane < a.top) {
+        rid[qw][lane] = my_id;
+        rwt[qw][lane] = my_w * wf;
+      }
+      if (part == 0 && k == 0 && wave == q && lane == 0) {
+        a.id_w[q] = idw * wf;
+        if (a.shared) a.sh_g[q] = sigmoid1(a.z[(size_t)q * a.ldz + a.n_out]);
+      }
+      __syncthreads();
+      id = rid[q][k];
+      bool first = id >= 0;
+#pragma unroll
+      for (int o = 0; o < B; ++o) {
+        const unsigned long long hit = __builtin_amdgcn_ballot_w64(lane < a.top && rid[o][lane < a.top ? lane : 0] == id);
+        if (o == q || !hit) continue;
+        if (o < q) first = false;
+        else mates |= (unsigned)(__builtin_ctzll(hit) + 1) << (8 * o);
+      }
+      if (part == 0 && threadIdx.x == 0) {
+        a.ids[q * a.top + k] = first ? id : -1;
+        a.mates[q * a.top + k] = (int)mates;
+      }
+      if (!first) return;  // the whole workgroup agrees
+      id = __builtin_amdgcn_readfirstlane(id);
+      mates = (unsigned)__builtin_amdgcn_readfirstlane((int)mates);
+      w = rwt[q][k];
+    } else {
     const float wf = moe_route<RP>(a.z + (size_t)q * a.ldz, a.corr, a.n_out, a.top, a.over_chosen, lane,
                                    [&](int kk, int i, float wt) __attribute__((always_inline)) {
       const bool ident = i >= a.n_expert;
@@ -477,6 +522,7 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
       }
     }
     if (id < 0) return;  // identity expert: no tensors (the whole workgroup agrees)
+    }
     const T* base = (const T*)a.gu + (size_t)id * 2 * a.ffp * a.ldw;
     const int items = a.ffp / 2;
     int it = part * 4 + wave;
@@ -494,22 +540,61 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
 #pragma unroll
     for (int j = 0; j < NV; ++j)
       if ((int)threadIdx.x + 256 * j < total4) ((f32x4*)xs)[ld_slot<T>(threadIdx.x + 256 * j)] = x[j];
-    __syncthreads();
-    while (it < items) {
-      float acc[R][1] = {};
-      ld_rows<T, R, U, 1>(t, row, nblk, nch, xs, 0, lane, acc);
-      const int cur = it;
-      it += a.nwg_e * 4;
-      if (it < items) {
-        set_rows(it);
-        ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
+    // vector j > 0: the j-th of the mates, in rising order of their sequences
+    int n = 1, dst[B];
+    float wj[B];
+    dst[0] = pair;
+    wj[0] = w;
+    if constexpr (B > 1) {
+#pragma unroll
+      for (int j = 1; j < B; ++j) {
+        dst[j] = pair;
+        wj[j] = 0.f;
       }
-      ld_reduce<R, 1>(acc);
-      if (lane < 2) {
-        const float g = ld_pick<R, 1>(acc, lane, 0), u = ld_pick<R, 1>(acc, lane + 2, 0);
-        a.he[(size_t)pair * a.ffp + cur * 2 + lane] = w * gated1(a.act, g, u);
+#pragma unroll
+      for (int o = 1; o < B; ++o) {
+        const int ko = (int)(mates >> (8 * o) & 255) - 1;
+        if (ko < 0) continue;  // uniform
+        f32x4* xo = (f32x4*)xs + (size_t)n * total4;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          const int i = threadIdx.x + 256 * j;
+          if (i < total4) xo[ld_slot<T>(i)] = i < n4 ? ((const f32x4*)(a.xn2 + (size_t)o * a.ldw))[i] : f4_zero();
+        }
+#pragma unroll
+        for (int j = 1; j < B; ++j)
+          if (j == n) {
+            dst[j] = o * a.top + ko;
+            wj[j] = rwt[o][ko];
+          }
+        ++n;
       }
     }
+    __syncthreads();
+    auto rows_of = [&](auto cnt) __attribute__((always_inline)) {
+      constexpr int N = decltype(cnt)::value;
+      while (it < items) {
+        float acc[R][N] = {};
+        ld_rows<T, R, U, N>(t, row, nblk, nch, xs, total4 * 4, lane, acc);
+        const int cur = it;
+        it += a.nwg_e * 4;
+        if (it < items) {
+          set_rows(it);
+          ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
+        }
+        ld_reduce<R, N>(acc);
+        if (lane < 2) {
+#pragma unroll
+          for (int j = 0; j < N; ++j) {
+            const float g = ld_pick<R, N>(acc, lane, j), u = ld_pick<R, N>(acc, lane + 2, j);
+            if (j < n) a.he[(size_t)dst[j] * a.ffp + cur * 2 + lane] = wj[j] * gated1(a.act, g, u);
+          }
+        }
+      }
+    };
+    if (n == 1) rows_of(std::integral_constant<int, 1>());
+    else if (B == 2 || n == 2) rows_of(std::integral_constant<int, B < 2 ? 1 : 2>());
+    else rows_of(std::integral_constant<int, B>());  // three of four: what the fourth place holds is finite or not, and not stored
     return;
   }
   wg -= ne;
@@ -867,7 +952,7 @@ struct LdOutArgs {
   const float* v;         // [B][ld_v] mixer vector
   const void *down, *sdown;  // experts [W][ffp] each; shared [W][sffp]
   const float *he, *hs;   // [B][top][ffp] (weighted), [B][sffp]
-  const int32_t* ids;     // [B][top]
+  const int32_t *ids, *mates;  // [B][top], see LdMidArgs
   const float *id_w, *sh_g, *xn2, *x_cur;  // id_w, sh_g: nullptr = none, 1
   const float* bias;      // of W_o, or nullptr
   float* x_out;           // [B][ld]
@@ -980,6 +1065,25 @@ __global__ __launch_bounds__(512, 4) void k_ld_out(const LdOutArgs a) {
           for (int p = 0; p < P; ++p) x[u][p] = in[u] ? x[u][p] : f4_zero();
 #pragma unroll
           for (int r = 0; r < R; ++r) acc[r][q] = dot(w[r][u], x[u], acc[r][q]);
+          if constexpr (B > 1) {
+            const unsigned mates = (unsigned)a.mates[q * a.top + k];
+            if (!mates) continue;  // uniform
+            bool other;
+            const int c = chunk(a.ffp, e + u - k * nbe, other);
+#pragma unroll
+            for (int o = q + 1; o < B; ++o) {
+              const int ko = (int)(mates >> (8 * o) & 255) - 1;
+              if (ko < 0) continue;
+              const float* v = a.he + (size_t)(o * a.top + ko) * a.ffp + (size_t)c * E;
+              f32x4 xo[P];
+#pragma unroll
+              for (int p = 0; p < P; ++p) xo[p] = *(const f32x4*)(v + 4 * p);
+#pragma unroll
+              for (int p = 0; p < P; ++p) xo[p] = in[u] ? xo[p] : f4_zero();
+#pragma unroll
+              for (int r = 0; r < R; ++r) acc[r][o] = dot(w[r][u], xo, acc[r][o]);
+            }
+          }
         }
       }
   }

@@ -90,6 +90,25 @@ def test_expert_tiles(gpu, dtype, n, kw):
 
 
 @BOTH
+@pytest.mark.parametrize("n,same", [(2, 2), (2, 1), (3, 3), (4, 4), (4, 2), (4, 3), (4, 1)])
+def test_batches_that_share_experts(gpu, dtype, n, same):
+    """Steps of sequences of which the first `same` are alike, so that they choose the same experts, the others a few of them."""
+    layers = [U.with_ff(U.mamba(), experts=6, identity=2, top=4), U.with_ff(U.latent(), experts=3, identity=0, top=2, shared=0),
+              U.with_ff(U.mamba(), experts=80, identity=4, top=7, ff=66)]
+    mod = U.Model(U.config(layers))
+    alike = mod.tokens(30, seed=1)
+    toks = [alike if i < same else mod.tokens(30, seed=10 + i) for i in range(n)]
+    want = [mod.logits(t) for t in toks]
+    m = mod.load(dtype)
+    seqs = [m.open_seq() for _ in toks]
+    m.forward([(s, t[:20], []) for s, t in zip(seqs, toks)])
+    for k in range(20, 30):
+        got = m.forward([(s, [t[k]], [0]) for s, t in zip(seqs, toks)])
+        U.check(got, np.stack([w[k] for w in want]), dtype, f"step {k}")
+    m.close()
+
+
+@BOTH
 @pytest.mark.parametrize("loop", [None, (0, 1, 1), (0, 2, 3), (1, 3, 2), (2, 3, 2)])
 def test_loop_ranges(gpu, dtype, loop):
     layers = [U.with_ff(U.latent()), U.mamba(), U.with_ff(U.latent(2), identity=0)]
