@@ -1160,8 +1160,9 @@ __global__ __launch_bounds__(256) void k_ld_head(const LdHeadArgs a) {
       get(q0, v[0], shift[0]);  // Q = 1
       __syncthreads();          // red is free again
     }
-    ld_norm<T, NV, Q>(v, nw, nb, shift, a.rms, a.W, n4, xstride >> 2, a.eps, red, (f32x4*)(xs + (size_t)q0 * xstride), xstride >> 2,
-                      nullptr, 0);
+    int W = a.W, m4 = n4, total4 = xstride >> 2;
+    if (Q < B) asm volatile("" : "+s"(W), "+s"(m4), "+s"(total4));  // or the lane masks of all pieces are kept over the rows: scratch
+    ld_norm<T, NV, Q>(v, nw, nb, shift, a.rms, W, m4, total4, a.eps, red, (f32x4*)(xs + (size_t)q0 * xstride), xstride >> 2, nullptr, 0);
   }
   __syncthreads();
   float bv = -INFINITY;
