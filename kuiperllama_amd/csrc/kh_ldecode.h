@@ -270,8 +270,8 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
       row[r] = w + (size_t)i * a.ld;
     }
   };
-  LdTile<T, R, U> t;
-  if (item < items) {
+  LdTile<T, R, U> t;  // (rows of more than 4096 columns first: the other way takes 322 registers)
+  if (NV < 8 && item < items) {
     set_rows(item);
     ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
   }
@@ -304,6 +304,10 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
       nw[j] = i < n4 ? wp[i] : f4_zero();
       nb[j] = bp && i < n4 ? bp[i] : f4_zero();
     }
+  }
+  if (NV == 8 && item < items) {
+    set_rows(item);
+    ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
   }
   // convolution operands of the wave's first item: requested with its weights (up to four taps)
   constexpr int CT = 4;
