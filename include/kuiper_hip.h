@@ -385,6 +385,10 @@ int kh_plan_decode_ring(int32_t dim, int32_t hidden_dim, int32_t vocab_size, int
  * workgroups that own timesteps at `pos`} (KH_ATTN_TLONG honoured). */
 int kh_plan_attention(int32_t head_num, int32_t kv_mul, int32_t head_size, int32_t seq_len, int32_t pos,
                       int32_t* out8);
+/* kh_plan_heads_lds: LDS bytes of a workgroup of the layer-list models' attention over grouped heads with `sets` sets of
+ * four waves (1; prompts 2, one decoded token 4, both for key + value sizes of at most 256, else KH_ERR_UNSUPPORTED) and a
+ * distance table of `table` bytes a group. */
+int kh_plan_heads_lds(int32_t key, int32_t value, int32_t sets, int32_t table, int32_t* bytes);
 int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32_t is_quant,
                           int32_t r2_ok, int32_t* out7);
 

@@ -95,13 +95,23 @@ struct HeadsArgs {
   PassTabs p;
 };
 
-// stages of a key tile of tb bytes, ks sets of them
-constexpr int heads_stages(int tb, int ks) { return tb <= 24 * 1024 && 3 * ks * tb <= 144 * 1024 ? 3 : 2; }
+#define KH_HEADS_MAX_DIM 256
+#define KH_HEADS_BIAS_LDS (32 * 1024)  // the largest distance table that is copied to LDS, behind the stages
+constexpr int kHeadsLds = 160 * 1024;  // of a workgroup: the stages of all sets of waves and the table
+// a tile holds 64 bytes of keys a column: 32 in bf16, 16 in fp32
+constexpr int heads_tile_bytes(int dkp, int dvp) { return 64 * (dkp + dvp); }
+// stages of a key tile of tb bytes, ks sets of them: three of small tiles, where the largest table still fits beside them
+constexpr int heads_stages(int tb, int ks) { return tb <= 24 * 1024 && 3 * ks * tb + KH_HEADS_BIAS_LDS <= kHeadsLds ? 3 : 2; }
+constexpr bool heads_table_lds(size_t table) { return table <= KH_HEADS_BIAS_LDS; }
+constexpr size_t heads_lds(int tb, int ks, size_t table) {
+  return (size_t)ks * heads_stages(tb, ks) * tb + (heads_table_lds(table) ? table : 0);
+}
 
-// KN, KV: key and value size in units of 64.  CP = 4: 16 rows per workgroup; CP = 1: 64 MR rows.  KS = 2: eight waves, the
-// second four take every other key tile of the same rows and are merged at the end through LDS.  A tile of 32 keys is a serial
-// chain (keys from LDS, scores, maximum, exponentials, values: 1.1 us for 0.1 us of products), so a wave needs another one on
-// its SIMD; where the rows of a launch make one workgroup per CU, KS = 2 is where it comes from.
+// KN, KV: key and value size in units of 64.  CP = 4: 16 rows per workgroup; CP = 1: 64 MR rows.  KS: sets of four waves; set k
+// takes key tiles k, k + KS, ... of the same rows, and the sets are merged at the end through LDS.  A tile of 32 keys is a
+// serial chain (keys from LDS, scores, maximum, exponentials, values: 1.1 us for 0.1 us of products), so a wave needs another
+// one on its SIMD; where the rows of a launch make one workgroup per CU, KS = 2 is where it comes from.  KS = 4 is a decoded
+// token whose keys nobody else shares (heads_one_split): the tiles of a workgroup side by side.
 // Two waves per SIMD where the accumulators allow it: within 256 registers the compiler keeps them where the rescaling can
 // reach them (beyond, it moves them between two register files in every tile).
 template <class T, int KN, int KV, int CP, int MR, int KS>
@@ -111,9 +121,11 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
   constexpr int E = TL::N, KT = 4 * E, NS = KT / 16, ES = (int)sizeof(T);
   constexpr int DK = 64 * KN, DV = 64 * KV, ROW = DK + DV, CB = ROW / E;
   constexpr int NQ = DK / (4 * E), NT = DV / 16 / CP, NL = ROW / 64;
-  constexpr int TB = KT * ROW * ES, NST = heads_stages(TB, KS), WR = 4 / CP, ROWS = 16 * MR * WR;
+  constexpr int TB = heads_tile_bytes(DK, DV), NST = heads_stages(TB, KS), WR = 4 / CP, ROWS = 16 * MR * WR;
   constexpr int BOX = 4 * MR * NT * 1024 + 2048 * MR;  // what a set of four waves hands over
   static_assert((KS - 1) * BOX <= KS * NST * TB, "fits the stages");
+  static_assert(TB == KT * ROW * ES, "a tile");
+  static_assert(heads_lds(TB, KS, KH_HEADS_BIAS_LDS) <= kHeadsLds, "fits a CU with the largest table");
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   const int lane = threadIdx.x & 63, wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave8 & 3, ks = KS == 1 ? 0 : wave8 >> 2;
@@ -438,8 +450,6 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
   }
 }
 
-#define KH_HEADS_MAX_DIM 256
-#define KH_HEADS_BIAS_LDS (32 * 1024)
 // One token per sequence over at most `keys` keys: is a group one workgroup, without splits and the launch that merges them?
 // Where its keys and values are 64 KB, two microseconds of what one CU can pull; the merge costs three (8 heads of 128 on 2
 // groups in fp32, 24 ... 64 keys: 6.7 + 4.7 -> 9.0 us a layer; Gusorax 1024 x 8, 24 + 40 tokens 12 255 -> 11 950).

@@ -11,9 +11,9 @@ int heads_attn_launch(hipStream_t s, HeadsArgs a, int ntiles, int rows) {
       a.dkr % 16 || a.dvr % 16 || a.ldr % 16 || a.G <= 0 || a.H % a.G || a.ring <= 0 || a.nsplit < 1 || ntiles <= 0)
     return KH_ERR_INTERNAL;
   const size_t table = (size_t)(a.H / a.G) * a.nbias * sizeof(float);
-  a.bias_lds = a.bias && table <= KH_HEADS_BIAS_LDS;
+  a.bias_lds = a.bias && heads_table_lds(table);
   auto go = [&](auto kern, size_t stage, int ks) -> int {
-    const size_t lds = stage * heads_stages((int)stage, ks) * ks + (a.bias_lds ? table : 0);
+    const size_t lds = heads_lds((int)stage, ks, a.bias ? table : 0);
     if (lds > 64 * 1024) {
       struct Done { int dev; const void* fn; size_t lds; };
       static thread_local std::vector<Done> done;
@@ -32,7 +32,7 @@ int heads_attn_launch(hipStream_t s, HeadsArgs a, int ntiles, int rows) {
   };
   auto by_rows = [&](auto kn, auto kv) -> int {
     constexpr int KN = decltype(kn)::value, KV = decltype(kv)::value;
-    const size_t stage = (size_t)4 * Tile<T>::N * (a.dkp + a.dvp) * sizeof(T);
+    const size_t stage = heads_tile_bytes(a.dkp, a.dvp);
     if constexpr (KN + KV <= 4)  // one token per sequence and one split: four sets of waves, a key tile each
       if (rows == 16 && !a.tiles && a.nsplit == 1) return go(k_heads_attn<T, KN, KV, 4, 1, 4>, stage, 4);
     if (rows == 16) return go(k_heads_attn<T, KN, KV, 4, 1, 1>, stage, 1);
@@ -65,3 +65,12 @@ template int heads_attn_launch<bf16>(hipStream_t, HeadsArgs, int, int);
 template int heads_attn_launch<float>(hipStream_t, HeadsArgs, int, int);
 
 }  // namespace khm
+
+extern "C" int kh_plan_heads_lds(int32_t key, int32_t value, int32_t sets, int32_t table, int32_t* bytes) {
+  using namespace khm;
+  if (!bytes || key <= 0 || value <= 0 || table < 0 || (sets != 1 && sets != 2 && sets != 4)) return KH_ERR_INVALID_ARG;
+  const int kp = (key + 63) / 64 * 64, vp = (value + 63) / 64 * 64;
+  if (kp > KH_HEADS_MAX_DIM || vp > KH_HEADS_MAX_DIM || (sets > 1 && kp + vp > KH_HEADS_MAX_DIM)) return KH_ERR_UNSUPPORTED;
+  *bytes = (int32_t)heads_lds(heads_tile_bytes(kp, vp), sets, (size_t)table);
+  return KH_OK;
+}

@@ -211,3 +211,19 @@ def test_attention_plan_and_split_geometry(monkeypatch):
     assert _ffi.plan_attention(32, 4, 64, 131072, 255)["active_splits"] == 1
     monkeypatch.delenv("KH_ATTN_TS")
 
+
+@pytest.mark.parametrize("sets", [1, 2, 4])
+def test_attention_over_heads_fits_a_cu(sets):
+    """Stages of every key and value size beside every distance table within the 160 KB of a CU (three stages of four sets of
+    waves once left 16 KB for a table of up to 32)."""
+    for key, value in itertools.product((1, 64, 65, 128, 192, 256), repeat=2):
+        pad = -(-key // 64) * 64 + -(-value // 64) * 64
+        if sets > 1 and pad > 256:
+            with pytest.raises(_ffi.KhError):
+                _ffi.plan_heads_lds(key, value, sets, 0)
+            continue
+        for table in (0, 4, 16384, 16388, 20000, 32764, 32768, 32772, 1 << 20):
+            lds = _ffi.plan_heads_lds(key, value, sets, table)
+            assert lds <= 160 * 1024, (key, value, sets, table, lds)
+            stages, rest = divmod(lds - (table if table <= 32768 else 0), sets * 64 * pad)
+            assert rest == 0 and stages in (2, 3)

@@ -177,10 +177,11 @@ def test_waves_that_share_keys(gpu, dtype, n, heads, kv_heads):
 
 
 @BOTH
-@pytest.mark.parametrize("kw", [dict(dim=20, vdim=28), dict(dim=100, vdim=70), dict(dim=200, vdim=40, heads=18, kv_heads=1)])
+@pytest.mark.parametrize("kw", [dict(dim=20, vdim=28), dict(dim=100, vdim=70), dict(dim=100, vdim=40), dict(dim=40, vdim=100),
+                                dict(dim=40, vdim=180), dict(dim=180, vdim=40), dict(dim=200, vdim=40, heads=18, kv_heads=1)])
 def test_steps_with_one_split_and_more(gpu, dtype, kw):
-    """Decode steps around the last position whose keys and values stay in one workgroup: 128, 64 and 51 positions in fp32, twice
-    that in bf16; steps of one and of four sequences, and the graphs of generate()."""
+    """Decode steps around the last position whose keys and values stay in one workgroup: 51 to 128 positions in fp32, twice that
+    in bf16; steps of one and of four sequences, and the graphs of generate()."""
     mod = U.Model(U.gusorax([U.windowed(window=70, rows=16, far=50.0, **kw), U.chunked(chunk=400, **kw)]))
     last = 64 * 1024 // ((-(-kw["dim"] // 64) + -(-kw["vdim"] // 64)) * 64 * (4 if dtype == "float32" else 2))
     toks = mod.tokens(last + 9)
@@ -199,6 +200,30 @@ def test_steps_with_one_split_and_more(gpu, dtype, kw):
         seq = toks[:n] + [int(t) for t in words[n - 1: steps - 1]]
         U.check(m.logits()[None], mod.logits(seq)[-1:], dtype, "generate")
         m.close()
+
+
+@BOTH
+@pytest.mark.parametrize("dim,vdim", [(128, 64), (50, 120), (128, 128), (60, 60)])
+@pytest.mark.parametrize("far", [250.0, 400.0, 500.0, 900.0])
+def test_large_distance_tables(gpu, dtype, dim, vdim, far):
+    """Tables of 15, 24, 29 and 52 KB (32 KB at most go to LDS), beside the stages of every kernel: prompts, steps of one
+    and of four sequences on one split and on several, generate()."""
+    mod = U.Model(U.gusorax([U.windowed(heads=16, kv_heads=1, dim=dim, vdim=vdim, scale=dim ** -0.5, window=1000, rows=64, far=far)]))
+    toks = mod.tokens(260)
+    want = mod.logits(toks)
+    m = mod.load(dtype, max_seqs=4)
+    U.check(U.run_alone(m, toks, (3, 4, 5, 90, 91, 258, 259)), want, dtype, "portions")
+    seqs = [m.open_seq() for _ in range(4)]
+    at = [30, 1, 80, 250]
+    m.forward([(s, toks[:n], []) for s, n in zip(seqs, at)])
+    for k in range(3):
+        U.check(m.forward([(s, [toks[n + k]], [0]) for s, n in zip(seqs, at)]), want[[n + k for n in at]], dtype, "batch")
+    m.close()
+    m = mod.load(dtype)
+    words, _ = m.generate(toks[:20], 30)
+    seq = toks[:20] + [int(t) for t in words[19:29]]
+    U.check(m.logits()[None], mod.logits(seq)[-1:], dtype, "generate")
+    m.close()
 
 
 def test_prompt_of_several_passes(gpu):
