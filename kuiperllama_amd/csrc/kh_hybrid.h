@@ -228,7 +228,7 @@ int hy_unfused_step(kh_model* m);
 int hy_argmax_partial(kh_model* m);
 // ---- kh_hybrid_step.hip
 int hy_step_init(kh_model* m);
-void hy_launch_step(kh_model* m, int advance, int n_forced);
+int hy_launch_step(kh_model* m, int advance, int n_forced);
 int hy_decode_max(const kh_model* m);  // sequences the fused step can take at once
 int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits);
 struct HyTail {  // device lists of the wanted tokens of a pass: their rows, ids, positions, slots

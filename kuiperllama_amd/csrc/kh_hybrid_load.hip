@@ -785,7 +785,7 @@ int finish(kh_model* m, Plan& pl) {
   // one eager step (token 0 at position 0 of slot 0, which every sequence starts by overwriting): kernel attributes and
   // the one-token tables exist before a step is ever captured
   if ((rc = hy_kv_ensure(m, 0, 1)) != KH_OK) return rc;
-  hy_launch_step(m, 0, 0);
+  if ((rc = hy_launch_step(m, 0, 0)) != KH_OK) return rc;
   if ((rc = kh_launch_status()) != KH_OK) return rc;
   KH_CHECK_HIP(hipStreamSynchronize(m->stream));
   return KH_OK;

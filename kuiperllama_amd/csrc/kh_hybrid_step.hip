@@ -444,16 +444,18 @@ int hy_step_init(kh_model* m) {
 }
 
 // the generate loop's step: (d_token, d_pos) of slot 0, sampler behind it
-void hy_launch_step(kh_model* m, int advance, int n_forced) {
+int hy_launch_step(kh_model* m, int advance, int n_forced) {
   Hybrid& hy = *m->hy;
+  if (dbg("KH_HY_STEP_FAIL")) return KH_ERR_INTERNAL;
   if (hy.step_st->bmax >= 1) {
     const LdTabs tb{m->d_token, m->d_pos, hy.step_st->tabs + TB_ZERO};
-    (void)step_any(m, 1, tb, m->logits);
+    TRY(step_any(m, 1, tb, m->logits));
   } else {  // the pass kernels leave logits; the sampler wants partials
-    (void)hy_unfused_step(m);
-    (void)hy_argmax_partial(m);
+    TRY(hy_unfused_step(m));
+    TRY(hy_argmax_partial(m));
   }
   launch_sample(m, advance, n_forced);
+  return KH_OK;
 }
 int hy_launches(const kh_model* m) {
   int n = 2;

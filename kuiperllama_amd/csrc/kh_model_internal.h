@@ -192,7 +192,7 @@ void launch_cls(kh_model* m);
 void launch_sample(kh_model* m, int advance, int n_forced);
 // variant (see kh_model::sg): which attention / wo pair the launches of a step use
 int step_variant(const kh_model* m, int pos_lo, int pos_hi);
-void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant);
+int launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant);
 int launch_step_unfused(kh_model* m, int pos);
 void set_state(kh_model* m, int token, int pos);
 int ensure_pinned_words(kh_model* m, int n);

@@ -113,7 +113,7 @@ extern "C" int kh_model_profile_step(kh_model* m, int32_t start_pos, int32_t n_s
   set_state(m, 1 % c.vocab_size, start_pos);
   int rc = KH_OK;
   for (int s = 0; s < n_steps && rc == KH_OK; ++s) {
-    launch_step_fused(m, 1, 0, ev.data(), step_variant(m, start_pos + s, start_pos + s));
+    if ((rc = launch_step_fused(m, 1, 0, ev.data(), step_variant(m, start_pos + s, start_pos + s))) != KH_OK) break;
     hipError_t e = hipStreamSynchronize(m->stream);
     if (e != hipSuccess) {
       rc = (int)e;

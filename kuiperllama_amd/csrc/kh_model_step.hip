@@ -424,7 +424,7 @@ static void launch_layer(kh_model* m, int l, F&& mark) {
   mark();
 }
 // one fused decode step = 5L + 2 launches.  ev (optional) receives an event after each launch.
-void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant) {
+int launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant) {
   m->step_var = variant;
   if (m->hy) return hy_launch_step(m, advance, n_forced);
   int e = 0;
@@ -437,6 +437,7 @@ void launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, i
   mark();
   launch_sample(m, advance, n_forced);
   mark();
+  return KH_OK;
 }
 
 // the reference's own launch sequence, one C-ABI op per reference kernel (llama3.cpp:147-167)
@@ -569,8 +570,14 @@ void destroy_step_graphs(kh_model* m) {
 
 int capture_steps(kh_model* m, int n_forced, int steps, int variant, hipGraph_t* g, hipGraphExec_t* ge) {
   KH_CHECK_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-  for (int i = 0; i < steps; ++i) launch_step_fused(m, /*advance=*/1, n_forced, nullptr, variant);
+  int rc = KH_OK;
+  for (int i = 0; i < steps && rc == KH_OK; ++i) rc = launch_step_fused(m, /*advance=*/1, n_forced, nullptr, variant);
   hipError_t e = hipStreamEndCapture(m->stream, g);
+  if (rc != KH_OK) {
+    if (e == hipSuccess && *g) (void)hipGraphDestroy(*g);
+    *g = nullptr;
+    return rc;
+  }
   if (e != hipSuccess) return (int)e;
   KH_CHECK_HIP(hipGraphInstantiate(ge, *g, nullptr, nullptr, 0));
   return KH_OK;
@@ -701,8 +708,8 @@ extern "C" int kh_model_predict(kh_model* m, int32_t token, int32_t pos, int32_t
   if (exec == KH_EXEC_UNFUSED) {
     rc = launch_step_unfused(m, pos);
   } else if (exec == KH_EXEC_FUSED || exec == KH_EXEC_GRAPH) {
-    launch_step_fused(m, /*advance=*/0, /*n_forced=*/0, nullptr, step_variant(m, pos, pos));
-    rc = kh_launch_status();
+    rc = launch_step_fused(m, /*advance=*/0, /*n_forced=*/0, nullptr, step_variant(m, pos, pos));
+    if (rc == KH_OK) rc = kh_launch_status();
   } else {
     return KH_ERR_INVALID_ARG;
   }
@@ -863,11 +870,15 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
     m->first_pos = start;
   }
   if (!last_row) set_state(m, h_prompt[start], start);
-  auto launch_chunk = [&](int s) -> int {  // enqueue the next 1 or KH_GRAPH_STEPS steps (positions s ..)
+  // enqueue the next 1 or KH_GRAPH_STEPS steps (positions s ..); -1: failed, the reason in rc
+  auto launch_chunk = [&](int s) -> int {
+    auto done = [&](int code, int n) { return (rc = code) == KH_OK ? n : -1; };
+    auto keep_logits = [&]() -> int {
+      return (int)hipMemcpyAsync(m->first_logits, m->logits, sizeof(float) * (size_t)c.vocab_size, hipMemcpyDeviceToDevice, m->stream);
+    };
     if (s == start && last_row) {
       launch_tail_step(m, h_prompt[s], s, last_row, n_forced);
-      return hipMemcpyAsync(m->first_logits, m->logits, sizeof(float) * (size_t)c.vocab_size, hipMemcpyDeviceToDevice,
-                            m->stream) == hipSuccess ? 1 : -1;
+      return done(keep_logits(), 1);
     }
     if (exec == KH_EXEC_GRAPH) {
       // the largest of 8 / 4 / 2 / 1 steps that still fits (a single-step launch costs ~15 us of graph-launch gap:
@@ -877,25 +888,18 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
       const bool keep = s == start && start > 0;  // first sampled step behind a prefill: alone, logits kept
       if (keep) n = 1;
       hipGraphExec_t ge = nullptr;
-      if (step_graph_n(m, n_forced, step_variant(m, s, s + n - 1), n, &ge) != KH_OK) return -1;
-      if (hipGraphLaunch(ge, m->stream) != hipSuccess) return -1;
-      if (keep && hipMemcpyAsync(m->first_logits, m->logits, sizeof(float) * (size_t)c.vocab_size,
-                                 hipMemcpyDeviceToDevice, m->stream) != hipSuccess)
-        return -1;
-      return n;
+      if ((rc = step_graph_n(m, n_forced, step_variant(m, s, s + n - 1), n, &ge)) != KH_OK) return -1;
+      if ((rc = (int)hipGraphLaunch(ge, m->stream)) != KH_OK) return -1;
+      return keep ? done(keep_logits(), n) : n;
     }
-    launch_step_fused(m, 1, n_forced, nullptr, step_variant(m, s, s));
-    if (s == start && start > 0 &&
-        hipMemcpyAsync(m->first_logits, m->logits, sizeof(float) * (size_t)c.vocab_size, hipMemcpyDeviceToDevice,
-                       m->stream) != hipSuccess)
-      return -1;
-    return 1;
+    if ((rc = launch_step_fused(m, 1, n_forced, nullptr, step_variant(m, s, s))) != KH_OK) return -1;
+    return s == start && start > 0 ? done(keep_logits(), 1) : 1;
   };
   int n_out = total_steps;
   if (n_stop == 0) {
     for (int s = start; s < total_steps;) {
       const int n = launch_chunk(s);
-      if (n < 0) return (int)hipErrorUnknown;
+      if (n < 0) return rc;
       s += n;
     }
     KH_CHECK_HIP(hipEventRecord(m->ev1, m->stream));
@@ -930,7 +934,7 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
     while (stop_at < 0 && (launched < total_steps || n_infl > 0)) {
       while (launched < total_steps && n_infl < 2) {
         const int n = launch_chunk(launched);
-        if (n < 0) return fail((int)hipErrorUnknown);
+        if (n < 0) return fail(rc);
         const int slot = (head + n_infl) & 1;
         KH_CHECK_DRAIN(hipMemcpyAsync(m->h_words_pin + launched, m->d_words + launched,
                                       sizeof(int32_t) * n, hipMemcpyDeviceToHost, m->stream));

@@ -226,6 +226,27 @@ def test_large_distance_tables(gpu, dtype, dim, vdim, far):
     m.close()
 
 
+def test_a_step_that_fails_is_reported(gpu, hook):
+    """A step that cannot be launched, in graphs as in eager calls, ends the call with its reason; the next call is as before."""
+    mod = U.Model(U.gusorax([U.windowed(), U.chunked()]))
+    toks = mod.tokens(5)
+    m, other = mod.load("float32"), mod.load("float32")
+    want, _ = other.generate(toks, 20)
+    for exec_ in ("graph", "fused"):
+        hook("KH_HY_STEP_FAIL", "1")
+        for call in (lambda: m.generate(toks, 20, exec=exec_), lambda: m.generate(toks, 20, exec=exec_, stop=[999]),
+                     lambda: m.predict(toks[0], 0, exec=exec_)):
+            with pytest.raises(_ffi.KhError) as e:
+                call()
+            assert e.value.code == _ffi.KH_ERR_INTERNAL
+        with pytest.raises(_ffi.KhError):
+            mod.load("float32")
+        _ffi.debug_set("KH_HY_STEP_FAIL", None)
+        assert m.generate(toks, 20, exec=exec_)[0] == want
+    other.close()
+    m.close()
+
+
 def test_prompt_of_several_passes(gpu):
     """More tokens than one pass holds."""
     mod = U.Model(U.gusorax([U.windowed(8, 2, 16, 16, 0.4, 300, 16, 100.0), dict(U.chunked(16, 8, 8, 8, 0.5, 256), mlp=U.clamped(3, 2, 8))],
