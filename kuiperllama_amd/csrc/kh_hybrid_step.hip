@@ -17,12 +17,12 @@ struct Hybrid::Step {
   float *x[3] = {nullptr, nullptr, nullptr}, *xn2 = nullptr, *in = nullptr, *xc = nullptr, *mid = nullptr, *v = nullptr,
         *he = nullptr, *hs = nullptr, *z = nullptr, *id_w = nullptr, *sh_g = nullptr, *part = nullptr, *logits = nullptr;
   void* Q = nullptr;
-  int32_t *ids = nullptr, *mates = nullptr, *tabs = nullptr;
+  int32_t *ids = nullptr, *tabs = nullptr;
   int32_t* h_tabs = nullptr;
   int nsplit = 1, head_wg = 1;
   ~Step() {
     for (void* p : {(void*)x[0], (void*)x[1], (void*)x[2], (void*)xn2, (void*)in, (void*)xc, (void*)mid, (void*)v, (void*)he,
-                    (void*)hs, (void*)z, (void*)id_w, (void*)sh_g, (void*)part, (void*)logits, Q, (void*)ids, (void*)mates, (void*)tabs})
+                    (void*)hs, (void*)z, (void*)id_w, (void*)sh_g, (void*)part, (void*)logits, Q, (void*)ids, (void*)tabs})
       if (p) (void)hipFree(p);
     if (h_tabs) (void)hipHostFree(h_tabs);
   }
@@ -205,7 +205,6 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.gu = f.gu.w;
         a.he = st.he;
         a.ids = st.ids;
-        a.mates = st.mates;
         a.id_w = st.id_w;
         a.sh_g = st.sh_g;
         a.top = f.top;
@@ -337,7 +336,6 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.he = st.he;
         a.hs = st.hs;
         a.ids = st.ids;
-        a.mates = st.mates;
         a.id_w = f.ident ? st.id_w : nullptr;
         a.sh_g = f.sgate ? st.sh_g : nullptr;
         a.xn2 = st.xn2;
@@ -431,7 +429,6 @@ int hy_step_init(kh_model* m) {
   TRY(f(&st.logits, B * (size_t)hy.c.vocab));
   TRY(f((float**)&st.Q, B * Q));
   TRY(dalloc(&st.ids, B * top));
-  TRY(dalloc(&st.mates, B * top));
   TRY(dalloc(&st.tabs, TB_N));
   KH_CHECK_HIP(hipHostMalloc((void**)&st.h_tabs, TB_N * 4, hipHostMallocDefault));
   memset(st.h_tabs, 0, TB_N * 4);

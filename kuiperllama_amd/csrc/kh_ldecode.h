@@ -416,9 +416,7 @@ struct LdMidArgs {
   const float *corr, *xn2;
   const void* gu;        // experts [2 ffp][ldw]
   float* he;             // [B][top][ffp], weighted
-  // [B][top], written for k_ld_out.  ids: -1 for an identity expert, and for one that an earlier sequence chose as well: the
-  // first of them multiplies its weights for all.  mates: byte q is 1 + the place where later sequence q chose the same expert
-  int32_t *ids, *mates;
+  int32_t* ids;          // [B][top] (-1: identity), written for k_ld_out
   float *id_w, *sh_g;    // [B]
   int nwg_e, top, n_out, n_expert, shared, ffp, ldz, W, ldw, over_chosen;
   GateAct act;
@@ -464,12 +462,13 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
       x[j] = i < n4 ? ((const f32x4*)(a.xn2 + (size_t)q * a.ldw))[i] : f4_zero();
     }
     // one sequence: every wave makes the choice for itself: its weight loads leave without a barrier.  Several: the waves make
-    // one sequence's each, and an expert that several chose is read once.  Bound by the bytes of the experts (2048 x 1024 in bf16,
-    // four sequences, 6 of 32 and 4 identities each: 21 choices of 17 experts): 39.4 -> 35.5 us in front of latent attention,
-    // 31.6 -> 28.3 of mamba, k_ld_out 26.3 -> 24.6
+    // one sequence's each, and an expert that several chose is read once, by the first of them.  Bound by the bytes of the
+    // experts (2048 x 1024 in bf16, four sequences, 6 of 32 and 4 identities each: 21 choices of 17 experts): 39.4 -> 35.5 us
+    // in front of latent attention, 31.6 -> 28.3 of mamba.  k_ld_out does not do so: there a sequence's sum would be taken in
+    // an order that depends on what the others chose (26.3 -> 24.6 us)
     float idw = 0.f, w = 0.f;
     int id = -1;
-    unsigned mates = 0;
+    unsigned mates = 0;  // byte q: 1 + the place where later sequence q chose the same expert
     if constexpr (B > 1) {
       const int qw = wave % B;
       int my_id = 0;
@@ -498,10 +497,7 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
         if (o < q) first = false;
         else mates |= (unsigned)(__builtin_ctzll(hit) + 1) << (8 * o);
       }
-      if (part == 0 && threadIdx.x == 0) {
-        a.ids[q * a.top + k] = first ? id : -1;
-        a.mates[q * a.top + k] = (int)mates;
-      }
+      if (part == 0 && threadIdx.x == 0) a.ids[q * a.top + k] = id;
       if (!first) return;  // the whole workgroup agrees
       id = __builtin_amdgcn_readfirstlane(id);
       mates = (unsigned)__builtin_amdgcn_readfirstlane((int)mates);
@@ -956,7 +952,7 @@ struct LdOutArgs {
   const float* v;         // [B][ld_v] mixer vector
   const void *down, *sdown;  // experts [W][ffp] each; shared [W][sffp]
   const float *he, *hs;   // [B][top][ffp] (weighted), [B][sffp]
-  const int32_t *ids, *mates;  // [B][top], see LdMidArgs
+  const int32_t* ids;     // [B][top]
   const float *id_w, *sh_g, *xn2, *x_cur;  // id_w, sh_g: nullptr = none, 1
   const float* bias;      // of W_o, or nullptr
   float* x_out;           // [B][ld]
@@ -1069,25 +1065,6 @@ __global__ __launch_bounds__(512, 4) void k_ld_out(const LdOutArgs a) {
           for (int p = 0; p < P; ++p) x[u][p] = in[u] ? x[u][p] : f4_zero();
 #pragma unroll
           for (int r = 0; r < R; ++r) acc[r][q] = dot(w[r][u], x[u], acc[r][q]);
-          if constexpr (B > 1) {
-            const unsigned mates = (unsigned)a.mates[q * a.top + k];
-            if (!mates) continue;  // uniform
-            bool other;
-            const int c = chunk(a.ffp, e + u - k * nbe, other);
-#pragma unroll
-            for (int o = q + 1; o < B; ++o) {
-              const int ko = (int)(mates >> (8 * o) & 255) - 1;
-              if (ko < 0) continue;
-              const float* v = a.he + (size_t)(o * a.top + ko) * a.ffp + (size_t)c * E;
-              f32x4 xo[P];
-#pragma unroll
-              for (int p = 0; p < P; ++p) xo[p] = *(const f32x4*)(v + 4 * p);
-#pragma unroll
-              for (int p = 0; p < P; ++p) xo[p] = in[u] ? xo[p] : f4_zero();
-#pragma unroll
-              for (int r = 0; r < R; ++r) acc[r][o] = dot(w[r][u], xo, acc[r][o]);
-            }
-          }
         }
       }
   }

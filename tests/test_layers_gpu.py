@@ -109,6 +109,33 @@ def test_batches_that_share_experts(gpu, dtype, n, same):
 
 
 @BOTH
+@pytest.mark.parametrize("kw", [dict(experts=6, identity=2, top=4), dict(experts=3, identity=0, top=2, shared=0),
+                                dict(experts=10, identity=4, top=7, ff=600)])
+def test_steps_do_not_depend_on_the_other_sequences(gpu, dtype, kw):
+    """The logits of a step are the same bit by bit alone and among one to three others, in front of them and behind them,
+    whose experts are the same, some of them the same, and none."""
+    mod = U.Model(U.config([U.with_ff(U.mamba(), **kw), U.with_ff(U.latent(), **kw)]))
+    mine = mod.tokens(30, seed=1)
+
+    def steps(others, at):
+        m = mod.load(dtype, max_seqs=4)
+        toks = list(others)
+        toks.insert(at, mine)
+        seqs = [m.open_seq() for _ in toks]
+        for s, t in zip(seqs, toks):
+            m.forward([(s, t[:20], [])])
+        out = [m.forward([(s, [t[k]], [0]) for s, t in zip(seqs, toks)])[at] for k in range(20, 30)]
+        m.close()
+        return np.stack(out)
+
+    alone = steps([], 0)
+    for n in (1, 2, 3):
+        for others in ([mine] * n, [mod.tokens(30, seed=5 + k) for k in range(n)], [mine] * (n - 1) + [mod.tokens(30, seed=9)]):
+            for at in (0, n):
+                np.testing.assert_array_equal(steps(others, at), alone, err_msg=f"{n} others, place {at}")
+
+
+@BOTH
 @pytest.mark.parametrize("loop", [None, (0, 1, 1), (0, 2, 3), (1, 3, 2), (2, 3, 2)])
 def test_loop_ranges(gpu, dtype, loop):
     layers = [U.with_ff(U.latent()), U.mamba(), U.with_ff(U.latent(2), identity=0)]
