@@ -198,7 +198,9 @@ inline HeadsArgs heads_args(const Hybrid& hy, const HyHeads& a, const void* cach
   return h;
 }
 
-// decode steps up to position pos_hi: no attention over heads is split (step variant 0; 1 else)
+// Decode steps up to position pos_hi: no attention over heads is split (step variant 0; 1 else).  The steps of generate() and
+// predict(), of one sequence, take variant 0 where they can; those of forward() always take 1, or a sequence's last bits would
+// depend on how far the others are.  A layer whose span alone bounds its keys is not split in either.
 inline bool hy_one_split(const Hybrid& hy, const HyHeads& a, int pos_hi) {
   int keys = pos_hi + 1;
   if (a.span.window > 0) keys = std::min(keys, a.span.window);

@@ -440,12 +440,7 @@ int run_pass(kh_model* m, const Pass& ps, float* h_logits) {
   Runner<T> r(m, ps);
   TRY(r.layers());
   if (!ps.n_want) return KH_OK;
-  if (ps.tail) {
-    int last = 0;
-    for (const PassSeg& sg : ps.segs) last = std::max(last, sg.pos0 + sg.n - 1);
-    m->step_var = hy_step_variant(hy, last);
-    return hy_tail(m, ps.wanted, ps.n_want, h_logits);
-  }
+  if (ps.tail) return hy_tail(m, ps.wanted, ps.n_want, h_logits);
   TRY(r.combine(nullptr, false, -1));
   for (int w = 0; w < ps.n_want; w += hy.wl_rows) {
     const int n = std::min(hy.wl_rows, ps.n_want - w);

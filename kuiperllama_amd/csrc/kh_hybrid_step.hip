@@ -480,6 +480,7 @@ int hy_tail(kh_model* m, const HyTail& t, int n, float* h_logits) {
   Hybrid::Step& st = *hy.step_st;
   const HyLayer& l = hy.layers[(size_t)hy.runs.back().layer];
   const bool mamba = l.mixer == HY_MAMBA1;
+  m->step_var = 1;  // as in hy_decode
   for (int i = 0; i < n;) {
     const int B = std::min(st.bmax, n - i >= 4 ? 4 : (n - i >= 2 ? 2 : 1));
     const LdTabs tb{t.tok + i, t.pos + i, t.slot + i};
@@ -508,7 +509,7 @@ int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits) {
     st.h_tabs[TB_SLOT + i] = e[i].slot;
   }
   KH_CHECK_HIP(hipMemcpyAsync(st.tabs, st.h_tabs, TB_ZERO * 4, hipMemcpyHostToDevice, m->stream));
-  m->step_var = hy_step_variant(hy, *std::max_element(st.h_tabs + TB_POS, st.h_tabs + TB_POS + n));
+  m->step_var = 1;  // whatever the positions: a sequence's bits are its own, alone and beside others
   for (int i = 0; i < n;) {  // n = 3: 2 + 1
     const int B = n - i >= 4 ? 4 : (n - i >= 2 ? 2 : 1);
     const LdTabs tb{st.tabs + TB_TOK + i, st.tabs + TB_POS + i, st.tabs + TB_SLOT + i};

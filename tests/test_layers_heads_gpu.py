@@ -181,7 +181,8 @@ def test_waves_that_share_keys(gpu, dtype, n, heads, kv_heads):
                                 dict(dim=40, vdim=180), dict(dim=180, vdim=40), dict(dim=200, vdim=40, heads=18, kv_heads=1)])
 def test_steps_with_one_split_and_more(gpu, dtype, kw):
     """Decode steps around the last position whose keys and values stay in one workgroup: 51 to 128 positions in fp32, twice that
-    in bf16; steps of one and of four sequences, and the graphs of generate()."""
+    in bf16: predict() and the graphs of generate(), which take one workgroup that far, and steps of one and of four sequences,
+    which take it for the window alone."""
     mod = U.Model(U.gusorax([U.windowed(window=70, rows=16, far=50.0, **kw), U.chunked(chunk=400, **kw)]))
     last = 64 * 1024 // ((-(-kw["dim"] // 64) + -(-kw["vdim"] // 64)) * 64 * (4 if dtype == "float32" else 2))
     toks = mod.tokens(last + 9)
@@ -193,6 +194,12 @@ def test_steps_with_one_split_and_more(gpu, dtype, kw):
     m.forward([(s, toks[:n], []) for s, n in zip(seqs, at)])
     for k in range(5):
         U.check(m.forward([(s, [toks[n + k]], [0]) for s, n in zip(seqs, at)]), want[[n + k for n in at]], dtype, "batch")
+    m.close()
+    m = mod.load(dtype)
+    for pos in range(last + 4):
+        m.predict(toks[pos], pos)
+        if pos < 4 or pos >= last - 3:
+            U.check(m.logits()[None], want[pos: pos + 1], dtype, f"predict {pos}")
     m.close()
     for n, steps in ((3, 30), (last - 5, last + 6), (last + 3, last + 9)):
         m = mod.load(dtype)
@@ -224,6 +231,32 @@ def test_large_distance_tables(gpu, dtype, dim, vdim, far):
     seq = toks[:20] + [int(t) for t in words[19:29]]
     U.check(m.logits()[None], mod.logits(seq)[-1:], dtype, "generate")
     m.close()
+
+
+@BOTH
+def test_steps_do_not_depend_on_the_other_sequences(gpu, dtype):
+    """The logits of a step bit by bit alone and beside others, in front of them and behind them, some of them far beyond the
+    keys that one workgroup takes."""
+    kw = dict(dim=100, vdim=100)
+    mod = U.Model(U.gusorax([dict(U.windowed(window=70, rows=16, far=50.0, **kw), mlp=U.clamped(7, 3, 600)),
+                             dict(U.chunked(chunk=400, **kw), mlp=U.clamped())]))
+    mine = mod.tokens(60, seed=1)
+
+    def steps(others, at):
+        m = mod.load(dtype, max_seqs=4)
+        rows = [(mod.tokens(n + 8, seed=n), n) for n in others]
+        rows.insert(at, (mine, 50))
+        seqs = [m.open_seq() for _ in rows]
+        for s, (t, n) in zip(seqs, rows):
+            m.forward([(s, t[:n], [])])
+        out = [m.forward([(s, [t[n + k]], [0]) for s, (t, n) in zip(seqs, rows)])[at] for k in range(8)]
+        m.close()
+        return np.stack(out)
+
+    alone = steps([], 0)
+    for others in ([20], [380], [21, 22], [400, 20, 300], [20, 30, 40]):
+        for at in (0, len(others)):
+            np.testing.assert_array_equal(steps(others, at), alone, err_msg=f"{others}, place {at}")
 
 
 def test_a_step_that_fails_is_reported(gpu, hook):
