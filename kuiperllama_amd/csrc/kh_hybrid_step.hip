@@ -198,6 +198,7 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       a.t = tb;
       a.eps = hy.c.eps;
       size_t lds = 0;
+      bool share = false;
       if (f.top) {
         a.z = st.z;
         a.corr = f.corr.p;
@@ -218,7 +219,8 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.W = W;
         a.ldw = f.gu.ld;
         a.nwg_e = cdiv(f.ffp / 2, 4 * cdiv(B * f.top * f.ffp / 2, 3072));
-        lds = B * vec_b<T>(Wp);
+        share = ld_shares(B, f.top, f.n_out());
+        lds = (share ? B : 1) * vec_b<T>(Wp);
       }
       a.ldv = mamba ? l.mb.innerp : in_ld;
       int extra = 0;
@@ -261,8 +263,11 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       }
       TRY(with_nv<T>(Wp, [&](auto nv) {
         return with_rp(f.top ? f.n_out() : 1, [&](auto rp) {
-          return go(k_ld_mid<T, B, decltype(nv)::value, decltype(rp)::value>, dim3(B * a.top * a.nwg_e + a.nwg_m + extra), 256, lds,
-                    s, a);
+          constexpr int NV = decltype(nv)::value, RP = decltype(rp)::value;
+          const dim3 grid(B * a.top * a.nwg_e + a.nwg_m + extra);
+          if constexpr (B > 1)
+            if (share) return go(k_ld_mid<T, B, NV, RP, true>, grid, 256, lds, s, a);
+          return go(k_ld_mid<T, B, NV, RP, false>, grid, 256, lds, s, a);
         });
       }));
     }

@@ -438,20 +438,31 @@ struct LdMidArgs {
   float eps;
   LdTabs t;
 };
-template <class T, int B, int NV, int RP>
+// Steps of B sequences: are the experts that several of them chose read once (k_ld_mid<.., SHARE>)?  That takes the LDS of B
+// vectors and a barrier in front of the first weight, so it has to save something: with even routing, one choice in sixteen is
+// also an earlier sequence's.  us a step of four mamba layers of 1024 columns with few choices alike, each sequence's own / read
+// once, two and four sequences: 4 of 128 132 / 140 and 168 / 175, 8 of 256 148 / 151 and 195 / 199, 8 of 512 with 128 columns
+// 141 / 147 and 177 / 187; with many (6 of 36 outputs) see k_ld_mid.
+static inline bool ld_shares(int B, int top, int n_out) {
+  const double p = (double)top / n_out;
+  double none = 1.0;  // that no one of B chose an expert
+  for (int q = 0; q < B; ++q) none *= 1.0 - p;
+  return 1.0 - (1.0 - none) / (B * p) >= 1.0 / 16;
+}
+template <class T, int B, int NV, int RP, bool SHARE>
 __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
-  constexpr int R = 4, U = 4;
+  constexpr int R = 4, U = 4, SB = SHARE ? B : 1;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float* xs = (float*)smem_raw;
   __shared__ float red[KH_WAVES_MAX];
-  __shared__ int32_t rid[B][KH_MOE_MAX_TOP];
-  __shared__ float rwt[B][KH_MOE_MAX_TOP];
+  __shared__ int32_t rid[SB][KH_MOE_MAX_TOP];
+  __shared__ float rwt[SB][KH_MOE_MAX_TOP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int wg = blockIdx.x;
   LdTile<T, R, U> t;
   const T* row[R];
   const int ne = B * a.top * a.nwg_e;
-  if (wg < ne) {  // ---- one chosen expert of one sequence, and of those behind it that chose it too
+  if (wg < ne) {  // ---- one chosen expert of one sequence (SHARE: and of those behind it that chose it too)
     const int pair = wg / a.nwg_e, part = wg - pair * a.nwg_e, q = pair / a.top, k = pair - q * a.top;
     const int nblk = Ld<T>::blocks(a.ldw), nch = a.ldw / Ld<T>::E;
     const int n4 = a.ldw >> 2, total4 = nblk * Ld<T>::BE / 4;
@@ -461,15 +472,15 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
       const int i = threadIdx.x + 256 * j;
       x[j] = i < n4 ? ((const f32x4*)(a.xn2 + (size_t)q * a.ldw))[i] : f4_zero();
     }
-    // one sequence: every wave makes the choice for itself: its weight loads leave without a barrier.  Several: the waves make
-    // one sequence's each, and an expert that several chose is read once, by the first of them.  Bound by the bytes of the
-    // experts (2048 x 1024 in bf16, four sequences, 6 of 32 and 4 identities each: 21 choices of 17 experts): 39.4 -> 35.5 us
-    // in front of latent attention, 31.6 -> 28.3 of mamba.  k_ld_out does not do so: there a sequence's sum would be taken in
-    // an order that depends on what the others chose (26.3 -> 24.6 us)
+    // Every wave makes the choice for itself: its weight loads leave without a barrier.  SHARE: the waves make one sequence's
+    // each, and an expert that several chose is read once, by the first of them.  Bound by the bytes of the experts (2048 x
+    // 1024 in bf16, four sequences, 6 of 32 and 4 identities each: 21 choices of 17 experts): 39.4 -> 35.5 us in front of latent
+    // attention, 31.6 -> 28.3 of mamba.  k_ld_out does not do so: there a sequence's sum would be taken in an order that depends
+    // on what the others chose (26.3 -> 24.6 us).
     float idw = 0.f, w = 0.f;
     int id = -1;
     unsigned mates = 0;  // byte q: 1 + the place where later sequence q chose the same expert
-    if constexpr (B > 1) {
+    if constexpr (SHARE) {
       const int qw = wave % B;
       int my_id = 0;
       float my_w = 0.f;
@@ -503,25 +514,25 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
       mates = (unsigned)__builtin_amdgcn_readfirstlane((int)mates);
       w = rwt[q][k];
     } else {
-    const float wf = moe_route<RP>(a.z + (size_t)q * a.ldz, a.corr, a.n_out, a.top, a.over_chosen, lane,
-                                   [&](int kk, int i, float wt) __attribute__((always_inline)) {
-      const bool ident = i >= a.n_expert;
-      if (ident) idw += wt;
-      if (kk == k) {
-        id = ident ? -1 : i;
-        w = wt;
+      const float wf = moe_route<RP>(a.z + (size_t)q * a.ldz, a.corr, a.n_out, a.top, a.over_chosen, lane,
+                                     [&](int kk, int i, float wt) __attribute__((always_inline)) {
+        const bool ident = i >= a.n_expert;
+        if (ident) idw += wt;
+        if (kk == k) {
+          id = ident ? -1 : i;
+          w = wt;
+        }
+      });
+      w *= wf;
+      idw *= wf;
+      if (part == 0 && threadIdx.x == 0) {
+        a.ids[q * a.top + k] = id;
+        if (k == 0) {
+          a.id_w[q] = idw;
+          if (a.shared) a.sh_g[q] = sigmoid1(a.z[(size_t)q * a.ldz + a.n_out]);
+        }
       }
-    });
-    w *= wf;
-    idw *= wf;
-    if (part == 0 && threadIdx.x == 0) {
-      a.ids[q * a.top + k] = id;
-      if (k == 0) {
-        a.id_w[q] = idw;
-        if (a.shared) a.sh_g[q] = sigmoid1(a.z[(size_t)q * a.ldz + a.n_out]);
-      }
-    }
-    if (id < 0) return;  // identity expert: no tensors (the whole workgroup agrees)
+      if (id < 0) return;  // identity expert: no tensors (the whole workgroup agrees)
     }
     const T* base = (const T*)a.gu + (size_t)id * 2 * a.ffp * a.ldw;
     const int items = a.ffp / 2;
@@ -541,11 +552,11 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
     for (int j = 0; j < NV; ++j)
       if ((int)threadIdx.x + 256 * j < total4) ((f32x4*)xs)[ld_slot<T>(threadIdx.x + 256 * j)] = x[j];
     // vector j > 0: the j-th of the mates, in rising order of their sequences
-    int n = 1, dst[B];
-    float wj[B];
+    int n = 1, dst[SB];
+    float wj[SB];
     dst[0] = pair;
     wj[0] = w;
-    if constexpr (B > 1) {
+    if constexpr (SHARE) {
 #pragma unroll
       for (int j = 1; j < B; ++j) {
         dst[j] = pair;
@@ -593,8 +604,8 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
       }
     };
     if (n == 1) rows_of(std::integral_constant<int, 1>());
-    else if (B == 2 || n == 2) rows_of(std::integral_constant<int, B < 2 ? 1 : 2>());
-    else rows_of(std::integral_constant<int, B>());  // three of four: what the fourth place holds is finite or not, and not stored
+    else if (SB == 2 || n == 2) rows_of(std::integral_constant<int, SB < 2 ? 1 : 2>());
+    else rows_of(std::integral_constant<int, SB>());  // three of four: what the fourth place holds is finite or not, and not stored
     return;
   }
   wg -= ne;

@@ -94,7 +94,8 @@ def test_expert_tiles(gpu, dtype, n, kw):
 def test_batches_that_share_experts(gpu, dtype, n, same):
     """Steps of sequences of which the first `same` are alike, so that they choose the same experts, the others a few of them."""
     layers = [U.with_ff(U.mamba(), experts=6, identity=2, top=4), U.with_ff(U.latent(), experts=3, identity=0, top=2, shared=0),
-              U.with_ff(U.mamba(), experts=80, identity=4, top=7, ff=66)]
+              U.with_ff(U.mamba(), experts=80, identity=4, top=7, ff=66),
+              U.with_ff(U.mamba(), experts=130, identity=2, top=3, ff=34)]  # too many for two sequences to share
     mod = U.Model(U.config(layers))
     alike = mod.tokens(30, seed=1)
     toks = [alike if i < same else mod.tokens(30, seed=10 + i) for i in range(n)]
@@ -110,10 +111,10 @@ def test_batches_that_share_experts(gpu, dtype, n, same):
 
 @BOTH
 @pytest.mark.parametrize("kw", [dict(experts=6, identity=2, top=4), dict(experts=3, identity=0, top=2, shared=0),
-                                dict(experts=10, identity=4, top=7, ff=600)])
+                                dict(experts=10, identity=4, top=7, ff=600), dict(experts=70, identity=5, top=4, ff=70)])
 def test_steps_do_not_depend_on_the_other_sequences(gpu, dtype, kw):
     """The logits of a step are the same bit by bit alone and among one to three others, in front of them and behind them,
-    whose experts are the same, some of them the same, and none."""
+    whose experts are the same, some of them the same, and none, where they are read once for several and where they are not."""
     mod = U.Model(U.config([U.with_ff(U.mamba(), **kw), U.with_ff(U.latent(), **kw)]))
     mine = mod.tokens(30, seed=1)
 
