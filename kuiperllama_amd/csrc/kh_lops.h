@@ -177,7 +177,9 @@ __global__ __launch_bounds__(256) void k_conv_silu(const ConvArgs<T> a, const Sc
   const int u0 = (int)(blockIdx.y % KH_CONV_PER) * TT, n = ck.n - u0;
   const int c = (blockIdx.x * 256 + threadIdx.x) * E;
   if (n <= 0 || c >= a.C) return;
-  const bool vec = (a.C & (E - 1)) == 0 && (a.ldx & (E - 1)) == 0;
+  // whole fragments, but for the last lane of a row that ends inside its channels (with scalar loads for all lanes there, 2048
+  // tokens of 4100 channels take 26.2 us instead of 21.5, of 1100 13.0 instead of 12.0)
+  const bool vec = c + E <= a.C && (a.ldx & (E - 1)) == 0;
   const int t0 = ck.row0 + u0, i0 = t0 - a.p.seg_row0[ck.seg];  // rows of the segment in front of the first token
   const int taps = TAPS ? TAPS : a.taps;
   const bool fresh = a.p.seg_pos0[ck.seg] == 0;
