@@ -7,6 +7,7 @@
 // Result: lane (j, h) holds elements (m = 4 h + 0..3, n = j), m from the first operand, n from the second.
 #pragma once
 #include "kh_common.h"
+#include "kh_softplus.h"
 
 namespace khm {
 typedef __bf16 bf16;
@@ -66,25 +67,7 @@ __device__ __forceinline__ float gated1(const GateAct& c, float g, float u) {
   u = fminf(fmaxf(u, -c.limit), c.limit);
   return g * sigmoid1(c.alpha * g) * (u + c.shift);
 }
-// log(1 + e^z) without overflow: max(z, 0) + log1p(e), e = e^-|z|, log1p(e) = 2 atanh(s), s = e / (2 + e) <= 1/3 by its series (the
-// first term left out is below 2^-26 of the sum).  The library's log1pf and expf cost three times as much.
 __device__ __forceinline__ float softplus1(float z) {
-  float a = fabsf(z);
-  a = a > 126.f ? 126.f : a;  // (NaN stays)
-  constexpr float L = 1.44269502f, L_lo = 1.92596299e-8f;  // log2(e)
-  const float t = -a * L, lo = __builtin_fmaf(-a, L_lo, __builtin_fmaf(-a, L, -t));
-  float e = __builtin_amdgcn_exp2f(t);
-  e = __builtin_fmaf(e, lo * 0.693147181f, e);
-  const float d = 2.0f + e;
-  float r = __builtin_amdgcn_rcpf(d);
-  r = __builtin_fmaf(r, __builtin_fmaf(-d, r, 1.0f), r);
-  const float s = e * r, q = s * s;
-  float p = __builtin_fmaf(q, 1.f / 13, 1.f / 11);
-  p = __builtin_fmaf(q, p, 1.f / 9);
-  p = __builtin_fmaf(q, p, 1.f / 7);
-  p = __builtin_fmaf(q, p, 1.f / 5);
-  p = __builtin_fmaf(q, p, 1.f / 3);
-  const float s2 = s + s;
-  return fmaxf(z, 0.f) + __builtin_fmaf(s2 * q, p, s2);
+  return softplus_of(z, [](float h) { return __builtin_amdgcn_rcpf(h); });
 }
 }  // namespace khm
