@@ -293,6 +293,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     if (KEEP && m == TM - 1) lost[n][i] += __builtin_fmaf(f, g, acc[n][m][i] - s);
     acc[n][m][i] = s;
   };
+  // (of a sum that has overflowed, what was lost is the opposite infinity, then NaN)
+  auto settle = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[n][TM - 1][i] += fabsf(lost[n][i]) < INFINITY ? lost[n][i] : 0.f;
+  };
   float sgn = 1.0f, xinv[TM];
   unsigned xe[TM];
   auto row_top = [&](float v) __attribute__((always_inline)) {  // over the four lanes of row fr
@@ -499,8 +506,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       }
       sgn = -sgn;
     }
-#pragma unroll
-    for (int n = 0; n < TN; ++n) acc[n][TM - 1] += lost[n];
+    settle();
   };
   const std::true_type first{};
   const std::false_type second{};
@@ -528,8 +534,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       close();
     }
   }
-#pragma unroll
-  for (int n = 0; n < TN; ++n) acc[n][TM - 1] += lost[n];
+  settle();
   if constexpr (!Q) {
     // a half that has overflowed has left infinities or NaN in its row
     float all = 0.f;

@@ -5,6 +5,7 @@ import dataclasses
 import numpy as np
 import pytest
 
+import exact_kv
 from kuiperllama_amd import _ffi, binfmt
 from test_model_gpu import _PF_SPECS, KV_ATOL_GEMM, _atol
 
@@ -51,6 +52,27 @@ def test_last_token_in_the_pass(gpu, name, chunk, monkeypatch):
     if later:
         assert m.generate(prompt, 60, stop=[words[later]])[0] == words[:later]
     m.close()
+
+
+def test_sums_beyond_fp32(gpu):
+    """A value column whose group scale takes its sums beyond fp32 is infinite in every row, also in those of the token whose
+    sums are kept longer and of the 15 beside it."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = dataclasses.replace(SPECS["int8"], seq_len=512)
+    img = binfmt.synth_image(spec, seed=43, device=gpu)
+    t = exact_kv.tensors(img, spec)
+    scales = t["wv.0.scales"].reshape(spec.kv_dim, -1)
+    scales[5] = 0.0
+    scales[5, 0] = 1e38
+    for n in (17, 33, 60, 130, 300):
+        toks = [int(i) for i in np.random.default_rng(n).integers(0, spec.vocab_size, n)]
+        m = KuiperModel.from_device_image(img, spec)
+        m.generate(toks, n, exec="fused")
+        v = m.read_kv(0, 0, n)[1]
+        m.close()
+        want = exact_kv.rows(img, spec, toks)[0][1][:, 5]
+        assert np.isinf(v[:, 5]).all() and np.array_equal(np.sign(v[:, 5]), np.sign(want)), n
+        assert np.isfinite(np.delete(v, 5, axis=1)).all()
 
 
 def test_prompt_of_the_whole_cache(gpu):
