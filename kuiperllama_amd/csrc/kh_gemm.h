@@ -566,7 +566,7 @@ __global__ __launch_bounds__(KH_WG) void k_pg_rmsnorm(float* __restrict__ X,
 }
 
 // RoPE of the T query rows and of the T fresh key rows, in place (cpu/rope_kernel.cpp:18-42 half,
-// :98-121 interleaved); token t sits at position pos0 + t.  blockIdx.x = token.
+// :98-121 interleaved); token t sits at position pos0 + t.  dim 0: keys alone.  blockIdx.x = token.
 static __global__ __launch_bounds__(KH_WG) void k_pg_rope(float* __restrict__ Q, float* __restrict__ kc,
                                                    const float* __restrict__ sin_cache,
                                                    const float* __restrict__ cos_cache, int dim,

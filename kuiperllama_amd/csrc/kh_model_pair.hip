@@ -293,7 +293,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
                : (c.rope_mode == KH_ROPE_HALF ? (c.head_size % 32 == 0 ? KH_PG_ROPE_TILES : KH_PG_ROPE_OFF) : KH_PG_ROPE_PAIRS);
       if ((rc = pair_launch<KH_PG_QKV>(m, a, nullptr)) != KH_OK) return rc;
       if (a.rope == KH_PG_ROPE_OFF)
-        hipLaunchKernelGGL(k_pg_rope, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_q, a.kc, m->sin_cache, m->cos_cache, c.dim, c.kv_dim,
+        hipLaunchKernelGGL(k_pg_rope, dim3(T), dim3(KH_WG), 0, m->stream, m->pg_q, a.kc, m->sin_cache, m->cos_cache, a.rows0, c.kv_dim,
                            c.head_size, pos0, c.rope_mode);
     }
     // the prompt phase leaves K/V rows and nothing else: the last layer's attention, wo and feed-forward feed nothing

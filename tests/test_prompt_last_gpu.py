@@ -54,6 +54,26 @@ def test_last_token_in_the_pass(gpu, name, chunk, monkeypatch):
     m.close()
 
 
+@pytest.mark.parametrize("name", ["mha-interleaved", "one-layer", "qwen-bias"])
+def test_rotation_of_its_own(gpu, name, monkeypatch):
+    """Rows and logits with the rotation behind the GEMM instead of in it; the last layer has keys and no queries."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = dataclasses.replace(SPECS.get(name) or _PF_SPECS[name], seq_len=512)
+    m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=44, device=gpu), spec)
+    for n in (18, 150):
+        toks = [int(t) for t in np.random.default_rng(n).integers(0, spec.vocab_size, n)]
+        out = []
+        for fuse in ("1", "0"):
+            monkeypatch.setenv("KH_PG_ROPE_FUSE", fuse)
+            m.generate(toks, n)
+            out.append((m.logits(), [m.read_kv(l, 0, n) for l in range(spec.n_layers)]))
+        np.testing.assert_allclose(out[1][0], out[0][0], rtol=0, atol=_atol(spec))
+        for a, b in zip(out[0][1], out[1][1]):
+            for x, y in zip(a, b):
+                np.testing.assert_allclose(y, x, rtol=0, atol=KV_ATOL_GEMM)
+    m.close()
+
+
 def test_sums_beyond_fp32(gpu):
     """A value column whose group scale takes its sums beyond fp32 is infinite in every row, also in those of the token whose
     sums are kept longer and of the 15 beside it."""
