@@ -225,7 +225,7 @@ bool pg_slice_attention(kh_model* m, int layer, int T, int pos0, int layout, int
 bool pair_geometry(const kh_config& c);
 int pair_part_rows(const kh_config& c, int rows);  // partial rows of passes of up to `rows` tokens
 void pair_prepare(kh_model* m, int n, int pos0);  // memory of the attention of a prompt's passes, if there is any
-int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0);
+int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0, bool last);
 bool pair_takes_last(const kh_config& c, int T);
 // kh_model_prefill_gemm of the first n - 1 tokens of a prompt, or of all n: then *last is the residual row of the last token
 // in front of the last layer (valid until the next pass), else nullptr

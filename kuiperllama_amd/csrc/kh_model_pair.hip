@@ -150,9 +150,10 @@ bool pair_geometry(const kh_config& c) {
 // Is the last of T tokens of a pass cheaper in the pass than as a step of its own?  The step reads a layer's weights once more
 // (5 TB/s behind 10 us of launches a layer); in the pass the token may open another row of tiles, and where the model of
 // pair_shape sees a near tie the step was faster.  Time to the first token, ms, step of its own / in the pass, T tokens:
-// Llama-3.2-1B 17 2.62 / 1.88, 193 3.75 / 2.99, 512 5.18 / 4.37, 641 6.45 / 5.96; Qwen2.5-0.5B 41 2.35 / 1.79; TinyLlama 1793
-// 13.9 / 13.2; Llama-2-7B int8 33 6.28 / 5.10, 225 12.1 / 10.7, 561 21.1 / 21.3 (the one length measured where the rule errs);
-// not taken: Llama-3.2-1B 513 5.18 / 5.43, 1025 8.10 / 9.05; Llama-2-7B int8 65 6.83 / 7.07, 449 17.1 / 17.3.
+// Llama-3.2-1B 17 2.71 / 2.10, 193 3.86 / 3.16, 512 5.43 / 4.57, 641 6.68 / 6.23; Qwen2.5-0.5B 41 2.41 / 1.92; TinyLlama 1793
+// 14.4 / 14.1; Llama-2-7B int8 33 6.37 / 5.36, 225 12.3 / 11.2, 617 24.1 / 22.3; of 55 lengths the rule erred at two, int8 561
+// 21.7 / 22.1 and Qwen 1025 5.59 / 5.73.  Not taken: Llama-3.2-1B 513 5.18 / 5.43, 1025 8.10 / 9.05; Llama-2-7B int8 65 6.83 /
+// 7.07, 449 17.1 / 17.3.
 bool pair_takes_last(const kh_config& c, int T) {
   if (T < 2) return false;
   const PairDims d = pair_dims(c);
@@ -254,8 +255,9 @@ bool pair_attention(kh_model* m, int l, int T, int pos0) {
 }
 }  // namespace
 
-// forward of T (<= pg_rows) prompt tokens at positions pos0..: fills their K/V cache rows
-int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0) {
+// forward of T (<= pg_rows) prompt tokens at positions pos0..: fills their K/V cache rows.  last: logits are taken from the last
+// token's row in front of the last layer
+int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0, bool last) {
   const kh_config& c = m->cfg;
   int rc;
   if ((rc = kh_embedding_f32_host(toks, T, m->tok_emb, m->pg_x, c.dim, c.vocab_size, (void*)m->stream)) != KH_OK) return rc;
@@ -274,6 +276,7 @@ int launch_prefill_pair_chunk(kh_model* m, const int32_t* toks, int T, int pos0)
     base.T = T;
     base.pos0 = pos0;
     base.tcap = T;
+    base.keep = last && l < c.layer_num - 1;
     base.xe_ld = m->pg_rows;
     base.xs = m->pg_xs;
     base.part = m->pg_part;

@@ -614,7 +614,7 @@ int khm::prefill_gemm(kh_model* m, const int32_t* h_tokens, int n, int pos0, con
   if (pair) {
     pair_prepare(m, n, pos0);
     for (int t0 = 0; t0 < n; t0 += chunk)
-      if ((rc = launch_prefill_pair_chunk(m, h_tokens + t0, n - t0 < chunk ? n - t0 : chunk, pos0 + t0)) != KH_OK) return rc;
+      if ((rc = launch_prefill_pair_chunk(m, h_tokens + t0, std::min(n - t0, chunk), pos0 + t0, last && n - t0 <= chunk)) != KH_OK) return rc;
     if (last) *last = m->pg_x + (size_t)((n - 1) % chunk) * c.dim;
     return kh_launch_status();
   }

@@ -24,7 +24,7 @@
 // 512 / 1900 tokens as without, 1.8 / 0.95 / 0.7 times as long as on the fp32 matrix cores.  (With one request in flight in
 // the second way and in the search for the scales: 3.5 / 3.3 / 3.2 times as long as without.  The workgroup once more through
 // its ring, decided by a vote: 2.35 / 2.0 / 1.95, and 1 % slower where nothing overflows.)
-// Where the last token of a prompt is in the pass (pair_takes_last), logits come from it: see fold.
+// Where the last token of a prompt is in the pass (pair_takes_last), logits come from it: see `product`.
 // K/V rows of models of eight layers and 400 tokens, rms against 64 bits: 4.3e-7 (int8), 5.6e-7 (fp32); on the fp32 matrix
 // cores 1.2e-6 and 1.3e-6.  That needs numbers that weigh alike in a result to lie within about 2^12 of one another where
 // they share a scale.
@@ -60,6 +60,7 @@ struct KhPairArgs {
   const unsigned char* xe;  // RESID: 1 / its scales, one per token and stage of columns, at pair_exp_at
   int xe_ld;
   int fine;            // RESID, fp32: the two stages of 64 columns may differ in scale
+  int keep;            // the last token's result goes into logits: its sums are kept longer
   float* out;          // QKV: Q [T][ldo]; RESID: X [T][ldo] (+=)
   char* pairs;         // SWIGLU: pair slab of the gated unit, [T][ldo / 32]
   unsigned char* out_e;  // SWIGLU: 1 / its scales
@@ -178,9 +179,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       }
     }
   };
-  // Row r of the tile -> token: as it comes, but for the last tile, whose 16-row tiles turn within a wave until the last token
-  // lies in the last of them: that one's sums are kept longer (fold).
-  const int turn = t0 + C::BM < a.T ? 0 : ((a.T - 1 - t0) >> 4) + 1;
+  // The tile with the token that logits come from: its 16-row tiles turn within a wave until that token lies in the last of
+  // them, whose sums are kept longer (fold).
+  constexpr bool KEEPS = EPI != KH_PG_QKV;
+  const bool keep = KEEPS && a.keep && t0 + C::BM >= a.T;  // uniform
+  const int turn = keep ? ((a.T - 1 - t0) >> 4) + 1 : 0;
   auto token_of = [&](int r) __attribute__((always_inline)) {
     const int m = r >> 4;
     return t0 + ((m / TM * TM + (m + turn) % TM) << 4) + (r & 15);
@@ -277,29 +280,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   // The matrix unit rounds its sums down: a bias that the mean over many cached rows keeps while it averages everything else
   // (logits behind 1900 prompt tokens: 1.7e-6 from 64 bits instead of 1.3e-6 on fp32 fma chains).  Every other group takes
   // its weights with the sign turned and is subtracted, which cancels it: 1.1e-6.
-  // Every group's sum is folded into the accumulators with one rounding of them, the largest error of a long dot product.
-  // For the last 16 tokens of a wave it is kept and added at the end (lost): the logits behind the prompt come from the last
-  // token, while the rows of the others are averaged over by those that attend to them.  Logits from 64 bits (mean of six
-  // models), steps of their own on fp32 fma chains / in the pass without this / with it, Llama-3.2-1B 40, 150, 512 tokens:
-  // 1.20 1.17 1.08e-6 / 1.29 1.36 1.23 / 1.02 1.13 1.00; Qwen2.5-0.5B 300: 7.1e-7 / - / 7.5; Llama-2-7B int8 60, 225: 3.7
-  // 3.4e-6 / 3.6 3.6 / 3.4 3.3.  It takes 1 to 2 % of a prompt.  The largest tile spills with it in RESID, whose sums are
-  // shorter (kz); int8 loses 3 % with it everywhere.
-  constexpr bool KEEP = Q ? EPI == KH_PG_QKV : EPI != KH_PG_RESID || TM <= 4;
-  f32x4 lost[TN];
-#pragma unroll
-  for (int n = 0; n < TN; ++n) lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto fold = [&](int n, int m, int i, float f, float g) __attribute__((always_inline)) {
-    const float s = __builtin_fmaf(f, g, acc[n][m][i]);
-    if (KEEP && m == TM - 1) lost[n][i] += __builtin_fmaf(f, g, acc[n][m][i] - s);
-    acc[n][m][i] = s;
-  };
-  // (of a sum that has overflowed, what was lost is the opposite infinity, then NaN)
-  auto settle = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int n = 0; n < TN; ++n)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[n][TM - 1][i] += fabsf(lost[n][i]) < INFINITY ? lost[n][i] : 0.f;
-  };
   float sgn = 1.0f, xinv[TM];
   unsigned xe[TM];
   auto row_top = [&](float v) __attribute__((always_inline)) {  // over the four lanes of row fr
@@ -331,220 +311,269 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
       wl[e] = lo.x; wl[e + 1] = lo.y;
     }
   };
-  auto stage = [&](int k, auto open) __attribute__((always_inline)) {
-    constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a sum
-    // stage k has landed when at most the requests of the stages behind it are outstanding
-    // (and with it the scales, which were requested before those)
-    if (NST > 2 && k + NST - 2 < nk) wait_vm<(NST - 2) * C::NL>();
-    else wait_vm<0>();
-    __syncthreads();
-    const int at = z0 + k;
-    if (GROUP && k > 0 && (at & 15) == 0 && ((at >> 4) + 1) * 16 < z1) issue_exps((at >> 4) + 1);
-    const unsigned char* exps = (const unsigned char*)smem_raw + NST * C::STAGE + ((at >> 4) & 1) * C::EX * 1024 + (at & 15);
-    if (k + NST - 1 < nk) issue(fill);
-    const char* st = smem_raw + slot * C::STAGE;
-    const char* wst = st + C::XR * 1024;
-    if constexpr (!Q) {
-      f16x8 xh[TM], xl[TM];
-      f32x4 wv[TN][2];
+  // Every group's sum is folded into the accumulators with one rounding of them, the largest error of a long dot product.  The
+  // rows of a prompt's tokens are averaged over by those that attend to them, but logits come from the last one's.  Its tile of
+  // 16 tokens (m = TM - 1) runs a loop of its own, in which what a fold rounds off is summed and added at the end (lost), and,
+  // with fp32 weights, every stage's sum starts from zero and has the product lo lo as well; the other tiles of the workgroup
+  // are as ever, and a pass without the last token has no such workgroup.  wq + wk + wv do without: it took 10 % of them behind
+  // 777 tokens (int8) and left fp32 models where they were.  Logits from 64 bits (mean of 4 to 16 models), the token as a step
+  // of its own on fp32 fma chains / in the pass with the sums of all others / with its own:
+  //   Qwen2.5-0.5B 41, 300 tokens 7.1 7.3e-7 / - - / 6.9 7.0; TinyLlama 700, 1900 1.13 1.09e-6 / - - / 0.98 0.92; Llama-3.2-1B
+  //   150, 512 1.17 1.08e-6 / 1.36 1.23 / 1.08 0.86; Llama-2-7B int8 60, 225, 777 3.8 3.7 3.0e-6 / 3.6 3.6 - / 3.4 3.5 2.9;
+  //   stories15M 60, 200 2.53 2.49e-7 / - - / 2.56 2.54 (40 models, deviation of a mean 0.04).
+  // Prompts without it: 1 to 3 % faster (Llama-2-7B int8 777 tokens 25.9 ms instead of 26.9, Qwen 41 1.84 instead of 1.91).
+  auto product = [&](auto kept) __attribute__((always_inline)) {
+    constexpr bool KEEP = decltype(kept)::value;
+    f32x4 lost[KEEP ? TN : 1];
 #pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        const int r = (wn * TN + n) * 16 + fr;
-        wv[n][0] = *(const f32x4*)(wst + r * 128 + (((2 * fh) ^ pair_swz(r)) << 4));
-        wv[n][1] = *(const f32x4*)(wst + r * 128 + (((2 * fh + 1) ^ pair_swz(r)) << 4));
-      }
+    for (int n = 0; n < (KEEP ? TN : 1); ++n) lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto fold = [&](int n, int m, int i, float f, float g) __attribute__((always_inline)) {
+      const float s = __builtin_fmaf(f, g, acc[n][m][i]);
+      if (KEEP && m == TM - 1) lost[n][i] += __builtin_fmaf(f, g, acc[n][m][i] - s);
+      acc[n][m][i] = s;
+    };
+    // (of a sum that has overflowed, what was lost is the opposite infinity, then NaN)
+    auto settle = [&]() __attribute__((always_inline)) {
+      if constexpr (!KEEP) return;
 #pragma unroll
-      for (int m = 0; m < TM; ++m) {
-        const int r = (wm * TM + m) * 16 + fr;
-        xh[m] = *(const f16x8*)(st + r * 128 + ((fh ^ pair_swz(r)) << 4));
-        xl[m] = *(const f16x8*)(st + r * 128 + (((4 + fh) ^ pair_swz(r)) << 4));
-      }
-      if constexpr (GROUP) {
+      for (int n = 0; n < TN; ++n)
 #pragma unroll
-        for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
-      }
-      if (OPEN && k == 0) {
+        for (int i = 0; i < 4; ++i) acc[n][TM - 1][i] += fabsf(lost[n][i]) < INFINITY ? lost[n][i] : 0.f;
+    };
+    auto stage = [&](int k, auto open) __attribute__((always_inline)) {
+      constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a sum
+      // stage k has landed when at most the requests of the stages behind it are outstanding
+      // (and with it the scales, which were requested before those)
+      if (NST > 2 && k + NST - 2 < nk) wait_vm<(NST - 2) * C::NL>();
+      else wait_vm<0>();
+      __syncthreads();
+      const int at = z0 + k;
+      if (GROUP && k > 0 && (at & 15) == 0 && ((at >> 4) + 1) * 16 < z1) issue_exps((at >> 4) + 1);
+      const unsigned char* exps = (const unsigned char*)smem_raw + NST * C::STAGE + ((at >> 4) & 1) * C::EX * 1024 + (at & 15);
+      if (k + NST - 1 < nk) issue(fill);
+      const char* st = smem_raw + slot * C::STAGE;
+      const char* wst = st + C::XR * 1024;
+      if constexpr (!Q) {
+        f16x8 xh[TM], xl[TM];
+        f32x4 wv[TN][2];
 #pragma unroll
         for (int n = 0; n < TN; ++n) {
-          const float t = row_top(fmaxf(pair_top4(wv[n][0]), pair_top4(wv[n][1])));
-          wsc[n] = pair_scale_to(t, 10);
-          if (__builtin_amdgcn_ballot_w64(t == 0.f)) wsc[n] = row_scale(n);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        f16x8 wh, wl;
-        split(wv[n], wsc[n], wh, wl);
-#pragma unroll
-        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wl, xh[m], OPEN ? f4_zero() : grp[n][m]);
-#pragma unroll
-        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wh, xl[m], grp[n][m]);
-#pragma unroll
-        for (int m = 0; m < TM; ++m) grp[n][m] = mfma_pair(wh, xh[m], grp[n][m]);
-      }
-    } else {
-      // lane (i, h) takes columns 16 h .. + 15 of its 64-column group; either product takes eight of them
-      f16x8 xh[TM][2], xl[TM][2];
-      i32x4 qv[TN];
-      f32x4 sc[TN];
-#pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        const int r = (wn * TN + n) * 16 + fr;
-        qv[n] = *(const i32x4*)(wst + r * 64 + ((fh ^ ((r & 4) >> 1)) << 4));
-        sc[n] = *(const f32x4*)(wst + C::WR * 1024 + ((wn * TN + n) * 16 + 4 * fh) * 4);
-      }
-#pragma unroll
-      for (int m = 0; m < TM; ++m) {
-        const int r = (wm * TM + m) * 16 + fr;
-        const char* row = st + ((fh >> 1) * C::BM + r) * 128;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          const int c = 2 * (fh & 1) + b;
-          xh[m][b] = *(const f16x8*)(row + ((c ^ pair_swz(r)) << 4));
-          xl[m][b] = *(const f16x8*)(row + (((4 + c) ^ pair_swz(r)) << 4));
-        }
-      }
-      if constexpr (GROUP) {
-#pragma unroll
-        for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int m = 0; m < TM; ++m)
-        if (GROUP) xinv[m] = sgn * __uint_as_float(xe[m] << 23);
-#pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        const f16x8 w0 = pair_q8((unsigned)qv[n].x, (unsigned)qv[n].y, sgn), w1 = pair_q8((unsigned)qv[n].z, (unsigned)qv[n].w, sgn);
-        const f32x4 sg = {sc[n].x * sgn, sc[n].y * sgn, sc[n].z * sgn, sc[n].w * sgn};
-        f32x4 g[TM];
-#pragma unroll
-        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w0, xl[m][0], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w1, xl[m][1], g[m]);
-#pragma unroll
-        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w0, xh[m][0], g[m]);
-#pragma unroll
-        for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w1, xh[m][1], g[m]);
-#pragma unroll
-        for (int m = 0; m < TM; ++m)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) fold(n, m, i, GROUP ? sc[n][i] * xinv[m] : sg[i], g[m][i]);
-      }
-    }
-    __builtin_amdgcn_s_setprio(0);
-    slot = slot + 1 == NST ? 0 : slot + 1;
-    fill = fill + 1 == NST ? 0 : fill + 1;
-  };
-  auto close = [&]() __attribute__((always_inline)) {
-    if constexpr (!Q) {
-#pragma unroll
-      for (int m = 0; m < TM; ++m) xinv[m] = GROUP ? sgn * __uint_as_float(xe[m] << 23) : sgn;
-#pragma unroll
-      for (int n = 0; n < TN; ++n) {
-#pragma unroll
-        for (int m = 0; m < TM; ++m)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) fold(n, m, i, xinv[m], grp[n][m][i]);
-        wsc[n] = -wsc[n];
-      }
-    }
-    sgn = -sgn;
-  };
-  // The wave's tiles once more, from memory, with scales from all columns (x * 0 above: also where the inputs are not finite).
-  auto again = [&]() __attribute__((always_inline)) {
-    const float* w[TN];
-    sgn = 1.0f;
-#pragma unroll
-    for (int n = 0; n < TN; ++n) {
-      wsc[n] = row_scale(n);
-      w[n] = row_at(n) + 8 * fh;
-      lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    constexpr int PART = GROUP && TM > 4 ? 4 : TM;  // token tiles requested at once (eight with their scales spill)
-#pragma nounroll
-    for (int k = z0; k < z1; ++k) {
-      f32x4 wv[TN][2];
-#pragma unroll
-      for (int n = 0; n < TN; ++n) {
-        wv[n][0] = *(const f32x4*)(w[n] + 32 * k);
-        wv[n][1] = *(const f32x4*)(w[n] + 32 * k + 4);
-      }
-      f16x8 wh[TN], wl[TN];
-#pragma unroll
-      for (int m0 = 0; m0 < TM; m0 += PART) {
-        f16x8 xh[PART], xl[PART];
-        unsigned e[PART];
-#pragma unroll
-        for (int m = 0; m < PART; ++m) {
-          int t = token_of((wm * TM + m0 + m) * 16 + fr);
-          t = t < a.T ? t : a.T - 1;
-          const char* x = a.X + ((unsigned)t * (unsigned)(4 * K) + 128u * k + 16u * fh);
-          xh[m] = *(const f16x8*)x;
-          xl[m] = *(const f16x8*)(x + 64);
-          e[m] = GROUP ? a.xe[pair_exp_at(k, t, a.xe_ld)] : 127u;
-        }
-        __builtin_amdgcn_sched_barrier(0);  // requests in front of products
-        if (m0 == 0) {
-#pragma unroll
-          for (int n = 0; n < TN; ++n) split(wv[n], sgn * wsc[n], wh[n], wl[n]);
+          const int r = (wn * TN + n) * 16 + fr;
+          wv[n][0] = *(const f32x4*)(wst + r * 128 + (((2 * fh) ^ pair_swz(r)) << 4));
+          wv[n][1] = *(const f32x4*)(wst + r * 128 + (((2 * fh + 1) ^ pair_swz(r)) << 4));
         }
 #pragma unroll
-        for (int m = 0; m < PART; ++m) {
-          const float f = sgn * __uint_as_float(e[m] << 23);
+        for (int m = 0; m < TM; ++m) {
+          const int r = (wm * TM + m) * 16 + fr;
+          xh[m] = *(const f16x8*)(st + r * 128 + ((fh ^ pair_swz(r)) << 4));
+          xl[m] = *(const f16x8*)(st + r * 128 + (((4 + fh) ^ pair_swz(r)) << 4));
+        }
+        if constexpr (GROUP) {
+#pragma unroll
+          for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
+        }
+        if (OPEN && k == 0) {
 #pragma unroll
           for (int n = 0; n < TN; ++n) {
-            const f32x4 g = mfma_pair(wh[n], xh[m], mfma_pair(wh[n], xl[m], mfma_pair(wl[n], xh[m], f4_zero())));
-#pragma unroll
-            for (int i = 0; i < 4; ++i) fold(n, m0 + m, i, f, g[i]);
+            const float t = row_top(fmaxf(pair_top4(wv[n][0]), pair_top4(wv[n][1])));
+            wsc[n] = pair_scale_to(t, 10);
+            if (__builtin_amdgcn_ballot_w64(t == 0.f)) wsc[n] = row_scale(n);
           }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          f16x8 wh, wl;
+          split(wv[n], wsc[n], wh, wl);
+          constexpr int PM = KEEP ? TM - 1 : TM;
+#pragma unroll
+          for (int m = 0; m < PM; ++m) grp[n][m] = mfma_pair(wl, xh[m], OPEN ? f4_zero() : grp[n][m]);
+#pragma unroll
+          for (int m = 0; m < PM; ++m) grp[n][m] = mfma_pair(wh, xl[m], grp[n][m]);
+#pragma unroll
+          for (int m = 0; m < PM; ++m) grp[n][m] = mfma_pair(wh, xh[m], grp[n][m]);
+          if constexpr (KEEP) {
+            constexpr int m = TM - 1;
+            f32x4 g = mfma_pair(wl, xl[m], f4_zero());
+            g = mfma_pair(wh, xh[m], mfma_pair(wh, xl[m], mfma_pair(wl, xh[m], g)));
+            if (OPEN) grp[n][m] = g;
+            else grp[n][m] += g;
+          }
+        }
+      } else {
+        // lane (i, h) takes columns 16 h .. + 15 of its 64-column group; either product takes eight of them
+        constexpr bool LATE = KEEP && GROUP && TM > 4;  // the scales of the weights behind the products, or it spills
+        f16x8 xh[TM][2], xl[TM][2];
+        i32x4 qv[TN];
+        f32x4 sc[TN];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          const int r = (wn * TN + n) * 16 + fr;
+          qv[n] = *(const i32x4*)(wst + r * 64 + ((fh ^ ((r & 4) >> 1)) << 4));
+          if (!LATE) sc[n] = *(const f32x4*)(wst + C::WR * 1024 + ((wn * TN + n) * 16 + 4 * fh) * 4);
+        }
+#pragma unroll
+        for (int m = 0; m < TM; ++m) {
+          const int r = (wm * TM + m) * 16 + fr;
+          const char* row = st + ((fh >> 1) * C::BM + r) * 128;
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            const int c = 2 * (fh & 1) + b;
+            xh[m][b] = *(const f16x8*)(row + ((c ^ pair_swz(r)) << 4));
+            xl[m][b] = *(const f16x8*)(row + (((4 + c) ^ pair_swz(r)) << 4));
+          }
+        }
+        if constexpr (GROUP) {
+#pragma unroll
+          for (int m = 0; m < TM; ++m) xe[m] = exps[((wm * TM + m) * 16 + fr) * 16];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+          if (GROUP) xinv[m] = sgn * __uint_as_float(xe[m] << 23);
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          const f16x8 w0 = pair_q8((unsigned)qv[n].x, (unsigned)qv[n].y, sgn), w1 = pair_q8((unsigned)qv[n].z, (unsigned)qv[n].w, sgn);
+          f32x4 g[TM];
+#pragma unroll
+          for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w0, xl[m][0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w1, xl[m][1], g[m]);
+#pragma unroll
+          for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w0, xh[m][0], g[m]);
+#pragma unroll
+          for (int m = 0; m < TM; ++m) g[m] = mfma_pair(w1, xh[m][1], g[m]);
+          if constexpr (LATE) {
+            __builtin_amdgcn_sched_barrier(0);
+            sc[n] = *(const f32x4*)(wst + C::WR * 1024 + ((wn * TN + n) * 16 + 4 * fh) * 4);
+          }
+          const f32x4 sg = {sc[n].x * sgn, sc[n].y * sgn, sc[n].z * sgn, sc[n].w * sgn};
+#pragma unroll
+          for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) fold(n, m, i, GROUP ? sc[n][i] * xinv[m] : sg[i], g[m][i]);
+        }
+      }
+      __builtin_amdgcn_s_setprio(0);
+      slot = slot + 1 == NST ? 0 : slot + 1;
+      fill = fill + 1 == NST ? 0 : fill + 1;
+    };
+    auto close = [&]() __attribute__((always_inline)) {
+      if constexpr (!Q) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m) xinv[m] = GROUP ? sgn * __uint_as_float(xe[m] << 23) : sgn;
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+#pragma unroll
+          for (int m = 0; m < TM; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) fold(n, m, i, xinv[m], grp[n][m][i]);
+          wsc[n] = -wsc[n];
         }
       }
       sgn = -sgn;
+    };
+    // The wave's tiles once more, from memory, with scales from all columns (x * 0 above: also where the inputs are not finite).
+    auto again = [&]() __attribute__((always_inline)) {
+      const float* w[TN];
+      sgn = 1.0f;
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        wsc[n] = row_scale(n);
+        w[n] = row_at(n) + 8 * fh;
+        if constexpr (KEEP) lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < TM; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      constexpr int PART = GROUP && TM > 4 ? 4 : TM;  // token tiles requested at once (eight with their scales spill)
+#pragma nounroll
+      for (int k = z0; k < z1; ++k) {
+        f32x4 wv[TN][2];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+          wv[n][0] = *(const f32x4*)(w[n] + 32 * k);
+          wv[n][1] = *(const f32x4*)(w[n] + 32 * k + 4);
+        }
+        f16x8 wh[TN], wl[TN];
+#pragma unroll
+        for (int m0 = 0; m0 < TM; m0 += PART) {
+          f16x8 xh[PART], xl[PART];
+          unsigned e[PART];
+#pragma unroll
+          for (int m = 0; m < PART; ++m) {
+            int t = token_of((wm * TM + m0 + m) * 16 + fr);
+            t = t < a.T ? t : a.T - 1;
+            const char* x = a.X + ((unsigned)t * (unsigned)(4 * K) + 128u * k + 16u * fh);
+            xh[m] = *(const f16x8*)x;
+            xl[m] = *(const f16x8*)(x + 64);
+            e[m] = GROUP ? a.xe[pair_exp_at(k, t, a.xe_ld)] : 127u;
+          }
+          __builtin_amdgcn_sched_barrier(0);  // requests in front of products
+          if (m0 == 0) {
+#pragma unroll
+            for (int n = 0; n < TN; ++n) split(wv[n], sgn * wsc[n], wh[n], wl[n]);
+          }
+#pragma unroll
+          for (int m = 0; m < PART; ++m) {
+            const float f = sgn * __uint_as_float(e[m] << 23);
+#pragma unroll
+            for (int n = 0; n < TN; ++n) {
+              const f32x4 g = mfma_pair(wh[n], xh[m], mfma_pair(wh[n], xl[m], mfma_pair(wl[n], xh[m], f4_zero())));
+#pragma unroll
+              for (int i = 0; i < 4; ++i) fold(n, m0 + m, i, f, g[i]);
+            }
+          }
+        }
+        sgn = -sgn;
+      }
+      settle();
+    };
+    const std::true_type first{};
+    const std::false_type second{};
+    if constexpr (Q) {
+      for (int k = 0; k < nk; ++k) {
+        stage(k, first);
+        close();
+      }
+    } else {
+      int k = 0;
+      for (; k + 1 < nk; k += 2) {
+        stage(k, first);
+        if (GROUP && a.fine) {  // uniform
+          close();
+#pragma unroll
+          for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int m = 0; m < TM; ++m) grp[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        stage(k + 1, second);
+        close();
+      }
+      if (k < nk) {
+        stage(k, first);
+        close();
+      }
     }
     settle();
+    if constexpr (!Q) {
+      // a half that has overflowed has left infinities or NaN in its row
+      float all = 0.f;
+#pragma unroll
+      for (int n = 0; n < TN; ++n)
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) all = __builtin_fmaf(acc[n][m][i], 0.f, all);
+      if (__builtin_amdgcn_ballot_w64(all != 0.f)) again();
+    }
   };
-  const std::true_type first{};
-  const std::false_type second{};
-  if constexpr (Q) {
-    for (int k = 0; k < nk; ++k) {
-      stage(k, first);
-      close();
-    }
+  if constexpr (KEEPS) {
+    if (keep) product(std::true_type());
+    else product(std::false_type());
   } else {
-    int k = 0;
-    for (; k + 1 < nk; k += 2) {
-      stage(k, first);
-      if (GROUP && a.fine) {  // uniform
-        close();
-#pragma unroll
-        for (int n = 0; n < TN; ++n)
-#pragma unroll
-          for (int m = 0; m < TM; ++m) grp[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      stage(k + 1, second);
-      close();
-    }
-    if (k < nk) {
-      stage(k, first);
-      close();
-    }
-  }
-  settle();
-  if constexpr (!Q) {
-    // a half that has overflowed has left infinities or NaN in its row
-    float all = 0.f;
-#pragma unroll
-    for (int n = 0; n < TN; ++n)
-#pragma unroll
-      for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) all = __builtin_fmaf(acc[n][m][i], 0.f, all);
-    if (__builtin_amdgcn_ballot_w64(all != 0.f)) again();
+    product(std::false_type());
   }
   // ---- epilogue: lane (fr, fh) of tile (n, m) holds rows 4 fh .. + 3 of the tile for token t0 + .. + fr
   f32x4 wi[TN];

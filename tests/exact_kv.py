@@ -34,8 +34,8 @@ def _rotate(x, spec, pos):
     return (torch.cat([p, q], -1) if half else torch.stack([p, q], -1).flatten(-2)).reshape(x.shape)
 
 
-def rows(img, spec, toks, front=None):
-    """[(K, V)] per layer of `toks` behind the cache rows front[layer] = (K, V)."""
+def rows(img, spec, toks, front=None, logits=None):
+    """[(K, V)] per layer of `toks` behind the cache rows front[layer] = (K, V).  logits: a list that gets the last token's."""
     w, hs, mul = _weights(img, spec), spec.head_size, spec.kv_mul
     old = 0 if front is None else len(front[0][0])
     pos, out = np.arange(old, old + len(toks)), []
@@ -57,6 +57,8 @@ def rows(img, spec, toks, front=None):
         x = x + torch.cat(att, 1) @ w[f"wo.{l}"].T
         h = norm(x, w[f"ffn_norm.{l}"])
         x = x + (torch.nn.functional.silu(h @ w[f"w1.{l}"].T) * (h @ w[f"w3.{l}"].T)) @ w[f"w2.{l}"].T
+    if logits is not None:
+        logits.append((norm(x[-1], w["final_norm"]) @ w["tok_emb" if spec.shared_classifier else "wcls"].T).numpy())
     return out
 
 
