@@ -314,7 +314,8 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
     // lane: keys k0 + 16 n + 4 fh + i of its rows
     frag p[MR];
     const bool edge = k0 + KT - 1 > p_lo || k0 < w_full || k0 + KT > k_hi;
-    const bool near = a.bias && p_lo - (k0 + KT - 1) < a.nbias - 1;
+    // (by the tile's last key, not its last row, as where the table is copied: or a wave would read what was not)
+    const bool near = a.bias && p_lo - ((k0 + KT < k_hi ? k0 + KT : k_hi) - 1) < a.nbias - 1;
 #pragma unroll
     for (int q = 0; q < MR; ++q) {
       if (near) {  // two loads of known address space, not one of a selected address

@@ -106,8 +106,8 @@ def distance_bucket(n, rows, far):
     """Row of a distance table of `rows` entries: one entry per distance below half of them, then entries of equal
     width in log distance up to `far`, the last one for everything beyond."""
     half = rows // 2
-    if n < half:
-        return n
+    if n < half or rows == 1:
+        return min(n, rows - 1)
     x = math.log(n / half) / math.log(far / half) * (rows - half)
     r = round(x)
     if abs(x - r) < 1e-9:  # a border up to rounding of the logarithms

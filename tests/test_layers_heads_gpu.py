@@ -71,6 +71,14 @@ def test_span_sizes(gpu, size):
 
 
 @BOTH
+@pytest.mark.parametrize("kw", [dict(window=45, rows=1), dict(window=1, rows=12), dict(window=45, rows=2), dict(window=300, rows=1)])
+def test_one_bias_for_every_distance(gpu, dtype, kw):
+    """Tables of one entry and two: no distance is nearer than the last entry's, in whole key tiles and where a tile reaches
+    beyond the last key."""
+    against_reference(U.Model(U.gusorax([U.windowed(heads=16, kv_heads=1, **kw), U.chunked(chunk=60)])), dtype, n=150)
+
+
+@BOTH
 @pytest.mark.parametrize("ff", [U.dense(1), U.dense(40), U.dense(130), U.clamped(1, 1, 5), U.clamped(6, 6, 64, 0.1),
                                 U.clamped(70, 5, 8, 3.0), U.clamped(300, 2, 4, 0.5)])
 def test_feed_forwards_alone(gpu, dtype, ff):
@@ -227,9 +235,10 @@ def test_large_distance_tables(gpu, dtype, dim, vdim, far):
         U.check(m.forward([(s, [toks[n + k]], [0]) for s, n in zip(seqs, at)]), want[[n + k for n in at]], dtype, "batch")
     m.close()
     m = mod.load(dtype)
-    words, _ = m.generate(toks[:20], 30)
-    seq = toks[:20] + [int(t) for t in words[19:29]]
-    U.check(m.logits()[None], mod.logits(seq)[-1:], dtype, "generate")
+    for n in (250, 20):  # the first call's graphs are of steps that are split
+        words, _ = m.generate(toks[:n], n + 10)
+        seq = toks[:n] + [int(t) for t in words[n - 1: n + 9]]
+        U.check(m.logits()[None], mod.logits(seq)[-1:], dtype, "generate")
     m.close()
 
 
