@@ -71,6 +71,39 @@ def test_experts_alone(gpu, dtype, kw):
 
 
 @BOTH
+@pytest.mark.parametrize("inner,state,lens", [(4100, 12, (2048,)), (2050, 20, (1000, 1047)), (300, 130, (2048,)), (260, 256, (700, 1, 65, 1282))])
+def test_scans_of_sixteen_states_a_lane(gpu, dtype, inner, state, lens):
+    """Launches with two waves a SIMD at 16 states a lane (csrc/kh_scan.h): one, two, sixteen lanes a channel, states and channels
+    that fill neither, sequences that end inside a chunk, of one token and of two chunks."""
+    mod = U.Model(U.config([U.mamba(inner, state, 3, 4)], width=24, vocab=40))
+    toks = [mod.tokens(n, seed=n) for n in lens]
+    wants = [sorted({0, n // 3, max(0, n - 70), n - 1}) for n in lens]
+    m = mod.load(dtype, max_seqs=len(lens), max_seq_len=2304)
+    seqs = [m.open_seq() for _ in lens]
+    got = m.forward(list(zip(seqs, toks, wants)))
+    more = m.forward([(s, [3], [0]) for s in seqs])  # the states that the pass left
+    m.close()
+    refs = [mod.logits(t + [3]) for t in toks]
+    U.check(got, np.concatenate([r[w] for r, w in zip(refs, wants)]), dtype, "pass")
+    U.check(more, np.stack([r[-1] for r in refs]), dtype, "step")
+
+
+@BOTH
+@pytest.mark.parametrize("n", [1, 2, 4])
+def test_rows_of_more_than_4096_columns(gpu, dtype, n):
+    """Prompts and steps of one, two and four sequences of 4160 columns, of which some choose the same experts."""
+    mod = U.Model(U.config([U.with_ff(U.mamba(), experts=4, top=2), U.with_ff(U.latent(), shared=0)], width=4160, vocab=60))
+    toks = [mod.tokens(14, seed=i // 2) for i in range(n)]
+    want = [mod.logits(t) for t in toks]
+    m = mod.load(dtype, max_seqs=n)
+    seqs = [m.open_seq() for _ in toks]
+    U.check(m.forward([(s, t[:8], [7]) for s, t in zip(seqs, toks)]), np.stack([w[7] for w in want]), dtype, "prompt")
+    for k in range(8, 14):
+        U.check(m.forward([(s, [t[k]], [0]) for s, t in zip(seqs, toks)]), np.stack([w[k] for w in want]), dtype, f"step {k}")
+    m.close()
+
+
+@BOTH
 @pytest.mark.parametrize("n,kw", [(15, dict(experts=2, top=1)), (16, dict(experts=2, top=2)), (17, dict(experts=3, top=2)),
                                   (129, dict(experts=1, top=1)), (130, dict(experts=2, top=2)), (209, dict(experts=3, top=2)),
                                   (257, dict(experts=5, identity=0, top=4)), (400, dict(experts=2, top=1, ff=70)),

@@ -11,7 +11,7 @@ from test_model_gpu import _PF_SPECS, KV_ATOL_GEMM, _atol
 
 pytestmark = pytest.mark.gpu
 
-SPECS = {n: _PF_SPECS[n] for n in ("gqa-half", "int8")}
+SPECS = {n: _PF_SPECS[n] for n in ("gqa-half", "int8", "qwen-bias", "gqa-half-hs128")}
 SPECS["one-layer"] = dataclasses.replace(_PF_SPECS["gqa-half"], n_layers=1)
 
 
