@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   };
   // The tile with the token that logits come from: its 16-row tiles turn within a wave until that token lies in the last of
   // them, whose sums are kept longer (fold).
-  constexpr bool KEEPS = EPI != KH_PG_QKV;
+  constexpr bool KEEPS = Q || EPI != KH_PG_QKV;
   const bool keep = KEEPS && a.keep && t0 + C::BM >= a.T;  // uniform
   const int turn = keep ? ((a.T - 1 - t0) >> 4) + 1 : 0;
   auto token_of = [&](int r) __attribute__((always_inline)) {
@@ -315,13 +315,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
   // rows of a prompt's tokens are averaged over by those that attend to them, but logits come from the last one's.  Its tile of
   // 16 tokens (m = TM - 1) runs a loop of its own, in which what a fold rounds off is summed and added at the end (lost), and,
   // with fp32 weights, every stage's sum starts from zero and has the product lo lo as well; the other tiles of the workgroup
-  // are as ever, and a pass without the last token has no such workgroup.  wq + wk + wv do without: it took 10 % of them behind
-  // 777 tokens (int8) and left fp32 models where they were.  Logits from 64 bits (mean of 4 to 16 models), the token as a step
-  // of its own on fp32 fma chains / in the pass with the sums of all others / with its own:
+  // are as ever, and a pass without the last token has no such workgroup.  wq + wk + wv of fp32 do without: their errors stay
+  // where they are.  Logits from 64 bits (mean of 4 to 16 models), the token as a step of its own on fp32 fma chains / in the
+  // pass with the sums of all others / with its own:
   //   Qwen2.5-0.5B 41, 300 tokens 7.1 7.3e-7 / - - / 6.9 7.0; TinyLlama 700, 1900 1.13 1.09e-6 / - - / 0.98 0.92; Llama-3.2-1B
-  //   150, 512 1.17 1.08e-6 / 1.36 1.23 / 1.08 0.86; Llama-2-7B int8 60, 225, 777 3.8 3.7 3.0e-6 / 3.6 3.6 - / 3.4 3.5 2.9;
+  //   150, 512 1.17 1.08e-6 / 1.36 1.23 / 1.08 0.86; Llama-2-7B int8 60, 225, 777 3.8 3.7 3.0e-6 / 3.6 3.6 - / 3.2 3.3 2.75;
   //   stories15M 60, 200 2.53 2.49e-7 / - - / 2.56 2.54 (40 models, deviation of a mean 0.04).
-  // Prompts without it: 1 to 3 % faster (Llama-2-7B int8 777 tokens 25.9 ms instead of 26.9, Qwen 41 1.84 instead of 1.91).
+  // Prompts without it: 1 to 4 % faster (Llama-2-7B int8 777 tokens 25.9 ms instead of 26.8, Qwen 41 1.84 instead of 1.91).
   auto product = [&](auto kept) __attribute__((always_inline)) {
     constexpr bool KEEP = decltype(kept)::value;
     f32x4 lost[KEEP ? TN : 1];
