@@ -255,7 +255,9 @@ int kh_seq_close(kh_model* m, int32_t seq);
 int kh_seq_length(const kh_model* m, int32_t seq); /* tokens held; < 0: not open */
 /* One step of a batch: every entry appends n_tokens tokens to its sequence (different lengths in one batch; prompts,
  * portions of prompts and single decoded tokens), each sequence at most once.  want = ascending places among an
- * entry's tokens whose logits are copied to h_logits [sum of n_want][vocab], in the order of entries and want. */
+ * entry's tokens whose logits are copied to h_logits [sum of n_want][vocab], in the order of entries and want.
+ * Steps of one token of each entry on the decode kernels (layer-list models, up to four entries, fewer where the vectors of
+ * four exceed the LDS): the bits of an entry's logits do not depend on the other entries. */
 typedef struct kh_batch_entry {
   int32_t seq, n_tokens;
   const int32_t* tokens;
@@ -399,8 +401,8 @@ int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32
  * KH_PAIR_ATTN (0 = attention of a prompt slice on the fp32 matrix cores; KH_PG_ATTN_QT selects it too),
  * KH_SHAPE_DEBUG, KH_HY_DECODE (0 = single-token batches of layer-list models run on the pass kernels), KH_HY_EXPAND (0 = latent
  * attention of prompts in its absorbed form), KH_HY_TMAX (tokens of one pass, 32 ... 2048), KH_HY_ROWS (16, 64 or 128: row tiles
- * of the attention kernels of a pass), KH_HY_STEP_FAIL (the step of their generate loop reports KH_ERR_INTERNAL before its
- * first launch)) lives in ONE process-wide key -> value table, seeded once from the KH_* variables of
+ * of the attention kernels of a pass), KH_HY_TAIL (0 = the last layer of a pass for all its tokens), KH_HY_STEP_FAIL (the step of
+ * their generate loop reports KH_ERR_INTERNAL before its first launch)) lives in ONE process-wide key -> value table, seeded once from the KH_* variables of
  * the environment when the library is first used and changed afterwards only through kh_debug_set
  * (value NULL = unset).  No launch path reads the environment.  Hooks that shape a model (KH_SHAPE_*,
  * KH_ATTN_*, KH_HY_TMAX) are read by kh_model_create_*; the others by the call they affect.  Keys must start with "KH_". */
