@@ -329,16 +329,18 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs 
     for (int n = 0; n < (KEEP ? TN : 1); ++n) lost[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto fold = [&](int n, int m, int i, float f, float g) __attribute__((always_inline)) {
       const float s = __builtin_fmaf(f, g, acc[n][m][i]);
-      if (KEEP && m == TM - 1) lost[n][i] += __builtin_fmaf(f, g, acc[n][m][i] - s);
+      if constexpr (KEEP)
+        if (m == TM - 1) lost[n][i] += __builtin_fmaf(f, g, acc[n][m][i] - s);
       acc[n][m][i] = s;
     };
     // (of a sum that has overflowed, what was lost is the opposite infinity, then NaN)
     auto settle = [&]() __attribute__((always_inline)) {
-      if constexpr (!KEEP) return;
+      if constexpr (KEEP) {
 #pragma unroll
-      for (int n = 0; n < TN; ++n)
+        for (int n = 0; n < TN; ++n)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[n][TM - 1][i] += fabsf(lost[n][i]) < INFINITY ? lost[n][i] : 0.f;
+          for (int i = 0; i < 4; ++i) acc[n][TM - 1][i] += fabsf(lost[n][i]) < INFINITY ? lost[n][i] : 0.f;
+      }
     };
     auto stage = [&](int k, auto open) __attribute__((always_inline)) {
       constexpr bool OPEN = decltype(open)::value;  // fp32: first stage of a sum
