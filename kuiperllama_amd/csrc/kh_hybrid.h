@@ -15,6 +15,7 @@
 
 #include "kh_heads.h"
 #include "kh_json.h"
+#include "kh_ldheads.h"
 #include "kh_latent.h"
 #include "kh_lgemm.h"
 #include "kh_model_internal.h"
@@ -68,6 +69,7 @@ struct HyHeads {  // attention over cached keys and values, grouped heads
   float scale = 1.f;
   KeySpan span{0, 0};
   int nbias = 0, ring = 0, nsplit = 1;
+  int beside = 0;  // splits of a decoded token's attention beside the experts (kh_ldheads.h); 0: launches of its own
   bool gate = false, sink = false;
   HyMat qkvg;  // query heads, key heads, value heads, gate rows
   HyMat o;     // columns head by head, dvr each
@@ -76,6 +78,7 @@ struct HyHeads {  // attention over cached keys and values, grouped heads
   int k_off() const { return H * dkr; }
   int v_off() const { return k_off() + G * dkr; }
   int g_off() const { return v_off() + G * dvr; }
+  int chunks() const { return (H / G + 3) / 4; }  // of four query heads of a group
   HeadRow head_row(float eps) const { return {kn.p, G, dk, dv, dkr, dvr, dkp, dvp, k_off(), v_off(), ring, eps}; }
 };
 // Feed-forward: routed experts and / or one every token takes (a dense feed-forward is the latter alone)
@@ -200,8 +203,10 @@ inline HeadsArgs heads_args(const Hybrid& hy, const HyHeads& a, const void* cach
 
 // Decode steps up to position pos_hi: no attention over heads is split (step variant 0; 1 else).  The steps of generate() and
 // predict(), of one sequence, take variant 0 where they can; those of forward() always take 1, or a sequence's last bits would
-// depend on how far the others are.  A layer whose span alone bounds its keys is not split in either.
+// depend on how far the others are.  A layer whose span alone bounds its keys is not split in either; one whose attention runs
+// beside the experts knows no variants.
 inline bool hy_one_split(const Hybrid& hy, const HyHeads& a, int pos_hi) {
+  if (a.beside) return true;
   int keys = pos_hi + 1;
   if (a.span.window > 0) keys = std::min(keys, a.span.window);
   if (a.span.chunk > 0) keys = std::min(keys, a.span.chunk);

@@ -750,6 +750,7 @@ int finish(kh_model* m, Plan& pl) {
     const int keys = span > 0 ? std::min(span, CL) : CL;
     a.nsplit = 2;
     while (a.nsplit < 128 && a.nsplit * KH_LAT_SPLIT_MIN < keys && a.nsplit * a.G < 512) a.nsplit *= 2;
+    a.beside = ldh_fits(keys, a.dkp, a.dvp) && !dbg_off("KH_HY_BESIDE") ? ldh_splits(a.G * a.chunks()) : 0;
     if ((double)a.ring * a.row() * hy.elem() >= 4294967296.0) return KH_ERR_UNSUPPORTED;  // 32-bit offsets within a run
   }
   build_runs(hy);
@@ -831,6 +832,10 @@ int create_impl(const char* config, size_t config_len, const void* tensors, size
   kh_model* m = new kh_model();
   m->opts = *o;
   m->opts.family = KH_FAMILY_LAYERS;
+  {
+    const char* e = dbg("KH_ATTN_FENCED");
+    m->attn_fenced = (m->opts.flags & KH_FLAG_ATTN_MERGE_FENCED) != 0 || (e && e[0] == '1');
+  }
   m->hy = hy.release();
   *out = m;
   KH_CHECK_HIP(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));

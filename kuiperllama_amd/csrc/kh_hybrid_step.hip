@@ -15,14 +15,16 @@ namespace khm {
 struct Hybrid::Step {
   int bmax = 0;  // sequences one fused step can take (0: the geometry does not fit; everything runs as passes)
   float *x[3] = {nullptr, nullptr, nullptr}, *xn2 = nullptr, *in = nullptr, *xc = nullptr, *mid = nullptr, *v = nullptr,
-        *he = nullptr, *hs = nullptr, *z = nullptr, *id_w = nullptr, *sh_g = nullptr, *part = nullptr, *logits = nullptr;
+        *he = nullptr, *hs = nullptr, *z = nullptr, *id_w = nullptr, *sh_g = nullptr, *part = nullptr, *logits = nullptr,
+        *hpart = nullptr;
   void* Q = nullptr;
-  int32_t *ids = nullptr, *tabs = nullptr;
+  int32_t *ids = nullptr, *tabs = nullptr, *tickets = nullptr;
   int32_t* h_tabs = nullptr;
   int nsplit = 1, head_wg = 1;
   ~Step() {
     for (void* p : {(void*)x[0], (void*)x[1], (void*)x[2], (void*)xn2, (void*)in, (void*)xc, (void*)mid, (void*)v, (void*)he,
-                    (void*)hs, (void*)z, (void*)id_w, (void*)sh_g, (void*)part, (void*)logits, Q, (void*)ids, (void*)tabs})
+                    (void*)hs, (void*)z, (void*)id_w, (void*)sh_g, (void*)part, (void*)logits, Q, (void*)ids, (void*)tabs, (void*)hpart,
+                    (void*)tickets})
       if (p) (void)hipFree(p);
     if (h_tabs) (void)hipHostFree(h_tabs);
   }
@@ -226,11 +228,16 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       int extra = 0;
       if (heads) {
         extra = cdiv(B * ha.G, 4);
-        a.heads = 1;
         a.hr = ha.head_row(hy.c.eps);
         a.raw = st.in;
         a.cache = (T*)m->kcache + r.kv_off;
         a.slot_elems = hy.kv_slot;
+        if (ha.beside) {
+          const int chunks = ha.chunks();
+          a.att = {ha.qn.p, ha.bias.p, st.hpart, st.v, st.tickets, B * ha.G * chunks * ha.beside, ha.H / ha.G, chunks, ha.beside,
+                   ha.nbias, ha.sink, ha.gate ? ha.g_off() : -1, ha.o.ld, m->attn_fenced, ha.span, ha.scale * 1.44269504088896f};
+          lds = std::max(lds, kLdhLds);
+        }
       } else if (!mixed) {
         const HyMat& wm = mamba ? l.mb.x : l.la.uq;
         a.wm = wm.w;
@@ -264,14 +271,17 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       TRY(with_nv<T>(Wp, [&](auto nv) {
         return with_rp(f.top ? f.n_out() : 1, [&](auto rp) {
           constexpr int NV = decltype(nv)::value, RP = decltype(rp)::value;
-          const dim3 grid(B * a.top * a.nwg_e + a.nwg_m + extra);
-          if constexpr (B > 1)
-            if (share) return go(k_ld_mid<T, B, NV, RP, true>, grid, 256, lds, s, a);
-          return go(k_ld_mid<T, B, NV, RP, false>, grid, 256, lds, s, a);
+          const dim3 grid(a.att.nwg + B * a.top * a.nwg_e + a.nwg_m + extra);
+          if constexpr (B > 1) {
+            if (share && heads) return go(k_ld_mid<T, B, NV, RP, true, true>, grid, 256, lds, s, a);
+            if (share) return go(k_ld_mid<T, B, NV, RP, true, false>, grid, 256, lds, s, a);
+          }
+          if (heads) return go(k_ld_mid<T, B, NV, RP, false, true>, grid, 256, lds, s, a);
+          return go(k_ld_mid<T, B, NV, RP, false, false>, grid, 256, lds, s, a);
         });
       }));
     }
-    if (mixed) {
+    if (mixed || (heads && ha.beside)) {
     } else if (mamba) {
       const HyMamba& mb = l.mb;
       LdScanArgs a{st.xc, st.in, st.mid, mb.dt.w, mb.dt_b.p, mb.A2.p, mb.D.p, hy.state + r.st_off, st.v, hy.st_slot,
@@ -387,7 +397,7 @@ int hy_step_init(kh_model* m) {
   for (int B : {1, 2, 4})
     if (hy.f32 ? fits<float>(hy, B) : fits<bf16>(hy, B)) st.bmax = B;
   const size_t B = KH_HY_DECODE_B, W = (size_t)hy.c.widthp;
-  size_t in = 1, xc = 1, mid = 1, v = 1, he = 1, hs = 1, z = 1, top = 1, Q = 1, part = 1, hpart = 1;
+  size_t in = 1, xc = 1, mid = 1, v = 1, he = 1, hs = 1, z = 1, top = 1, Q = 1, part = 1, hpart = 1, units = 0, ldh = 0;
   auto up = [](size_t& a, size_t n) { a = a > n ? a : n; };
   for (auto& l : hy.layers) {
     if (l.mixer == HY_MAMBA1) {
@@ -398,7 +408,13 @@ int hy_step_init(kh_model* m) {
     } else if (l.mixer == HY_HEADS) {
       up(in, (size_t)l.ha.qkvg.N);
       up(v, (size_t)l.ha.o.ld);
-      up(hpart, (size_t)l.ha.H * (l.ha.dvp + 4) * l.ha.nsplit);
+      if (l.ha.beside) {
+        const size_t n = (size_t)l.ha.G * l.ha.chunks();
+        up(units, n);
+        up(ldh, n * l.ha.beside * 4 * kLdhPart);
+      } else {
+        up(hpart, (size_t)l.ha.H * (l.ha.dvp + 4) * l.ha.nsplit);
+      }
     } else {
       up(in, (size_t)l.la.dqkv.N);
       up(mid, (size_t)l.la.uq.N);
@@ -432,6 +448,10 @@ int hy_step_init(kh_model* m) {
   TRY(f(&st.sh_g, B));
   TRY(f(&st.part, B * std::max(part * (size_t)st.nsplit, hpart)));
   TRY(f(&st.logits, B * (size_t)hy.c.vocab));
+  if (units) {
+    TRY(f(&st.hpart, B * ldh));
+    TRY(f((float**)&st.tickets, B * units));
+  }
   TRY(f((float**)&st.Q, B * Q));
   TRY(dalloc(&st.ids, B * top));
   TRY(dalloc(&st.tabs, TB_N));
@@ -463,7 +483,7 @@ int hy_launches(const kh_model* m) {
   int n = 2;
   for (const HyRun& r : m->hy->runs) {
     const int mixer = m->hy->layers[(size_t)r.layer].mixer;
-    n += mixer == HY_MAMBA1 ? 4 : (mixer == HY_LATENT ? 6 : 5);
+    n += mixer == HY_MAMBA1 ? 4 : (mixer == HY_LATENT ? 6 : (m->hy->layers[(size_t)r.layer].ha.beside ? 3 : 5));
     if (r.pass >= 0 && m->hy->enter.N) ++n;
   }
   return n;

@@ -1,13 +1,13 @@
 // kh_ldecode.h — fused decode step of the layer-list models: B sequences (1, 2 or 4), one token each.
 //
-// Per layer   mixer mamba1: 4 launches      latent attention: 6      attention over heads: 5
+// Per layer   mixer mamba1: 4 launches      latent attention: 6      attention over heads: 3, or 5
 //   k_ld_in   norms -> LDS ; every projection that reads them: mixer input (+ bias), router (+ shared gate row), dense
 //             or shared feed-forward's gate / up ; mamba x rows go through the convolution and silu in the epilogue
 //   k_ld_mid  router choice, chosen experts' gate / up ; mamba: W_x ; latent: W_uq behind its RMS norm, cache row ;
-//             heads: cache row
+//             heads: cache row, attention (kh_ldheads.h)
 //   mamba     k_ld_scan   dt projection, softplus, one step of the selective scan, gate
 //   latent    k_ld_absorb W_uk^T q per head, rotation ; k_latent_attn (time splits) ; k_ld_values merge + W_uv per head
-//   heads     k_heads_attn (time splits) ; k_ld_merge merge and output gate
+//   heads     of more than 128 elements or over more than 4096 keys: k_heads_attn (time splits) ; k_ld_merge merge and output gate
 //   k_ld_out  W_o . v (+ bias) + experts' down + shared down + identity experts, times the residual multiplier, +
 //             residual: one dot product per row over a concatenation of weight rows
 // A loop that enters through a matrix: k_ld_enter in front of each pass.  Then k_ld_head (final norm, head, soft cap,
@@ -20,6 +20,7 @@
 #pragma once
 #include "kh_heads.h"
 #include "kh_hybrid.h"
+#include "kh_ldheads.h"
 
 namespace khm {
 
@@ -427,8 +428,9 @@ struct LdMidArgs {
   float* om;             // [B][ldo]
   int nwg_m, rows, ldm, n, n4, ldv, ldo;  // n4: float4 of a row that may be read (no norm)
   // cache rows: the last workgroups (latent attention: one per sequence; heads: one wave per key / value head)
-  int latent, heads;
+  int latent;
   HeadRow hr;
+  LdHeads att;           // attention over heads: the first workgroups
   const float* raw;      // [B][ldv]: q latent, kv latent, rotated part
   const float* kvn;
   const float2* rope;
@@ -449,7 +451,9 @@ static inline bool ld_shares(int B, int top, int n_out) {
   for (int q = 0; q < B; ++q) none *= 1.0 - p;
   return 1.0 - (1.0 - none) / (B * p) >= 1.0 / 16;
 }
-template <class T, int B, int NV, int RP, bool SHARE>
+// HEADS: the layer's mixer is attention over heads (its workgroups' registers, 151 in bf16 and 175 in fp32, would take a fourth
+// workgroup per CU from the other mixers')
+template <class T, int B, int NV, int RP, bool SHARE, bool HEADS>
 __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
   constexpr int R = 4, U = 4, SB = SHARE ? B : 1;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -459,6 +463,13 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
   __shared__ float rwt[SB][KH_MOE_MAX_TOP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int wg = blockIdx.x;
+  if constexpr (HEADS) {
+    if (wg < a.att.nwg) {  // ---- attention over heads, a chain of round trips: in front
+      ld_heads<T>(a.att, a.hr, a.raw, a.ldv, (const T*)a.cache, a.slot_elems, a.t.pos, a.t.slot, wg, smem_raw);
+      return;
+    }
+    wg -= a.att.nwg;
+  }
   LdTile<T, R, U> t;
   const T* row[R];
   const int ne = B * a.top * a.nwg_e;
@@ -609,6 +620,12 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
     return;
   }
   wg -= ne;
+  if constexpr (HEADS) {  // ---- cache rows
+    const int i = wg * 4 + wave, q = i / a.hr.G, g = i - q * a.hr.G;
+    if (q < B)
+      heads_cache_row(a.hr, a.raw + (size_t)q * a.ldv, (T*)a.cache + (size_t)a.t.slot[q] * a.slot_elems, a.t.pos[q], g, lane);
+    return;
+  }
   if (wg < a.nwg_m) {  // ---- the mixer's second projection
     const int nblk = Ld<T>::blocks(a.ldm), nch = a.ldm / Ld<T>::E, xstride = nblk * Ld<T>::BE;
     const int items = (a.rows + R - 1) / R;
@@ -658,12 +675,6 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
     return;
   }
   wg -= a.nwg_m;
-  if (a.heads) {
-    const int i = wg * 4 + wave, q = i / a.hr.G, g = i - q * a.hr.G;
-    if (q < B)
-      heads_cache_row(a.hr, a.raw + (size_t)q * a.ldv, (T*)a.cache + (size_t)a.t.slot[q] * a.slot_elems, a.t.pos[q], g, lane);
-    return;
-  }
   if (!a.latent || wg >= B) return;  // ---- cache row of sequence wg
   const float* rr = a.raw + (size_t)wg * a.ldv + a.qr;
   const int pos = a.t.pos[wg];
