@@ -70,9 +70,9 @@ int go(K kern, dim3 grid, int wg, size_t lds, hipStream_t s, A... args) {
   hipLaunchKernelGGL(kern, grid, dim3(wg), lds, s, args...);
   return KH_OK;
 }
-#define TRY(e)                    \
+#define TRY(...)                  \
   do {                            \
-    const int _rc = (e);          \
+    const int _rc = (__VA_ARGS__); \
     if (_rc != KH_OK) return _rc; \
   } while (0)
 
@@ -87,13 +87,13 @@ int launch_scan(const LdScanArgs& a, int B, hipStream_t s) {
   if (a.N <= 128) return go(k_ld_scan<T, 8>, grid, 256, 0, s, a);
   return go(k_ld_scan<T, 16>, grid, 256, 0, s, a);
 }
-// staging depth (float4 per thread) that covers a padded row of the residual stream
-template <class T, class F>
+// staging depth (float4 per thread of NT) that covers a padded row of the residual stream
+template <class T, int NT, class F>
 int with_nv(int ld, F&& f) {
   const int n = cdiv(Ld<T>::blocks(ld) * Ld<T>::BE / 4, 256);
-  if (n <= 2) return f(std::integral_constant<int, 2>());
-  if (n <= 4) return f(std::integral_constant<int, 4>());
-  return f(std::integral_constant<int, 8>());
+  if (n <= 2) return f(std::integral_constant<int, 512 / NT>());
+  if (n <= 4) return f(std::integral_constant<int, 1024 / NT>());
+  return f(std::integral_constant<int, 2048 / NT>());
 }
 template <class F>
 int with_rp(int n_out, F&& f) {
@@ -157,14 +157,19 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       if (f.top) seg(f.zr, st.z, f.zr.N, f.zr.N, LDI_PLAIN, 1);
       if (f.sff) seg(f.sgu, st.hs, f.sffp, f.sffp, LDI_GATED, 1);
       a.act = f.sact;
-      int total = 0, wg = 0;
+      // at most one workgroup per CU, each with as many items as the others: the fewest with which 256 workgroups hold them all
+      int total = 0, wg = 0, m = 1;
       auto items = [&](const LdInSeg& g) { return cdiv(g.rows, g.kind == LDI_GATED ? 2 : 4); };
       for (int i = 0; i < a.nseg; ++i) total += items(a.seg[i]);
-      const int ipw = cdiv(total, 2048);
-      for (int i = 0; i < a.nseg; ++i) {
-        a.seg[i].wg0 = wg;
-        a.seg[i].nwg = cdiv(items(a.seg[i]), 4 * ipw);
-        wg += a.seg[i].nwg;
+      m = std::max(1, cdiv(total, 256));
+      for (;; ++m) {
+        wg = 0;
+        for (int i = 0; i < a.nseg; ++i) {
+          a.seg[i].wg0 = wg;
+          a.seg[i].nwg = cdiv(items(a.seg[i]), m);
+          wg += a.seg[i].nwg;
+        }
+        if (wg <= 256) break;
       }
       a.x_in = through ? x_cur : x_in;
       a.x_cur = changed ? x_cur : nullptr;
@@ -193,7 +198,7 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.taps = l.mb.taps;
         a.xc_ld = l.mb.innerp;
       }
-      if (wg) TRY(with_nv<T>(Wp, [&](auto nv) { return go(k_ld_in<T, B, decltype(nv)::value>, dim3(wg), 256, B * vec_b<T>(Wp), s, a); }));
+      if (wg) TRY(with_nv<T, kLdNorm>(Wp, [&](auto nv) { return go(k_ld_in<T, B, decltype(nv)::value>, dim3(wg), ld_in_wg(B, decltype(nv)::value), B * vec_b<T>(Wp), s, a); }));
     }
     if (!mixed || f.top) {
       LdMidArgs a{};
@@ -268,7 +273,7 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.row = la.row();
         a.dims = la.dims;
       }
-      TRY(with_nv<T>(Wp, [&](auto nv) {
+      TRY(with_nv<T, 256>(Wp, [&](auto nv) {
         return with_rp(f.top ? f.n_out() : 1, [&](auto rp) {
           constexpr int NV = decltype(nv)::value, RP = decltype(rp)::value;
           const dim3 grid(a.att.nwg + B * a.top * a.nwg_e + a.nwg_m + extra);
@@ -358,17 +363,16 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.ffp = f.ffp;
         a.sffp = f.sffp;
       }
-      // two workgroups per CU at most: 16 waves a CU hide the latency, a second round would not (four sequences, us a step:
-      // width 1024: 535 with ks 4, 520 with 8; width 2048: 606 with 4, 616 with 8)
+      // two workgroups per CU at most: 16 waves a CU hide the latency, a second round would not
       a.ks = 1;
-      while (a.ks < 8 && cdiv(cdiv(W, 2) * a.ks * 2, 8) <= 512) a.ks *= 2;
-      TRY(go(k_ld_out<T, B>, dim3(cdiv(cdiv(W, 2) * a.ks, 8)), 512, 0, s, a));
+      while (a.ks < 8 && cdiv(cdiv(W, kLdOutRows) * a.ks * 2, 8) <= 512) a.ks *= 2;
+      TRY(go(k_ld_out<T, B>, dim3(cdiv(cdiv(W, kLdOutRows) * a.ks, 8)), 512, 0, s, a));
     }
     x_in = x_out;
   }
   LdHeadArgs h{x_in, hy.fnorm.p, hy.fnorm_b.p, hy.head.w, logits, m->part_val, m->part_idx, W, Wp, hy.c.vocab, hy.c.rms, hy.c.eps,
                hy.c.cap};
-  return with_nv<T>(Wp, [&](auto nv) { return go(k_ld_head<T, B, decltype(nv)::value>, dim3(st.head_wg), 256, B * vec_b<T>(Wp), s, h); });
+  return with_nv<T, kLdNorm>(Wp, [&](auto nv) { return go(k_ld_head<T, B, decltype(nv)::value>, dim3(st.head_wg), ld_in_wg(B, decltype(nv)::value), B * vec_b<T>(Wp), s, h); });
 }
 template <class T>
 int step_b(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail) {
@@ -458,7 +462,7 @@ int hy_step_init(kh_model* m) {
   KH_CHECK_HIP(hipHostMalloc((void**)&st.h_tabs, TB_N * 4, hipHostMallocDefault));
   memset(st.h_tabs, 0, TB_N * 4);
   KH_CHECK_HIP(hipMemcpyAsync(st.tabs, st.h_tabs, TB_N * 4, hipMemcpyHostToDevice, m->stream));
-  st.head_wg = std::min(cdiv(cdiv(hy.c.vocab, 4), 4), 1024);
+  st.head_wg = std::min(cdiv(hy.c.vocab, 4), 256);
   m->nparts = st.head_wg;
   TRY(dalloc(&m->part_val, (size_t)m->nparts));
   TRY(dalloc(&m->part_idx, (size_t)m->nparts));

@@ -60,46 +60,108 @@ __device__ __forceinline__ void ld_stage(f32x4* xs, const float* src, int n4, in
       if (i0 + j * NT < total4) xs[ld_slot<T>(i0 + j * NT)] = v[j] * g;
   }
 }
-// Layer norm (rms: RMS norm, shift 0) of Q rows (256 threads, NV float4 of a row each, rows padded with zeros to ld) into LDS
+// Sums over the wave of R B values per lane, value n = R q + r for row r and vector q.  Two values share each exchange: halves of
+// the wave, then rows of 16 lanes, then four steps within a row - 4 + 4 + 2 + 2 + 16 instructions for 16 values where a
+// sum of its own for each takes twelve times 16, on vector units that four products per weight keep busy (k_ld_in, k_ld_head).
+// The order of a value's additions does not depend on R and B.  Lane l ends with value ld_own(l).n, if it is one's owner.
+__device__ __forceinline__ float ld_fold32(float a, float b) {  // lanes 0 .. 31: of a, 32 .. 63: of b
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+}
+__device__ __forceinline__ float ld_fold16(float a, float b) {  // even rows: of a, odd rows: of b
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+  return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+}
+template <int N>
+__device__ __forceinline__ float ld_fold(const float (&v)[N], int lane) {
+  static_assert(N == 2 || N == 4 || N == 8 || N == 16 || N == 32, "values");
+  if constexpr (N == 2) {
+    return group_sum<16>(xor16_sum(ld_fold32(v[0], v[1])));
+  } else {
+    float s[N / 4], x = 0.f;
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) s[i] = group_sum<16>(ld_fold16(ld_fold32(v[4 * i], v[4 * i + 1]), ld_fold32(v[4 * i + 2], v[4 * i + 3])));
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) x = (lane & 15) == i ? s[i] : x;
+    return x;
+  }
+}
+struct LdOwn {
+  int n, r, q;
+  bool on;
+};
+template <int R, int B>
+__device__ __forceinline__ LdOwn ld_own(int lane) {
+  constexpr int N = R * B;
+  const int k = lane & 15, g = lane >> 4;
+  const int n = N == 2 ? lane >> 5 : 4 * k + ((g & 1) << 1 | g >> 1);
+  return {n, n % R, n / R, N == 2 ? (lane & 31) == 0 : k < N / 4};
+}
+template <int R, int B>
+__device__ __forceinline__ float ld_sums(const float (&acc)[R][B], int lane) {
+  float v[R * B];
+#pragma unroll
+  for (int q = 0; q < B; ++q)
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[q * R + r] = acc[r][q];
+  return ld_fold(v, lane);
+}
+// Rows 0, 1 of four are gates, rows 2, 3 their ups: an owner of row r < 2 gets the other's value in u (and its own in g).
+__device__ __forceinline__ void ld_gate_up(float v, float& g, float& u) { KH_SWAP16(v, g, u); }
+
+// Layer norm (rms: RMS norm, shift 0) of Q rows (NT threads, NV float4 of a row each, rows padded with zeros to ld) into LDS
 // slots, rows xstride4 slots apart.  v: the rows in registers; the normalised values also go to `out` (ldo4 apart) when given.
 // Mean and variance come from ONE workgroup reduction of (x - shift) and (x - shift)^2 for all rows, shift = an element of the
-// row: no cancellation beyond the distance of that element from the mean.  red: 8 Q floats.
-template <class T, int NV, int Q>
+// row: no cancellation beyond the distance of that element from the mean.  Every wave finishes the statistics for itself, those of
+// all rows at once in its lanes.  red: 64 floats.  Waves behind the first NT threads only meet the barrier.
+template <class T, int NT, int NV, int Q>
 __device__ __forceinline__ void ld_norm(const f32x4 (&v)[Q][NV], const f32x4 (&w)[NV], const f32x4 (&b)[NV], const float (&shift)[Q],
                                         bool rms, int W, int n4, int total4, float eps, float* red, f32x4* xs, int xstride4,
                                         f32x4* out, int ldo4) {
-  const int wave = threadIdx.x >> 6;
+  static_assert(NT == 512 && Q <= 4, "eight waves of eight values are the lanes of one");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (wave >= NT / 64) {  // uniform
+    __syncthreads();
+    return;
+  }
+  float s[2 * Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    float s1 = 0.f, s2 = 0.f;
+    s[2 * q] = s[2 * q + 1] = 0.f;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int i = threadIdx.x + 256 * j;
+      const int i = threadIdx.x + NT * j;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const float d = 4 * i + k < W ? v[q][j][k] - shift[q] : 0.f;
-        s1 += d;
-        s2 = __builtin_fmaf(d, d, s2);
+        s[2 * q] += d;
+        s[2 * q + 1] = __builtin_fmaf(d, d, s[2 * q + 1]);
       }
     }
-    s1 = wave_sum(s1);
-    s2 = wave_sum(s2);
-    if ((threadIdx.x & 63) == 0) {
-      red[8 * q + wave] = s1;
-      red[8 * q + 4 + wave] = s2;
-    }
+  }
+  {
+    const float x = ld_fold(s, lane);
+    const LdOwn o = ld_own<2, Q>(lane);
+    if (o.on) red[8 * wave + o.n] = x;
   }
   __syncthreads();
+  const int c = lane & 7;  // value c = 2 q (+ 1) of wave lane / 8
+  float x = c < 2 * Q ? red[lane] : 0.f;
+  x += __shfl_xor(x, 8, 64);
+  x = xor32_sum(xor16_sum(x));
+  const float y = dpp_f32<KH_DPP_XOR1>(x), s1 = c & 1 ? y : x, s2 = c & 1 ? x : y;
+  const float m = rms ? 0.f : s1 / (float)W;
+  const float var = fmaxf(s2 / (float)W - m * m, 0.f);
+  const float rs = 1.0f / sqrtf(var + eps);
+  auto of_row = [&](float z, int q) __attribute__((always_inline)) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, z), 2 * q));
+  };
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    const float* r = red + 8 * q;
-    const float s1 = (r[0] + r[1]) + (r[2] + r[3]), s2 = (r[4] + r[5]) + (r[6] + r[7]);
-    const float m = rms ? 0.f : s1 / (float)W, mean = rms ? 0.f : shift[q] + m;
-    const float var = fmaxf(s2 / (float)W - m * m, 0.f);
-    const float rstd = 1.0f / sqrtf(var + eps);
+    const float mean = rms ? 0.f : shift[q] + of_row(m, q), rstd = of_row(rs, q);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int i = threadIdx.x + 256 * j;
+      const int i = threadIdx.x + NT * j;
       f32x4 y;
 #pragma unroll
       for (int k = 0; k < 4; ++k) y[k] = (v[q][j][k] - mean) * rstd * w[j][k] + b[j][k];  // pads: zero weight and bias
@@ -109,9 +171,8 @@ __device__ __forceinline__ void ld_norm(const f32x4 (&v)[Q][NV], const f32x4 (&w
   }
 }
 // The rows of how many of B sequences are requested at once and normed behind one reduction: all, where the registers hold them.
-// (One after the other they are a load and a reduction each: k_ld_in of four sequences of 2048 21.9 -> 20.6 us in front of a
-// mamba mixer, 14.8 -> 13.7 of latent attention.)
-constexpr int ld_rows_at_once(int B, int NV) { return B * NV <= 16 ? B : 1; }
+// (One after the other they are a load and a reduction each.)
+constexpr int ld_rows_at_once(int B, int NV) { return B * NV <= 8 ? B : 1; }
 
 template <class T, int R, int U>
 struct LdTile {
@@ -167,22 +228,43 @@ __device__ __forceinline__ void ld_rows(LdTile<T, R, U>& t, const T* const (&row
     ld_fma<T, R, U, B>(t, xs, xstride, b0, nblk, lane, acc);
   }
 }
-template <int R, int B>
-__device__ __forceinline__ void ld_reduce(float (&acc)[R][B]) {
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int q = 0; q < B; ++q) acc[r][q] = wave_sum(acc[r][q]);
+// A wave's items, `step` apart.  A tile is requested again as soon as its products are done; sixteen waves a CU keep requests in
+// flight meanwhile.  set_rows(item, row) gives an item's rows, early(item) requests what done(item, sum) needs beside the sums
+// (ld_sums).  ld_items_begin requests the first tile and may come long before.
+template <class T, int R, int U, class S>
+__device__ __forceinline__ void ld_items_begin(LdTile<T, R, U>& t, int item, int items, int nblk, int nch, int lane, S&& set_rows) {
+  if (item >= items) return;
+  const T* row[R];
+  set_rows(item, row);
+  ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
 }
-// value (r, q) picked by a lane-dependent index without dynamic register indexing
-template <int R, int B>
-__device__ __forceinline__ float ld_pick(const float (&acc)[R][B], int r, int q) {
-  float v = 0.f;
+template <int B, class T, int R, int U, class S, class E, class D>
+__device__ __forceinline__ void ld_items(LdTile<T, R, U>& t, int item, int step, int items, int nblk, int nch, const float* xs, int xstride,
+                                         int lane, S&& set_rows, E&& early, D&& done) {
+  if (item >= items) return;
+  float acc[R][B] = {};
+  int b = 0;
+  early(item);
+  for (;;) {
+    ld_fma<T, R, U, B>(t, xs, xstride, b, nblk, lane, acc);
+    const bool last = b + U >= nblk;
+    const int it2 = last ? item + step : item;
+    b = last ? 0 : b + U;
+    if (it2 < items) {
+      const T* row[R];
+      set_rows(it2, row);
+      ld_load<T, R, U>(t, row, b, nblk, nch, lane);
+    }
+    if (!last) continue;
+    done(item, ld_sums(acc, lane));
+    if (it2 >= items) return;
+    item = it2;
+    early(item);
 #pragma unroll
-  for (int i = 0; i < R; ++i)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int j = 0; j < B; ++j) v = (i == r && j == q) ? acc[i][j] : v;
-  return v;
+      for (int q = 0; q < B; ++q) acc[r][q] = 0.f;
+  }
 }
 
 struct LdTabs {
@@ -231,13 +313,27 @@ struct LdInArgs {
   int inner, taps, xc_ld;
 };
 
+// k_ld_in and k_ld_head: one workgroup of sixteen waves per CU, which stages the rows once.  The first eight request the rows and
+// norm them, the others meanwhile weights: a wave that has requested more than the memory pipe takes (32 KB a CU are in
+// flight) is held up where it is, and the norm was done 5 ... 10 us into the launch where every wave asked for weights first.
+// As workgroups of four waves, up to four per CU and one CU with twice the items of another (us, before / now): k_ld_in of 2048
+// columns in bf16, four sequences, 50 and 26 MB 20.8 / 16.3 and 13.9 / 11.5; in fp32, one sequence, 100 and 51 MB 21.9 / 19.1 and
+// 17.5 / 11.9; 1024 columns, 10 and 6 MB 6.5 / 5.3 and 5.8 / 4.7.  k_ld_head, 131 MB: four sequences 35.2 / 28.6 (one
+// in fp32, 262 MB: 42.8 / 44.4).
+// (Four rows of more than 4096 columns, NV = 4: eight waves; sixteen would have too few registers.)
+constexpr int kLdNorm = 512;
+constexpr int ld_in_wg(int B, int NV) { return B * NV >= 16 ? kLdNorm : 1024; }
+// blocks of a tile: 128 registers a wave hold them beside the rows (more than 4096 columns: NV = 4).  One vector: all of a row of
+// 2048 at once, a launch of two items a CU is one round trip (k_ld_in of 1024 columns in fp32, 6 and 10 MB: 6.9 and 7.2 us with
+// two, 4.7 and 5.3 with four).
+constexpr int ld_in_tile(int B, int NV) { return B == 1 && NV < 4 ? 4 : 2; }
 template <class T, int B, int NV>
-__global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
-  constexpr int R = 4, U = 4;
+__global__ __launch_bounds__(ld_in_wg(B, NV)) void k_ld_in(const LdInArgs a) {
+  constexpr int R = 4, U = ld_in_tile(B, NV), NT = kLdNorm, NW = ld_in_wg(B, NV) / 64;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float* xs = (float*)smem_raw;
-  __shared__ float red[8 * B];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wg = blockIdx.x;
+  __shared__ float red[64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wg = blockIdx.x;
   int si = 0;
   if (a.nseg > 1 && wg >= a.seg[1].wg0) si = 1;
   if (a.nseg > 2 && wg >= a.seg[2].wg0) si = 2;
@@ -254,9 +350,10 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
   const int nblk = Ld<T>::blocks(a.ld), nch = a.ld / Ld<T>::E;
   const int per = kind == LDI_GATED ? R / 2 : R;  // outputs per item
   const int items = (rows + per - 1) / per;
-  int item = (wg - wg0) * 4 + wave;
-  const T* row[R];
-  auto set_rows = [&](int it) __attribute__((always_inline)) {
+  // dealt over the workgroups in turn: every CU draws the same number of them, give or take one; first those of the waves that
+  // do not norm
+  const int item = ((wave + NW / 2) % NW) * nwg + (wg - wg0), step = NW * nwg;
+  auto set_rows = [&](int it, const T* (&row)[R]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       int i;
@@ -271,11 +368,6 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
       row[r] = w + (size_t)i * a.ld;
     }
   };
-  LdTile<T, R, U> t;  // (rows of more than 4096 columns first: the other way takes 322 registers)
-  if (NV < 8 && item < items) {
-    set_rows(item);
-    ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
-  }
   // ---- the rows
   constexpr int Q = ld_rows_at_once(B, NV);
   const int xstride = nblk * Ld<T>::BE, n4 = a.ld >> 2, total4 = xstride >> 2;
@@ -284,7 +376,7 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
   auto get = [&](int q, f32x4 (&x)[NV], float& sh) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int i = threadIdx.x + 256 * j;
+      const int i = threadIdx.x + NT * j;
       x[j] = f4_zero();
       if (i < n4) {
         x[j] = a.from_embed ? ld_embed<T>(a.emb, a.t.tok[q], a.t.pos[q], a.ld, i) : ((const f32x4*)(a.x_in + (size_t)q * a.ld))[i];
@@ -295,119 +387,115 @@ __global__ __launch_bounds__(256) void k_ld_in(const LdInArgs a) {
     sh = 0.f;
     if (!a.rms) sh = a.from_embed ? (float)((const T*)a.emb.embed)[(size_t)a.t.tok[q] * a.ld] : a.x_in[(size_t)q * a.ld];
   };
-#pragma unroll
-  for (int q = 0; q < Q; ++q) get(q, v[q], shift[q]);
-  {
+  auto weights = [&]() __attribute__((always_inline)) {
     const f32x4 *wp = (const f32x4*)(norm2 ? a.w2 : a.w1), *bp = (const f32x4*)(norm2 ? a.b2 : a.b1);
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int i = threadIdx.x + 256 * j;
+      const int i = threadIdx.x + NT * j;
       nw[j] = i < n4 ? wp[i] : f4_zero();
       nb[j] = bp && i < n4 ? bp[i] : f4_zero();
     }
-  }
-  if (NV == 8 && item < items) {
-    set_rows(item);
-    ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
-  }
-  // convolution operands of the wave's first item: requested with its weights (up to four taps)
-  constexpr int CT = 4;
-  float cw[CT], cs[CT];
-  float cb = 0.f;
-  const bool conv_pre = kind == LDI_CONV && a.taps <= CT;
-  if (conv_pre && item < items && lane < R * B) {
-    const int c = item * R + (lane & (R - 1)), q = lane / R;
-    if (c < a.inner) {
-      const float* st = a.conv_st + (size_t)a.t.slot[q] * a.slot_stride + c;
-      const bool fresh = a.t.pos[q] == 0;
-      cb = a.conv_b[c];
+  };
+  const bool norms = wave < NT / 64;
+  if (norms && Q == B) {
 #pragma unroll
-      for (int k = 0; k < CT; ++k) {
-        cw[k] = k < a.taps ? a.conv_w[(size_t)c * a.taps + k] : 0.f;
-        cs[k] = k + 1 < a.taps && !fresh ? st[(size_t)k * a.inner] : 0.f;
-      }
-    }
+    for (int q = 0; q < Q; ++q) get(q, v[q], shift[q]);
+    weights();
   }
-  const int first_item = item;
+  LdTile<T, R, U> t;
+  if (!norms) ld_items_begin(t, item, items, nblk, nch, lane, set_rows);
   // ---- layer norm of B rows
+#pragma unroll 1
   for (int q0 = 0; q0 < B; q0 += Q) {
-    if (q0) {
-      get(q0, v[0], shift[0]);  // Q = 1
-      __syncthreads();          // red is free again
+    if (Q < B) {
+      if (norms) {
+        get(q0, v[0], shift[0]);  // Q = 1
+        __builtin_amdgcn_sched_barrier(0);
+        weights();  // behind what get() adds up: the registers do not hold both
+      }
+      if (q0) __syncthreads();  // red is free again
     }
-    if (a.x_cur && wg == 0) {
+    if (a.x_cur && wg == 0 && norms) {
 #pragma unroll
       for (int q = 0; q < Q; ++q)
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-          if ((int)threadIdx.x + 256 * j < n4) ((f32x4*)(a.x_cur + (size_t)(q0 + q) * a.ld))[threadIdx.x + 256 * j] = v[q][j];
+          if ((int)threadIdx.x + NT * j < n4) ((f32x4*)(a.x_cur + (size_t)(q0 + q) * a.ld))[threadIdx.x + NT * j] = v[q][j];
     }
     // the router's first workgroup leaves the second norm for the launches that follow
     f32x4* keep = a.xn2 && wg == a.xn2_wg ? (f32x4*)(a.xn2 + (size_t)q0 * a.ld) : nullptr;
-    ld_norm<T, NV, Q>(v, nw, nb, shift, a.rms, a.W, n4, total4, a.eps, red, (f32x4*)(xs + (size_t)q0 * xstride), total4, keep, n4);
+    int W = a.W, m4 = n4, t4 = total4;
+    if (Q < B) asm volatile("" : "+s"(W), "+s"(m4), "+s"(t4));  // or the lane masks of all pieces are kept over the rows: scratch
+    ld_norm<T, NT, NV, Q>(v, nw, nb, shift, a.rms, W, m4, t4, a.eps, red, (f32x4*)(xs + (size_t)q0 * xstride), total4, keep, n4);
   }
+  if (norms) ld_items_begin(t, item, items, nblk, nch, lane, set_rows);
   __syncthreads();
-  while (item < items) {
-    float acc[R][B] = {};
-    float bi = 0.f;
-    if (bias && lane < R * B) {
-      const int i = item * R + (lane & (R - 1));
-      bi = bias[i < rows ? i : rows - 1];
-    }
-    ld_rows<T, R, U, B>(t, row, nblk, nch, xs, xstride, lane, acc);
-    const int cur = item;
-    item += nwg * 4;
-    if (item < items) {  // the next row set travels while this one is reduced
-      set_rows(item);
-      ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
-    }
-    ld_reduce<R, B>(acc);
-    if (lane < R * B) {
-      const int r = lane & (R - 1), q = lane / R;
-      if (kind == LDI_GATED) {
-        const int j = cur * 2 + r;
-        if (r < 2 && j < rows) {
-          const float g = ld_pick<R, B>(acc, r, q), u = ld_pick<R, B>(acc, r + 2, q);
-          out[(size_t)q * ldo + j] = gated1(a.act, g, u);
-        }
-      } else {
-        const int i = cur * R + r;
-        const float v = ld_pick<R, B>(acc, r, q);
-        if (i < rows) {
-          if (kind == LDI_CONV && i < a.inner) {
-            float* st = a.conv_st + (size_t)a.t.slot[q] * a.slot_stride + i;
-            float c;
-            if (conv_pre && cur == first_item) {
-              c = cb;
+  // the owner of sum (r, q) finishes output r of sequence q: operands of a convolution of up to CT taps are requested early
+  constexpr int CT = 4;
+  const LdOwn own = ld_own<R, B>(lane);
+  const int lr = own.r, lq = own.q;
+  const bool conv_pre = kind == LDI_CONV && a.taps <= CT;
+  float cw[CT], cs[CT], cb = 0.f, bi = 0.f;
+  bool fresh = false;
+  float* st0 = nullptr;
+  if (kind == LDI_CONV && own.on) {
+    fresh = a.t.pos[lq] == 0;
+    st0 = a.conv_st + (size_t)a.t.slot[lq] * a.slot_stride;
+  }
+  auto early = [&](int it) __attribute__((always_inline)) {
+    if (!own.on) return;
+    const int i = it * R + lr;
+    if (bias) bi = bias[i < rows ? i : rows - 1];
+    if (conv_pre && i < a.inner) {
+      cb = a.conv_b[i];
 #pragma unroll
-              for (int k = 0; k < CT; ++k) {
-                if (k + 1 < a.taps) {
-                  c = __builtin_fmaf(cw[k], cs[k], c);
-                  if (k) st[(size_t)(k - 1) * a.inner] = cs[k];
-                } else if (k + 1 == a.taps) {
-                  c = __builtin_fmaf(cw[k], v, c);
-                }
-              }
-            } else {
-              const bool fresh = a.t.pos[q] == 0;
-              const float* w1 = a.conv_w + (size_t)i * a.taps;
-              c = a.conv_b[i];
-              for (int k = 0; k + 1 < a.taps; ++k) {
-                const float in = fresh ? 0.f : st[(size_t)k * a.inner];
-                c = __builtin_fmaf(w1[k], in, c);
-                if (k) st[(size_t)(k - 1) * a.inner] = in;
-              }
-              c = __builtin_fmaf(w1[a.taps - 1], v, c);
-            }
-            if (a.taps > 1) st[(size_t)(a.taps - 2) * a.inner] = v;
-            a.xc[(size_t)q * a.xc_ld + i] = silu1(c);
-          } else {
-            out[(size_t)q * ldo + i] = v + bi;
-          }
-        }
+      for (int k = 0; k < CT; ++k) {
+        cw[k] = k < a.taps ? a.conv_w[(size_t)i * a.taps + k] : 0.f;
+        cs[k] = k + 1 < a.taps && !fresh ? st0[(size_t)k * a.inner + i] : 0.f;
       }
     }
-  }
+  };
+  auto done = [&](int it, float v) __attribute__((always_inline)) {
+    if (kind == LDI_GATED) {
+      float g, u;
+      ld_gate_up(v, g, u);
+      const int j = it * 2 + lr;
+      if (own.on && lr < 2 && j < rows) out[(size_t)lq * ldo + j] = gated1(a.act, g, u);
+      return;
+    }
+    const int i = it * R + lr;
+    if (!own.on || i >= rows) return;
+    if (kind != LDI_CONV || i >= a.inner) {
+      out[(size_t)lq * ldo + i] = v + bi;
+      return;
+    }
+    float* st = st0 + i;
+    float c;
+    if (conv_pre) {
+      c = cb;
+#pragma unroll
+      for (int k = 0; k < CT; ++k) {
+        if (k + 1 < a.taps) {
+          c = __builtin_fmaf(cw[k], cs[k], c);
+          if (k) st[(size_t)(k - 1) * a.inner] = cs[k];
+        } else if (k + 1 == a.taps) {
+          c = __builtin_fmaf(cw[k], v, c);
+        }
+      }
+    } else {
+      const float* w1 = a.conv_w + (size_t)i * a.taps;
+      c = a.conv_b[i];
+      for (int k = 0; k + 1 < a.taps; ++k) {
+        const float in = fresh ? 0.f : st[(size_t)k * a.inner];
+        c = __builtin_fmaf(w1[k], in, c);
+        if (k) st[(size_t)(k - 1) * a.inner] = in;
+      }
+      c = __builtin_fmaf(w1[a.taps - 1], v, c);
+    }
+    if (a.taps > 1) st[(size_t)(a.taps - 2) * a.inner] = v;
+    a.xc[(size_t)lq * a.xc_ld + i] = silu1(c);
+  };
+  ld_items<B>(t, item, step, items, nblk, nch, xs, xstride, lane, set_rows, early, done);
 }
 
 // ---- k_ld_mid ----------------------------------------------------------------------------------------------------
@@ -454,8 +542,8 @@ static inline bool ld_shares(int B, int top, int n_out) {
 // HEADS: the layer's mixer is attention over heads (its workgroups' registers, 151 in bf16 and 175 in fp32, would take a fourth
 // workgroup per CU from the other mixers')
 template <class T, int B, int NV, int RP, bool SHARE, bool HEADS>
-__global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
-  constexpr int R = 4, U = 4, SB = SHARE ? B : 1;
+__global__ __launch_bounds__(256, B > 1 && sizeof(T) == 2 ? 3 : 1) void k_ld_mid(const LdMidArgs a) {
+  constexpr int R = 4, U = B > 1 ? 2 : 4, SB = SHARE ? B : 1;  // (three blocks spill, and so do four workgroups per CU: 35 and 40 us for 30.5)
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float* xs = (float*)smem_raw;
   __shared__ float red[KH_WAVES_MAX];
@@ -486,8 +574,9 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
     // Every wave makes the choice for itself: its weight loads leave without a barrier.  SHARE: the waves make one sequence's
     // each, and an expert that several chose is read once, by the first of them.  Bound by the bytes of the experts (2048 x
     // 1024 in bf16, four sequences, 6 of 32 and 4 identities each: 21 choices of 17 experts): 39.4 -> 35.5 us in front of latent
-    // attention, 31.6 -> 28.3 of mamba.  k_ld_out does not do so: there a sequence's sum would be taken in an order that depends
-    // on what the others chose (26.3 -> 24.6 us).
+    // attention, 31.6 -> 28.3 of mamba; with tiles of two blocks, three workgroups per CU instead of two and no second round of
+    // them, 30.5 and 26.4.  k_ld_out does not do so: there a sequence's sum would be taken in an order that depends on what the
+    // others chose.
     float idw = 0.f, w = 0.f;
     int id = -1;
     unsigned mates = 0;  // byte q: 1 + the place where later sequence q chose the same expert
@@ -604,13 +693,18 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
           set_rows(it);
           ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
         }
-        ld_reduce<R, N>(acc);
-        if (lane < 2) {
+        float g, u;
+        ld_gate_up(ld_sums(acc, lane), g, u);
+        const LdOwn own = ld_own<R, N>(lane);
+        if (own.on && own.r < 2 && own.q < n) {
+          int d = dst[0];
+          float wt = wj[0];
 #pragma unroll
-          for (int j = 0; j < N; ++j) {
-            const float g = ld_pick<R, N>(acc, lane, j), u = ld_pick<R, N>(acc, lane + 2, j);
-            if (j < n) a.he[(size_t)dst[j] * a.ffp + cur * 2 + lane] = wj[j] * gated1(a.act, g, u);
+          for (int j = 1; j < N; ++j) {
+            d = own.q == j ? dst[j] : d;
+            wt = own.q == j ? wj[j] : wt;
           }
+          a.he[(size_t)d * a.ffp + cur * 2 + own.r] = wt * gated1(a.act, g, u);
         }
       }
     };
@@ -665,12 +759,10 @@ __global__ __launch_bounds__(256) void k_ld_mid(const LdMidArgs a) {
         set_rows(item);
         ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
       }
-      ld_reduce<R, B>(acc);
-      if (lane < R * B) {
-        const int r = lane & (R - 1), q = lane / R, i = cur * R + r;
-        const float v = ld_pick<R, B>(acc, r, q);
-        if (i < a.rows) a.om[(size_t)q * a.ldo + i] = v;
-      }
+      const float v = ld_sums(acc, lane);
+      const LdOwn own = ld_own<R, B>(lane);
+      const int i = cur * R + own.r;
+      if (own.on && i < a.rows) a.om[(size_t)own.q * a.ldo + i] = v;
     }
     return;
   }
@@ -883,8 +975,9 @@ __global__ __launch_bounds__(256) void k_ld_values(const LdValuesArgs a) {
       set_rows(item);
       ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
     }
-    ld_reduce<R, 1>(acc);
-    if (lane < R) a.o[((size_t)b * a.H + h) * a.dvp + cur * R + lane] = ld_pick<R, 1>(acc, lane, 0);
+    const float v = ld_sums(acc, lane);
+    const LdOwn own = ld_own<R, 1>(lane);
+    if (own.on) a.o[((size_t)b * a.H + h) * a.dvp + cur * R + own.r] = v;
   }
 }
 
@@ -957,8 +1050,11 @@ __global__ __launch_bounds__(512) void k_ld_enter(const LdEnterArgs a) {
     if (b != b0) ld_load<T, R, U>(t, row, b, b1, nch, lane);
     ld_fma<T, R, U, B>(t, xs, nblk * BE, b, b1, lane, acc);
   }
-  ld_reduce<R, B>(acc);
-  if (lane < R * B) comb[wave][lane] = ld_pick<R, B>(acc, lane & (R - 1), lane / R);
+  {
+    const float v = ld_sums(acc, lane);
+    const LdOwn own = ld_own<R, B>(lane);
+    if (own.on) comb[wave][own.n] = v;
+  }
   __syncthreads();
   if (kp == 0 && lane < R * B) {
     float v = 0.f;
@@ -986,10 +1082,13 @@ struct LdOutArgs {
 // from the caches as they are needed, lanes behind a row's end repeat its last chunk against zeros: no LDS but the final sum,
 // no barrier before it, and 16 waves a CU run freely.  Bound by latency: with the vectors staged in LDS, four sequences of
 // 2048 columns took 96 KB (8 waves a CU, two rounds of workgroups) and a load, a staging and two barriers per sequence:
-// 44.9 -> 26.3 us a layer at four (bf16, 105 ... 139 MB of weights), 8.0 -> 6.1 at one of 1024 (fp32).
+// 44.9 -> 26.3 us a layer at four (bf16, 105 ... 139 MB of weights), 8.0 -> 6.1 at one of 1024 (fp32).  Four rows a wave: with
+// two, the vectors were half of what a CU draws through its L1 (31 ... 40 bytes a ns): 26.2 -> 20.9 us at four sequences, 15.7 ->
+// 13.9 at two, 9.7 -> 8.8 at four of 1024, 5.96 -> 5.62 at one of 1024 in fp32; with eight, the waves are too few: 22.6, 13.3, 12.0.
+constexpr int kLdOutRows = 4;
 template <class T, int B>
 __global__ __launch_bounds__(512, 4) void k_ld_out(const LdOutArgs a) {
-  constexpr int R = 2, U = 4;
+  constexpr int R = kLdOutRows, U = 2;
   typedef typename Tile<T>::frag frag;
   constexpr int E = Ld<T>::E, P = Ld<T>::P;
   __shared__ float comb[8][R * B];
@@ -1090,8 +1189,11 @@ __global__ __launch_bounds__(512, 4) void k_ld_out(const LdOutArgs a) {
         }
       }
   }
-  ld_reduce<R, B>(acc);
-  if (lane < R * B) comb[wave][lane] = ld_pick<R, B>(acc, lane & (R - 1), lane / R);
+  {
+    const float v = ld_sums(acc, lane);
+    const LdOwn own = ld_own<R, B>(lane);
+    if (own.on) comb[wave][own.n] = v;
+  }
   __syncthreads();
   if (kp == 0 && lane < R * B) {
     float v = 0.f;
@@ -1113,20 +1215,18 @@ struct LdHeadArgs {
   float eps, cap;
 };
 template <class T, int B, int NV>
-__global__ __launch_bounds__(256) void k_ld_head(const LdHeadArgs a) {
-  constexpr int R = 4, U = 4;
+__global__ __launch_bounds__(ld_in_wg(B, NV)) void k_ld_head(const LdHeadArgs a) {
+  constexpr int R = 4, U = ld_in_tile(B, NV), NT = kLdNorm, NW = ld_in_wg(B, NV) / 64;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   float* xs = (float*)smem_raw;
-  __shared__ float red[8 * B];
-  __shared__ float sv[4];
-  __shared__ int si[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ float red[64];
+  __shared__ float sv[NW];
+  __shared__ int si[NW];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nblk = Ld<T>::blocks(a.ld), nch = a.ld / Ld<T>::E, xstride = nblk * Ld<T>::BE;
   const int items = (a.V + R - 1) / R;
-  int item = blockIdx.x * 4 + wave;
-  const T* row[R];
-  LdTile<T, R, U> t;
-  auto set_rows = [&](int it) __attribute__((always_inline)) {
+  const int item = ((wave + NW / 2) % NW) * (int)gridDim.x + (int)blockIdx.x, step = NW * (int)gridDim.x;  // as in k_ld_in
+  auto set_rows = [&](int it, const T* (&row)[R]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       int i = it * R + r;
@@ -1136,60 +1236,54 @@ __global__ __launch_bounds__(256) void k_ld_head(const LdHeadArgs a) {
   };
   constexpr int Q = ld_rows_at_once(B, NV);
   const int n4 = a.ld >> 2;
-  f32x4 nw[NV], nb[NV], v[Q][NV];  // in front of the weights: 35.4 -> 32.6 us for four rows of 2048 (in k_ld_in one row alone loses)
+  f32x4 nw[NV], nb[NV], v[Q][NV];
   float shift[Q];
   auto get = [&](int q, f32x4 (&x)[NV], float& sh) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int i = threadIdx.x + 256 * j;
+      const int i = threadIdx.x + NT * j;
       x[j] = i < n4 ? ((const f32x4*)(a.x + (size_t)q * a.ld))[i] : f4_zero();
     }
     sh = a.rms ? 0.f : a.x[(size_t)q * a.ld];
   };
+  const bool norms = wave < NT / 64;
+  if (norms) {
+    if (Q == B) {
 #pragma unroll
-  for (int q = 0; q < Q; ++q) get(q, v[q], shift[q]);
-#pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    const int i = threadIdx.x + 256 * j;
-    nw[j] = i < n4 ? ((const f32x4*)a.w)[i] : f4_zero();
-    nb[j] = a.b && i < n4 ? ((const f32x4*)a.b)[i] : f4_zero();
-  }
-  if (item < items) {
-    set_rows(item);
-    ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
-  }
-  for (int q0 = 0; q0 < B; q0 += Q) {
-    if (q0) {
-      get(q0, v[0], shift[0]);  // Q = 1
-      __syncthreads();          // red is free again
+      for (int q = 0; q < Q; ++q) get(q, v[q], shift[q]);
     }
-    int W = a.W, m4 = n4, total4 = xstride >> 2;
-    if (Q < B) asm volatile("" : "+s"(W), "+s"(m4), "+s"(total4));  // or the lane masks of all pieces are kept over the rows: scratch
-    ld_norm<T, NV, Q>(v, nw, nb, shift, a.rms, W, m4, total4, a.eps, red, (f32x4*)(xs + (size_t)q0 * xstride), xstride >> 2, nullptr, 0);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int i = threadIdx.x + NT * j;
+      nw[j] = i < n4 ? ((const f32x4*)a.w)[i] : f4_zero();
+      nb[j] = a.b && i < n4 ? ((const f32x4*)a.b)[i] : f4_zero();
+    }
   }
+  LdTile<T, R, U> t;
+  if (!norms) ld_items_begin(t, item, items, nblk, nch, lane, set_rows);
+#pragma unroll 1
+  for (int q0 = 0; q0 < B; q0 += Q) {
+    if (Q < B) {
+      if (norms) get(q0, v[0], shift[0]);  // Q = 1
+      if (q0) __syncthreads();             // red is free again
+    }
+    ld_norm<T, NT, NV, Q>(v, nw, nb, shift, a.rms, a.W, n4, xstride >> 2, a.eps, red, (f32x4*)(xs + (size_t)q0 * xstride), xstride >> 2,
+                          nullptr, 0);
+  }
+  if (norms) ld_items_begin(t, item, items, nblk, nch, lane, set_rows);
   __syncthreads();
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  while (item < items) {
-    float acc[R][B] = {};
-    ld_rows<T, R, U, B>(t, row, nblk, nch, xs, xstride, lane, acc);
-    const int cur = item;
-    item += gridDim.x * 4;
-    if (item < items) {
-      set_rows(item);
-      ld_load<T, R, U>(t, row, 0, nblk, nch, lane);
+  const LdOwn own = ld_own<R, B>(lane);
+  ld_items<B>(t, item, step, items, nblk, nch, xs, xstride, lane, set_rows, [](int) {}, [&](int it, float v) __attribute__((always_inline)) {
+    if (!own.on) return;
+    const int i = it * R + own.r;
+    if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
+    if (i < a.V) {
+      a.logits[(size_t)own.q * a.V + i] = v;
+      if (own.q == 0) amax_merge(bv, bi, v, i);
     }
-    ld_reduce<R, B>(acc);
-    if (lane < R * B) {
-      const int r = lane & (R - 1), q = lane / R, i = cur * R + r;
-      float v = ld_pick<R, B>(acc, r, q);
-      if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
-      if (i < a.V) {
-        a.logits[(size_t)q * a.V + i] = v;
-        if (q == 0) amax_merge(bv, bi, v, i);
-      }
-    }
-  }
+  });
   if (a.part_val) {
     wave_amax(bv, bi);
     if (lane == 0) {
@@ -1199,7 +1293,7 @@ __global__ __launch_bounds__(256) void k_ld_head(const LdHeadArgs a) {
     __syncthreads();
     if (threadIdx.x == 0) {
 #pragma unroll
-      for (int w = 1; w < 4; ++w) amax_merge(bv, bi, sv[w], si[w]);
+      for (int w = 1; w < NW; ++w) amax_merge(bv, bi, sv[w], si[w]);
       a.part_val[blockIdx.x] = bv;
       a.part_idx[blockIdx.x] = bi;
     }

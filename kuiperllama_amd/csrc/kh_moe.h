@@ -51,21 +51,22 @@ __device__ __forceinline__ float moe_route(const float* z, const float* corr, in
 #pragma unroll
     for (int j = 1; j < PER; ++j) v = fmaxf(v, key[j]);
     v = wave_max(v);
-    // lowest index that holds the maximum (indices are exact in fp32)
-    float first = 1e9f;
-#pragma unroll
-    for (int j = PER - 1; j >= 0; --j) first = key[j] == v ? (float)(j * 64 + lane) : first;
-    const int id = (int)(-wave_max(-first));
+    // the lowest index that holds the maximum, and its weight, without a second and a third reduction
+    int id = 1 << 30;  // nobody's (a NaN): an identity expert of no weight
     float w = 0.f;
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const bool mine = j * 64 + lane == id;
-      w = mine ? s[j] : w;
-      key[j] = mine ? -INFINITY : key[j];
+    for (int j = PER - 1; j >= 0; --j) {
+      const unsigned long long has = __builtin_amdgcn_ballot_w64(key[j] == v);
+      if (has) {
+        const int at = __builtin_ctzll(has);
+        id = j * 64 + at;
+        w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[j]), at));
+      }
     }
-    w = wave_sum(w);  // one lane holds it, the others zero
+#pragma unroll
+    for (int j = 0; j < PER; ++j) key[j] = j * 64 + lane == id ? -INFINITY : key[j];
     chosen += w;
-    pick(k, __builtin_amdgcn_readfirstlane(id), w);
+    pick(k, id, w);
   }
   return over_chosen ? 1.0f / chosen : 1.0f;  // the largest z contributes exp(0)
 }
