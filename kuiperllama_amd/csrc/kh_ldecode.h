@@ -958,7 +958,7 @@ __global__ __launch_bounds__(256) void k_ld_values(const LdValuesArgs a) {
   const int c4 = a.Rp >> 2;
   f32x4* sum = (f32x4*)(xs + (size_t)nblk * Ld<T>::BE);  // [grp][c4]
   int grp;
-  const float inv = ld_merge_splits(p, lat_active_splits(a.pos[b] + 1, a.nsplit), a.Rp, fac, red, sum, grp);
+  const float inv = ld_merge_splits(p, lat_active_splits(a.pos[b] + 1, a.nsplit, LatCfg<T>::KT), a.Rp, fac, red, sum, grp);
   for (int i = threadIdx.x; i < nblk * Ld<T>::BE / 4; i += 256) {
     f32x4 v = f4_zero();
     if (i < c4)
