@@ -62,10 +62,12 @@ struct LgArgs {
   GateAct act;          // LG_GATED
 };
 
-template <class T, int BM, int BN, bool GROUPED>
+// WM x WN: waves along the tokens and the features
+template <class T, int BM, int BN, bool GROUPED, int WM = 2, int WN = 2>
 struct LgCfg {
-  static constexpr int XS = BM + BN >= 192 ? 2 : (BM + BN >= 128 ? 3 : 4);  // stages of the tokens' ring
-  static constexpr int WS = BM + BN >= 256 && GROUPED ? 3 : XS;             // ... of the weights'
+  static constexpr bool WIDE = WM * WN == 8;  // one workgroup of eight waves per CU: the whole LDS is its
+  static constexpr int XS = WIDE ? 160 * 8 / (BM + BN) : BM + BN >= 192 ? 2 : (BM + BN >= 128 ? 3 : 4);  // stages of the tokens' ring
+  static constexpr int WS = !WIDE && BM + BN >= 256 && GROUPED ? 3 : XS;                                 // ... of the weights'
   static constexpr int LDS = (XS * BM + WS * BN) * 128;
 };
 
@@ -116,14 +118,17 @@ __device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 
   }
 }
 
-template <class T, int BM, int BN, int EPI, bool GROUPED>
-__global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
+template <class T, int BM, int BN, int EPI, bool GROUPED, int WM = 2, int WN = 2>
+__global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
   typedef Tile<T> TL;
   typedef typename TL::frag frag;
-  constexpr int XS = LgCfg<T, BM, BN, GROUPED>::XS, WS = LgCfg<T, BM, BN, GROUPED>::WS;
+  constexpr int NWV = WM * WN;
+  constexpr int XS = LgCfg<T, BM, BN, GROUPED, WM, WN>::XS, WS = LgCfg<T, BM, BN, GROUPED, WM, WN>::WS;
   static_assert(XS >= 2 && WS >= XS, "order of the requests");
-  constexpr int TM = BM / 32, TN = BN / 32;  // 16-wide tiles per wave: tokens, features
-  constexpr int NX = BM / 32, NW = BN / 32;  // LDS-DMA requests per wave and stage
+  static_assert(LgCfg<T, BM, BN, GROUPED, WM, WN>::LDS <= 160 * 1024, "fits a CU");
+  constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN);    // 16-wide tiles per wave: tokens, features
+  constexpr int NX = BM / (8 * NWV), NW = BN / (8 * NWV);    // LDS-DMA requests per wave and stage
+  static_assert(EPI != LG_GATED || TN % 2 == 0, "a gate tile and its up tile are one wave's");
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const char* W = (const char*)a.W;
@@ -144,19 +149,19 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   X += (size_t)blockIdx.z * a.x_z * sizeof(T);
   const int f0 = (int)blockIdx.x * BN;
   const int m_last = m_lo + m_n - 1;
-  // ---- staging addresses: request j of wave w covers rows 8 (4 j + w) .. +8 of the token tile, or of the feature tile
+  // ---- staging addresses: request j of wave w covers rows 8 (NWV j + w) .. +8 of the token tile, or of the feature tile
   unsigned xoff[NX], woff[NW];
   const int sub = lane >> 3, ch = (lane & 7) ^ sub;
 #pragma unroll
   for (int j = 0; j < NX; ++j) {
-    int m = mt0 + 8 * (4 * j + wave) + sub;
+    int m = mt0 + 8 * (NWV * j + wave) + sub;
     m = m < m_last ? m : m_last;
     const int row = GROUPED && a.gather ? a.gather[m] : m;
     xoff[j] = (unsigned)row * (unsigned)(a.ldx * (int)sizeof(T)) + 16u * ch;
   }
 #pragma unroll
   for (int j = 0; j < NW; ++j) {
-    int f = f0 + 8 * (4 * j + wave) + sub;
+    int f = f0 + 8 * (NWV * j + wave) + sub;
     f = f < a.N ? f : a.N - 1;
     woff[j] = (unsigned)f * (unsigned)(a.ldw * (int)sizeof(T)) + 16u * ch;
   }
@@ -164,14 +169,14 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
   auto issue_x = [&](int slot) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NX; ++j) {
-      dma_x4_keep(X, xoff[j], lds0 + (unsigned)(slot * BM * 128 + j * 4096));
+      dma_x4_keep(X, xoff[j], lds0 + (unsigned)(slot * BM * 128 + j * 1024 * NWV));
       xoff[j] += 128;
     }
   };
   auto issue_w = [&](int slot) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NW; ++j) {
-      dma_x4_keep(W, woff[j], lds0 + (unsigned)(XS * BM * 128 + slot * BN * 128 + j * 4096));
+      dma_x4_keep(W, woff[j], lds0 + (unsigned)(XS * BM * 128 + slot * BN * 128 + j * 1024 * NWV));
       woff[j] += 128;
     }
   };
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
     if (j >= WS - XS && j - (WS - XS) < nk) issue_x(j - (WS - XS));
     if (j < nk) issue_w(j);
   }
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % WM, wn = wave / WM;
   const int fr = lane & 15, fh = lane >> 4;
   const int fo0 = fr * 128 + ((fh ^ (fr & 7)) << 4);  // this lane's fragment within 16 rows, first half of the stage
   constexpr int LATER = WS > XS ? NW : 0;             // requests of a step behind the ones that are waited for
@@ -210,7 +215,7 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
         const char* sx = smem_raw + xslot * BM * 128 + (fo0 ^ (b << 6));
         const char* sw = smem_raw + XS * BM * 128 + wslot * BN * 128 + (fo0 ^ (b << 6));
 #pragma unroll
-        for (int m = 0; m < LIVE; ++m) fx[b][m] = *(const frag*)(sx + (2 * m + wm) * 2048);
+        for (int m = 0; m < LIVE; ++m) fx[b][m] = *(const frag*)(sx + (WM * m + wm) * 2048);
 #pragma unroll
         for (int n = 0; n < TN; ++n) fw[b][n] = *(const frag*)(sw + (wn * TN + n) * 2048);
       }
@@ -228,20 +233,20 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
     }
   };
   const int tiles_m = (m_last - mt0) / 16 + 1;  // of the workgroup, with rows in them; they go to the waves in turn
-  const int live = (tiles_m - wm + 1) / 2;
-  if (TM == 1 || live <= 1) loop(std::integral_constant<int, 1>{});
-  else if (TM == 2 || live == 2) loop(std::integral_constant<int, TM < 2 ? 1 : 2>{});
-  else if (live == 3) loop(std::integral_constant<int, TM < 3 ? 1 : 3>{});
+  const int live = (tiles_m - wm + WM - 1) / WM;
+  if (TM == 1 || (TM <= 4 && live <= 1)) loop(std::integral_constant<int, 1>{});
+  else if (TM == 2 || (TM <= 4 && live == 2)) loop(std::integral_constant<int, TM < 2 ? 1 : 2>{});
+  else if (TM <= 4 && live == 3) loop(std::integral_constant<int, TM < 3 ? 1 : 3>{});
   else loop(std::integral_constant<int, TM>{});
   // ---- epilogue: lane (fr, fh) of tile (n, m): token mt0 + .. + fr, features f .. f + 3
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
-    const int tok = mt0 + (2 * m + wm) * 16 + fr;
+    const int tok = mt0 + (WM * m + wm) * 16 + fr;
     if (tok > m_last) continue;
     if (EPI == LG_GATED) {
 #pragma unroll
       for (int n = 0; n + 1 < TN; n += 2) {
-        const int f = f0 + wn * (BN / 2) + n * 16;  // a multiple of 32: gate tile; the up tile follows
+        const int f = f0 + wn * (BN / WN) + n * 16;  // a multiple of 32: gate tile; the up tile follows
         const int c = (f >> 1) + 4 * fh;
         f32x4 v;
 #pragma unroll
@@ -250,20 +255,25 @@ __global__ __launch_bounds__(256) void k_lgemm(const LgArgs a) {
       }
     } else {
 #pragma unroll
-      for (int n = 0; n < TN; ++n) lg_store<T, EPI>(a, tok, f0 + wn * (BN / 2) + n * 16 + 4 * fh, acc[n][m]);
+      for (int n = 0; n < TN; ++n) lg_store<T, EPI>(a, tok, f0 + wn * (BN / WN) + n * 16 + 4 * fh, acc[n][m]);
     }
   }
 }
 
-// Tile choice.  Plain / batched launches: the largest tile that still gives the chip enough workgroups (one per CU is not:
-// nobody covers its barriers).  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
+// Tile choice.  Plain / batched launches: the largest tile that still gives the chip enough workgroups (one of four waves per CU is
+// not: nobody covers its barriers).  In bf16 there are two forms of eight waves, one workgroup per CU with the whole LDS, where
+// the tiles fill the CUs once: 256 x 256 in two stages, which a CU reads half as much for (2048 tokens x 8192 x 2048: 69.8 -> 64.9 us;
+// with rounds that are less than 200 of 256 full it loses that), and 128 x 128 in five, from 129 tiles on (2048 x 2048, K 4096 /
+// 2048: 57 / 31 us as 512 workgroups of 64 x 128, 44 / 25 so; 144 tiles of 1100 tokens, K 4096 / 2048 43 / 24 -> 38 / 22; 128
+// tiles: 12.7 us instead of 9.9).  Experts gain nothing from either (130 us of gate and up with 256 x 256, 137 with 256 x 128): their
+// tiles are a third empty or wait for HBM.  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
 static inline int lg_group_bm(long rows, int groups) {
   const long per = rows / (groups > 0 ? groups : 1);
   return per > 64 ? 128 : (per > 24 ? 64 : 32);
 }
 template <class T, int EPI>
 int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, int max_tiles = 0) {
-  auto go = [&](auto kern, int BM, int BN, int lds) -> int {
+  auto go = [&](auto kern, int BM, int BN, int lds, int wg) -> int {
     if (lds > 64 * 1024) {  // the dynamic-LDS opt-in is per (device, kernel): once
       struct Done { int dev; const void* fn; };
       static thread_local std::vector<Done> done;
@@ -278,11 +288,12 @@ int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, in
       }
     }
     const int gy = a.tiles ? max_tiles : (a.M + BM - 1) / BM;
-    hipLaunchKernelGGL(kern, dim3((a.N + BN - 1) / BN, gy, zdim), dim3(256), lds, s, a);
+    hipLaunchKernelGGL(kern, dim3((a.N + BN - 1) / BN, gy, zdim), dim3(wg), lds, s, a);
     return KH_OK;
   };
   auto tiles = [&](int BM, int BN) { return (long)((a.N + BN - 1) / BN) * ((a.M + BM - 1) / BM) * zdim; };
-#define KH_LG_GO(BM, BN, G) return go(k_lgemm<T, BM, BN, EPI, G>, BM, BN, LgCfg<T, BM, BN, G>::LDS)
+#define KH_LG_GO(BM, BN, G) return go(k_lgemm<T, BM, BN, EPI, G>, BM, BN, LgCfg<T, BM, BN, G>::LDS, 256)
+#define KH_LG_WIDE(BM, BN) return go(k_lgemm<T, BM, BN, EPI, false, 2, 4>, BM, BN, LgCfg<T, BM, BN, false, 2, 4>::LDS, 512)
   if constexpr (EPI == LG_T || EPI == LG_GATED) {
     if (a.tiles) {
       if (group_bm == 128) KH_LG_GO(128, 128, true);
@@ -292,10 +303,17 @@ int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, in
   } else if (a.tiles) {
     return KH_ERR_INTERNAL;
   }
+  if constexpr (sizeof(T) == 2 && (EPI == LG_T || EPI == LG_F32)) {
+    const long t = tiles(128, 128), w = tiles(256, 256);
+    auto full = [&](int bm) { return 4L * ((a.M + bm - 1) / bm * bm) <= 5L * a.M; };  // a fifth of the rows empty at most
+    if ((w % 256 == 0 || w % 256 >= 200) && full(256)) KH_LG_WIDE(256, 256);
+    if (t > 128 && t <= 256 && full(128)) KH_LG_WIDE(128, 128);
+  }
   if (a.M > 64 && tiles(128, 128) >= 400) KH_LG_GO(128, 128, false);
   if (a.M <= 32) KH_LG_GO(32, 64, false);
   if (tiles(64, 128) >= 400) KH_LG_GO(64, 128, false);
   KH_LG_GO(64, 64, false);
 #undef KH_LG_GO
+#undef KH_LG_WIDE
 }
 }  // namespace khm
