@@ -15,6 +15,7 @@ _PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_PKG, "csrc")
 LIB_DIR = os.path.join(_PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libkuiper_hip.so")
+PYOPS_PATH = os.path.join(LIB_DIR, "kh_pyops.so")
 SOURCES = ["kh_ops.hip", "kh_model_load.hip", "kh_model_step.hip", "kh_model_prefill.hip", "kh_model_pair.hip", "kh_model_profile.hip", "kh_model_selftest.hip",
            "kh_hybrid_load.hip", "kh_hybrid_pass.hip", "kh_hybrid_step.hip", "kh_heads.hip",
            "kh_tokenizer.cpp", "kh_bpe.cpp", "kh_debug.cpp"]
@@ -45,7 +46,20 @@ def _stale() -> bool:
     return False
 
 
+def build_pyops(force: bool = False) -> str:
+    """The operator calls without ctypes (csrc/kh_pyops.c): a CPython extension that needs the interpreter's headers alone."""
+    import sysconfig
+    src = os.path.join(CSRC, "kh_pyops.c")
+    if not force and os.path.exists(PYOPS_PATH) and os.path.getmtime(src) <= os.path.getmtime(PYOPS_PATH):
+        return PYOPS_PATH
+    os.makedirs(LIB_DIR, exist_ok=True)
+    subprocess.check_call([shutil.which("gcc") or _hipcc(), "-O2", "-std=gnu11", "-shared", "-fPIC", "-Wall",
+                           f"-I{sysconfig.get_paths()['include']}", src, "-o", PYOPS_PATH])
+    return PYOPS_PATH
+
+
 def build_lib(force: bool = False, verbose: bool = False) -> str:
+    build_pyops(force)
     if not force and not _stale():
         return LIB_PATH
     os.makedirs(LIB_DIR, exist_ok=True)

@@ -7,6 +7,7 @@ torch's current stream.  There is no eager/CPU fallback: a CPU tensor is an erro
 """
 from __future__ import annotations
 
+import os
 from typing import Optional
 
 import torch
@@ -39,26 +40,42 @@ def _stream():
     return _raw_stream(torch.cuda.current_device())
 
 
+class _Unbound:
+    """Stands for csrc/kh_pyops.c, the calls that a decoder layer is made of, until the first of them loads it."""
+
+    def __getattr__(self, name):
+        global _n
+        import ctypes as C
+        import importlib.machinery
+        import importlib.util
+        L = _ffi.lib()
+        path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "kh_pyops.so")
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: build it with `python -m kuiperllama_amd.build`")
+        spec = importlib.util.spec_from_loader("kh_pyops", importlib.machinery.ExtensionFileLoader("kh_pyops", path))
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind(tuple(C.cast(f, C.c_void_p).value for f in (L.kh_add_f32, L.kh_swiglu_f32, L.kh_matmul_f32, L.kh_matmul_q8,
+                                                             L.kh_rmsnorm_f32, L.kh_rope_f32, L.kh_mha_f32)),
+                 (torch.float32, torch.int32, torch.int8, torch.Tensor, getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device),
+                  _raw_stream, _stream, _ffi.check, C.ArgumentError))
+        _n = mod
+        return getattr(mod, name)
+
+
+_n = _Unbound()
+
+
 def add(in1, in2, out):
-    _ffi.check(_ffi.lib().kh_add_f32(_p(in1, torch.float32), _p(in2, torch.float32),
-                                     _p(out, torch.float32), in1.numel(), _stream()), "kh_add_f32")
-    return out
+    return _n.add(in1, in2, out)
 
 
 def matmul(x, w, out, scale: float = 1.0):
-    K, M = w.shape
-    _ffi.check(_ffi.lib().kh_matmul_f32(_p(x, torch.float32), _p(w, torch.float32),
-                                        _p(out, torch.float32), M, K, scale, _stream()),
-               "kh_matmul_f32")
-    return out
+    return _n.matmul(x, w, out, scale)
 
 
 def matmul_q8(x, w8, scales, group_size: int, out):
-    K, M = w8.shape
-    _ffi.check(_ffi.lib().kh_matmul_q8(_p(x, torch.float32), _p(w8, torch.int8),
-                                       _p(scales, torch.float32), group_size,
-                                       _p(out, torch.float32), M, K, _stream()), "kh_matmul_q8")
-    return out
+    return _n.matmul_q8(x, w8, scales, group_size, out)
 
 
 def embedding(tokens, w, out):
@@ -79,26 +96,16 @@ def embedding_host_tokens(tokens, w, out):
 
 
 def swiglu(a, b, out):
-    _ffi.check(_ffi.lib().kh_swiglu_f32(_p(a, torch.float32), _p(b, torch.float32),
-                                        _p(out, torch.float32), a.numel(), _stream()),
-               "kh_swiglu_f32")
-    return out
+    return _n.swiglu(a, b, out)
 
 
 def rmsnorm(x, w, out, eps: float):
-    _ffi.check(_ffi.lib().kh_rmsnorm_f32(_p(x, torch.float32), _p(w, torch.float32),
-                                         _p(out, torch.float32), x.numel(), eps, _stream()),
-               "kh_rmsnorm_f32")
-    return out
+    return _n.rmsnorm(x, w, out, eps)
 
 
 def rope(q, k, pos, sin_cache, cos_cache, head_size: int, mode: int):
     """pos: python int, or a 1-element int32 GPU tensor (graph-capturable form)."""
-    d_pos, ipos = (None, int(pos)) if not torch.is_tensor(pos) else (_p(pos, torch.int32), 0)
-    _ffi.check(_ffi.lib().kh_rope_f32(q.numel(), k.numel(), head_size, _p(q, torch.float32),
-                                      _p(k, torch.float32), d_pos, ipos,
-                                      _p(sin_cache, torch.float32), _p(cos_cache, torch.float32),
-                                      mode, _stream()), "kh_rope_f32")
+    _n.rope(q, k, pos, sin_cache, cos_cache, head_size, mode)
     return q, k
 
 
@@ -112,13 +119,7 @@ def sincos_cache(head_size: int, seq_len: int, theta: float, sin_cache, cos_cach
 
 def mha(pos, head_num, layer_index, seq_len, kv_dim, kv_mul, head_size, mha_out, q, score,
         kcache, vcache):
-    d_pos, ipos = (None, int(pos)) if not torch.is_tensor(pos) else (_p(pos, torch.int32), 0)
-    _ffi.check(_ffi.lib().kh_mha_f32(d_pos, ipos, head_num, layer_index, seq_len, kv_dim, kv_mul,
-                                     head_size, _p(mha_out, torch.float32), _p(q, torch.float32),
-                                     _p(score, torch.float32) if score is not None else None,
-                                     _p(kcache, torch.float32),
-                                     _p(vcache, torch.float32), _stream()), "kh_mha_f32")
-    return mha_out
+    return _n.mha(pos, head_num, layer_index, seq_len, kv_dim, kv_mul, head_size, mha_out, q, score, kcache, vcache)
 
 
 def mha_prefill(pos0, n_tokens, head_num, layer_index, seq_len, kv_dim, kv_mul, head_size, mha_out, q,
