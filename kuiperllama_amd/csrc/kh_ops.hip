@@ -88,8 +88,8 @@ extern "C" int kh_scale_f32(float scale, float* x, int32_t n, void* stream) {
 // =============================================================================================
 // matmul fp32 (GEMV).  reference: cuda/matmul_kernel.cu:7-54 = one 128-thread block per row,
 // x re-read from global by every block.  Here: wave per row pair, x staged once per WG in LDS.
-template <int U, int MAXV>
-__global__ __launch_bounds__(KH_WG) void k_matmul_f32(const float* __restrict__ x,
+template <int U, int MAXV, int SPLIT>
+__global__ __launch_bounds__(KH_WG_MAX, 4) void k_matmul_f32(const float* __restrict__ x,
                                                       const float* __restrict__ w,
                                                       float* __restrict__ y, int M, int K,
                                                       float scale) {
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(KH_WG) void k_matmul_f32(const float* __restrict__ 
     y[r0] = s0 * scale;
     if (r1 != r0) y[r1] = s1 * scale;
   };
-  gemv_pairs<1, /*ROLL=*/false>(g, xs, (K + 1) >> 1, lane, nullptr, pair, [](int) __attribute__((always_inline)) { return NoAux{}; },
+  gemv_pairs<SPLIT, /*ROLL=*/false>(g, xs, (K + 1) >> 1, lane, red + KH_WAVES_MAX, pair, [](int) __attribute__((always_inline)) { return NoAux{}; },
                        [&]() __attribute__((always_inline)) { st.issue(); }, [&]() __attribute__((always_inline)) { (void)st.finish(xs, 0.f, red); }, epi);
 }
 
@@ -136,6 +136,47 @@ static inline int gemv_grid(int nitems_per_wave_unit) {
   return g;
 }
 
+// Launch of a matrix of K rows of M: waves that share a row pair, tiles, threads, workgroups.  Rows are split over waves as the
+// decode step splits them (kh_model_step.hip::pick_shape): until 4096 waves (short rows: 2048) have work and while each still
+// streams 8 KB of its pair (int8: 4 KB); vectors that 256 threads cannot hold in registers are staged by 512.  Llama-3.2-1B's
+// layer, us alone in the row / split: 2048 x 8192 16.6 / 12.0, 2048 x 2048 5.2 / 4.8, 512 x 2048 4.0 / 3.6.
+struct MmShape {
+  int split, u, mv, wg, grid;
+  size_t lds;
+};
+static MmShape mm_shape(bool quant, int M, int K) {
+  MmShape s{1, 2, 4, KH_WG, 1, 0};
+  const int pairs = (K + 1) / 2, Mc = quant ? M / 16 : M / 4;
+  const long bytes = 2L * M * (quant ? 1 : 4), least = quant ? 4096 : 8192;
+  const size_t vec = quant ? kh_q8_lds_bytes(M) : (size_t)M * 4, sums = 2 * KH_WAVES_MAX * 4 + KH_WAVES_MAX * 4;
+  const int target = bytes >= 16384 ? 4096 : 2048;
+  if (vec + sums <= 64 * 1024)
+    while (s.split < 4 && (long)pairs * s.split < target && bytes / (s.split * 2) >= least) s.split *= 2;
+  s.wg = kh_stage_fits4(M) ? KH_WG : KH_WG_MAX;
+  s.mv = kh_stage_maxv(M, s.wg);
+  const int per_lane = ((Mc + s.split - 1) / s.split + KH_WAVE - 1) / KH_WAVE;
+  s.u = !quant && per_lane >= 8 ? 8 : (per_lane >= 3 ? 4 : 2);
+  const int ppw = s.wg / KH_WAVE / s.split, need = (pairs + ppw - 1) / ppw, most = 1024 * KH_WG / s.wg;
+  s.grid = need < most ? need : most;
+  s.lds = vec + (s.split > 1 ? sums : 16);
+  return s;
+}
+
+#define KH_MM_SPLITS(GO, sh, UU, MV)      \
+  if ((sh).mv == MV) {                    \
+    if ((sh).split == 1) GO(UU, MV, 1);   \
+    else if ((sh).split == 2) GO(UU, MV, 2); \
+    else GO(UU, MV, 4);                   \
+  }
+#define KH_MM_TILES(GO, sh, UU)  \
+  if ((sh).u == UU) {            \
+    KH_MM_SPLITS(GO, sh, UU, 1)  \
+    KH_MM_SPLITS(GO, sh, UU, 2)  \
+    KH_MM_SPLITS(GO, sh, UU, 4)  \
+    KH_MM_SPLITS(GO, sh, UU, 6)  \
+    KH_MM_SPLITS(GO, sh, UU, 0)  \
+  }
+
 extern "C" int kh_matmul_f32(const float* x, const float* w, float* y, int32_t M, int32_t K,
                              float scale, void* stream) {
   if (!x || !w || !y || M <= 0 || K <= 0) return KH_ERR_INVALID_ARG;
@@ -147,19 +188,12 @@ extern "C" int kh_matmul_f32(const float* x, const float* w, float* y, int32_t M
                        K, scale);
     return kh_launch_status();
   }
-  const size_t lds = (size_t)M * 4 + 16;
-  const int grid = gemv_grid((K + 1) / 2);
-  const int per_lane = (M / 4 + KH_WAVE - 1) / KH_WAVE;
-#define KH_MM(UU, MV) \
-  hipLaunchKernelGGL((k_matmul_f32<UU, MV>), dim3(grid), dim3(KH_WG), lds, s, x, w, y, M, K, scale)
-  const bool inreg = kh_stage_fits4(M);
-  if (per_lane >= 8) {
-    if (inreg) KH_MM(8, 4); else KH_MM(8, 0);
-  } else if (per_lane >= 3) {
-    if (inreg) KH_MM(4, 4); else KH_MM(4, 0);
-  } else {
-    KH_MM(2, 4);  // per_lane < 3 implies M <= 512
-  }
+  const MmShape sh = mm_shape(false, M, K);
+#define KH_MM(UU, MV, SP) \
+  hipLaunchKernelGGL((k_matmul_f32<UU, MV, SP>), dim3(sh.grid), dim3(sh.wg), sh.lds, s, x, w, y, M, K, scale)
+  KH_MM_TILES(KH_MM, sh, 8)
+  KH_MM_TILES(KH_MM, sh, 4)
+  KH_MM_TILES(KH_MM, sh, 2)
 #undef KH_MM
   return kh_launch_status();
 }
@@ -167,8 +201,8 @@ extern "C" int kh_matmul_f32(const float* x, const float* w, float* y, int32_t M
 // =============================================================================================
 // matmul int8 group-dequant.  reference: cuda/matmul_kernel.cu:56-87 (scalar byte loads, an
 // integer divide and a scale load per element).
-template <int U, int MAXV>
-__global__ __launch_bounds__(KH_WG) void k_matmul_q8(const float* __restrict__ x,
+template <int U, int MAXV, int SPLIT>
+__global__ __launch_bounds__(KH_WG_MAX, 4) void k_matmul_q8(const float* __restrict__ x,
                                                      const int8_t* __restrict__ w,
                                                      const float* __restrict__ scales,
                                                      int gshift, float* __restrict__ y, int M,
@@ -188,7 +222,7 @@ __global__ __launch_bounds__(KH_WG) void k_matmul_q8(const float* __restrict__ x
     y[r0] = s0;
     if (r1 != r0) y[r1] = s1;
   };
-  gemv_pairs<1, /*ROLL=*/false>(g, xs, (K + 1) >> 1, lane, nullptr, pair, [](int) __attribute__((always_inline)) { return NoAux{}; },
+  gemv_pairs<SPLIT, /*ROLL=*/false>(g, xs, (K + 1) >> 1, lane, red + KH_WAVES_MAX, pair, [](int) __attribute__((always_inline)) { return NoAux{}; },
                       [&]() __attribute__((always_inline)) { st.issue(); }, [&]() __attribute__((always_inline)) { (void)st.finish(xs, 0.f, red); }, epi);
 }
 
@@ -234,18 +268,11 @@ extern "C" int kh_matmul_q8(const float* x, const int8_t* w8, const float* scale
                        scales, group_size, y, M, K);
     return kh_launch_status();
   }
-  const size_t lds = kh_q8_lds_bytes(M) + 16;
-  const int grid = gemv_grid((K + 1) / 2);
-  const int per_lane = (M / 16 + KH_WAVE - 1) / KH_WAVE;
-#define KH_MMQ(UU, MV)                                                                        \
-  hipLaunchKernelGGL((k_matmul_q8<UU, MV>), dim3(grid), dim3(KH_WG), lds, s, x, w8, scales, gshift, \
-                     y, M, K)
-  const bool inreg = kh_stage_fits4(M);
-  if (per_lane >= 3) {
-    if (inreg) KH_MMQ(4, 4); else KH_MMQ(4, 0);
-  } else {
-    KH_MMQ(2, 4);  // per_lane < 3 implies M <= 2048
-  }
+  const MmShape sh = mm_shape(true, M, K);
+#define KH_MMQ(UU, MV, SP)                                                                                              \
+  hipLaunchKernelGGL((k_matmul_q8<UU, MV, SP>), dim3(sh.grid), dim3(sh.wg), sh.lds, s, x, w8, scales, gshift, y, M, K)
+  KH_MM_TILES(KH_MMQ, sh, 4)
+  KH_MM_TILES(KH_MMQ, sh, 2)
 #undef KH_MMQ
   return kh_launch_status();
 }
