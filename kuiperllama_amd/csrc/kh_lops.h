@@ -55,44 +55,68 @@ __device__ __forceinline__ f32x4 fma_s(float s, f32x4 a, f32x4 b) {
 }
 template <class T>
 __global__ __launch_bounds__(256) void k_combine(const CombineArgs<T> a) {
+  typedef typename Tile<T>::quad quad;
+  constexpr int U = 4;  // expert rows requested together
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f32x4* row = (f32x4*)smem_raw;  // [ld / 4]
   __shared__ float red[KH_WAVES_MAX];
-  const int t = blockIdx.x, n4 = a.ld >> 2;
+  const int t = blockIdx.x, n4 = a.ld >> 2, lane = threadIdx.x & 63;
   const size_t o = (size_t)t * a.ld;
   float s = 0.f;
+  const int top = a.add.y ? a.add.top : 0;
+  // lane k: choice k
+  const int my_slot = lane < top ? a.add.y_slot[(size_t)t * top + lane] : -1;
+  const float my_w = lane < top ? a.add.y_w[(size_t)t * top + lane] : 0.f;
   const T* e = a.from_embed ? a.embed + (size_t)a.tok[t] * a.ld : nullptr;
   const T* ep = a.from_embed && a.pos_emb ? a.pos_emb + (size_t)a.pos[t] * a.ld : nullptr;
   const float idw = a.add.y && a.add.id_w ? a.add.id_w[t] : 0.f, shg = a.add.sh && a.add.sh_g ? a.add.sh_g[t] : 1.f;
-  const int top = a.add.y ? a.add.top : 0;
   for (int i = threadIdx.x; i < n4; i += 256) {
     const int c = 4 * i;
-    f32x4 v;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v, d = zero, x0 = zero, st = zero;
+    quad idq{}, shq{};
+    if (a.add.mix) d = *(const f32x4*)(a.add.mix + o + c);
+    if (!a.from_embed) v = *(const f32x4*)(a.x + o + c);
+    if (a.add_x0 || (a.cat && !a.from_embed)) x0 = *(const f32x4*)(a.x0 + o + c);
+    if (a.step) st = *(const f32x4*)(a.step + c);
+    if (a.add.sh) shq = *(const quad*)(a.add.sh + o + c);
+    if (idw != 0.f) idq = *(const quad*)(a.xn2_prev + o + c);
     if (a.from_embed) {
       v = quad_f(e + c) * a.emb_scale;
       if (ep) v += quad_f(ep + c);
       *(f32x4*)(a.x0 + o + c) = v;
-    } else {
-      v = *(const f32x4*)(a.x + o + c);
+      x0 = v;
     }
     if (a.add.mix) {
-      f32x4 d = *(const f32x4*)(a.add.mix + o + c);
-      f32x4 f = {0.f, 0.f, 0.f, 0.f};
-      for (int k = 0; k < top; ++k) {
-        const int sl = a.add.y_slot[(size_t)t * top + k];
-        if (sl >= 0) f = fma_s(a.add.y_w[(size_t)t * top + k], quad_f(a.add.y + (size_t)sl * a.ld + c), f);
+      f32x4 f = zero;
+      for (int k0 = 0; k0 < top; k0 += U) {
+        quad r[U];
+        int sl[U];
+        float w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = k0 + u < top ? k0 + u : 63;  // lanes behind `top` hold -1
+          sl[u] = __builtin_amdgcn_readlane(my_slot, k);
+          w[u] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_w), k));
+          r[u] = *(const quad*)(a.add.y + (size_t)max(sl[u], 0) * a.ld + c);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const f32x4 q = {(float)r[u].x, (float)r[u].y, (float)r[u].z, (float)r[u].w};
+          if (sl[u] >= 0) f = fma_s(w[u], q, f);
+        }
       }
-      if (idw != 0.f) f = fma_s(idw, quad_f(a.xn2_prev + o + c), f);
-      if (a.add.sh) f = fma_s(shg, quad_f(a.add.sh + o + c), f);
+      if (idw != 0.f) f = fma_s(idw, f32x4{(float)idq.x, (float)idq.y, (float)idq.z, (float)idq.w}, f);
+      if (a.add.sh) f = fma_s(shg, f32x4{(float)shq.x, (float)shq.y, (float)shq.z, (float)shq.w}, f);
       d += f;
       v = fma_s(a.mult, d, v);
     }
-    if (a.add_x0) v += *(const f32x4*)(a.x0 + o + c);
-    if (a.step) v += *(const f32x4*)(a.step + c);
+    if (a.add_x0) v += x0;
+    if (a.step) v += st;
     *(f32x4*)(a.x + o + c) = v;
     if (a.cat) {
-      *(typename Tile<T>::quad*)(a.cat + 2 * o + c) = to_quad<T>(v);
-      *(typename Tile<T>::quad*)(a.cat + 2 * o + a.ld + c) = to_quad<T>(a.from_embed ? v : *(const f32x4*)(a.x0 + o + c));
+      *(quad*)(a.cat + 2 * o + c) = to_quad<T>(v);
+      *(quad*)(a.cat + 2 * o + a.ld + c) = to_quad<T>(a.from_embed ? v : x0);
     }
     row[i] = v;
     s += (v.x + v.y) + (v.z + v.w);
@@ -117,12 +141,12 @@ __global__ __launch_bounds__(256) void k_combine(const CombineArgs<T> a) {
     const f32x4 w1 = *(const f32x4*)(a.w1 + c), b1 = a.b1 ? *(const f32x4*)(a.b1 + c) : zero;
 #pragma unroll
     for (int k = 0; k < 4; ++k) y[k] = (v[k] - mean) * rstd * w1[k] + b1[k];  // pads: weights and biases are zero
-    *(typename Tile<T>::quad*)(a.xn1 + o + c) = to_quad<T>(y);
+    *(quad*)(a.xn1 + o + c) = to_quad<T>(y);
     if (a.w2) {
       const f32x4 w2 = *(const f32x4*)(a.w2 + c), b2 = a.b2 ? *(const f32x4*)(a.b2 + c) : zero;
 #pragma unroll
       for (int k = 0; k < 4; ++k) y[k] = (v[k] - mean) * rstd * w2[k] + b2[k];
-      *(typename Tile<T>::quad*)(a.xn2 + o + c) = to_quad<T>(y);
+      *(quad*)(a.xn2 + o + c) = to_quad<T>(y);
     }
   }
 }
