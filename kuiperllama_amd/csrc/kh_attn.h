@@ -50,27 +50,47 @@ static inline size_t attn_lds_bytes(int head_size, int wg = KH_WG) {
 // the reference's score tensor.  smem: attn_lds_bytes(hs) bytes, 16-B aligned.
 // U timesteps per thread and batch; the next batch is requested before the current one is used, and the first values
 // before the softmax statistics.
-template <int U>
+// GC: lanes per timestep, a power of two >= hs / 4 (0: found here).
+// part of parts: all scores, then that part of the value's columns, with as many more timesteps side by side.
+template <int U, int GC = 0>
 __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
                                                  const float* __restrict__ k_base,
                                                  const float* __restrict__ v_base, int kv_stride,
                                                  int hs, int pos, float* __restrict__ out_h,
-                                                 float* __restrict__ score_out, float* smem) {
+                                                 float* __restrict__ score_out, float* smem, int part = 0,
+                                                 int parts = 1) {
   float* sc = smem;                    // [KH_ATTN_TC]
   float* red = smem + KH_ATTN_TC;      // [8]
-  float* opart = red + 8;              // [4][hs]
+  float* opart = red + 8;              // [waves][hs / parts]
   const int tid = threadIdx.x;
-  const int hs4 = hs >> 2;
-  int G = 1;
-  while (G < hs4) G <<= 1;             // lanes per timestep (<= 64 since hs <= 256)
-  const int TPI = kh_wg() / G;         // timesteps per workgroup iteration
-  const int tg = tid / G, dl = tid - tg * G;
-  const bool active = dl < hs4;
   const int stride4 = kv_stride >> 2;
   const f32x4* K4 = (const f32x4*)k_base;
   const f32x4* V4 = (const f32x4*)v_base;
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  const f32x4 q4 = active ? ((const f32x4*)q_h)[dl] : zero4;
+  auto lanes_of = [](int n) __attribute__((always_inline)) {
+    int g = 1;
+    while (g < n) g <<= 1;
+    return g;
+  };
+  struct Lanes {  // of a timestep's row: `cols` float4 of it by G lanes (<= 64 since hs <= 256)
+    int G, TPI, tg, dl, cols, at;  // TPI: timesteps per workgroup iteration; at: the lane's float4
+    bool active;
+  };
+  auto lanes_for = [&](int G, int cols, int first) __attribute__((always_inline)) {
+    Lanes r;
+    r.G = G;
+    r.TPI = kh_wg() / G;
+    r.tg = tid / G;
+    r.dl = tid - r.tg * G;
+    r.cols = cols;
+    r.active = r.dl < cols;
+    r.at = first + r.dl;
+    return r;
+  };
+  const int hs4 = hs >> 2, vc4 = hs4 / parts;
+  const Lanes kl = lanes_for(GC ? GC : lanes_of(hs4), hs4, 0);
+  const Lanes vl = parts == 1 ? kl : lanes_for(lanes_of(vc4), vc4, part * vc4);
+  const f32x4 q4 = kl.active ? ((const f32x4*)q_h)[kl.dl] : zero4;
   const float scale = 1.0f / sqrtf((float)hs);   // cpu/mha_kernel.cpp:11
   const int nT = pos + 1;
   const bool single = nT <= KH_ATTN_TC;
@@ -81,63 +101,69 @@ __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
   for (int t0 = 0; t0 < nT; t0 += KH_ATTN_TC) {
     const int tc = min(KH_ATTN_TC, nT - t0);
     // row of timestep t0 + tb + u TPI + tg, clamped to the chunk; nothing is requested behind its end
-    auto load_as = [&](f32x4(&r)[U], const f32x4* base, int tb, auto f) __attribute__((always_inline)) {
+    auto load_as = [&](f32x4(&r)[U], const f32x4* base, const Lanes& ln, int tb, auto f) __attribute__((always_inline)) {
       constexpr bool full = decltype(f)::value;  // a whole batch: no guards between the requests
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         r[u] = zero4;
-        if (!full && tb + u * TPI >= tc) continue;  // uniform
-        const int t = tb + u * TPI + tg, tt = t < tc ? t : tc - 1;
-        if (active) r[u] = base[(size_t)(t0 + tt) * stride4 + dl];
+        if (!full && tb + u * ln.TPI >= tc) continue;  // uniform
+        const int t = tb + u * ln.TPI + ln.tg, tt = t < tc ? t : tc - 1;
+        if (ln.active) r[u] = base[(size_t)(t0 + tt) * stride4 + ln.at];
       }
     };
-    const int step = TPI * U;
-    auto load = [&](f32x4(&r)[U], const f32x4* base, int tb) __attribute__((always_inline)) {
-      if (tb + step <= tc) load_as(r, base, tb, std::true_type{});
-      else load_as(r, base, tb, std::false_type{});
+    auto load = [&](f32x4(&r)[U], const f32x4* base, const Lanes& ln, int tb) __attribute__((always_inline)) {
+      if (tb + ln.TPI * U <= tc) load_as(r, base, ln, tb, std::true_type{});
+      else load_as(r, base, ln, tb, std::false_type{});
     };
-    auto apply = [&](const f32x4(&r)[U], int tb, auto&& use) __attribute__((always_inline)) {
-      if (tb + step <= tc) {
+    auto apply = [&](const f32x4(&r)[U], const Lanes& ln, int tb, auto&& use) __attribute__((always_inline)) {
+      if (tb + ln.TPI * U <= tc) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) use(r[u], tb + u * TPI + tg);
+        for (int u = 0; u < U; ++u) use(r[u], tb + u * ln.TPI + ln.tg);
       } else {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (tb + u * TPI >= tc) break;  // uniform
-          use(r[u], tb + u * TPI + tg);
+          if (tb + u * ln.TPI >= tc) break;  // uniform
+          use(r[u], tb + u * ln.TPI + ln.tg);
         }
       }
     };
     // batches 0, step, ... through two register sets
-    auto stream = [&](const f32x4* base, f32x4(&r0)[U], auto&& use) __attribute__((always_inline)) {
+    auto stream = [&](const f32x4* base, const Lanes& ln, f32x4(&r0)[U], auto&& use) __attribute__((always_inline)) {
       f32x4 r1[U];
+      const int step = ln.TPI * U;
       for (int tb = 0; tb < tc; tb += 2 * step) {
-        if (tb + step < tc) load(r1, base, tb + step);
-        apply(r0, tb, use);
+        asm volatile("" : "+s"(tb));  // or a batch's addresses are kept beside the next ones' (k_mha: 227 registers, 0.5 us slower)
+        if (tb + step < tc) load(r1, base, ln, tb + step);
+        apply(r0, ln, tb, use);
         if (tb + step < tc) {
-          if (tb + 2 * step < tc) load(r0, base, tb + 2 * step);
-          apply(r1, tb + step, use);
+          if (tb + 2 * step < tc) load(r0, base, ln, tb + 2 * step);
+          apply(r1, ln, tb + step, use);
         }
       }
     };
     f32x4 kv[U], vv[U];
-    load(kv, K4, 0);
+    float mx = -INFINITY;
+    load(kv, K4, kl, 0);
     // ---- scores: s[t] = (q . K[t]) * scale ---------------------------------------------
-    stream(K4, kv, [&](const f32x4& k4, int t) __attribute__((always_inline)) {
+    stream(K4, kl, kv, [&](const f32x4& k4, int t) __attribute__((always_inline)) {
       float d = fma4(q4, k4, 0.f);
-      for (int off = G >> 1; off > 0; off >>= 1) d += __shfl_xor(d, off, KH_WAVE);
-      if (dl == 0 && t < tc) {
+      if constexpr (GC) {
+        d = group_sum<GC>(d);
+      } else {
+        for (int off = kl.G >> 1; off > 0; off >>= 1) d += __shfl_xor(d, off, KH_WAVE);
+      }
+      if (t < tc) {
         const float s = d * scale;
-        sc[t] = s;
-        if (score_out && !single) score_out[t0 + t] = s;  // raw score; normalised in the last pass
+        mx = fmaxf(mx, s);
+        if (kl.dl == 0) {
+          sc[t] = s;
+          if (score_out && !single) score_out[t0 + t] = s;  // raw score; normalised in the last pass
+        }
       }
     });
-    load(vv, V4, 0);
-    __syncthreads();
+    load(vv, V4, vl, 0);
     // ---- running softmax statistics --------------------------------------------------------
-    float mx = -INFINITY;
-    for (int t = tid; t < tc; t += kh_wg()) mx = fmaxf(mx, sc[t]);
-    mx = block_max(mx, red);
+    mx = block_max(mx, red);  // its barriers publish the scores as well
     const float m_new = fmaxf(m_run, mx);
     float s = 0.f;
     for (int t = tid; t < tc; t += kh_wg()) {
@@ -156,7 +182,7 @@ __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
       __syncthreads();
     }
     // ---- o += sum_t p[t] * V[t] --------------------------------------------------------------
-    stream(V4, vv, [&](const f32x4& v4, int t) __attribute__((always_inline)) {
+    stream(V4, vl, vv, [&](const f32x4& v4, int t) __attribute__((always_inline)) {
       const float p = t < tc ? sc[t] : 0.f;
       o4.x = __builtin_fmaf(p, v4.x, o4.x);
       o4.y = __builtin_fmaf(p, v4.y, o4.y);
@@ -166,23 +192,23 @@ __device__ __forceinline__ void attn_head_decode(const float* __restrict__ q_h,
     __syncthreads();  // sc is rewritten by the next chunk
   }
 
-  // ---- fold the timestep groups: lanes with equal dl inside a wave, then the 4 waves --------
-  for (int off = G; off < KH_WAVE; off <<= 1) {
+  // ---- fold the timestep groups: lanes with equal dl inside a wave, then the waves --------
+  for (int off = vl.G; off < KH_WAVE; off <<= 1) {
     o4.x += __shfl_xor(o4.x, off, KH_WAVE);
     o4.y += __shfl_xor(o4.y, off, KH_WAVE);
     o4.z += __shfl_xor(o4.z, off, KH_WAVE);
     o4.w += __shfl_xor(o4.w, off, KH_WAVE);
   }
-  const int lane = tid & 63, wave = tid >> 6;
-  if (G <= KH_WAVE && lane < G && active) ((f32x4*)(opart + wave * hs))[dl] = o4;
+  const int lane = tid & 63, wave = tid >> 6, vw = 4 * vl.cols;
+  if (lane < vl.G && vl.active) ((f32x4*)(opart + wave * vw))[vl.dl] = o4;
   __syncthreads();
-  if (tid < hs) {
+  if (tid < vw) {
     float r = 0.f;
-    // when G == 256/TPI... every wave holds a partial for every d (TPI >= 4 <=> G <= 64)
+    // every wave holds a partial for every column (at most 64 lanes per timestep)
     const int nw = kh_nwaves();
 #pragma unroll
-    for (int w = 0; w < KH_WAVES_MAX; ++w) r += w < nw ? opart[(w < nw ? w : 0) * hs + tid] : 0.f;
-    out_h[tid] = single ? r : r / l_run;
+    for (int w = 0; w < KH_WAVES_MAX; ++w) r += w < nw ? opart[(w < nw ? w : 0) * vw + tid] : 0.f;
+    out_h[part * vw + tid] = single ? r : r / l_run;
   }
   if (score_out) {
     // probabilities as the reference leaves them in the score tensor

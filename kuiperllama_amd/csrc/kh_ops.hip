@@ -139,7 +139,7 @@ static inline int gemv_grid(int nitems_per_wave_unit) {
 // Launch of a matrix of K rows of M: waves that share a row pair, tiles, threads, workgroups.  Rows are split over waves as the
 // decode step splits them (kh_model_step.hip::pick_shape): until 4096 waves (short rows: 2048) have work and while each still
 // streams 8 KB of its pair (int8: 4 KB); vectors that 256 threads cannot hold in registers are staged by 512.  Llama-3.2-1B's
-// layer, us alone in the row / split: 2048 x 8192 16.6 / 12.0, 2048 x 2048 5.2 / 4.8, 512 x 2048 4.0 / 3.6.
+// layer, us alone in the row / split: 2048 x 8192 16.6 / 11.9, 2048 x 2048 5.2 / 4.5, 512 x 2048 4.0 / 3.6.
 struct MmShape {
   int split, u, mv, wg, grid;
   size_t lds;
@@ -488,12 +488,19 @@ extern "C" int kh_sincos_cache_f32(int32_t head_size, int32_t max_seq_len, float
 
 // =============================================================================================
 // multi-head attention (decode).  Device core in kh_attn.h.
-// One workgroup of eight waves per head, eight timesteps per thread and batch, two batches in flight: the launch is a chain
-// of memory trips (scores, then values), so their number counts.  Back to back on Llama-3.2-1B's geometry, us at positions
-// 30 / 255 / 700 / 4000: 5.5 / 11.0 / 24.2 / 148 with four waves, four timesteps and one batch, 5.4 / 7.9 / 15.1 / 81 now.
+// Workgroups of eight waves, eight timesteps per thread and batch, two batches in flight: the launch is a chain of memory trips
+// (scores, then values), and a CU pulls 30-40 B/ns.  A head is `parts` workgroups: every one takes all scores and a part of the
+// value's columns, the first one writes the probabilities.  Blocks go round the XCDs, so with block -> group b % groups the
+// workgroups that read the same rows (the heads of a group and their parts) share an L2.  Llama-3.2-1B's geometry in a layer of
+// operators, us at position 700 / 1900: 17.6 / 39.0 with a workgroup a head in head order and sums over lanes through LDS, 11.4 /
+// 22.0 in group order with sums by DPP, 9.8 / 17.9 with four parts; 32 heads on 32 groups of 128 at 200: 12.5, 9.0, 7.8; where
+// all is one trip (TinyLlama at 20) 5.9, 5.7, 5.9.
+// (The parts' batches begun one behind the other, so that one's misses are the next one's hits: 1.0 us slower.)
+// GC: lanes per timestep (attn_lanes), 0: found in the kernel (heads of at most 32).
+template <int GC>
 __global__ __launch_bounds__(KH_WG_MAX) void k_mha(const int32_t* __restrict__ d_pos, int pos_val,
                                                int layer_index, int seq_len, int kv_dim,
-                                               int kv_mul, int head_size,
+                                               int kv_mul, int head_size, int heads, int parts,
                                                float* __restrict__ mha_out,
                                                const float* __restrict__ q,
                                                float* __restrict__ score,
@@ -501,13 +508,16 @@ __global__ __launch_bounds__(KH_WG_MAX) void k_mha(const int32_t* __restrict__ d
                                                const float* __restrict__ vcache) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   const int pos = d_pos ? *d_pos : pos_val;
-  const int h = blockIdx.x;
+  const int groups = (heads + kv_mul - 1) / kv_mul;
+  const int g = (int)blockIdx.x % groups, r = (int)blockIdx.x / groups, part = r / kv_mul;
+  const int h = g * kv_mul + r % kv_mul;
+  if (h >= heads) return;
   const size_t layer_off = (size_t)layer_index * (size_t)seq_len * (size_t)kv_dim;
-  const size_t head_off = (size_t)(h / kv_mul) * head_size;
-  attn_head_decode<8>(q + (size_t)h * head_size, kcache + layer_off + head_off,
-                   vcache + layer_off + head_off, kv_dim, head_size, pos,
-                   mha_out + (size_t)h * head_size, score ? score + (size_t)h * seq_len : nullptr,
-                   (float*)smem_raw);
+  const size_t head_off = (size_t)g * head_size;
+  attn_head_decode<8, GC>(q + (size_t)h * head_size, kcache + layer_off + head_off,
+                          vcache + layer_off + head_off, kv_dim, head_size, pos,
+                          mha_out + (size_t)h * head_size, score && part == 0 ? score + (size_t)h * seq_len : nullptr,
+                          (float*)smem_raw, part, parts);
 }
 
 // decode attention through the launch the fused step uses (kh_attn.h); ns_g == 0: per-head only
@@ -560,9 +570,22 @@ extern "C" int kh_mha_f32(const int32_t* d_pos, int32_t pos, int32_t head_num,
     // one workgroup per head (kh_mha_decode_f32 adds the long-context time split)
     return launch_mha_fast(d_pos, pos, head_num, layer_index, seq_len, kv_dim, kv_mul, head_size,
                            mha_out, q, kcache, vcache, 1, 0, 1, 1 << 30, nullptr, s);
-  hipLaunchKernelGGL(k_mha, dim3(head_num), dim3(KH_WG_MAX), attn_lds_bytes(head_size, KH_WG_MAX), s, d_pos,
-                     pos, layer_index, seq_len, kv_dim, kv_mul, head_size, mha_out, q, score,
-                     kcache, vcache);
+  kv_mul = kv_mul < head_num ? kv_mul : head_num;
+  const int groups = (head_num + kv_mul - 1) / kv_mul;
+  int parts = 4;  // of whole float4, at most a workgroup per CU (MI355X: 256)
+  while (parts > 1 && (head_size % (4 * parts) || (long)groups * kv_mul * parts > 256)) parts /= 2;
+  const size_t dim = (size_t)head_num * head_size;
+  if (mha_out < q + dim && q < mha_out + dim) parts = 1;  // in place: the workgroup that writes a head has read its query
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(groups * kv_mul * parts), dim3(KH_WG_MAX), attn_lds_bytes(head_size, KH_WG_MAX), s, d_pos, pos,
+                       layer_index, seq_len, kv_dim, kv_mul, head_size, head_num, parts, mha_out, q, score, kcache, vcache);
+  };
+  switch (head_size <= 32 ? 0 : attn_lanes(head_size)) {
+    case 16: go(k_mha<16>); break;
+    case 32: go(k_mha<32>); break;
+    case 64: go(k_mha<64>); break;
+    default: go(k_mha<0>);
+  }
   return kh_launch_status();
 }
 

@@ -615,6 +615,61 @@ def test_mha_score_form_batch_edges(gpu, oracle, heads, kv_heads, hs):
         np.testing.assert_allclose(host(score)[:, : pos + 1], so[:, : pos + 1], rtol=0, atol=3e-6, err_msg=str(pos))
 
 
+@pytest.mark.parametrize("heads,kv_mul,hs", [(6, 3, 40), (5, 2, 36), (3, 8, 64), (72, 8, 64), (160, 40, 48), (64, 1, 96)])
+def test_mha_score_form_parts(gpu, oracle, heads, kv_mul, hs):
+    """k_mha: heads of one, two and four workgroups (columns that divide, launches that fill the chip), a last group of fewer
+    heads, a group of more heads than there are, the result over the query."""
+    from kuiperllama_amd import ops
+    seq, groups = 300, -(-heads // kv_mul)
+    rng = np.random.default_rng(heads)
+    kc = rng.standard_normal((1, seq, groups * hs)).astype(np.float32)
+    vc = rng.standard_normal((1, seq, groups * hs)).astype(np.float32)
+    q = rng.standard_normal(heads * hs).astype(np.float32)
+    kcd, vcd = dev(kc, gpu), dev(vc, gpu)
+    for pos in (0, 130, 299):
+        oo, so = oracle.mha(pos, heads, 0, seq, groups * hs, kv_mul, hs, q, kc, vc, acc=oracle.ACC_F64)
+        for inplace in (False, True):
+            qd = dev(q, gpu)
+            out = qd if inplace else torch.full((heads * hs,), float("nan"), device=gpu)
+            score = torch.full((heads, seq), float("nan"), device=gpu)
+            ops.mha(pos, heads, 0, seq, groups * hs, kv_mul, hs, out, qd, score, kcd, vcd)
+            np.testing.assert_allclose(host(out), oo, rtol=0, atol=3e-5, err_msg=f"{pos} {inplace}")
+            np.testing.assert_allclose(host(score)[:, : pos + 1], so[:, : pos + 1], rtol=0, atol=3e-6, err_msg=f"{pos} {inplace}")
+            assert np.isnan(host(score)[:, pos + 1:]).all()
+
+
+def _mm_case(rng, K, M, quant):
+    w = rng.standard_normal((K, M)).astype(np.float32)
+    x = rng.standard_normal(M).astype(np.float32)
+    if not quant:
+        return w, x, w.astype(np.float64) @ x.astype(np.float64), np.abs(w.astype(np.float64)) @ np.abs(x.astype(np.float64))
+    q = rng.integers(-127, 128, (K, M)).astype(np.int8)
+    s = rng.uniform(0.5, 2.0, K * M // 64).astype(np.float32) / 127
+    wd = q.astype(np.float64) * np.repeat(s.astype(np.float64), 64).reshape(K, M)
+    return (q, s), x, wd @ x.astype(np.float64), np.abs(wd) @ np.abs(x.astype(np.float64))
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("K", [1, 3, 512, 515, 2048, 8209])
+def test_matmul_rows_over_waves(gpu, K, quant):
+    """k_matmul_f32 / k_matmul_q8: rows of one, two and four waves, vectors at the edges of what is staged in registers and of
+    what is not, rows that no whole batch and no whole workgroup fills.  A sum of M products in fp32 is within M/64 + 16
+    roundings (a lane's chain, the folds) of the sum of their sizes."""
+    from kuiperllama_amd import ops
+    rng = np.random.default_rng(K)
+    edges = (64, 192, 1024, 4096, 4160, 8192, 8256, 12288, 12352, 16320) if K <= 515 else (64, 2048, 4096, 8192)
+    for M in edges if quant else sorted({m + d for m in edges for d in (0, 4) if m + d >= 4}):
+        w, x, want, size = _mm_case(rng, K, M, quant)
+        out = torch.full((K,), float("nan"), device=gpu)
+        xd = dev(x, gpu)
+        if quant:
+            ops.matmul_q8(xd, dev(w[0], gpu), dev(w[1], gpu), 64, out)
+        else:
+            ops.matmul(xd, dev(w, gpu), out)
+        bound = (M / 64 + 16) * 2.0 ** -24 * size
+        assert (np.abs(host(out) - want) <= bound).all(), (K, M, float((np.abs(host(out) - want) / size).max() * 2 ** 24))
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 511, 512, 513, 576, 577, 1500])
 def test_embedding_host_tokens_launch_edges(gpu, n):
     """Lists that fill a launch of 64 or of 512 ids, and one more; an id out of range leaves its row alone."""
