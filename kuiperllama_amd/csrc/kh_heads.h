@@ -122,6 +122,7 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
   constexpr int DK = 64 * KN, DV = 64 * KV, ROW = DK + DV, CB = ROW / E;
   constexpr int NQ = DK / (4 * E), NT = DV / 16 / CP, NL = ROW / 64;
   constexpr int TB = heads_tile_bytes(DK, DV), NST = heads_stages(TB, KS), WR = 4 / CP, ROWS = 16 * MR * WR;
+  constexpr bool LATE = KS == 4 && CP == 1;  // values behind the softmax: four waves on a SIMD have 128 registers
   constexpr int BOX = 4 * MR * NT * 1024 + 2048 * MR;  // what a set of four waves hands over
   static_assert((KS - 1) * BOX <= KS * NST * TB, "fits the stages");
   static_assert(TB == KT * ROW * ES, "a tile");
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
       }
     frag fv[NT];  // requested with the keys: they arrive under the scores and the softmax
 #pragma unroll
-    for (int n = 0; n < NT; ++n) fv[n] = lat_col<CB>(Kt, DK + (wc * NT + n) * 16, lane, T());
+    for (int n = 0; n < (LATE ? 0 : NT); ++n) fv[n] = lat_col<CB>(Kt, DK + (wc * NT + n) * 16, lane, T());
 #pragma unroll
     for (int b = 0; b < NQ; ++b)
 #pragma unroll
@@ -369,6 +370,11 @@ __global__ __launch_bounds__(256 * KS, KN + KV > 4 && KS == 1 ? 1 : 2) void k_he
           p[q][4 * n + i] = (T)e;
         }
       l[q] += sum;
+    }
+    if constexpr (LATE) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int n = 0; n < NT; ++n) fv[n] = lat_col<CB>(Kt, DK + (wc * NT + n) * 16, lane, T());
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n)

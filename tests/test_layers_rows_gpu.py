@@ -1,0 +1,44 @@
+"""Per-token kernels of layer-list prompts (csrc/kh_lops.h, kh_latent.h, kh_scan.h) and the attention of four sets of waves
+(csrc/kh_heads.h): rows with and without a remainder, segments shorter than the convolution, launches that leave CUs idle."""
+import pytest
+
+import layers_util as U
+
+pytestmark = pytest.mark.gpu
+BOTH = pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+
+
+def _prompt(mod, dtype, n, cuts, **kw):
+    m = mod.load(dtype, **kw)
+    toks = mod.tokens(n)
+    U.check(U.run_alone(m, toks, cuts), mod.logits(toks), dtype, f"{n} {cuts}")
+    m.close()
+
+
+@BOTH
+@pytest.mark.parametrize("q_rank,kv_rank,rot", [(1024, 512, 64), (2044, 40, 12), (2052, 36, 6), (2300, 260, 10), (1026, 64, 8)])
+def test_latent_rows(gpu, dtype, q_rank, kv_rank, rot):
+    """In registers, beyond them, quads that the rotated part does not fill, and rows that are no quads."""
+    _prompt(U.Model(U.config([U.latent(2, 20, rot, 28, kv_rank, q_rank, 0.3)], width=48, vocab=60)), dtype, 40, (7, 8, 30))
+
+
+@BOTH
+@pytest.mark.parametrize("inner,conv", [(72, 4), (75, 4), (2060, 4), (72, 2), (40, 6)])
+def test_convolution_state(gpu, dtype, inner, conv):
+    """Pieces of one, two and three tokens behind one another, where the state is made of the state before it."""
+    _prompt(U.Model(U.config([U.mamba(inner, 5, 3, conv), U.mamba(24, 3, 2, 4)], width=40, vocab=50)), dtype, 150, (1, 2, 4, 7, 70, 135))
+
+
+@BOTH
+@pytest.mark.parametrize("top", [4, 5, 8, 9])
+def test_rows_of_experts(gpu, dtype, top):
+    """Chosen rows in batches of four, with outputs that are no stored row among them."""
+    _prompt(U.Model(U.config([U.with_ff(U.mamba(), experts=9, identity=3, top=top, ff=20)], width=1100, vocab=60)), dtype, 33, (20,))
+
+
+@pytest.mark.parametrize("dim,vdim,window,n,cuts", [(128, 128, 40, 65, ()), (128, 128, 600, 700, (63, 64, 400)), (100, 90, 200, 300, (129,)),
+                                                    (128, 128, 700, 33, (1, 2)), (65, 128, 31, 200, (31, 190))])
+def test_heads_of_four_sets(gpu, dim, vdim, window, n, cuts):
+    """bf16 heads of 65 to 128 columns: fewer key tiles than sets, masks inside a set's tile, rows in front of the piece."""
+    layers = [U.windowed(8, 2, dim, vdim, 0.1, window, 20, 50.0), U.chunked(4, 1, dim, vdim, 0.1, window)]
+    _prompt(U.Model(U.gusorax(layers, width=64, vocab=70, positions=800)), "bfloat16", n, cuts, max_seq_len=800)
