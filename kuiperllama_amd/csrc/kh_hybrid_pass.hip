@@ -209,7 +209,6 @@ struct Runner {
     cv.taps = mb.taps;
     cv.p = ps.p;
     conv_launch<T>(s, cv, ps.chunks, ps.n_chunks);
-    hipLaunchKernelGGL(k_conv_state<T>, dim3((I + 255) / 256, ps.S), dim3(256), 0, s, cv);
     {
       LgArgs a = gemm(mb.x, hy.a1, mb.innerp, hy.a2, mb.rankp);
       a.n_split = mb.rankp;
@@ -241,6 +240,9 @@ struct Runner {
     sc.ldx = mb.innerp;
     sc.ldz = 2 * I;
     sc.ldo = mb.innerp;
+    sc.cx = cv.xz;
+    sc.conv = cv.state;
+    sc.taps = mb.taps;
     if (ps.n_multi_segs) {
       TRY((scan_launch<T, false>(s, sc, ps.n_multi_chunks)));
       hipLaunchKernelGGL(k_scan_carry<T>, dim3((unsigned)(((size_t)I * N + 255) / 256), ps.n_multi_segs), dim3(256), 0, s, sc,

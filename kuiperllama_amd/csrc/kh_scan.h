@@ -31,6 +31,10 @@ struct ScanArgs {
   const ScanChunk* chunks;
   PassTabs p;
   int C, N, ldx, ldz, ldo, gshift;
+  // with outputs: the last taps - 1 inputs of the convolution become its sequence's state, where a segment ends
+  const T* cx;           // [T][ldz]
+  float* conv;           // + slot * slot_stride: [taps - 1][C]
+  int taps;
 };
 
 template <int G>
@@ -39,7 +43,8 @@ __device__ __forceinline__ float scan_group_sum(float v) { return group_sum<G>(v
 // B and C rows of the chunk go to LDS: [n_tok][2 N].  A state costs 28 cycles of a wave a token (36 with its output), half of
 // them the exponential, a token about 200 more (loads, conversions, silu): NS states a lane share those.  Inputs are requested
 // U tokens ahead.  2048 tokens of 4096 x 16: 45 + 61 us with 8 states a lane, requests in front of their own tokens and the
-// library's exponential in the gate; 44 + 52 us with 16.
+// library's exponential in the gate; 44 + 52 us with 16.  The convolution's state is written here, 1.8 us, not by a launch of
+// its own, 4.7 and its start.
 template <class T, bool OUT, int NS, int G>
 __global__ __launch_bounds__(256) void k_scan(const ScanArgs<T> a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -128,6 +133,16 @@ __global__ __launch_bounds__(256) void k_scan(const ScanArgs<T> a) {
     }
   }
   if (!OUT && g == 0) a.dtsum[(size_t)blockIdx.y * a.C + c] = dts;
+  if (OUT && (ck.flags & 2) && g == 0) {
+    const int n = a.p.seg_n[ck.seg], last = ck.row0 + ck.n, m = a.taps - 1;
+    float* cs = a.conv + (size_t)slot * a.slot_stride + c;
+    for (int j = 0; j < m; ++j) {  // ascending: entry j reads entry j + n > j of the old state
+      float v = 0.f;
+      if (n - m + j >= 0) v = (float)a.cx[(size_t)(last - m + j) * a.ldz + c];
+      else if (!fresh) v = cs[(size_t)(j + n) * a.C];
+      cs[(size_t)j * a.C] = v;
+    }
+  }
 }
 
 // ends[k] (end of chunk k from zero) -> start state of chunk k, for every segment's chunks in order.
