@@ -71,13 +71,23 @@ struct LgCfg {
   static constexpr int LDS = (XS * BM + WS * BN) * 128;
 };
 
-// features f .. f + 3 of one token, f a multiple of four
-template <class T, int EPI>
-__device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 v) {
-  typedef Tile<T> TL;
-  if ((EPI == LG_T || EPI == LG_F32) && a.bias) {
+// biases of features f .. f + 3, f a multiple of four (no bias: zeros)
+template <int EPI>
+__device__ __forceinline__ f32x4 lg_bias(const LgArgs& a, int f) {
+  f32x4 b = f4_zero();
+  if (EPI == LG_SOFTPLUS || ((EPI == LG_T || EPI == LG_F32) && a.bias)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] += a.bias[f + i < a.N ? f + i : 0];
+    for (int i = 0; i < 4; ++i) b[i] = a.bias[f + i < a.N ? f + i : 0];
+  }
+  return b;
+}
+// features f .. f + 3 of one token, bias b
+template <class T, int EPI>
+__device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 v, const f32x4& b) {
+  typedef Tile<T> TL;
+  if (EPI == LG_T || EPI == LG_F32) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += b[i];
   }
   if (EPI == LG_T) {
     T* o = (T*)a.out + (size_t)blockIdx.z * a.o_z + (size_t)tok * a.ldo + f;
@@ -92,7 +102,7 @@ __device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 
     f32x4 y = v;
     if (EPI == LG_SOFTPLUS) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = softplus1(v[i] + a.bias[f + i < a.N ? f + i : 0]);
+      for (int i = 0; i < 4; ++i) y[i] = softplus1(v[i] + b[i]);
     } else if (EPI == LG_SOFTCAP) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) y[i] = a.cap > 0.f ? a.cap * tanhf(v[i] / a.cap) : v[i];
@@ -239,6 +249,13 @@ __global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
   else if (TM <= 4 && live == 3) loop(std::integral_constant<int, TM < 3 ? 1 : 3>{});
   else loop(std::integral_constant<int, TM>{});
   // ---- epilogue: lane (fr, fh) of tile (n, m): token mt0 + .. + fr, features f .. f + 3
+  auto feature = [&](int n) __attribute__((always_inline)) { return f0 + wn * (BN / WN) + n * 16 + 4 * fh; };
+  constexpr bool BIAS = EPI == LG_T || EPI == LG_F32 || EPI == LG_SOFTPLUS;
+  f32x4 bias[BIAS ? TN : 1];  // ahead of the stores: a load behind them waits for them
+  if constexpr (BIAS) {
+#pragma unroll
+    for (int n = 0; n < TN; ++n) bias[n] = lg_bias<EPI>(a, feature(n));
+  }
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
     const int tok = mt0 + (WM * m + wm) * 16 + fr;
@@ -255,7 +272,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
       }
     } else {
 #pragma unroll
-      for (int n = 0; n < TN; ++n) lg_store<T, EPI>(a, tok, f0 + wn * (BN / WN) + n * 16 + 4 * fh, acc[n][m]);
+      for (int n = 0; n < TN; ++n) lg_store<T, EPI>(a, tok, feature(n), acc[n][m], bias[BIAS ? n : 0]);
     }
   }
 }
