@@ -283,7 +283,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
 // with rounds that are less than 200 of 256 full it loses that), and 128 x 128 in five, from 129 tiles on (2048 x 2048, K 4096 /
 // 2048: 57 / 31 us as 512 workgroups of 64 x 128, 44 / 25 so; 144 tiles of 1100 tokens, K 4096 / 2048 43 / 24 -> 38 / 22; 128
 // tiles: 12.7 us instead of 9.9).  Experts gain nothing from either (130 us of gate and up with 256 x 256, 137 with 256 x 128): their
-// tiles are a third empty or wait for HBM.  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
+// tiles are a third empty or wait for HBM.  Where 64 x 64 leaves half of the CUs idle, 32 x 64: what one CU pulls is the time (160
+// features of K 4096, 2048 / 732 tokens: 25.2 / 24.0 -> 18.6 / 17.1 us).  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
 static inline int lg_group_bm(long rows, int groups) {
   const long per = rows / (groups > 0 ? groups : 1);
   return per > 64 ? 128 : (per > 24 ? 64 : 32);
@@ -327,7 +328,7 @@ int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, in
     if (t > 128 && t <= 256 && full(128)) KH_LG_WIDE(128, 128);
   }
   if (a.M > 64 && tiles(128, 128) >= 400) KH_LG_GO(128, 128, false);
-  if (a.M <= 32) KH_LG_GO(32, 64, false);
+  if (a.M <= 32 || tiles(64, 64) <= 128) KH_LG_GO(32, 64, false);
   if (tiles(64, 128) >= 400) KH_LG_GO(64, 128, false);
   KH_LG_GO(64, 64, false);
 #undef KH_LG_GO
