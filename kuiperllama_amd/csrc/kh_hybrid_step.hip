@@ -332,7 +332,7 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
       at.p.seg_slot = tb.slot;
       at.p.seg_pos0 = tb.pos;
       TRY(lat_attn_launch<T>(s, at, tiles, cp));
-      LdValuesArgs va{st.part, la.uv.w, st.v, la.H, std::max(1, std::min(cdiv(la.dvp, 16), cdiv(128, la.H * B))), st.nsplit,
+      LdValuesArgs va{st.part, la.uv.w, st.v, la.H, std::max(1, std::min(cdiv(la.dvp, 16), cdiv(256, la.H * B))), st.nsplit,
                       la.Rp, la.dvp, tb.pos};
       TRY(go(k_ld_values<T>, dim3(la.H * va.nwg, B), 256, vec_b<T>(la.Rp) + 256 * 16 + (size_t)la.Rp * 4, s, va));
     }

@@ -891,32 +891,61 @@ __global__ __launch_bounds__(256) void k_ld_absorb(const LdAbsorbArgs a) {
 // sum [256 / (C / 4) groups][C / 4], summed over the groups by the caller.  Returns 1 / sum of the weights and, in grp, the
 // number of groups.  fac: one factor per split, ns <= 256
 __device__ __forceinline__ float ld_merge_splits(const float* p, int ns, int C, float* fac, float* red, f32x4* sum, int& grp) {
-  float m = -INFINITY;
-  for (int s = threadIdx.x; s < ns; s += 256) m = fmaxf(m, p[(size_t)s * (C + 4) + C]);
-  m = block_max(m, red);
-  float l = 0.f;
-  for (int s = threadIdx.x; s < ns; s += 256) {
-    const float* ps = p + (size_t)s * (C + 4) + C;
-    const float f = __builtin_amdgcn_exp2f(ps[0] - m);  // an empty split: exp2(-inf) = 0
-    fac[s] = f;
-    l = __builtin_fmaf(f, ps[1], l);
-  }
-  l = block_sum(l, red);
   // column groups of four; 256 / (C / 4) thread groups share the splits and meet in LDS
-  const int c4 = C >> 2, g = (int)threadIdx.x / c4;
+  const int c4 = C >> 2, g = (int)threadIdx.x / c4, lane = threadIdx.x & 63;
   grp = c4 < 256 ? 256 / c4 : 1;
-  if (g < grp) {
-    for (int i = (int)threadIdx.x - g * c4; i < c4; i += 256) {
+  const int ahead = g < grp ? grp : 0;
+  constexpr int U = 8;
+  f32x4 x[U];
+  const int i0 = (int)threadIdx.x - g * c4;
+  auto request = [&](int i, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int k = s + j * grp;
+      x[j] = *(const f32x4*)(p + (size_t)(k < ns ? k : ns - 1) * (C + 4) + 4 * i);
+    }
+  };
+  float l;
+  const float* f;
+  if (ns <= 64) {  // uniform: every wave has all maxima and sums in its lanes, and no barrier before the columns
+    if (ahead) request(i0, g);
+    float mk = -INFINITY, lk = 0.f;
+    if (lane < ns) {
+      const float2 ml = *(const float2*)(p + (size_t)lane * (C + 4) + C);
+      mk = ml.x;
+      lk = ml.y;
+    }
+    const float m = wave_max(mk);
+    const float fk = lane < ns ? __builtin_amdgcn_exp2f(mk - m) : 0.f;  // an empty split: exp2(-inf) = 0
+    l = wave_sum(fk * lk);
+    float* own = fac + (threadIdx.x & ~63u);
+    own[lane] = fk;
+    f = own;
+  } else {
+    float m = -INFINITY;
+    for (int s = threadIdx.x; s < ns; s += 256) m = fmaxf(m, p[(size_t)s * (C + 4) + C]);
+    m = block_max(m, red);
+    l = 0.f;
+    for (int s = threadIdx.x; s < ns; s += 256) {
+      const float* ps = p + (size_t)s * (C + 4) + C;
+      const float fs = __builtin_amdgcn_exp2f(ps[0] - m);
+      fac[s] = fs;
+      l = __builtin_fmaf(fs, ps[1], l);
+    }
+    l = block_sum(l, red);
+    f = fac;
+    if (ahead) request(i0, g);
+  }
+  if (ahead) {
+    for (int i = i0; i < c4; i += 256) {
+      if (i != i0) request(i, g);
       f32x4 v = f4_zero();
-      int s = g;
-      for (; s + 7 * grp < ns; s += 8 * grp) {
-        f32x4 x[8];
+      for (int s = g; s < ns; s += U * grp) {
+        if (s != g) request(i, s);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = *(const f32x4*)(p + (size_t)(s + j * grp) * (C + 4) + 4 * i);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v = fma_s(fac[s + j * grp], x[j], v);
+        for (int j = 0; j < U; ++j)
+          if (s + j * grp < ns) v = fma_s(f[s + j * grp], x[j], v);
       }
-      for (; s < ns; s += grp) v = fma_s(fac[s], *(const f32x4*)(p + (size_t)s * (C + 4) + 4 * i), v);
       sum[g * c4 + i] = v;
     }
   }
@@ -925,6 +954,9 @@ __device__ __forceinline__ float ld_merge_splits(const float* p, int ns, int C, 
 }
 
 // ---- k_ld_values: merge of the time splits, then W_uv of the head.  grid (H nwg, B) ----------------------------------
+// A chain of trips (position; maxima, sums and columns of the splits; W_uv beside them), so a head is cut until the launch has 256
+// workgroups or a wave one group of rows: 4 x 16 heads of 128 over 512 latents and 10 splits 7.2 us with the maxima and sums behind
+// barriers of their own in front of the columns, 6.9 with both at once, 5.5 with 256 workgroups instead of 128.
 struct LdValuesArgs {
   const float* part;  // [B H][nsplit][Rp + 4]
   const void* uv;     // [H][dvp][Rp]
