@@ -199,7 +199,7 @@ typedef struct kh_config {
   int32_t family, rope_mode, cache_len;
   float rope_theta, rms_eps;
   int64_t weight_bytes; /* bytes of the weight arena resident in HBM */
-  int32_t launches_per_token; /* 5 per layer + classifier + sampler */
+  int32_t launches_per_token; /* .bin models: 5 per layer + classifier + sampler */
   /* Self-checks run once at the end of kh_model_create_* (csrc/kh_model_selftest.hip), about a millisecond:
    *   ring_selftest        the int8 LDS-DMA ring kernels against the register-tile kernels of the same launches on
    *                        this model's own weights: 0 = no ring kernel planned (fp32, geometry, KH_RING=0) or skipped,

@@ -42,3 +42,23 @@ def test_heads_of_four_sets(gpu, dim, vdim, window, n, cuts):
     """bf16 heads of 65 to 128 columns: fewer key tiles than sets, masks inside a set's tile, rows in front of the piece."""
     layers = [U.windowed(8, 2, dim, vdim, 0.1, window, 20, 50.0), U.chunked(4, 1, dim, vdim, 0.1, window)]
     _prompt(U.Model(U.gusorax(layers, width=64, vocab=70, positions=800)), "bfloat16", n, cuts, max_seq_len=800)
+
+
+@pytest.mark.parametrize("dtype,n", [("float32", 1024), ("bfloat16", 2048)])
+def test_latent_steps_of_many_splits(gpu, dtype, n):
+    """Steps of one and of four sequences around 64 filled splits of one key tile, in lanes and beyond them."""
+    import numpy as np
+    mod = U.Model(U.config([U.latent(3, 20, 8, 28, 72, 40, 0.4)], width=40, vocab=50))
+    m = mod.load(dtype, max_seq_len=n + 16)
+    toks = mod.tokens(n + 3)
+    want = mod.logits(toks)
+    for others in (0, 3):
+        s = m.open_seq()
+        rest = [m.open_seq() for _ in range(others)]
+        m.forward([(s, toks[:n - 2], [n - 3])])
+        for i in range(n - 2, n + 3):
+            got = m.forward([(s, [toks[i]], [0])] + [(r, [toks[i]], [0]) for r in rest])
+            U.check(np.asarray(got)[:1], want[i:i + 1], dtype, f"{i} {others}")
+        for r in [s] + rest:
+            m.close_seq(r)
+    m.close()
