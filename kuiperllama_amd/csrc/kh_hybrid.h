@@ -240,6 +240,7 @@ int hy_decode_max(const kh_model* m);  // sequences the fused step can take at o
 int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits);
 struct HyTail {  // device lists of the wanted tokens of a pass: their rows, ids, positions, slots
   const int32_t *rows, *tok, *pos, *slot;
+  bool mates;  // several of them are one sequence's
 };
 bool hy_tail_pays(const kh_model* m, int T, int want);
 int hy_tail(kh_model* m, const HyTail& t, int n, float* h_logits);

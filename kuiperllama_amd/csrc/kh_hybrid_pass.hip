@@ -555,6 +555,8 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
     o.wtok = of_wanted([&](size_t r) { return tok[r]; });
     o.wpos = of_wanted([&](size_t r) { return pos[r]; });
     o.wslot = of_wanted([&](size_t r) { return slot[(size_t)seg[r]]; });
+    for (size_t i = 1; i < wr.size(); ++i)  // ascending rows, one segment per sequence
+      p.wanted.mates = p.wanted.mates || seg[(size_t)wr[i]] == seg[(size_t)wr[i - 1]];
     for (const RowKind& kd : kinds) {
       RowTiles t{kd, row_tiles(sn, kd, &lt), 0, (int)lt.size() / 2};
       t.off = tb.put(lt);
@@ -591,7 +593,7 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
     p.multi0 = b + o.m0;
     p.multin = b + o.mn;
     p.want = b + o.want;
-    p.wanted = HyTail{b + o.want, b + o.wtok, b + o.wpos, b + o.wslot};
+    p.wanted = HyTail{b + o.want, b + o.wtok, b + o.wpos, b + o.wslot, p.wanted.mates};
     TRY(hy.f32 ? run_pass<float>(m, p, out) : run_pass<bf16>(m, p, out));
     if (out) out += (size_t)p.n_want * hy.c.vocab;
   }

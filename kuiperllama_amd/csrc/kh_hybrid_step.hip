@@ -115,9 +115,10 @@ int split_waves(int rows, int nblk) {
 // One token of B sequences: tables at (tok, pos, slot); logits to `logits` [B][V]; argmax partials of sequence 0 to
 // the model's sampler buffers.
 // tail: the last layer run only, behind a pass that has left the residual rows in front of it in x[0] (complete: nothing of a
-// loop's entry is missing) and, where its mixer is a scan, that one's outputs in v.
+// loop's entry is missing) and, where its mixer is a scan, that one's outputs in v.  mates: several of the tokens are one
+// sequence's (of a tail alone): one attends over another's cache row.
 template <class T, int B>
-int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
+int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false, bool mates = false) {
   Hybrid& hy = *m->hy;
   Hybrid::Step& st = *hy.step_st;
   hipStream_t s = m->stream;
@@ -273,18 +274,27 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
         a.row = la.row();
         a.dims = la.dims;
       }
-      TRY(with_nv<T, 256>(Wp, [&](auto nv) {
-        return with_rp(f.top ? f.n_out() : 1, [&](auto rp) {
-          constexpr int NV = decltype(nv)::value, RP = decltype(rp)::value;
-          const dim3 grid(a.att.nwg + B * a.top * a.nwg_e + a.nwg_m + extra);
-          if constexpr (B > 1) {
-            if (share && heads) return go(k_ld_mid<T, B, NV, RP, true, true>, grid, 256, lds, s, a);
-            if (share) return go(k_ld_mid<T, B, NV, RP, true, false>, grid, 256, lds, s, a);
-          }
-          if (heads) return go(k_ld_mid<T, B, NV, RP, false, true>, grid, 256, lds, s, a);
-          return go(k_ld_mid<T, B, NV, RP, false, false>, grid, 256, lds, s, a);
+      auto launch = [&](const LdMidArgs& a, int extra) {
+        return with_nv<T, 256>(Wp, [&](auto nv) {
+          return with_rp(f.top ? f.n_out() : 1, [&](auto rp) {
+            constexpr int NV = decltype(nv)::value, RP = decltype(rp)::value;
+            const dim3 grid(a.att.nwg + B * a.top * a.nwg_e + a.nwg_m + extra);
+            if constexpr (B > 1) {
+              if (share && heads) return go(k_ld_mid<T, B, NV, RP, true, true>, grid, 256, lds, s, a);
+              if (share) return go(k_ld_mid<T, B, NV, RP, true, false>, grid, 256, lds, s, a);
+            }
+            if (heads) return go(k_ld_mid<T, B, NV, RP, false, true>, grid, 256, lds, s, a);
+            return go(k_ld_mid<T, B, NV, RP, false, false>, grid, 256, lds, s, a);
+          });
         });
-      }));
+      };
+      if (mates && a.att.nwg) {  // the cache rows alone, ahead of the launch that reads them
+        LdMidArgs rows = a;
+        rows.att.nwg = rows.top = 0;
+        TRY(launch(rows, extra));
+        extra = 0;
+      }
+      TRY(launch(a, extra));
     }
     if (mixed || (heads && ha.beside)) {
     } else if (mamba) {
@@ -375,13 +385,13 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false) {
   return with_nv<T, kLdNorm>(Wp, [&](auto nv) { return go(k_ld_head<T, B, decltype(nv)::value>, dim3(st.head_wg), ld_in_wg(B, decltype(nv)::value), B * vec_b<T>(Wp), s, h); });
 }
 template <class T>
-int step_b(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail) {
+int step_b(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail, bool mates) {
   if (B == 1) return step<T, 1>(m, tb, logits, tail);
-  if (B == 2) return step<T, 2>(m, tb, logits, tail);
-  return step<T, 4>(m, tb, logits, tail);
+  if (B == 2) return step<T, 2>(m, tb, logits, tail, mates);
+  return step<T, 4>(m, tb, logits, tail, mates);
 }
-int step_any(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail = false) {
-  return m->hy->f32 ? step_b<float>(m, B, tb, logits, tail) : step_b<bf16>(m, B, tb, logits, tail);
+int step_any(kh_model* m, int B, const LdTabs& tb, float* logits, bool tail = false, bool mates = false) {
+  return m->hy->f32 ? step_b<float>(m, B, tb, logits, tail, mates) : step_b<bf16>(m, B, tb, logits, tail, mates);
 }
 // rows of the residual stream, and of a scan's outputs (mix nullptr: none), to the step's buffers; grid (rows of the step)
 template <class T>
@@ -520,7 +530,7 @@ int hy_tail(kh_model* m, const HyTail& t, int n, float* h_logits) {
     };
     if (hy.f32) rows(0.f);
     else rows((bf16)0.f);
-    TRY(step_any(m, B, tb, st.logits, true));
+    TRY(step_any(m, B, tb, st.logits, true, t.mates));
     KH_CHECK_HIP(hipMemcpyAsync(h_logits + (size_t)i * hy.c.vocab, st.logits, (size_t)B * hy.c.vocab * 4, hipMemcpyDeviceToHost, m->stream));
     i += B;
   }

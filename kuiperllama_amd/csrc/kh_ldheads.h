@@ -9,7 +9,9 @@
 //   softmax   wave w has head w: a lane per key, running maximum and sum over the tiles of 64
 //   values    16 bytes of a row per thread, all four heads; the rows of a wave meet by lane swaps, the waves in LDS
 // The newest key and value come from the projected row, not from the cache row that another workgroup of the launch is writing;
-// they are rounded as that one is.  Everything else is fp32.
+// they are rounded as that one is.  Everything else is fp32.  Older keys come from the cache: no two tokens of a launch that also
+// writes cache rows are one sequence's.  Where several of a prompt's tokens take the last layer together, a launch of the cache rows
+// alone comes first (kh_hybrid_step.hip, `mates`).
 // A layer has a fixed number of splits, and how long they are follows from the position: a sequence's bits are its own.  The
 // last split of a group to arrive merges them all, in their order (kh_attn.h::attn_publish_barrier has the hand-over).
 #pragma once
