@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void k_scan(const ScanArgs<T> a) {
   request(0);
   float A2[NS], S[NS];
   const size_t sbase = (size_t)cc * N;
-  const bool first = ck.flags & 1;
+  const bool alone = (ck.flags & 3) == 3;
   const int slot = a.p.seg_slot[ck.seg];
   float* st = a.state + (size_t)slot * a.slot_stride + sbase;
   const bool fresh = a.p.seg_pos0[ck.seg] == 0;
@@ -86,7 +86,9 @@ __global__ __launch_bounds__(256) void k_scan(const ScanArgs<T> a) {
     A2[j] = n < N ? a.A2[sbase + n] : 0.f;
     S[j] = 0.f;
     if (OUT && n < N) {
-      if (!first) S[j] = a.ends[(size_t)blockIdx.y * a.C * N + sbase + n];  // start state (k_scan_carry)
+      // start state: a segment of several chunks has all of them from k_scan_carry, its first too - the last one's workgroup
+      // writes the slot's state in this launch
+      if (!alone) S[j] = a.ends[(size_t)blockIdx.y * a.C * N + sbase + n];
       else if (!fresh) S[j] = st[n];
     }
   }

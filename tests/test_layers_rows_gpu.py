@@ -62,3 +62,19 @@ def test_latent_steps_of_many_splits(gpu, dtype, n):
         for r in [s] + rest:
             m.close_seq(r)
     m.close()
+
+
+@BOTH
+@pytest.mark.parametrize("inner,state", [(72, 5), (2050, 16)])
+def test_scans_that_continue(gpu, dtype, inner, state):
+    """Pieces of several chunks behind others, of two and of one chunk more: the same bits every time."""
+    import numpy as np
+    mod = U.Model(U.config([U.mamba(inner, state, 3, 4), U.mamba(24, 3, 2, 4)], width=40, vocab=50))
+    toks = mod.tokens(330)
+    want = mod.logits(toks)
+    m = mod.load(dtype)
+    out = [U.run_alone(m, toks, (70, 199, 200, 265)) for _ in range(5)]
+    m.close()
+    U.check(out[0], want, dtype)
+    for o in out[1:]:
+        np.testing.assert_array_equal(o, out[0])
