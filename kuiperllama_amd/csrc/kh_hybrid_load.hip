@@ -750,7 +750,8 @@ int finish(kh_model* m, Plan& pl) {
     const int keys = span > 0 ? std::min(span, CL) : CL;
     a.nsplit = 2;
     while (a.nsplit < 128 && a.nsplit * KH_LAT_SPLIT_MIN < keys && a.nsplit * a.G < 512) a.nsplit *= 2;
-    a.beside = ldh_fits(keys, a.dkp, a.dvp) && !dbg_off("KH_HY_BESIDE") ? ldh_splits(a.G * a.chunks()) : 0;
+    const int groups = a.G * a.chunks();
+    a.beside = ldh_fits(keys, groups, a.dkp, a.dvp, hy.elem()) && !dbg_off("KH_HY_BESIDE") ? ldh_splits(groups) : 0;
     if ((double)a.ring * a.row() * hy.elem() >= 4294967296.0) return KH_ERR_UNSUPPORTED;  // 32-bit offsets within a run
   }
   build_runs(hy);

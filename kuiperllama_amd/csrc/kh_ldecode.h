@@ -7,7 +7,8 @@
 //             heads: cache row, attention (kh_ldheads.h)
 //   mamba     k_ld_scan   dt projection, softplus, one step of the selective scan, gate
 //   latent    k_ld_absorb W_uk^T q per head, rotation ; k_latent_attn (time splits) ; k_ld_values merge + W_uv per head
-//   heads     of more than 128 elements or over more than 4096 keys: k_heads_attn (time splits) ; k_ld_merge merge and output gate
+//   heads     of more than 128 elements or over more keys than kh_ldheads.h takes: k_heads_attn (time splits) ; k_ld_merge merge
+//             and output gate
 //   k_ld_out  W_o . v (+ bias) + experts' down + shared down + identity experts, times the residual multiplier, +
 //             residual: one dot product per row over a concatenation of weight rows
 // A loop that enters through a matrix: k_ld_enter in front of each pass.  Then k_ld_head (final norm, head, soft cap,

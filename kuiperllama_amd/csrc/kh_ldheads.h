@@ -21,7 +21,7 @@
 namespace khm {
 
 #define KH_LDH_SPLITS 16   // splits of a group, at most (a power of two)
-#define KH_LDH_KEYS 4096   // visible keys up to which 16 splits are enough (256 keys: four tiles, 8 us in fp32)
+#define KH_LDH_WGS 128     // workgroups of a sequence, at most
 #define KH_LDH_DIM 128     // key and value size that a thread's registers are laid out for
 
 struct LdHeads {
@@ -39,13 +39,26 @@ struct LdHeads {
 constexpr int kLdhPart = KH_LDH_DIM + 4;  // o, m, l of one head in one split
 constexpr size_t kLdhLds = (4 * KH_LDH_DIM + 4 * 64 + 64 * 4 + 16 + 16 * KH_LDH_DIM) * 4;
 
-// Does a layer's attention run this way?  keys: the most that any position sees.
-__host__ __device__ inline bool ldh_fits(int keys, int dkp, int dvp) { return keys <= KH_LDH_KEYS && dkp <= KH_LDH_DIM && dvp <= KH_LDH_DIM; }
-// splits: 256 workgroups a sequence at most, most of which leave at once while the sequence is short
+// Workgroups of a sequence stand in front of the experts' in any case, most of them to leave at once while the sequence is short,
+// and a split's tiles of 64 keys are a chain: so 128 workgroups a sequence, and this route for as many visible keys as its splits
+// take 256 of each, in bf16 with less than 16 splits (more than 8 groups of four heads) 128.  Four layers of width 1024 with 7 of
+// 32 experts of 512, heads of 128 over visible keys of that bound, us a step in launches of its own / so, one and four sequences:
+//   keys                          30                       300                      1000                    4000
+//   8 heads on 2, bf16     127 / 101  177 / 137     126 / 110  174 / 139     123 / 112  175 / 141    136 / 134  202 / 160
+//   32 on 8, fp32          175 / 143  242 / 223     178 / 144  251 / 227     177 / 145  282 / 232    208 / 180  392 / 292
+//   64 on 16, bf16         184 / 142  237 / 210     173 / 149  242 / 212     171 / 162  277 / 207
+// Beyond: 64 on 16 as 256 workgroups a sequence 230 / 250 at 30 keys, four sequences; in bf16 with 256 keys a split, one
+// sequence at the last of them 163 / 168 (32 on 16, eight splits), 171 / 182 (32 on 32, four); 128 heads of 64 on 128 as one split,
+// 4000 keys 262 / 528 and 616 / 977.
 __host__ __device__ inline int ldh_splits(int groups) {
   int n = KH_LDH_SPLITS;
-  while (n > 1 && n * groups > 256) n >>= 1;
+  while (n > 1 && n * groups > KH_LDH_WGS) n >>= 1;
   return n;
+}
+// Does a layer's attention run this way?  keys: the most that any position sees.
+inline bool ldh_fits(int keys, int groups, int dkp, int dvp, size_t elem) {
+  const int splits = ldh_splits(groups), each = elem == 2 && splits < KH_LDH_SPLITS ? 128 : 256;
+  return keys <= each * splits && dkp <= KH_LDH_DIM && dvp <= KH_LDH_DIM;
 }
 // keys of a split: at least 32 KB of a group's keys and values of 128, in whole steps of 16
 template <class T>

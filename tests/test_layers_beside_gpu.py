@@ -65,6 +65,26 @@ def test_most_keys(gpu, dtype, rows, beside):
     m.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dtype,keys,most", [
+    (8, 8, "bfloat16", 4096, 4096), (9, 9, "bfloat16", 1024, 1024), (9, 9, "float32", 2048, 2048), (36, 4, "bfloat16", 1024, 1024),
+    (33, 33, "float32", 512, 512), (33, 33, "bfloat16", 256, 256), (65, 65, "float32", 256, 256), (130, 65, "bfloat16", 128, 128)])
+def test_more_groups_than_splits_for_them(gpu, heads, kv_heads, dtype, keys, most):
+    """The bound follows the splits, which many groups of heads share: at the bound beside the experts, above it as launches of
+    their own; steps up to it, and behind a window that has moved on."""
+    for window, launches in ((keys, 5), (keys + 1, 7)):
+        kw = dict(heads=heads, kv_heads=kv_heads, dim=6, vdim=5)
+        mod = U.Model(U.gusorax([dict(U.windowed(window=window, rows=8, far=60.0, **kw), mlp=U.clamped())], positions=4400))
+        m = mod.load(dtype, max_seq_len=min(max(2 * most, 300), 4400), max_seqs=4)
+        assert m.cfg.launches_per_token == launches
+        if most <= 512:
+            toks = mod.tokens(most + 40)
+            want = mod.logits(toks)
+            for at in ([most - 3], [0, 30, most // 2, most + 20]):
+                for k, g in zip(at, steps(m, toks, at, 6)):
+                    U.check(g, want[k: k + 6], dtype, f"{window} {at} {k}")
+        m.close()
+
+
 def test_fences_give_the_same_bits(gpu):
     """The hand-over of the splits with release and acquire fences and without, many steps beside a stream of experts."""
     mod = U.Model(U.gusorax([dict(U.windowed(heads=8, kv_heads=2, dim=128, vdim=128, window=400, rows=16, far=90.0),
