@@ -2,7 +2,8 @@
 
     python -m kuiperllama_amd.build [--force]
 
-Output: kuiperllama_amd/lib/libkuiper_hip.so (git-ignored, shipped to the GPU box by gpurun).
+Output: kuiperllama_amd/lib/libkuiper_hip.so, and beside it the operator calls of kuiperllama_amd.ops as an extension of this
+interpreter, where its headers are installed (both git-ignored).
 """
 from __future__ import annotations
 
@@ -10,12 +11,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_PKG, "csrc")
 LIB_DIR = os.path.join(_PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libkuiper_hip.so")
-PYOPS_PATH = os.path.join(LIB_DIR, "kh_pyops.so")
+# code for one interpreter's ABI, which its name says
+PYOPS_PATH = os.path.join(LIB_DIR, "kh_pyops" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 SOURCES = ["kh_ops.hip", "kh_model_load.hip", "kh_model_step.hip", "kh_model_prefill.hip", "kh_model_pair.hip", "kh_model_profile.hip", "kh_model_selftest.hip",
            "kh_hybrid_load.hip", "kh_hybrid_pass.hip", "kh_hybrid_step.hip", "kh_heads.hip",
            "kh_tokenizer.cpp", "kh_bpe.cpp", "kh_debug.cpp"]
@@ -46,21 +49,30 @@ def _stale() -> bool:
     return False
 
 
-def build_pyops(force: bool = False) -> str:
-    """The operator calls without ctypes (csrc/kh_pyops.c): a CPython extension that needs the interpreter's headers alone."""
-    import sysconfig
+def build_pyops(force: bool = False) -> str | None:
+    """The operator calls without ctypes (csrc/kh_pyops.c): a CPython extension that needs the interpreter's headers alone.
+    None, and a line on stderr, without them: the library and its models do not need it, kuiperllama_amd.ops does."""
     src = os.path.join(CSRC, "kh_pyops.c")
     if not force and os.path.exists(PYOPS_PATH) and os.path.getmtime(src) <= os.path.getmtime(PYOPS_PATH):
         return PYOPS_PATH
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"kuiperllama_amd.build: no Python.h in {include}: the operator calls (kuiperllama_amd.ops) are not built", file=sys.stderr)
+        return None
     os.makedirs(LIB_DIR, exist_ok=True)
-    subprocess.check_call([shutil.which("gcc") or _hipcc(), "-O2", "-std=gnu11", "-shared", "-fPIC", "-Wall",
-                           f"-I{sysconfig.get_paths()['include']}", src, "-o", PYOPS_PATH])
+    part = f"{PYOPS_PATH}.{os.getpid()}"  # whole before it has the name that is loaded
+    try:
+        subprocess.check_call([shutil.which("gcc") or _hipcc(), "-O2", "-std=gnu11", "-shared", "-fPIC", "-Wall", f"-I{include}", src, "-o", part])
+        os.replace(part, PYOPS_PATH)
+    finally:
+        if os.path.exists(part):
+            os.remove(part)
     return PYOPS_PATH
 
 
 def build_lib(force: bool = False, verbose: bool = False) -> str:
-    build_pyops(force)
     if not force and not _stale():
+        build_pyops()
         return LIB_PATH
     os.makedirs(LIB_DIR, exist_ok=True)
     objs, procs = [], []
@@ -83,6 +95,7 @@ def build_lib(force: bool = False, verbose: bool = False) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    build_pyops(force)  # behind the library, which it is no part of
     return LIB_PATH
 
 

@@ -48,10 +48,11 @@ class _Unbound:
         import ctypes as C
         import importlib.machinery
         import importlib.util
+        from .build import PYOPS_PATH as path
         L = _ffi.lib()
-        path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "kh_pyops.so")
         if not os.path.exists(path):
-            raise ImportError(f"{path} is missing: build it with `python -m kuiperllama_amd.build`")
+            raise ImportError(f"{path} is missing: build it with `python -m kuiperllama_amd.build`, which needs this "
+                              "interpreter's headers")
         spec = importlib.util.spec_from_loader("kh_pyops", importlib.machinery.ExtensionFileLoader("kh_pyops", path))
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
