@@ -162,20 +162,30 @@ static MmShape mm_shape(bool quant, int M, int K) {
   return s;
 }
 
-#define KH_MM_SPLITS(GO, sh, UU, MV)      \
-  if ((sh).mv == MV) {                    \
-    if ((sh).split == 1) GO(UU, MV, 1);   \
-    else if ((sh).split == 2) GO(UU, MV, 2); \
-    else GO(UU, MV, 4);                   \
+// The (U, MAXV, SPLIT) that mm_shape comes to, over all lengths and numbers of rows; nothing else is compiled.
+#define KH_MM_FORMS_F32(X)                                                                                                  \
+  X(2, 1, 1) X(4, 1, 1) X(4, 2, 1) X(4, 2, 2) X(4, 4, 2) X(4, 4, 4) X(8, 2, 1) X(8, 4, 1) X(8, 4, 2) X(8, 4, 4) X(8, 6, 1) \
+  X(8, 6, 2) X(8, 6, 4) X(8, 0, 1) X(8, 0, 2) X(8, 0, 4)
+#define KH_MM_FORMS_Q8(X)                                                                                                   \
+  X(2, 1, 1) X(2, 2, 1) X(2, 4, 2) X(2, 4, 4) X(4, 4, 1) X(4, 4, 2) X(4, 6, 1) X(4, 6, 2) X(4, 6, 4) X(4, 0, 1) X(4, 0, 2)  \
+  X(4, 0, 4)
+
+extern "C" int kh_plan_matmul(int32_t is_quant, int32_t M, int32_t K, int32_t* out5) {
+  if (!out5 || M <= 0 || K <= 0) return KH_ERR_INVALID_ARG;
+  if (is_quant ? M % 16 || kh_q8_lds_bytes(M) + 16 > 64 * 1024 : M % 4 || (size_t)M * 4 + 16 > 64 * 1024) return KH_ERR_UNSUPPORTED;
+  const MmShape sh = mm_shape(is_quant != 0, M, K);
+  const int32_t o[5] = {sh.u, sh.mv, sh.split, sh.wg, sh.grid};
+  for (int i = 0; i < 5; ++i) out5[i] = o[i];
+#define KH_MM(UU, MV, SP) \
+  if (sh.u == UU && sh.mv == MV && sh.split == SP) return KH_OK;
+  if (is_quant) {
+    KH_MM_FORMS_Q8(KH_MM)
+  } else {
+    KH_MM_FORMS_F32(KH_MM)
   }
-#define KH_MM_TILES(GO, sh, UU)  \
-  if ((sh).u == UU) {            \
-    KH_MM_SPLITS(GO, sh, UU, 1)  \
-    KH_MM_SPLITS(GO, sh, UU, 2)  \
-    KH_MM_SPLITS(GO, sh, UU, 4)  \
-    KH_MM_SPLITS(GO, sh, UU, 6)  \
-    KH_MM_SPLITS(GO, sh, UU, 0)  \
-  }
+#undef KH_MM
+  return KH_ERR_INTERNAL;
+}
 
 extern "C" int kh_matmul_f32(const float* x, const float* w, float* y, int32_t M, int32_t K,
                              float scale, void* stream) {
@@ -189,13 +199,14 @@ extern "C" int kh_matmul_f32(const float* x, const float* w, float* y, int32_t M
     return kh_launch_status();
   }
   const MmShape sh = mm_shape(false, M, K);
-#define KH_MM(UU, MV, SP) \
-  hipLaunchKernelGGL((k_matmul_f32<UU, MV, SP>), dim3(sh.grid), dim3(sh.wg), sh.lds, s, x, w, y, M, K, scale)
-  KH_MM_TILES(KH_MM, sh, 8)
-  KH_MM_TILES(KH_MM, sh, 4)
-  KH_MM_TILES(KH_MM, sh, 2)
+#define KH_MM(UU, MV, SP)                                                                                                        \
+  if (sh.u == UU && sh.mv == MV && sh.split == SP) {                                                                           \
+    hipLaunchKernelGGL((k_matmul_f32<UU, MV, SP>), dim3(sh.grid), dim3(sh.wg), sh.lds, s, x, w, y, M, K, scale);               \
+    return kh_launch_status();                                                                                                 \
+  }
+  KH_MM_FORMS_F32(KH_MM)
 #undef KH_MM
-  return kh_launch_status();
+  return KH_ERR_INTERNAL;
 }
 
 // =============================================================================================
@@ -269,12 +280,14 @@ extern "C" int kh_matmul_q8(const float* x, const int8_t* w8, const float* scale
     return kh_launch_status();
   }
   const MmShape sh = mm_shape(true, M, K);
-#define KH_MMQ(UU, MV, SP)                                                                                              \
-  hipLaunchKernelGGL((k_matmul_q8<UU, MV, SP>), dim3(sh.grid), dim3(sh.wg), sh.lds, s, x, w8, scales, gshift, y, M, K)
-  KH_MM_TILES(KH_MMQ, sh, 4)
-  KH_MM_TILES(KH_MMQ, sh, 2)
-#undef KH_MMQ
-  return kh_launch_status();
+#define KH_MM(UU, MV, SP)                                                                                                        \
+  if (sh.u == UU && sh.mv == MV && sh.split == SP) {                                                                           \
+    hipLaunchKernelGGL((k_matmul_q8<UU, MV, SP>), dim3(sh.grid), dim3(sh.wg), sh.lds, s, x, w8, scales, gshift, y, M, K);      \
+    return kh_launch_status();                                                                                                 \
+  }
+  KH_MM_FORMS_Q8(KH_MM)
+#undef KH_MM
+  return KH_ERR_INTERNAL;
 }
 
 // =============================================================================================

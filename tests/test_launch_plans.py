@@ -227,3 +227,19 @@ def test_attention_over_heads_fits_a_cu(sets):
             assert lds <= 160 * 1024, (key, value, sets, table, lds)
             stages, rest = divmod(lds - (table if table <= 32768 else 0), sets * 64 * pad)
             assert rest == 0 and stages in (2, 3)
+
+
+@pytest.mark.parametrize("quant,step,most,forms", [(False, 4, 16380, 16), (True, 16, 16352, 12)])
+def test_every_matmul_has_its_kernel(quant, step, most, forms):
+    """kh_matmul_f32 / kh_matmul_q8: every length of the vector path and every split has a compiled kernel, and no more are
+    compiled than some length reaches.  Rows around the numbers where the split changes: 2048 and 4096 waves have work."""
+    seen = set()
+    for M in range(step, most + 1, step):
+        for K in (1, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 1 << 20):
+            p = _ffi.plan_matmul(quant, M, K)
+            assert p["wg"] // 64 % p["split"] == 0 and p["grid"] * (p["wg"] // 64) <= 4096 * p["split"], (M, K, p)
+            assert p["staged"] == 0 or 4 * p["staged"] * p["wg"] >= M, (M, K, p)
+            seen.add((p["u"], p["staged"], p["split"]))
+    assert len(seen) == forms
+    with pytest.raises(_ffi.KhError):
+        _ffi.plan_matmul(quant, most + step, 1)
