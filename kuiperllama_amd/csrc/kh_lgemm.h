@@ -71,23 +71,31 @@ struct LgCfg {
   static constexpr int LDS = (XS * BM + WS * BN) * 128;
 };
 
+// Biases ahead of the stores, because a load behind them waits for them (LG_SOFTPLUS, 2048 x 4096 of K 128 in bf16 28.7 -> 23.7 us)?
+// Not in fp32 outside LG_SOFTPLUS: there the loop's registers come out differently, and 64 x 64 tiles are slower as a whole (606
+// tokens x 2048 of K 7168 241 -> 257 us, x 3072 of K 2048 75.4 -> 79.4; 2048 x 1024 of K 3584 130 -> 138), 64 x 128 2 % faster.
+template <class T, int EPI>
+constexpr bool lg_bias_first() { return EPI == LG_SOFTPLUS || (sizeof(T) == 2 && (EPI == LG_T || EPI == LG_F32)); }
 // biases of features f .. f + 3, f a multiple of four (no bias: zeros)
 template <int EPI>
 __device__ __forceinline__ f32x4 lg_bias(const LgArgs& a, int f) {
   f32x4 b = f4_zero();
-  if (EPI == LG_SOFTPLUS || ((EPI == LG_T || EPI == LG_F32) && a.bias)) {
+  if (EPI == LG_SOFTPLUS || a.bias) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) b[i] = a.bias[f + i < a.N ? f + i : 0];
   }
   return b;
 }
-// features f .. f + 3 of one token, bias b
+// features f .. f + 3 of one token; b: their biases, where they come first
 template <class T, int EPI>
 __device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 v, const f32x4& b) {
   typedef Tile<T> TL;
-  if (EPI == LG_T || EPI == LG_F32) {
+  if (lg_bias_first<T, EPI>() && EPI != LG_SOFTPLUS) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] += b[i];
+  } else if ((EPI == LG_T || EPI == LG_F32) && a.bias) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += a.bias[f + i < a.N ? f + i : 0];
   }
   if (EPI == LG_T) {
     T* o = (T*)a.out + (size_t)blockIdx.z * a.o_z + (size_t)tok * a.ldo + f;
@@ -250,8 +258,8 @@ __global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
   else loop(std::integral_constant<int, TM>{});
   // ---- epilogue: lane (fr, fh) of tile (n, m): token mt0 + .. + fr, features f .. f + 3
   auto feature = [&](int n) __attribute__((always_inline)) { return f0 + wn * (BN / WN) + n * 16 + 4 * fh; };
-  constexpr bool BIAS = EPI == LG_T || EPI == LG_F32 || EPI == LG_SOFTPLUS;
-  f32x4 bias[BIAS ? TN : 1];  // ahead of the stores: a load behind them waits for them
+  constexpr bool BIAS = lg_bias_first<T, EPI>();
+  f32x4 bias[BIAS ? TN : 1];
   if constexpr (BIAS) {
 #pragma unroll
     for (int n = 0; n < TN; ++n) bias[n] = lg_bias<EPI>(a, feature(n));
