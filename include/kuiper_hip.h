@@ -205,7 +205,8 @@ typedef struct kh_config {
    *                        this model's own weights: 0 = no ring kernel planned (fp32, geometry, KH_RING=0) or skipped,
    *                        1 = outputs identical, -1 = mismatch: this model runs the register-tile kernels;
    *   attn_merge_selftest  the fence-free in-launch merge of the decode-attention time splits against the fenced
-   *                        form: 0 = not applicable (no time splits in this cache) or skipped, 1 = identical,
+   *                        form (layer-list models: the splits that a launch with experts merges, csrc/kh_ldheads.h):
+   *                        0 = not applicable (no time splits in this cache) or skipped, 1 = identical,
    *                        -1 = mismatch: this model uses the fenced form, 2 = the fenced form was requested
    *                        (KH_FLAG_ATTN_MERGE_FENCED / KH_ATTN_FENCED=1).
    * Hook KH_SELFTEST=0 skips both, KH_SELFTEST_FAIL="ring,attn" injects a failure (tests). */

@@ -235,6 +235,7 @@ int hy_unfused_step(kh_model* m);
 int hy_argmax_partial(kh_model* m);
 // ---- kh_hybrid_step.hip
 int hy_step_init(kh_model* m);
+int hy_selftest(kh_model* m);  // cfg.attn_merge_selftest; a mismatch turns the fences on
 int hy_launch_step(kh_model* m, int advance, int n_forced);
 int hy_decode_max(const kh_model* m);  // sequences the fused step can take at once
 int hy_decode(kh_model* m, const HyEntry* e, int n, float* h_logits);

@@ -792,7 +792,7 @@ int finish(kh_model* m, Plan& pl) {
   m->step_var = 0;
   if ((rc = kh_launch_status()) != KH_OK) return rc;
   KH_CHECK_HIP(hipStreamSynchronize(m->stream));
-  return KH_OK;
+  return hy_selftest(m);
 }
 
 int create_impl(const char* config, size_t config_len, const void* tensors, size_t nbytes, const kh_model_opts* o,

@@ -112,6 +112,13 @@ int split_waves(int rows, int nblk) {
   return ks;
 }
 
+// attention over heads beside the experts, of B sequences
+LdHeads beside(const kh_model* m, const Hybrid::Step& st, const HyHeads& ha, int B) {
+  const int chunks = ha.chunks();
+  return {ha.qn.p, ha.bias.p, st.hpart, st.v, st.tickets, B * ha.G * chunks * ha.beside, ha.H / ha.G, chunks, ha.beside,
+          ha.nbias, ha.sink, ha.gate ? ha.g_off() : -1, ha.o.ld, m->attn_fenced, ha.span, ha.scale * 1.44269504088896f};
+}
+
 // One token of B sequences: tables at (tok, pos, slot); logits to `logits` [B][V]; argmax partials of sequence 0 to
 // the model's sampler buffers.
 // tail: the last layer run only, behind a pass that has left the residual rows in front of it in x[0] (complete: nothing of a
@@ -239,9 +246,7 @@ int step(kh_model* m, const LdTabs tb, float* logits, bool tail = false, bool ma
         a.cache = (T*)m->kcache + r.kv_off;
         a.slot_elems = hy.kv_slot;
         if (ha.beside) {
-          const int chunks = ha.chunks();
-          a.att = {ha.qn.p, ha.bias.p, st.hpart, st.v, st.tickets, B * ha.G * chunks * ha.beside, ha.H / ha.G, chunks, ha.beside,
-                   ha.nbias, ha.sink, ha.gate ? ha.g_off() : -1, ha.o.ld, m->attn_fenced, ha.span, ha.scale * 1.44269504088896f};
+          a.att = beside(m, st, ha, B);
           lds = std::max(lds, kLdhLds);
         }
       } else if (!mixed) {
@@ -402,7 +407,88 @@ __global__ __launch_bounds__(256) void k_tail_rows(const int32_t* rows, const fl
   if (!mix) return;
   for (int i = threadIdx.x; i < ldv / 4; i += 256) ((f32x4*)(v + to * ldv))[i] = quad_f(mix + from * ldv + 4 * i);
 }
+// ---- self-check of the splits' hand-over without fences (kh_ldheads.h), as kh_model_selftest.hip checks the .bin models' ----
+template <class T>
+__global__ __launch_bounds__(256) void k_check_fill(T* p, size_t n, uint32_t seed) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    uint32_t h = (uint32_t)i * 2654435761u ^ seed;
+    h ^= h >> 15;
+    h *= 2246822519u;
+    h ^= h >> 13;
+    p[i] = (T)((float)(h & 0xffffu) / 32768.0f - 1.0f);
+  }
+}
+__global__ __launch_bounds__(256) void k_check_diff(const uint32_t* a, const uint32_t* b, int n, int32_t* flag) {
+  bool d = false;
+  for (int i = threadIdx.x; i < n; i += 256) d |= a[i] != b[i];
+  if (d) *flag = 1;
+}
+// One launch with fences, then 24 without, over pseudo-random rows 0 .. pos of slot 0; what it borrows is zero again behind it.
+// out: [o.ld] and a flag behind it, zeroed
+template <class T>
+int check_beside(kh_model* m, const HyRun& r, const HyHeads& ha, int pos, float* out) {
+  Hybrid& hy = *m->hy;
+  Hybrid::Step& st = *hy.step_st;
+  hipStream_t s = m->stream;
+  T* rows = (T*)m->kcache + r.kv_off;
+  const size_t n = (size_t)(pos + 1) * ha.row();
+  TRY(kv_map_range(m, 0, r.kv_off * sizeof(T), (r.kv_off + n) * sizeof(T), r.layer));
+  st.h_tabs[TB_POS] = pos;
+  KH_CHECK_HIP(hipMemcpyAsync(st.tabs, st.h_tabs, TB_ZERO * 4, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_check_fill<T>, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1024)), dim3(256), 0, s, rows, n, 0x9e3779b9u);
+  hipLaunchKernelGGL(k_check_fill<float>, dim3(16), dim3(256), 0, s, st.in, (size_t)ha.qkvg.N, 0xc2b2ae35u);
+  LdMidArgs a{};
+  a.t = {st.tabs + TB_TOK, st.tabs + TB_POS, st.tabs + TB_SLOT};
+  a.hr = ha.head_row(hy.c.eps);
+  a.raw = st.in;
+  a.ldv = ha.qkvg.N;
+  a.cache = rows;
+  a.slot_elems = hy.kv_slot;
+  a.att = beside(m, st, ha, 1);
+  for (int i = 0; i < 25; ++i) {
+    a.att.fenced = i == 0;
+    TRY(go(k_ld_mid<T, 1, 2, 1, false, true>, dim3(a.att.nwg), 256, kLdhLds, s, a));
+    if (i == 0) KH_CHECK_HIP(hipMemcpyAsync(out, st.v, (size_t)ha.o.ld * 4, hipMemcpyDeviceToDevice, s));
+    else hipLaunchKernelGGL(k_check_diff, dim3(1), dim3(256), 0, s, (const uint32_t*)st.v, (const uint32_t*)out, ha.o.ld, (int32_t*)out + ha.o.ld);
+  }
+  KH_CHECK_HIP(hipMemsetAsync(rows, 0, n * sizeof(T), s));
+  KH_CHECK_HIP(hipMemsetAsync(st.in, 0, (size_t)ha.qkvg.N * 4, s));
+  KH_CHECK_HIP(hipMemsetAsync(st.v, 0, (size_t)ha.o.ld * 4, s));
+  int32_t flag = 0;
+  KH_CHECK_HIP(hipMemcpyAsync(&flag, (int32_t*)out + ha.o.ld, 4, hipMemcpyDeviceToHost, s));
+  KH_CHECK_HIP(hipStreamSynchronize(s));
+  st.h_tabs[TB_POS] = 0;
+  TRY(kh_launch_status());
+  const char* inject = dbg("KH_SELFTEST_FAIL");
+  const bool ok = !flag && !(inject && strstr(inject, "attn"));
+  m->cfg.attn_merge_selftest = ok ? 1 : -1;
+  m->attn_fenced = !ok;
+  return KH_OK;
+}
 }  // namespace
+
+// the first layer whose attention beside the experts has several splits within its first 256 keys; without one there is nothing
+// to check
+int hy_selftest(kh_model* m) {
+  Hybrid& hy = *m->hy;
+  m->cfg.attn_merge_selftest = m->attn_fenced ? 2 : 0;
+  if (m->attn_fenced || dbg_off("KH_SELFTEST") || hy.step_st->bmax < 1) return KH_OK;
+  for (const HyRun& r : hy.runs) {
+    const HyLayer& l = hy.layers[(size_t)r.layer];
+    if (l.mixer != HY_HEADS || l.ha.beside < 2) continue;
+    const HyHeads& ha = l.ha;
+    const int span = ha.span.window > 0 ? ha.span.window : ha.span.chunk;
+    const int keys = std::min({span > 0 ? span : INT_MAX, m->cfg.cache_len, 256});
+    if ((hy.f32 ? ldh_split_len<float>(keys, ha.beside) : ldh_split_len<bf16>(keys, ha.beside)) >= keys) continue;
+    float* out = nullptr;
+    TRY(dalloc(&out, (size_t)ha.o.ld + 1));
+    hipError_t e = hipMemsetAsync(out, 0, ((size_t)ha.o.ld + 1) * 4, m->stream);
+    const int rc = e != hipSuccess ? (int)e : hy.f32 ? check_beside<float>(m, r, ha, keys - 1, out) : check_beside<bf16>(m, r, ha, keys - 1, out);
+    (void)hipFree(out);
+    return rc;
+  }
+  return KH_OK;
+}
 
 int hy_step_init(kh_model* m) {
   Hybrid& hy = *m->hy;

@@ -10,7 +10,8 @@
 //      form): it leans on gfx950 behaviour the HIP memory model does not spell out.  One fenced launch gives the
 //      reference, KH_SELFTEST_ATTN_LAUNCHES back-to-back fence-free launches of the same merge (per-head path and,
 //      where the geometry has one, the GQA group path) must reproduce it word for word.  A mismatch makes this
-//      model use the fenced form (kh_config.attn_merge_selftest = -1).
+//      model use the fenced form (kh_config.attn_merge_selftest = -1).  Layer-list models check theirs, of one layer that
+//      attends beside its experts, by themselves (kh_hybrid_step.hip, hy_selftest).
 //
 // Both run on scratch state the model owns at that moment (activation buffers, rows of layer 0 of the still
 // empty KV cache, which are zeroed again) in about a millisecond.  This is a tripwire for a part, a compiler or a

@@ -101,3 +101,34 @@ def test_fences_give_the_same_bits(gpu):
         m.close()
     for got in out[0] + out[1]:
         np.testing.assert_array_equal(got, out[1][0])
+
+
+@BOTH
+def test_hand_over_is_checked_at_creation(gpu, dtype):
+    """Splits merged without fences against the fenced form, on the model's own device: the result in the configuration, the fenced
+    form where the check fails (injected), nothing where no launch has several splits."""
+    kw = dict(heads=8, kv_heads=2, dim=128, vdim=64)
+    mod = U.Model(U.gusorax([dict(U.chunked(), mlp=U.dense()), dict(U.windowed(window=400, rows=16, far=90.0, **kw), mlp=U.clamped())]))
+    toks = mod.tokens(310)
+    out = {}
+    for hooks, want in (((), 1), ((("KH_SELFTEST_FAIL", "attn"),), -1), ((("KH_SELFTEST", "0"),), 0), ((("KH_ATTN_FENCED", "1"),), 2)):
+        for k, v in hooks:
+            _ffi.debug_set(k, v)
+        try:
+            m = mod.load(dtype, max_seqs=4)
+        finally:
+            for k, _ in hooks:
+                _ffi.debug_set(k, None)
+        assert m.cfg.attn_merge_selftest == want and m.cfg.ring_selftest == 0
+        out[want] = steps(m, toks, [300, 0, 63, 64], 6)
+        m.close()
+    U.check(out[1][0], mod.logits(toks)[300:306], dtype)
+    for v in out.values():
+        np.testing.assert_array_equal(v, out[1])
+    split = 32 if dtype == "float32" else 64
+    for layer, rows, want in ((U.windowed(window=split, **kw), 512, 0), (U.windowed(window=split + 1, **kw), 512, 1),
+                              (U.chunked(chunk=300, **kw), split, 0), (U.latent(), 512, 0)):
+        one = U.Model(U.config([layer]) if layer["type"] == "latent_attention" else U.gusorax([dict(layer, mlp=U.dense())]))
+        m = one.load(dtype, max_seq_len=rows)
+        assert m.cfg.attn_merge_selftest == want, (layer, rows)
+        m.close()
