@@ -433,7 +433,7 @@ __device__ __forceinline__ float stage_vec(const float* __restrict__ x,
 //   MAXV = 1 / 2 / 4  vectors up to 4 / 8 / 16 floats per thread (4096 at 256 threads: dim of every
 //             BASELINE config)
 //   MAXV = 6  up to 24 floats per thread (12288 at 512 threads: the 11008-float hidden vector of
-//             Llama-2-7B's w2; k_gemv_res only)
+//             Llama-2-7B's w2; k_gemv_res and the operators k_matmul_*)
 //   MAXV = 0  any length: single-phase stage_vec AFTER the first weight loads were issued - its x
 //             loads sit behind the weight loads in the in-order vmcnt queue, so the staging (and
 //             everything after it) waits for the whole first tile
@@ -504,8 +504,8 @@ struct Stager {
   }
 };
 // float4 of the vector per staging thread: the smallest of 1 / 2 / 4 / 6 that covers M (0: single-phase staging)
-// does the 4-deep in-register staging cover M?  (the op-level kernels, the B-token prefill and the int8 ring
-// kernels use that depth whatever the length; a slot beyond the vector adds an exact 0 to the sum of
+// does the 4-deep in-register staging cover M?  (the B-token prefill and the int8 ring kernels use that depth whatever
+// the length; a slot beyond the vector adds an exact 0 to the sum of
 // squares, so every depth that covers the vector stages the same bits)
 static inline bool kh_stage_fits4(int M, int wg = KH_WG) { return M <= 4 * 4 * wg; }
 #ifndef KH_STAGE_MAXV_MIN  // experiment hook (profiles/r6_staging_ab.txt): 4 = the depth of rounds 1-5

@@ -110,8 +110,8 @@ constexpr size_t heads_lds(int tb, int ks, size_t table) {
 // KN, KV: key and value size in units of 64.  CP = 4: 16 rows per workgroup; CP = 1: 64 MR rows.  KS: sets of four waves; set k
 // takes key tiles k, k + KS, ... of the same rows, and the sets are merged at the end through LDS.  A tile of 32 keys is a
 // serial chain (keys from LDS, scores, maximum, exponentials, values: 1.1 us for 0.1 us of products), so a wave needs another
-// one on its SIMD; where the rows of a launch make one workgroup per CU, KS = 2 is where it comes from.  KS = 4 is a decoded
-// token whose keys nobody else shares (heads_one_split): the tiles of a workgroup side by side.
+// one on its SIMD; where the rows of a launch make one workgroup per CU, KS = 2 is where it comes from.  KS = 4: a decoded
+// token whose keys nobody else shares (heads_one_split), the tiles of a workgroup side by side, or such a launch of rows in bf16.
 // Two waves per SIMD where the accumulators allow it: within 256 registers the compiler keeps them where the rescaling can
 // reach them (beyond, it moves them between two register files in every tile).
 template <class T, int KN, int KV, int CP, int MR, int KS>

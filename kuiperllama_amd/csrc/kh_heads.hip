@@ -37,9 +37,9 @@ int heads_attn_launch(hipStream_t s, HeadsArgs a, int ntiles, int rows) {
       if (rows == 16 && !a.tiles && a.nsplit == 1) return go(k_heads_attn<T, KN, KV, 4, 1, 4>, stage, 4);
     if (rows == 16) return go(k_heads_attn<T, KN, KV, 4, 1, 1>, stage, 1);
     // at most one workgroup per CU: two sets of waves, which share the keys (1100 tokens of 2 x 4 heads of 128, 138 workgroups:
-    // 37.2 -> 27.9 us; four sets on tiles of 32 rows 25.9, at twice the key traffic), or four in bf16, where heads of 128 leave
-    // the registers (25.1; in fp32 they spill) and what the sets hand over fits the stages.  Keys and values of more than 256
-    // elements together need the registers of a wave alone on its SIMD.
+    // 37.2 -> 27.6 us; four sets on tiles of 32 rows 25.9, at twice the key traffic), or four in bf16, where heads of 128 leave
+    // the registers (27.9 -> 25.1 in another session; in fp32 they spill) and what the sets hand over fits the stages.  Keys and
+    // values of more than 256 elements together need the registers of a wave alone on its SIMD.
     if constexpr (KN + KV <= 4)
       if (rows == 64 && a.tiles && (long)ntiles * a.G <= 256) {
         if constexpr (sizeof(T) == 2 && KN == 2 && KV == 2) return go(k_heads_attn<T, KN, KV, 1, 1, 4>, stage, 4);

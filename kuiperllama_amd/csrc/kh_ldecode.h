@@ -501,7 +501,7 @@ __global__ __launch_bounds__(ld_in_wg(B, NV)) void k_ld_in(const LdInArgs a) {
 
 // ---- k_ld_mid ----------------------------------------------------------------------------------------------------
 struct LdMidArgs {
-  // experts: workgroups [0, B top nwg_e)
+  // experts: workgroups [0, B top nwg_e), behind those of attention over heads
   const float* z;        // [B][ldz]
   const float *corr, *xn2;
   const void* gu;        // experts [2 ffp][ldw]
@@ -519,7 +519,7 @@ struct LdMidArgs {
   // cache rows: the last workgroups (latent attention: one per sequence; heads: one wave per key / value head)
   int latent;
   HeadRow hr;
-  LdHeads att;           // attention over heads: the first workgroups
+  LdHeads att;           // attention over heads: the first workgroups (none: it has launches of its own)
   const float* raw;      // [B][ldv]: q latent, kv latent, rotated part
   const float* kvn;
   const float2* rope;
