@@ -432,7 +432,7 @@ int kh_model_time_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32
 int kh_model_profile_kernel(kh_model* m, int32_t kclass, int32_t pos, int32_t reps,
                             float* h_avg_us);
 
-/* Latency of ONE decode step at position `pos` (per-token latency at pos 0/64/127):
+/* Latency of ONE decode step at position `pos`:
  * the 1-step hipGraph replayed `reps` times with the device state reset to `pos` before each,
  * HIP events around each replay; h_us[reps] in microseconds.  KV rows below pos must exist and
  * a graph-mode generate of more than `pos` steps must have run on this model. */

@@ -45,7 +45,7 @@ inline void check(int code, const char* what) {
   if (code != KH_OK) error_handler()(code, what);
 }
 
-// Runtime replacements for the reference's compile-time switches (SURVEY.md §0.4):
+// Runtime replacements for the reference's compile-time switches:
 //   LLAMA3_SUPPORT -> {KH_ROPE_HALF, eps 1e-5, theta 5e5}; QWEN2_SUPPORT -> {KH_ROPE_HALF, eps 1e-6,
 //   theta 1e6}; neither -> {KH_ROPE_INTERLEAVED, eps 1e-5, theta 1e4}
 //   (cpu/rope_kernel.cpp:3-16,43,83; cpu/rmsnorm_kernel.cpp:24-28).

@@ -17,7 +17,7 @@ against each other and (in the build container only) against files written by th
 reference's own exporter.  No reference code is imported here.
 
 There are no real checkpoints on disk and no network, so benchmarks and parity tests use
-:func:`synth_image`: a seeded random model of the exact BASELINE shape written straight
+:func:`synth_image`: a seeded random model of a preset's exact shape written straight
 into an in-memory image with the byte layout above.
 """
 from __future__ import annotations
@@ -80,12 +80,12 @@ class ModelSpec:
         return HEADER_INT8_BYTES if self.quant else HEADER_FP32_BYTES
 
     def weight_elems(self) -> int:
-        """W_elems of SURVEY.md §8(d): matmul weights streamed per decoded token."""
+        """Matmul weights streamed per decoded token."""
         d, kv, h, L, v = self.dim, self.kv_dim, self.hidden_dim, self.n_layers, self.vocab_size
         return L * (2 * d * d + 2 * kv * d + 3 * h * d) + v * d
 
     def algorithmic_bytes_per_token(self, pos: float) -> float:
-        """Algorithmic HBM bytes for one decode step at position ``pos`` (SURVEY.md §8d):
+        """Algorithmic HBM bytes for one decode step at position ``pos``:
         weights once + KV read/write + norms/embedding row/biases/logits."""
         d, kv, L, v = self.dim, self.kv_dim, self.n_layers, self.vocab_size
         we = self.weight_elems()
@@ -100,7 +100,7 @@ class ModelSpec:
         return float(wbytes + small + kvb)
 
     def kernel_bytes(self) -> Dict[str, float]:
-        """Algorithmic HBM bytes of ONE launch of each weight-streaming kernel of the decode step (DESIGN 3.2):
+        """Algorithmic HBM bytes of ONE launch of each weight-streaming kernel of the decode step:
         the rows of its matrices once (+ group scales), its input vector (+ norm weight) once, its output once."""
         d, kv, h, v = self.dim, self.kv_dim, self.hidden_dim, self.vocab_size
 
@@ -114,7 +114,7 @@ class ModelSpec:
                 "cls": w(v * d) + 2 * d * 4 + v * 4}
 
 
-# BASELINE.json configs -------------------------------------------------
+# The geometries that the benchmark and the tests run ----------------------------------------
 PRESETS: Dict[str, ModelSpec] = {
     "stories15M": ModelSpec(288, 768, 6, 6, 6, 32000, 256, True, FAMILY_LLAMA, False, 64,
                             ROPE_INTERLEAVED, 10000.0, 1e-5, "stories15M"),
@@ -256,7 +256,7 @@ def synth_image(spec: ModelSpec, seed: int = 1234, device: str | torch.device = 
     ents, total = layout(spec)
     # Place the image so that the bytes BEHIND the header - what the library uses in place when the image is handed
     # over on the device - start on a 4-KiB boundary, as they do in the arena kh_model_create_from_file /
-    # _from_host_image allocate.  Every tensor of an exported image is a multiple of 256 bytes long in the BASELINE
+    # _from_host_image allocate.  Every tensor of an exported image is a multiple of 256 bytes long in the presets'
     # geometries, so all weight rows then start on a line boundary; with the int8 header (32 bytes: a 16-byte
     # aligned, usable address) every row sat 32 bytes off one and each 1-KiB wave request straddled nine 128-byte
     # lines instead of eight (measured on ffn13 int8: 18.0 vs 17.4 us, profiles/r5_int8_ring_ab.txt).

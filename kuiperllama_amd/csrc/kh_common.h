@@ -46,7 +46,7 @@ inline bool dbg_off(const char* key) {  // hook present and starting with '0'
 }  // namespace khm
 
 // Weight rows are streamed exactly once per token: non-temporal loads keep them from
-// displacing the activations in L2 (MI355X guide: nt-weights row).
+// displacing the activations in L2.
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) {
   return __builtin_nontemporal_load(p);

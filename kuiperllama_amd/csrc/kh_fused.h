@@ -1,7 +1,7 @@
 // kh_fused.h — the fused decode-step kernels (5 per layer + classifier + sampler).
 //
 // The reference issues 14 launches per layer (17 for Qwen2) from host code that also reads
-// `pos` on the CPU (SURVEY.md §2a, §0.5).  Here one token = 5L+2 launches whose every
+// `pos` on the CPU.  Here one token = 5L+2 launches whose every
 // offset derives from the DEVICE scalar *d_pos, so the whole step is a replayable hipGraph:
 //
 //   k_qkv    rmsnorm(x) -> LDS ; [wq|wk|wv] row pairs ; +bias ; RoPE ; q -> q_buf,
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(KH_WG_MAX, 4) void k_qkv(const KhQkvArgs a) {
   float* red = lds_red_ptr<QUANT>(xs, dim);
   const int lane = threadIdx.x & 63;
   const int hs = a.head_size, half = hs >> 1;
-  // head sizes are powers of two in every BASELINE config: shifts instead of the ~25-instruction
+  // head sizes are powers of two in every preset: shifts instead of the ~25-instruction
   // integer division the work-item decode would otherwise run three times per row pair
   const bool half_pow2 = (half & (half - 1)) == 0;
   const int half_sh = __builtin_ctz((unsigned)half | 0x40000000u);

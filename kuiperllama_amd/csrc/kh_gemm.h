@@ -204,7 +204,7 @@ __device__ __forceinline__ void pg_kloop_f32(const float* const (&wrow)[R], cons
 // latency of the activations.  The phase scheme above prefetches the activations ONE step ahead -
 // enough when a step holds >= 64 MFMAs (R x NT = 16), far too little for the 16-MFMA steps of the
 // (1,4) / (2,2) tiles the small-M GEMMs (wo, w2, QKV) need to fill the chip (0.24 us per step against
-// ~0.5 us of L2 latency: MfmaUtil 28-33 % in round 2).  Needs (b1 - b0) % D == 0 and >= 2 D blocks;
+// ~0.5 us of L2 latency: MfmaUtil 28-33 %).  Needs (b1 - b0) % D == 0 and >= 2 D blocks;
 // D * (R + NT) float4 of ring registers.
 template <int R, int NT, int D>
 __device__ __forceinline__ void pg_kloop_f32_ring(const float* const (&wrow)[R], const PgBAddr& B, int b0,

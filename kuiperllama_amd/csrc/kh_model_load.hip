@@ -51,8 +51,8 @@ int ilog2_exact(int v) {
 // Host image (typically the mmap of a .bin file: pageable, possibly not yet paged in) -> HBM.
 // A plain hipMemcpy from pageable memory is staged by the driver in small pieces.  Here a ring of four pinned
 // 32-MiB buffers is filled by a team of host threads - each chunk is cut into one slice per thread, so the page
-// faults and the memcpy of ONE chunk run on all of them (a single filler thread moves 6-9 GB/s: rounds 1-4
-// uploaded at 14-17 GB/s) - while up to three earlier chunks are in flight on the copy engine.  The main thread
+// faults and the memcpy of ONE chunk run on all of them (a single filler thread moves 6-9 GB/s, an upload
+// by one was 14-17 GB/s) - while up to three earlier chunks are in flight on the copy engine.  The main thread
 // only sequences: chunk c is handed to the DMA engine when all of its slices are staged, and its buffer goes back
 // to the fillers when that transfer has completed.  Matters for the 27 GB fp32 7B image of the 8-replica config.
 int upload_threads() {

@@ -303,7 +303,7 @@ int ensure_pg_buffers(kh_model* m, int n) {
   return done(rows) ? KH_OK : alloc_pg_buffers(m, rows, part(rows));
 }
 // The split workspace of the decode-attention FALLBACK (one per token of a pass, ~270 KB per token at
-// Llama-3.2-1B geometry: 136 MB for a 512-token pass).  Every BASELINE head size has an MFMA
+// Llama-3.2-1B geometry: 136 MB for a 512-token pass).  Every preset's head size has an MFMA
 // instantiation, so it is allocated on the first pass that actually takes the fallback.
 int ensure_pg_ws(kh_model* m) {
   if (m->pg_ws || pg_mfma_attn(m)) return KH_OK;

@@ -2,7 +2,7 @@
 // construction, executed once at the end of kh_model_create_* on the model's own device, weights and geometry:
 //
 //  (a) the int8 LDS-DMA ring kernels (kh_q8ring.h): their input-vector staging uses asm loads whose destination
-//      registers the compiler believes written at the asm statement (DESIGN 3.1b).  One launch of every adopted
+//      registers the compiler believes written at the asm statement.  One launch of every adopted
 //      ring kernel (ffn13 on the first layer's w1 / w3, the classifier) against the register-tile kernel of the same
 //      launch on the same input, outputs compared word for word.  A mismatch turns the ring off for this model
 //      (kh_config.ring_selftest = -1; the register-tile kernels are bit-identical by design, so nothing else changes).

@@ -48,8 +48,7 @@ kh_model::Shape pick_shape(bool quant, int pairs, int M, int max_split, const ch
   // requests the next tile in a burst right after the current tile's FMAs (kh_fused.h: ROLL = false everywhere but
   // the int8 QKV kernel), so a wave that walks several chunks of a long row keeps loads in flight across them and
   // fewer, longer-lived waves beat many short ones (r3 sweeps, profiles/r3_shape_sweep.txt: Llama-2-7B w2 int8
-  // split 4 -> 2: 12.6 -> 10.8 us, fp32 33.6 -> 31.4; wo int8 split 2 -> 1: 5.6 -> 5.25); rounds 1-2 aimed at
-  // twice as many.
+  // split 4 -> 2: 12.6 -> 10.8 us, fp32 33.6 -> 31.4; wo int8 split 2 -> 1: 5.6 -> 5.25).
   const int target_waves = pair_bytes >= 16384 ? 4096 : 2048;
   while (sh.split < max_split && pairs * sh.split < target_waves &&
          pair_bytes / (sh.split * 2) >= min_bytes)
@@ -60,7 +59,7 @@ kh_model::Shape pick_shape(bool quant, int pairs, int M, int max_split, const ch
     // one chunk when it covers the column range; ranges that need several chunks anyway take the
     // small one (less padding in the last chunk, finer refill: w2 int8 u4 -> u2 11.9 -> 10.8 us)
     sh.u = per_lane > 4 ? 2 : (per_lane >= 3 ? 4 : 2);
-    // [r6] w2 only (u3): a column range of 5 or 6 loads per lane as TWO exact tiles of 3 instead of three tiles of
+    // w2 only (u3): a column range of 5 or 6 loads per lane as TWO exact tiles of 3 instead of three tiles of
     // 2 - Llama-2-7B int8's w2 (5.4 loads per lane): 10.45 -> 10.25 us, +0.4 % tok/s, four alternations on one box
     // (profiles/r6_w2_u3_ab.txt); ONE tile of 6 is slower (10.95 us: the whole item requested in one burst)
     if (u3 && per_lane > 4 && per_lane <= 6) sh.u = 3;
@@ -914,7 +913,7 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
     memcpy(h_words, m->h_words_pin, sizeof(int32_t) * (size_t)total_steps);
     for (int i = 0; i < start; ++i) h_words[i] = h_prompt[i + 1];  // forced, main.cpp:36-38
   } else {
-    // Stop-token check without a per-step host round trip (SURVEY 8f.2): the words of every
+    // Stop-token check without a per-step host round trip: the words of every
     // chunk of steps are mirrored into pinned memory behind the chunk, and the host inspects
     // chunk k while chunk k+1 is already queued, so the GPU never waits for the check.  At
     // most two chunks of steps run past the stop token; their words are discarded.

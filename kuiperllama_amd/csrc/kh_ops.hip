@@ -760,8 +760,8 @@ extern "C" int kh_argmax_f32(const float* logits, int64_t n, int32_t* d_out_inde
   return kh_launch_status();
 }
 // The reference's sampler path (ArgmaxSampler::sample -> argmax_kernel_cu, argmax_kernel.cu:53-77) allocates 8 bytes
-// per token and never frees them; rounds 1-4 of this library allocated and freed 4 bytes per call, i.e. a
-// device-wide synchronisation per token.  One 4-byte device word per (device, stream), created on first use and
+// per token and never frees them; allocating and freeing 4 bytes per call would be a device-wide
+// synchronisation per token.  One 4-byte device word per (device, stream), created on first use and
 // kept for the life of the process (a few bytes per stream ever used).  Calls on different streams use different
 // words; two host threads calling on the SAME stream (the null stream, say) are serialised by the word's own mutex,
 // held from the kernel launch to the stream synchronisation - otherwise kernel A, kernel B, copy A, copy B would hand

@@ -1,4 +1,4 @@
-// kh_pattn.h — causal attention of a prompt slice on the matrix cores (GEMM prefill, SURVEY.md §8f-4).
+// kh_pattn.h — causal attention of a prompt slice on the matrix cores (GEMM prefill).
 //
 // The reference computes attention one query token at a time (cpu/mha_kernel.cpp:5-61,
 // cuda/mha_kernel.cu:47-110: score = q.k * 1/sqrt(hs), softmax over 0..pos, out = sum p_t v_t).

@@ -1,4 +1,4 @@
-"""Multi-GPU = independent replicas (SURVEY.md §8e): batch-1 greedy decode is single-stream and
+"""Multi-GPU = independent replicas: batch-1 greedy decode is single-stream and
 autoregressive, the reference has no sharding and pins device 0 (llama3.cpp:118), so N GPUs run
 N copies of the path with NO data-path collective.  The only communication is the timing
 protocol of the benchmark: barrier, then max-over-ranks of the per-rank wall time.
@@ -13,8 +13,8 @@ from typing import Callable, Tuple
 import torch
 
 
-# the 8-GPU number is Llama-2-7B fp32, one independent replica per GPU
-# (the reference pins device 0, llama3.cpp:118); N = 1 is configs[1].
+# Several GPUs: Llama-2-7B in fp32, one independent replica per GPU (the reference pins device 0, llama3.cpp:118); one GPU:
+# Llama-3.2-1B.
 REPLICA_WORKLOAD = "llama2-7b"
 SINGLE_WORKLOAD = "llama3.2-1b"
 
@@ -102,7 +102,7 @@ def gather_per_replica(value: float, world: int, device: torch.device) -> list:
 
 
 def spread(per_replica: list) -> dict:
-    """min / max / relative spread of per-replica throughputs (SURVEY.md §8e)."""
+    """min / max / relative spread of per-replica throughputs."""
     lo, hi = min(per_replica), max(per_replica)
     return {"per_replica": [round(v, 3) for v in per_replica], "min": lo, "max": hi,
             "spread_frac": (hi - lo) / hi if hi > 0 else 0.0}

@@ -8,7 +8,7 @@
  *
  * Summation order note: the reference computes every dot product through Armadillo ->
  * BLAS sgemv/sdot (cpu/matmul_kernel.cpp:37-40), whose internal order is unspecified and
- * whose version is unpinned (SURVEY.md §8c).  dot_f32() below uses a fixed 16-way blocked
+ * whose version is unpinned.  dot_f32() below uses a fixed 16-way blocked
  * order (what a vectorised BLAS kernel does); dot_f64() is the fp64-accumulated "gold"
  * used to judge which of {HIP, this fp32 restatement} is closer to exact.
  */
@@ -82,7 +82,7 @@ static float arma_accumulate(const float* x, int n) {
 /* ---- cpu/matmul_kernel.cpp:5-41 ---------------------------------------------------
  * weight is [K rows, M cols] row-major (wei_dim0=K, wei_dim1=M); arma views it as M x K
  * column-major, so output[p] = sum_i input[i]*weight[p*M+i]; then "* scale" (line 40). */
-/* Timing-only variant (bench.py cpu_baseline, SURVEY 8d(ii)): the reference's CPU matmul is
+/* Timing-only variant (bench.py cpu_baseline): the reference's CPU matmul is
  * Armadillo -> BLAS sgemv (cpu/matmul_kernel.cpp:37-40), so a caller may plug in a
  * cblas_sgemv-compatible ILP64 entry point (numpy's bundled OpenBLAS).  Never set by tests:
  * BLAS summation order is not the pinned one. */

@@ -9,7 +9,7 @@
  * reference repo root, zjhellofss/KuiperLLama @ 2025-02-19).  This is a *port* ("kind":
  * "port" in bench.py), pinned by (a) the reference tests' integer-exact golden vectors,
  * (b) logits produced by the reference's own Python model (tools/model.py, tools/export.py)
- * — see tests/golden/make_golden.py — and, since round 5, (c) the reference's OWN C++ CPU
+ * — see tests/golden/make_golden.py — and (c) the reference's OWN C++ CPU
  * backend: its ten CPU kernel files (cpu/<op>_kernel.cpp), operator and model classes compiled where they lie
  * (oracle/Makefile `ref_cpu` -> oracle/_ref/ref_cpu_model*; Armadillo, absent here, is
  * answered by tests/cpp/ref_stubs/armadillo over numpy's OpenBLAS): this oracle and that
