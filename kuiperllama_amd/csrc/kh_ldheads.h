@@ -47,6 +47,8 @@ constexpr size_t kLdhLds = (4 * KH_LDH_DIM + 4 * 64 + 64 * 4 + 16 + 16 * KH_LDH_
 //   8 heads on 2, bf16     127 / 101  177 / 137     126 / 110  174 / 139     123 / 112  175 / 141    136 / 134  202 / 160
 //   32 on 8, fp32          175 / 143  242 / 223     178 / 144  251 / 227     177 / 145  282 / 232    208 / 180  392 / 292
 //   64 on 16, bf16         184 / 142  237 / 210     173 / 149  242 / 212     171 / 162  277 / 207
+// In layers without experts, where it stands alone in its launch, 10-18 % less at 30 keys, as much at 3000 and in bf16 2-7 % more at
+// 4000 keys of one sequence (8 on 2 130 / 138, 4 on 4 130 / 134).
 // Beyond: 64 on 16 as 256 workgroups a sequence 230 / 250 at 30 keys, four sequences; in bf16 with 256 keys a split, one
 // sequence at the last of them 163 / 168 (32 on 16, eight splits), 171 / 182 (32 on 32, four); 128 heads of 64 on 128 as one split,
 // 4000 keys 262 / 528 and 616 / 977.
