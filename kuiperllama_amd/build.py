@@ -19,10 +19,10 @@ LIB_DIR = os.path.join(_PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libkuiper_hip.so")
 # code for one interpreter's ABI, which its name says
 PYOPS_PATH = os.path.join(LIB_DIR, "kh_pyops" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
-SOURCES = ["kh_ops.hip", "kh_model_load.hip", "kh_model_step.hip", "kh_model_prefill.hip", "kh_model_pair.hip", "kh_model_profile.hip", "kh_model_selftest.hip",
+SOURCES = ["kh_ops.hip", "kh_model_load.hip", "kh_model_step.hip", "kh_attn_wo.hip", "kh_model_prefill.hip", "kh_model_pair.hip", "kh_model_profile.hip", "kh_model_selftest.hip",
            "kh_hybrid_load.hip", "kh_hybrid_pass.hip", "kh_hybrid_step.hip", "kh_heads.hip",
            "kh_tokenizer.cpp", "kh_bpe.cpp", "kh_debug.cpp"]
-HEADERS = ["kh_common.h", "kh_gemv.h", "kh_attn.h", "kh_fused.h", "kh_q8ring.h", "kh_fused_ring.h", "kh_prefill.h", "kh_gemm.h", "kh_pair.h", "kh_pattn.h", "kh_pattn_pair.h", "kh_unicode_tables.h", "kh_json.h",
+HEADERS = ["kh_common.h", "kh_gemv.h", "kh_attn.h", "kh_fused.h", "kh_q8ring.h", "kh_fused_ring.h", "kh_prefill.h", "kh_gemm.h", "kh_attn_wo.h", "kh_pair.h", "kh_pattn.h", "kh_pattn_pair.h", "kh_unicode_tables.h", "kh_json.h",
            "kh_tile.h", "kh_softplus.h", "kh_lgemm.h", "kh_lops.h", "kh_scan.h", "kh_moe.h", "kh_latent.h", "kh_expanded.h", "kh_heads.h", "kh_hybrid.h", "kh_ldheads.h", "kh_ldecode.h",
            "kh_model_internal.h",
            "../../include/kuiper_hip.h"]

@@ -1,0 +1,107 @@
+// kh_attn_wo.hip - launches of kh_attn_wo.h: attention and the output projection of a decoded token in one launch.
+#include "kh_attn_wo.h"
+
+#include "kh_model_internal.h"
+
+namespace khm {
+
+// Which models take it, and in what shape.  fp32 weights; at most eight key / value groups of at most 16 heads and 512 columns
+// (two float4 a lane), head sizes that the attention is instantiated for, vectors that two float4 a thread cover: every group is
+// one vector more that k_ffn13_parts stages (eight of 2048 floats cost it 0.9 us), and its keys and values are read by every
+// slice.  us a launch at position 48, attention + wo -> one launch | ffn13: Llama-3.2-1B 3.4 + 4.5 -> 5.0 | 21.3 -> 22.2;
+// TinyLlama 3.3 + 4.5 -> 4.9 | 15.5 -> 15.9; Qwen2.5-0.5B 3.4 + 2.6 -> 4.2 | 6.95 -> 7.15; stories15M 3.6 + 2.3 -> 3.9 | 2.4 -> 2.75.
+// A token: -3.9 / -6.1 / -8.4 / -12 %; with 200 - 240 positions -1.5 / -3 / -2 / -4 %.  From KH_ATTN_MIN_TS on attention is split over time.
+kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long) {
+  kh_model::AttnWoPlan p;
+  const int hs = c.head_size, cols = c.kv_mul * hs, mv = kh_stage_maxv(c.dim, ffn_wg);
+  if (c.is_quant || dbg_off("KH_ATTN_WO") || (hs != 48 && hs != 64)) return p;
+  if (c.kv_mul > 16 || c.kv_head_num > KH_AWO_PARTS_MAX || cols > 512 || c.dim != c.head_num * hs || mv < 1 || mv > 2) return p;
+  p.parts = c.kv_head_num;
+  p.cols4 = cols / 4;
+  p.lpr = p.cols4 <= 16 ? 16 : (p.cols4 <= 32 ? 32 : 64);
+  p.nu = (p.cols4 + p.lpr - 1) / p.lpr;
+  const int rows = KH_AWO_WAVES * (64 / p.lpr);
+  auto slices = [&](int rw) { return (c.dim + rows * rw - 1) / (rows * rw); };
+  // the most rows a workgroup (its attention is the same for few) that leave three quarters of the CUs with one: two rounds of
+  // half as many took 7.8 instead of 5.6 us (Llama-3.2-1B)
+  for (p.rw = p.lpr == 64 ? 8 / p.nu : 2; p.rw > 1 && p.parts * slices(p.rw) < 192;) p.rw /= 2;
+  p.slices = slices(p.rw);
+  p.lds = attn_wo_lds_bytes(hs, c.kv_mul);
+  p.end = t_long - 1 < KH_ATTN_MIN_TS ? t_long - 1 : KH_ATTN_MIN_TS;  // one split, and no group path
+  return p;
+}
+
+namespace {
+KhAttnWoArgs attn_args(kh_model* m, int l) {
+  const kh_config& c = m->cfg;
+  KhAttnWoArgs a{};
+  a.kcache_layer = m->kcache + (size_t)l * c.cache_len * c.kv_dim;
+  a.vcache_layer = m->vcache + (size_t)l * c.cache_len * c.kv_dim;
+  a.wo = (const float*)m->layers[l].wo.w;
+  a.dim = c.dim;
+  a.kv_dim = c.kv_dim;
+  a.kv_mul = c.kv_mul;
+  return a;
+}
+template <int DN>
+void go(const kh_model::AttnWoPlan& p, hipStream_t s, const KhAttnWoArgs& a) {
+  auto l = [&](auto k) { hipLaunchKernelGGL(k, dim3(p.parts, p.slices), dim3(128 * KH_AWO_WAVES), p.lds, s, a); };
+  if (p.lpr == 16) p.rw == 2 ? l(k_attn_wo<DN, 16, 1, 2>) : l(k_attn_wo<DN, 16, 1, 1>);
+  else if (p.lpr == 32) p.rw == 2 ? l(k_attn_wo<DN, 32, 1, 2>) : l(k_attn_wo<DN, 32, 1, 1>);
+  else if (p.nu == 2) p.rw == 4 ? l(k_attn_wo<DN, 64, 2, 4>) : p.rw == 2 ? l(k_attn_wo<DN, 64, 2, 2>) : l(k_attn_wo<DN, 64, 2, 1>);
+  else if (p.rw >= 4) p.rw == 8 ? l(k_attn_wo<DN, 64, 1, 8>) : l(k_attn_wo<DN, 64, 1, 4>);
+  else p.rw == 2 ? l(k_attn_wo<DN, 64, 1, 2>) : l(k_attn_wo<DN, 64, 1, 1>);
+}
+}  // namespace
+
+void launch_attn_wo(kh_model* m, int l) {
+  KhAttnWoArgs a = attn_args(m, l);
+  a.q = m->q;
+  a.d_pos = m->d_pos;
+  a.out = m->wo_part;
+  if (m->cfg.head_size == 48) go<3>(m->awo, m->stream, a);
+  else go<4>(m->awo, m->stream, a);
+}
+
+void launch_ffn13_parts(kh_model* m, const KhFfn13Args& f) {
+  KhFfn13PartsArgs a{f, m->wo_part, m->x1, m->awo.parts};
+  const int wg = m->sh_ffn.wg, mv = kh_stage_maxv(f.dim, wg), pn = (m->awo.parts + 1) / 2;
+  auto l = [&](auto k) { hipLaunchKernelGGL(k, dim3(m->sh_ffn.grid), dim3(wg), fused_lds_bytes(false, f.dim), m->stream, a); };
+  auto by_parts = [&](auto u, auto v) {
+    constexpr int U = decltype(u)::value, MV = decltype(v)::value;
+    if (pn == 1) l(k_ffn13_parts<U, MV, 2>);
+    else if (pn == 2) l(k_ffn13_parts<U, MV, 4>);
+    else if (pn == 3) l(k_ffn13_parts<U, MV, 6>);
+    else l(k_ffn13_parts<U, MV, 8>);
+  };
+  auto by_depth = [&](auto u) {
+    if (mv == 1) by_parts(u, std::integral_constant<int, 1>{});
+    else by_parts(u, std::integral_constant<int, 2>{});
+  };
+  if (m->sh_ffn.u >= 8) by_depth(std::integral_constant<int, 8>{});
+  else if (m->sh_ffn.u >= 4) by_depth(std::integral_constant<int, 4>{});
+  else by_depth(std::integral_constant<int, 2>{});
+}
+
+void launch_pf_attn_parts(kh_model* m, int l, int nvalid, int pos0) {
+  KhAttnWoArgs a = attn_args(m, l);
+  a.q = m->pf_q;
+  a.out = m->pf_att;
+  a.pos0 = pos0;
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, dim3(m->awo.parts, nvalid), dim3(64 * KH_AWO_WAVES), m->awo.lds, m->stream, a); };
+  if (m->cfg.head_size == 48) go(k_pf_attn_parts<3>);
+  else go(k_pf_attn_parts<4>);
+}
+void launch_pf_wo_parts(kh_model* m, int l, int nvalid) {
+  const kh_model::AttnWoPlan& p = m->awo;
+  KhPfWoPartsArgs a{m->pf_att, (const float*)m->layers[l].wo.w, m->pf_x, m->cfg.dim, p.parts, p.cols4, nvalid};
+  const int rows = KH_AWO_WAVES * (64 / p.lpr), lds = nvalid * m->cfg.dim * 4;  // at most 8 * 2048 floats: 64 KB
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3((m->cfg.dim + rows - 1) / rows), dim3(64 * KH_AWO_WAVES), lds, m->stream, a);
+  };
+  if (p.lpr == 16) go(k_pf_wo_parts<16, 1>);
+  else if (p.lpr == 32) go(k_pf_wo_parts<32, 1>);
+  else if (p.nu == 1) go(k_pf_wo_parts<64, 1>);
+  else go(k_pf_wo_parts<64, 2>);
+}
+}  // namespace khm

@@ -183,7 +183,8 @@ static __global__ __launch_bounds__(KH_WG_MAX) void k_attn_generic(const KhAttnA
 struct KhGemvResArgs {
   const float* vec;  // [M]
   KhLin w;           // [K, M]
-  float* x;          // [K] residual stream, updated in place
+  float* x;          // [K] residual stream
+  const float* xin;  // what the product is added to: x, or the sum that k_ffn13_parts left
   int M, K, gshift;
 };
 // STAGER(a, M): the staging of the input vector - Stager<false, ...> over a.vec, or CombStager over the
@@ -194,6 +195,7 @@ __device__ __forceinline__ void gemv_res_body(const KhGemvResArgs& a, St& st, f3
   const void* const w = a.w.w;
   const float* const scales = a.w.scales;
   float* const x = a.x;
+  const float* const xin = a.xin;
   const int M = a.M;
   const int lane = threadIdx.x & 63;
   const Gemv<QUANT, U> g(M, a.gshift);
@@ -201,7 +203,7 @@ __device__ __forceinline__ void gemv_res_body(const KhGemvResArgs& a, St& st, f3
   struct Aux {
     float x0, x1;
   };
-  auto pre = [&](int p) __attribute__((always_inline)) { return Aux{x[2 * p], x[2 * p + 1]}; };  // residual, fetched early
+  auto pre = [&](int p) __attribute__((always_inline)) { return Aux{xin[2 * p], xin[2 * p + 1]}; };  // residual, fetched early
   auto epi = [&](int p, float s0, float s1, const Aux& r) __attribute__((always_inline)) {
     if (lane != 0) return;
     x[2 * p] = r.x0 + s0;

@@ -18,6 +18,8 @@
 #include "kh_attn.h"
 #include "kh_common.h"
 
+struct KhFfn13Args;  // kh_fused.h
+
 namespace khm {
 // No C++ exception crosses the C ABI: the entry points that allocate host containers or start threads run their
 // body through this (std::bad_alloc -> hipErrorOutOfMemory, anything else -> KH_ERR_INTERNAL).
@@ -51,7 +53,7 @@ using khm::LayerW;
 
 #define KH_PAIR_TMAX 2048   // prompt tokens of one pass on the pair GEMMs
 #define KH_PA_WS_MAX ((size_t)256 << 20)  // the most memory for one layer's K / V as pairs
-#define KH_STEP_VARIANTS 3  // kh_model_step.hip::step_variant
+#define KH_STEP_VARIANTS 4  // kh_model_step.hip::step_variant
 struct kh_model {
   khm::Hybrid* hy = nullptr;  // layer-list model (checkpoint folder); nullptr: a .bin image
   std::vector<int> seq_len;   // .bin models: tokens of the one sequence kh_seq_open handed out
@@ -148,14 +150,23 @@ struct kh_model {
     int ffn_r = 0, ffn_grid = 0, cls_r = 0, cls_grid = 0;
   };
   RingPlan ring;
+  // attention and wo of a decoded token in one launch (kh_attn_wo.h; step variant 3); chosen by plan_attn_wo
+  struct AttnWoPlan {
+    int end = 0;  // positions below it take it (0: none)
+    int parts = 0, cols4 = 0, lpr = 0, nu = 0, rw = 0, slices = 0;
+    size_t lds = 0;
+  };
+  AttnWoPlan awo;
+  float *wo_part = nullptr, *x1 = nullptr;  // its partial sums [parts][dim]; the residual behind them
   // graph
   // the decode step captured once as a 1-step graph and once as a KH_GRAPH_STEPS-step graph:
   // consecutive hipGraphLaunch calls leave the GPU idle for ~8 us (measured), so the long
   // graph amortises that gap over several tokens
-  // ... each in three VARIANTS of the attention / wo pair (kh_model_step.hip::step_variant): 0 = the
+  // ... each in VARIANTS of the attention / wo pair (kh_model_step.hip::step_variant): 0 = the
   // attention launch merges its time splits itself (valid at every position; nothing to merge below
   // position 256), 1 = the splits are merged by k_wo_comb (positions on the per-head path only), 2 = as 0
-  // with the per-head-only attention instantiation (positions below the group path, merge not deferrable)
+  // with the per-head-only attention instantiation (positions below the group path, merge not deferrable),
+  // 3 = attention and wo in one launch (kh_attn_wo.h, positions below 256)
   struct StepGraph {
     hipGraph_t g = nullptr;
     hipGraphExec_t e = nullptr;
@@ -204,6 +215,12 @@ void destroy_step_graphs(kh_model* m);
 int step_graph(kh_model* m, int n_forced, int variant, bool steps8, hipGraphExec_t* out);
 // the same for a graph of `nsteps` in {1, 2, 4, 8} steps (the tail of a run: 20 steps = 8 + 8 + 4)
 int step_graph_n(kh_model* m, int n_forced, int variant, int nsteps, hipGraphExec_t* out);
+// ---- kh_attn_wo.hip -------------------------------------------------------------------------
+kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long);
+void launch_attn_wo(kh_model* m, int l);
+void launch_ffn13_parts(kh_model* m, const KhFfn13Args& f);
+void launch_pf_attn_parts(kh_model* m, int l, int nvalid, int pos0);  // pf_q -> pf_att
+void launch_pf_wo_parts(kh_model* m, int l, int nvalid);              // pf_x += wo . pf_att
 // ---- kh_model_load.hip ----------------------------------------------------------------------
 // Make rows [0, rows) of the K / V cache usable before anything that touches them is enqueued: every layer, or one
 // (layer >= 0).  No-op for rows that are mapped already and for caches that are plainly allocated.  Newly mapped

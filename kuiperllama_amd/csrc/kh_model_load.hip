@@ -585,6 +585,11 @@ int finish_create(kh_model* m, SinCosJob* sincos = nullptr) {
   }
   KH_ALLOC(m->part_val, (size_t)m->nparts);
   KH_ALLOC(m->part_idx, (size_t)m->nparts);
+  m->awo = plan_attn_wo(c, m->sh_ffn.wg, m->attn_t_long);
+  if (m->awo.end > 0) {
+    KH_ALLOC(m->wo_part, (size_t)m->awo.parts * c.dim);
+    KH_ALLOC(m->x1, (size_t)c.dim);
+  }
 #undef KH_ALLOC
   pc.lap("caches, tables, plans, workspace");
   if (!m->kv.on) {  // a mapped-on-demand cache zeroes what it maps (kv_ensure)
@@ -675,7 +680,7 @@ extern "C" void kh_model_destroy(kh_model* m) {
   void* bufs[] = {m->x,      m->rms,    m->q,         m->att,       m->h1,       m->h3,
                   m->w2o,    m->logits, m->score,     m->sin_cache,
                   m->cos_cache, m->part_val, m->part_idx, m->d_pos, m->d_token,  m->d_next,
-                  m->d_forced, m->d_words, m->attn_ws};
+                  m->d_forced, m->d_words, m->attn_ws, m->wo_part, m->x1};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   kv_release(m);

@@ -192,7 +192,10 @@ void launch_prefill_chunk(kh_model* m, const int32_t* toks, int nvalid, int pos0
     // the prompt phase leaves K/V rows and nothing else (no logits): the last layer's K/V rows are
     // written, its attention, wo and FFN feed nothing
     if (l == c.layer_num - 1) break;
-    {
+    if (pos0 + nvalid <= m->awo.end) {  // as steps at these positions
+      launch_pf_attn_parts(m, l, nvalid, pos0);
+      launch_pf_wo_parts(m, l, nvalid);
+    } else {
       KhAttnArgs a = fill_attn(m, l);
       a.defer = 0;  // multi-token slices merge in the launch
       a.nsplit_g = m->attn_ns_g;  // not the decode step's variant: launch_attn_decode decides from the slice's positions
@@ -203,8 +206,8 @@ void launch_prefill_chunk(kh_model* m, const int32_t* toks, int nvalid, int pos0
       a.tok_stride = c.dim;
       a.ws_tok_bytes = m->pf_ws_tok_bytes;
       launch_attn_decode(a, pos0, m->attn_wg, m->stream, nvalid, pos0 + nvalid - 1);
+      pf_gemv_res(m, m->sh_wo, W.wo, m->pf_att, m->pf_x, c.dim, c.dim, nvalid, B);
     }
-    pf_gemv_res(m, m->sh_wo, W.wo, m->pf_att, m->pf_x, c.dim, c.dim, nvalid, B);
     {
       KhPfFfn13Args a;
       a.X = m->pf_x;
@@ -670,8 +673,13 @@ extern "C" int kh_model_prefill(kh_model* m, const int32_t* h_tokens, int32_t n,
   if ((rc = kv_ensure(m, pos0 + n)) != KH_OK) return rc;
   if ((rc = ensure_prefill_buffers(m)) != KH_OK) return rc;
   const int B = prefill_batch(m);
-  for (int t0 = 0; t0 < n; t0 += B)
-    launch_prefill_chunk(m, h_tokens + t0, n - t0 < B ? n - t0 : B, pos0 + t0, B);
+  for (int t0 = 0; t0 < n;) {
+    int k = n - t0 < B ? n - t0 : B;
+    const int one = m->awo.end - (pos0 + t0);  // positions left of attention and wo in one launch: a chunk ends there
+    if (one > 0 && k > one) k = one;
+    launch_prefill_chunk(m, h_tokens + t0, k, pos0 + t0, B);
+    t0 += k;
+  }
   return kh_launch_status();
 }
 

@@ -238,6 +238,10 @@ int attn_group_lanes(const kh_config& c) {
   return G < 16 ? 16 : G;
 }
 void launch_attn(kh_model* m, int l) {
+  if (m->step_var == 3) {
+    launch_attn_wo(m, l);
+    return;
+  }
   const kh_config& c = m->cfg;
   const KhAttnArgs a = fill_attn(m, l);
   const int wg = m->attn_wg;
@@ -253,6 +257,7 @@ KhGemvResArgs fill_wo(kh_model* m, int l) {
   a.vec = m->att;
   a.w = m->layers[l].wo;
   a.x = m->x;
+  a.xin = m->x;
   a.M = c.dim;
   a.K = c.dim;
   a.gshift = m->gshift;
@@ -278,6 +283,7 @@ KhGemvResArgs fill_wo(kh_model* m, int l) {
       KH_SEL_SP5C(Q, UU, 4, SP, __VA_ARGS__);               \
   } while (0)
 void launch_wo(kh_model* m, int l) {
+  if (m->step_var == 3) return;  // part of the attention launch
   const kh_config& c = m->cfg;
   const bool qn = c.is_quant;
   const int kh_launch_wg = m->sh_wo.wg;
@@ -315,6 +321,10 @@ void launch_ffn13(kh_model* m, int l) {
   a.hidden = c.hidden_dim;
   a.gshift = m->gshift;
   a.eps = c.rms_eps;
+  if (m->step_var == 3) {
+    launch_ffn13_parts(m, a);
+    return;
+  }
   const bool qn = c.is_quant;
   if (m->ring.ffn_r == 2) {  // plan_ring: int8, dim a multiple of 256 floats and at most 16 per thread
     hipLaunchKernelGGL((k_ffn13_ring<2, 4>), dim3(m->ring.ffn_grid), dim3(KH_WG),
@@ -331,6 +341,7 @@ void launch_w2(kh_model* m, int l) {
   a.vec = m->h1;
   a.w = m->layers[l].w2;
   a.x = m->x;
+  a.xin = m->step_var == 3 ? m->x1 : m->x;
   a.M = c.hidden_dim;
   a.K = c.dim;
   a.gshift = m->gshift;
@@ -400,6 +411,7 @@ void launch_sample(kh_model* m, int advance, int n_forced) {
 int step_variant(const kh_model* m, int pos_lo, int pos_hi) {
   (void)pos_lo;
   if (m->hy) return hy_step_variant(*m->hy, pos_hi);
+  if (pos_hi < m->awo.end) return 3;
   if (pos_hi < KH_ATTN_MIN_TS) return 0;         // pos + 1 <= 256 everywhere: one split
   if (pos_hi + 1 >= m->attn_t_long) return 0;    // some step runs the group path
   if (m->attn_defer && attn_active_splits(pos_hi, m->attn_ns, m->attn_ts_shift) <= m->attn_defer_max) return 1;
@@ -799,7 +811,7 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
   }
   const int n_forced = m->seq_cap + 1;
   if (exec == KH_EXEC_GRAPH) {
-    // all four graphs of variant 0 (1 / 2 / 4 / 8 steps) exist after the first generate of a .bin model, whatever its
+    // all four graphs of the first positions' variant (1 / 2 / 4 / 8 steps) exist after the first generate of a .bin model, whatever its
     // length (a warm-up run of 5 steps must leave the 8-step graph behind: capturing 656 nodes costs ~0.8 ms, which a
     // 20-step run would otherwise pay inside its timed loop); the other variants are captured when a run first
     // reaches position 256
@@ -816,7 +828,8 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
     // captured when a run first reaches it, by a host that is ahead of the steps before it: 120 steps of Gusorax 1024 x 8
     // across the border take 27.9 ms on the first call and 27.5 afterwards, and with both variants captured in front of the
     // loop the first call as a whole took 37.4 ms instead of 33.3.
-    const int v0 = m->hy ? step_variant(m, n_prompt - 1, std::min(total_steps, n_prompt - 1 + KH_GRAPH_STEPS) - 1) : 0;
+    const int v0 = m->hy ? step_variant(m, n_prompt - 1, std::min(total_steps, n_prompt - 1 + KH_GRAPH_STEPS) - 1)
+                         : step_variant(m, 0, KH_GRAPH_STEPS - 1);
     bool fresh[4] = {false, false, false, false};
     hipGraphExec_t ge = nullptr;
     for (int n = 1, k = 0; n <= KH_GRAPH_STEPS; n *= 2, ++k) {
@@ -887,6 +900,9 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
       // the 20-step form of the bench ran 8 + 8 + 1 + 1 + 1 + 1 and lost 0.3 % to it; now 8 + 8 + 4)
       int n = KH_GRAPH_STEPS;
       while (n > total_steps - s) n >>= 1;
+      // a position's bits follow from the position: no graph across the end of attention and wo in one launch
+      if (s < m->awo.end)
+        while (s + n > m->awo.end) n >>= 1;
       const bool keep = s == start && start > 0;  // first sampled step behind a prefill: alone, logits kept
       if (keep) n = 1;
       hipGraphExec_t ge = nullptr;

@@ -1,0 +1,65 @@
+"""Attention and wo of a decoded token in one launch (csrc/kh_attn_wo.h): positions at the edges of its 16-timestep tiles, of
+its two tiles a wave and of its range, and every shape of its rows."""
+import numpy as np
+import pytest
+import torch
+
+from kuiperllama_amd import binfmt
+
+pytestmark = pytest.mark.gpu
+
+
+def _spec(dim, hidden, heads, kv, name):
+    return binfmt.ModelSpec(dim, hidden, 2, heads, kv, 700, 512, True, binfmt.FAMILY_LLAMA, False, 64, binfmt.ROPE_HALF, 500000.0,
+                            1e-5, name)
+
+
+# head size 48: 16 and 32 lanes a row (stories15M's; two heads a group); 64: one float4 a lane (32 lanes, 64 lanes), two of them,
+# of which the second is half empty (seven heads), one and two rows, rows past the end of the last slice (dim 896, 1088)
+_SPECS = {s.name: s for s in (
+    _spec(288, 768, 6, 6, "48x6-6"), _spec(384, 768, 8, 4, "48x8-4"), _spec(512, 1408, 8, 4, "64x8-4"),
+    _spec(448, 1216, 7, 1, "64x7-1"), _spec(896, 1216, 14, 2, "64x14-2"), _spec(1024, 1408, 16, 8, "64x16-8"),
+    _spec(1088, 1408, 17, 1, "64x17-1"),  # seventeen heads a group: the launches of their own
+    _spec(2048, 1408, 32, 8, "64x32-8"), _spec(2048, 1408, 32, 4, "64x32-4"))}
+
+
+@pytest.mark.parametrize("name", sorted(_SPECS))
+def test_against_the_oracle_and_the_prompt_path(gpu, oracle, name):
+    """Logits within the bound of fp32 decode steps (4e-5, as for the attention in launches of its own); the prompt path of
+    several tokens a weight pass leaves the same bits, also where a chunk would cross the end of the range; words of captured and
+    eager steps are the same across it."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = _SPECS[name]
+    img_d = binfmt.synth_image(spec, seed=31, device=gpu, final_norm_std=1.0)  # words that wander
+    torch.cuda.synchronize()
+    img_h = img_d.cpu().numpy()
+    a, b = KuiperModel.from_device_image(img_d, spec), KuiperModel.from_device_image(img_d, spec)
+    om = oracle.OracleModel.from_spec(img_h, spec)
+    ko, vo = om.kv_cache()
+    rng = np.random.default_rng(3)
+    for l in range(spec.n_layers):
+        k, v = (rng.standard_normal((300, spec.kv_dim), dtype=np.float32) for _ in range(2))
+        k[rng.integers(0, 300, 6)] *= 6.0  # a few dominant keys: the waves' maxima differ
+        ko[l, :300], vo[l, :300] = k, v
+        a.write_kv(l, 0, k, v)
+        b.write_kv(l, 0, k, v)
+    for pos in (0, 1, 15, 16, 63, 127, 128, 143, 254, 255, 256):
+        tok = int(rng.integers(0, spec.vocab_size))
+        a.predict(tok, pos, exec="fused")
+        b.predict(tok, pos, exec="fused")
+        err = np.abs(a.logits() - om.forward(tok, pos)).max()
+        assert err <= 4e-5, f"position {pos}: {err:.3e}"
+    toks = [int(t) for t in rng.integers(0, spec.vocab_size, 24)]
+    a.prefill(toks[:-1], 240)  # 240 .. 262
+    for i, t in enumerate(toks):
+        b.predict(t, 240 + i, exec="fused")
+    a.predict(toks[-1], 263, exec="fused")
+    for l in range(spec.n_layers):
+        for x, y in zip(a.read_kv(l, 0, 264), b.read_kv(l, 0, 264)):
+            assert np.array_equal(x, y), l
+    assert np.array_equal(a.logits(), b.logits())
+    words, _ = a.generate(toks[:3], 270, exec="graph")
+    assert words == b.generate(toks[:3], 270, exec="fused")[0]
+    assert np.array_equal(a.logits(), b.logits())
+    a.close()
+    b.close()

@@ -965,14 +965,14 @@ int main(int argc, char** argv) {
     at.ws_stride = 1; at.nsplit_g = 0; at.t_long = 1 << 30; at.defer = 0; at.tok_stride = 0; at.ws_tok_bytes = 0;
     launch_attn_decode(at, 0, attn_wg, s);
     KhGemvResArgs w{};
-    w.vec = attc; w.w = KhLin{b.wo, nullptr, nullptr}; w.x = xc; w.M = dim; w.K = dim; w.gshift = 0;
+    w.vec = attc; w.w = KhLin{b.wo, nullptr, nullptr}; w.x = xc; w.xin = xc; w.M = dim; w.K = dim; w.gshift = 0;
     launch_res(w, cf->wo, fused_lds_bytes(false, dim), s);
     KhFfn13Args f{};
     f.x = xc; f.ffn_norm = b.fn; f.w1 = KhLin{b.w1, nullptr, nullptr}; f.w3 = KhLin{b.w3, nullptr, nullptr}; f.h = hc;
     f.dim = dim; f.hidden = hidden; f.gshift = 0; f.eps = 1e-5f;
     launch_ffn(f, cf->ffn, fused_lds_bytes(false, dim), s);
     KhGemvResArgs w2{};
-    w2.vec = hc; w2.w = KhLin{b.w2, nullptr, nullptr}; w2.x = xc; w2.M = hidden; w2.K = dim; w2.gshift = 0;
+    w2.vec = hc; w2.w = KhLin{b.w2, nullptr, nullptr}; w2.x = xc; w2.xin = xc; w2.M = hidden; w2.K = dim; w2.gshift = 0;
     launch_res(w2, cf->w2, fused_lds_bytes(false, hidden), s);
   };
   auto engine_layer = [&](int l, hipStream_t s) {
@@ -1051,7 +1051,7 @@ int main(int argc, char** argv) {
       CK(hipMemcpy(xc, x0, dim * 4, hipMemcpyDeviceToDevice));
       hipLaunchKernelGGL(k_ungran, dim3((dim + 255) / 256), dim3(256), 0, st, g_att, attc, dim);
       KhGemvResArgs w{};
-      w.vec = attc; w.w = KhLin{b.wo, nullptr, nullptr}; w.x = xc; w.M = dim; w.K = dim; w.gshift = 0;
+      w.vec = attc; w.w = KhLin{b.wo, nullptr, nullptr}; w.x = xc; w.xin = xc; w.M = dim; w.K = dim; w.gshift = 0;
       launch_res(w, cf->wo, fused_lds_bytes(false, dim), st);
       CK(hipStreamSynchronize(st));
       cmp_gran("x after wo", g_x2, xc, dim, true);
@@ -1062,7 +1062,7 @@ int main(int argc, char** argv) {
       CK(hipStreamSynchronize(st));
       cmp_gran("hidden*", g_h, hc, hidden, true);
       KhGemvResArgs w2{};
-      w2.vec = hc; w2.w = KhLin{b.w2, nullptr, nullptr}; w2.x = xc; w2.M = hidden; w2.K = dim; w2.gshift = 0;
+      w2.vec = hc; w2.w = KhLin{b.w2, nullptr, nullptr}; w2.x = xc; w2.xin = xc; w2.M = hidden; w2.K = dim; w2.gshift = 0;
       launch_res(w2, cf->w2, fused_lds_bytes(false, hidden), st);
       CK(hipStreamSynchronize(st));
       CK(hipMemcpy(ha.data(), xc, dim * 4, hipMemcpyDeviceToHost));

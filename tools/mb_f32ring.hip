@@ -139,7 +139,7 @@ int main(int argc, char** argv) {
     const int M = hidden, K = dim;
     const double bytes = (double)K * M * 4 + M * 4.0 + 2.0 * K * 4;
     auto args = [&](int l, float* xres) {
-      KhGemvResArgs a{}; a.vec = xh; a.w = KhLin{w + slab * l, nullptr, nullptr}; a.x = xres; a.M = M; a.K = K; a.gshift = 0; return a;
+      KhGemvResArgs a{}; a.vec = xh; a.w = KhLin{w + slab * l, nullptr, nullptr}; a.x = xres; a.xin = xres; a.M = M; a.K = K; a.gshift = 0; return a;
     };
     const size_t lds0 = fused_lds_bytes(false, M);
     optin(k_gemv_res<false, 8, 4, 4>, lds0);

@@ -262,7 +262,7 @@ int main(int argc, char** argv) {
     const double bytes = (double)wb + sb * 4.0 + M * 4.0 + 2.0 * K * 4;
     float* vec = which == 2 ? x : xh;
     auto args = [&](int l, float* xres) {
-      KhGemvResArgs a{}; a.vec = vec; a.w = KhLin{w + wb * l, sc + sb * l, nullptr}; a.x = xres; a.M = M; a.K = K; a.gshift = gshift; return a;
+      KhGemvResArgs a{}; a.vec = vec; a.w = KhLin{w + wb * l, sc + sb * l, nullptr}; a.x = xres; a.xin = xres; a.M = M; a.K = K; a.gshift = gshift; return a;
     };
     const size_t lds0 = fused_lds_bytes(true, M);
     optin(k_gemv_res<true, 2, 6, 2>, lds0);

@@ -80,7 +80,7 @@ int main() {
                            a.h = out; a.dim = dim; a.hidden = hidden; a.gshift = 0; a.eps = 1e-5f; return a; };
     const size_t lds0 = fused_lds_bytes(false, dim);
     report("1B fp32 ffn13 <false,8,2> 512x256", 512, 4, 9, [&](int l) { hipLaunchKernelGGL((k_ffn13<false, 8, 2>), dim3(512), dim3(256), lds0, S, fa(l)); }, NL);
-    auto wa = [&](int l) { KhGemvResArgs a{}; a.vec = xh; a.w = KhLin{w + slab * l, nullptr, nullptr}; a.x = out; a.M = hidden; a.K = dim; a.gshift = 0; return a; };
+    auto wa = [&](int l) { KhGemvResArgs a{}; a.vec = xh; a.w = KhLin{w + slab * l, nullptr, nullptr}; a.x = out; a.xin = out; a.M = hidden; a.K = dim; a.gshift = 0; return a; };
     const size_t lds1 = fused_lds_bytes(false, hidden);
     CK(hipFuncSetAttribute((const void*)k_gemv_res<false, 8, 4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds1));
     report("1B fp32 w2 <false,8,4,4> 512x512", 512, 8, 9, [&](int l) { hipLaunchKernelGGL((k_gemv_res<false, 8, 4, 4>), dim3(512), dim3(512), lds1, S, wa(l)); }, NL);
