@@ -621,7 +621,14 @@ void plan_decode_shapes(bool quant, int dim, int hidden_dim, int kv_dim, int voc
   // w2 re-stages the hidden-sized input in every workgroup: 512-thread workgroups halve that
   // L2 -> LDS traffic for the same number of waves (measured 14.1 -> 11.8 us on Llama-3.2-1B)
   out[3] = pick_shape(quant, dim / 2, hidden_dim, 4, "KH_SHAPE_W2", KH_WG_MAX, KH_WG_MAX, true, /*u3=*/true);
-  out[4] = pick_shape(quant, (vocab_size + 1) / 2, dim, 1, "KH_SHAPE_CLS", quant ? KH_WG : KH_WG_MAX, KH_WG_MAX);
+  // ... but not where it leaves three quarters of the CUs without one (stories15M, 288 rows of 768: 18 workgroups 2.55 us, 36
+  // of 256 threads 2.16)
+  if (out[3].grid < 64) out[3] = pick_shape(quant, dim / 2, hidden_dim, 4, "KH_SHAPE_W2", KH_WG, KH_WG_MAX, true, /*u3=*/true);
+  // rows of less than 2 KB keep less in flight per wave than a trip to memory hides: 16 waves per CU instead of 8 (32000 rows of
+  // 288 floats: 9.8 -> 7.8 us; 151936 rows of 896, 3.5 KB, lose 3 %)
+  const bool short_rows = !quant && dim < 512;
+  out[4] = pick_shape(quant, (vocab_size + 1) / 2, dim, 1, "KH_SHAPE_CLS", quant || short_rows ? KH_WG : KH_WG_MAX, KH_WG_MAX,
+                      short_rows);
 }
 
 // The int8 ffn13 and classifier launches run on the LDS-DMA ring kernels (kh_fused_ring.h) when the geometry fits
