@@ -367,7 +367,7 @@ struct Runner {
       TRY((lg_launch<T, LG_F32>(s, zr)));
       moe_route_launch(s, ra);
     }
-    const int bm = lg_group_bm((long)ps.T * f.top, f.n_out());
+    const int bm = lg_group_bm((long)ps.T * f.top, f.n_out(), f.E, 2 * f.ffp, (size_t)f.E * 2 * f.ffp * f.gu.ld * sizeof(T));
     ListArgs li{hy.moe_id, hy.moe_count, hy.moe_rows, hy.moe_slot, hy.tiles, hy.n_tiles, ps.T, f.top, f.E, bm};
     hipLaunchKernelGGL(k_moe_lists, dim3(moe_blocks(ps.T)), dim3(KH_MOE_LT), 0, s, li);
     const long rows = (long)ps.T * f.top;

@@ -23,6 +23,7 @@
 //   * Grouped form (experts): a device-side tile list maps blockIdx.y to (expert, first row, rows); the rows of X are
 //     gathered through an index list.  Batched form (heads): blockIdx.z strides.
 #pragma once
+#include <math.h>
 #include <type_traits>
 #include <vector>
 
@@ -67,7 +68,7 @@ template <class T, int BM, int BN, bool GROUPED, int WM = 2, int WN = 2>
 struct LgCfg {
   static constexpr bool WIDE = WM * WN == 8;  // one workgroup of eight waves per CU: the whole LDS is its
   static constexpr int XS = WIDE ? 160 * 8 / (BM + BN) : BM + BN >= 192 ? 2 : (BM + BN >= 128 ? 3 : 4);  // stages of the tokens' ring
-  static constexpr int WS = !WIDE && BM + BN >= 256 && GROUPED ? 3 : XS;                                 // ... of the weights'
+  static constexpr int WS = !WIDE && BM + BN == 256 && GROUPED ? 3 : XS;                                 // ... of the weights'
   static constexpr int LDS = (XS * BM + WS * BN) * 128;
 };
 
@@ -137,7 +138,7 @@ __device__ __forceinline__ void lg_store(const LgArgs& a, int tok, int f, f32x4 
 }
 
 template <class T, int BM, int BN, int EPI, bool GROUPED, int WM = 2, int WN = 2>
-__global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
+__global__ __launch_bounds__(64 * WM * WN, BM == 192 ? 2 : 1) void k_lgemm(const LgArgs a) {
   typedef Tile<T> TL;
   typedef typename TL::frag frag;
   constexpr int NWV = WM * WN;
@@ -255,6 +256,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
   if (TM == 1 || (TM <= 4 && live <= 1)) loop(std::integral_constant<int, 1>{});
   else if (TM == 2 || (TM <= 4 && live == 2)) loop(std::integral_constant<int, TM < 2 ? 1 : 2>{});
   else if (TM <= 4 && live == 3) loop(std::integral_constant<int, TM < 3 ? 1 : 3>{});
+  else if (TM == 6 && live <= 2) loop(std::integral_constant<int, TM < 2 ? 1 : 2>{});
+  else if (TM == 6 && live <= 4) loop(std::integral_constant<int, TM < 4 ? 1 : 4>{});
+  else if (TM == 6 && live == 5) loop(std::integral_constant<int, TM < 5 ? 1 : 5>{});
   else loop(std::integral_constant<int, TM>{});
   // ---- epilogue: lane (fr, fh) of tile (n, m): token mt0 + .. + fr, features f .. f + 3
   auto feature = [&](int n) __attribute__((always_inline)) { return f0 + wn * (BN / WN) + n * 16 + 4 * fh; };
@@ -293,8 +297,16 @@ __global__ __launch_bounds__(64 * WM * WN) void k_lgemm(const LgArgs a) {
 // tiles: 12.7 us instead of 9.9).  Experts gain nothing from either (130 us of gate and up with 256 x 256, 137 with 256 x 128): their
 // tiles are a third empty or wait for HBM.  Where 64 x 64 leaves half of the CUs idle, 32 x 64: what one CU pulls is the time (160
 // features of K 4096, 2048 / 732 tokens: 25.2 / 24.0 -> 18.6 / 17.1 us).  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
-static inline int lg_group_bm(long rows, int groups) {
+// (rows: token and choice pairs, over `groups` outputs; w_bytes: weights of all experts of the gate and up product, N columns)
+// 192 rows for 128 where an expert's share lies so close below 128 or 256 that some of them pass it, and all tiles are one round of two
+// workgroups per CU: a tile more for one expert in eight is a second round for 34 workgroups.  1100 tokens, 7 of 32 experts, 1024 x
+// 1024: 36.1 -> 30.6 and 26.4 -> 21.8 us (fp32: the prompt 2791 -> 2418).  Several rounds hide it (2048 tokens: 128.7 / 131.5), and more weights
+// wait for HBM longer than the two stages of them that 192 rows leave room for (740 tokens, 6 of 36, 2048 x 2048, 268 MB: the prompt 1299 / 1354).
+static inline int lg_group_bm(long rows, int groups, int experts, int N, size_t w_bytes) {
   const long per = rows / (groups > 0 ? groups : 1);
+  const double most = per + 2.0 * sqrt((double)per);  // of even choices: two deviations
+  const long n = (per + 127) / 128;
+  if (per > 64 && most > 128.0 * n && most <= 192.0 * n && experts * n * ((N + 127) / 128) <= 512 && w_bytes <= (128u << 20)) return 192;
   return per > 64 ? 128 : (per > 24 ? 64 : 32);
 }
 template <class T, int EPI>
@@ -322,6 +334,7 @@ int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, in
 #define KH_LG_WIDE(BM, BN) return go(k_lgemm<T, BM, BN, EPI, false, 2, 4>, BM, BN, LgCfg<T, BM, BN, false, 2, 4>::LDS, 512)
   if constexpr (EPI == LG_T || EPI == LG_GATED) {
     if (a.tiles) {
+      if (group_bm == 192) KH_LG_GO(192, 128, true);
       if (group_bm == 128) KH_LG_GO(128, 128, true);
       if (group_bm == 64) KH_LG_GO(64, 128, true);
       KH_LG_GO(32, 64, true);

@@ -36,6 +36,13 @@ def test_rows_of_experts(gpu, dtype, top):
     _prompt(U.Model(U.config([U.with_ff(U.mamba(), experts=9, identity=3, top=top, ff=20)], width=1100, vocab=60)), dtype, 33, (20,))
 
 
+@BOTH
+@pytest.mark.parametrize("experts,top,n", [(4, 2, 240), (3, 1, 345), (5, 1, 610), (2, 1, 490)])
+def test_expert_tiles_of_192_rows(gpu, dtype, experts, top, n):
+    """Shares just below 128 and 256 rows (csrc/kh_lgemm.h::lg_group_bm), spread by the choices: tiles of few and of many 16-row units."""
+    _prompt(U.Model(U.config([U.with_ff(U.mamba(), experts=experts, top=top, ff=72)], width=136, vocab=60)), dtype, n, (), max_seq_len=640)
+
+
 @pytest.mark.parametrize("dim,vdim,window,n,cuts", [(128, 128, 40, 65, ()), (128, 128, 600, 700, (63, 64, 400)), (100, 90, 200, 300, (129,)),
                                                     (128, 128, 700, 33, (1, 2)), (65, 128, 31, 200, (31, 190))])
 def test_heads_of_four_sets(gpu, dim, vdim, window, n, cuts):
