@@ -406,7 +406,7 @@ int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32
  * KH_PAIR_ATTN (0 = attention of a prompt slice on the fp32 matrix cores; KH_PG_ATTN_QT selects it too),
  * KH_SHAPE_DEBUG, KH_HY_DECODE (0 = single-token batches of layer-list models run on the pass kernels), KH_HY_EXPAND (0 = latent
  * attention of prompts in its absorbed form), KH_HY_TMAX (tokens of one pass, 32 ... 2048), KH_HY_ROWS (16, 64 or 128: row tiles
- * of the attention kernels of a pass), KH_HY_TAIL (0 = the last layer of a pass for all its tokens), KH_HY_STEP_FAIL (the step of
+ * of the attention kernels of a pass), KH_HY_TAIL (0 = the last layer of a pass for all its tokens), KH_HY_FORK (0 = a pass on one stream), KH_HY_STEP_FAIL (the step of
  * their generate loop reports KH_ERR_INTERNAL before its first launch)) lives in ONE process-wide key -> value table, seeded once from the KH_* variables of
  * the environment when the library is first used and changed afterwards only through kh_debug_set
  * (value NULL = unset).  No launch path reads the environment.  Hooks that shape a model (KH_SHAPE_*,

@@ -156,6 +156,9 @@ struct Hybrid {
   LgTile* tiles = nullptr;
   int max_tiles = 0;
   int wl_rows = 0;        // rows wlogits / xw hold
+  // a pass's mixers run beside its feed-forwards, on a stream of their own (kh_hybrid_pass.hip, Runner::fork)
+  hipStream_t aux = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   // pass tables: pinned staging and device copy
   int32_t *h_tab = nullptr, *d_tab = nullptr;
   size_t tab_cap = 0;

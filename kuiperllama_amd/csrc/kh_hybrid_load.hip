@@ -688,6 +688,11 @@ int alloc_workspace(kh_model* m) {
   TRY(zi(&hy.moe_slot, T * top));
   TRY(zi(&hy.moe_count, (size_t)moe_blocks((int)T) * experts));
   TRY(zi(&hy.n_tiles, 1));
+  {
+    TRY((int)hipStreamCreateWithFlags(&hy.aux, hipStreamNonBlocking));
+    TRY((int)hipEventCreateWithFlags(&hy.ev_fork, hipEventDisableTiming));
+    TRY((int)hipEventCreateWithFlags(&hy.ev_join, hipEventDisableTiming));
+  }
   TRY(zi((int32_t**)&hy.tiles, tiles * 4));
   hy.max_tiles = (int)tiles;
   hy.wl_rows = 64;
@@ -885,6 +890,7 @@ int hy_create(const char* config, size_t config_len, const void* tensors, size_t
 void hy_destroy(kh_model* m) {
   Hybrid* h = m->hy;
   if (!h) return;
+  if (h->aux) (void)hipStreamSynchronize(h->aux);
   void* dev[] = {h->farena, h->state, h->x, h->x0, h->mix, h->f32a, h->y, h->sh, h->dt, h->bc, h->z, h->ends, h->dtsum,
                  h->moe_w, h->id_w, h->sh_g, h->wlogits, h->xn1, h->xn2, h->a0, h->a1, h->a2, h->h, h->hs, h->xw,
                  h->moe_id, h->moe_rows, h->moe_slot, h->moe_count, h->n_tiles, h->tiles, h->kx, h->vx, h->d_tab, h->d_one};
@@ -892,6 +898,9 @@ void hy_destroy(kh_model* m) {
     if (p) (void)hipFree(p);
   for (float2* t : h->rope_tabs) (void)hipFree(t);
   if (h->h_tab) (void)hipHostFree(h->h_tab);
+  if (h->ev_fork) (void)hipEventDestroy(h->ev_fork);
+  if (h->ev_join) (void)hipEventDestroy(h->ev_join);
+  if (h->aux) (void)hipStreamDestroy(h->aux);
   delete h;
   m->hy = nullptr;
 }

@@ -1,6 +1,7 @@
 // kh_hybrid_pass.hip — layer-list models: one pass over T tokens of any number of sequences.  The tokens of all
 // entries are concatenated (no padding); linear layers see one [T, K] matrix, the mixers find each token's sequence
 // through the pass tables, and every sequence continues from the cache rows and the recurrent state of its slot.
+#include <math.h>
 #include <stdio.h>
 #include <string.h>
 
@@ -398,6 +399,52 @@ struct Runner {
     return KH_OK;
   }
 
+  // Does a layer's mixer run beside its feed-forward, on the other stream?  Two pairs of event and wait cost the shorter branch some
+  // 17 us and the host 20, so the layer has to be worth it: about 14 us of weights and products beside its launches.  us a
+  // prompt in one stream / two: Gusorax 1024 x 8, 3 tokens 524 / 569, 8 568 / 567, 16 577 / 565, 150 677 / 621, 1100 1097 / 930, 512 x 8, 50
+  // 445 / 524; Gufanex 2048 x 4, 20 tokens 733 / 650, 400 1136 / 964, 2048 2060 / 1889, 512 x 4, 17 338 / 349.
+  bool beside(const HyLayer& l) const {
+    const HyMoe& f = l.ff;
+    if (ps.T < 2 || !f.on || dbg_off("KH_HY_FORK")) return false;  // (one token: hy_unfused_step, which may be captured)
+    auto size = [](const HyMat& w) { return (double)w.N * w.ld; };
+    double all = size(l.out_mat()) + size(f.sgu) + size(f.sdown), one = 0.0, met = 0.0, mine = 0.0;
+    if (l.mixer == HY_MAMBA1) all += size(l.mb.in) + size(l.mb.x) + size(l.mb.dt);
+    else if (l.mixer == HY_LATENT) all += size(l.la.dqkv) + size(l.la.uq) + size(l.la.uk) + size(l.la.uv);
+    else all += size(l.ha.qkvg);
+    if (f.top) {
+      const double p = (double)f.top / f.n_out();  // of an expert to be a token's choice, routed evenly
+      one = 2.0 * f.ffp * f.gu.ld + (double)hy.c.width * f.down.ld;
+      met = f.E * (1.0 - pow(1.0 - p, ps.T));
+      mine = f.E * p;
+    }
+    const double us = (all + met * one) * sizeof(T) / 5e6 + 2.0 * ps.T * (all + mine * one) / (sizeof(T) == 2 ? 6e8 : 1e8);
+    return us >= 14.0;
+  }
+  bool forked = false;
+  // A layer's mixer and its feed-forward read the same norms and write nothing in common: in a parallel block neither needs the other.
+  template <class F>
+  int fork(F&& mixer) {
+    KH_CHECK_HIP(hipEventRecord(hy.ev_fork, s));
+    KH_CHECK_HIP(hipStreamWaitEvent(hy.aux, hy.ev_fork, 0));
+    forked = true;
+    hipStream_t main = s;
+    s = hy.aux;
+    const int rc = mixer();
+    s = main;
+    if (rc != KH_OK) return rc;
+    KH_CHECK_HIP(hipEventRecord(hy.ev_join, hy.aux));
+    return KH_OK;
+  }
+  int join() {
+    if (!forked) return KH_OK;
+    forked = false;
+    KH_CHECK_HIP(hipStreamWaitEvent(s, hy.ev_join, 0));
+    return KH_OK;
+  }
+  ~Runner() {
+    if (forked) (void)hipStreamSynchronize(hy.aux);  // an error between fork and join
+  }
+
   int layers() {
     for (size_t i = 0; i < hy.runs.size(); ++i) {
       const HyRun& r = hy.runs[i];
@@ -406,11 +453,19 @@ struct Runner {
       const bool through = r.pass >= 0 && hy.enter.N;
       if (through) TRY(enter(i == 0));
       TRY(combine(&l, i == 0 && !through, r.pass));
-      TRY(l.mixer == HY_MAMBA1 ? mamba(r, l.mb, state_only)
-          : l.mixer == HY_LATENT ? latent(r, l.la, state_only) : heads(r, l.ha, state_only));
-      if (state_only) break;
+      auto mixer = [&]() -> int {
+        return l.mixer == HY_MAMBA1 ? mamba(r, l.mb, state_only)
+               : l.mixer == HY_LATENT ? latent(r, l.la, state_only) : heads(r, l.ha, state_only);
+      };
+      if (state_only) {
+        TRY(mixer());
+        break;
+      }
+      if (beside(l)) TRY(fork(mixer));
+      else TRY(mixer());
       pend.mix = hy.mix;
       if (l.ff.on) TRY(feed_forward(l.ff, l.n2.on ? hy.xn2 : hy.xn1));
+      TRY(join());
       if (hy.probe) {
         TRY(combine(nullptr, false, -1));
         const int64_t n = (int64_t)ps.T * hy.c.width;
