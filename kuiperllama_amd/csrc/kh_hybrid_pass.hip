@@ -637,7 +637,8 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
   }
   memcpy(hy.h_tab, all.data(), all.size() * 4);
   KH_CHECK_HIP(hipMemcpyAsync(hy.d_tab, hy.h_tab, all.size() * 4, hipMemcpyHostToDevice, m->stream));
-  float* out = h_logits;
+  float* const pin = h_logits ? logits_pin(m, (size_t)n_want * hy.c.vocab) : nullptr;
+  float* out = pin ? pin : h_logits;
   for (size_t i = 0; i < passes.size(); ++i) {
     Pass& p = passes[i];
     const Off& o = offs[i];
@@ -652,7 +653,9 @@ int hy_forward(kh_model* m, const HyEntry* e, int n, const int32_t* want, int n_
     TRY(hy.f32 ? run_pass<float>(m, p, out) : run_pass<bf16>(m, p, out));
     if (out) out += (size_t)p.n_want * hy.c.vocab;
   }
-  if (h_logits) KH_CHECK_HIP(hipStreamSynchronize(m->stream));
+  if (!h_logits) return KH_OK;
+  KH_CHECK_HIP(hipStreamSynchronize(m->stream));
+  if (pin) memcpy(h_logits, pin, (size_t)n_want * hy.c.vocab * sizeof(float));
   return KH_OK;
 }
 
