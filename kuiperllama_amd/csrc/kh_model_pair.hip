@@ -13,11 +13,14 @@
 using namespace khm;
 
 namespace {
-// Tile and K split of one GEMM from a model of the busiest CU: a workgroup's stage takes at least `lat` (one or more stages
-// in flight against memory latency), and `n` workgroups side by side on a CU take n `sat` per stage together.  Both numbers
-// (us) were fitted to 18 tile / split combinations of the four GEMMs of Llama-3.2-1B fp32 and Llama-2-7B int8 at 40 ... 2000
-// tokens: the choice was on average 0.6 % (fp32) and 0.3 % (int8) behind the fastest combination measured, 5 % at worst.  They
-// belong to the tile and the 256 CUs, not to a model; other widths take them as they are.
+// Tile and K split of one GEMM from a model of its time (us): a workgroup's stage takes at least `lat` (one or more stages in
+// flight against memory latency), `n` workgroups side by side on a CU take n `sat` per stage together, every workgroup of a CU has
+// a start and an end, and partial rows are written and read back.  Where some CUs have a workgroup more than others, n lies
+// between the most and the mean: they compete for what lies behind the CUs as well.  The numbers were fitted to all twelve tile
+// and split combinations of the four GEMMs of five models (Llama-3.2-1B, TinyLlama, Qwen2.5-0.5B, stories15M; Llama-2-7B int8) at 40 ...
+// 2000 tokens, 44 lengths: the choice is on average 0.4 % (fp32, 14 % at worst) and 0.01 % (int8, 0.2 %) behind the fastest
+// combination measured, their sum 0.2 and 0.00 %; with the busiest CU alone and numbers from 18 combinations of two models 2.4
+// (29) and 0.7 (16), the sum 2.1 and 0.5 %.  They belong to the tile and the 256 CUs, not to a model; other widths take them as they are.
 // The largest tile of a type is the largest whose registers do not spill: 8 x 2 fragments a wave for fp32, 7 x 2 (112
 // tokens) for int8, where 8 x 2 spills 18 to 24 registers, the sums of a 64-column group standing beside the accumulators.
 // Against the tiled fp32-MFMA kernel (k_pg_gemm), us at 40 / 128 / 512 / 2000 tokens, w1 + w3 of either model:
@@ -33,10 +36,16 @@ struct PairTile {
   double lat, sat;
 };
 const PairTile kPairTiles[2][4] = {
-    {{128, 128, 2, 1.44, 0.73}, {64, 128, 2, 0.57, 0.445}, {32, 128, 2, 0.40, 0.315}, {32, 64, 2, 0.20, 0.30}},  // fp32
-    {{112, 128, 2, 1.22, 0.95}, {64, 128, 2, 0.72, 0.63}, {32, 128, 2, 0.53, 0.42}, {128, 256, 1, 1.95, 1.95}}};  // int8
+    {{128, 128, 2, 1.028, 0.752}, {64, 128, 2, 0.592, 0.471}, {32, 128, 2, 0.484, 0.348}, {32, 64, 2, 0.389, 0.228}},  // fp32
+    {{112, 128, 2, 1.346, 0.885}, {64, 128, 2, 0.850, 0.592}, {32, 128, 2, 0.615, 0.414}, {128, 256, 1, 2.116, 2.116}}};  // int8
+// of a workgroup: its start and end; of partial rows: of their time at 4 TB/s; weight of the busiest CU against the mean
+const struct {
+  double ends, part, most;
+} kPairCost[2] = {{1.833, 0.650, 0.444}, {2.167, 0.929, 1.0}};
 
-PairShape pair_shape(bool q, int T, int N, int K, bool resid, double* time_us = nullptr) {
+// resid: a product that is added to the residual (wo, w2).  gated: w1 + w3, whose scales the product behind it has to fold in twice
+// as often where a tile leaves them per 32 columns (Qwen2.5-0.5B, 41 tokens, 32 x 64 instead of 32 x 128 there: w2 24 -> 25 us).
+PairShape pair_shape(bool q, int T, int N, int K, bool resid, bool gated, double* time_us = nullptr) {
   PairShape best{0, 1};
   double best_us = -1.0;
   for (int i = 0; i < 4; ++i)
@@ -45,11 +54,12 @@ PairShape pair_shape(bool q, int T, int N, int K, bool resid, double* time_us = 
       const int stages = K / (q ? 64 : 32);
       if (kz > 1 && stages / kz < 4) break;
       const long wgs = (long)((N + t.bn - 1) / t.bn) * ((T + t.bm - 1) / t.bm) * kz;
-      const long per_cu = (wgs + 255) / 256, rest = per_cu % t.occ;
-      double us = (double)(per_cu / t.occ) * std::max(t.lat, t.occ * t.sat);
-      if (rest) us += std::max(t.lat, (double)rest * t.sat);
-      us *= (double)stages / kz;
-      if (kz > 1) us += (double)kz * T * N * 8 / 4.0e6;  // partial rows, written and read back at 4 TB/s
+      const long most = (wgs + 255) / 256, rounds = (most - 1) / t.occ;
+      const double last = kPairCost[q].most * most + (1.0 - kPairCost[q].most) * std::max(wgs / 256.0, 1.0) - (double)(rounds * t.occ);
+      double us = rounds * std::max(t.lat, t.occ * t.sat) + std::max(t.lat, last * t.sat);
+      us = us * stages / kz + kPairCost[q].ends * most;
+      if (kz > 1) us += kPairCost[q].part * kz * T * N * 8 / 4.0e6;
+      if (gated && t.bn < 128) us *= 1.06;
       if (best_us < 0 || us < best_us) {
         best_us = us;
         best = PairShape{i, kz};
@@ -83,14 +93,14 @@ int pair_go(hipStream_t s, KhPairArgs a, int kz) {
   }
   a.tiles_t = (a.T + C::BM - 1) / C::BM;
   a.tiles_f = (a.N + C::BN - 1) / C::BN;
-  hipLaunchKernelGGL(kern, dim3((a.tiles_f + 7) / 8 * 8 * a.tiles_t, kz), dim3(64 * C::NW), C::LDS, s, a);
+  hipLaunchKernelGGL(kern, dim3((a.tiles_f * a.tiles_t + 7) / 8 * 8, kz), dim3(64 * C::NW), C::LDS, s, a);
   return KH_OK;
 }
 // *kz_out: K slices whose partial rows the next RMSNorm has to add (0: the epilogue added itself)
 // *fine_out: SWIGLU left a scale per 32 columns instead of 64
 template <int EPI>
 int pair_launch(kh_model* m, const KhPairArgs& a, int* kz_out, int* fine_out = nullptr) {
-  PairShape sh = pair_shape(m->cfg.is_quant, a.T, a.N, a.K, EPI == KH_PG_RESID);
+  PairShape sh = pair_shape(m->cfg.is_quant, a.T, a.N, a.K, EPI == KH_PG_RESID, EPI == KH_PG_SWIGLU);
   if (const char* e = dbg("KH_PAIR_SHAPE")) {  // test hook "tile,kz"
     int t = 0, kz = 1;
     if (sscanf(e, "%d,%d", &t, &kz) == 2 && t >= 0 && t < 4 && (kz == 1 || kz == 2 || kz == 4))
@@ -127,7 +137,7 @@ extern "C" int kh_plan_pair_shapes(int32_t dim, int32_t hidden_dim, int32_t kv_d
   if (!pair_geometry(c)) return KH_ERR_UNSUPPORTED;
   const PairDims d = pair_dims(c);
   for (int i = 0; i < 4; ++i) {
-    const PairShape s = pair_shape(c.is_quant, T, d.N[i], d.K[i], i & 1);
+    const PairShape s = pair_shape(c.is_quant, T, d.N[i], d.K[i], i & 1, i == 2);
     const PairTile& t = kPairTiles[c.is_quant][s.tile];
     int32_t* o = out16 + 4 * i;
     o[0] = t.bm;
@@ -148,31 +158,31 @@ bool pair_geometry(const kh_config& c) {
 }
 
 // Is the last of T tokens of a pass cheaper in the pass than as a step of its own?  The step reads a layer's weights once more
-// (5 TB/s behind 10 us of launches a layer); in the pass the token may open another row of tiles, and where the model of
-// pair_shape sees a near tie the step was faster.  Time to the first token, ms, step of its own / in the pass, T tokens:
-// Llama-3.2-1B 17 2.71 / 2.10, 193 3.86 / 3.16, 512 5.43 / 4.57, 641 6.68 / 6.23; Qwen2.5-0.5B 41 2.41 / 1.92; TinyLlama 1793
-// 14.4 / 14.1; Llama-2-7B int8 33 6.37 / 5.36, 225 12.3 / 11.2, 617 24.1 / 22.3; of 55 lengths the rule erred at two, int8 561
-// 21.7 / 22.1 and Qwen 1025 5.59 / 5.73.  Not taken: Llama-3.2-1B 513 5.18 / 5.43, 1025 8.10 / 9.05; Llama-2-7B int8 65 6.83 /
-// 7.07, 449 17.1 / 17.3.
+// (5 TB/s behind 10 us of launches a layer); in the pass the token may open another row of tiles.  Time to the first token, ms,
+// step of its own / in the pass, T tokens.  Taken: Llama-3.2-1B 193 3.65 / 3.12, 257 3.96 / 3.86, 641 6.50 / 6.12; TinyLlama 641
+// 6.95 / 6.58, 705 7.50 / 7.31, 1473 13.3 / 11.9; Qwen2.5-0.5B 513 3.88 / 3.32, 833 4.74 / 4.48, 1153 5.62 / 5.19; Llama-2-7B
+// int8 113 8.93 / 7.51, 225 12.0 / 11.0, 673 26.4 / 25.9.  Not taken: Llama-3.2-1B 513 5.33 / 5.63, 1025 8.17 / 8.59; TinyLlama 1409
+// 11.65 / 11.95; Llama-2-7B int8 65 6.88 / 7.22, 321 14.5 / 15.3, 641 23.4 / 24.8.  Of 34 lengths, most of them where the last token
+// opens a row of tiles, the rule errs at one, Qwen2.5-0.5B 1665 6.96 / 6.77.
 bool pair_takes_last(const kh_config& c, int T) {
   if (T < 2) return false;
   const PairDims d = pair_dims(c);
   double more = 0.0, bytes = 0.0;
   for (int i = 0; i < 4; ++i) {
     double with = 0.0, without = 0.0;
-    (void)pair_shape(c.is_quant, T, d.N[i], d.K[i], i & 1, &with);
-    (void)pair_shape(c.is_quant, T - 1, d.N[i], d.K[i], i & 1, &without);
+    (void)pair_shape(c.is_quant, T, d.N[i], d.K[i], i & 1, i == 2, &with);
+    (void)pair_shape(c.is_quant, T - 1, d.N[i], d.K[i], i & 1, i == 2, &without);
     more += with - without;
     bytes += (double)d.N[i] * d.K[i] * (c.is_quant ? 1 : 4);
   }
-  return more < 0.8 * (10.0 + bytes / 5.0e6);
+  return more < 10.0 + bytes / 5.0e6;
 }
 
 int pair_part_rows(const kh_config& c, int rows) {
   int most = 0;
   for (int T = 1; T <= rows; ++T)
     for (int K : {c.dim, c.hidden_dim}) {
-      const int kz = pair_shape(c.is_quant, T, c.dim, K, true).kz;
+      const int kz = pair_shape(c.is_quant, T, c.dim, K, true, false).kz;
       if (kz > 1) most = std::max(most, kz * T);
     }
   return most;

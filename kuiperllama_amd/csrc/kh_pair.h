@@ -144,17 +144,19 @@ struct PairCfg {
   static_assert(NW % 2 == 0 && XR % NW == 0 && WR % NW == 0, "every wave issues the same number of requests");
 };
 
-// blockIdx.x -> (row tile, token tile): the token tiles of a row tile run on one XCD (blocks go round the XCDs) one after
-// the other, so its weights cross HBM once.  blockIdx.y = K slice (RESID).
+// blockIdx.x -> (row tile, token tile): every XCD (blocks go round them) takes an eighth of the tiles, row tile by row tile, so the
+// token tiles of a row tile run on one XCD, or on two, and its weights cross HBM once or twice.  (Whole row tiles an XCD leave some
+// with one more than others: 20 of them by 25 token tiles, wq + wk + wv of TinyLlama at 777 tokens, 72.8 -> 48.1 us.)  blockIdx.y = K
+// slice (RESID).
 template <bool Q, int EPI, int TM, int TN, int WM, int WN, int NST>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_pair_gemm(const KhPairArgs a) {
   constexpr bool GROUP = EPI == KH_PG_RESID;
   typedef PairCfg<Q, GROUP, TM, TN, WM, WN, NST> C;
   extern __shared__ __attribute__((aligned(1024))) char smem_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int xcd = (int)blockIdx.x & 7, bj = (int)blockIdx.x >> 3;
-  const int ft = bj / a.tiles_t * 8 + xcd, tt = bj % a.tiles_t;
-  if (ft >= a.tiles_f) return;  // uniform: the grid is rounded up to eight row tiles
+  const int xcd = (int)blockIdx.x & 7, all = a.tiles_f * a.tiles_t, tile = (xcd * all >> 3) + ((int)blockIdx.x >> 3);
+  if (tile >= (xcd + 1) * all >> 3) return;  // uniform: the grid is rounded up
+  const int ft = tile / a.tiles_t, tt = tile % a.tiles_t;
   const int t0 = tt * C::BM, f0 = ft * C::BN;
   const int K = a.K;
   // place f of the stacked rows -> matrix, row.  Runs of 16 places are runs of 16 rows: SWIGLU takes 16 rows of w1, the
