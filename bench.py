@@ -52,7 +52,7 @@ import torch
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-from kuiperllama_amd import binfmt  # noqa: E402
+from kuiperllama_amd import _ffi, binfmt  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0  # MI355X_MICROARCH.md: 8.0 TB/s spec (6.29 TB/s measured float4 copy)
 # logits vs the oracle at one greedy step (tests/test_model_gpu.py holds the same bounds at full size)
@@ -64,12 +64,13 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def ffn13_bytes(spec: binfmt.ModelSpec) -> float:
+def ffn13_bytes(spec: binfmt.ModelSpec, parts: int = 0) -> float:
     """Algorithmic bytes of one ffn13 launch: w1 and w3 rows once (+ scales), x and the norm
-    weight once, h written once."""
+    weight once, h written once.  parts: partial sums of wo that the launch adds to x (k_ffn13_parts), each
+    read once, and their sum written once."""
     n = 2 * spec.hidden_dim * spec.dim
     w = n + (n // spec.group_size) * 4 if spec.quant else n * 4
-    return float(w + 2 * spec.dim * 4 + spec.hidden_dim * 4)
+    return float(w + 2 * spec.dim * 4 + spec.hidden_dim * 4 + (parts + 1 if parts else 0) * spec.dim * 4)
 
 
 def build_model(spec, device_index, seed=1234, max_seq_len=0):
@@ -446,18 +447,21 @@ def long_context(m, spec, dev):
             m.write_kv_device(l, r0, kv[0], kv[1])
     torch.cuda.synchronize(dev)
     out = {}
-    wo_short = m.profile_kernel("wo", 64, reps=4)  # wo with a plain input vector (nothing to merge)
+    # wo with a plain input vector (nothing to merge): as the GQA group path launches it (below position 256 it may be
+    # part of the attention launch)
+    grouped = [p for p in poss if _ffi.plan_attention(spec.n_heads, spec.kv_mul, spec.head_size, cache_len, p)["group_path"]]
+    wo_short = m.profile_kernel("wo", grouped[0], reps=4) if grouped else None
     for p in poss:
         us = sorted(m.time_step(p, 9))
         attn_us = m.profile_kernel("attn", p, reps=4)
         wo_us = m.profile_kernel("wo", p, reps=4)
         # between position 256 and the GQA group path the split partials are merged by the wo kernel
         # (k_wo_comb): what that adds to wo is attention time and is charged to it here
-        merge_us = max(0.0, wo_us - wo_short)
+        merge_us = max(0.0, wo_us - wo_short) if grouped and p not in grouped else 0.0
         kv_bytes = 2.0 * (p + 1) * spec.kv_dim * 4
         out[str(p)] = {"step_us": round(us[len(us) // 2], 2), "attn_us_per_layer": round(attn_us + merge_us, 2),
                        "attn_kernel_us": round(attn_us, 2), "wo_us": round(wo_us, 2),
-                       "wo_us_plain_input": round(wo_short, 2),
+                       "wo_us_plain_input": round(wo_short, 2) if grouped else None,
                        "attn_kv_bytes_per_layer": kv_bytes,
                        "attn_kv_frac": kv_bytes / ((attn_us + merge_us) * 1e-6) / (HBM_PEAK_GBS * 1e9)}
     return out
@@ -595,12 +599,13 @@ def measure(spec, args, rank, world, local_rank, primary):
     ppos = min(args.steps - 1, 64)
     b2b = m.profile_kernels(ppos, reps=8)
     k_us = b2b["ffn13"]
-    kb = ffn13_bytes(spec)
+    parts = spec.n_kv_heads if "attn_wo" in b2b else 0  # attention and wo in one launch: the sums are this kernel's
+    kb = ffn13_bytes(spec, parts)
     achieved = kb / (k_us * 1e-6) / 1e9
-    tr, tr_src = load_traffic(f"{spec.name}:ffn13")
+    tr, tr_src = load_traffic(f"{spec.name}:{'ffn13_parts' if parts else 'ffn13'}")
     L = spec.n_layers
     out["roofline"] = {
-        "bound": "hbm", "kernel": "k_ffn13 (w1,w3 GEMV + SwiGLU)", "achieved": achieved,
+        "bound": "hbm", "kernel": f"{'k_ffn13_parts' if parts else 'k_ffn13'} (w1,w3 GEMV + SwiGLU)", "achieved": achieved,
         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
         "traffic": tr, "traffic_source": tr_src, "bytes_per_launch": kb, "avg_launch_us": k_us,
         "step": {"achieved": out["step_gbs"], "frac": out["step_gbs"] / HBM_PEAK_GBS,

@@ -429,7 +429,9 @@ int kh_model_time_prefill(kh_model* m, const int32_t* h_tokens, int32_t n, int32
  * launches; a graph because a 3-4 us kernel outruns eager host enqueues); consecutive
  * launches read different layers' weights, so nothing is served from cache.  This is the
  * number bench.py's roofline uses and the one rocprofv3's per-kernel average must agree with.
- * Destroys the activation state and KV row `pos` (a later generate/predict resets both). */
+ * Destroys the activation state and KV row `pos` (a later generate/predict resets both).
+ * KH_ERR_UNSUPPORTED: KH_K_WO at a position whose step has no such launch (KH_K_ATTN is attention and wo there,
+ * csrc/kh_attn_wo.h), and layer-list models. */
 int kh_model_profile_kernel(kh_model* m, int32_t kclass, int32_t pos, int32_t reps,
                             float* h_avg_us);
 
@@ -442,7 +444,8 @@ int kh_model_time_step(kh_model* m, int32_t pos, int32_t reps, float* h_us);
 /* Per-kernel-class timing of the fused step with HIP events (eager launches, one event
  * between every kernel).  n_steps decode steps starting at position start_pos (KV rows
  * below start_pos must already exist).  Writes avg microseconds per launch for each
- * class into h_avg_us[KH_NUM_KCLASS] and launches-per-step into h_count. */
+ * class into h_avg_us[KH_NUM_KCLASS] and launches-per-step into h_count (KH_K_WO: 0 of both where attention and wo
+ * are one launch, KH_K_ATTN). */
 enum {
   KH_K_QKV = 0, KH_K_ATTN = 1, KH_K_WO = 2, KH_K_FFN13 = 3, KH_K_W2 = 4, KH_K_CLS = 5,
   KH_K_SAMPLE = 6, KH_NUM_KCLASS = 7

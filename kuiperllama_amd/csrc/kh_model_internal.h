@@ -212,6 +212,7 @@ float* logits_pin(kh_model* m, size_t n);
 int ensure_seq_cap(kh_model* m, int n);
 void destroy_step_graphs(kh_model* m);
 // the captured graph of 1 (steps8 = false) or KH_GRAPH_STEPS decode steps in `variant`, captured on first use
+int step_launches(const kh_model* m, int variant);  // of one step of a .bin model
 int step_graph(kh_model* m, int n_forced, int variant, bool steps8, hipGraphExec_t* out);
 // the same for a graph of `nsteps` in {1, 2, 4, 8} steps (the tail of a run: 20 steps = 8 + 8 + 4)
 int step_graph_n(kh_model* m, int n_forced, int variant, int nsteps, hipGraphExec_t* out);

@@ -18,8 +18,10 @@ extern "C" int kh_model_profile_kernel(kh_model* m, int32_t kclass, int32_t pos,
     const int rc = kv_ensure(m, pos + 1);
     if (rc != KH_OK) return rc;
   }
+  const int variant = step_variant(m, pos, pos);  // the attention / wo pair a step at `pos` launches
+  if (kclass == KH_K_WO && variant == 3) return KH_ERR_UNSUPPORTED;  // no launch of its own: part of KH_K_ATTN's
   set_state(m, 1 % c.vocab_size, pos);
-  m->step_var = step_variant(m, pos, pos);  // the attention / wo pair a step at `pos` launches
+  m->step_var = variant;
   const bool per_layer = kclass < KH_K_CLS;
   const int n_inner = per_layer ? c.layer_num : 1;
   auto sweep = [&]() {
@@ -105,28 +107,31 @@ extern "C" int kh_model_profile_step(kh_model* m, int32_t start_pos, int32_t n_s
     if (rc != KH_OK) return rc;
   }
   const int L = c.layer_num;
-  const int nk = 5 * L + 2;
-  std::vector<hipEvent_t> ev((size_t)nk + 1);
+  std::vector<hipEvent_t> ev((size_t)5 * L + 3);
   for (auto& e : ev) KH_CHECK_HIP(hipEventCreate(&e));
   double acc[KH_NUM_KCLASS] = {0};
   int cnt[KH_NUM_KCLASS] = {0};
   set_state(m, 1 % c.vocab_size, start_pos);
   int rc = KH_OK;
   for (int s = 0; s < n_steps && rc == KH_OK; ++s) {
-    if ((rc = launch_step_fused(m, 1, 0, ev.data(), step_variant(m, start_pos + s, start_pos + s))) != KH_OK) break;
+    const int variant = step_variant(m, start_pos + s, start_pos + s);
+    if ((rc = launch_step_fused(m, 1, 0, ev.data(), variant)) != KH_OK) break;
     hipError_t e = hipStreamSynchronize(m->stream);
     if (e != hipSuccess) {
       rc = (int)e;
       break;
     }
+    static const int kOfLayer[5] = {KH_K_QKV, KH_K_ATTN, KH_K_WO, KH_K_FFN13, KH_K_W2};
+    static const int kOfLayerWo[4] = {KH_K_QKV, KH_K_ATTN, KH_K_FFN13, KH_K_W2};  // attention and wo are one launch
+    const int per = variant == 3 ? 4 : 5, nk = step_launches(m, variant);
     for (int k = 0; k < nk; ++k) {
       float ms = 0.f;
       (void)hipEventElapsedTime(&ms, ev[k], ev[k + 1]);
       int cls;
-      if (k < 5 * L)
-        cls = k % 5;  // qkv, attn, wo, ffn13, w2
+      if (k < per * L)
+        cls = (per == 4 ? kOfLayerWo : kOfLayer)[k % per];
       else
-        cls = k == 5 * L ? KH_K_CLS : KH_K_SAMPLE;
+        cls = k == per * L ? KH_K_CLS : KH_K_SAMPLE;
       acc[cls] += (double)ms * 1000.0;
       cnt[cls] += 1;
     }

@@ -1,4 +1,4 @@
-// kh_model_step.hip — the decode step of the model level: launch shapes, the fused (5L+2 launches)
+// kh_model_step.hip — the decode step of the model level: launch shapes, the fused (4L+2 or 5L+2 launches)
 // and unfused (the reference's own sequence) step, hipGraph capture, predict and the generate loop.
 // Replaces, for the decode path,
 //   LLama2Model::forward / predict                         kuiper/source/model/llama3.cpp:147-167, 642-650
@@ -428,13 +428,14 @@ static void launch_layer(kh_model* m, int l, F&& mark) {
   launch_attn(m, l);
   mark();
   launch_wo(m, l);
-  mark();
+  if (m->step_var != 3) mark();  // 3: part of the attention launch
   launch_ffn13(m, l);
   mark();
   launch_w2(m, l);
   mark();
 }
-// one fused decode step = 5L + 2 launches.  ev (optional) receives an event after each launch.
+int step_launches(const kh_model* m, int variant) { return (variant == 3 ? 4 : 5) * m->cfg.layer_num + 2; }
+// one fused decode step = step_launches().  ev (optional) receives an event ahead of the first and after each launch.
 int launch_step_fused(kh_model* m, int advance, int n_forced, hipEvent_t* ev, int variant) {
   m->step_var = variant;
   if (m->hy) return hy_launch_step(m, advance, n_forced);

@@ -301,12 +301,16 @@ class KuiperModel:
 
     def profile_kernels(self, pos: int, reps: int = 8):
         """Back-to-back average launch duration (us) of every kernel class at position `pos`
-        (kh_model_profile_kernel); clobbers activations and KV row `pos`."""
+        (kh_model_profile_kernel); clobbers activations and KV row `pos`.  Where attention and wo are one
+        launch it is "attn_wo", in the place of "attn" and "wo"."""
         out = {}
         for i in range(_ffi.KH_NUM_KCLASS):
             us = C.c_float(0.0)
-            _ffi.check(_ffi.lib().kh_model_profile_kernel(self._h, i, pos, reps, C.byref(us)),
-                       "kh_model_profile_kernel")
+            rc = _ffi.lib().kh_model_profile_kernel(self._h, i, pos, reps, C.byref(us))
+            if rc == _ffi.KH_ERR_UNSUPPORTED and "attn" in out:
+                out["attn_wo"] = out.pop("attn")
+                continue
+            _ffi.check(rc, "kh_model_profile_kernel")
             out[_ffi.lib().kh_kclass_name(i).decode()] = float(us.value)
         return out
 
@@ -319,14 +323,17 @@ class KuiperModel:
         return float(us.value)
 
     def profile_step(self, start_pos: int, n_steps: int):
-        """Per-kernel-class average launch duration (us) of the fused step, HIP events."""
+        """Per-kernel-class average launch duration (us) of the fused step, HIP events ("attn_wo" as in
+        profile_kernels)."""
         avg = (C.c_float * _ffi.KH_NUM_KCLASS)()
         cnt = (C.c_int32 * _ffi.KH_NUM_KCLASS)()
         _ffi.check(_ffi.lib().kh_model_profile_step(self._h, start_pos, n_steps, avg, cnt),
                    "kh_model_profile_step")
         names = [_ffi.lib().kh_kclass_name(i).decode() for i in range(_ffi.KH_NUM_KCLASS)]
+        if cnt[names.index("wo")] == 0:
+            names[names.index("attn")] = "attn_wo"
         return {n: {"avg_us": float(avg[i]), "launches_per_step": int(cnt[i])}
-                for i, n in enumerate(names)}
+                for i, n in enumerate(names) if n != "wo" or cnt[i]}
 
     @property
     def load_ms(self) -> float:

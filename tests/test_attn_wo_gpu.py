@@ -23,6 +23,31 @@ _SPECS = {s.name: s for s in (
     _spec(2048, 1408, 32, 8, "64x32-8"), _spec(2048, 1408, 32, 4, "64x32-4"))}
 
 
+def test_profiles_name_what_is_launched(gpu):
+    """Below position 256 attention and wo are one launch and are reported as one; behind it each has its own time."""
+    from kuiperllama_amd import _ffi
+    from kuiperllama_amd.model import KuiperModel
+    spec = _SPECS["64x8-4"]
+    m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=31, device=gpu), spec)
+    m.generate([1, 2], 300)
+    joint, apart = ["qkv", "attn_wo", "ffn13", "w2", "cls", "sample"], ["qkv", "attn", "wo", "ffn13", "w2", "cls", "sample"]
+    for pos, names in ((0, joint), (64, joint), (255, joint), (256, apart), (290, apart)):
+        us = m.profile_kernels(pos)
+        assert sorted(us) == sorted(names) and min(us.values()) > 0.5, (pos, us)
+        if names is joint:
+            with pytest.raises(_ffi.KhError) as e:
+                m.profile_kernel("wo", pos)
+            assert e.value.code == _ffi.KH_ERR_UNSUPPORTED
+            assert m.profile_kernel("attn", pos) > 0.5
+        else:
+            assert m.profile_kernel("wo", pos) > 0.5
+        step = m.profile_step(pos, 1)
+        assert sorted(step) == sorted(names)
+        for k, v in step.items():
+            assert v["launches_per_step"] == (1 if k in ("cls", "sample") else spec.n_layers) and v["avg_us"] > 0.5, (pos, k, v)
+    m.close()
+
+
 @pytest.mark.parametrize("name", sorted(_SPECS))
 def test_against_the_oracle_and_the_prompt_path(gpu, oracle, name):
     """Logits within the bound of fp32 decode steps (4e-5, as for the attention in launches of its own); the prompt path of

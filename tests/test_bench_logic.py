@@ -66,6 +66,42 @@ def test_algorithmic_bytes_match_survey_table():
         assert abs(per_tok / sp.algorithmic_bytes_per_token(0) - 1) < 0.005
 
 
+def test_long_context_charges_attention_with_the_merge_alone(monkeypatch):
+    """The part of the wo launch that merges time splits is attention's; wo's own time is not, wherever it is measured.  Below
+    position 256 wo may be no launch at all: no baseline comes from there."""
+    import dataclasses
+
+    import torch
+    from kuiperllama_amd import binfmt
+    bench = _bench()
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    spec = dataclasses.replace(binfmt.PRESETS["llama3.2-1b"], n_layers=1)
+
+    class Model:
+        class cfg:
+            cache_len = 8192
+
+        def write_kv_device(self, *a):
+            pass
+
+        def time_step(self, pos, reps):
+            return [900.0] * reps
+
+        def profile_kernel(self, name, pos, reps=8):
+            if name == "wo":
+                return 0.07 if pos < 256 else 7.9 if pos < 4095 else 4.6
+            return 20.0
+
+    out = bench.long_context(Model(), spec, torch.device("cpu"))
+    assert out["2047"]["attn_us_per_layer"] == 23.3 and out["2047"]["wo_us_plain_input"] == 4.6
+    for pos in ("4095", "4096"):  # the group path: nothing is merged in wo
+        assert out[pos]["attn_us_per_layer"] == out[pos]["attn_kernel_us"] == 20.0
+        kv = 2 * (int(pos) + 1) * spec.kv_dim * 4
+        assert abs(out[pos]["attn_kv_frac"] - kv / 20e-6 / 8e12) < 1e-9
+    # the sums that k_ffn13_parts adds: eight parts read, one vector written
+    assert bench.ffn13_bytes(spec, 8) == bench.ffn13_bytes(spec) + 9 * 2048 * 4
+
+
 def test_traffic_provenance_names_the_kernel_sources():
     """roofline.traffic is read from profiles/pmc_traffic.json (separate PMC passes).  The file carries the sha1 of
     the device-code headers it was collected on and bench.py compares it with the tree it runs from, so a kernel change

@@ -36,6 +36,8 @@ def run(tag, env):
     return row
 
 
+if any(arg.startswith("WO=") for arg in sys.argv[2:]):
+    os.environ["KH_ATTN_WO"] = "0"  # a launch of its own
 base = run("default", {})
 for arg in sys.argv[2:]:
     cls, cands = arg.split("=")

@@ -43,6 +43,8 @@ def run(tag, env):
 
 
 classes = sys.argv[2].split(",") if len(sys.argv) > 2 else ["W2", "WO", "QKV"]
+if {"WO", "ATTN"} & set(classes):
+    os.environ["KH_ATTN_WO"] = "0"  # launches of their own
 run("default", {})
 us = (2, 4) if spec.quant else (4, 8)
 for cls in classes:
