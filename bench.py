@@ -523,6 +523,7 @@ def measure(spec, args, rank, world, local_rank, primary):
         "replicas": replicas.spread(per),
     }
     cfg = getattr(m, "cfg", None)  # kh_config: what the self-checks of kh_model_create_* decided for this model
+    out["launches_per_token"] = getattr(cfg, "launches_per_token", None)
     out["selftests"] = {"ring": getattr(cfg, "ring_selftest", None), "attn_merge": getattr(cfg, "attn_merge_selftest", None),
                         "legend": "0 n/a, 1 passed, -1 failed: fallback in use, 2 (attn_merge) fenced form requested"}
     if hasattr(m, "kv_bytes"):
@@ -714,7 +715,7 @@ def assemble_line(spec, args, world, res, secondary, others, skipped, timing_bac
               "parallelism": f"replicas{world} (no shard, no data-path collective; one process "
                              f"per GPU, HIP_VISIBLE_DEVICES/LOCAL_RANK pinning)",
               "timing_backend": timing_backend,
-              "exec": "hipGraph replay, 5L+2 fused HIP kernels per token",
+              "exec": f"hipGraph replay, {res.get('launches_per_token')} fused HIP kernels per token at position 0",
               "kv_cache_rows": spec.seq_len,
               "tok_s_128_steps": summary["tok_s_128_steps"],
               "secondary_workload": summary["secondary_workload"],

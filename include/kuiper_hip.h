@@ -199,8 +199,9 @@ typedef struct kh_config {
   int32_t family, rope_mode, cache_len;
   float rope_theta, rms_eps;
   int64_t weight_bytes; /* bytes of the weight arena resident in HBM */
-  int32_t launches_per_token; /* .bin models: 5 per layer + classifier + sampler (4 per layer below
-                               * position 256 where attention and wo are one launch, csrc/kh_attn_wo.h) */
+  int32_t launches_per_token; /* of a step at the first positions.  .bin models: 5 per layer + classifier + sampler, or 4
+                               * per layer where attention and wo are one launch there (csrc/kh_attn_wo.h: below
+                               * position 256, and 5 behind it) */
   /* Self-checks run once at the end of kh_model_create_* (csrc/kh_model_selftest.hip), about a millisecond:
    *   ring_selftest        the int8 LDS-DMA ring kernels against the register-tile kernels of the same launches on
    *                        this model's own weights: 0 = no ring kernel planned (fp32, geometry, KH_RING=0) or skipped,

@@ -854,7 +854,7 @@ extern "C" int kh_model_create_from_file(const char* path, const kh_model_opts* 
 extern "C" int kh_model_get_config(const kh_model* m, kh_config* out) {
   if (!m || !out) return KH_ERR_INVALID_ARG;
   *out = m->cfg;
-  out->launches_per_token = m->hy ? hy_launches(m) : 5 * m->cfg.layer_num + 2;
+  out->launches_per_token = m->hy ? hy_launches(m) : step_launches(m, step_variant(m, 0, 0));
   return KH_OK;
 }
 extern "C" float kh_model_get_load_ms(const kh_model* m) { return m ? m->load_ms : -1.f; }

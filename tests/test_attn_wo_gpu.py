@@ -23,6 +23,19 @@ _SPECS = {s.name: s for s in (
     _spec(2048, 1408, 32, 8, "64x32-8"), _spec(2048, 1408, 32, 4, "64x32-4"))}
 
 
+@pytest.mark.parametrize("name,hook,per", [("48x6-6", None, 4), ("64x32-8", None, 4), ("64x17-1", None, 5), ("64x32-8", "0", 5)])
+def test_launches_per_token(gpu, name, hook, per, monkeypatch):
+    """The count that the configuration reports is that of the step at position 0."""
+    from kuiperllama_amd.model import KuiperModel
+    if hook:
+        monkeypatch.setenv("KH_ATTN_WO", hook)
+    spec = _SPECS[name]
+    m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=31, device=gpu), spec)
+    assert m.cfg.launches_per_token == per * spec.n_layers + 2
+    assert sum(v["launches_per_step"] for v in m.profile_step(0, 1).values()) == m.cfg.launches_per_token
+    m.close()
+
+
 def test_profiles_name_what_is_launched(gpu):
     """Below position 256 attention and wo are one launch and are reported as one; behind it each has its own time."""
     from kuiperllama_amd import _ffi
