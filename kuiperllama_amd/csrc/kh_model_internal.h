@@ -214,6 +214,7 @@ void destroy_step_graphs(kh_model* m);
 // the captured graph of 1 (steps8 = false) or KH_GRAPH_STEPS decode steps in `variant`, captured on first use
 int step_launches(const kh_model* m, int variant);  // of one step of a .bin model
 int step_graph(kh_model* m, int n_forced, int variant, bool steps8, hipGraphExec_t* out);
+int graph_run(const kh_model* m, int s, int left);  // steps of the next graph at position s, of at most `left`
 // the same for a graph of `nsteps` in {1, 2, 4, 8} steps (the tail of a run: 20 steps = 8 + 8 + 4)
 int step_graph_n(kh_model* m, int n_forced, int variant, int nsteps, hipGraphExec_t* out);
 // ---- kh_attn_wo.hip -------------------------------------------------------------------------

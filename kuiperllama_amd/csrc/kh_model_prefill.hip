@@ -709,17 +709,15 @@ extern "C" int kh_model_time_prefill(kh_model* m, const int32_t* h_tokens, int32
     // capture (first use) outside the timed region
     hipGraphExec_t ge = nullptr;
     for (int s = 0; s < n;) {
-      const bool n8 = n - s >= KH_GRAPH_STEPS;
-      const int k = n8 ? KH_GRAPH_STEPS : 1;
-      if ((rc = step_graph(m, n_forced, step_variant(m, pos0 + s, pos0 + s + k - 1), n8, &ge)) != KH_OK) return rc;
+      const int k = graph_run(m, pos0 + s, n - s);
+      if ((rc = step_graph_n(m, n_forced, step_variant(m, pos0 + s, pos0 + s + k - 1), k, &ge)) != KH_OK) return rc;
       s += k;
     }
     set_state(m, h_tokens[0], pos0);
     KH_CHECK_HIP(hipEventRecord(m->ev0, m->stream));
     for (int s = 0; s < n;) {
-      const bool n8 = n - s >= KH_GRAPH_STEPS;
-      const int k = n8 ? KH_GRAPH_STEPS : 1;
-      if ((rc = step_graph(m, n_forced, step_variant(m, pos0 + s, pos0 + s + k - 1), n8, &ge)) != KH_OK) return rc;
+      const int k = graph_run(m, pos0 + s, n - s);
+      if ((rc = step_graph_n(m, n_forced, step_variant(m, pos0 + s, pos0 + s + k - 1), k, &ge)) != KH_OK) return rc;
       KH_CHECK_HIP(hipGraphLaunch(ge, m->stream));
       s += k;
     }

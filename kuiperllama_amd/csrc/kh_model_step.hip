@@ -612,6 +612,16 @@ int step_graph_n(kh_model* m, int n_forced, int variant, int nsteps, hipGraphExe
   *out = sg.e;
   return KH_OK;
 }
+// the largest of 8 / 4 / 2 / 1 steps from position s on that still fits (a single-step launch costs ~15 us of graph-launch gap:
+// the 20-step form of the bench ran 8 + 8 + 1 + 1 + 1 + 1 and lost 0.3 % to it; now 8 + 8 + 4)
+int graph_run(const kh_model* m, int s, int left) {
+  int n = KH_GRAPH_STEPS;
+  while (n > left) n >>= 1;
+  // a position's bits follow from the position: no graph across the end of attention and wo in one launch
+  if (s < m->awo.end)
+    while (s + n > m->awo.end) n >>= 1;
+  return n;
+}
 int step_graph(kh_model* m, int n_forced, int variant, bool steps8, hipGraphExec_t* out) {
   return step_graph_n(m, n_forced, variant, steps8 ? KH_GRAPH_STEPS : 1, out);
 }
@@ -906,13 +916,7 @@ extern "C" int kh_model_generate_until(kh_model* m, const int32_t* h_prompt, int
       return done(keep_logits(), 1);
     }
     if (exec == KH_EXEC_GRAPH) {
-      // the largest of 8 / 4 / 2 / 1 steps that still fits (a single-step launch costs ~15 us of graph-launch gap:
-      // the 20-step form of the bench ran 8 + 8 + 1 + 1 + 1 + 1 and lost 0.3 % to it; now 8 + 8 + 4)
-      int n = KH_GRAPH_STEPS;
-      while (n > total_steps - s) n >>= 1;
-      // a position's bits follow from the position: no graph across the end of attention and wo in one launch
-      if (s < m->awo.end)
-        while (s + n > m->awo.end) n >>= 1;
+      int n = graph_run(m, s, total_steps - s);
       const bool keep = s == start && start > 0;  // first sampled step behind a prefill: alone, logits kept
       if (keep) n = 1;
       hipGraphExec_t ge = nullptr;

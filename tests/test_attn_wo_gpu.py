@@ -61,6 +61,27 @@ def test_profiles_name_what_is_launched(gpu):
     m.close()
 
 
+@pytest.mark.parametrize("pos0,n", [(4, 300), (251, 9), (0, 261)])
+def test_token_by_token_prompt_across_the_end(gpu, pos0, n):
+    """The prompt phase one token a step leaves the cache rows of predict() at every position, whatever its first one is: no graph
+    of several steps crosses position 256."""
+    from kuiperllama_amd.model import KuiperModel
+    spec = _SPECS["64x8-4"]
+    img = binfmt.synth_image(spec, seed=31, device=gpu, final_norm_std=1.0)
+    a, b = KuiperModel.from_device_image(img, spec), KuiperModel.from_device_image(img, spec)
+    toks = [int(t) for t in np.random.default_rng(4).integers(0, spec.vocab_size, pos0 + n)]
+    for pos, t in enumerate(toks):
+        a.predict(t, pos, exec="fused")
+        if pos < pos0:
+            b.predict(t, pos, exec="fused")
+    assert b.time_prefill(toks[pos0:], pos0, "token") > 0
+    for l in range(spec.n_layers):
+        for x, y in zip(a.read_kv(l, 0, pos0 + n), b.read_kv(l, 0, pos0 + n)):
+            np.testing.assert_array_equal(x, y)
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("name", sorted(_SPECS))
 def test_against_the_oracle_and_the_prompt_path(gpu, oracle, name):
     """Logits within the bound of fp32 decode steps (4e-5, as for the attention in launches of its own); the prompt path of
