@@ -5,17 +5,18 @@
 
 namespace khm {
 
-// Which models take it, and in what shape.  fp32 weights; at most eight key / value groups of at most 16 heads and 512 columns
-// (two float4 a lane), head sizes that the attention is instantiated for, vectors that two float4 a thread cover: every group is
+// Which models take it, and in what shape.  fp32 weights; at most eight key / value groups of at most 512 columns (two float4 a
+// lane, ten heads), head sizes that the attention is instantiated for, vectors that two float4 a thread cover: every group is
 // one vector more that k_ffn13_parts stages (eight of 2048 floats cost it 0.9 us), and its keys and values are read by every
-// slice.  us a launch at position 48, attention + wo -> one launch | ffn13: Llama-3.2-1B 3.4 + 4.5 -> 5.0 | 21.3 -> 22.2;
+// slice.  At most 2048 columns, whatever the threads of ffn13: k_pf_wo_parts keeps eight tokens' vectors in 64 KB.  us a launch at position 48, attention + wo -> one launch | ffn13: Llama-3.2-1B 3.4 + 4.5 -> 5.0 | 21.3 -> 22.2;
 // TinyLlama 3.3 + 4.5 -> 4.9 | 15.5 -> 15.9; Qwen2.5-0.5B 3.4 + 2.6 -> 4.2 | 6.95 -> 7.15; stories15M 3.6 + 2.3 -> 3.9 | 2.4 -> 2.75.
 // A token: -3.9 / -6.1 / -8.4 / -12 %; with 200 - 240 positions -1.5 / -3 / -2 / -4 %.  From KH_ATTN_MIN_TS on attention is split over time.
 kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long) {
   kh_model::AttnWoPlan p;
   const int hs = c.head_size, cols = c.kv_mul * hs, mv = kh_stage_maxv(c.dim, ffn_wg);
   if (c.is_quant || dbg_off("KH_ATTN_WO") || (hs != 48 && hs != 64)) return p;
-  if (c.kv_mul > 16 || c.kv_head_num > KH_AWO_PARTS_MAX || cols > 512 || c.dim != c.head_num * hs || mv < 1 || mv > 2) return p;
+  if (c.kv_head_num > KH_AWO_PARTS_MAX || cols > 512 || c.dim != c.head_num * hs || mv < 1 || mv > 2) return p;
+  if ((size_t)KH_PF_BMAX * c.dim * sizeof(float) > (64u << 10)) return p;
   p.parts = c.kv_head_num;
   p.cols4 = cols / 4;
   p.lpr = p.cols4 <= 16 ? 16 : (p.cols4 <= 32 ? 32 : 64);
@@ -95,7 +96,7 @@ void launch_pf_attn_parts(kh_model* m, int l, int nvalid, int pos0) {
 void launch_pf_wo_parts(kh_model* m, int l, int nvalid) {
   const kh_model::AttnWoPlan& p = m->awo;
   KhPfWoPartsArgs a{m->pf_att, (const float*)m->layers[l].wo.w, m->pf_x, m->cfg.dim, p.parts, p.cols4, nvalid};
-  const int rows = KH_AWO_WAVES * (64 / p.lpr), lds = nvalid * m->cfg.dim * 4;  // at most 8 * 2048 floats: 64 KB
+  const int rows = KH_AWO_WAVES * (64 / p.lpr), lds = nvalid * m->cfg.dim * 4;  // at most 64 KB: plan_attn_wo
   auto go = [&](auto k) {
     hipLaunchKernelGGL(k, dim3((m->cfg.dim + rows - 1) / rows), dim3(64 * KH_AWO_WAVES), lds, m->stream, a);
   };

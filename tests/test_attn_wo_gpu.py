@@ -36,6 +36,27 @@ def test_launches_per_token(gpu, name, hook, per, monkeypatch):
     m.close()
 
 
+@pytest.mark.parametrize("heads,kv,joint", [(32, 8, True), (35, 7, False), (36, 6, False), (40, 8, False)])
+def test_wide_models_with_wide_workgroups(gpu, heads, kv, joint, monkeypatch):
+    """With 512 threads in ffn13 two float4 a thread cover 4096 columns; eight prompt tokens of more than 2048 do not fit the LDS of
+    the joint form's prompt launch, so such models keep their launches apart."""
+    from kuiperllama_amd.model import KuiperModel
+    monkeypatch.setenv("KH_SHAPE_FFN", "1,8,256,512")
+    spec = _spec(64 * heads, 1408, heads, kv, "wide")
+    img = binfmt.synth_image(spec, seed=31, device=gpu)
+    a, b = KuiperModel.from_device_image(img, spec), KuiperModel.from_device_image(img, spec)
+    assert a.cfg.launches_per_token == (4 if joint else 5) * spec.n_layers + 2
+    toks = [int(t) for t in np.random.default_rng(4).integers(0, spec.vocab_size, 21)]
+    a.prefill(toks, 0)
+    for pos, t in enumerate(toks):
+        b.predict(t, pos, exec="fused")
+    for l in range(spec.n_layers):
+        for x, y in zip(a.read_kv(l, 0, len(toks)), b.read_kv(l, 0, len(toks))):
+            np.testing.assert_array_equal(x, y)
+    a.close()
+    b.close()
+
+
 def test_profiles_name_what_is_launched(gpu):
     """Below position 256 attention and wo are one launch and are reported as one; behind it each has its own time."""
     from kuiperllama_amd import _ffi
