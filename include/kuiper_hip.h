@@ -394,6 +394,9 @@ int kh_plan_attention(int32_t head_num, int32_t kv_mul, int32_t head_size, int32
  * four waves (1; prompts 2, one decoded token 4, both for key + value sizes of at most 256, else KH_ERR_UNSUPPORTED) and a
  * distance table of `table` bytes a group. */
 int kh_plan_heads_lds(int32_t key, int32_t value, int32_t sets, int32_t table, int32_t* bytes);
+/* kh_plan_expert_rows: rows of a tile of the experts' products in a prompt pass (32, 64, 128 or 192), for `choices` pairs of token and
+ * choice over `outputs` of the router; `columns` and `weight_bytes` are those of gate and up, the bytes of all experts together. */
+int kh_plan_expert_rows(int64_t choices, int32_t outputs, int32_t experts, int32_t columns, int64_t weight_bytes, int32_t* rows);
 /* kh_plan_matmul: {tiles of a row in flight, float4 staged per thread (0: in one phase), waves that share a row pair, threads,
  * workgroups} of kh_matmul_f32 / kh_matmul_q8 for K rows of M; KH_ERR_UNSUPPORTED for lengths of the scalar kernels. */
 int kh_plan_matmul(int32_t is_quant, int32_t M, int32_t K, int32_t* out5);

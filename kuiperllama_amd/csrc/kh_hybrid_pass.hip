@@ -696,3 +696,9 @@ int hy_unfused_step(kh_model* m) {
   return hy.f32 ? go(Runner<float>(m, p)) : go(Runner<bf16>(m, p));
 }
 }  // namespace khm
+
+extern "C" int kh_plan_expert_rows(int64_t choices, int32_t outputs, int32_t experts, int32_t columns, int64_t weight_bytes, int32_t* rows) {
+  if (!rows || choices < 0 || outputs <= 0 || experts <= 0 || columns <= 0 || weight_bytes < 0) return KH_ERR_INVALID_ARG;
+  *rows = khm::lg_group_bm((long)choices, outputs, experts, columns, (size_t)weight_bytes);
+  return KH_OK;
+}

@@ -298,16 +298,24 @@ __global__ __launch_bounds__(64 * WM * WN, BM == 192 ? 2 : 1) void k_lgemm(const
 // tiles are a third empty or wait for HBM.  Where 64 x 64 leaves half of the CUs idle, 32 x 64: what one CU pulls is the time (160
 // features of K 4096, 2048 / 732 tokens: 25.2 / 24.0 -> 18.6 / 17.1 us).  Grouped launches: BM = the row granule the tile list was built with (lg_group_bm).
 // (rows: token and choice pairs, over `groups` outputs; w_bytes: weights of all experts of the gate and up product, N columns)
-// 192 rows for 128 where an expert's share lies so close below 128 or 256 that some of them pass it, and all tiles are one round of two
-// workgroups per CU: a tile more for one expert in eight is a second round for 34 workgroups.  1100 tokens, 7 of 32 experts, 1024 x
-// 1024: 36.1 -> 30.6 and 26.4 -> 21.8 us (fp32: the prompt 2791 -> 2418).  Several rounds hide it (2048 tokens: 128.7 / 131.5), and more weights
-// wait for HBM longer than the two stages of them that 192 rows leave room for (740 tokens, 6 of 36, 2048 x 2048, 268 MB: the prompt 1299 / 1354).
+// 192 rows for 128 where an expert's share lies so close below 128 or 256 that some of them pass it, and what those bring is a second
+// round of workgroups (two fit a CU): more than 512 tiles of 128 rows are expected, the experts' rows spread as independent choices
+// would, and those of 192 are one round.  us a prompt with 128 / 192 rows, 32 experts of 1024 x 1024: Gusorax, 7 choices, 1036 / 1100 / 1165
+// tokens in fp32 2042 / 2110 / 2200 -> 1971 / 2000 / 2144, in bf16 700 / 707 / 733 -> 700 / 717 / 733; Gufanex, 6 choices, 1360 / 1450 / 1530
+// tokens in fp32 3395 / 3555 / 3685 -> 3364 / 3566 / 3761, in bf16 1268 / 1296 / 1292 -> 1219 / 1260 / 1325; 28 experts of 1152 x 640, fp32, 930 /
+// 960 / 1010 tokens 1369 / 1427 / 1457 -> 1340 / 1357 / 1390.  Where 128 rows are one round as well, 192 only make the longest workgroup longer and
+// the ring of weights shorter: experts of 512 x 512, 540 / 1700 tokens in fp32 894 / 1820 -> 988 / 1992, of 1024 x 1024, Gufanex, 700 tokens
+// 2911 -> 3167, 540 tokens in bf16 715 -> 748 (in fp32 the other way, 1858 -> 1780).  Several rounds hide the second (2048
+// tokens: 128.7 / 131.5), and more weights wait for HBM longer than two stages of them cover (740 tokens, 6 of 36, 2048 x 2048, 268
+// MB: the prompt 1299 / 1354).
 static inline int lg_group_bm(long rows, int groups, int experts, int N, size_t w_bytes) {
   const long per = rows / (groups > 0 ? groups : 1);
-  const double most = per + 2.0 * sqrt((double)per);  // of even choices: two deviations
-  const long n = (per + 127) / 128;
-  if (per > 64 && most > 128.0 * n && most <= 192.0 * n && experts * n * ((N + 127) / 128) <= 512 && w_bytes <= (128u << 20)) return 192;
-  return per > 64 ? 128 : (per > 24 ? 64 : 32);
+  if (per <= 64) return per > 24 ? 64 : 32;
+  const double sd = sqrt((double)per), most = per + 2.0 * sd;
+  const long n = (per + 127) / 128, tiles = experts * n * ((N + 127) / 128);
+  const double pass = 0.5 * erfc((128.0 * n + 0.5 - per) / (sd * sqrt(2.0)));  // share of the experts with a tile more
+  const bool second = most > 128.0 * n && tiles * (n + pass) > 512.0 * n;
+  return second && most <= 192.0 * n && tiles <= 512 && w_bytes <= (128u << 20) ? 192 : 128;
 }
 template <class T, int EPI>
 int lg_launch(hipStream_t s, const LgArgs& a, int zdim = 1, int group_bm = 0, int max_tiles = 0) {

@@ -35,6 +35,22 @@ def test_decode_plan_invariants(name):
         assert s["grid"] <= -(-max(pairs, 1) // pairs_per_wg) or s["grid"] % 256 == 0, (k, s)
 
 
+@pytest.mark.parametrize("arch,width,elem,tokens,rows", [
+    # a second round of 128-row tiles, one round of 192-row tiles
+    ("gusorax", 1024, 2, 1036, 192), ("gusorax", 1024, 2, 1100, 192), ("gusorax", 1024, 4, 1100, 192), ("gusorax", 1024, 2, 1165, 192),
+    ("gufanex", 1024, 2, 1360, 192), ("gufanex", 1024, 4, 1450, 192),
+    # one round of either
+    ("gusorax", 512, 2, 540, 128), ("gusorax", 512, 4, 1100, 128), ("gusorax", 512, 4, 1700, 128), ("gusorax", 1024, 4, 540, 128),
+    ("gufanex", 512, 2, 700, 128), ("gufanex", 512, 2, 1450, 128), ("gufanex", 1024, 4, 700, 128),
+    # shares far below the edge, more than one round of 192, more weights than two stages cover
+    ("gusorax", 1024, 2, 800, 128), ("gusorax", 1024, 2, 1000, 128), ("gusorax", 1024, 2, 1700, 128), ("gusorax", 2048, 2, 1100, 128),
+    ("gufanex", 2048, 2, 740, 128), ("gusorax", 1024, 2, 290, 64), ("gusorax", 1024, 2, 100, 32)])
+def test_expert_tiles_take_192_rows_for_a_second_round_alone(arch, width, elem, tokens, rows):
+    """32 experts of half a width, 7 of 32 outputs chosen (Gusorax) or 6 of 36 (Gufanex)."""
+    top, outputs = (7, 32) if arch == "gusorax" else (6, 36)
+    assert _ffi.plan_expert_rows(tokens * top, outputs, 32, width, 32 * width * width * elem) == rows
+
+
 def test_decode_plan_int8_wide_rows_keep_the_small_tile():
     """int8 rows that need more than four 16-byte loads per lane walk several tiles of TWO loads (qkv / wo / ffn13 /
     cls; w2 takes two tiles of three where that is exact) - never the fp32 rule's 4 or 8.  Geometries wider than any

@@ -3,6 +3,7 @@
 import pytest
 
 import layers_util as U
+from kuiperllama_amd import _ffi
 
 pytestmark = pytest.mark.gpu
 BOTH = pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
@@ -38,9 +39,19 @@ def test_rows_of_experts(gpu, dtype, top):
 
 @BOTH
 @pytest.mark.parametrize("experts,top,n", [(4, 2, 240), (3, 1, 345), (5, 1, 610), (2, 1, 490)])
-def test_expert_tiles_of_192_rows(gpu, dtype, experts, top, n):
-    """Shares just below 128 and 256 rows (csrc/kh_lgemm.h::lg_group_bm), spread by the choices: tiles of few and of many 16-row units."""
+def test_expert_shares_below_an_edge(gpu, dtype, experts, top, n):
+    """Shares just below 128 and 256 rows, spread by the choices: tiles of few and of many 16-row units."""
     _prompt(U.Model(U.config([U.with_ff(U.mamba(), experts=experts, top=top, ff=72)], width=136, vocab=60)), dtype, n, (), max_seq_len=640)
+
+
+@BOTH
+@pytest.mark.parametrize("ff,n", [(512, 1100), (512, 1036), (1024, 540)])
+def test_expert_tiles_of_192_rows_in_one_round(gpu, dtype, ff, n):
+    """Shares just below 256 and 128 rows whose tiles of 128 would be a second round of workgroups: the tiles that the rule of
+    csrc/kh_lgemm.h::lg_group_bm makes 192 rows long, of experts with two tiles and with one, below and beyond their share."""
+    width, size = 136, {"bfloat16": 2, "float32": 4}[dtype]
+    assert _ffi.plan_expert_rows(7 * n, 32, 32, 2 * ff, 32 * 2 * ff * width * size) == 192
+    _prompt(U.Model(U.config([U.with_ff(U.mamba(), experts=32, top=7, ff=ff)], width=width, vocab=60)), dtype, n, (), max_seq_len=1152)
 
 
 @pytest.mark.parametrize("dim,vdim,window,n,cuts", [(128, 128, 40, 65, ()), (128, 128, 600, 700, (63, 64, 400)), (100, 90, 200, 300, (129,)),
