@@ -397,6 +397,11 @@ int kh_plan_heads_lds(int32_t key, int32_t value, int32_t sets, int32_t table, i
 /* kh_plan_expert_rows: rows of a tile of the experts' products in a prompt pass (32, 64, 128 or 192), for `choices` pairs of token and
  * choice over `outputs` of the router; `columns` and `weight_bytes` are those of gate and up, the bytes of all experts together. */
 int kh_plan_expert_rows(int64_t choices, int32_t outputs, int32_t experts, int32_t columns, int64_t weight_bytes, int32_t* rows);
+/* kh_plan_mixer_beside: does a layer of a prompt pass of `tokens` run its mixer beside its feed-forward (1), on a second stream?
+ * mixer, dense, expert: elements of the matrices of the mixer, of the dense or shared feed-forward (0: none) and of one expert;
+ * experts, top, outputs: those of the router (top 0: none). */
+int kh_plan_mixer_beside(int64_t mixer, int64_t dense, int64_t expert, int32_t experts, int32_t top, int32_t outputs,
+                         int32_t tokens, int32_t is_f32, int32_t* beside);
 /* kh_plan_matmul: {tiles of a row in flight, float4 staged per thread (0: in one phase), waves that share a row pair, threads,
  * workgroups} of kh_matmul_f32 / kh_matmul_q8 for K rows of M; KH_ERR_UNSUPPORTED for lengths of the scalar kernels. */
 int kh_plan_matmul(int32_t is_quant, int32_t M, int32_t K, int32_t* out5);
@@ -410,7 +415,7 @@ int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32
  * KH_PAIR_ATTN (0 = attention of a prompt slice on the fp32 matrix cores; KH_PG_ATTN_QT selects it too),
  * KH_SHAPE_DEBUG, KH_HY_DECODE (0 = single-token batches of layer-list models run on the pass kernels), KH_HY_EXPAND (0 = latent
  * attention of prompts in its absorbed form), KH_HY_TMAX (tokens of one pass, 32 ... 2048), KH_HY_ROWS (16, 64 or 128: row tiles
- * of the attention kernels of a pass), KH_HY_TAIL (0 = the last layer of a pass for all its tokens), KH_HY_FORK (0 = a pass on one stream), KH_HY_STEP_FAIL (the step of
+ * of the attention kernels of a pass), KH_HY_TAIL (0 = the last layer of a pass for all its tokens), KH_HY_FORK (0 = a pass on one stream, 1 = every layer of several tokens on two), KH_HY_STEP_FAIL (the step of
  * their generate loop reports KH_ERR_INTERNAL before its first launch)) lives in ONE process-wide key -> value table, seeded once from the KH_* variables of
  * the environment when the library is first used and changed afterwards only through kh_debug_set
  * (value NULL = unset).  No launch path reads the environment.  Hooks that shape a model (KH_SHAPE_*,

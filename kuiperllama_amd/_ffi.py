@@ -27,7 +27,7 @@ EXPORTS = [
     "kh_bpe_create_from_file", "kh_bpe_create_from_memory", "kh_bpe_destroy", "kh_bpe_vocab_size",
     "kh_bpe_bos_id", "kh_bpe_eos_id", "kh_bpe_stop_id", "kh_bpe_encode", "kh_bpe_decode",
     "kh_model_generate", "kh_model_generate_until", "kh_model_first_sample", "kh_model_time_step", "kh_model_prefill", "kh_model_prefill_gemm", "kh_model_time_prefill", "kh_model_profile_kernel", "kh_model_profile_step", "kh_kclass_name",
-    "kh_plan_decode_shapes", "kh_plan_decode_ring", "kh_plan_pair_shapes", "kh_plan_prefill_shape", "kh_plan_attention", "kh_plan_heads_lds", "kh_plan_expert_rows", "kh_plan_matmul",
+    "kh_plan_decode_shapes", "kh_plan_decode_ring", "kh_plan_pair_shapes", "kh_plan_prefill_shape", "kh_plan_attention", "kh_plan_heads_lds", "kh_plan_expert_rows", "kh_plan_mixer_beside", "kh_plan_matmul",
     "kh_model_create_from_checkpoint", "kh_seq_open", "kh_seq_close", "kh_seq_length", "kh_model_forward",
     "kh_model_generate_batch", "kh_model_probe_residual",
     "kh_debug_set", "kh_debug_get", "kh_debug_list",
@@ -157,6 +157,7 @@ def lib() -> C.CDLL:
     L.kh_plan_pair_shapes.argtypes = [_i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_attention.argtypes = [_i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_heads_lds.argtypes = [_i32, _i32, _i32, _i32, C.POINTER(_i32)]
+    L.kh_plan_mixer_beside.argtypes = [C.c_int64, C.c_int64, C.c_int64, _i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_expert_rows.argtypes = [C.c_int64, _i32, _i32, _i32, C.c_int64, C.POINTER(_i32)]
     L.kh_plan_matmul.argtypes = [_i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_spm_create_from_file.argtypes = [C.c_char_p, C.POINTER(_vp)]
@@ -328,6 +329,15 @@ def plan_expert_rows(choices: int, outputs: int, experts: int, columns: int, wei
     if rc != 0:
         raise KhError(rc, "kh_plan_expert_rows")
     return out.value
+
+
+def plan_mixer_beside(mixer: int, dense: int, expert: int, experts: int, top: int, outputs: int, tokens: int, f32: bool) -> bool:
+    """Does a layer of a prompt pass run its mixer beside its feed-forward; host-only."""
+    out = _i32()
+    rc = lib().kh_plan_mixer_beside(mixer, dense, expert, experts, top, outputs, tokens, int(f32), C.byref(out))
+    if rc != 0:
+        raise KhError(rc, "kh_plan_mixer_beside")
+    return bool(out.value)
 
 
 def plan_matmul(quant: bool, M: int, K: int) -> dict:

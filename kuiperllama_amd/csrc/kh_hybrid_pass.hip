@@ -93,6 +93,21 @@ int row_tiles(const std::vector<int32_t>& seg_n, const RowKind& kind, std::vecto
 }
 
 // ---- the pass ----------------------------------------------------------------------------------------------------
+// Does a layer's mixer run beside its feed-forward, on the other stream?  Two pairs of event and wait cost the shorter branch some
+// 17 us and the host 20, so the layer has to be worth it: about 14 us of weights and products beside its launches, and a
+// feed-forward without experts - two launches of 4.5 us; four at least are a mixer, and so are experts - 8 us of its own.  us
+// a prompt in one stream / two: Gusorax 1024 x 8, 3 tokens 524 / 569, 8 568 / 567, 16 577 / 565, 150 677 / 621, 1100 1097 / 930, 512 x 8, 50
+// 445 / 524; Gufanex 2048 x 4, 20 tokens 733 / 650, 400 1136 / 964, 2048 2060 / 1889, 512 x 4, 17 338 / 349.  Mixers of one head of
+// 64, Gusorax 1024 x 8, 17 tokens 598 / 548, 1100 1192 / 1050.  Feed-forwards of 256 columns: Gusorax 1024 x 8, 1100 tokens 633 / 676, 2048 x
+// 4, 400 333 / 360, in fp32 17 429 / 439, 100 480 / 487, 400 767 / 754; of 4096, 17 tokens 285 / 285, 100 311 / 307, 400 463 / 440.
+// mix, dense, expert: elements of the mixer's matrices, of the shared or dense feed-forward's, of one expert's.
+bool mixer_beside(double mix, double dense, double expert, int experts, int top, int outputs, int T, bool f32) {
+  auto us = [&](double read, double used) { return read * (f32 ? 4 : 2) / 5e6 + 2.0 * T * used / (f32 ? 1e8 : 6e8); };
+  if (!top) return us(dense, dense) >= 8.0 && us(mix + dense, mix + dense) >= 14.0;
+  const double p = (double)top / outputs;  // of an expert to be a token's choice, routed evenly
+  const double met = experts * (1.0 - pow(1.0 - p, T));
+  return us(mix + dense + met * expert, mix + dense + experts * p * expert) >= 14.0;
+}
 template <class T>
 struct Runner {
   kh_model* m;
@@ -399,26 +414,18 @@ struct Runner {
     return KH_OK;
   }
 
-  // Does a layer's mixer run beside its feed-forward, on the other stream?  Two pairs of event and wait cost the shorter branch some
-  // 17 us and the host 20, so the layer has to be worth it: about 14 us of weights and products beside its launches.  us a
-  // prompt in one stream / two: Gusorax 1024 x 8, 3 tokens 524 / 569, 8 568 / 567, 16 577 / 565, 150 677 / 621, 1100 1097 / 930, 512 x 8, 50
-  // 445 / 524; Gufanex 2048 x 4, 20 tokens 733 / 650, 400 1136 / 964, 2048 2060 / 1889, 512 x 4, 17 338 / 349.
   bool beside(const HyLayer& l) const {
     const HyMoe& f = l.ff;
-    if (ps.T < 2 || !f.on || dbg_off("KH_HY_FORK")) return false;  // (one token: hy_unfused_step, which may be captured)
+    const char* hook = dbg("KH_HY_FORK");
+    if (ps.T < 2 || !f.on || (hook && hook[0] == '0')) return false;  // (one token: hy_unfused_step, which may be captured)
+    if (hook && hook[0] == '1') return true;
     auto size = [](const HyMat& w) { return (double)w.N * w.ld; };
-    double all = size(l.out_mat()) + size(f.sgu) + size(f.sdown), one = 0.0, met = 0.0, mine = 0.0;
-    if (l.mixer == HY_MAMBA1) all += size(l.mb.in) + size(l.mb.x) + size(l.mb.dt);
-    else if (l.mixer == HY_LATENT) all += size(l.la.dqkv) + size(l.la.uq) + size(l.la.uk) + size(l.la.uv);
-    else all += size(l.ha.qkvg);
-    if (f.top) {
-      const double p = (double)f.top / f.n_out();  // of an expert to be a token's choice, routed evenly
-      one = 2.0 * f.ffp * f.gu.ld + (double)hy.c.width * f.down.ld;
-      met = f.E * (1.0 - pow(1.0 - p, ps.T));
-      mine = f.E * p;
-    }
-    const double us = (all + met * one) * sizeof(T) / 5e6 + 2.0 * ps.T * (all + mine * one) / (sizeof(T) == 2 ? 6e8 : 1e8);
-    return us >= 14.0;
+    double mix = size(l.out_mat());
+    if (l.mixer == HY_MAMBA1) mix += size(l.mb.in) + size(l.mb.x) + size(l.mb.dt);
+    else if (l.mixer == HY_LATENT) mix += size(l.la.dqkv) + size(l.la.uq) + size(l.la.uk) + size(l.la.uv);
+    else mix += size(l.ha.qkvg);
+    const double expert = f.top ? 2.0 * f.ffp * f.gu.ld + (double)hy.c.width * f.down.ld : 0.0;
+    return mixer_beside(mix, size(f.sgu) + size(f.sdown), expert, f.E, f.top, f.n_out(), ps.T, sizeof(T) == 4);
   }
   bool forked = false;
   // A layer's mixer and its feed-forward read the same norms and write nothing in common: in a parallel block neither needs the other.
@@ -700,5 +707,13 @@ int hy_unfused_step(kh_model* m) {
 extern "C" int kh_plan_expert_rows(int64_t choices, int32_t outputs, int32_t experts, int32_t columns, int64_t weight_bytes, int32_t* rows) {
   if (!rows || choices < 0 || outputs <= 0 || experts <= 0 || columns <= 0 || weight_bytes < 0) return KH_ERR_INVALID_ARG;
   *rows = khm::lg_group_bm((long)choices, outputs, experts, columns, (size_t)weight_bytes);
+  return KH_OK;
+}
+
+extern "C" int kh_plan_mixer_beside(int64_t mixer, int64_t dense, int64_t expert, int32_t experts, int32_t top, int32_t outputs,
+                                    int32_t tokens, int32_t is_f32, int32_t* beside) {
+  if (!beside || mixer < 0 || dense < 0 || expert < 0 || experts < 0 || top < 0 || tokens < 1 || (top && (outputs < top || !experts)))
+    return KH_ERR_INVALID_ARG;
+  *beside = tokens > 1 && mixer_beside((double)mixer, (double)dense, (double)expert, experts, top, outputs, tokens, is_f32 != 0);
   return KH_OK;
 }

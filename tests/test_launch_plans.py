@@ -51,6 +51,27 @@ def test_expert_tiles_take_192_rows_for_a_second_round_alone(arch, width, elem, 
     assert _ffi.plan_expert_rows(tokens * top, outputs, 32, width, 32 * width * width * elem) == rows
 
 
+@pytest.mark.parametrize("width,ff,f32,tokens,beside", [
+    (1024, 256, False, 1100, False), (2048, 256, False, 400, False), (2048, 256, True, 17, False), (2048, 256, True, 100, False),
+    (2048, 256, True, 400, True), (2048, 4096, False, 17, True), (2048, 4096, False, 400, True), (1024, 3584, False, 17, False),
+    (1024, 3584, False, 1100, True)])
+def test_mixers_run_beside_a_dense_feed_forward_of_some_size(width, ff, f32, tokens, beside):
+    """Heads of 128, a quarter of them with keys and values.  The shorter branch pays for the events: a short feed-forward gains
+    nothing beside a mixer however long that is."""
+    mixer = width * (2 * width + 2 * width // 4 + width)
+    assert _ffi.plan_mixer_beside(mixer, 3 * width * ff, 0, 0, 0, 0, tokens, f32) is beside
+    assert not _ffi.plan_mixer_beside(100 * mixer, 3 * 64 * 256, 0, 0, 0, 0, tokens, f32)
+
+
+def test_mixers_run_beside_experts():
+    """Experts are launches enough for a mixer of any size: what counts is the layer's work in all."""
+    gusorax = lambda width, tokens, mixer=None: _ffi.plan_mixer_beside(  # noqa: E731
+        3 * width * width if mixer is None else mixer, 0, 3 * width * width // 2, 32, 7, 32, tokens, False)
+    assert [gusorax(1024, t) for t in (1, 3, 17, 150, 1100)] == [False, False, True, True, True]
+    assert [gusorax(1024, t, 4 * 64 * 1024) for t in (17, 1100)] == [True, True]
+    assert not gusorax(512, 50) and gusorax(512, 1100)
+
+
 def test_decode_plan_int8_wide_rows_keep_the_small_tile():
     """int8 rows that need more than four 16-byte loads per lane walk several tiles of TWO loads (qkv / wo / ffn13 /
     cls; w2 takes two tiles of three where that is exact) - never the fp32 rule's 4 or 8.  Geometries wider than any
