@@ -634,14 +634,16 @@ void plan_decode_shapes(bool quant, int dim, int hidden_dim, int kv_dim, int voc
   // w2 re-stages the hidden-sized input in every workgroup: 512-thread workgroups halve that
   // L2 -> LDS traffic for the same number of waves (measured 14.1 -> 11.8 us on Llama-3.2-1B)
   out[3] = pick_shape(quant, dim / 2, hidden_dim, 4, "KH_SHAPE_W2", KH_WG_MAX, KH_WG_MAX, true, /*u3=*/true);
-  // ... but not where it leaves three quarters of the CUs without one (stories15M, 288 rows of 768: 18 workgroups 2.55 us, 36
-  // of 256 threads 2.16)
+  // ... but not where it leaves three quarters of the CUs without one (rows of the model x hidden, as workgroups of 512 / 256
+  // threads, us: 288 x 768 2.60 / 2.14, 384 x 1024 2.87 / 2.39, 448 x 1216 3.5 / 2.84, 512 x 1376 3.66 / 3.12)
   if (out[3].grid < 64) out[3] = pick_shape(quant, dim / 2, hidden_dim, 4, "KH_SHAPE_W2", KH_WG, KH_WG_MAX, true, /*u3=*/true);
-  // rows of less than 2 KB keep less in flight per wave than a trip to memory hides: 16 waves per CU instead of 8 (32000 rows of
-  // 288 floats: 9.8 -> 7.8 us; 151936 rows of 896, 3.5 KB, lose 3 %)
-  const bool short_rows = !quant && dim < 512;
-  out[4] = pick_shape(quant, (vocab_size + 1) / 2, dim, 1, "KH_SHAPE_CLS", quant || short_rows ? KH_WG : KH_WG_MAX, KH_WG_MAX,
-                      short_rows);
+  // rows of less than 1.5 KB keep less in flight per wave than a trip to memory hides: 16 waves per CU instead of 8, in workgroups
+  // of 512 threads (of 256 they leave the sampler twice as many partial maxima).  64 steps of 8 layers, us, 8 waves / 16 / 16 in
+  // workgroups of 256, 32000 and 151936 rows: 192 floats 6521 / 6450 / 6469 and 8043 / 7423 / 7734, 288 6901 / 6813 / 6841 and 8598 /
+  // 8212 / 8316, 336 7051 / 7008 / 7074 and 8876 / 8683 / 8781; not 384, 6986 / 6977 / 7030 and 8780 / 8866 / 8981, nor 448, 7875 / - / 7985
+  // and 10017 / - / 10155
+  const bool short_rows = !quant && dim < 384;
+  out[4] = pick_shape(quant, (vocab_size + 1) / 2, dim, 1, "KH_SHAPE_CLS", quant ? KH_WG : KH_WG_MAX, KH_WG_MAX, short_rows);
 }
 
 // The int8 ffn13 and classifier launches run on the LDS-DMA ring kernels (kh_fused_ring.h) when the geometry fits

@@ -72,6 +72,14 @@ def test_mixers_run_beside_experts():
     assert not gusorax(512, 50) and gusorax(512, 1100)
 
 
+@pytest.mark.parametrize("vocab", [32000, 151936])
+@pytest.mark.parametrize("dim,grid", [(192, 512), (288, 512), (336, 512), (384, 256), (448, 256), (512, 256), (896, 256)])
+def test_classifiers_of_short_rows(dim, grid, vocab):
+    """fp32 rows of less than 1.5 KB: 16 waves a CU, in workgroups of 512 threads like the longer ones."""
+    cls = _ffi.plan_decode_shapes(dim, 3 * dim, dim, vocab, False)["cls"]
+    assert (cls["grid"], cls["wg"], cls["split"]) == (grid, 512, 1)
+
+
 def test_decode_plan_int8_wide_rows_keep_the_small_tile():
     """int8 rows that need more than four 16-byte loads per lane walk several tiles of TWO loads (qkv / wo / ffn13 /
     cls; w2 takes two tiles of three where that is exact) - never the fp32 rule's 4 or 8.  Geometries wider than any
