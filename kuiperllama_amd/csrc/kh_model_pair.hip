@@ -44,7 +44,9 @@ const struct {
 } kPairCost[2] = {{1.833, 0.650, 0.444}, {2.167, 0.929, 1.0}};
 
 // resid: a product that is added to the residual (wo, w2).  gated: w1 + w3, whose scales the product behind it has to fold in twice
-// as often where a tile leaves them per 32 columns (Qwen2.5-0.5B, 41 tokens, 32 x 64 instead of 32 x 128 there: w2 24 -> 25 us).
+// as often where a tile leaves them per 32 columns.  With and without 1.15 for it: passes of 33 to 64 tokens take 32 x 128 instead of 32
+// x 64, us, TinyLlama 33 2172 / 2158, 50 2229 / 2184, 64 2279 / 2208, Qwen2.5-0.5B 41 1597 / 1580, 64 1651 / 1612; elsewhere the choice
+// is the same (Llama-3.2-1B and the shortest passes of all three, where 32 x 64 are more workgroups on idle CUs).
 PairShape pair_shape(bool q, int T, int N, int K, bool resid, bool gated, double* time_us = nullptr) {
   PairShape best{0, 1};
   double best_us = -1.0;
@@ -59,7 +61,7 @@ PairShape pair_shape(bool q, int T, int N, int K, bool resid, bool gated, double
       double us = rounds * std::max(t.lat, t.occ * t.sat) + std::max(t.lat, last * t.sat);
       us = us * stages / kz + kPairCost[q].ends * most;
       if (kz > 1) us += kPairCost[q].part * kz * T * N * 8 / 4.0e6;
-      if (gated && t.bn < 128) us *= 1.06;
+      if (gated && t.bn < 128) us *= 1.15;
       if (best_us < 0 || us < best_us) {
         best_us = us;
         best = PairShape{i, kz};

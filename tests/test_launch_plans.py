@@ -80,6 +80,14 @@ def test_classifiers_of_short_rows(dim, grid, vocab):
     assert (cls["grid"], cls["wg"], cls["split"]) == (grid, 512, 1)
 
 
+@pytest.mark.parametrize("name,narrow,wide", [("tinyllama-1.1b", (17, 32), (33, 50, 64)), ("qwen2.5-0.5b", (17, 32), (33, 41, 64))])
+def test_gated_tiles_of_short_prompts(name, narrow, wide):
+    """w1 + w3: tiles of 64 rows only where they win by more than their finer scales cost the product behind them."""
+    sp = binfmt.PRESETS[name]
+    bn = lambda n: _ffi.plan_pair_shapes(sp.dim, sp.hidden_dim, sp.kv_dim, False, n)["w13"]["bn"]  # noqa: E731
+    assert [bn(n) for n in narrow] == [64] * len(narrow) and [bn(n) for n in wide] == [128] * len(wide)
+
+
 def test_decode_plan_int8_wide_rows_keep_the_small_tile():
     """int8 rows that need more than four 16-byte loads per lane walk several tiles of TWO loads (qkv / wo / ffn13 /
     cls; w2 takes two tiles of three where that is exact) - never the fp32 rule's 4 or 8.  Geometries wider than any
