@@ -796,6 +796,7 @@ int finish(kh_model* m, Plan& pl) {
     if ((rc = hy_launch_step(m, 0, 0)) != KH_OK) return rc;
   m->step_var = 0;
   if ((rc = kh_launch_status()) != KH_OK) return rc;
+  (void)logits_pin(m, std::min<size_t>((size_t)hy.slots * hy.c.vocab, 1u << 20));  // a row a sequence: no prompt's first call pays for it
   KH_CHECK_HIP(hipStreamSynchronize(m->stream));
   return hy_selftest(m);
 }
