@@ -1,7 +1,7 @@
-// kh_fused.h — the fused decode-step kernels (5 per layer + classifier + sampler).
+// kh_fused.h — the fused decode-step kernels (5 per layer, or 4, + classifier + sampler).
 //
 // The reference issues 14 launches per layer (17 for Qwen2) from host code that also reads
-// `pos` on the CPU.  Here one token = 5L+2 launches whose every
+// `pos` on the CPU.  Here one token = 5L+2 launches (4L+2 where kh_attn_wo.h joins k_attn and k_wo) whose every
 // offset derives from the DEVICE scalar *d_pos, so the whole step is a replayable hipGraph:
 //
 //   k_qkv    rmsnorm(x) -> LDS ; [wq|wk|wv] row pairs ; +bias ; RoPE ; q -> q_buf,

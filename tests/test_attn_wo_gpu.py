@@ -82,6 +82,30 @@ def test_profiles_name_what_is_launched(gpu):
     m.close()
 
 
+@pytest.mark.parametrize("name", ["48x6-6", "64x8-4", "64x32-8"])
+def test_launches_of_their_own(gpu, oracle, name, monkeypatch):
+    """The same models with attention and wo apart at every position: the oracle's logits, and the prompt path's bits."""
+    from kuiperllama_amd.model import KuiperModel
+    monkeypatch.setenv("KH_ATTN_WO", "0")
+    spec = _SPECS[name]
+    img_d = binfmt.synth_image(spec, seed=31, device=gpu, final_norm_std=1.0)
+    torch.cuda.synchronize()
+    a, b = KuiperModel.from_device_image(img_d, spec), KuiperModel.from_device_image(img_d, spec)
+    om = oracle.OracleModel.from_spec(img_d.cpu().numpy(), spec)
+    toks = [int(t) for t in np.random.default_rng(5).integers(0, spec.vocab_size, 140)]
+    for pos, t in enumerate(toks):
+        a.predict(t, pos, exec="fused")
+        want = om.forward(t, pos)
+        if pos in (0, 1, 15, 16, 63, 127, 128, 139):
+            err = np.abs(a.logits() - want).max()
+            assert err <= 4e-5, f"position {pos}: {err:.3e}"
+    b.prefill(toks[:-1], 0)
+    b.predict(toks[-1], 139, exec="fused")
+    assert np.array_equal(a.logits(), b.logits())
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("pos0,n", [(4, 300), (251, 9), (0, 261)])
 def test_token_by_token_prompt_across_the_end(gpu, pos0, n):
     """The prompt phase one token a step leaves the cache rows of predict() at every position, whatever its first one is: no graph
