@@ -390,6 +390,10 @@ int kh_plan_decode_ring(int32_t dim, int32_t hidden_dim, int32_t vocab_size, int
  * workgroups that own timesteps at `pos`} (KH_ATTN_TLONG honoured). */
 int kh_plan_attention(int32_t head_num, int32_t kv_mul, int32_t head_size, int32_t seq_len, int32_t pos,
                       int32_t* out8);
+/* kh_plan_attn_wo: attention and wo of a decoded token in one launch (csrc/kh_attn_wo.h) for a .bin model of these sizes: out4 =
+ * {positions below it take it (0: none do), parts of wo, rows of a part a workgroup, workgroups}. */
+int kh_plan_attn_wo(int32_t dim, int32_t hidden_dim, int32_t head_num, int32_t kv_head_num, int32_t seq_len, int32_t is_quant,
+                    int32_t* out4);
 /* kh_plan_heads_lds: LDS bytes of a workgroup of the layer-list models' attention over grouped heads with `sets` sets of
  * four waves (1; prompts 2, one decoded token 4, both for key + value sizes of at most 256, else KH_ERR_UNSUPPORTED) and a
  * distance table of `table` bytes a group. */

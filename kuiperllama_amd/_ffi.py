@@ -27,7 +27,7 @@ EXPORTS = [
     "kh_bpe_create_from_file", "kh_bpe_create_from_memory", "kh_bpe_destroy", "kh_bpe_vocab_size",
     "kh_bpe_bos_id", "kh_bpe_eos_id", "kh_bpe_stop_id", "kh_bpe_encode", "kh_bpe_decode",
     "kh_model_generate", "kh_model_generate_until", "kh_model_first_sample", "kh_model_time_step", "kh_model_prefill", "kh_model_prefill_gemm", "kh_model_time_prefill", "kh_model_profile_kernel", "kh_model_profile_step", "kh_kclass_name",
-    "kh_plan_decode_shapes", "kh_plan_decode_ring", "kh_plan_pair_shapes", "kh_plan_prefill_shape", "kh_plan_attention", "kh_plan_heads_lds", "kh_plan_expert_rows", "kh_plan_mixer_beside", "kh_plan_matmul",
+    "kh_plan_decode_shapes", "kh_plan_decode_ring", "kh_plan_pair_shapes", "kh_plan_prefill_shape", "kh_plan_attention", "kh_plan_attn_wo", "kh_plan_heads_lds", "kh_plan_expert_rows", "kh_plan_mixer_beside", "kh_plan_matmul",
     "kh_model_create_from_checkpoint", "kh_seq_open", "kh_seq_close", "kh_seq_length", "kh_model_forward",
     "kh_model_generate_batch", "kh_model_probe_residual",
     "kh_debug_set", "kh_debug_get", "kh_debug_list",
@@ -156,6 +156,7 @@ def lib() -> C.CDLL:
     L.kh_plan_prefill_shape.argtypes = [_i32, _i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_pair_shapes.argtypes = [_i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_attention.argtypes = [_i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
+    L.kh_plan_attn_wo.argtypes = [_i32, _i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_heads_lds.argtypes = [_i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_mixer_beside.argtypes = [C.c_int64, C.c_int64, C.c_int64, _i32, _i32, _i32, _i32, _i32, C.POINTER(_i32)]
     L.kh_plan_expert_rows.argtypes = [C.c_int64, _i32, _i32, _i32, C.c_int64, C.POINTER(_i32)]
@@ -311,6 +312,16 @@ def plan_pair_shapes(dim: int, hidden_dim: int, kv_dim: int, quant: bool, T: int
     if rc != 0:
         raise KhError(rc, "kh_plan_pair_shapes")
     return {k: dict(zip(("bm", "bn", "kz", "workgroups"), out[4 * i: 4 * i + 4])) for i, k in enumerate(("qkv", "wo", "w13", "w2"))}
+
+
+def plan_attn_wo(dim: int, hidden_dim: int, head_num: int, kv_head_num: int, seq_len: int, quant: bool = False) -> dict:
+    """Attention and wo of a decoded token in one launch: the positions that take it (below `end`) and its shape; host-only."""
+    sync_env()
+    out = (_i32 * 4)()
+    rc = lib().kh_plan_attn_wo(dim, hidden_dim, head_num, kv_head_num, seq_len, int(quant), out)
+    if rc != 0:
+        raise KhError(rc, "kh_plan_attn_wo")
+    return dict(zip(("end", "parts", "rows", "workgroups"), list(out)))
 
 
 def plan_heads_lds(key: int, value: int, sets: int, table: int) -> int:

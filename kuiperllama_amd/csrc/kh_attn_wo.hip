@@ -23,10 +23,13 @@ kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long) {
   p.nu = (p.cols4 + p.lpr - 1) / p.lpr;
   const int rows = KH_AWO_WAVES * (64 / p.lpr);
   auto slices = [&](int rw) { return (c.dim + rows * rw - 1) / (rows * rw); };
-  // the most rows a workgroup (its attention is the same for few) that leave three quarters of the CUs with one: two rounds of
-  // half as many took 7.8 instead of 5.6 us (Llama-3.2-1B)
-  for (p.rw = p.lpr == 64 ? 8 / p.nu : 2; p.rw > 1 && p.parts * slices(p.rw) < 192;) p.rw /= 2;
+  // the most rows a workgroup (its attention is the same for few) that leave three quarters of the CUs with one, or fewer CUs
+  // where half as many rows would be more than one workgroup a CU: sixteen waves of up to 115 registers are alone there, and two
+  // rounds take 7.8 instead of 5.6 us (Llama-3.2-1B).  256 steps of 8 layers, 288 / 144 workgroups: 768 columns, 12-6 heads 45.8 / 39.8
+  // ms, 1536, 24-3 heads 72.4 / 65.0; apart 40.6 and 67.0
+  for (p.rw = p.lpr == 64 ? 8 / p.nu : 2; p.rw > 1 && p.parts * slices(p.rw) < 192 && p.parts * slices(p.rw / 2) <= 256;) p.rw /= 2;
   p.slices = slices(p.rw);
+  if (p.parts * p.slices > 256) return kh_model::AttnWoPlan{};
   p.lds = attn_wo_lds_bytes(hs, c.kv_mul);
   p.end = t_long - 1 < KH_ATTN_MIN_TS ? t_long - 1 : KH_ATTN_MIN_TS;  // one split, and no group path
   return p;
@@ -106,3 +109,29 @@ void launch_pf_wo_parts(kh_model* m, int l, int nvalid) {
   else go(k_pf_wo_parts<64, 2>);
 }
 }  // namespace khm
+
+extern "C" int kh_plan_attn_wo(int32_t dim, int32_t hidden_dim, int32_t head_num, int32_t kv_head_num, int32_t seq_len, int32_t is_quant,
+                               int32_t* out4) {
+  if (!out4 || dim <= 0 || hidden_dim <= 0 || head_num <= 0 || kv_head_num <= 0 || head_num % kv_head_num || dim % head_num || seq_len <= 0)
+    return KH_ERR_INVALID_ARG;
+  kh_config c{};
+  c.dim = dim;
+  c.hidden_dim = hidden_dim;
+  c.head_num = head_num;
+  c.kv_head_num = kv_head_num;
+  c.kv_mul = head_num / kv_head_num;
+  c.head_size = dim / head_num;
+  c.kv_dim = c.head_size * kv_head_num;
+  c.is_quant = is_quant;
+  kh_model::Shape sh[5];
+  khm::plan_decode_shapes(is_quant != 0, dim, hidden_dim, c.kv_dim, dim, sh);
+  int32_t at[8];
+  const int rc = kh_plan_attention(head_num, c.kv_mul, c.head_size, seq_len, 0, at);
+  if (rc != KH_OK) return rc;
+  const kh_model::AttnWoPlan p = khm::plan_attn_wo(c, sh[2].wg, at[3]);
+  out4[0] = p.end > 0 ? p.end : 0;
+  out4[1] = p.end > 0 ? p.parts : 0;
+  out4[2] = p.end > 0 ? KH_AWO_WAVES * (64 / p.lpr) * p.rw : 0;
+  out4[3] = p.end > 0 ? p.parts * p.slices : 0;
+  return KH_OK;
+}

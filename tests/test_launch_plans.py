@@ -88,6 +88,27 @@ def test_gated_tiles_of_short_prompts(name, narrow, wide):
     assert [bn(n) for n in narrow] == [64] * len(narrow) and [bn(n) for n in wide] == [128] * len(wide)
 
 
+@pytest.mark.parametrize("head_size", [48, 64])
+def test_attention_and_wo_in_one_round_of_workgroups(head_size, monkeypatch):
+    """A CU holds one of its workgroups: never more than 256, every row somebody's; and what does not take the joint launch."""
+    monkeypatch.delenv("KH_ATTN_WO", raising=False)
+    taken = 0
+    for heads in range(1, 45):
+        for kv in range(1, heads + 1):
+            if heads % kv:
+                continue
+            dim = heads * head_size
+            p = _ffi.plan_attn_wo(dim, 11 * dim // 4 // 16 * 16 + 16, heads, kv, 512)
+            if kv > 8 or heads // kv * head_size > 512 or dim > 2048:
+                assert p == dict(end=0, parts=0, rows=0, workgroups=0), (heads, kv, p)
+            elif p["end"]:
+                taken += 1
+                assert p["parts"] == kv and p["end"] <= 256
+                assert p["workgroups"] == kv * -(-dim // p["rows"]) <= 256, (heads, kv, p)
+    assert taken > 40
+    assert not _ffi.plan_attn_wo(2048, 8192, 32, 8, 512, True)["end"] and not _ffi.plan_attn_wo(2048, 8192, 16, 8, 512)["end"]
+
+
 def test_decode_plan_int8_wide_rows_keep_the_small_tile():
     """int8 rows that need more than four 16-byte loads per lane walk several tiles of TWO loads (qkv / wo / ffn13 /
     cls; w2 takes two tiles of three where that is exact) - never the fp32 rule's 4 or 8.  Geometries wider than any
