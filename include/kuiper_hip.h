@@ -200,8 +200,8 @@ typedef struct kh_config {
   float rope_theta, rms_eps;
   int64_t weight_bytes; /* bytes of the weight arena resident in HBM */
   int32_t launches_per_token; /* of a step at the first positions.  .bin models: 5 per layer + classifier + sampler, or 4
-                               * per layer where attention and wo are one launch there (csrc/kh_attn_wo.h: below
-                               * position 256, and 5 behind it) */
+                               * per layer where attention and wo are one launch there (kh_plan_attn_wo: below
+                               * position 256 at most, and 5 behind it) */
   /* Self-checks run once at the end of kh_model_create_* (csrc/kh_model_selftest.hip), about a millisecond:
    *   ring_selftest        the int8 LDS-DMA ring kernels against the register-tile kernels of the same launches on
    *                        this model's own weights: 0 = no ring kernel planned (fp32, geometry, KH_RING=0) or skipped,
@@ -414,7 +414,7 @@ int kh_plan_prefill_shape(int32_t epi, int32_t T, int32_t rows, int32_t K, int32
 
 /* Tuning / test hooks.  Every hook the library honours (KH_SHAPE_<QKV|WO|FFN|W2|CLS>, KH_RING, KH_ATTN_WG, KH_ATTN_FENCED,
  * KH_ATTN_TLONG, KH_ATTN_DEFER (0 = never merge time splits in the wo kernel), KH_ATTN_DEFER_MAX (active splits up to
- * which it does), KH_ATTN_WO (0 = attention and wo in launches of their own), KH_PREFILL, KH_PG_<CHUNK|ROWS (the most slab rows that memory is given for)|PAIR|SHAPE_*|SOLO|KZ|ATTN|ATTN_QT|ROPE_FUSE|DEBUG> (SHAPE_*, SOLO, KZ and
+ * which it does), KH_ATTN_WO (attention and wo in one launch at positions below it; 0 = in launches of their own), KH_PREFILL, KH_PG_<CHUNK|ROWS (the most slab rows that memory is given for)|PAIR|SHAPE_*|SOLO|KZ|ATTN|ATTN_QT|ROPE_FUSE|DEBUG> (SHAPE_*, SOLO, KZ and
  * DEBUG belong to the fp32-MFMA GEMMs; a SHAPE_* hook selects them), KH_PAIR_SHAPE (tile,K split of the pair GEMMs),
  * KH_PAIR_ATTN (0 = attention of a prompt slice on the fp32 matrix cores; KH_PG_ATTN_QT selects it too),
  * KH_SHAPE_DEBUG, KH_HY_DECODE (0 = single-token batches of layer-list models run on the pass kernels), KH_HY_EXPAND (0 = latent

@@ -1,6 +1,10 @@
 // kh_attn_wo.hip - launches of kh_attn_wo.h: attention and the output projection of a decoded token in one launch.
 #include "kh_attn_wo.h"
 
+#include <stdlib.h>
+
+#include <algorithm>
+
 #include "kh_model_internal.h"
 
 namespace khm {
@@ -8,13 +12,33 @@ namespace khm {
 // Which models take it, and in what shape.  fp32 weights; at most eight key / value groups of at most 512 columns (two float4 a
 // lane, ten heads), head sizes that the attention is instantiated for, vectors that two float4 a thread cover: every group is
 // one vector more that k_ffn13_parts stages (eight of 2048 floats cost it 0.9 us), and its keys and values are read by every
-// slice.  At most 2048 columns, whatever the threads of ffn13: k_pf_wo_parts keeps eight tokens' vectors in 64 KB.  us a launch at position 48, attention + wo -> one launch | ffn13: Llama-3.2-1B 3.4 + 4.5 -> 5.0 | 21.3 -> 22.2;
+// slice.  At most 2048 columns, whatever the threads of ffn13: k_pf_wo_parts keeps eight tokens' vectors in 64 KB.  us a launch at
+// position 48, attention + wo -> one launch | ffn13: Llama-3.2-1B 3.4 + 4.5 -> 5.0 | 21.3 -> 22.2;
 // TinyLlama 3.3 + 4.5 -> 4.9 | 15.5 -> 15.9; Qwen2.5-0.5B 3.4 + 2.6 -> 4.2 | 6.95 -> 7.15; stories15M 3.6 + 2.3 -> 3.9 | 2.4 -> 2.75.
-// A token: -3.9 / -6.1 / -8.4 / -12 %; with 200 - 240 positions -1.5 / -3 / -2 / -4 %.  From KH_ATTN_MIN_TS on attention is split over time.
-kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long) {
+// A token: -3.9 / -6.1 / -8.4 / -12 %; with 200 - 240 positions -2 / -2.4 / -1.9 / -3 %.  From KH_ATTN_MIN_TS on attention is split over time.
+namespace {
+// Positions below which the joint launch is the faster form.  Its time grows by some 1 us a layer from position 48 to 127 and by 0.4
+// more with the second tile a wave, for every slice reads its group's keys and values; what it saves is 1.3 - 2 us, less 0.1 a
+// part in ffn13, and up to 1 us more where wo has 1536 rows.  Slices of a part run on 8 / gcd(parts, 8) of the XCDs: 3, 5 and 7 parts
+// bring their keys into all of them.  Fitted to 85 geometries at eleven positions, us a layer saved at 16 / 112 / 192 (head size x heads -
+// groups; a layer is 14 - 32 us, models of one geometry differ by 0.2 among themselves): 64 x 8-8 1.6 / 0.7 / 0, 64 x 8-4 1.8 / 0.8 /
+// 0.1, 64 x 14-2 2.0 / 0.9 / 0.3, 64 x 16-4 1.5 / 0.6 / -0.1, 64 x 6-3 1.5 / 0.4 / -0.9, 64 x 12-6 1.3 / 0.1 / -0.6, 64 x 7-7 1.5 / -0.3 / -0.8, 64 x
+// 16-8 1.0 / 0.1 / -0.7, 64 x 24-8 2.0 / 0.9 / 0.4, 48 x 6-6 of stories15M 1.7 / 1.0 / 0.5, 48 x 16-8 1.2 / 0.4 / -0.1, 48 x 14-7 1.3 / -0.1 / -0.1,
+// 48 x 24-8 -0.3 / -0.9 / -1.3.  Of 85, 256 for all costs 29 up to 7 % at some position; these limits cost four 1 %, and one 3 %.
+// `staged`: floats of parts that the workgroups of ffn13 read.  From 1536 columns on they decide: 16 - 35 MB (Llama-3.2-1B 33.5) 1.6 / 0.7 / 0
+// and more, 38 MB 1.1 / 0.5 / -0.3, 50 - 67 MB 0.5 / 0 / -0.6.
+int joint_end(int dim, int head_size, int parts, long staged) {
+  if (dim >= 1536) return staged <= 8750000 ? 256 : (staged <= 11000000 ? 128 : 64);
+  if (parts == 8 && dim > 1024) return 0;
+  if (parts == 5 || parts == 7) return 64;
+  if (head_size == 48) return parts <= 4 || (parts == 6 && dim <= 576) ? 256 : 128;
+  return parts == 2 ? 256 : (parts == 1 || parts == 4 ? 192 : 128);
+}
+}  // namespace
+kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, const kh_model::Shape& ffn, int t_long) {
   kh_model::AttnWoPlan p;
-  const int hs = c.head_size, cols = c.kv_mul * hs, mv = kh_stage_maxv(c.dim, ffn_wg);
-  if (c.is_quant || dbg_off("KH_ATTN_WO") || (hs != 48 && hs != 64)) return p;
+  const int hs = c.head_size, cols = c.kv_mul * hs, mv = kh_stage_maxv(c.dim, ffn.wg);
+  if (c.is_quant || (hs != 48 && hs != 64)) return p;
   if (c.kv_head_num > KH_AWO_PARTS_MAX || cols > 512 || c.dim != c.head_num * hs || mv < 1 || mv > 2) return p;
   if ((size_t)KH_PF_BMAX * c.dim * sizeof(float) > (64u << 10)) return p;
   p.parts = c.kv_head_num;
@@ -31,8 +55,10 @@ kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long) {
   p.slices = slices(p.rw);
   if (p.parts * p.slices > 256) return kh_model::AttnWoPlan{};
   p.lds = attn_wo_lds_bytes(hs, c.kv_mul);
-  p.end = t_long - 1 < KH_ATTN_MIN_TS ? t_long - 1 : KH_ATTN_MIN_TS;  // one split, and no group path
-  return p;
+  const char* hook = dbg("KH_ATTN_WO");
+  const int pays = hook ? atoi(hook) : joint_end(c.dim, hs, p.parts, (long)ffn.grid * p.parts * c.dim);
+  p.end = std::min(pays, std::min(KH_ATTN_MIN_TS, t_long - 1));  // one split, and no group path
+  return p.end > 0 ? p : kh_model::AttnWoPlan{};
 }
 
 namespace {
@@ -128,7 +154,7 @@ extern "C" int kh_plan_attn_wo(int32_t dim, int32_t hidden_dim, int32_t head_num
   int32_t at[8];
   const int rc = kh_plan_attention(head_num, c.kv_mul, c.head_size, seq_len, 0, at);
   if (rc != KH_OK) return rc;
-  const kh_model::AttnWoPlan p = khm::plan_attn_wo(c, sh[2].wg, at[3]);
+  const kh_model::AttnWoPlan p = khm::plan_attn_wo(c, sh[2], at[3]);
   out4[0] = p.end > 0 ? p.end : 0;
   out4[1] = p.end > 0 ? p.parts : 0;
   out4[2] = p.end > 0 ? KH_AWO_WAVES * (64 / p.lpr) * p.rw : 0;

@@ -218,7 +218,7 @@ int graph_run(const kh_model* m, int s, int left);  // steps of the next graph a
 // the same for a graph of `nsteps` in {1, 2, 4, 8} steps (the tail of a run: 20 steps = 8 + 8 + 4)
 int step_graph_n(kh_model* m, int n_forced, int variant, int nsteps, hipGraphExec_t* out);
 // ---- kh_attn_wo.hip -------------------------------------------------------------------------
-kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, int ffn_wg, int t_long);
+kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, const kh_model::Shape& ffn, int t_long);
 void launch_attn_wo(kh_model* m, int l);
 void launch_ffn13_parts(kh_model* m, const KhFfn13Args& f);
 void launch_pf_attn_parts(kh_model* m, int l, int nvalid, int pos0);  // pf_q -> pf_att

@@ -585,7 +585,7 @@ int finish_create(kh_model* m, SinCosJob* sincos = nullptr) {
   }
   KH_ALLOC(m->part_val, (size_t)m->nparts);
   KH_ALLOC(m->part_idx, (size_t)m->nparts);
-  m->awo = plan_attn_wo(c, m->sh_ffn.wg, m->attn_t_long);
+  m->awo = plan_attn_wo(c, m->sh_ffn, m->attn_t_long);
   if (m->awo.end > 0) {
     KH_ALLOC(m->wo_part, (size_t)m->awo.parts * c.dim);
     KH_ALLOC(m->x1, (size_t)c.dim);

@@ -58,14 +58,16 @@ def test_wide_models_with_wide_workgroups(gpu, heads, kv, joint, monkeypatch):
 
 
 def test_profiles_name_what_is_launched(gpu):
-    """Below position 256 attention and wo are one launch and are reported as one; behind it each has its own time."""
+    """Below the end of their range attention and wo are one launch and are reported as one; behind it each has its own time."""
     from kuiperllama_amd import _ffi
     from kuiperllama_amd.model import KuiperModel
     spec = _SPECS["64x8-4"]
+    end = _ffi.plan_attn_wo(spec.dim, spec.hidden_dim, spec.n_heads, spec.n_kv_heads, spec.seq_len)["end"]
+    assert end == 192
     m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=31, device=gpu), spec)
     m.generate([1, 2], 300)
     joint, apart = ["qkv", "attn_wo", "ffn13", "w2", "cls", "sample"], ["qkv", "attn", "wo", "ffn13", "w2", "cls", "sample"]
-    for pos, names in ((0, joint), (64, joint), (255, joint), (256, apart), (290, apart)):
+    for pos, names in ((0, joint), (64, joint), (end - 1, joint), (end, apart), (290, apart)):
         us = m.profile_kernels(pos)
         assert sorted(us) == sorted(names) and min(us.values()) > 0.5, (pos, us)
         if names is joint:
@@ -106,12 +108,12 @@ def test_launches_of_their_own(gpu, oracle, name, monkeypatch):
     b.close()
 
 
-@pytest.mark.parametrize("pos0,n", [(4, 300), (251, 9), (0, 261)])
-def test_token_by_token_prompt_across_the_end(gpu, pos0, n):
+@pytest.mark.parametrize("name,pos0,n", [("64x8-4", 4, 300), ("64x8-4", 187, 9), ("64x8-4", 0, 197), ("64x32-8", 251, 9)])
+def test_token_by_token_prompt_across_the_end(gpu, name, pos0, n):
     """The prompt phase one token a step leaves the cache rows of predict() at every position, whatever its first one is: no graph
-    of several steps crosses position 256."""
+    of several steps crosses the end of the range, 192 or 256."""
     from kuiperllama_amd.model import KuiperModel
-    spec = _SPECS["64x8-4"]
+    spec = _SPECS[name]
     img = binfmt.synth_image(spec, seed=31, device=gpu, final_norm_std=1.0)
     a, b = KuiperModel.from_device_image(img, spec), KuiperModel.from_device_image(img, spec)
     toks = [int(t) for t in np.random.default_rng(4).integers(0, spec.vocab_size, pos0 + n)]
@@ -127,12 +129,38 @@ def test_token_by_token_prompt_across_the_end(gpu, pos0, n):
     b.close()
 
 
+@pytest.mark.parametrize("heads,kv,end", [(8, 4, 192), (12, 6, 128), (7, 7, 64), (14, 2, 256)])
+def test_bits_follow_from_the_position(gpu, heads, kv, end):
+    """Steps, graphs of several and the prompt path of several tokens across an end of the range that is not 256."""
+    from kuiperllama_amd import _ffi
+    from kuiperllama_amd.model import KuiperModel
+    spec = _spec(64 * heads, 1408, heads, kv, "end")
+    assert _ffi.plan_attn_wo(spec.dim, 1408, heads, kv, spec.seq_len)["end"] == end
+    img = binfmt.synth_image(spec, seed=31, device=gpu, final_norm_std=1.0)
+    a, b = KuiperModel.from_device_image(img, spec), KuiperModel.from_device_image(img, spec)
+    toks = [int(t) for t in np.random.default_rng(6).integers(0, spec.vocab_size, end + 11)]
+    for pos, t in enumerate(toks):
+        a.predict(t, pos, exec="fused")
+    b.prefill(toks[:-1], 0)
+    b.predict(toks[-1], len(toks) - 1, exec="fused")
+    for l in range(spec.n_layers):
+        for x, y in zip(a.read_kv(l, 0, len(toks)), b.read_kv(l, 0, len(toks))):
+            np.testing.assert_array_equal(x, y)
+    assert np.array_equal(a.logits(), b.logits())
+    words, _ = a.generate(toks[:3], end + 21, exec="graph")
+    assert words == b.generate(toks[:3], end + 21, exec="fused")[0]
+    assert np.array_equal(a.logits(), b.logits())
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("name", sorted(_SPECS))
-def test_against_the_oracle_and_the_prompt_path(gpu, oracle, name):
+def test_against_the_oracle_and_the_prompt_path(gpu, oracle, name, monkeypatch):
     """Logits within the bound of fp32 decode steps (4e-5, as for the attention in launches of its own); the prompt path of
     several tokens a weight pass leaves the same bits, also where a chunk would cross the end of the range; words of captured and
     eager steps are the same across it."""
     from kuiperllama_amd.model import KuiperModel
+    monkeypatch.setenv("KH_ATTN_WO", "256")  # the whole range that the kernels have, wherever they pay
     spec = _SPECS[name]
     img_d = binfmt.synth_image(spec, seed=31, device=gpu, final_norm_std=1.0)  # words that wander
     torch.cuda.synchronize()

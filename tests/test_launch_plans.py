@@ -109,6 +109,25 @@ def test_attention_and_wo_in_one_round_of_workgroups(head_size, monkeypatch):
     assert not _ffi.plan_attn_wo(2048, 8192, 32, 8, 512, True)["end"] and not _ffi.plan_attn_wo(2048, 8192, 16, 8, 512)["end"]
 
 
+def test_attention_and_wo_in_one_launch_as_far_as_it_pays(monkeypatch):
+    """The presets take it at all positions below 256; geometries of many parts as far as they gain."""
+    monkeypatch.delenv("KH_ATTN_WO", raising=False)
+    for name, end in (("stories15M", 256), ("qwen2.5-0.5b", 256), ("tinyllama-1.1b", 256), ("llama3.2-1b", 256), ("llama2-7b", 0)):
+        sp = binfmt.PRESETS[name]
+        assert _ffi.plan_attn_wo(sp.dim, sp.hidden_dim, sp.n_heads, sp.n_kv_heads, 512)["end"] == end, name
+    for size, heads, kv, end in ((64, 8, 8, 128), (64, 8, 4, 192), (64, 8, 2, 256), (64, 8, 1, 192), (64, 7, 7, 64), (64, 6, 3, 128), (64, 12, 6, 128),
+                                 (64, 16, 8, 128), (64, 24, 8, 256), (48, 16, 8, 128), (48, 14, 7, 64), (48, 24, 8, 0), (48, 12, 6, 256), (48, 18, 6, 128)):
+        assert _ffi.plan_attn_wo(size * heads, 8192, heads, kv, 512)["end"] == end, (size, heads, kv)
+    for dim, hidden, heads, kv, end in ((1536, 4096, 24, 8, 64), (1536, 3072, 24, 8, 128), (1536, 4096, 24, 4, 256), (2048, 4096, 32, 8, 64),
+                                        (2048, 4096, 32, 4, 256), (1536, 4224, 24, 8, 256)):  # 1024, 768 or 512 workgroups in ffn13
+        assert _ffi.plan_attn_wo(dim, hidden, heads, kv, 512)["end"] == end, (dim, hidden, kv)
+    assert _ffi.plan_attn_wo(2048, 8192, 32, 8, 512)["end"] == 256 and _ffi.plan_attn_wo(2048, 8192, 32, 8, 100)["end"] == 256
+    monkeypatch.setenv("KH_ATTN_WO", "100")
+    assert _ffi.plan_attn_wo(64 * 16, 2816, 16, 8, 512)["end"] == 100
+    monkeypatch.setenv("KH_ATTN_WO", "0")
+    assert _ffi.plan_attn_wo(2048, 8192, 32, 8, 512)["end"] == 0
+
+
 def test_decode_plan_int8_wide_rows_keep_the_small_tile():
     """int8 rows that need more than four 16-byte loads per lane walk several tiles of TWO loads (qkv / wo / ffn13 /
     cls; w2 takes two tiles of three where that is exact) - never the fp32 rule's 4 or 8.  Geometries wider than any
