@@ -20,19 +20,39 @@ namespace {
 // Positions below which the joint launch is the faster form.  Its time grows by some 1 us a layer from position 48 to 127 and by 0.4
 // more with the second tile a wave, for every slice reads its group's keys and values; what it saves is 1.3 - 2 us, less 0.1 a
 // part in ffn13, and up to 1 us more where wo has 1536 rows.  Slices of a part run on 8 / gcd(parts, 8) of the XCDs: 3, 5 and 7 parts
-// bring their keys into all of them.  Fitted to 85 geometries at eleven positions, us a layer saved at 16 / 112 / 192 (head size x heads -
-// groups; a layer is 14 - 32 us, models of one geometry differ by 0.2 among themselves): 64 x 8-8 1.6 / 0.7 / 0, 64 x 8-4 1.8 / 0.8 /
-// 0.1, 64 x 14-2 2.0 / 0.9 / 0.3, 64 x 16-4 1.5 / 0.6 / -0.1, 64 x 6-3 1.5 / 0.4 / -0.9, 64 x 12-6 1.3 / 0.1 / -0.6, 64 x 7-7 1.5 / -0.3 / -0.8, 64 x
-// 16-8 1.0 / 0.1 / -0.7, 64 x 24-8 2.0 / 0.9 / 0.4, 48 x 6-6 of stories15M 1.7 / 1.0 / 0.5, 48 x 16-8 1.2 / 0.4 / -0.1, 48 x 14-7 1.3 / -0.1 / -0.1,
-// 48 x 24-8 -0.3 / -0.9 / -1.3.  Of 85, 256 for all costs 29 up to 7 % at some position; these limits cost four 1 %, and one 3 %.
-// `staged`: floats of parts that the workgroups of ffn13 read.  From 1536 columns on they decide: 16 - 35 MB (Llama-3.2-1B 33.5) 1.6 / 0.7 / 0
-// and more, 38 MB 1.1 / 0.5 / -0.3, 50 - 67 MB 0.5 / 0 / -0.6.
+// bring their keys into all of them.  `staged`: floats of parts that the workgroups of ffn13 read; from 1536 columns on they decide.
+// Fitted to 85 geometries at eight positions, each as a model of 8 layers and as one of 18 - 24, which gain more behind position 100.
+// Per cent of a step saved at position 16 / 80 / 144 / 208 (head size x heads - groups; 1 % from one instance of a model to the next):
+//                             8 layers                   18 - 24 layers
+//   48 x 6-6 (stories15M)     11.9   7.0   4.1   2.5     12.7   4.6   0.9   1.8
+//   48 x 15-5                  8.3   4.8   1.6  -0.8      9.2   5.0   4.5   4.5
+//   48 x 24-6                  1.8  -0.3  -1.0  -1.3      2.2   0.8  -0.9  -1.6
+//   48 x 28-7                  0.8  -1.6  -2.9  -2.1      0.6   0.1  -1.3  -1.6
+//   48 x 24-8                 -1.9  -4.3  -6.0  -6.5     -1.2  -3.0  -4.0  -4.6
+//   64 x 12-3                 10.2   5.1   2.5  -0.2     10.9   4.3   3.4   3.2
+//   64 x 16-4                  7.0   2.2  -0.6  -2.0      8.0   4.0   2.0   0.8
+//   64 x 15-5                  6.5   2.4  -3.2  -3.3      6.3   3.3   1.2   0.3
+//   64 x 12-6                  8.3   3.7   0.6  -1.3      8.6   3.0   1.7   1.2
+//   64 x 18-6                  1.7  -1.0  -3.5  -4.4      2.6   0.8  -1.6  -2.6
+//   64 x 14-7                  5.4  -0.9  -4.1  -4.1      5.0   1.8   0.4  -0.3
+//   64 x 8-8                  10.5   4.9   1.2   0.1     10.6   4.9   2.7   1.5
+//   64 x 16-8                  4.9   0.5  -2.7  -3.6      5.6   2.1   0.1  -1.0
+//   64 x 24-8, 3072 hidden     3.8   0.6  -1.5  -2.3      4.0   1.3  -0.4  -0.4    9.4 million staged
+//   64 x 32-8, 4096            1.8  -0.4  -1.1  -2.3      2.0   0.0  -0.4  -0.9   16.8 million
+//   64 x 32-8, 8192            3.6   1.9   1.1   0.3      5.0   3.2   2.5   2.0    8.4 million (Llama-3.2-1B)
+// Mean of positions 0 - 255 over all 85: 3.3 and 4.2 %; with 256 for all of them 3.0 and 4.1, 19 of them slower at some position.
 int joint_end(int dim, int head_size, int parts, long staged) {
   if (dim >= 1536) return staged <= 8750000 ? 256 : (staged <= 11000000 ? 128 : 64);
-  if (parts == 8 && dim > 1024) return 0;
-  if (parts == 5 || parts == 7) return 64;
-  if (head_size == 48) return parts <= 4 || (parts == 6 && dim <= 576) ? 256 : 128;
-  return parts == 2 ? 256 : (parts == 1 || parts == 4 ? 192 : 128);
+  const bool wide = dim >= 1024;
+  if (head_size == 48) return !wide || parts <= 5 ? 256 : (parts == 6 ? 128 : (parts == 7 ? 64 : 0));
+  switch (parts) {
+    case 4: return wide ? 192 : 256;
+    case 5: return 128;
+    case 6: return wide ? 64 : 192;
+    case 7: return wide ? 64 : 128;
+    case 8: return wide ? 128 : 256;
+    default: return 256;
+  }
 }
 }  // namespace
 kh_model::AttnWoPlan plan_attn_wo(const kh_config& c, const kh_model::Shape& ffn, int t_long) {

@@ -18,7 +18,7 @@ def _spec(dim, hidden, heads, kv, name):
 # of which the second is half empty (seven heads), one and two rows, rows past the end of the last slice (dim 896, 1088)
 _SPECS = {s.name: s for s in (
     _spec(288, 768, 6, 6, "48x6-6"), _spec(384, 768, 8, 4, "48x8-4"), _spec(512, 1408, 8, 4, "64x8-4"),
-    _spec(448, 1216, 7, 1, "64x7-1"), _spec(896, 1216, 14, 2, "64x14-2"), _spec(1024, 1408, 16, 8, "64x16-8"),
+    _spec(448, 1216, 7, 1, "64x7-1"), _spec(768, 2112, 12, 6, "64x12-6"), _spec(896, 1216, 14, 2, "64x14-2"), _spec(1024, 1408, 16, 8, "64x16-8"),
     _spec(1088, 1408, 17, 1, "64x17-1"),  # seventeen heads a group: the launches of their own
     _spec(2048, 1408, 32, 8, "64x32-8"), _spec(2048, 1408, 32, 4, "64x32-4"))}
 
@@ -61,7 +61,7 @@ def test_profiles_name_what_is_launched(gpu):
     """Below the end of their range attention and wo are one launch and are reported as one; behind it each has its own time."""
     from kuiperllama_amd import _ffi
     from kuiperllama_amd.model import KuiperModel
-    spec = _SPECS["64x8-4"]
+    spec = _SPECS["64x12-6"]
     end = _ffi.plan_attn_wo(spec.dim, spec.hidden_dim, spec.n_heads, spec.n_kv_heads, spec.seq_len)["end"]
     assert end == 192
     m = KuiperModel.from_device_image(binfmt.synth_image(spec, seed=31, device=gpu), spec)
@@ -108,7 +108,7 @@ def test_launches_of_their_own(gpu, oracle, name, monkeypatch):
     b.close()
 
 
-@pytest.mark.parametrize("name,pos0,n", [("64x8-4", 4, 300), ("64x8-4", 187, 9), ("64x8-4", 0, 197), ("64x32-8", 251, 9)])
+@pytest.mark.parametrize("name,pos0,n", [("64x12-6", 4, 300), ("64x12-6", 187, 9), ("64x12-6", 0, 197), ("64x32-8", 251, 9)])
 def test_token_by_token_prompt_across_the_end(gpu, name, pos0, n):
     """The prompt phase one token a step leaves the cache rows of predict() at every position, whatever its first one is: no graph
     of several steps crosses the end of the range, 192 or 256."""
@@ -129,7 +129,7 @@ def test_token_by_token_prompt_across_the_end(gpu, name, pos0, n):
     b.close()
 
 
-@pytest.mark.parametrize("heads,kv,end", [(8, 4, 192), (12, 6, 128), (7, 7, 64), (14, 2, 256)])
+@pytest.mark.parametrize("heads,kv,end", [(12, 6, 192), (10, 5, 128), (21, 7, 64), (14, 2, 256)])
 def test_bits_follow_from_the_position(gpu, heads, kv, end):
     """Steps, graphs of several and the prompt path of several tokens across an end of the range that is not 256."""
     from kuiperllama_amd import _ffi

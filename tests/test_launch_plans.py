@@ -115,8 +115,9 @@ def test_attention_and_wo_in_one_launch_as_far_as_it_pays(monkeypatch):
     for name, end in (("stories15M", 256), ("qwen2.5-0.5b", 256), ("tinyllama-1.1b", 256), ("llama3.2-1b", 256), ("llama2-7b", 0)):
         sp = binfmt.PRESETS[name]
         assert _ffi.plan_attn_wo(sp.dim, sp.hidden_dim, sp.n_heads, sp.n_kv_heads, 512)["end"] == end, name
-    for size, heads, kv, end in ((64, 8, 8, 128), (64, 8, 4, 192), (64, 8, 2, 256), (64, 8, 1, 192), (64, 7, 7, 64), (64, 6, 3, 128), (64, 12, 6, 128),
-                                 (64, 16, 8, 128), (64, 24, 8, 256), (48, 16, 8, 128), (48, 14, 7, 64), (48, 24, 8, 0), (48, 12, 6, 256), (48, 18, 6, 128)):
+    for size, heads, kv, end in ((64, 8, 1, 256), (64, 14, 2, 256), (64, 18, 3, 256), (64, 15, 5, 128), (64, 20, 5, 128), (64, 8, 4, 256), (64, 16, 4, 192),
+                                 (64, 12, 6, 192), (64, 18, 6, 64), (64, 14, 7, 128), (64, 21, 7, 64), (64, 8, 8, 256), (64, 16, 8, 128), (64, 24, 8, 256),
+                                 (48, 30, 5, 256), (48, 18, 6, 256), (48, 24, 6, 128), (48, 21, 7, 256), (48, 28, 7, 64), (48, 16, 8, 256), (48, 24, 8, 0)):
         assert _ffi.plan_attn_wo(size * heads, 8192, heads, kv, 512)["end"] == end, (size, heads, kv)
     for dim, hidden, heads, kv, end in ((1536, 4096, 24, 8, 64), (1536, 3072, 24, 8, 128), (1536, 4096, 24, 4, 256), (2048, 4096, 32, 8, 64),
                                         (2048, 4096, 32, 4, 256), (1536, 4224, 24, 8, 256)):  # 1024, 768 or 512 workgroups in ffn13
